@@ -158,7 +158,7 @@ pack_means_bf16_kernel(const float* __restrict__ means, size_t stride_means, flo
 bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev)
 {
 	const uint32_t kb = pick_kb(a.dim);
-	if (kb == 0) return false;
+	if (kb == 0) return !a.ranking_only && wide_supports(a, dev);
 	/* two tiles (the double-buffered stream of the centroid block) plus the static flag lists must fit */
 	return (size_t)(tile_floats(KBLOCK * kb + ROW_PAD) + NORM_TILE) * 4 * 2 + 2 * FLAG_CAP * MFMA_WAVES * 4 + 1024 <= dev.lds_bytes;
 }
@@ -192,6 +192,7 @@ int launch_screen_bf16(const float* rows, const Workspace* ws, const uint32_t* r
 
 int launch_assign_bf16(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
+	if (args.dim > 256) return launch_assign_wide(args, exec, ws, dev);
 	AssignArgs a = args;
 	/* wide rows and many centroids: a second sweep screens the queued points (narrow rows fit the registers of the
 	 * lane-per-centroid kernels, which then need fewer launches); so do the packed rows, whose sweep queues more points

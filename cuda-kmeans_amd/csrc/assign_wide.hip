@@ -1,0 +1,584 @@
+/*
+ * Assignment of rows of more than 256 dimensions on the matrix cores. The sweeps of the narrower rows (assign_bf16_impl.h)
+ * keep the split operands of whole point rows in registers; a row of 512 dimensions does not fit there. Here a work-group
+ * stages the rows of its points in LDS instead, 64 dimensions at a time, converted to bf16 once, and its eight wavefronts
+ * share them: every wavefront owns centroid tiles of its own, whose packed operands it reads straight from the caches (no two
+ * wavefronts of a work-group want the same ones, so LDS would only add a copy).
+ *
+ * Ranking, split operands and certificates are those of assign_bf16.hip: a[j] = |c_j|^2 - 2 c_j . x by
+ * v_mfma_f32_32x32x16_bf16, either the hi parts alone (the first level: all points) or three products (the second level: the
+ * points the first could not settle; the only level of small inputs). What three products cannot settle goes to the exact pass.
+ *
+ * Split of the work. Per block of 16 dimensions a wavefront reads the operands of its NT centroid tiles (1 KB each, global)
+ * and of the PT point tiles (1 KB each, LDS) for NT * PT MFMAs of 32 cycles; with NT = 2, PT = 4 the four SIMDs of a compute
+ * unit ask the LDS for 64 and the vector cache for 32 of their 128 / 64 bytes per cycle, and all centroids pass by 128 points
+ * at a time. The alternatives: PT = 2 doubles the cache traffic (at its limit), NT = 4 does not fit the registers.
+ * The rows of a unit are read from memory once while 512 centroids go by; with more centroids the converted rows stay in LDS
+ * if they fit (d <= 512 in the first level), otherwise they are staged again per group of 512.
+ *
+ * N = 131071, d = 512, k = 400, one iteration: the lane-per-point kernel that took these rows before needed 147 ms.
+ */
+#include "assign_bf16_impl.h"
+
+namespace kmx {
+
+constexpr uint32_t WIDE_THREADS = 512;
+constexpr uint32_t WIDE_WAVES = WIDE_THREADS / WAVE;
+constexpr uint32_t WIDE_CHUNK = 64;                       /* dimensions staged at a time */
+constexpr uint32_t WIDE_BLOCKS = WIDE_CHUNK / KBLOCK;     /* MFMA blocks of a chunk */
+constexpr uint32_t WIDE_LIST = 512;                       /* points waiting for the queue, per work-group */
+constexpr uint32_t WIDE_ROW_PAD = 4;                      /* 16-byte units: the two half-waves' units of a block start 64 bytes apart modulo the banks */
+
+/* the norms array: tiles of |c - m|^2, per row sum c'mid^2 and sum c'rest^2, the frame m (dp floats, |m|^2, an upper bound of |m|), tiles of |c|^2 */
+__host__ __device__ __forceinline__ size_t wide_exact_norms_offset(uint32_t kp, uint32_t dp) { return frame_offset(kp) + dp + 4; }
+__host__ __device__ __forceinline__ size_t wide_norms_floats(uint32_t kp, uint32_t dp) { return wide_exact_norms_offset(kp, dp) + split_norms_offset(kp); }
+/* the packed centroids: plane of hi parts, plane of mid parts of -2 (c - m); inside a plane per tile and block the 64 lanes' 16-byte operands */
+__host__ __device__ __forceinline__ size_t wide_plane_units(uint32_t kp, uint32_t dp) { return (size_t)(kp / TILE) * (dp / KBLOCK) * WAVE; }
+
+struct WideArgs {
+	const float* data; size_t stride;
+	const bf16x8* packed; const float* norms;
+	uint32_t* assignment; uint32_t* queue; uint32_t* counters;
+	const uint32_t* list; const uint32_t* list_length;
+	uint32_t dim, dp, k, kp, n, buffers;
+	float kd, kd_unmoved;
+};
+
+/* One wavefront per (padded) centroid row; the frame as in sweep_frame, for any row length, computed by every work-group into LDS. */
+template <int LM>
+__global__ void __launch_bounds__(256)
+pack_means_wide_kernel(const float* __restrict__ means, size_t stride_means, __bf16* __restrict__ packed, float* __restrict__ norms,
+                       float* __restrict__ means_t, uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t moved, uint32_t* __restrict__ counters)
+{
+	extern __shared__ float m[]; /* dp floats */
+	constexpr uint32_t SAMPLE = 16;
+	const uint32_t lane = threadIdx.x & (WAVE - 1);
+	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; }
+	const uint32_t sample = min(k, SAMPLE);
+	for (uint32_t q = threadIdx.x; q < dp; q += 256) {
+		float sum = 0.0f;
+		if (moved && q < dim) {
+			float v[SAMPLE];
+#pragma unroll
+			for (uint32_t r = 0; r < SAMPLE; ++r) v[r] = r < sample ? means[elem<LM>(stride_means, r, q)] : 0.0f;
+#pragma unroll
+			for (uint32_t r = 0; r < SAMPLE; ++r) sum += __builtin_fabsf(v[r]) < __builtin_inff() ? v[r] : 0.0f;
+			sum = sum / (float)sample;
+			sum = __builtin_fabsf(sum) < __builtin_inff() ? sum : 0.0f;
+		}
+		m[q] = sum;
+	}
+	__syncthreads();
+	if (blockIdx.x == 0) {
+		float* stored = norms + frame_offset(kp);
+		for (uint32_t q = threadIdx.x; q < dp; q += 256) stored[q] = m[q];
+		if (threadIdx.x < WAVE) {
+			float m2 = 0.0f;
+			for (uint32_t q = threadIdx.x; q < dp; q += WAVE) m2 += m[q] * m[q];
+			for (int off = 32; off > 0; off >>= 1) m2 += __shfl_xor(m2, off);
+			if (threadIdx.x == 0) { stored[dp] = m2; stored[dp + 1] = __builtin_sqrtf(m2) * 1.0001f; }
+		}
+	}
+	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+	if (j >= kp) return;
+	const size_t plane = wide_plane_units(kp, dp) * 8;
+	float c2 = 0.0f, mid2 = 0.0f, rest2 = 0.0f, exact2 = 0.0f;
+	for (uint32_t q = lane; q < dp; q += WAVE) {
+		const bool there = j < k && q < dim;
+		const float exact = there ? means[elem<LM>(stride_means, j, q)] : 0.0f;
+		const float v = there ? exact - m[q] : 0.0f;
+		exact2 += exact * exact;
+		c2 += v * v;
+		__bf16 hi, mid;
+		const float rest = split_bf16(-2.0f * v, hi, mid);
+		mid2 += (float)mid * (float)mid;
+		rest2 += rest * rest;
+		const size_t at = (((size_t)(j / TILE) * (dp / KBLOCK) + q / KBLOCK) * WAVE + (q % KBLOCK) / 8 * TILE + j % TILE) * 8 + q % 8;
+		packed[at] = hi;
+		packed[plane + at] = mid;
+		if (q < dim) means_t[(size_t)q * kp + j] = exact; /* exact copy for the exact pass */
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) {
+		c2 += __shfl_xor(c2, off);
+		mid2 += __shfl_xor(mid2, off);
+		rest2 += __shfl_xor(rest2, off);
+		exact2 += __shfl_xor(exact2, off);
+	}
+	if (lane == 0) {
+		norms[norm_at(j)] = j < k ? c2 : __builtin_inff();
+		norms[wide_exact_norms_offset(kp, dp) + norm_at(j)] = j < k ? exact2 : __builtin_inff();
+		norms[split_norms_offset(kp) + j] = mid2;
+		norms[split_norms_offset(kp) + kp + j] = rest2;
+	}
+	if (lane < NORM_TILE - TILE && j % TILE == 0) {
+		norms[(j / TILE) * NORM_TILE + TILE + lane] = __builtin_inff();
+		norms[wide_exact_norms_offset(kp, dp) + (j / TILE) * NORM_TILE + TILE + lane] = __builtin_inff();
+	}
+}
+
+/*
+ * PT point tiles of 32 per unit, NT centroid tiles per wavefront and group (a group: the WIDE_WAVES * NT tiles that go by together),
+ * X3: three products instead of the hi parts alone. LISTED: the points of a list (entries of two words, the first the point number).
+ *
+ * Order of a step (one chunk of 64 dimensions against one group): the operands of the chunk's four blocks are in registers,
+ * each block's are replaced by those of the next step as soon as its MFMAs have been issued; the B operands of block b + 1
+ * are requested from LDS before the MFMAs of block b. After the step the rows requested a step ago are converted and written to the next
+ * buffer, and the chunk after them is requested: every load has a whole step (NT * PT * 4 MFMAs per wavefront, two wavefronts
+ * on a SIMD: about a microsecond in the first level) to arrive. Loads retire in order, hence the rows are requested after all of
+ * the step's operand loads.
+ * Ranking values carry the number of their result (4 or 5 bits) in the lowest mantissa bits, as in the single-pass kernels
+ * (cert_kd_keyed): three operations per value for the two smallest and the place of the smallest. A NaN anywhere makes the smallest
+ * NaN (v_minimum3_f32 passes it on), which certifies nothing.
+ */
+template <int PT, int NT, bool X3, int LD, bool VEC, bool LISTED>
+__global__ void __launch_bounds__(WIDE_THREADS)
+wide_sweep_kernel(const WideArgs w)
+{
+	constexpr uint32_t ROWS = PT * TILE;
+	constexpr uint32_t SUBS = WIDE_THREADS / ROWS;          /* lanes that stage one row */
+	constexpr uint32_t VECS = WIDE_CHUNK / 4 / SUBS;        /* 4-dimension pieces per lane and chunk */
+	constexpr uint32_t UNIT_STRIDE = ROWS + WIDE_ROW_PAD;   /* 16-byte units between the half-blocks of a chunk */
+	constexpr uint32_t PART_UNITS = 2 * WIDE_BLOCKS * UNIT_STRIDE;
+	constexpr uint32_t BUFFER_UNITS = (X3 ? 2 : 1) * PART_UNITS;
+	constexpr uint32_t GROUP_TILES = WIDE_WAVES * NT;
+	constexpr uint32_t KEY_MASK = NT * 16 - 1;
+	static_assert(VECS * SUBS * 4 == WIDE_CHUNK && NT <= 2, "shape");
+
+	extern __shared__ __attribute__((aligned(16))) float dyn[];
+	float* frame = dyn;                            /* dp floats (a multiple of 64) */
+	bf16x8* rows_lds = (bf16x8*)(dyn + w.dp);      /* w.buffers buffers of BUFFER_UNITS */
+	__shared__ float cand_first[WIDE_WAVES][ROWS], cand_second[WIDE_WAVES][ROWS];
+	__shared__ uint32_t cand_idx[WIDE_WAVES][ROWS];
+	__shared__ float row_info[3][ROWS];            /* |x|^2, squared norm of the part the products drop, (x - m) . m */
+	__shared__ __attribute__((aligned(16))) float norm_stage[WIDE_WAVES][NT * TILE];
+	__shared__ uint32_t flags[2 * WIDE_LIST];
+	__shared__ uint32_t flag_count, flag_base;
+	__shared__ uint32_t wave_max[3][WIDE_WAVES];
+
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
+	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	const uint32_t col = lane & 31, h = lane >> 5;
+	const uint32_t n = LISTED ? min(w.list_length[0], w.n) : w.n;
+	const uint32_t units = (n + ROWS - 1) / ROWS;
+	const uint32_t tiles = w.kp / TILE;
+	const uint32_t groups = (tiles + GROUP_TILES - 1) / GROUP_TILES;
+	const uint32_t chunks = w.dp / WIDE_CHUNK;
+	const uint32_t blocks = w.dp / KBLOCK;
+	const bool resident = w.buffers >= chunks;
+	const uint32_t steps = groups * chunks;
+	const uint32_t staged_steps = resident ? chunks : steps;
+	if (blockIdx.x >= units) return; /* the whole work-group */
+
+	/* the certificate's maxima over the centroids (bit patterns: NaN and infinity win) and the frame */
+	if (tid == 0) flag_count = 0u;
+	for (uint32_t q = tid; q < w.dp; q += WIDE_THREADS) frame[q] = w.norms[frame_offset(w.kp) + q];
+	const float m2 = w.norms[frame_offset(w.kp) + w.dp], mnorm = w.norms[frame_offset(w.kp) + w.dp + 1];
+	CertCoeffs cert;
+	{
+		const float* part_norms = w.norms + split_norms_offset(w.kp);
+		uint32_t most[3] = { 0u, 0u, 0u };
+		for (uint32_t j = tid; j < w.k; j += WIDE_THREADS) {
+			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
+			most[1] = max(most[1], __float_as_uint(part_norms[j]));
+			most[2] = max(most[2], __float_as_uint(part_norms[w.kp + j]));
+		}
+#pragma unroll
+		for (int q = 0; q < 3; ++q) {
+			for (int off = WAVE / 2; off > 0; off >>= 1) most[q] = max(most[q], (uint32_t)__shfl_xor((int)most[q], off));
+			if (lane == 0) wave_max[q][wave] = most[q];
+		}
+		__syncthreads();
+#pragma unroll
+		for (int q = 0; q < 3; ++q) {
+			most[q] = 0;
+			for (uint32_t v = 0; v < WIDE_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
+		}
+		const CentroidBounds cb{ __uint_as_float(most[0]), __uint_as_float(most[1]), __uint_as_float(most[2]) };
+		cert = X3 ? cert_coeffs_split(cb) : cert_coeffs_level1(cb);
+	}
+
+	/* staging: this lane's row of the unit and its pieces of a chunk */
+	const uint32_t row = LD == KMX_AOS ? tid / SUBS : tid % ROWS;
+	const uint32_t sub = LD == KMX_AOS ? tid % SUBS : tid / ROWS;
+	f32x4 piece[VECS];
+	auto point_of = [&](uint32_t unit) -> uint32_t { /* rows beyond the end repeat the last one */
+		const uint32_t slot = min(unit * ROWS + row, n - 1);
+		return LISTED ? w.list[2 * (size_t)slot] : slot;
+	};
+	auto request_rows = [&](uint32_t pt, uint32_t chunk) {
+#pragma unroll
+		for (uint32_t i = 0; i < VECS; ++i) {
+			const uint32_t d = chunk * WIDE_CHUNK + (i * SUBS + sub) * 4;
+			f32x4 v = { 0.0f, 0.0f, 0.0f, 0.0f };
+			/* (pieces beyond the row repeat its end: no branches around the loads; store_rows puts zeros there) */
+			if (LD == KMX_AOS) {
+				typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4))); /* 16-byte loads need no more than 4-byte alignment */
+				const float* at = w.data + (size_t)pt * w.stride + min(d, w.dim - 4);
+				if constexpr (VEC) v = *(const f32x4*)at;
+				else v = *(const f32x4_any*)at;
+			}
+			else {
+#pragma unroll
+				for (uint32_t e = 0; e < 4; ++e) v[e] = w.data[elem<LD>(w.stride, pt, min(d + e, w.dim - 1))];
+			}
+			piece[i] = v;
+		}
+	};
+	float xx = 0.0f, xpart = 0.0f, xalong = 0.0f;
+	auto store_rows = [&](uint32_t buffer, uint32_t chunk, bool first_pass) {
+		typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+		char* base = (char*)(rows_lds + (size_t)buffer * BUFFER_UNITS);
+#pragma unroll
+		for (uint32_t i = 0; i < VECS; ++i) {
+			const uint32_t f = i * SUBS + sub;
+			const f32x4 mv = *(const f32x4*)(frame + chunk * WIDE_CHUNK + f * 4);
+			if constexpr (LD == KMX_AOS && !VEC) {
+				/* the piece that holds the end of a row whose length is no multiple of four came from up to three places before */
+				const uint32_t d = chunk * WIDE_CHUNK + f * 4;
+				if ((chunk + 1) * WIDE_CHUNK > w.dim && d + 4 > w.dim && d < w.dim) {
+					const f32x4 p = piece[i];
+					const uint32_t s = d + 4 - w.dim;
+					piece[i].x = s == 1 ? p.y : s == 2 ? p.z : p.w;
+					piece[i].y = s == 1 ? p.z : p.w;
+					piece[i].z = p.w;
+				}
+			}
+			bf16x4 hi, mid;
+			float a = 0.0f, b = 0.0f, c = 0.0f;
+#pragma unroll
+			for (int e = 0; e < 4; ++e) {
+				const float v = chunk * WIDE_CHUNK + f * 4 + e < w.dim ? piece[i][e] - mv[e] : 0.0f;
+				__bf16 vh, vm;
+				split_bf16(v, vh, vm);
+				hi[e] = vh;
+				mid[e] = vm;
+				const float low = X3 ? (float)vm : v - (float)vh;
+				a += v * v;
+				b += low * low;
+				c += v * mv[e];
+			}
+			if (first_pass) { xx += a; xpart += b; xalong += c; }
+			char* at = base + ((f / 2) * UNIT_STRIDE + row) * 16 + (f % 2) * 8;
+			*(bf16x4*)at = hi;
+			if constexpr (X3) *(bf16x4*)(at + PART_UNITS * 16) = mid;
+		}
+	};
+
+	/* this wavefront's tile of a group (beyond the last tile: the last one again, with infinite norms) */
+	auto tile_of = [&](uint32_t group, int nt) -> uint32_t { return group * GROUP_TILES + nt * WIDE_WAVES + wave; };
+	const size_t plane = wide_plane_units(w.kp, w.dp);
+	const bf16x8* next_ops[NT]; /* operands of the next step */
+	uint32_t next_chunk = 0, next_group = 0;
+	auto seek = [&]() {
+#pragma unroll
+		for (int nt = 0; nt < NT; ++nt)
+			next_ops[nt] = w.packed + ((size_t)min(tile_of(next_group, nt), tiles - 1) * blocks + next_chunk * WIDE_BLOCKS) * WAVE;
+	};
+	auto advance = [&]() {
+		if (++next_chunk == chunks) {
+			next_chunk = 0;
+			if (++next_group == groups) next_group = 0;
+		}
+		seek();
+	};
+	bf16x8 ahi[WIDE_BLOCKS][NT], amid[X3 ? WIDE_BLOCKS : 1][NT];
+	auto fetch_ops = [&](int b) {
+#pragma unroll
+		for (int nt = 0; nt < NT; ++nt) {
+			ahi[b][nt] = next_ops[nt][b * WAVE + lane];
+			if constexpr (X3) amid[b][nt] = (next_ops[nt] + plane)[b * WAVE + lane];
+		}
+	};
+	/* |c|^2 of this wavefront's tiles of a group, one per lane; requested a group ahead */
+	float norm_reg = 0.0f;
+	auto request_norms = [&](uint32_t group) {
+		const uint32_t tile = tile_of(group, NT == 2 ? (int)h : 0);
+		/* rows that do not exist: beyond all values, but finite (a number in the low bits would make infinity a NaN) */
+		norm_reg = tile * TILE + col < w.k ? w.norms[tile * NORM_TILE + col] : 1.7e38f;
+	};
+
+	uint32_t unit = blockIdx.x;
+	uint32_t pt = point_of(unit);
+	request_norms(0);
+	seek();
+#pragma unroll
+	for (int b = 0; b < (int)WIDE_BLOCKS; ++b) fetch_ops(b);
+	advance();
+	request_rows(pt, 0);
+	const uint32_t uniform_n = n;
+
+	for (; unit < units; unit += gridDim.x) {
+		const uint32_t next_pt = unit + gridDim.x < units ? point_of(unit + gridDim.x) : pt;
+		float best[PT], second[PT];
+		uint32_t best_idx[PT];
+#pragma unroll
+		for (int p = 0; p < PT; ++p) { best[p] = __builtin_inff(); second[p] = __builtin_inff(); best_idx[p] = 0; }
+		xx = xpart = xalong = 0.0f;
+		store_rows(0, 0, true);
+		if (staged_steps > 1) request_rows(pt, 1 % chunks);
+		else request_rows(next_pt, 0);
+		__syncthreads();
+		if (flag_count + ROWS > WIDE_LIST) { /* (the same in every lane: the barrier above) */
+			__syncthreads();
+			if (tid == 0) { flag_base = atomicAdd(&w.counters[0], flag_count); }
+			__syncthreads();
+			for (uint32_t i = tid; i < 2 * flag_count; i += WIDE_THREADS) w.queue[2 * (size_t)flag_base + i] = flags[i];
+			__syncthreads();
+			if (tid == 0) flag_count = 0u;
+			/* (the next lane to add to the list does so behind at least one more barrier) */
+		}
+
+		uint32_t step = 0, write_chunk = 1 % chunks, write_buffer = 1, read_buffer = 0;
+		for (uint32_t group = 0; group < groups; ++group) {
+			f32x16 acc[NT][PT];
+			norm_stage[wave][NT == 2 ? lane : col] = norm_reg;
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+#pragma unroll
+			for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+				for (int g = 0; g < 4; ++g) {
+					const f32x4 v = *(const f32x4*)&norm_stage[wave][nt * TILE + 8 * g + 4 * h];
+					acc[nt][0][4 * g] = v.x; acc[nt][0][4 * g + 1] = v.y; acc[nt][0][4 * g + 2] = v.z; acc[nt][0][4 * g + 3] = v.w;
+				}
+#pragma unroll
+				for (int p = 1; p < PT; ++p) acc[nt][p] = acc[nt][0];
+			}
+			request_norms(group + 1 < groups ? group + 1 : 0);
+			bool busy[NT]; /* uniform: which tiles of this wavefront exist in this group */
+#pragma unroll
+			for (int nt = 0; nt < NT; ++nt) busy[nt] = tile_of(group, nt) < tiles;
+
+			for (uint32_t chunk = 0; chunk < chunks; ++chunk, ++step) {
+				const bf16x8* rows_at = rows_lds + (size_t)read_buffer * BUFFER_UNITS + h * UNIT_STRIDE + col;
+				bf16x8 bhi[2][PT], bmid[2][X3 ? PT : 1];
+				auto fetch_points = [&](int b) {
+#pragma unroll
+					for (int p = 0; p < PT; ++p) {
+						bhi[b & 1][p] = rows_at[2 * b * UNIT_STRIDE + p * TILE];
+						if constexpr (X3) bmid[b & 1][p] = rows_at[PART_UNITS + 2 * b * UNIT_STRIDE + p * TILE];
+					}
+				};
+				fetch_points(0);
+#pragma unroll
+				for (int b = 0; b < (int)WIDE_BLOCKS; ++b) {
+					if (b + 1 < (int)WIDE_BLOCKS) fetch_points(b + 1);
+					__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+					for (int nt = 0; nt < NT; ++nt) {
+						if (!busy[nt]) continue;
+						if constexpr (X3) {
+#pragma unroll
+							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b][nt], bmid[b & 1][p], acc[nt][p], 0, 0, 0);
+#pragma unroll
+							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(amid[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
+						}
+#pragma unroll
+						for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
+					}
+					__builtin_amdgcn_sched_barrier(0);
+					fetch_ops(b);
+					__builtin_amdgcn_sched_barrier(0);
+				}
+				advance();
+				if (step + 1 < staged_steps) {
+					store_rows(write_buffer, write_chunk, step + 1 < chunks);
+					if (step + 2 < staged_steps) request_rows(pt, write_chunk + 1 == chunks ? 0 : write_chunk + 1);
+					else request_rows(next_pt, 0);
+					write_chunk = write_chunk + 1 == chunks ? 0 : write_chunk + 1;
+					write_buffer = write_buffer + 1 == w.buffers ? 0 : write_buffer + 1;
+					__syncthreads();
+				}
+				read_buffer = read_buffer + 1 == w.buffers ? 0 : read_buffer + 1;
+			}
+
+			if (busy[0]) {
+#pragma unroll
+				for (int p = 0; p < PT; ++p) {
+					__builtin_amdgcn_sched_barrier(0); /* one point tile at a time: the keyed values of all of them do not fit the registers */
+					float g1 = __builtin_inff(), g2 = __builtin_inff();
+#pragma unroll
+					for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+						for (int r = 0; r < 16; ++r) {
+							const float v = __uint_as_float((__float_as_uint(acc[nt][p][r]) & ~KEY_MASK) | (uint32_t)(nt * 16 + r));
+							g2 = __builtin_amdgcn_fmed3f(g1, g2, v);
+							g1 = __builtin_elementwise_minimum(g1, v);
+							asm volatile("" : "+v"(g1), "+v"(g2)); /* value by value: left alone the compiler takes all minima first and spills the values for the medians */
+						}
+					}
+					const uint32_t key = __float_as_uint(g1) & KEY_MASK, r = key % 16;
+					const uint32_t idx = (group * GROUP_TILES + (key / 16) * WIDE_WAVES + wave) * TILE + 8 * (r / 4) + 4 * h + r % 4;
+					const bool wins = g1 < best[p];
+					second[p] = fminf(fminf(second[p], g2), fmaxf(best[p], g1));
+					best_idx[p] = wins ? idx : best_idx[p];
+					best[p] = __builtin_elementwise_minimum(best[p], g1);
+				}
+			}
+		}
+
+		/* the two half-waves of a wavefront, then the wavefronts */
+#pragma unroll
+		for (int p = 0; p < PT; ++p) {
+			const float ob = __shfl_xor(best[p], 32), os = __shfl_xor(second[p], 32);
+			const uint32_t oi = (uint32_t)__shfl_xor((int)best_idx[p], 32);
+			if (h == 0) {
+				cand_second[wave][p * TILE + col] = fminf(fminf(second[p], os), fmaxf(best[p], ob));
+				cand_idx[wave][p * TILE + col] = ob < best[p] ? oi : best_idx[p];
+				cand_first[wave][p * TILE + col] = __builtin_elementwise_minimum(best[p], ob);
+			}
+		}
+		if (LD == KMX_AOS) {
+			for (int off = SUBS / 2; off > 0; off >>= 1) {
+				xx += __shfl_xor(xx, off);
+				xpart += __shfl_xor(xpart, off);
+				xalong += __shfl_xor(xalong, off);
+			}
+			if (sub == 0) { row_info[0][row] = xx; row_info[1][row] = xpart; row_info[2][row] = xalong; }
+		}
+		else {
+			/* the lanes of a row sit in different wavefronts: their shares meet in LDS, in a fixed order */
+			float* share = (float*)rows_lds; /* (all wavefronts are past their last read after the barrier) */
+			__syncthreads();
+			share[(0 * SUBS + sub) * ROWS + row] = xx;
+			share[(1 * SUBS + sub) * ROWS + row] = xpart;
+			share[(2 * SUBS + sub) * ROWS + row] = xalong;
+			__syncthreads();
+			if (tid < ROWS) {
+				for (int q = 0; q < 3; ++q) {
+					float s = 0.0f;
+					for (uint32_t i = 0; i < SUBS; ++i) s += share[(q * SUBS + i) * ROWS + tid];
+					row_info[q][tid] = s;
+				}
+			}
+		}
+		__syncthreads();
+		if (tid < ROWS) {
+			float first = cand_first[0][tid], next = cand_second[0][tid];
+			uint32_t idx = cand_idx[0][tid];
+#pragma unroll
+			for (uint32_t v = 1; v < WIDE_WAVES; ++v) {
+				const float cf = cand_first[v][tid];
+				next = fminf(fminf(next, cand_second[v][tid]), fmaxf(first, cf));
+				idx = cf < first ? cand_idx[v][tid] : idx;
+				first = __builtin_elementwise_minimum(first, cf);
+			}
+			const float x2 = row_info[0][tid], along = row_info[2][tid];
+			const float tau = cert_tau(w.kd, x2, row_info[1][tid], cert);
+			const uint32_t slot = unit * ROWS + tid;
+			const bool mine = slot < uniform_n;
+			const uint32_t point = LISTED ? w.list[2 * (size_t)min(slot, uniform_n - 1)] : slot;
+			const bool decided = (next - first > tau) && (x2 + cert.c2max > 1e-30f) && idx < w.k;
+			if (mine) w.assignment[point] = idx < w.k ? idx : 0u;
+			if (mine && !decided) {
+				const uint32_t at = atomicAdd(&flag_count, 1u);
+				flags[2 * at] = point;
+				flags[2 * at + 1] = w.kd_unmoved > 0.0f
+					? screening_threshold(cert_unmoved_threshold(first, tau, x2, along, cert.c2max, m2, mnorm, w.kd_unmoved), 0.0f)
+					: screening_threshold(first, tau);
+			}
+		}
+		pt = next_pt;
+	}
+	__syncthreads();
+	if (flag_count) {
+		if (tid == 0) flag_base = atomicAdd(&w.counters[0], flag_count);
+		__syncthreads();
+		for (uint32_t i = tid; i < 2 * flag_count; i += WIDE_THREADS) w.queue[2 * (size_t)flag_base + i] = flags[i];
+	}
+}
+
+constexpr uint32_t WIDE_MAX_DIM = 2560; /* what the exact pass takes */
+
+static uint32_t wide_buffer_bytes(uint32_t pt, bool x3) { return (x3 ? 2u : 1u) * 2 * WIDE_BLOCKS * (pt * TILE + WIDE_ROW_PAD) * 16; }
+static uint32_t wide_static_bytes(uint32_t pt, uint32_t nt) { return (3 * WIDE_WAVES * pt * TILE + 3 * pt * TILE + WIDE_WAVES * nt * TILE + 2 * WIDE_LIST + 3 * WIDE_WAVES + 64) * 4; }
+
+bool wide_supports(const AssignArgs& a, const DeviceInfo& dev)
+{
+	const uint32_t dp = round_up(a.dim, WIDE_CHUNK);
+	return a.dim > 256 && a.dim <= WIDE_MAX_DIM && dp * 4 + 2 * wide_buffer_bytes(4, true) + wide_static_bytes(4, 2) <= dev.lds_bytes;
+}
+
+template <int PT, int NT, bool X3, bool LISTED>
+static int launch_wide_sweep(const AssignArgs& a, WideArgs w, const DeviceInfo& dev, kmx_exec_params* exec)
+{
+	const bool vec = a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data & 15) == 0;
+	void (*kernel)(WideArgs) = a.layout == KMX_SOA ? wide_sweep_kernel<PT, NT, X3, KMX_SOA, false, LISTED>
+	                           : vec ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, true, LISTED> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, false, LISTED>;
+	const uint32_t chunks = w.dp / WIDE_CHUNK, groups = (w.kp / TILE + WIDE_WAVES * NT - 1) / (WIDE_WAVES * NT);
+	const uint32_t buffer = wide_buffer_bytes(PT, X3);
+	const uint32_t room = dev.lds_bytes - wide_static_bytes(PT, NT) - w.dp * 4;
+	/* all chunks of a unit stay in LDS where another group of centroids wants them again */
+	w.buffers = std::min(chunks, (groups > 1 && (uint64_t)chunks * buffer <= room) ? chunks : 2u);
+	const uint32_t lds_bytes = w.dp * 4 + w.buffers * buffer;
+	const uint32_t units = (a.n + PT * TILE - 1) / (PT * TILE);
+	const uint32_t grid = std::min(units, dev.compute_units);
+	if (exec) exec->block_count = grid;
+	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+	KMX_LAUNCH_KERNEL(kernel, dim3(grid), dim3(WIDE_THREADS), lds_bytes, stream(), w);
+	KMX_LAUNCH_CHECK("wide_sweep_kernel");
+	return KMX_OK;
+}
+
+/* every offset the kernels form must lie inside its allocation (see check_sweep_plan) */
+static int check_wide_plan(const AssignArgs& a, const WideArgs& w, const Workspace* ws, bool two_level)
+{
+#define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (wide rows): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u)", #cond, a.dim, a.k, w.kp, a.n); } while (0)
+	KMX_PLAN(w.dp % WIDE_CHUNK == 0 && w.dp >= a.dim && w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1);
+	KMX_PLAN(ws->packed_means && wide_plane_units(w.kp, w.dp) * 2 * 4 <= ws->packed_cap);
+	KMX_PLAN(ws->norms && wide_norms_floats(w.kp, w.dp) <= ws->norms_cap);
+	KMX_PLAN(ws->means_t && (size_t)w.kp * a.dim <= ws->means_t_cap);
+	KMX_PLAN(ws->queue && 2 * (size_t)a.n <= ws->queue_cap && ws->counters);
+	KMX_PLAN(!two_level || (ws->listed && 2 * (size_t)a.n <= ws->listed_cap));
+#undef KMX_PLAN
+	return KMX_OK;
+}
+
+/* Two levels pay from about a hundred units of 128 points and two centroid tiles on: below that the second launch costs more
+ * than the products it saves. Few points are swept in units of 32, so that they reach more compute units. */
+constexpr uint32_t WIDE_TWO_LEVEL_POINTS = 1u << 14;
+
+int launch_assign_wide(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	AssignArgs a = args;
+	const uint32_t dp = round_up(a.dim, WIDE_CHUNK), kp = round_up(a.k, TILE);
+	const bool moved = !a.ranking_only; /* (the double path hands over copies it has moved itself) */
+	const int mode = two_level_mode();
+	const bool two_level = a.two_level && mode != 0 && (mode == 2 || (a.n >= WIDE_TWO_LEVEL_POINTS && kp > 2 * TILE));
+	int rc = reserve_packed(ws, wide_plane_units(kp, dp) * 2 * 4, wide_norms_floats(kp, dp), (size_t)kp * a.dim);
+	if (rc) return rc;
+	if ((rc = reserve_queue(ws, 2 * (size_t)a.n))) return rc;
+	if (two_level && (rc = reserve_listed(ws, 2 * (size_t)a.n))) return rc;
+	auto pack = a.layout_means == KMX_AOS ? pack_means_wide_kernel<KMX_AOS> : pack_means_wide_kernel<KMX_SOA>;
+	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), dp * 4, stream(),
+	                   a.means, a.stride_means, (__bf16*)ws->packed_means, ws->norms, ws->means_t, a.dim, a.k, kp, dp, moved ? 1u : 0u, ws->counters);
+	KMX_LAUNCH_CHECK("pack_means_wide_kernel");
+
+	const float extra = (moved ? 8.0f * CERT_UNIT : 0.0f) + a.kd_extra;
+	WideArgs w = { a.data, a.stride, (const bf16x8*)ws->packed_means, ws->norms, a.assignment, ws->queue, ws->counters, nullptr, nullptr,
+	               a.dim, dp, a.k, kp, a.n, 0, 0.0f, moved ? cert_kd_unmoved(a.dim) : 0.0f };
+	if (!sizing_only() && (rc = check_wide_plan(a, w, ws, two_level))) return rc;
+	if ((rc = profile_begin(0))) return rc;
+	if (two_level) {
+		WideArgs first = w;
+		first.queue = ws->listed;
+		first.counters = ws->counters + LISTED_COUNTER;
+		first.kd = cert_kd_level1(a.dim) + cert_kd_keyed(5) + extra;
+		if ((rc = launch_wide_sweep<4, 2, false, false>(a, first, dev, exec))) return rc;
+		w.list = ws->listed;
+		w.list_length = ws->counters + LISTED_COUNTER;
+	}
+	w.kd = cert_kd_split(a.dim) + cert_kd_keyed(4) + extra;
+	const bool large = a.n >= 128 * dev.compute_units;
+	if (two_level) rc = a.n >= (1u << 18) ? launch_wide_sweep<4, 1, true, true>(a, w, dev, nullptr) : launch_wide_sweep<1, 1, true, true>(a, w, dev, nullptr);
+	else rc = large ? launch_wide_sweep<4, 1, true, false>(a, w, dev, exec) : launch_wide_sweep<1, 1, true, false>(a, w, dev, exec);
+	if (rc) return rc;
+	if ((rc = profile_end(0))) return rc;
+	if (a.ranking_only) return KMX_OK; /* the caller resolves the queued points */
+	ws->exact_norms = ws->norms + wide_exact_norms_offset(kp, dp);
+	rc = launch_recheck(a, ws, kp);
+	ws->exact_norms = nullptr;
+	return rc;
+}
+
+} // namespace kmx

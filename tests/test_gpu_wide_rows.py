@@ -1,0 +1,55 @@
+"""Rows of more than 256 dimensions (csrc/assign_wide.hip) against the serial oracle, bit for bit: both levels, both unit sizes,
+one and several groups of centroids, rows kept in LDS and rows staged again, ragged ends everywhere (-m gpu)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def flat(rows, layout):
+    return np.ascontiguousarray(rows if layout == 0 else rows.T).ravel()
+
+
+@pytest.mark.parametrize("kind", ["clustered", "grid", "offset"])
+@pytest.mark.parametrize("dim,k,n", [
+    (257, 1, 1), (300, 5, 31), (320, 33, 130), (511, 400, 700), (257, 290, 1500),   # units of 32 points, one level
+    (384, 520, 16500), (512, 545, 16384), (515, 100, 16421),                         # two levels; groups of 512; resident rows
+    (1030, 600, 16400), (2560, 40, 300),                                             # rows staged again per group; the widest
+    (300, 40, 33000),                                                                # units of 128 points, one level (two tiles)
+])
+def test_wide_rows_match_the_oracle(km, orc, gpu, dim, k, n, kind):
+    rng = np.random.default_rng(dim * 31 + k)
+    centres = rng.uniform(-3, 3, size=(k, dim)).astype(np.float32)
+    rows = (centres[rng.integers(0, k, n)] + rng.normal(size=(n, dim))).astype(np.float32)
+    means = (centres + rng.normal(size=(k, dim)) * 0.3).astype(np.float32)
+    if kind == "grid":       # many exact ties: duplicated centroids, points on bisectors
+        rows, means = np.round(rows * 0.5).astype(np.float32), np.round(means * 0.5).astype(np.float32)
+        means[k // 2:] = means[:k - k // 2]
+    elif kind == "offset":
+        rows, means = (rows + np.float32(1000)).astype(np.float32), (means + np.float32(1000)).astype(np.float32)
+    if n > 20:
+        rows[7, 3] = np.nan
+        rows[11, dim - 1] = np.inf
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    a = km.DeviceBuffer(4 * n)
+    for layout, layout_means, pad in [(0, 0, 0), (0, 1, 5), (1, 0, 0)]:
+        stride = dim + pad if layout == 0 else n
+        if pad:
+            padded = np.full((n, stride), np.float32(np.nan)); padded[:, :dim] = rows
+        else:
+            padded = rows
+        d = km.DeviceBuffer(padded.nbytes); d.write(flat(padded, layout))
+        m = km.DeviceBuffer(4 * k * dim); m.write(flat(means, layout_means))
+        for mode in (1, 2):  # two levels where they pay, two levels always
+            km.set_two_level_sweep(mode)
+            try:
+                a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+                km.assign(km.ASSIGN_BEST, d, layout, stride, m, layout_means, km.layout_stride(layout_means, k, dim), a, dim, k, n)
+                km.sync()
+            finally:
+                km.set_two_level_sweep(1)
+            got = a.read(np.uint32, n)
+            assert km.last_assign_variant() == km.ASSIGN_MFMA_BF16X3
+            assert np.array_equal(got, want), "layouts %d/%d, mode %d: %d mismatches" % (layout, layout_means, mode, int((got != want).sum()))
+        d.free(); m.free()
+    a.free()
