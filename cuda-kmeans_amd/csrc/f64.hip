@@ -1291,6 +1291,14 @@ extern "C" int kmx_assign_f64(int variant,
 	const DeviceInfo* dev = nullptr;
 	rc = device_info(&dev);
 	if (rc) return rc;
+	if (variant == KMX_ASSIGN_BEST && small_assign_fits<double>(dim, k, n, lds_budget_of(exec, *dev))) {
+		/* small inputs: the serial arithmetic for every pair in one launch (small.hip) */
+		Workspace* ws = nullptr;
+		if ((rc = workspace(&ws))) return rc;
+		if ((rc = profile_begin(0))) return rc;
+		rc = launch_assign_small<double>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, ws->counters, &exec->block_count, *dev);
+		return rc ? rc : profile_end(0);
+	}
 	const bool float_ranking = variant == KMX_ASSIGN_MFMA || variant == KMX_ASSIGN_MFMA_BF16X3 || variant == KMX_ASSIGN_BEST;
 
 	const uint32_t kp = round_up_u32(k, WIDE_GROUP);
@@ -1398,6 +1406,10 @@ static int update_f64_call(const char* who, bool divide, int variant,
 
 	rc = profile_begin(1);
 	if (rc) return rc;
+	if (variant == KMX_UPDATE_ATOMIC_SHM && small_update_fits<double>(dim, k, n, lds_budget_of(exec, *dev), *dev)) {
+		rc = launch_update_small<double>(data, layout, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n, divide, &exec->block_count, *dev);
+		return rc ? rc : profile_end(1);
+	}
 #define KMX_F64_UPDATE(LD, LM) \
 	launch_update_f64_t<LD, LM>(variant, data, stride, assignment, means, stride_means, cluster_sizes, dim, k, n, exec, *dev, divide)
 	if (layout == KMX_AOS) rc = layout_means == KMX_AOS ? KMX_F64_UPDATE(KMX_AOS, KMX_AOS) : KMX_F64_UPDATE(KMX_AOS, KMX_SOA);

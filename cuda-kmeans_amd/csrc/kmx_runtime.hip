@@ -182,6 +182,16 @@ namespace kmx {
 
 int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, int* chosen)
 {
+	if (variant == KMX_ASSIGN_BEST && !a.ranking_only && small_assign_fits<float>(a.dim, a.k, a.n, lds_budget_of(exec, dev))) {
+		/* small inputs: the serial arithmetic for every pair in one launch (small.hip) */
+		g_last_assign_variant = KMX_ASSIGN_BASE;
+		if (chosen) *chosen = KMX_ASSIGN_BASE;
+		int rc = profile_begin(0);
+		if (rc) return rc;
+		rc = launch_assign_small<float>(a.data, a.layout, a.stride, a.means, a.layout_means, a.stride_means, a.assignment, a.dim, a.k, a.n,
+		                                ws->counters, &exec->block_count, dev);
+		return rc ? rc : profile_end(0);
+	}
 	if (variant == KMX_ASSIGN_BEST) {
 		/* counterpart of BestCachedAssignmentKernel::run (reference kernels.cu:706-717): pick by shape.
 		 * Measured (one call, exact pass included, N = 2-4M): the split-bf16 sweep is about twice as fast as the fp32 one
@@ -229,6 +239,20 @@ int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Wor
 	default:
 		return fail(KMX_ERR_INVALID_ARGUMENT, "kmx_assign_f32: unknown variant %d", variant);
 	}
+}
+
+/* the single-pass iteration of small inputs: every work-group assigns its points and adds them up, one launch folds and divides */
+static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	const size_t elements = (size_t)a.k * a.dim, most = assign_small_max_blocks(a.n);
+	int rc = reserve_partials(ws, most * (elements + a.k));
+	if (rc) return rc;
+	g_last_assign_variant = KMX_ASSIGN_BASE;
+	uint32_t* partial_counts = (uint32_t*)(ws->partials + most * elements);
+	if ((rc = profile_begin(0))) return rc;
+	if ((rc = launch_assign_small_sums(a, ws->partials, partial_counts, &exec->block_count, ws->counters, dev))) return rc;
+	if ((rc = profile_end(0))) return rc;
+	return launch_reduce_partials(u, ws->partials, partial_counts, exec->block_count);
 }
 
 } // namespace kmx
@@ -625,6 +649,8 @@ int kmx_fused_f32(int variant,
 		rc = device_info(&dev);
 		if (rc) return rc;
 		AssignArgs a{ data, layout, stride, means_in, layout_means, stride_means, ws->fused_assignment, dim, k, n };
+		UpdateArgs small{ data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
+		if (small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) return launch_iteration_small(a, small, exec, ws, *dev);
 		rc = launch_fused_small(a, means_out, cluster_sizes, exec, ws, *dev);
 		if (rc) return rc;
 		UpdateArgs u{ data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
@@ -663,6 +689,11 @@ int kmx_iteration_f32(const float* data, int layout, size_t stride,
 		rc = workspace(&ws);
 		if (rc) return rc;
 		UpdateArgs u{ data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
+		if (small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) {
+			AssignArgs small{ data, layout, stride, means_in, layout_means, stride_means, assignment, dim, k, n };
+			g_last_iteration_passes = 1;
+			return launch_iteration_small(small, u, exec, ws, *dev);
+		}
 		rc = clear_update_outputs(u); /* the single-pass kernel accumulates into them */
 		if (rc) return rc;
 		AssignArgs a{ data, layout, stride, means_in, layout_means, stride_means, assignment, dim, k, n };
@@ -673,7 +704,19 @@ int kmx_iteration_f32(const float* data, int layout, size_t stride,
 		g_last_iteration_passes = 1;
 		return launch_divide_means(u);
 	}
-	int rc = kmx_assign_f32(KMX_ASSIGN_BEST, data, layout, stride, means_in, layout_means, stride_means, nullptr, assignment, dim, k, n, exec);
+	const DeviceInfo* dev = nullptr;
+	int rc = device_info(&dev);
+	if (rc) return rc;
+	if (n > 0 && small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) {
+		if ((rc = check_layout("kmx_iteration_f32", "data", layout, stride, n, dim))) return rc;
+		if ((rc = check_layout("kmx_iteration_f32", "means", layout_means, stride_means, k, dim))) return rc;
+		Workspace* ws = nullptr;
+		if ((rc = workspace(&ws))) return rc;
+		const AssignArgs small{ data, layout, stride, means_in, layout_means, stride_means, assignment, dim, k, n };
+		const UpdateArgs u{ data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
+		return launch_iteration_small(small, u, exec, ws, *dev);
+	}
+	rc = kmx_assign_f32(KMX_ASSIGN_BEST, data, layout, stride, means_in, layout_means, stride_means, nullptr, assignment, dim, k, n, exec);
 	if (rc) return rc;
 	return kmx_update_f32(KMX_UPDATE_ATOMIC_SHM, data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n, exec);
 }

@@ -1,0 +1,544 @@
+/*
+ * Small inputs, floats and doubles: what a call costs there is launches and latency, not arithmetic. The general paths take five
+ * to seven dependent launches (pack, sweep, exact pass, clear, accumulate, fold or divide), each of them a few microseconds of
+ * its own; N = 10240, d = 20, k = 128 was 34 us per iteration for 26 M multiply-adds. Two kernels instead:
+ *
+ *   assign_small_kernel  the serial arithmetic for every pair, nothing to pack, certify or re-evaluate. With `sums` it also adds
+ *                        up its points (rows are still in LDS) into per-work-group partial sums for reduce_partials_kernel:
+ *                        the single-pass iteration of small inputs.
+ *   update_small_kernel  a work-group per range of clusters reads ALL memberships, lists its members, adds their rows and writes
+ *                        finished centroids and sizes: no partial sums, nothing cleared before, nothing divided after.
+ *
+ * Where the general paths take over is measured; see small_assign_fits and small_update_fits.
+ */
+#include "kmx_internal.h"
+
+#include <algorithm>
+#include <type_traits>
+
+#pragma clang fp contract(off)
+
+namespace kmx {
+
+constexpr uint32_t SMALL_THREADS = 512;
+constexpr uint32_t SMALL_WAVES = SMALL_THREADS / WAVE;
+
+template <typename F> struct SmallVec;
+template <> struct SmallVec<float> { typedef float type __attribute__((ext_vector_type(4))); };
+template <> struct SmallVec<double> { typedef double type __attribute__((ext_vector_type(4))); };
+
+template <typename F> __device__ __forceinline__ F small_sqrt(F v);
+template <> __device__ __forceinline__ float small_sqrt<float>(float v) { return __builtin_sqrtf(v); }
+template <> __device__ __forceinline__ double small_sqrt<double>(double v) { return __builtin_sqrt(v); }
+
+/* The serial scan compares correctly rounded square roots. Two sums whose ratio is below this differ in their roots by more
+ * than one unit in the last place, so comparing the sums decides; between this and 1 the roots themselves are compared. (Below
+ * `tiny` the sums may be subnormal and their ratio means nothing.) */
+template <typename F> struct SqrtMargin;
+template <> struct SqrtMargin<float> { static constexpr float ratio = 0.9999995f, tiny = 1e-30f; };
+template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e-15, tiny = 1e-290; };
+
+/*
+ * A work-group owns 64 points, whose rows it stages in LDS next to a chunk of the centroids. A wavefront is 16 x 4 lanes with
+ * T points times T centroids each, so it covers 16 T points and 4 T centroids at a time; the eight wavefronts are 4 / T groups of
+ * points times 2 T shares of the centroids. Per four dimensions a lane reads 2 T pieces of 16 bytes for its T^2 pairs: with T = 2
+ * (192 ALU cycles against 128 of the LDS that four SIMDs share) the vector ALU sets the pace, T = 1 (48 against 64) is for a
+ * dozen centroids at most, which would leave most of the larger tile empty. (A lane per point with the centroids broadcast is
+ * bound by the LDS; with the centroids as scalar operands every scalar load waits for all earlier ones: N = 2588, d = 60, k = 1288
+ * 135 us.) The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
+ * ascending dimension, every operation rounded separately. Global loads are issued in batches of eight per lane: one after the
+ * other they cost a microsecond each.
+ *
+ * SUMS: membership (clusters x 64 points) times rows (64 points x coordinates) on v_mfma_f32_16x16x4_f32: 1.0 times a coordinate is
+ * exact, the accumulators add in fp32. A wavefront keeps the memberships of 16 clusters in registers and goes over the coordinates 16
+ * at a time. 0.0 times an infinity or a NaN would reach every cluster: a work-group that sees one adds its points up again, an
+ * element of the sums per lane.
+ */
+constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading the memberships again (update_small_kernel) is cheaper than as many partial sums */
+constexpr uint32_t SMALL_POINTS = WAVE;
+constexpr int SMALL_BATCH = 8;
+
+/* count rows of dim elements into LDS rows of row_stride: AoS rows `stride` apart, or columns (row r of column q at src[q * stride + r]).
+ * magic = ceil(2^32 / dim): i / dim = umulhi(i, magic) for the few ten thousand elements of a work-group. */
+template <typename F, int L>
+__device__ __forceinline__ void stage_rows(F* __restrict__ to, const F* __restrict__ src, size_t stride, uint32_t count, uint32_t last, uint32_t dim,
+                                           uint32_t row_stride, uint32_t magic, uint32_t vec4)
+{
+	typedef typename SmallVec<F>::type F4;
+	if (L == KMX_AOS && vec4) { /* rows of whole, aligned pieces of four */
+		const uint32_t pieces = dim / 4, total = count * pieces;
+		for (uint32_t i0 = threadIdx.x; i0 < total; i0 += SMALL_THREADS * SMALL_BATCH) {
+			F4 v[SMALL_BATCH];
+			uint32_t at[SMALL_BATCH];
+#pragma unroll
+			for (int u = 0; u < SMALL_BATCH; ++u) {
+				const uint32_t i = min(i0 + u * SMALL_THREADS, total - 1);
+				const uint32_t r = __umulhi(i * 4, magic), q = i * 4 - r * dim;
+				at[u] = r * row_stride + q;
+				v[u] = *(const F4*)(src + (size_t)min(r, last) * stride + q);
+			}
+#pragma unroll
+			for (int u = 0; u < SMALL_BATCH; ++u) *(F4*)(to + at[u]) = v[u];
+		}
+	}
+	else if (L == KMX_AOS) {
+		const uint32_t total = count * dim;
+		for (uint32_t i0 = threadIdx.x; i0 < total; i0 += SMALL_THREADS * SMALL_BATCH) {
+			F v[SMALL_BATCH];
+			uint32_t at[SMALL_BATCH];
+#pragma unroll
+			for (int u = 0; u < SMALL_BATCH; ++u) {
+				const uint32_t i = min(i0 + u * SMALL_THREADS, total - 1);
+				const uint32_t r = dim == 1 ? i : __umulhi(i, magic), q = i - r * dim;
+				at[u] = r * row_stride + q;
+				v[u] = src[(size_t)min(r, last) * stride + q];
+			}
+#pragma unroll
+			for (int u = 0; u < SMALL_BATCH; ++u) to[at[u]] = v[u];
+		}
+	}
+	else {
+		/* a wavefront takes 64 rows of one column at a time */
+		const uint32_t lane = threadIdx.x & (WAVE - 1);
+		for (uint32_t r0 = 0; r0 < count; r0 += WAVE) {
+			const uint32_t r = min(r0 + lane, count - 1);
+			for (uint32_t q0 = threadIdx.x / WAVE; q0 < dim; q0 += SMALL_WAVES * SMALL_BATCH) {
+				F v[SMALL_BATCH];
+#pragma unroll
+				for (int u = 0; u < SMALL_BATCH; ++u) v[u] = src[(size_t)min(q0 + u * SMALL_WAVES, dim - 1) * stride + min(r, last)];
+#pragma unroll
+				for (int u = 0; u < SMALL_BATCH; ++u) to[r * row_stride + min(q0 + u * SMALL_WAVES, dim - 1)] = v[u];
+			}
+		}
+	}
+}
+
+template <typename F, int T, int LD, int LM, bool SUMS>
+__global__ void __launch_bounds__(SMALL_THREADS)
+assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restrict__ means, size_t stride_means,
+                    uint32_t* __restrict__ assignment, uint32_t dim, uint32_t k, uint32_t n, uint32_t row_stride, uint32_t chunk,
+                    uint32_t magic, uint32_t vec4, uint32_t* __restrict__ counters, F* __restrict__ partial, uint32_t* __restrict__ partial_counts)
+{
+	typedef typename SmallVec<F>::type F4;
+	constexpr uint32_t POINTS = SMALL_POINTS;
+	constexpr uint32_t PG = 4 / T, CW = SMALL_WAVES / PG; /* groups of points, shares of the centroids */
+	extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+	F* rows = (F*)lds_raw;
+	F* cents = rows + (size_t)POINTS * row_stride; /* chunk rows; with SUMS later k * dim sums and k counts */
+	__shared__ F cand_dist[CW][POINTS];
+	__shared__ uint32_t cand_idx[CW][POINTS];
+	__shared__ __attribute__((aligned(16))) uint32_t member[POINTS];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
+	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	const uint32_t pg = wave % PG, cw = wave / PG;
+	const uint32_t lp = lane & 15, lc = lane >> 4; /* points lp + 16 p of the group, centroids T lc + u of the wavefront's 4 T */
+	const uint32_t first = blockIdx.x * POINTS;
+	const uint32_t here = min(POINTS, n - first);
+	if (blockIdx.x == 0 && tid == 0) counters[0] = 0u; /* nothing is left to an exact pass */
+
+	stage_rows<F, LD>(rows, LD == KMX_AOS ? data + (size_t)first * stride : data + first, stride, POINTS, here - 1, dim, row_stride, magic, vec4 & 1u);
+
+	F low[T];
+	uint32_t at[T];
+#pragma unroll
+	for (int p = 0; p < T; ++p) { low[p] = (F)__builtin_inff(); at[p] = 0xFFFFFFFFu; }
+	const F* mine = rows + (pg * (16 * T) + lp) * row_stride;
+	for (uint32_t base = 0; base < k; base += chunk) {
+		const uint32_t count = min(chunk, k - base);
+		if (base) __syncthreads(); /* the previous chunk is no longer needed */
+		stage_rows<F, LM>(cents, LM == KMX_AOS ? means + (size_t)base * stride_means : means + base, stride_means, count, count - 1, dim, row_stride, magic, vec4 & 2u);
+		__syncthreads();
+		for (uint32_t c0 = cw * (4 * T); c0 < count; c0 += CW * (4 * T)) {
+			F sum[T][T];
+			uint32_t centre[T];
+#pragma unroll
+			for (int u = 0; u < T; ++u) {
+				centre[u] = min(c0 + T * lc + u, count - 1) * row_stride; /* beyond the last centroid: the last one again */
+#pragma unroll
+				for (int p = 0; p < T; ++p) sum[u][p] = (F)0;
+			}
+			auto add = [&](uint32_t q, auto width) {
+				constexpr int W = decltype(width)::value;
+				F x[T][W], cv[T][W];
+				auto fetch = [&](F (&to)[W], const F* from) {
+					if constexpr (W == 4) {
+						const F4 v = *(const F4*)from;
+						to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+					}
+					else to[0] = from[0];
+				};
+#pragma unroll
+				for (int p = 0; p < T; ++p) fetch(x[p], mine + p * (16 * row_stride) + q);
+#pragma unroll
+				for (int u = 0; u < T; ++u) fetch(cv[u], cents + centre[u] + q);
+#pragma unroll
+				for (int e = 0; e < W; ++e)
+#pragma unroll
+					for (int u = 0; u < T; ++u)
+#pragma unroll
+						for (int p = 0; p < T; ++p) {
+							const F diff = x[p][e] - cv[u][e];
+							const F sq = diff * diff;
+							sum[u][p] = sum[u][p] + sq;
+						}
+			};
+			uint32_t q = 0;
+#pragma unroll 4
+			for (; q + 4 <= dim; q += 4) add(q, std::integral_constant<int, 4>());
+			for (; q < dim; ++q) add(q, std::integral_constant<int, 1>());
+#pragma unroll
+			for (int u = 0; u < T; ++u) {
+				const uint32_t c = base + min(c0 + T * lc + u, count - 1);
+#pragma unroll
+				for (int p = 0; p < T; ++p) {
+					const F s = sum[u][p];
+					const bool start = c == 0; /* where the serial scan starts: a NaN stays */
+					bool less = s < low[p];
+					const bool close = less && !(s < low[p] * SqrtMargin<F>::ratio && low[p] > SqrtMargin<F>::tiny);
+					if (__builtin_amdgcn_ballot_w64(close)) less = close ? small_sqrt(s) < small_sqrt(low[p]) : less;
+					less = less || start;
+					low[p] = less ? s : low[p];
+					at[p] = less ? c : at[p];
+				}
+			}
+		}
+	}
+	/* the four lanes of a point, then the wavefronts: the smaller root, then the smaller number. The share that holds centroid 0
+	 * keeps a NaN root of it against everything. */
+#pragma unroll
+	for (int p = 0; p < T; ++p) {
+		F d = small_sqrt(low[p]);
+		uint32_t i = at[p];
+#pragma unroll
+		for (int off = 16; off < WAVE; off <<= 1) {
+			const F od = __shfl_xor(d, off);
+			const uint32_t oi = (uint32_t)__shfl_xor((int)i, off);
+			const bool pinned = i == 0 && d != d, other_pinned = oi == 0 && od != od;
+			const bool wins = other_pinned || (!pinned && oi != 0xFFFFFFFFu && (i == 0xFFFFFFFFu || od < d || (od == d && oi < i)));
+			d = wins ? od : d;
+			i = wins ? oi : i;
+		}
+		if (lc == 0) { cand_dist[cw][pg * (16 * T) + lp + 16 * p] = d; cand_idx[cw][pg * (16 * T) + lp + 16 * p] = i; }
+	}
+	__syncthreads();
+	if (tid < POINTS) {
+		F best = cand_dist[0][tid];
+		uint32_t idx = cand_idx[0][tid];
+#pragma unroll
+		for (uint32_t w = 1; w < CW; ++w) {
+			const F d = cand_dist[w][tid];
+			const uint32_t i = cand_idx[w][tid];
+			const bool wins = i != 0xFFFFFFFFu && (d < best || (d == best && i < idx));
+			best = wins ? d : best;
+			idx = wins ? i : idx;
+		}
+		if (tid < here) assignment[first + tid] = idx;
+		if (SUMS) member[tid] = tid < here ? idx : 0xFFFFFFFFu;
+	}
+
+	if constexpr (SUMS) {
+		typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+		uint32_t* counts = (uint32_t*)cents; /* k words; the centroids are no longer needed */
+		__shared__ uint32_t not_finite;
+		if (tid == 0) not_finite = 0u;
+		for (uint32_t i = tid; i < k; i += SMALL_THREADS) counts[i] = 0u;
+		__syncthreads();
+		if (tid < here) atomicAdd(&counts[member[tid]], 1u);
+		F* out = partial + (size_t)blockIdx.x * k * dim;
+		const uint32_t l16 = lane & 15, quad = lane >> 4;
+		bool bad = false;
+		for (uint32_t cluster = wave * 16; cluster < k; cluster += SMALL_WAVES * 16) {
+			float in[POINTS / 4]; /* point 4 i + quad belongs to cluster + l16 */
+#pragma unroll
+			for (uint32_t i = 0; i < POINTS / 4; ++i) in[i] = member[4 * i + quad] == cluster + l16 ? 1.0f : 0.0f;
+			for (uint32_t d0 = 0; d0 < dim; d0 += 16) {
+				const F* at_row = rows + quad * row_stride + min(d0 + l16, dim - 1);
+				f32x4 sum = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+				for (uint32_t i = 0; i < POINTS / 4; ++i) {
+					const float x = at_row[4 * i * row_stride];
+					bad = bad || !(__builtin_fabsf(x) < __builtin_inff());
+					sum = __builtin_amdgcn_mfma_f32_16x16x4f32(in[i], x, sum, 0, 0, 0);
+				}
+#pragma unroll
+				for (uint32_t r = 0; r < 4; ++r)
+					if (cluster + 4 * quad + r < k && d0 + l16 < dim) out[(size_t)(cluster + 4 * quad + r) * dim + d0 + l16] = sum[r];
+			}
+		}
+		if (bad) not_finite = 1u;
+		__syncthreads();
+		for (uint32_t i = tid; i < k; i += SMALL_THREADS) partial_counts[(size_t)blockIdx.x * k + i] = counts[i];
+		if (not_finite) { /* (the stores above have left before the barrier) */
+			for (uint32_t e = tid; e < k * dim; e += SMALL_THREADS) {
+				const uint32_t cl = e / dim, d = e - cl * dim;
+				F s = (F)0;
+				for (uint32_t p = 0; p < POINTS; p += 4) {
+					const u4 m = *(const u4*)(member + p);
+#pragma unroll
+					for (uint32_t i = 0; i < 4; ++i)
+						if (m[i] == cl) s += rows[(p + i) * row_stride + d];
+				}
+				out[e] = s;
+			}
+		}
+	}
+}
+
+/*
+ * blockIdx.x owns the clusters [per * blockIdx.x, + per). Its 1024 lanes read all n memberships (ITEMS 16-byte pieces each, one
+ * round trip to the caches); every wavefront lists the points of its share that belong to these clusters in a region of LDS of
+ * its own (ballots, no atomics), the lists are joined, sorted by cluster where there are several, and the listed rows are added:
+ * groups of gw lanes (a lane: VEC consecutive coordinates) take equal shares of the list, 8 rows in flight, and add what they
+ * have of a cluster to its sums in LDS when the cluster changes. Rows wider than a group go by in slices.
+ * One hot cluster holding everything is bound by what one compute unit reads (about 0.1 TB/s), which small_update_fits bounds.
+ */
+constexpr uint32_t UPDATE_SMALL_THREADS = 1024;
+constexpr uint32_t UPDATE_SMALL_WAVES = UPDATE_SMALL_THREADS / WAVE;
+constexpr uint32_t UPDATE_SMALL_MAX_PER = 64;
+
+template <typename F, int ITEMS, int VEC, int LD, int LM>
+__global__ void __launch_bounds__(UPDATE_SMALL_THREADS)
+update_small_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment, F* __restrict__ means, size_t stride_means,
+                    uint32_t* __restrict__ sizes, uint32_t dim, uint32_t k, uint32_t n, uint32_t per, uint32_t gw, uint32_t divide, uint32_t vec4)
+{
+	typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+	extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+	F* acc = (F*)lds_raw;                                                     /* per x dim sums */
+	constexpr uint32_t REGION = WAVE * 4 * ITEMS;                             /* points a wavefront looks at */
+	unsigned short* found = (unsigned short*)(acc + (size_t)per * dim);       /* UPDATE_SMALL_WAVES regions */
+	unsigned short* list = found + UPDATE_SMALL_WAVES * REGION;               /* all of them, sorted by cluster */
+	__shared__ uint32_t count[UPDATE_SMALL_MAX_PER], cursor[UPDATE_SMALL_MAX_PER], begin[UPDATE_SMALL_MAX_PER + 1];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+	const uint32_t c0 = blockIdx.x * per, mine = min(per, k - c0);
+
+	u4 a[ITEMS];
+#pragma unroll
+	for (int i = 0; i < ITEMS; ++i) {
+		const uint32_t p = (i * UPDATE_SMALL_THREADS + tid) * 4;
+		a[i] = u4{ 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu };
+		if (vec4 && p + 4 <= n) a[i] = *(const u4*)(assignment + p);
+		else {
+#pragma unroll
+			for (int e = 0; e < 4; ++e)
+				if (p + e < n) a[i][e] = assignment[p + e];
+		}
+	}
+	if (tid < per) count[tid] = 0u;
+	for (uint32_t i = tid; i < per * dim; i += UPDATE_SMALL_THREADS) acc[i] = (F)0;
+	uint32_t have = 0; /* wave-uniform */
+	unsigned short* region = found + wave * REGION;
+#pragma unroll
+	for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+		for (int e = 0; e < 4; ++e) {
+			const bool match = a[i][e] - c0 < mine; /* (a membership beyond k belongs to nobody) */
+			const unsigned long long mask = __builtin_amdgcn_ballot_w64(match);
+			if (mask == 0) continue;
+			if (match) region[have + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] = (unsigned short)((i * UPDATE_SMALL_THREADS + tid) * 4 + e);
+			have += (uint32_t)__popcll(mask);
+		}
+	__syncthreads();
+	for (uint32_t i = lane; i < have; i += WAVE) atomicAdd(&count[mine > 1 ? assignment[region[i]] - c0 : 0u], 1u);
+	__syncthreads();
+	if (tid < WAVE) {
+		const uint32_t v = tid < mine ? count[tid] : 0u;
+		uint32_t incl = v;
+		for (int off = 1; off < WAVE; off <<= 1) {
+			const uint32_t up = (uint32_t)__shfl_up((int)incl, off);
+			if (tid >= (uint32_t)off) incl += up;
+		}
+		if (tid < mine) { begin[tid] = incl - v; cursor[tid] = incl - v; }
+		if (tid == mine - 1) begin[mine] = incl;
+	}
+	__syncthreads();
+	for (uint32_t i = lane; i < have; i += WAVE) list[atomicAdd(&cursor[mine > 1 ? assignment[region[i]] - c0 : 0u], 1u)] = region[i];
+	__syncthreads();
+
+	const uint32_t groups = UPDATE_SMALL_THREADS / gw, group = tid / gw, gl = tid % gw;
+	const uint32_t entries = begin[mine];
+	const uint32_t e_begin = (uint32_t)((uint64_t)group * entries / groups), e_end = (uint32_t)((uint64_t)(group + 1) * entries / groups);
+	for (uint32_t slice = 0; slice < dim; slice += gw * VEC) {
+		const uint32_t d0 = slice + gl * VEC;
+		const bool on = d0 < dim;
+		/* (the last piece of a row that is no multiple of VEC starts early enough to end with the row; its first coordinates are the previous lane's) */
+		const uint32_t d = on ? (VEC > 1 ? min(d0, dim - VEC) : d0) : 0u;
+		if (!on || e_begin == e_end) continue;
+		F s[VEC];
+#pragma unroll
+		for (int v = 0; v < VEC; ++v) s[v] = (F)0;
+		uint32_t cl = 0;
+		while (begin[cl + 1] <= e_begin) ++cl;
+		auto flush = [&]() {
+#pragma unroll
+			for (int v = 0; v < VEC; ++v) {
+				if (VEC == 1 || d + v >= d0) unsafeAtomicAdd(&acc[cl * dim + d + v], s[v]);
+				s[v] = (F)0;
+			}
+		};
+		constexpr int AHEAD = 8;
+		for (uint32_t e = e_begin; e < e_end; e += AHEAD) {
+			F x[AHEAD][VEC];
+#pragma unroll
+			for (int u = 0; u < AHEAD; ++u) {
+				const uint32_t p = list[min(e + u, e_end - 1)];
+#pragma unroll
+				for (int v = 0; v < VEC; ++v) x[u][v] = data[elem<LD>(stride, p, d + v)];
+			}
+#pragma unroll
+			for (int u = 0; u < AHEAD; ++u) {
+				if (e + u < e_end) {
+					while (begin[cl + 1] <= e + u) { flush(); ++cl; }
+#pragma unroll
+					for (int v = 0; v < VEC; ++v) s[v] += x[u][v];
+				}
+			}
+		}
+		flush();
+	}
+	__syncthreads();
+	for (uint32_t i = tid; i < mine * dim; i += UPDATE_SMALL_THREADS) {
+		const uint32_t cl = i / dim, d = i - cl * dim;
+		const uint32_t members = count[cl];
+		const F s = acc[i];
+		means[elem<LM>(stride_means, c0 + cl, d)] = !divide ? s : (members ? s / (F)members : (F)0);
+	}
+	if (tid < mine) sizes[c0 + tid] = count[tid];
+}
+
+static uint32_t small_row_stride(uint32_t dim) { return (((dim + 3) / 4) | 1u) * 4; }
+template <typename F> static uint32_t assign_small_static()
+{
+	return SMALL_WAVES * SMALL_POINTS * ((uint32_t)sizeof(F) + 4) + SMALL_POINTS * 4 + 64;
+}
+/* LDS next to the static arrays: the rows of the points and as many centroids as 32 KB hold (at least 32: one step of all wavefronts) */
+template <typename F> static uint32_t assign_small_chunk(uint32_t dim, uint32_t k)
+{
+	const uint32_t fit = 32 * 1024 / (small_row_stride(dim) * (uint32_t)sizeof(F)) / 32 * 32;
+	return std::min(k, std::max(32u, fit));
+}
+template <typename F> static uint32_t assign_small_lds(uint32_t dim, uint32_t k)
+{
+	return (SMALL_POINTS + assign_small_chunk<F>(dim, k)) * small_row_stride(dim) * (uint32_t)sizeof(F);
+}
+
+constexpr uint32_t SMALL_FEW_CENTROIDS = 12; /* up to here a tile of one point times one centroid per lane */
+
+/*
+ * Every pair costs 3 dim operations and about 30 to compare and keep, four cycles each on a SIMD; a work-group of 64 points keeps one
+ * compute unit, so fewer than 256 of them leave units idle. Fitted: 12 us + effort / 2.6e7 per us. The general path takes 30 to
+ * 35 us for rows of up to 32 dimensions, 50 to 75 us for wider ones (N = 30000, d = 32: k = 40 18.5 against 42.8 us, k = 150 31.9
+ * against 35.5, k = 600 76 against 46; d = 100: k = 40 30.6 against 55.6, k = 150 54.8 against 65.3), twice that for doubles.
+ * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
+ */
+constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
+#ifndef KMX_SMALL_EFFORT
+#define KMX_SMALL_EFFORT 450000000ull
+#endif
+template <typename F>
+bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
+{
+	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
+	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
+	const uint64_t limit = KMX_SMALL_EFFORT * (dim > 32 ? 3 : 2) / 2 * (sizeof(F) / 4);
+	return effort <= limit && assign_small_lds<F>(dim, k) + assign_small_static<F>() <= lds_budget;
+}
+
+template <typename F, bool SUMS>
+static int launch_assign_small_t(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
+                                 uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, F* partial, uint32_t* partial_counts, uint32_t* blocks, const DeviceInfo& dev)
+{
+	const uint32_t lds = assign_small_lds<F>(dim, k);
+	*blocks = (n + SMALL_POINTS - 1) / SMALL_POINTS;
+	const uint32_t align = 4 * sizeof(F) - 1;
+	const uint32_t vec4 = (dim % 4 == 0 && stride % 4 == 0 && ((uintptr_t)data & align) == 0 ? 1u : 0u) | (dim % 4 == 0 && stride_means % 4 == 0 && ((uintptr_t)means & align) == 0 ? 2u : 0u);
+	void (*kernel)(const F*, size_t, const F*, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t*, F*, uint32_t*) = nullptr;
+#define KMX_PICK(P) (layout == KMX_AOS ? (layout_means == KMX_AOS ? assign_small_kernel<F, P, KMX_AOS, KMX_AOS, SUMS> : assign_small_kernel<F, P, KMX_AOS, KMX_SOA, SUMS>) \
+                                       : (layout_means == KMX_AOS ? assign_small_kernel<F, P, KMX_SOA, KMX_AOS, SUMS> : assign_small_kernel<F, P, KMX_SOA, KMX_SOA, SUMS>))
+	kernel = k > SMALL_FEW_CENTROIDS ? KMX_PICK(2) : KMX_PICK(1);
+#undef KMX_PICK
+	if (lds > 48 * 1024) KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(SMALL_THREADS), lds, stream(), data, stride, means, stride_means, assignment, dim, k, n,
+	                   small_row_stride(dim), assign_small_chunk<F>(dim, k), (uint32_t)((0x100000000ull + dim - 1) / dim), vec4, counters, partial, partial_counts);
+	KMX_LAUNCH_CHECK("assign_small_kernel");
+	return KMX_OK;
+}
+
+template <typename F>
+int launch_assign_small(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
+                        uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, uint32_t* blocks, const DeviceInfo& dev)
+{
+	return launch_assign_small_t<F, false>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, counters, nullptr, nullptr, blocks, dev);
+}
+
+/* the single-pass iteration of small inputs: partial sums and counts of *blocks work-groups, for launch_reduce_partials */
+int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, const DeviceInfo& dev)
+{
+	return launch_assign_small_t<float, true>(a.data, a.layout, a.stride, a.means, a.layout_means, a.stride_means, a.assignment, a.dim, a.k, a.n,
+	                                          counters, partial, partial_counts, blocks, dev);
+}
+uint32_t assign_small_max_blocks(uint32_t n) { return (n + SMALL_POINTS - 1) / SMALL_POINTS; }
+/* (the partial sums of all work-groups are written and read once) */
+bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
+{
+	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * assign_small_max_blocks(n) <= (2u << 20) && small_assign_fits<float>(dim, k, n, lds_budget);
+}
+
+/*
+ * The members of a cluster come from one compute unit, so the largest cluster sets the time: everything in one cluster is
+ * n * dim * sizeof(F) bytes at about 0.1 TB/s. 2 MB keeps that worst case near 20 us, what the general path takes anyway.
+ */
+constexpr uint32_t SMALL_UPDATE_POINTS = 1u << 15;
+constexpr uint64_t SMALL_UPDATE_BYTES = 2u << 20;
+
+static uint32_t update_small_per(uint32_t k, const DeviceInfo& dev) { return (k + dev.compute_units - 1) / dev.compute_units; }
+static uint32_t update_small_items(uint32_t n)
+{
+	const uint32_t items = (n + 4 * UPDATE_SMALL_THREADS - 1) / (4 * UPDATE_SMALL_THREADS);
+	return items <= 1 ? 1 : items <= 3 ? 3 : 8;
+}
+template <typename F> static uint64_t update_small_lds(uint32_t dim, uint32_t k, uint32_t n, const DeviceInfo& dev)
+{
+	return (uint64_t)update_small_per(k, dev) * dim * sizeof(F) + (uint64_t)update_small_items(n) * UPDATE_SMALL_THREADS * 4 * 2 * 2;
+}
+
+template <typename F>
+bool small_update_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget, const DeviceInfo& dev)
+{
+	return n > 0 && n <= SMALL_UPDATE_POINTS && (uint64_t)n * dim * sizeof(F) <= SMALL_UPDATE_BYTES && update_small_per(k, dev) <= UPDATE_SMALL_MAX_PER &&
+	       update_small_lds<F>(dim, k, n, dev) + 1024 <= lds_budget;
+}
+
+template <typename F>
+int launch_update_small(const F* data, int layout, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
+                        uint32_t dim, uint32_t k, uint32_t n, bool divide, uint32_t* blocks, const DeviceInfo& dev)
+{
+	const uint32_t per = update_small_per(k, dev);
+	*blocks = (k + per - 1) / per;
+	const uint32_t lds = (uint32_t)update_small_lds<F>(dim, k, n, dev);
+	constexpr int VEC = sizeof(F) == 4 ? 4 : 2;
+	const bool vec = layout == KMX_AOS && dim >= (uint32_t)VEC;
+	uint32_t gw = 1;
+	while (gw < 64 && gw * (vec ? VEC : 1) < dim) gw <<= 1;
+	const uint32_t items = update_small_items(n);
+	void (*kernel)(const F*, size_t, const uint32_t*, F*, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t) = nullptr;
+#define KMX_PICK_LM(I, V, L) (layout_means == KMX_AOS ? update_small_kernel<F, I, V, L, KMX_AOS> : update_small_kernel<F, I, V, L, KMX_SOA>)
+#define KMX_PICK(I) (layout == KMX_SOA ? KMX_PICK_LM(I, 1, KMX_SOA) : vec ? KMX_PICK_LM(I, VEC, KMX_AOS) : KMX_PICK_LM(I, 1, KMX_AOS))
+	kernel = items == 1 ? KMX_PICK(1) : items == 3 ? KMX_PICK(3) : KMX_PICK(8);
+#undef KMX_PICK
+#undef KMX_PICK_LM
+	if (lds > 48 * 1024) KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(UPDATE_SMALL_THREADS), lds, stream(), data, stride, assignment, means, stride_means, sizes, dim, k, n, per, gw,
+	                   divide ? 1u : 0u, ((uintptr_t)assignment & 15) == 0 ? 1u : 0u);
+	KMX_LAUNCH_CHECK("update_small_kernel");
+	return KMX_OK;
+}
+
+#define KMX_SMALL_INSTANCES(F)                                                                                                                                   \
+	template bool small_assign_fits<F>(uint32_t, uint32_t, uint32_t, uint32_t);                                                                                  \
+	template bool small_update_fits<F>(uint32_t, uint32_t, uint32_t, uint32_t, const DeviceInfo&);                                                               \
+	template int launch_assign_small<F>(const F*, int, size_t, const F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, const DeviceInfo&); \
+	template int launch_update_small<F>(const F*, int, size_t, const uint32_t*, F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, uint32_t*, const DeviceInfo&);
+KMX_SMALL_INSTANCES(float)
+KMX_SMALL_INSTANCES(double)
+
+} // namespace kmx

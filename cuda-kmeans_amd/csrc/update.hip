@@ -718,28 +718,32 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
 
 /*
  * means[c][d] = (sum over the chunks of partial[chunk][c][d]) / count[c]  (0 for an empty cluster).
- * Block = 64 consecutive elements x 16 chunk shares; every lane keeps up to 16 loads in flight; the shares meet in LDS.
+ * Block = COLS consecutive elements x up to 1024 / COLS chunk shares; every lane keeps up to 16 loads in flight, the rest of its
+ * share too (one after the other they cost a trip to memory each: 469 chunks 12 -> 7 us); the shares meet in LDS. COLS = 64, or
+ * 16 where few elements and many chunks would leave a handful of work-groups with long shares (512 elements, 1024 chunks: 9.4 us
+ * with 8 work-groups).
  * Overwrites means: the sorted path needs neither zeroed centroids nor the separate divide kernel.
  * divide = 0 stores the sums themselves.
  */
-constexpr uint32_t REDUCE_SHARES = 16;
+constexpr uint32_t REDUCE_THREADS = 1024;
 
-template <int LM>
-__global__ void __launch_bounds__(64 * REDUCE_SHARES)
+template <int LM, uint32_t COLS>
+__global__ void __launch_bounds__(REDUCE_THREADS)
 reduce_partials_kernel(const float* __restrict__ partial, const uint32_t* __restrict__ partial_counts, float* __restrict__ means, size_t stride_means,
                        uint32_t* __restrict__ sizes, uint32_t dim, uint32_t k, uint32_t chunks, uint32_t divide)
 {
-	__shared__ float part[REDUCE_SHARES][64];
-	__shared__ uint32_t part_count[REDUCE_SHARES][64];
-	const uint32_t col = threadIdx.x & 63, share = threadIdx.x >> 6;
-	const uint32_t shares = blockDim.x >> 6; /* 1 to REDUCE_SHARES: the launcher gives every share at least 8 chunks */
-	const uint32_t e = blockIdx.x * 64 + col;
+	constexpr uint32_t MAX_SHARES = REDUCE_THREADS / COLS;
+	__shared__ float part[MAX_SHARES][COLS];
+	__shared__ uint32_t part_count[MAX_SHARES][COLS];
+	const uint32_t col = threadIdx.x % COLS, share = threadIdx.x / COLS;
+	const uint32_t shares = blockDim.x / COLS; /* the launcher gives every share at least 8 chunks */
+	const uint32_t e = blockIdx.x * COLS + col;
 	const size_t kd = (size_t)k * dim;
 	const uint32_t per = (chunks + shares - 1) / shares;
 	const uint32_t c0 = min(share * per, chunks), c1 = min(c0 + per, chunks);
-	/* the clusters the 64 elements of this work-group belong to (at most 64): lane `col` counts cluster cl_lo + col */
-	const uint32_t cl_lo = (uint32_t)(((size_t)blockIdx.x * 64) / dim);
-	const uint32_t cl_hi = (uint32_t)min((size_t)k - 1, ((size_t)blockIdx.x * 64 + 63) / dim);
+	/* the clusters the elements of this work-group belong to (at most COLS): lane `col` counts cluster cl_lo + col */
+	const uint32_t cl_lo = (uint32_t)(((size_t)blockIdx.x * COLS) / dim);
+	const uint32_t cl_hi = (uint32_t)min((size_t)k - 1, ((size_t)blockIdx.x * COLS + COLS - 1) / dim);
 	/* the count partials of this lane's cluster are requested first and added up after the sums, so that both sets of
 	 * loads are in flight together */
 	const bool counting = cl_lo + col <= cl_hi;
@@ -757,13 +761,24 @@ reduce_partials_kernel(const float* __restrict__ partial, const uint32_t* __rest
 #pragma unroll
 			for (int u = 0; u < 16; ++u) s += v[u];
 		}
-		for (; c < c1; ++c) s += partial[(size_t)c * kd + e];
+		if (c < c1) {
+			float v[16];
+#pragma unroll
+			for (int u = 0; u < 16; ++u) v[u] = c + u < c1 ? partial[(size_t)(c + u) * kd + e] : 0.0f;
+#pragma unroll
+			for (int u = 0; u < 16; ++u) s += v[u];
+		}
 	}
 	uint32_t members = 0;
 #pragma unroll
 	for (int u = 0; u < 16; ++u) members += cv[u];
 	if (counting)
-		for (uint32_t c = c0 + 16; c < c1; ++c) members += pc[(size_t)c * k];
+		for (uint32_t c = c0 + 16; c < c1; c += 16) {
+#pragma unroll
+			for (int u = 0; u < 16; ++u) cv[u] = c + u < c1 ? pc[(size_t)(c + u) * k] : 0u;
+#pragma unroll
+			for (int u = 0; u < 16; ++u) members += cv[u];
+		}
 	part_count[share][col] = members;
 	part[share][col] = s;
 	__syncthreads();
@@ -841,6 +856,19 @@ static uint32_t pow2_at_least(uint32_t v)
 	return p;
 }
 
+int launch_reduce_partials(const UpdateArgs& u, const float* partial, const uint32_t* partial_counts, uint32_t chunks)
+{
+	const uint32_t total = u.k * u.dim;
+	const uint32_t cols = chunks > 256 && total <= 16384 ? 16 : 64;
+	const uint32_t shares = std::max<uint32_t>(64 / cols, std::min<uint32_t>(REDUCE_THREADS / cols, chunks / 8));
+	auto kernel = u.layout_means == KMX_AOS ? (cols == 16 ? reduce_partials_kernel<KMX_AOS, 16> : reduce_partials_kernel<KMX_AOS, 64>)
+	                                        : (cols == 16 ? reduce_partials_kernel<KMX_SOA, 16> : reduce_partials_kernel<KMX_SOA, 64>);
+	KMX_LAUNCH_KERNEL(kernel, dim3((total + cols - 1) / cols), dim3(cols * shares), 0, stream(),
+	                   partial, partial_counts, u.means, u.stride_means, u.cluster_sizes, u.dim, u.k, chunks, u.divide ? 1u : 0u);
+	KMX_LAUNCH_CHECK("reduce_partials_kernel");
+	return KMX_OK;
+}
+
 template <int ITEMS, int LM>
 static int launch_sorted(const UpdateArgs& u, Workspace* ws, uint32_t chunks, uint32_t slices, uint32_t chunk_points, uint32_t gw, uint32_t vec, uint32_t lds_bytes, bool whole_rows)
 {
@@ -872,12 +900,7 @@ static int launch_sorted(const UpdateArgs& u, Workspace* ws, uint32_t chunks, ui
 	KMX_LAUNCH_KERNEL(kernel, dim3(chunks, slices), dim3(1024), lds_bytes, stream(),
 	                   u.data, u.stride, u.assignment, ws->partials, partial_counts, u.dim, u.k, u.n, chunk_points);
 	KMX_LAUNCH_CHECK("update_sorted_kernel");
-	const uint32_t total = u.k * u.dim;
-	const uint32_t shares = std::max<uint32_t>(1, std::min<uint32_t>(REDUCE_SHARES, chunks / 8));
-	KMX_LAUNCH_KERNEL((reduce_partials_kernel<LM>), dim3((total + 63) / 64), dim3(64 * shares), 0, stream(),
-	                   ws->partials, partial_counts, u.means, u.stride_means, u.cluster_sizes, u.dim, u.k, chunks, u.divide ? 1u : 0u);
-	KMX_LAUNCH_CHECK("reduce_partials_kernel");
-	return KMX_OK;
+	return launch_reduce_partials(u, ws->partials, partial_counts, chunks);
 }
 
 /* Picks and launches the kernel of KMX_UPDATE_ATOMIC_SHM. *state: 0 = no LDS variant fits the shape, 1 = sums and
@@ -1202,6 +1225,13 @@ int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Works
 	if (variant == KMX_UPDATE_SERIAL_ORDER)
 		return launch_update_serial_order<float>(u.data, u.layout, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes,
 		                                         u.dim, u.k, u.n, u.divide, exec, ws, dev);
+	if (variant == KMX_UPDATE_ATOMIC_SHM && small_update_fits<float>(u.dim, u.k, u.n, lds_budget_of(exec, dev), dev)) {
+		int rc = profile_begin(1);
+		if (rc) return rc;
+		rc = launch_update_small<float>(u.data, u.layout, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes,
+		                                u.dim, u.k, u.n, u.divide, &exec->block_count, dev);
+		return rc ? rc : profile_end(1);
+	}
 	/* (the fixed work space has no room for a copy of the points: SoA points then stay with the element-wise kernels) */
 	if (!ws->fixed && u.layout == KMX_SOA && (variant & ~KMX_UPDATE_EMULATED_ATOMICS) == KMX_UPDATE_ATOMIC_SHM && u.n > 0 && u.dim >= 8 &&
 	    (size_t)u.n * u.dim * sizeof(float) <= ROWS_COPY_MAX_BYTES) {

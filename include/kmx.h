@@ -246,7 +246,7 @@ int kmx_fused_f32(int variant,
  * one call buys: where a single kernel can hold all centroids (k <= 32, dim <= 32 -- the shapes bound by HBM, where reading
  * the points twice is what an iteration costs) it reads every point ONCE, assigns it, accumulates it and writes its
  * assignment; everywhere else the call is the two calls it stands for. kmx_iteration_last_passes tells which of the two
- * ran (1 or 2 passes over the points; 0 before the first call).
+ * ran (1 or 2 passes over the points; 0 before the first call; small inputs of other shapes may be read once as well and count as 2).
  */
 int kmx_iteration_f32(const float* data, int layout, size_t stride,
                       const float* means_in, float* means_out, int layout_means, size_t stride_means,
