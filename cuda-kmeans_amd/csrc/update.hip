@@ -14,7 +14,7 @@
  *                              of the k x dim block in LDS and accumulates with plain read-add-write; the
  *                              copies are merged at the end, one global atomic per element and work-group.
  *                              (update_private_vec_kernel: the same with 16-byte row pieces per lane, for
- *                              a million points or more: N = 16.7M, d = 16, k = 16 in 0.205 instead of 0.250 ms.)
+ *                              millions of points: N = 16.7M, d = 16, k = 16 in 0.205 instead of 0.250 ms.)
  *       update_sorted_kernel   larger k: the work-group counting-sorts its chunk of points by cluster
  *                              with integer LDS atomics, then lane groups walk the sorted list and sum each
  *                              cluster's rows in registers (no atomics at all); per-chunk sums go to a partial
@@ -389,21 +389,27 @@ update_private_kernel(const float* __restrict__ data, size_t stride, const uint3
 }
 
 /*
- * The same with 16-byte pieces of a row per lane (dim a multiple of 4, aligned rows): a group is GW4 = dim / 4 lanes (rounded
+ * The same with 16-byte pieces of a row per lane: a group is GW4 = dim / 4 lanes (rounded
  * up to a power of two), so a wavefront reads 64 / GW4 consecutive rows with one instruction -- a quarter of the load
  * instructions, and of the loads of the assignment, that one lane per dimension issues. Every group still needs a copy of its
  * own (lanes of one instruction that met in one copy would lose updates), so a work-group of 256 lanes holds 256 / GW4 copies:
  * more LDS per work-group, fewer work-groups per compute unit, the same bytes in flight.
  */
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int UPDATE_UNROLL_VEC = 8; /* row pieces in flight per lane (16 measured the same) */
 
-template <int LM>
+/*
+ * FULL: dim a multiple of 4 and aligned rows. Otherwise the last piece of a row is read so that it ends with the row (16-byte
+ * loads need 4-byte alignment only) and shifted into place; the sums in LDS have rows of whole pieces, whose surplus is never read.
+ */
+template <int LM, bool FULL>
 __global__ void __launch_bounds__(256)
 update_private_vec_kernel(const float* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment,
                           float* __restrict__ means, size_t stride_means, uint32_t* __restrict__ sizes,
                           uint32_t dim, uint32_t k, uint32_t n, uint32_t gw, uint32_t copy_stride, uint32_t chunk_points)
 {
 	extern __shared__ __attribute__((aligned(16))) float lds[];
+	const uint32_t dim4 = (dim + 3) & ~3u;
 	const uint32_t groups = blockDim.x / gw;
 	const uint32_t group = threadIdx.x / gw;
 	const uint32_t gl = threadIdx.x - group * gw;
@@ -411,14 +417,26 @@ update_private_vec_kernel(const float* __restrict__ data, size_t stride, const u
 	__syncthreads();
 
 	float* acc = lds + (size_t)group * copy_stride;
-	uint32_t* cnt = (uint32_t*)(acc + (size_t)k * dim);
+	uint32_t* cnt = (uint32_t*)(acc + (size_t)k * dim4);
 	const uint32_t p_begin = (uint32_t)min((uint64_t)blockIdx.x * chunk_points, (uint64_t)n);
 	const uint32_t p_end = (uint32_t)min((uint64_t)p_begin + chunk_points, (uint64_t)n);
 	const bool lane_on = gl * 4 < dim;
-	const float* src = data + (lane_on ? gl * 4 : 0);
-	auto add_row = [&](uint32_t target, const f32x4& v) {
+	const uint32_t d0 = lane_on ? gl * 4 : 0;
+	const uint32_t shift = FULL ? 0u : d0 + 4 > dim ? d0 + 4 - dim : 0u; /* places the piece was read too early */
+	const float* src = data + d0 - shift;
+	auto load = [&](uint32_t p) -> f32x4 {
+		if constexpr (FULL) return *(const f32x4*)(src + (size_t)p * stride);
+		else return *(const f32x4_any*)(src + (size_t)p * stride);
+	};
+	auto add_row = [&](uint32_t target, const f32x4& w) {
 		if (lane_on) {
-			f32x4* at = (f32x4*)(acc + target * dim + gl * 4);
+			f32x4 v = w;
+			if constexpr (!FULL) {
+				v.x = shift == 0 ? w.x : shift == 1 ? w.y : shift == 2 ? w.z : w.w;
+				v.y = shift == 0 ? w.y : shift == 1 ? w.z : w.w;
+				v.z = shift == 0 ? w.z : w.w;
+			}
+			f32x4* at = (f32x4*)(acc + target * dim4 + gl * 4);
 			f32x4 a = *at;
 			a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
 			*at = a;
@@ -431,24 +449,24 @@ update_private_vec_kernel(const float* __restrict__ data, size_t stride, const u
 		uint32_t t[UPDATE_UNROLL_VEC];
 #pragma unroll
 		for (int u = 0; u < UPDATE_UNROLL_VEC; ++u) {
-			v[u] = *(const f32x4*)(src + (size_t)(p + u * groups) * stride);
+			v[u] = load(p + u * groups);
 			t[u] = assignment[p + u * groups];
 		}
 #pragma unroll
 		for (int u = 0; u < UPDATE_UNROLL_VEC; ++u) add_row(t[u], v[u]);
 	}
-	for (; p < p_end; p += groups) add_row(assignment[p], *(const f32x4*)(src + (size_t)p * stride));
+	for (; p < p_end; p += groups) add_row(assignment[p], load(p));
 	__syncthreads();
 
 	for (uint32_t e = threadIdx.x; e < k * dim; e += blockDim.x) {
-		float s = 0.0f;
-		for (uint32_t g = 0; g < groups; ++g) s += lds[(size_t)g * copy_stride + e];
 		const uint32_t c = e / dim, d = e - c * dim;
+		float s = 0.0f;
+		for (uint32_t g = 0; g < groups; ++g) s += lds[(size_t)g * copy_stride + c * dim4 + d];
 		if (s != 0.0f) atomic_add_f32(&means[elem<LM>(stride_means, c, d)], s);
 	}
 	for (uint32_t c = threadIdx.x; c < k; c += blockDim.x) {
 		uint32_t s = 0;
-		for (uint32_t g = 0; g < groups; ++g) s += ((const uint32_t*)lds)[(size_t)g * copy_stride + (size_t)k * dim + c];
+		for (uint32_t g = 0; g < groups; ++g) s += ((const uint32_t*)lds)[(size_t)g * copy_stride + (size_t)k * dim4 + c];
 		if (s) atomicAdd(&sizes[c], s);
 	}
 }
@@ -469,15 +487,15 @@ update_private_vec_kernel(const float* __restrict__ data, size_t stride, const u
 constexpr uint32_t SORT_SHIFT = 15; /* local point index bits: chunk_points <= 32768 */
 constexpr int SORT_UNROLL = 8;      /* row loads per batch and lane group in the segment-sum phase (two batches in flight; 16 measured slower) */
 
-/* VEC consecutive floats of a row per lane: one 16-byte load when VEC = 4 (needs dim, stride % 4 == 0 and an aligned base). */
+/* VEC consecutive floats of a row per lane: one 16-byte load when VEC = 4. In global memory those need 4-byte alignment only, in
+ * LDS all of it. */
 template <int VEC> struct RowPart { float v[VEC]; };
-
 template <int VEC>
 __device__ __forceinline__ RowPart<VEC> load_part(const float* p)
 {
 	RowPart<VEC> r;
 	if constexpr (VEC == 4) {
-		const f32x4 t = *(const f32x4*)p;
+		const f32x4 t = *(const f32x4_any*)p;
 		r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
 	} else {
 #pragma unroll
@@ -492,12 +510,16 @@ __device__ __forceinline__ void store_part(float* p, const RowPart<VEC>& r)
 	if constexpr (VEC == 4) {
 		f32x4 t;
 		t.x = r.v[0]; t.y = r.v[1]; t.z = r.v[2]; t.w = r.v[3];
-		*(f32x4*)p = t;
+		*(f32x4_any*)p = t;
 	} else {
 #pragma unroll
 		for (int i = 0; i < VEC; ++i) p[i] = r.v[i];
 	}
 }
+
+/* the same in LDS, at multiples of VEC floats */
+template <int VEC> struct alignas(4 * VEC) LdsPart { RowPart<VEC> part; };
+template <int VEC> __device__ __forceinline__ LdsPart<VEC>& lds_part(float* p) { return *(LdsPart<VEC>*)p; }
 
 template <int ITEMS, int GW, int VEC, bool WHOLE_ROWS = false>
 __global__ void __launch_bounds__(1024)
@@ -577,8 +599,11 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
 	const uint32_t group = tid / GW, gl = tid % GW;
 	const uint32_t entries = offsets[k];
 	const bool lane_on = gl * VEC < width;
-	const float* src = data + (size_t)p_begin * stride + d0 + (lane_on ? gl * VEC : 0);
-	float* out = partial + ((size_t)blockIdx.x * k) * dim + d0 + gl * VEC;
+	/* the last piece of a row that is no whole number of pieces ends with the row: the coordinates it shares with the piece
+	 * before it are summed by both lanes in the same order and stored twice with the same value */
+	const uint32_t d_lane = lane_on ? min(gl * VEC, width - VEC) : 0u;
+	const float* src = data + (size_t)p_begin * stride + d0 + d_lane;
+	float* out = partial + ((size_t)blockIdx.x * k) * dim + d0 + d_lane;
 	constexpr uint32_t LOCAL_MASK = (1u << SORT_SHIFT) - 1u;
 
 	/* the clusters [c_begin, c_stop) and their entries [e_begin, e_stop) that this work-group sums: all of them, or (WHOLE_ROWS)
@@ -601,7 +626,10 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
 	}
 	const uint32_t e_begin = offsets[c_begin], e_stop = offsets[c_stop];
 	auto cluster_at = [&](uint32_t e) -> uint32_t { return e < e_stop ? sorted[e] >> SORT_SHIFT : c_stop; };
-	auto range_begin = [&](uint32_t g) -> uint32_t { return e_begin + (uint32_t)((uint64_t)g * (e_stop - e_begin) / GROUPS); };
+	/* at least a batch of entries per group: with fewer, one cluster spans many groups whose pieces are then added one after the
+	 * other (d = 4, k = 8, N = 70000: 83 us with an entry per group) */
+	const uint32_t per_group = max((uint32_t)SORT_UNROLL, (e_stop - e_begin + GROUPS - 1) / GROUPS);
+	auto range_begin = [&](uint32_t g) -> uint32_t { return min(e_begin + g * per_group, e_stop); };
 
 	/* Lane group g takes the entries [range_begin(g), range_begin(g + 1)): every group the same number of rows, whatever
 	 * the cluster sizes (cut at cluster boundaries the ranges differed by a cluster's size, and the last group to finish set
@@ -633,7 +661,7 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
 	auto flush_to = [&](uint32_t t) {
 		while (cur < t) {
 			if (head_pending) {
-				store_part<VEC>(heads + (size_t)group * (GW * VEC) + gl * VEC, acc);
+				lds_part<VEC>(heads + (size_t)group * (GW * VEC) + gl * VEC).part = acc;
 				head_pending = false;
 			}
 			else if (lane_on) store_part<VEC>(out + (size_t)cur * dim, acc);
@@ -697,7 +725,7 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
 	if (tail_open) {
 		if (head_pending) {
 			/* the whole range lies inside one cluster that began before it and goes on behind it */
-			store_part<VEC>(heads + (size_t)group * (GW * VEC) + gl * VEC, acc);
+			lds_part<VEC>(heads + (size_t)group * (GW * VEC) + gl * VEC).part = acc;
 			if (gl == 0) whole[group] = 1u;
 		}
 		else collect = true;
@@ -707,7 +735,7 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
 	if (collect) {
 		for (uint32_t g = group + 1; g < GROUPS; ++g) {
 			if (range_begin(g) == range_begin(g + 1)) continue;
-			const RowPart<VEC> piece = load_part<VEC>(heads + (size_t)g * (GW * VEC) + gl * VEC);
+			const RowPart<VEC> piece = lds_part<VEC>(heads + (size_t)g * (GW * VEC) + gl * VEC).part;
 #pragma unroll
 			for (int i = 0; i < VEC; ++i) acc.v[i] += piece.v[i];
 			if (!whole[g]) break;
@@ -859,7 +887,7 @@ static uint32_t pow2_at_least(uint32_t v)
 int launch_reduce_partials(const UpdateArgs& u, const float* partial, const uint32_t* partial_counts, uint32_t chunks)
 {
 	const uint32_t total = u.k * u.dim;
-	const uint32_t cols = chunks > 256 && total <= 16384 ? 16 : 64;
+	const uint32_t cols = chunks > 256 && total <= 4096 ? 16 : 64;
 	const uint32_t shares = std::max<uint32_t>(64 / cols, std::min<uint32_t>(REDUCE_THREADS / cols, chunks / 8));
 	auto kernel = u.layout_means == KMX_AOS ? (cols == 16 ? reduce_partials_kernel<KMX_AOS, 16> : reduce_partials_kernel<KMX_AOS, 64>)
 	                                        : (cols == 16 ? reduce_partials_kernel<KMX_SOA, 16> : reduce_partials_kernel<KMX_SOA, 64>);
@@ -903,6 +931,19 @@ static int launch_sorted(const UpdateArgs& u, Workspace* ws, uint32_t chunks, ui
 	return launch_reduce_partials(u, ws->partials, partial_counts, chunks);
 }
 
+/*
+ * Private copies or sorted chunks (us per call, private / sorted). Clearing and folding the copies costs a work-group the same
+ * whatever its points, so 16-byte pieces pay from here on: d = 16, k = 16: 1 M 29 / 32, 2 M 37 / 50, 4 M 53 / 87; d = 13,
+ * k = 20: 1 M 29 / 24, 2 M 42 / 47, 4 M 66 / 94; d = 32, k = 16: 1 M 37 / 34, 2 M 52 / 54; d = 60, k = 3: 1 M 67 / 62, 2 M 100 / 133.
+ */
+constexpr uint32_t PRIVATE_VEC_MIN_POINTS = 3u << 19;
+/* Single words per lane are for short rows: d = 4, k = 8 12 us (70 k points) to 62 (12 M) against 18 to 228; d = 8, k = 64:
+ * 70 k 14 / 12, 500 k 26 / 15, 2 M 43 / 38, 4 M 66 / 72. From nine dimensions on the sorted chunks are ahead everywhere the
+ * pieces above do not fit (d = 32, k = 64: 70 k 22 / 12, 4 M 238 / 99; d = 64, k = 32: 200 k 57 / 19, 4 M 287 / 199). */
+static bool private_words_pay(uint32_t dim, uint32_t k, uint32_t n)
+{
+	return dim <= 4 || (dim <= 8 && (k <= 32 || n >= (3u << 20)));
+}
 /* Picks and launches the kernel of KMX_UPDATE_ATOMIC_SHM. *state: 0 = no LDS variant fits the shape, 1 = sums and
  * counts accumulated (divide still to do), 2 = centroids finished (the sorted path divides while it folds the partials). */
 template <int LD, int LM>
@@ -911,12 +952,12 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 	*state = 1;
 	const uint32_t budget = exec->shared_mem_bytes ? std::min(exec->shared_mem_bytes, dev.lds_bytes) : dev.lds_bytes;
 
-	if (LD == KMX_AOS && u.dim >= 8 && u.dim <= 64 && u.dim % 4 == 0 && u.stride % 4 == 0 && ((uintptr_t)u.data & 15) == 0 && u.n >= (1u << 20)) {
-		/* private copies for groups of dim / 4 lanes with 16-byte row pieces (from a million points on: clearing and folding four
-		 * times as many copies costs small inputs more than the wider loads save) */
-		const uint32_t gw = pow2_at_least(u.dim / 4);
+	if (LD == KMX_AOS && u.dim >= 8 && u.dim <= 64 && u.n >= PRIVATE_VEC_MIN_POINTS) {
+		/* private copies for groups of dim / 4 lanes with 16-byte row pieces */
+		const uint32_t gw = pow2_at_least((u.dim + 3) / 4);
+		const bool full = u.dim % 4 == 0 && u.stride % 4 == 0 && ((uintptr_t)u.data & 15) == 0;
 		const uint32_t groups = 256 / gw;
-		const uint64_t copy_words = (uint64_t)u.k * (u.dim + 1);
+		const uint64_t copy_words = (uint64_t)u.k * ((u.dim + 3) / 4 * 4 + 1);
 		const uint64_t copy_stride = (copy_words + 31) / 32 * 32 + 4 * gw; /* groups of one 128-byte LDS cycle start 4 gw banks apart */
 		const uint64_t lds_bytes = groups * copy_stride * 4;
 		if (lds_bytes <= std::min<uint32_t>(budget, 96 * 1024)) {
@@ -929,8 +970,9 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 			exec->block_count = chunks;
 			int rc = clear_outputs(u);
 			if (rc) return rc;
-			KMX_HIP(hipFuncSetAttribute((const void*)update_private_vec_kernel<LM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-			KMX_LAUNCH_KERNEL((update_private_vec_kernel<LM>), dim3(chunks), dim3(256), (uint32_t)lds_bytes, stream(),
+			auto kernel = full ? update_private_vec_kernel<LM, true> : update_private_vec_kernel<LM, false>;
+			KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+			KMX_LAUNCH_KERNEL(kernel, dim3(chunks), dim3(256), (uint32_t)lds_bytes, stream(),
 			                   u.data, u.stride, u.assignment, u.means, u.stride_means, u.cluster_sizes,
 			                   u.dim, u.k, u.n, gw, (uint32_t)copy_stride, chunk_points);
 			KMX_LAUNCH_CHECK("update_private_vec_kernel");
@@ -938,7 +980,7 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 		}
 	}
 
-	if (LD == KMX_AOS && u.dim <= 64) {
+	if (LD == KMX_AOS && private_words_pay(u.dim, u.k, u.n)) {
 		/* private copies: 256 / gw groups, each k*dim sums + k counts, padded so that groups start gw banks apart */
 		const uint32_t gw = pow2_at_least(u.dim);
 		const uint32_t groups = 256 / gw;
@@ -965,14 +1007,12 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 
 	if (LD == KMX_AOS && u.k < (1u << (32 - SORT_SHIFT)) && (uint64_t)(u.k + 36) * 4 + 1024 * 4 + 1024 * 5 * 4 <= budget) {
 		const uint32_t slices = (u.dim + 31) / 32;
-		/* 16-byte row parts where one slice covers the row and its alignment allows it (measured: no gain for sliced rows) */
-		const bool aligned4 = u.dim % 4 == 0 && u.stride % 4 == 0 && ((uintptr_t)u.data & 15) == 0;
 		/* rows of 33 to 256 dimensions: the work-groups of a chunk take ranges of clusters and read whole rows (measured at
 		 * N = 1M, d = 256, k = 1024: 0.29 ms in slices of 32 dimensions) */
-		const bool whole_rows = u.dim > 32 && u.dim <= 256 && aligned4;
-		/* 16-byte row parts where one slice covers the row and its alignment allows it (measured: no gain for sliced rows) */
-		const uint32_t vec = ((u.dim <= 32 && aligned4) || whole_rows) ? 4 : 1;
-		const uint32_t gw = whole_rows ? std::max<uint32_t>(16, pow2_at_least(u.dim / 4)) : (u.dim > 16 ? 32 : pow2_at_least(std::max<uint32_t>(u.dim, 4))) / vec;
+		const bool whole_rows = u.dim > 32 && u.dim <= 256;
+		/* 16-byte row parts where one slice covers the row, whatever its alignment (measured: no gain for sliced rows) */
+		const uint32_t vec = u.dim >= 4 && u.dim <= 256 ? 4 : 1;
+		const uint32_t gw = whole_rows ? std::max<uint32_t>(16, pow2_at_least((u.dim + 3) / 4)) : (u.dim > 16 ? 32 : pow2_at_least(std::max<uint32_t>(u.dim, 4))) / vec;
 		const uint32_t pieces_bytes = 1024u * (vec + 1) * 4; /* sums of clusters cut by a range boundary, and a flag per lane group */
 		const uint32_t max_points = std::min<uint32_t>(1u << SORT_SHIFT, (budget - (u.k + 36) * 4 - pieces_bytes) / 4 / 1024 * 1024);
 		/* one chunk per compute unit; two for rows of at most 16 bytes, whose chunks are bound by the sorting, not by their
