@@ -134,6 +134,21 @@ __device__ __forceinline__ void load_packed_points(SplitPoints<1> (&b)[P], float
 	convert_packed_points<P>(b, xx, raw, h, frame);
 }
 
+/* four coordinates from `d` on of an AoS row of any alignment (16-byte loads need 4-byte alignment only), zeros beyond the row:
+ * word by word only where the row ends inside the piece (N = 300 k, d = 50, k = 300: sweep 60 us with eight loads per half-wave and block) */
+__device__ __forceinline__ void load_piece_any(float* v, const float* __restrict__ src, bool valid, uint32_t d, uint32_t dim)
+{
+	typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+	f32x4 t = { 0.0f, 0.0f, 0.0f, 0.0f };
+	if (valid && d + 4 <= dim) t = *(const f32x4_any*)src;
+	else if (valid && d < dim) {
+		t.x = src[0];
+		if (d + 1 < dim) t.y = src[1];
+		if (d + 2 < dim) t.z = src[2];
+	}
+	v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+}
+
 /* LISTED: the sweep covers the points of a list (entries of two words, the first one the point number); position
  * base + p TILE + col of the list stands where the point number itself stands otherwise, n is the length of the list */
 template <int KB, int P, int LD, bool VEC, bool LISTED = false>
@@ -170,8 +185,8 @@ __device__ __forceinline__ void request_split_points(RawPoints<KB, false> (&raw)
 				if (KB > 4 && kb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
 			}
 			else {
-#pragma unroll
-				for (int j = 0; j < 8; ++j) v[j] = (valid && d0 + j < dim) ? data[elem<LD>(stride, pt, d0 + j)] : 0.0f;
+				load_piece_any(v, data + (size_t)pt * stride + d0, valid, d0, dim);
+				load_piece_any(v + 4, data + (size_t)pt * stride + d0 + 4, valid, d0 + 4, dim);
 			}
 		}
 	}
@@ -251,8 +266,8 @@ __device__ __forceinline__ void load_split_points(SplitPoints<KB> (&b)[P], float
 				if (KB > 4 && kb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
 			}
 			else {
-#pragma unroll
-				for (int j = 0; j < 8; ++j) v[kb][j] = (valid && d0 + j < dim) ? data[elem<LD>(stride, pt, d0 + j)] : 0.0f;
+				load_piece_any(v[kb], data + (size_t)pt * stride + d0, valid, d0, dim);
+				load_piece_any(v[kb] + 4, data + (size_t)pt * stride + d0 + 4, valid, d0 + 4, dim);
 			}
 		};
 		float part = 0.0f, along = 0.0f, low = 0.0f;
