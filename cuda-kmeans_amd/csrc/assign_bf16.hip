@@ -34,6 +34,22 @@
 
 namespace kmx {
 
+/*
+ * Where the half-precision sweep (rank16.hip) beats the sweeps of this file (us, here -> there):
+ *   - one tile of centroids and narrow rows are bound by reading the points, which three products hide better, and leave fewer points to
+ *     the exact pass (N = 4M, d = 20, k = 16: 106 -> 141; d = 64, k = 20, N = 1M: 81 -> 67; d = 32, k = 64: 62 -> 51);
+ *   - small narrow calls are latency, the same either way (N = 131072, d = 24, k = 128: 24.5 -> 25.5; N = 200k, d = 40, k = 16: 27.5 ->
+ *     28.3; N = 65536, d = 20, k = 2000: 62 -> 45; N = 30000, d = 200, k = 512: 81 -> 65);
+ *   - SoA points are written out as rows on the way, which many centroids have to pay for (N = 1M, d = 64, k = 64: 116 -> 160;
+ *     d = 32, k = 128: 134 -> 82; N = 250k, d = 50, k = 300: 66 -> 55).
+ */
+static bool rank16_pays(const AssignArgs& a)
+{
+	if (a.layout == KMX_SOA && a.k < 128) return false;
+	if (a.dim > 32) return true;
+	return a.k > 32 && (double)a.n * a.k * a.dim >= 5e8;
+}
+
 /* supported blocks of 16 dimensions per row */
 static uint32_t pick_kb(uint32_t dim)
 {
@@ -193,6 +209,9 @@ int launch_screen_bf16(const float* rows, const Workspace* ws, const uint32_t* r
 int launch_assign_bf16(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	if (args.dim > 256) return launch_assign_wide(args, exec, ws, dev);
+	const int mode = two_level_mode(); /* kmx_set_two_level_sweep: 0 never, 1 where it pays, 2 wherever the kernels allow it */
+	if (!args.ranking_only && args.two_level && mode != 0 && (mode == 2 || rank16_pays(args)) && rank16_supports(args, lds_budget_of(exec, dev)))
+		return launch_assign_rank16(args, exec, ws, dev);
 	AssignArgs a = args;
 	/* wide rows and many centroids: a second sweep screens the queued points (narrow rows fit the registers of the
 	 * lane-per-centroid kernels, which then need fewer launches); so do the packed rows, whose sweep queues more points

@@ -674,6 +674,7 @@ static int launch_recheck_l(const AssignArgs& a, Workspace* ws, uint32_t kp)
 static size_t g_queued_rows_bytes = (size_t)1 << 30; /* upper bound of the block of copied rows */
 
 void set_queued_rows_limit(size_t bytes) { g_queued_rows_bytes = bytes; }
+size_t queued_rows_limit() { return g_queued_rows_bytes; }
 
 /* a group of `1 << group_shift` lanes (the smallest power of two that covers the row, at most a wavefront) copies one row */
 template <int LD>

@@ -55,7 +55,9 @@ struct Workspace {
 	uint32_t* queue = nullptr;      size_t queue_cap = 0;      /* entries */
 	uint32_t* counters = nullptr;                               /* 16 words */
 	float* packed_means = nullptr;  size_t packed_cap = 0;     /* floats  */
+	float* packed16 = nullptr;      size_t packed16_cap = 0;   /* floats: half-precision operands of the centroids (rank16.hip) */
 	float* norms = nullptr;         size_t norms_cap = 0;      /* floats  */
+	float* norms16 = nullptr;       size_t norms16_cap = 0;    /* floats: norms, frame and scale of the half-precision sweep */
 	float* means_t = nullptr;       size_t means_t_cap = 0;    /* floats: exact transposed centroids [dim][kp] */
 	float* partials = nullptr;      size_t partials_cap = 0;   /* floats  */
 	uint32_t* fused_assignment = nullptr; size_t fused_cap = 0; /* entries: assignment vector of kmx_fused_f32 */
@@ -71,6 +73,7 @@ struct Workspace {
 int workspace(Workspace** ws);
 int reserve_queue(Workspace* ws, size_t entries);
 int reserve_packed(Workspace* ws, size_t packed_floats, size_t norm_floats, size_t transposed_floats);
+int reserve_packed16(Workspace* ws, size_t packed_floats, size_t norm_floats);
 int reserve_partials(Workspace* ws, size_t floats);
 int reserve_fused_assignment(Workspace* ws, size_t entries);
 int reserve_bucket_sizes(Workspace* ws, size_t entries);
@@ -153,6 +156,7 @@ int launch_assign_base(const AssignArgs& a, kmx_exec_params* exec);
  * exact transposed centroids ws->means_t ([dim][kp]) that pack_means wrote for this call. */
 int launch_recheck(const AssignArgs& a, Workspace* ws, uint32_t kp);
 void set_queued_rows_limit(size_t bytes); /* bound of the block of copied rows */
+size_t queued_rows_limit();
 /* The exact pass behind the split-bf16 sweep for k >= 128 and rows of more than 32 dimensions: the queued rows are copied into a compact block, a second
  * split-bf16 sweep over them notes the (row, centroid) pairs within the threshold (assign_bf16.hip), and one lane
  * per pair evaluates the serial arithmetic. */
@@ -171,6 +175,9 @@ bool mfma_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_mfma(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_bf16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
+/* rank16.hip: one half-precision product per dimension for all points, the serial result for what that leaves */
+bool rank16_supports(const AssignArgs& a, uint32_t lds_budget);
+int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */
 bool wide_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_wide(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);

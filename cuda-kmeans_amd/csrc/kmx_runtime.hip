@@ -120,6 +120,12 @@ int reserve_packed(Workspace* ws, size_t packed_floats, size_t norm_floats, size
 	return grow(&ws->means_t, &ws->means_t_cap, transposed_floats);
 }
 
+int reserve_packed16(Workspace* ws, size_t packed_floats, size_t norm_floats)
+{
+	int rc = grow(&ws->packed16, &ws->packed16_cap, packed_floats);
+	return rc ? rc : grow(&ws->norms16, &ws->norms16_cap, norm_floats);
+}
+
 int reserve_partials(Workspace* ws, size_t floats)
 {
 	if (ws->fixed) {
@@ -151,6 +157,8 @@ static int release_workspace()
 	if (g_ws.counters) KMX_HIP(hipFree(g_ws.counters));
 	if (g_ws.packed_means) KMX_HIP(hipFree(g_ws.packed_means));
 	if (g_ws.norms) KMX_HIP(hipFree(g_ws.norms));
+	if (g_ws.packed16) KMX_HIP(hipFree(g_ws.packed16));
+	if (g_ws.norms16) KMX_HIP(hipFree(g_ws.norms16));
 	if (g_ws.means_t) KMX_HIP(hipFree(g_ws.means_t));
 	if (g_ws.partials) KMX_HIP(hipFree(g_ws.partials));
 	if (g_ws.fused_assignment) KMX_HIP(hipFree(g_ws.fused_assignment));

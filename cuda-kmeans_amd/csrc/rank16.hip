@@ -1,0 +1,226 @@
+/*
+ * Assignment of rows of 5 to 256 dimensions by one half-precision product per dimension, and the exact pass behind it.
+ *
+ * Ranking. Points and centroids are moved to the middle of the centroids and scaled by a power of two S that brings the centroids'
+ * coordinates to about 16..32, then rounded to half precision (11 significant bits): a[j] = S^2 (|c_j|^2 - 2 c_j . x) is one
+ * v_mfma_f32_32x32x16_f16 per 16 dimensions, a third of what three bf16 products cost. The certificate is the one-product form of
+ * certificate.h with the norms of what the roundings actually dropped, |x - x_half| of the point and max_j |c'_j - c'_half| of the
+ * centroids; overflow to infinity and values lost below the smallest half-precision number are covered by the same norms (an
+ * infinite one certifies nothing). Eleven bits instead of the eight of a bf16 make it eight times narrower: at N = 2M, d = 32,
+ * k = 1024 it leaves 0.5 to 4 % of the points, where hi * hi in bf16 left 12 to 26 % to a second sweep with three products.
+ *
+ * Exact pass (rank16_exact_impl.h). One kernel for the listed points: it ranks them again with the same instruction on the same
+ * operands, notes the centroids within the point's threshold (two or three of k) and evaluates the serial arithmetic for those.
+ * Gather, screen, evaluate and scatter were four launches (63 us at N = 1M, d = 256, k = 1024, behind a second sweep of 188).
+ *
+ * What bounds it: the sweep by the matrix instructions and the tracking of the minima that shares the issue slots with them
+ * (N = 1M, d = 256, k = 1024: 630 us, 0.87 PFLOP/s; d = 32, k = 1024, N = 2M: 185 us); the exact pass by reading centroid operands
+ * and rows (12 % of N = 1M, d = 256 listed: 131 us). Whole calls, two bf16 levels before -> now: N = 1M, d = 256, k = 1024 1713 ->
+ * 743 us; N = 2M, d = 128, k = 1024 1443 -> 683 (SoA 1629 -> 940); N = 2M, d = 32, k = 1024 332 -> 230; N = 1M, d = 64, k = 512 203 -> 122;
+ * N = 100k, d = 256, k = 32 92 -> 51.
+ */
+#include "rank16_exact_impl.h"
+
+namespace kmx {
+
+/* ws->packed16: the operands, then the centroids' rows as they are, padded with zeros to whole blocks */
+static size_t rank16_rows_offset(uint32_t kp, uint32_t dp) { return (size_t)kp * dp / 2; }
+
+/* blocks of 16 dimensions the sweep is built for */
+static uint32_t rank16_kb(uint32_t dim)
+{
+	const uint32_t need = (dim + KBLOCK - 1) / KBLOCK;
+	for (uint32_t o : { 1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u })
+		if (need <= o) return o;
+	return 0;
+}
+
+#define KMX_DECLARE_RANK16(W) int launch_rank16_##W(const AssignArgs& a, const Rank16Args& w, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
+KMX_DECLARE_RANK16(1) KMX_DECLARE_RANK16(2) KMX_DECLARE_RANK16(3) KMX_DECLARE_RANK16(4)
+KMX_DECLARE_RANK16(6) KMX_DECLARE_RANK16(8) KMX_DECLARE_RANK16(12) KMX_DECLARE_RANK16(16)
+#define KMX_DECLARE_EXACT16(W) int launch_listed_exact_##W(const AssignArgs& a, const ExactArgs& w, const DeviceInfo& dev);
+KMX_DECLARE_EXACT16(1) KMX_DECLARE_EXACT16(2) KMX_DECLARE_EXACT16(3) KMX_DECLARE_EXACT16(4)
+KMX_DECLARE_EXACT16(6) KMX_DECLARE_EXACT16(8) KMX_DECLARE_EXACT16(12) KMX_DECLARE_EXACT16(16)
+
+/*
+ * One wavefront per (padded) centroid row: its half-precision operands, S^2 |c|^2, the squared norms of what half precision and the
+ * bf16 parts leave out. Every work-group computes the frame m (sweep_frame) and S from the first 16 centroids: S max |c - m| over them
+ * is in [16, 32), so that a coordinate may be 2000 times larger before it overflows.
+ * norms: tiles of S^2 |c - m|^2, then per row low2, mid2, rest2, then the frame (sweep_frame), S and 1 / S^2.
+ */
+__host__ __device__ __forceinline__ size_t rank16_low_offset(uint32_t kp) { return (size_t)(kp / TILE) * NORM_TILE; }
+__host__ __device__ __forceinline__ size_t rank16_frame_offset(uint32_t kp) { return rank16_low_offset(kp) + 3 * (size_t)kp; }
+__host__ __device__ __forceinline__ size_t rank16_scale_offset(uint32_t kp) { return rank16_frame_offset(kp) + FRAME_FLOATS; }
+static size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) + 4; }
+
+template <int LM>
+__global__ void __launch_bounds__(256)
+pack_means16_kernel(const float* __restrict__ means, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
+                    uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t moved, uint32_t* __restrict__ counters)
+{
+	__shared__ float frame[FRAME_DIMS];
+	__shared__ float wave_far[4];
+	const uint32_t lane = threadIdx.x & (WAVE - 1);
+	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; }
+	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+	/* this row's coordinates are requested ahead of the frame they will be moved to */
+	float exact[FRAME_DIMS / WAVE];
+#pragma unroll
+	for (uint32_t i = 0; i < FRAME_DIMS / WAVE; ++i) {
+		const uint32_t q = lane + i * WAVE;
+		exact[i] = (j < k && q < dim) ? means[elem<LM>(stride_means, j, q)] : 0.0f;
+	}
+	sweep_frame<LM>(means, stride_means, dim, k, dp, moved ? FRAME_MOVED : FRAME_KEPT, frame, norms + rank16_frame_offset(kp));
+	float far = 0.0f;
+	for (uint32_t q = threadIdx.x; q < dim; q += 256) {
+		float v[16];
+#pragma unroll
+		for (uint32_t r = 0; r < 16; ++r) v[r] = means[elem<LM>(stride_means, min(r, k - 1), q)];
+#pragma unroll
+		for (uint32_t r = 0; r < 16; ++r) {
+			const float d = __builtin_fabsf(v[r] - frame[q]);
+			if (d < __builtin_inff()) far = fmaxf(far, d);
+		}
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) far = fmaxf(far, __shfl_xor(far, off));
+	if (lane == 0) wave_far[threadIdx.x / WAVE] = far;
+	__syncthreads();
+	far = fmaxf(fmaxf(wave_far[0], wave_far[1]), fmaxf(wave_far[2], wave_far[3]));
+	/* 2^(131 - exponent) puts the largest into [16, 32); kept inside what S and 1 / S^2 can be as normal numbers */
+	const int exponent = (int)(__float_as_uint(far) >> 23);
+	const int shift = far > 0.0f ? min(max(131 - exponent, -60), 60) : 0;
+	const float scale = __uint_as_float((uint32_t)(127 + shift) << 23);
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		norms[rank16_scale_offset(kp)] = scale;
+		norms[rank16_scale_offset(kp) + 1] = __uint_as_float((uint32_t)(127 - 2 * shift) << 23);
+	}
+	if (j >= kp) return;
+	float c2 = 0.0f, low2 = 0.0f, mid2 = 0.0f, rest2 = 0.0f;
+#pragma unroll
+	for (uint32_t i = 0; i < FRAME_DIMS / WAVE; ++i) {
+		const uint32_t q = lane + i * WAVE;
+		if (q >= dp) break;
+		const float v = (j < k && q < dim) ? __builtin_fmaf(exact[i], scale, -(frame[q] * scale)) : 0.0f;
+		c2 += v * v;
+		const float cv = -2.0f * v;
+		const _Float16 half = (_Float16)cv;
+		const float low = cv - (float)half;
+		low2 += low * low;
+		__bf16 hi, mid;
+		const float rest = split_bf16(cv, hi, mid);
+		mid2 += (float)mid * (float)mid;
+		rest2 += rest * rest;
+		rows[(size_t)j * dp + q] = exact[i];
+		packed[(((size_t)(j / TILE) * (dp / KBLOCK) + q / KBLOCK) * WAVE + (q % KBLOCK) / 8 * TILE + j % TILE) * 8 + q % 8] = half;
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) {
+		c2 += __shfl_xor(c2, off);
+		low2 += __shfl_xor(low2, off);
+		mid2 += __shfl_xor(mid2, off);
+		rest2 += __shfl_xor(rest2, off);
+	}
+	if (lane == 0) {
+		norms[norm_at(j)] = j < k ? c2 : 1.7e38f; /* rows that do not exist: beyond all values, but finite (keyed values) */
+		norms[rank16_low_offset(kp) + j] = low2;
+		norms[rank16_low_offset(kp) + kp + j] = mid2;
+		norms[rank16_low_offset(kp) + 2 * kp + j] = rest2;
+	}
+	if (lane < NORM_TILE - TILE && j % TILE == 0) norms[(j / TILE) * NORM_TILE + TILE + lane] = 1.7e38f;
+}
+
+bool rank16_supports(const AssignArgs& a, uint32_t lds_budget)
+{
+	const uint32_t kb = rank16_kb(a.dim);
+	if (a.dim <= 4 || kb == 0 || a.k >= (1u << 25) || a.n > (1u << 31)) return false;
+	const uint32_t sweep = (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + kb * KBLOCK) * 4 + 64 + 2 * (kb * WAVE * 4 + NORM_TILE) * 4; /* two tiles */
+	return sweep <= lds_budget && std::max<uint32_t>(EXACT_GROUPS * kb * WAVE * 16, EXACT_SQUARES * 4) + EXACT_STATIC_BYTES <= lds_budget;
+}
+
+/* the centroids for launch_rank16_sweep */
+static int launch_pack16(const AssignArgs& a, Workspace* ws)
+{
+	const uint32_t dp = rank16_kb(a.dim) * KBLOCK, kp = round_up(a.k, TILE);
+	const int rc = reserve_packed16(ws, rank16_rows_offset(kp, dp) + (size_t)kp * dp, rank16_norms_floats(kp));
+	if (rc) return rc;
+	auto pack = a.layout_means == KMX_AOS ? pack_means16_kernel<KMX_AOS> : pack_means16_kernel<KMX_SOA>;
+	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), 0, stream(),
+	                   a.means, a.stride_means, (_Float16*)ws->packed16, ws->packed16 + rank16_rows_offset(kp, dp), ws->norms16, a.dim, a.k, kp, dp, a.ranking_only ? 0u : 1u, ws->counters);
+	KMX_LAUNCH_CHECK("pack_means16_kernel");
+	return KMX_OK;
+}
+
+/* sweeps the points; what is left goes to ws->listed (length in counters[LISTED_COUNTER]), rows of SoA points to ws->queued_rows */
+static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	const uint32_t kb = rank16_kb(a.dim), kp = round_up(a.k, TILE), copy_stride = round_up(a.dim, 8);
+	int rc = reserve_listed(ws, 2 * (size_t)a.n);
+	if (rc) return rc;
+	if (a.layout == KMX_SOA && (rc = reserve_queued_rows(ws, a.n, copy_stride, 0))) return rc;
+	const float* norms = ws->norms16;
+	const Rank16Args w = { a.data, a.stride, (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp), norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp),
+	                       a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->queued_rows, copy_stride, a.dim, a.k, kp, a.n, 0,
+	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + (a.ranking_only ? 0.0f : 8.0f * CERT_UNIT) + a.kd_extra };
+	switch (kb) {
+	case 1: return launch_rank16_1(a, w, exec, ws, dev);
+	case 2: return launch_rank16_2(a, w, exec, ws, dev);
+	case 3: return launch_rank16_3(a, w, exec, ws, dev);
+	case 4: return launch_rank16_4(a, w, exec, ws, dev);
+	case 6: return launch_rank16_6(a, w, exec, ws, dev);
+	case 8: return launch_rank16_8(a, w, exec, ws, dev);
+	case 12: return launch_rank16_12(a, w, exec, ws, dev);
+	case 16: return launch_rank16_16(a, w, exec, ws, dev);
+	default: return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): dim %u is not supported", a.dim);
+	}
+}
+
+/* the serial result for the points in ws->listed, after launch_rank16_sweep */
+static int launch_listed_exact(const AssignArgs& a, Workspace* ws, const DeviceInfo& dev)
+{
+	const uint32_t kb = rank16_kb(a.dim), dp = kb * KBLOCK, kp = round_up(a.k, TILE);
+	const float* norms = ws->norms16;
+	const bool aos = a.layout == KMX_AOS;
+	const uint32_t row_dim = aos ? a.dim : round_up(a.dim, 8);
+	const ExactArgs w = { aos ? a.data : ws->queued_rows, aos ? a.stride : row_dim, row_dim,
+	                      ws->packed16 + rank16_rows_offset(kp, dp), (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp),
+	                      norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
+	                      a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT };
+	switch (kb) {
+	case 1: return launch_listed_exact_1(a, w, dev);
+	case 2: return launch_listed_exact_2(a, w, dev);
+	case 3: return launch_listed_exact_3(a, w, dev);
+	case 4: return launch_listed_exact_4(a, w, dev);
+	case 6: return launch_listed_exact_6(a, w, dev);
+	case 8: return launch_listed_exact_8(a, w, dev);
+	case 12: return launch_listed_exact_12(a, w, dev);
+	case 16: return launch_listed_exact_16(a, w, dev);
+	default: return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): dim %u is not supported", a.dim);
+	}
+}
+
+static __global__ void clear_word_kernel(uint32_t* word) { *word = 0u; }
+
+int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	int rc = launch_pack16(a, ws);
+	if (rc) return rc;
+	/* SoA points go in parts whose copied rows fit the bound of the workspace (1 GiB unless it was set) */
+	const size_t row_bytes = round_up(a.dim, 8) * sizeof(float);
+	const uint32_t part = a.layout == KMX_AOS ? a.n : (uint32_t)std::min<size_t>(a.n, std::max<size_t>(1024, queued_rows_limit() / row_bytes));
+	for (uint32_t first = 0; first < a.n; first += std::min(part, a.n - first)) {
+		AssignArgs p = a;
+		p.n = std::min(part, a.n - first);
+		p.data = a.data + first;
+		p.assignment = a.assignment + first;
+		if (first) {
+			KMX_LAUNCH_KERNEL(clear_word_kernel, dim3(1), dim3(1), 0, stream(), ws->counters + LISTED_COUNTER);
+			KMX_LAUNCH_CHECK("clear_word_kernel");
+		}
+		if (first == 0 && (rc = profile_begin(0))) return rc;
+		if ((rc = launch_rank16_sweep(p, exec, ws, dev))) return rc;
+		if (first == 0 && (rc = profile_end(0))) return rc;
+		if ((rc = launch_listed_exact(p, ws, dev))) return rc;
+	}
+	return KMX_OK;
+}
+
+} // namespace kmx

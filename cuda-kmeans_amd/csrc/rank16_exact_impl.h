@@ -1,0 +1,342 @@
+/*
+ * The exact pass behind the half-precision sweep (rank16_impl.h): the serial result for the points it listed. Device code,
+ * instantiated per row width (rank16_inst.hip).
+ */
+#ifndef KMX_RANK16_EXACT_IMPL_H
+#define KMX_RANK16_EXACT_IMPL_H
+
+#include "rank16_impl.h"
+
+namespace kmx {
+
+constexpr uint32_t EXACT_THREADS = 512;
+constexpr uint32_t EXACT_WAVES = EXACT_THREADS / WAVE;
+constexpr uint32_t EXACT_GROUPS = 4;                       /* most groups of 32 points per unit */
+constexpr uint32_t EXACT_ROWS = EXACT_GROUPS * TILE;
+constexpr uint32_t EXACT_HITS = 256;                       /* pairs per wavefront and unit that wait for the common evaluation */
+constexpr uint32_t EXACT_PAIR_FLOATS = KBLOCK + 4;         /* a pair's squares of one block of 16 dimensions; the padding spreads 16 lanes' reads over all banks */
+constexpr uint32_t EXACT_SQUARES = EXACT_WAVES * WAVE * EXACT_PAIR_FLOATS;
+
+constexpr uint32_t EXACT_STATIC_BYTES = (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + 3 * EXACT_WAVES) * 4 + 64;
+
+struct ExactArgs {
+	const float* data; size_t stride; uint32_t row_dim; /* AoS, row_dim coordinates (zeros behind the first dim) */
+	const float* means;                     /* rows of KB * 16 floats, zeros behind the coordinates */
+	const f16x8* packed; const float* norms; const float* low; const float* frame; const float* scale;
+	uint32_t* assignment; const uint32_t* list; const uint32_t* length; uint32_t* undecided;
+	uint32_t dim, k, kp;
+	float kd_split;
+};
+
+__device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
+{
+	const float dist = __builtin_sqrtf(sum);
+	return (c == 0 && dist != dist) ? 0ull : (((unsigned long long)__float_as_uint(dist) << 32) | c); /* see evaluate_pair */
+}
+
+/*
+ * A unit is 32, 64 or 128 listed points of a work-group of eight wavefronts: as many as leave every work-group something to do, since
+ * all of a unit's points share one reading of the centroids' operands (512 KB at k = 1024, d = 256).
+ *   1. The rows, moved, scaled and rounded as in the sweep, go to LDS as operands of the ranking.
+ *   2. The wavefronts share out the centroid tiles: operands from the caches to registers, then one chain of matrix instructions per
+ *      group of points. A centroid at or below the point's threshold is noted in the wavefront's list; NaN passes.
+ *   3. The lists are evaluated together, up to 64 pairs per wavefront: for a block of 16 dimensions four lanes per pair fetch 16
+ *      bytes each of point and centroid and square the differences (64 consecutive bytes per row: a lane of its own per row would
+ *      touch 64 lines per load), the squares go through LDS to the pair's lane, which adds them in order. The results merge into
+ *      the point's two smallest keys (distance bits << 32 | centroid, see evaluate_pair) in LDS.
+ * A wavefront whose list fills up (data that the thresholds tell nothing about) evaluates it on the spot, one lane per pair.
+ *
+ * counters[0] receives the number of points whose two smallest serial distances are closer than the three-product certificate.
+ */
+template <int KB>
+__global__ void __launch_bounds__(EXACT_THREADS, 4)
+listed_exact_kernel(const ExactArgs w)
+{
+	constexpr uint32_t DP = KB * KBLOCK;
+	extern __shared__ __attribute__((aligned(16))) float lds[];
+	f16x8* ops = (f16x8*)lds;                                   /* groups x KB x 64 lanes; the squares afterwards */
+	__shared__ unsigned long long best[EXACT_ROWS], second[EXACT_ROWS];
+	__shared__ float threshold[EXACT_ROWS], tau3[EXACT_ROWS];
+	__shared__ uint32_t point[EXACT_ROWS];
+	__shared__ uint32_t hits[EXACT_WAVES][EXACT_HITS];          /* row << 25 | centroid (supports: k < 2^25) */
+	__shared__ uint32_t wave_max[3][EXACT_WAVES];
+	constexpr uint32_t CENTROID = (1u << 25) - 1u;
+	const uint32_t count = w.length[0];
+	if (count == 0) return;
+	uint32_t groups = 1;
+	while (groups < EXACT_GROUPS && groups * TILE * gridDim.x < count) groups *= 2;
+	const uint32_t unit_rows = groups * TILE, units = (count + unit_rows - 1) / unit_rows;
+	if (blockIdx.x >= units) return;
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
+	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	const uint32_t col = lane & 31, h = lane >> 5;
+	const float scale = w.scale[0], unscale = w.scale[1];
+	const uint32_t tiles = w.kp / TILE;
+	const bool ragged = w.row_dim < DP;
+
+	CertCoeffs cert; /* of the three-product ranking: only what is counted depends on it */
+	{
+		uint32_t most[3] = { 0u, 0u, 0u };
+		for (uint32_t j = tid; j < w.k; j += EXACT_THREADS) {
+			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
+			most[1] = max(most[1], __float_as_uint(w.low[w.kp + j]));
+			most[2] = max(most[2], __float_as_uint(w.low[2 * w.kp + j]));
+		}
+#pragma unroll
+		for (int q = 0; q < 3; ++q) {
+			for (int off = WAVE / 2; off > 0; off >>= 1) most[q] = max(most[q], (uint32_t)__shfl_xor((int)most[q], off));
+			if (lane == 0) wave_max[q][wave] = most[q];
+		}
+		__syncthreads();
+#pragma unroll
+		for (int q = 0; q < 3; ++q) {
+			most[q] = 0;
+			for (uint32_t v = 0; v < EXACT_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
+		}
+		cert = cert_coeffs_split(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), __uint_as_float(most[2]) });
+	}
+
+	/* four coordinates of a row at its coordinate d, as they come from memory (d brought inside the row) ... */
+	auto source = [&](uint32_t row) -> const float* { return w.data + (size_t)point[row] * w.stride; };
+	auto request = [&](f32x4& v, const float* src, uint32_t d) {
+		typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+		v = *(const f32x4_any*)(src + min(d, w.row_dim - 4));
+	};
+	/* ... and in their places, zeros beyond the row */
+	auto place = [&](f32x4& v, uint32_t d) {
+		const int shift = (int)(d + 4) - (int)w.row_dim;
+		const f32x4 t = v;
+		v.x = shift <= 0 ? t.x : shift == 1 ? t.y : shift == 2 ? t.z : shift == 3 ? t.w : 0.0f;
+		v.y = shift <= 0 ? t.y : shift == 1 ? t.z : shift == 2 ? t.w : 0.0f;
+		v.z = shift <= 0 ? t.z : shift == 1 ? t.w : 0.0f;
+		v.w = shift <= 0 ? t.w : 0.0f;
+	};
+	uint32_t close_here = 0;
+	for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+		const uint32_t first = unit * unit_rows;
+		__syncthreads(); /* the previous unit has been written out */
+		if (tid < unit_rows) {
+			const uint32_t e = min(first + tid, count - 1);
+			point[tid] = w.list[2 * (size_t)e];
+			threshold[tid] = first + tid < count ? __uint_as_float(w.list[2 * (size_t)e + 1]) : -__builtin_inff(); /* rows beyond the list pass nothing */
+			best[tid] = ~0ull;
+			second[tid] = ~0ull;
+		}
+		__syncthreads();
+
+		{
+			uint32_t me = tid;
+			asm volatile("" : "+v"(me)); /* (what follows is not worth keeping in registers from one unit to the next) */
+			const uint32_t lanes = EXACT_THREADS / unit_rows; /* per row: 16, 8 or 4, a piece of four coordinates each */
+			const uint32_t row = me / lanes, sub = me % lanes;
+			const float* src = source(row);
+			f16x8* dst = ops + (row / TILE) * (KB * WAVE) + row % TILE;
+			float x2 = 0.0f, xmid2 = 0.0f;
+#pragma unroll 1
+			for (uint32_t f0 = sub; f0 < DP / 4; f0 += 4 * lanes) {
+				f32x4 v[4];
+#pragma unroll
+				for (int i = 0; i < 4; ++i) request(v[i], src, (f0 + i * lanes) * 4);
+#pragma unroll
+				for (int i = 0; i < 4; ++i) {
+					const uint32_t d = (f0 + i * lanes) * 4;
+					if (d >= DP) break;
+					if (ragged) place(v[i], d);
+					const f32x4 m = *(const f32x4*)(w.frame + d);
+					typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+					f16x4 half;
+#pragma unroll
+					for (int e = 0; e < 4; ++e) {
+						const float s = __builtin_fmaf(v[i][e], scale, -(m[e] * scale));
+						half[e] = (_Float16)s;
+						__bf16 hi, mid;
+						split_bf16(s, hi, mid);
+						x2 += s * s;
+						xmid2 += (float)mid * (float)mid;
+					}
+					/* block d / 16, half-wave (d % 16) / 8: four of its eight values */
+					*(f16x4*)((char*)(dst + (d / KBLOCK) * WAVE + (d % KBLOCK) / 8 * TILE) + (d % 8) * 2) = half;
+				}
+			}
+			for (uint32_t off = lanes / 2; off > 0; off >>= 1) { x2 += __shfl_xor(x2, off); xmid2 += __shfl_xor(xmid2, off); }
+			if (sub == 0) tau3[row] = cert_tau(w.kd_split, x2, xmid2, cert);
+		}
+		__syncthreads();
+
+		auto merge = [&](uint32_t row, unsigned long long key) {
+			const unsigned long long before = atomicMin(&best[row], key);
+			atomicMin(&second[row], before < key ? key : before);
+		};
+		uint32_t noted = 0; /* wave-uniform */
+		auto evaluate_alone = [&]() {
+#pragma clang fp contract(off)
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+			for (uint32_t i = lane; i < noted; i += WAVE) {
+				const uint32_t hit = hits[wave][i], row = hit >> 25, c = hit & CENTROID;
+				const float* src = source(row);
+				const float* mean = w.means + (size_t)c * DP;
+				float sum = 0.0f;
+#pragma unroll 1
+				for (uint32_t d = 0; d < w.dim; ++d) {
+					const float diff = src[d] - mean[d];
+					const float sq = diff * diff;
+					sum = sum + sq;
+				}
+				merge(row, exact_key(sum, c));
+			}
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+			noted = 0;
+		};
+		/* few tiles: the wavefronts share out the groups of points as well */
+		const uint32_t parts = tiles < EXACT_WAVES ? groups : 1;
+#pragma unroll 1
+		for (uint32_t t = wave / parts; t < tiles; t += EXACT_WAVES / parts) {
+			f32x16 start;
+#pragma unroll
+			for (int g = 0; g < 4; ++g) {
+				const f32x4 n0 = *(const f32x4*)(w.norms + t * NORM_TILE + 8 * g + 4 * h);
+				start[4 * g] = n0.x; start[4 * g + 1] = n0.y; start[4 * g + 2] = n0.z; start[4 * g + 3] = n0.w;
+			}
+			const f16x8* operand = w.packed + (size_t)t * (KB * WAVE) + lane;
+			f16x8 c[KB];
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb) c[kb] = operand[kb * WAVE];
+#pragma unroll 1
+			for (uint32_t g = wave % parts; g < groups; g += parts) {
+				f32x16 a = start;
+				const f16x8* x = ops + g * (KB * WAVE) + lane;
+#pragma unroll
+				for (int kb = 0; kb < KB; ++kb) a = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], x[kb * WAVE], a, 0, 0, 0);
+				const float limit = threshold[g * TILE + col];
+				float low = a[0]; /* NaN-propagating minimum */
+#pragma unroll
+				for (int r = 1; r < 16; ++r) low = __builtin_elementwise_minimum(low, a[r]);
+				const bool near = !(low > limit);
+				if (__builtin_amdgcn_ballot_w64(near) == 0) continue;
+				uint32_t passed = 0; /* bit r: result r */
+#pragma unroll
+				for (int r = 0; r < 16; ++r) passed |= !(a[r] > limit) ? 1u << r : 0u;
+				if (t + 1 == tiles) { /* rows that do not exist */
+#pragma unroll
+					for (int r = 0; r < 16; ++r)
+						if (t * TILE + 8 * (r / 4) + 4 * h + (r % 4) >= w.k) passed &= ~(1u << r);
+				}
+				for (;;) { /* the lanes' next results */
+					const unsigned long long mask = __builtin_amdgcn_ballot_w64(passed != 0);
+					if (mask == 0) break;
+					const uint32_t more = (uint32_t)__popcll(mask);
+					if (noted + more > EXACT_HITS) evaluate_alone();
+					if (passed) {
+						const uint32_t r = (uint32_t)__builtin_ctz(passed);
+						hits[wave][noted + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (g * TILE + col) << 25 | (t * TILE + 8 * (r / 4) + 4 * h + r % 4);
+						passed &= passed - 1;
+					}
+					noted += more;
+				}
+			}
+		}
+		if (lane == 0) wave_max[0][wave] = noted;
+		__syncthreads(); /* all pairs are listed, the operands are no longer needed */
+
+		{
+#pragma clang fp contract(off)
+			uint32_t total = 0;
+#pragma unroll
+			for (uint32_t v = 0; v < EXACT_WAVES; ++v) total += wave_max[0][v];
+			/* equal shares of the pairs, in groups of 16 */
+			const uint32_t share = ((total + 15) / 16 + EXACT_WAVES - 1) / EXACT_WAVES * 16;
+			const uint32_t end = min((wave + 1) * share, total);
+			float* squares = lds + wave * (WAVE * EXACT_PAIR_FLOATS);
+#pragma unroll 1
+			for (uint32_t p0 = wave * share; p0 < end; p0 += WAVE) {
+				/* this lane's pair (the last one again behind the end), and the four it fetches for */
+				uint32_t at = min(p0 + lane, end - 1), list = 0;
+				while (at >= wave_max[0][list]) at -= wave_max[0][list++];
+				const uint32_t hit = hits[list][at];
+				const uint32_t fours = min((end - p0 + 15) / 16, 4u);
+				const float* x[4]; const float* m[4];
+#pragma unroll
+				for (uint32_t g = 0; g < 4; ++g) {
+					const uint32_t other = (uint32_t)__shfl((int)hit, (int)(16 * g + lane / 4));
+					x[g] = source(other >> 25);
+					m[g] = w.means + (size_t)(other & CENTROID) * DP + lane % 4 * 4;
+				}
+				f32x4 xv[4], mv[4];
+#pragma unroll
+				for (int g = 0; g < 4; ++g) asm volatile("" : "=v"(xv[g]), "=v"(mv[g])); /* no values yet */
+				auto fetch = [&](uint32_t kb) {
+#pragma unroll
+					for (uint32_t g = 0; g < 4; ++g)
+						if (g < fours) {
+							request(xv[g], x[g], kb * KBLOCK + lane % 4 * 4);
+							mv[g] = *(const f32x4*)(m[g] + kb * KBLOCK);
+						}
+				};
+				fetch(0);
+				float sum = 0.0f;
+#pragma unroll 1
+				for (uint32_t kb = 0; kb < KB; ++kb) {
+#pragma unroll
+					for (uint32_t g = 0; g < 4; ++g)
+						if (g < fours) {
+							if (ragged && (kb + 1) * KBLOCK > w.row_dim) place(xv[g], kb * KBLOCK + lane % 4 * 4);
+							f32x4 sq;
+#pragma unroll
+							for (int e = 0; e < 4; ++e) {
+								const float diff = xv[g][e] - mv[g][e];
+								sq[e] = diff * diff;
+							}
+							*(f32x4*)(squares + (16 * g + lane / 4) * EXACT_PAIR_FLOATS + lane % 4 * 4) = sq;
+						}
+					if (kb + 1 < KB) fetch(kb + 1);
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+					__builtin_amdgcn_wave_barrier();
+					const float* mine = squares + lane * EXACT_PAIR_FLOATS;
+					if (lane < 16 * fours) {
+						f32x4 s[4];
+#pragma unroll
+						for (int q = 0; q < 4; ++q) s[q] = *(const f32x4*)(mine + 4 * q);
+#pragma unroll
+						for (int q = 0; q < 4; ++q)
+#pragma unroll
+							for (int e = 0; e < 4; ++e) sum = sum + s[q][e]; /* (zeros behind the row change nothing) */
+					}
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+					__builtin_amdgcn_wave_barrier();
+				}
+				if (p0 + lane < end) merge(hit >> 25, exact_key(sum, hit & CENTROID));
+			}
+		}
+		__syncthreads();
+		if (tid < unit_rows && first + tid < count) {
+			const unsigned long long key = best[tid], next = second[tid];
+			w.assignment[point[tid]] = key == ~0ull ? 0u : (uint32_t)key;
+			const float d1 = __uint_as_float((uint32_t)(key >> 32)), d2 = __uint_as_float((uint32_t)(next >> 32));
+			if (next != ~0ull && !((d2 * d2 - d1 * d1) / unscale > tau3[tid])) ++close_here;
+		}
+	}
+	if (wave < EXACT_ROWS / WAVE) {
+		for (int off = WAVE / 2; off > 0; off >>= 1) close_here += (uint32_t)__shfl_xor((int)close_here, off);
+		if (lane == 0 && close_here) atomicAdd(w.undecided, close_here);
+	}
+}
+
+template <int KB> constexpr uint32_t exact_dynamic_bytes() { return std::max<uint32_t>(EXACT_GROUPS * KB * WAVE * 16, EXACT_SQUARES * 4); }
+
+template <int KB>
+static int launch_listed_exact_kb(const AssignArgs& a, const ExactArgs& w, const DeviceInfo& dev)
+{
+	void (*kernel)(ExactArgs) = listed_exact_kernel<KB>;
+	const uint32_t lds = exact_dynamic_bytes<KB>();
+	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+	const uint32_t grid = std::min<uint32_t>((a.n + TILE - 1) / TILE, 2 * dev.compute_units);
+	KMX_LAUNCH_KERNEL(kernel, dim3(grid), dim3(EXACT_THREADS), lds, stream(), w);
+	KMX_LAUNCH_CHECK("listed_exact_kernel");
+	return KMX_OK;
+}
+
+} // namespace kmx
+
+#endif

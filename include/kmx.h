@@ -333,18 +333,20 @@ int kmx_last_kernel_ms(int which, float* ms);
 
 /*
  * Work-space bound (no counterpart in the reference: its kernels evaluate every point directly). With SoA points the
- * exact pass of the tuned assignment variants copies the rows of the points it has to re-evaluate into a compact
- * block in the library's work space; `bytes` bounds that block (default 1 GiB, at least 1024 rows are always kept).
- * Points beyond the bound are still re-evaluated, reading the SoA data directly (slower, same results).
+ * tuned assignment variants copy rows into a compact block in the library's work space: those of the points the exact pass
+ * has to re-evaluate, or, in the half-precision sweep, all of them on the way; `bytes` bounds that block (default 1 GiB, at
+ * least 1024 rows are always kept). Points beyond the bound are still re-evaluated, reading the SoA data directly (slower,
+ * same results); the half-precision sweep goes over the points in parts that fit.
  */
 int kmx_set_queued_rows_limit(size_t bytes);
 
 /*
- * The split-bf16 sweep of rows of 17 to 32 dimensions may run in two levels (no counterpart in the reference): one product
- * per dimension (hi * hi) for all points, a third of the matrix work, with a certificate wide enough for it; then the three
- * products for the points that level could not settle; then the exact pass as always. The results are the same at every
- * setting. mode 0: one level always; 1 (default): two levels where they pay (resident centroids, 97 centroids or more,
- * 2^18 points or more); 2: two levels wherever the kernels allow it (for tests and measurements on small inputs).
+ * Where KMX_ASSIGN_MFMA_BF16X3 takes one product per dimension for all points (no counterpart in the reference): rows of up to
+ * 256 dimensions in half precision, a third of the matrix work of the three bf16 products, followed by the exact pass for what
+ * its wider certificate leaves; wider rows, and the float ranking of double rows, with a second level of three products for
+ * those points in between. The results are the same at every setting. mode 0: three products for all points always; 1
+ * (default): one product where it pays (by size, see rank16_pays in csrc/assign_bf16.hip); 2: wherever the kernels allow it
+ * (for tests and measurements on small inputs).
  */
 int kmx_set_two_level_sweep(int mode);
 
@@ -386,7 +388,8 @@ int kmx_certificate_unmoved_threshold(uint32_t dim, float first, float tau, floa
  * block by block in ascending q, one instruction per block, with the instructions, operand layout and order of the
  * sweeps: kind 0 = v_mfma_f32_32x32x2_f32 (depth = 2 blocks), kind 1 = v_mfma_f32_32x32x16_bf16 (depth = 16 blocks; the
  * values of a and b must be exactly representable in bf16, the low 16 bits of their words are dropped), kind 2 =
- * v_mfma_f32_16x16x4_f32 (depth = 4 blocks; the 32 x 32 result as four tiles of 16 x 16).
+ * v_mfma_f32_16x16x4_f32 (depth = 4 blocks; the 32 x 32 result as four tiles of 16 x 16), kind 3 = v_mfma_f32_32x32x16_f16
+ * (depth = 16 blocks; the values of a and b must be exactly representable in half precision).
  * a: 32 x depth row-major; b: 32 x depth, the depth values of column j contiguous; c, d: 32 x 32 row-major. Device pointers.
  */
 int kmx_probe_matrix_chain(int kind, const float* a, const float* b, const float* c, float* d, uint32_t blocks);

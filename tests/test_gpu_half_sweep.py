@@ -1,0 +1,75 @@
+"""The half-precision ranking sweep and its exact pass (csrc/rank16.hip) against the serial oracle, bit for bit: every number of
+blocks of 16 dimensions, resident and streamed centroids, one to four groups of listed points per unit, lists that overflow,
+SoA points in one part and in several (-m gpu)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def flat(rows, layout):
+    return np.ascontiguousarray(rows if layout == 0 else rows.T).ravel()
+
+
+@pytest.mark.parametrize("kind", ["clustered", "grid", "same"])
+@pytest.mark.parametrize("dim,k,n", [
+    (5, 33, 1), (16, 1, 64), (17, 40, 65), (32, 1024, 3001), (33, 31, 500), (48, 700, 2049), (49, 65, 4100),
+    (64, 1300, 1025), (65, 64, 600), (96, 300, 515), (97, 33, 513), (128, 700, 1030), (129, 250, 1000),
+    (192, 32, 700), (193, 900, 600), (256, 330, 1025), (20, 5000, 1500), (40, 16, 70001),
+])
+def test_half_precision_sweep_matches_the_oracle(km, orc, gpu, dim, k, n, kind):
+    rng = np.random.default_rng(dim * 37 + k)
+    centres = rng.uniform(-3, 3, size=(k, dim)).astype(np.float32)
+    rows = (centres[rng.integers(0, k, n)] + rng.normal(size=(n, dim))).astype(np.float32)
+    means = (centres + rng.normal(size=(k, dim)) * 0.3).astype(np.float32)
+    if kind == "grid":       # many exact ties: duplicated centroids, points on bisectors
+        rows, means = np.round(rows * 0.5).astype(np.float32), np.round(means * 0.5).astype(np.float32)
+        means[k // 2:] = means[:k - k // 2]
+    elif kind == "same":     # every centroid within every threshold: the lists of pairs overflow
+        means[:] = means[0]
+    if n > 20:
+        rows[7, 3] = np.nan
+        rows[11, dim - 1] = np.inf
+        rows[13] *= np.float32(1e-30)
+        rows[17, 0] = 1e30
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    a = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for layout, layout_means, pad, limit in [(0, 0, 0, 1 << 30), (0, 1, 5, 1 << 30), (1, 0, 0, 1 << 30), (1, 1, 0, 1)]:
+            stride = dim + pad if layout == 0 else n
+            padded = rows
+            if pad:
+                padded = np.full((n, stride), np.float32(np.nan)); padded[:, :dim] = rows
+            d = km.DeviceBuffer(padded.nbytes); d.write(flat(padded, layout))
+            m = km.DeviceBuffer(4 * k * dim); m.write(flat(means, layout_means))
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            km.set_queued_rows_limit(limit)  # (1 byte: parts of 1024 points)
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, layout, stride, m, layout_means, km.layout_stride(layout_means, k, dim), a, dim, k, n)
+            km.sync()
+            got = a.read(np.uint32, n)
+            d.free(); m.free()
+            assert np.array_equal(got, want), "layouts %d/%d: %d mismatches" % (layout, layout_means, int((got != want).sum()))
+    finally:
+        km.set_two_level_sweep(1)
+        km.set_queued_rows_limit(1 << 30)
+    a.free()
+
+
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -18, 2.0 ** 10])
+def test_half_precision_products_accumulate_as_the_certificate_assumes(km, gpu, scale):
+    """At most one 2^-23 of the running magnitude per accumulated product; operands down to the smallest subnormal (2^-24) count."""
+    rng = np.random.default_rng(5)
+    depth = 256
+    a = (rng.normal(size=(32, depth)) * scale * np.exp2(rng.integers(-8, 3, (32, depth)))).astype(np.float16).astype(np.float32)
+    b = (rng.normal(size=(32, depth)) * scale * np.exp2(rng.integers(-8, 3, (32, depth)))).astype(np.float16).astype(np.float32)
+    a[:, 1::2] = -a[:, 0::2]; b[:, 1::2] = b[:, 0::2]          # cancelling pairs ...
+    a[:, 5] = 2.0 ** -24; b[:, 5] = 2.0 ** -24                 # ... next to the smallest numbers there are
+    c = (rng.normal(size=(32, 32)) * scale * scale).astype(np.float32)
+    d = km.probe_matrix_chain(3, a, b, c).astype(np.float64)
+    exact = c.astype(np.float64) + a.astype(np.float64) @ b.astype(np.float64).T
+    magnitude = np.abs(c).astype(np.float64) + np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+    assert (np.abs(d - exact) <= (depth + 1) * 2.0 ** -23 * magnitude).all()
+    only = np.zeros((32, 16), np.float32); only[:, 3] = 2.0 ** -24
+    alone = km.probe_matrix_chain(3, only, np.full((32, 16), 1024.0, np.float32), np.zeros((32, 32), np.float32))
+    assert (alone == np.float32(2.0 ** -14)).all()             # subnormal operands are not flushed
