@@ -50,6 +50,18 @@ static bool rank16_pays(const AssignArgs& a)
 	return a.k > 32 && (double)a.n * a.k * a.dim >= 5e8;
 }
 
+static bool takes_rank16(const AssignArgs& a, uint32_t lds_budget)
+{
+	const int mode = two_level_mode(); /* kmx_set_two_level_sweep: 0 never, 1 where it pays, 2 wherever the kernels allow it */
+	return a.dim <= 256 && !a.ranking_only && a.two_level && mode != 0 && (mode == 2 || rank16_pays(a)) && rank16_supports(a, lds_budget);
+}
+
+bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
+{
+	return a.layout == KMX_SOA && bf16_supports(a, dev) && takes_rank16(a, lds_budget_of(exec, dev)) &&
+	       (size_t)a.n * round_up(a.dim, 8) * sizeof(float) <= queued_rows_limit();
+}
+
 /* supported blocks of 16 dimensions per row */
 static uint32_t pick_kb(uint32_t dim)
 {
@@ -209,9 +221,7 @@ int launch_screen_bf16(const float* rows, const Workspace* ws, const uint32_t* r
 int launch_assign_bf16(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	if (args.dim > 256) return launch_assign_wide(args, exec, ws, dev);
-	const int mode = two_level_mode(); /* kmx_set_two_level_sweep: 0 never, 1 where it pays, 2 wherever the kernels allow it */
-	if (!args.ranking_only && args.two_level && mode != 0 && (mode == 2 || rank16_pays(args)) && rank16_supports(args, lds_budget_of(exec, dev)))
-		return launch_assign_rank16(args, exec, ws, dev);
+	if (takes_rank16(args, lds_budget_of(exec, dev))) return launch_assign_rank16(args, exec, ws, dev);
 	AssignArgs a = args;
 	/* wide rows and many centroids: a second sweep screens the queued points (narrow rows fit the registers of the
 	 * lane-per-centroid kernels, which then need fewer launches); so do the packed rows, whose sweep queues more points

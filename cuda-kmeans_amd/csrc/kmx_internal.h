@@ -113,6 +113,11 @@ __host__ __device__ __forceinline__ size_t elem(size_t stride, size_t idx, size_
 	return LAYOUT == KMX_AOS ? idx * stride + dim : dim * stride + idx;
 }
 
+/* AoS copy of SoA points in the work space */
+struct AosRows {
+	const float* data; size_t stride;
+};
+
 /* Argument bundle of one assignment call after validation. */
 struct AssignArgs {
 	const float* data; int layout; size_t stride;
@@ -136,6 +141,8 @@ struct AssignArgs {
 	bool two_level = true;
 	/* the single-pass fused kernel: write the result of every point to `assignment`, not only those of the exact pass */
 	bool emit_assignment = false;
+	/* SoA points: filled in by a sweep that wrote all rows as AoS on the way (left alone by the others) */
+	AosRows* rows_out = nullptr;
 };
 
 struct UpdateArgs {
@@ -177,6 +184,7 @@ bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_bf16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* rank16.hip: one half-precision product per dimension for all points, the serial result for what that leaves */
 bool rank16_supports(const AssignArgs& a, uint32_t lds_budget);
+bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST would write a.rows_out */
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */
 bool wide_supports(const AssignArgs& a, const DeviceInfo& dev);
@@ -211,6 +219,9 @@ int launch_reduce_partials(const UpdateArgs& u, const float* partial, const uint
 int noalloc_workspace(Workspace** ws);
 bool recording_graph(); /* between kmx_graph_begin and kmx_graph_end */
 int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
+/* whether launch_update would copy the SoA points of u into AoS rows first, and that copy: ws->rows_copy, rows of dim floats */
+bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev);
+int launch_rows_from_soa(const float* data, size_t stride, uint32_t dim, uint32_t n, Workspace* ws, const DeviceInfo& dev);
 int launch_divide_means(const UpdateArgs& u);
 int clear_update_outputs(const UpdateArgs& u); /* means (replica 0) and cluster sizes := 0 in one launch */
 

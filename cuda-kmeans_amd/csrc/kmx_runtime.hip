@@ -263,9 +263,35 @@ static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_
 	return launch_reduce_partials(u, ws->partials, partial_counts, exec->block_count);
 }
 
+/*
+ * Assignment and update of SoA points. The update reads whole rows and copies the points for that (27 us at N = 250k, d = 50); so the
+ * copy comes from the half-precision sweep where that writes one anyway, and otherwise first, for the assignment to read as well.
+ */
+static int launch_two_passes_soa(AssignArgs a, UpdateArgs u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	AosRows rows = { nullptr, 0 };
+	if (update_wants_rows(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev)) {
+		if (sweep_writes_rows(a, exec, dev)) a.rows_out = &rows;
+		else {
+			const int rc = launch_rows_from_soa(u.data, u.stride, u.dim, u.n, ws, dev);
+			if (rc) return rc;
+			rows = AosRows{ ws->rows_copy, u.dim };
+			a.data = rows.data; a.stride = rows.stride; a.layout = KMX_AOS;
+		}
+	}
+	const int rc = dispatch_assign(KMX_ASSIGN_BEST, a, exec, ws, dev, nullptr);
+	if (rc) return rc;
+	if (rows.data) { u.data = rows.data; u.stride = rows.stride; u.layout = KMX_AOS; }
+	return launch_update(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev);
+}
+
 } // namespace kmx
 
 extern "C" {
+
+/* kmx_assign_f32 (KMX_ASSIGN_BEST) and kmx_update_f32 (KMX_UPDATE_ATOMIC_SHM) in one */
+static int two_passes(const float* data, int layout, size_t stride, const float* means_in, float* means_out, int layout_means, size_t stride_means,
+                      uint32_t* assignment, uint32_t* cluster_sizes, uint32_t dim, uint32_t k, uint32_t n, kmx_exec_params* exec);
 
 const char* kmx_last_error(void) { return g_error; }
 
@@ -487,6 +513,8 @@ int kmx_reserve_f32(int assign_variant, int update_variant, int layout, int layo
 	g_sizing = true;
 	int rc = kmx_assign_f32(assign_variant, points, layout, stride, points, layout_means, stride_means, nullptr, words, dim, k, n, &exec);
 	if (rc == KMX_OK) rc = kmx_update_f32(update_variant, points, layout, stride, words, points, layout_means, stride_means, words, dim, k, n, &exec);
+	/* an iteration on SoA points may run on an AoS copy of them */
+	if (rc == KMX_OK && layout == KMX_SOA) rc = two_passes(points, layout, stride, points, points, layout_means, stride_means, words, words, dim, k, n, &exec);
 	if (rc == KMX_OK) {
 		Workspace* ws = nullptr;
 		rc = workspace(&ws);
@@ -664,11 +692,7 @@ int kmx_fused_f32(int variant,
 		UpdateArgs u{ data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
 		return launch_divide_means(u);
 	}
-	/* argument checks of the two halves apply unchanged (their messages name the half that objects) */
-	rc = kmx_assign_f32(KMX_ASSIGN_BEST, data, layout, stride, means_in, layout_means, stride_means, nullptr, ws->fused_assignment, dim, k, n, exec);
-	if (rc) return rc;
-	return kmx_update_f32(KMX_UPDATE_ATOMIC_SHM, data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means,
-	                      cluster_sizes, dim, k, n, exec);
+	return two_passes(data, layout, stride, means_in, means_out, layout_means, stride_means, ws->fused_assignment, cluster_sizes, dim, k, n, exec);
 }
 
 static int g_last_iteration_passes = 0;
@@ -724,7 +748,27 @@ int kmx_iteration_f32(const float* data, int layout, size_t stride,
 		const UpdateArgs u{ data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
 		return launch_iteration_small(small, u, exec, ws, *dev);
 	}
-	rc = kmx_assign_f32(KMX_ASSIGN_BEST, data, layout, stride, means_in, layout_means, stride_means, nullptr, assignment, dim, k, n, exec);
+	return two_passes(data, layout, stride, means_in, means_out, layout_means, stride_means, assignment, cluster_sizes, dim, k, n, exec);
+}
+
+static int two_passes(const float* data, int layout, size_t stride, const float* means_in, float* means_out, int layout_means, size_t stride_means,
+                      uint32_t* assignment, uint32_t* cluster_sizes, uint32_t dim, uint32_t k, uint32_t n, kmx_exec_params* exec)
+{
+	if (layout == KMX_SOA && n > 0 && dim > 0 && k > 0 && data) {
+		int rc = check_layout("kmx_assign_f32", "data", layout, stride, n, dim);
+		if (rc) return rc;
+		if ((rc = check_layout("kmx_assign_f32", "means", layout_means, stride_means, k, dim))) return rc;
+		if (exec->privatized_copies == 0) exec->privatized_copies = 1;
+		const DeviceInfo* dev = nullptr;
+		if ((rc = device_info(&dev))) return rc;
+		Workspace* ws = nullptr;
+		if ((rc = workspace(&ws))) return rc;
+		const AssignArgs a{ data, layout, stride, means_in, layout_means, stride_means, assignment, dim, k, n };
+		const UpdateArgs u{ data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
+		return launch_two_passes_soa(a, u, exec, ws, *dev);
+	}
+	/* argument checks of the two halves apply unchanged (their messages name the half that objects) */
+	const int rc = kmx_assign_f32(KMX_ASSIGN_BEST, data, layout, stride, means_in, layout_means, stride_means, nullptr, assignment, dim, k, n, exec);
 	if (rc) return rc;
 	return kmx_update_f32(KMX_UPDATE_ATOMIC_SHM, data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n, exec);
 }

@@ -220,6 +220,7 @@ int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 		if (first == 0 && (rc = profile_end(0))) return rc;
 		if ((rc = launch_listed_exact(p, ws, dev))) return rc;
 	}
+	if (a.rows_out && a.layout == KMX_SOA && part == a.n) *a.rows_out = AosRows{ ws->queued_rows, round_up(a.dim, 8) };
 	return KMX_OK;
 }
 

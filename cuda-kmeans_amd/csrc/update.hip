@@ -1260,6 +1260,25 @@ int noalloc_workspace(Workspace** ws)
 
 int clear_update_outputs(const UpdateArgs& u) { return clear_outputs(u); }
 
+bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev)
+{
+	/* (the fixed work space has no room for a copy of the points: SoA points then stay with the element-wise kernels) */
+	return !ws->fixed && u.layout == KMX_SOA && (variant & ~KMX_UPDATE_EMULATED_ATOMICS) == KMX_UPDATE_ATOMIC_SHM && u.n > 0 && u.dim >= 8 &&
+	       (size_t)u.n * u.dim * sizeof(float) <= ROWS_COPY_MAX_BYTES &&
+	       !(variant == KMX_UPDATE_ATOMIC_SHM && small_update_fits<float>(u.dim, u.k, u.n, lds_budget_of(exec, dev), dev));
+}
+
+int launch_rows_from_soa(const float* data, size_t stride, uint32_t dim, uint32_t n, Workspace* ws, const DeviceInfo& dev)
+{
+	int rc = reserve_rows_copy(ws, (size_t)n * dim);
+	if (rc) return rc;
+	const size_t tiles = (size_t)((n + 63) / 64) * ((dim + 31) / 32);
+	KMX_LAUNCH_KERNEL(rows_from_soa_kernel, dim3((uint32_t)std::min<size_t>(tiles, (size_t)dev.compute_units * 32)), dim3(256), 0, stream(),
+	                   data, stride, ws->rows_copy, dim, n);
+	KMX_LAUNCH_CHECK("rows_from_soa_kernel");
+	return KMX_OK;
+}
+
 int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	if (variant == KMX_UPDATE_SERIAL_ORDER)
@@ -1272,15 +1291,9 @@ int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Works
 		                                u.dim, u.k, u.n, u.divide, &exec->block_count, dev);
 		return rc ? rc : profile_end(1);
 	}
-	/* (the fixed work space has no room for a copy of the points: SoA points then stay with the element-wise kernels) */
-	if (!ws->fixed && u.layout == KMX_SOA && (variant & ~KMX_UPDATE_EMULATED_ATOMICS) == KMX_UPDATE_ATOMIC_SHM && u.n > 0 && u.dim >= 8 &&
-	    (size_t)u.n * u.dim * sizeof(float) <= ROWS_COPY_MAX_BYTES) {
-		int rc = reserve_rows_copy(ws, (size_t)u.n * u.dim);
+	if (update_wants_rows(variant, u, exec, ws, dev)) {
+		const int rc = launch_rows_from_soa(u.data, u.stride, u.dim, u.n, ws, dev);
 		if (rc) return rc;
-		const size_t tiles = (size_t)((u.n + 63) / 64) * ((u.dim + 31) / 32);
-		KMX_LAUNCH_KERNEL(rows_from_soa_kernel, dim3((uint32_t)std::min<size_t>(tiles, (size_t)dev.compute_units * 32)), dim3(256), 0, stream(),
-		                   u.data, u.stride, ws->rows_copy, u.dim, u.n);
-		KMX_LAUNCH_CHECK("rows_from_soa_kernel");
 		UpdateArgs rows = u;
 		rows.data = ws->rows_copy; rows.layout = KMX_AOS; rows.stride = u.dim;
 		return u.layout_means == KMX_AOS ? launch_update_t<KMX_AOS, KMX_AOS>(variant, rows, exec, ws, dev)

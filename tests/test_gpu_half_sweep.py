@@ -73,3 +73,29 @@ def test_half_precision_products_accumulate_as_the_certificate_assumes(km, gpu, 
     only = np.zeros((32, 16), np.float32); only[:, 3] = 2.0 ** -24
     alone = km.probe_matrix_chain(3, only, np.full((32, 16), 1024.0, np.float32), np.zeros((32, 32), np.float32))
     assert (alone == np.float32(2.0 ** -14)).all()             # subnormal operands are not flushed
+
+
+@pytest.mark.parametrize("dim,k,n,mode", [(8, 130, 40001, 1), (50, 300, 70007, 1), (50, 60, 40003, 1), (9, 40, 33000, 1), (256, 129, 33001, 1), (300, 20, 33003, 1), (50, 300, 40000, 0)])
+def test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, mode):
+    """The assignment's copy of the rows, or the one made ahead of it, is what the update adds up."""
+    rng = np.random.default_rng(dim + k)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    means = np.ascontiguousarray(rows[rng.choice(n, k, replace=False)])
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, 1))
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 1))
+    o = km.DeviceBuffer(means.nbytes); a = km.DeviceBuffer(4 * n); s = km.DeviceBuffer(4 * k)
+    km.set_two_level_sweep(mode)
+    try:
+        km.iteration(d, 1, n, m, o, 1, k, a, s, dim, k, n)
+        km.sync()
+    finally:
+        km.set_two_level_sweep(1)
+    assert np.array_equal(a.read(np.uint32, n), want)
+    counts = np.bincount(want, minlength=k)
+    assert np.array_equal(s.read(np.uint32, k), counts)
+    sums = np.zeros((k, dim)); np.add.at(sums, want, rows.astype(np.float64))
+    got = o.read(np.float32, k * dim).reshape(dim, k).T
+    assert np.allclose(got, sums / counts[:, None], rtol=1e-5, atol=1e-6)
+    for b in (d, m, o, a, s):
+        b.free()
