@@ -15,12 +15,13 @@
  * reference's serial run. The price is the length of the longest chain: a cluster of m members is m dependent
  * additions, whatever the machine.
  *
- * Kernels: ordered_histogram_kernel, ordered_range_sums_kernel, ordered_offsets_kernel, ordered_starts_kernel,
- * ordered_scatter_kernel, ordered_sum_kernel.
+ * Kernels: ordered_histogram_kernel, ordered_offsets_kernel, ordered_starts_kernel, ordered_scatter_kernel,
+ * ordered_staged_sum_kernel / ordered_sum_kernel.
  */
 #include "kmx_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace kmx {
 
@@ -59,72 +60,89 @@ ordered_histogram_kernel(const uint32_t* __restrict__ assignment, uint32_t* __re
 	}
 }
 
-/* range_sums[r][c] = sum of hist[chunk][c] over the chunks of range r (ranges of `per` chunks): first half of the scan
- * along the chunks, which for few clusters has too few columns to fill the machine with one lane per column */
-__global__ void __launch_bounds__(256)
-ordered_range_sums_kernel(const uint32_t* __restrict__ hist, uint32_t* __restrict__ range_sums, uint32_t k, uint32_t chunks, uint32_t ranges, uint32_t per)
+/*
+ * hist[chunk][c] := number of members of cluster c in the chunks before `chunk` (exclusive scan along the chunks, in place), and the
+ * sizes. A work-group takes 16 clusters (64 bytes of every row), 64 lanes share out the rows of a cluster: each adds its share,
+ * the shares are scanned in LDS, each walks its share again (from L2). Loads go out SCAN_BATCH at a time: what bounds it is their
+ * latency (one lane per cluster and 128 rows, one load after the other, in two launches: 52 us at 2048 chunks, k = 1024).
+ */
+constexpr uint32_t SCAN_COLUMNS = 16, SCAN_SHARES = 64, SCAN_BATCH = 16;
+
+__global__ void __launch_bounds__(SCAN_COLUMNS * SCAN_SHARES)
+ordered_offsets_kernel(uint32_t* __restrict__ hist, uint32_t* __restrict__ sizes, uint32_t k, uint32_t chunks)
 {
-	const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-	if (e >= (size_t)ranges * k) return;
-	const uint32_t c = (uint32_t)(e % k), r = (uint32_t)(e / k);
-	const uint32_t c0 = min(chunks, r * per), c1 = min(chunks, c0 + per);
+	__shared__ uint32_t share_sum[SCAN_SHARES][SCAN_COLUMNS];
+	const uint32_t column = threadIdx.x % SCAN_COLUMNS, share = threadIdx.x / SCAN_COLUMNS;
+	const uint32_t c = min(blockIdx.x * SCAN_COLUMNS + column, k - 1);
+	const bool mine = blockIdx.x * SCAN_COLUMNS + column < k;
+	const uint32_t per = (chunks + SCAN_SHARES - 1) / SCAN_SHARES;
+	const uint32_t c0 = min(chunks, share * per), c1 = min(chunks, c0 + per);
 	uint32_t sum = 0;
-	for (uint32_t chunk = c0; chunk < c1; ++chunk) sum += hist[(size_t)chunk * k + c];
-	range_sums[e] = sum;
-}
-
-/* second half: hist[chunk][c] := number of members of cluster c in the chunks before `chunk` (exclusive scan along the
- * chunks, in place); the lane of the last range publishes the cluster's size */
-__global__ void __launch_bounds__(256)
-ordered_offsets_kernel(uint32_t* __restrict__ hist, const uint32_t* __restrict__ range_sums, uint32_t* __restrict__ sizes,
-                       uint32_t k, uint32_t chunks, uint32_t ranges, uint32_t per)
-{
-	const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-	if (e >= (size_t)ranges * k) return;
-	const uint32_t c = (uint32_t)(e % k), r = (uint32_t)(e / k);
-	uint32_t running = 0;
-	for (uint32_t q = 0; q < r; ++q) running += range_sums[(size_t)q * k + c];
-	const uint32_t c0 = min(chunks, r * per), c1 = min(chunks, c0 + per);
-	for (uint32_t chunk = c0; chunk < c1; ++chunk) {
-		const uint32_t members = hist[(size_t)chunk * k + c];
-		hist[(size_t)chunk * k + c] = running;
-		running += members;
+	for (uint32_t base = c0; base < c1; base += SCAN_BATCH) {
+		uint32_t v[SCAN_BATCH];
+#pragma unroll
+		for (uint32_t u = 0; u < SCAN_BATCH; ++u) v[u] = hist[(size_t)min(base + u, c1 - 1) * k + c];
+#pragma unroll
+		for (uint32_t u = 0; u < SCAN_BATCH; ++u) sum += base + u < c1 ? v[u] : 0u;
 	}
-	if (r + 1 == ranges) sizes[c] = running;
+	uint32_t upto = sum; /* of this share and those before it */
+	share_sum[share][column] = sum;
+#pragma unroll
+	for (uint32_t off = 1; off < SCAN_SHARES; off <<= 1) {
+		__syncthreads();
+		const uint32_t before = share >= off ? share_sum[share - off][column] : 0u;
+		__syncthreads();
+		upto += before;
+		share_sum[share][column] = upto;
+	}
+	if (mine && share == SCAN_SHARES - 1) sizes[c] = upto;
+	uint32_t running = upto - sum;
+	for (uint32_t base = c0; base < c1; base += SCAN_BATCH) {
+		uint32_t v[SCAN_BATCH];
+#pragma unroll
+		for (uint32_t u = 0; u < SCAN_BATCH; ++u) v[u] = hist[(size_t)min(base + u, c1 - 1) * k + c];
+#pragma unroll
+		for (uint32_t u = 0; u < SCAN_BATCH; ++u) {
+			if (base + u < c1 && mine) hist[(size_t)(base + u) * k + c] = running;
+			running += base + u < c1 ? v[u] : 0u;
+		}
+	}
 }
 
-/* starts[c] = sizes[0] + ... + sizes[c - 1]: one work-group; every lane scans a contiguous piece, the pieces meet in LDS */
+/* starts[c] = sizes[0] + ... + sizes[c - 1]: one work-group, 1024 clusters per step, wavefront sums meet in LDS */
 __global__ void __launch_bounds__(1024)
 ordered_starts_kernel(const uint32_t* __restrict__ sizes, uint32_t* __restrict__ starts, uint32_t k)
 {
-	__shared__ uint32_t piece_sum[1024];
-	const uint32_t per = (k + 1023) / 1024;
-	const uint32_t c0 = min(k, threadIdx.x * per), c1 = min(k, c0 + per);
-	uint32_t sum = 0;
-	for (uint32_t c = c0; c < c1; ++c) sum += sizes[c];
-	piece_sum[threadIdx.x] = sum;
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		uint32_t running = 0;
-		for (uint32_t t = 0; t < 1024; ++t) {
-			const uint32_t s = piece_sum[t];
-			piece_sum[t] = running;
-			running += s;
+	__shared__ uint32_t wave_sum[2][16];
+	const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+	uint32_t running = 0, buffer = 0;
+	for (uint32_t base = 0; base < k; base += 1024, buffer ^= 1) {
+		const uint32_t c = base + threadIdx.x;
+		const uint32_t members = c < k ? sizes[c] : 0u;
+		uint32_t upto = members; /* inclusive within the wavefront */
+#pragma unroll
+		for (uint32_t off = 1; off < WAVE; off <<= 1) {
+			const uint32_t below = (uint32_t)__shfl_up((int)upto, off);
+			if (lane >= off) upto += below;
 		}
-	}
-	__syncthreads();
-	uint32_t running = piece_sum[threadIdx.x];
-	for (uint32_t c = c0; c < c1; ++c) {
-		starts[c] = running;
-		running += sizes[c];
+		if (lane == WAVE - 1) wave_sum[buffer][wave] = upto;
+		__syncthreads(); /* (two buffers: the next step writes the other one) */
+		uint32_t before = running;
+		for (uint32_t v = 0; v < 16; ++v) {
+			const uint32_t sum = wave_sum[buffer][v];
+			before += v < wave ? sum : 0u;
+			running += sum;
+		}
+		if (c < k) starts[c] = before + upto - members;
 	}
 }
 
 /*
  * sorted[starts[c] + members of c in earlier chunks + rank inside the chunk] = point number. One wavefront per chunk
  * walks its points in ascending order, 64 per step. Inside a step the lanes that share a cluster are ranked by lane
- * number: the lanes still waiting read the cluster of the first of them, a ballot names all lanes with that cluster,
- * a lane's rank is the number of those below it. The cluster's counter then moves on by the size of the group (written
+ * number: one ballot per bit of the cluster number leaves every lane the mask of the lanes with its cluster, a lane's rank is
+ * the number of those below it (naming the clusters of a step one after the other took up to 64 ballots, 48 instead of 32 us at
+ * N = 2M, k = 1024). The cluster's counter then moves on by the size of the group (written
  * by its last lane, after every lane of the group has read it: one wavefront, in program order). The order inside a
  * cluster is therefore the point order, which no returning atomic would promise.
  */
@@ -136,31 +154,41 @@ ordered_scatter_kernel(const uint32_t* __restrict__ assignment, uint32_t* __rest
 	extern __shared__ uint32_t counters[];
 	const uint32_t lane = threadIdx.x;
 	uint32_t* row = hist + (size_t)blockIdx.x * k;
-	for (uint32_t c = lane; c < k; c += WAVE) {
-		const uint32_t first = starts[c] + row[c];
-		if (IN_LDS) counters[c] = first;
-		else __hip_atomic_store(&row[c], first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	if (IN_LDS) {
+		constexpr uint32_t BATCH = 8; /* loads in flight (one pair of loads at a time was a third of the kernel) */
+		for (uint32_t c0 = lane; c0 < k; c0 += BATCH * WAVE) {
+			uint32_t first[BATCH];
+#pragma unroll
+			for (uint32_t u = 0; u < BATCH; ++u) {
+				const uint32_t c = min(c0 + u * WAVE, k - 1);
+				first[u] = starts[c] + row[c];
+			}
+#pragma unroll
+			for (uint32_t u = 0; u < BATCH; ++u)
+				if (c0 + u * WAVE < k) counters[c0 + u * WAVE] = first[u];
+		}
 	}
+	else
+		for (uint32_t c = lane; c < k; c += WAVE) __hip_atomic_store(&row[c], starts[c] + row[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	if (!IN_LDS) __threadfence();
 	__syncthreads();
 	uint32_t* next = IN_LDS ? counters : row;
 	const unsigned long long below = (1ull << lane) - 1ull;
+	const uint32_t bits = 32 - (uint32_t)__builtin_clz(k - 1 | 1u);
 	const uint32_t begin = blockIdx.x * chunk_points;
 	const uint32_t end = min(n, begin + chunk_points);
+	uint32_t cluster = begin + lane < end ? assignment[begin + lane] : 0xFFFFFFFFu;
 	for (uint32_t base = begin; base < end; base += WAVE) {
-		const uint32_t i = base + lane;
-		const uint32_t c = i < end ? assignment[i] : 0xFFFFFFFFu;
-		bool waiting = c < k;
-		uint32_t rank = 0, group = 0;
-		while (waiting) {
-			const uint32_t first = __builtin_amdgcn_readfirstlane(c); /* cluster of the first lane still waiting */
-			const unsigned long long same = __ballot(c == first);     /* the waiting lanes with that cluster: all lanes that have it */
-			if (c == first) {
-				rank = (uint32_t)__popcll(same & below);
-				group = (uint32_t)__popcll(same);
-				waiting = false;
-			}
+		const uint32_t i = base + lane, c = cluster;
+		if (base + WAVE < end) cluster = i + WAVE < end ? assignment[i + WAVE] : 0xFFFFFFFFu; /* of the next step */
+		/* the lanes with this lane's cluster: those that agree in every bit of it */
+		unsigned long long same = __ballot(c < k);
+		for (uint32_t bit = 0; bit < bits; ++bit) {
+			const bool set = (c >> bit) & 1u;
+			const unsigned long long with = __ballot(set);
+			same &= set ? with : ~with;
 		}
+		const uint32_t rank = (uint32_t)__popcll(same & below), group = (uint32_t)__popcll(same);
 		if (c < k) {
 			/* counters in global memory: read and written past the vector cache, and fenced below, so that the lanes of the
 			 * next step see what this step wrote */
@@ -225,15 +253,120 @@ ordered_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __
 		means[elem<LM>(stride_means, c, d + i)] = !divide ? sum.v[i] : (members ? sum.v[i] / (F)members : (F)0);
 }
 
+/*
+ * The same for clusters of many members: a work-group per cluster and block of up to 32 coordinates. All eight wavefronts fetch the
+ * members' pieces (16 bytes each, STAGED_PIECES per lane) of the next few hundred rows into registers while the first one adds
+ * the last fetch from LDS, a lane per coordinate, four members per LDS read. The chain then runs at the latency of an addition and an LDS read
+ * instead of a trip to memory per 32 rows; what bounds it is that chain for the largest cluster, or the gathering of the rows
+ * (N = 2M, d = 32, k = 1024: 389 -> 125 us, 2.1 TB/s; N = 4M, d = 16, k = 16, all of it 33 -> 7.5 ms).
+ * ELEMENTS: SoA points, rows shorter than a piece: single coordinates, consecutive lanes take consecutive members.
+ */
+constexpr uint32_t STAGED_THREADS = 512, STAGED_PIECES = 8;
+
+template <typename F, int LD, int LM, bool ELEMENTS>
+__global__ void __launch_bounds__(STAGED_THREADS, 4)
+ordered_staged_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ starts,
+                          const uint32_t* __restrict__ sizes, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t blocks, uint32_t block_dims, uint32_t divide)
+{
+	constexpr uint32_t PIECE = ELEMENTS ? 1 : 16 / sizeof(F), QUAD = 16 / sizeof(F); /* (QUAD: members per LDS read) */
+	typedef F piece_any __attribute__((ext_vector_type(PIECE), aligned(sizeof(F))));
+	typedef F quad_t __attribute__((ext_vector_type(QUAD)));
+	extern __shared__ __attribute__((aligned(16))) char staged_lds[];
+	F* columns = (F*)staged_lds;
+	const uint32_t c = blockIdx.x / blocks, block = blockIdx.x % blocks;
+	const uint32_t d0 = block * block_dims, width = min(block_dims, dim - d0); /* (ELEMENTS = false: width >= PIECE, see the launcher) */
+	const uint32_t members = sizes[c], begin = starts[c];
+	const uint32_t tid = threadIdx.x;
+	const uint32_t pieces = (width + PIECE - 1) / PIECE;
+	const uint32_t step = STAGED_THREADS * STAGED_PIECES / pieces / QUAD * QUAD; /* members per fetch */
+	const uint32_t column = step + QUAD;                                         /* (the padding spreads the columns over the banks) */
+	/* piece q of a fetch: its member there and its coordinate; the last piece ends with the block */
+	uint32_t member_of[STAGED_PIECES], at_of[STAGED_PIECES];
+#pragma unroll
+	for (uint32_t i = 0; i < STAGED_PIECES; ++i) {
+		const uint32_t q = tid + i * STAGED_THREADS;
+		member_of[i] = ELEMENTS ? q % step : q / pieces;
+		const uint32_t piece = ELEMENTS ? q / step : q % pieces;
+		at_of[i] = min(piece * PIECE, width - PIECE);
+		if (member_of[i] >= step || piece >= pieces) member_of[i] = 0xFFFFFFFFu; /* beyond the fetch */
+	}
+	uint32_t point[STAGED_PIECES];
+	piece_any v[STAGED_PIECES];
+	auto name = [&](uint32_t first) { /* the points of the fetch that starts with member `first` */
+#pragma unroll
+		for (uint32_t i = 0; i < STAGED_PIECES; ++i)
+			if (member_of[i] < step && first + member_of[i] < members) point[i] = sorted[begin + first + member_of[i]];
+	};
+	auto fetch = [&](uint32_t first) {
+#pragma unroll
+		for (uint32_t i = 0; i < STAGED_PIECES; ++i)
+			if (member_of[i] < step && first + member_of[i] < members) v[i] = *(const piece_any*)(data + elem<LD>(stride, point[i], d0 + at_of[i]));
+	};
+	F sum = (F)0;
+	if (members) {
+		name(0);
+		fetch(0);
+		if (step < members) name(step);
+	}
+	for (uint32_t first = 0; first < members; first += step) {
+		__syncthreads(); /* the members in LDS have been added */
+#pragma unroll
+		for (uint32_t i = 0; i < STAGED_PIECES; ++i)
+			if (member_of[i] < step && first + member_of[i] < members) {
+#pragma unroll
+				for (uint32_t e = 0; e < PIECE; ++e) columns[(at_of[i] + e) * column + member_of[i]] = v[i][e];
+			}
+		__syncthreads();
+		if (first + step < members) {
+			fetch(first + step);
+			if (first + 2 * step < members) name(first + 2 * step);
+		}
+		if (tid < width) {
+			const uint32_t here = min(step, members - first);
+			const F* mine = columns + tid * column;
+			constexpr uint32_t READS = 4;
+			uint32_t r = 0;
+			for (; r + READS * QUAD <= here; r += READS * QUAD) {
+				quad_t x[READS];
+#pragma unroll
+				for (uint32_t u = 0; u < READS; ++u) x[u] = *(const quad_t*)(mine + r + u * QUAD);
+#pragma unroll
+				for (uint32_t u = 0; u < READS; ++u)
+#pragma unroll
+					for (uint32_t e = 0; e < QUAD; ++e) sum = sum + x[u][e];
+			}
+			for (; r < here; ++r) sum = sum + mine[r];
+		}
+	}
+	if (tid < width) means[elem<LM>(stride_means, c, d0 + tid)] = !divide ? sum : (members ? sum / (F)members : (F)0);
+}
+
 /* Work-groups of one wavefront: what bounds this kernel is the number of cache lines a compute unit keeps in flight, so
  * the chains are spread over as many compute units as there are wavefronts (measured at N = 2M, d = 32, k = 1024: 32
  * work-groups of four wavefronts with 16-byte pieces 0.85 ms). The 16-byte pieces, which need a quarter of the lanes, are
  * taken only where they still leave two wavefronts per compute unit. */
 template <typename F, int LD, int LM>
 static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sorted, const uint32_t* starts, const uint32_t* sizes,
-                              F* means, size_t stride_means, uint32_t dim, uint32_t k, bool divide, const DeviceInfo& dev)
+                              F* means, size_t stride_means, uint32_t dim, uint32_t k, uint32_t n, bool divide, const DeviceInfo& dev)
 {
 	constexpr int WIDE = 16 / sizeof(F);
+	/* Clusters of a few dozen members leave a work-group of eight wavefronts nothing to overlap, the more so the more clusters there are
+	 * (all of the update, us, staged and not: N = 80k, d = 32, k = 1024 31, 37; N = 40k 31, 30; d = 4, k = 4096: N = 1M 114, 116; N = 270k 77, 64).
+	 * Blocks of 32 coordinates are whole cache lines; of 16, twice as many work-groups and half the pieces per member, which long
+	 * chains want (N = 2M, d = 32, k = 1024 261 -> 231; N = 1M, d = 64, k = 100 388 -> 274) and the others do not (N = 500k, d = 500,
+	 * k = 200 432 -> 479; N = 100k, d = 32, k = 1024 34 -> 38). */
+	const uint32_t members = n / k;
+	const uint32_t block_dims = members >= 512 && (uint64_t)k * ((dim + 31) / 32) <= 1024 ? 16 : 32;
+	const uint32_t blocks = (dim + block_dims - 1) / block_dims;
+	if (members >= ((uint64_t)k * blocks <= 2048 ? 64u : 256u) && (uint64_t)k * blocks <= 0x7FFFFFFFu) {
+		const bool elements = LD == KMX_SOA || dim < (uint32_t)WIDE || (dim % block_dims != 0 && dim % block_dims < (uint32_t)WIDE);
+		const uint32_t lds = STAGED_THREADS * STAGED_PIECES * (elements ? sizeof(F) : 16) + std::min(dim, block_dims) * 16;
+		auto kernel = elements ? ordered_staged_sum_kernel<F, LD, LM, true> : ordered_staged_sum_kernel<F, KMX_AOS, LM, false>;
+		KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+		KMX_LAUNCH_KERNEL(kernel, dim3(k * blocks), dim3(STAGED_THREADS), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, blocks, block_dims, divide ? 1u : 0u);
+		KMX_LAUNCH_CHECK("ordered_staged_sum_kernel");
+		return KMX_OK;
+	}
 	const bool fits = LD == KMX_AOS && dim % WIDE == 0 && stride % WIDE == 0 && ((uintptr_t)data & 15) == 0;
 	const bool wide = fits && (size_t)k * (dim / WIDE) >= (size_t)2 * WAVE * dev.compute_units;
 	const size_t total = (size_t)k * (wide ? dim / WIDE : dim);
@@ -263,18 +396,23 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 		chunk_points = ((n + chunks - 1) / chunks + WAVE - 1) / WAVE * WAVE;
 		chunks = (n + chunk_points - 1) / chunk_points;
 	}
-	const uint32_t ranges = std::max<uint32_t>(1, std::min<uint32_t>({ 64u, chunks, (16384 + k - 1) / k }));
-	const uint32_t per = chunks ? (chunks + ranges - 1) / ranges : 0;
-	const size_t hist_words = (size_t)std::max(chunks, 1u) * k, range_words = (size_t)ranges * k;
-	int rc = reserve_partials(ws, hist_words + range_words + k + n);
+	const size_t hist_words = (size_t)std::max(chunks, 1u) * k;
+	int rc = reserve_partials(ws, hist_words + k + n);
 	if (rc) return rc;
 	uint32_t* hist = (uint32_t*)ws->partials;
-	uint32_t* range_sums = hist + hist_words;
-	uint32_t* starts = range_sums + range_words;
+	uint32_t* starts = hist + hist_words;
 	uint32_t* sorted = starts + k;
 	const bool in_lds = k <= ORDERED_LDS_CLUSTERS;
 	const uint32_t lds_bytes = in_lds ? k * 4 : 0;
 
+	if constexpr (std::is_same<F, float>::value) {
+		/* members are read row by row: SoA points go through an AoS copy like those of the other updates */
+		UpdateArgs u{ data, layout, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n };
+		if (update_wants_rows(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev)) {
+			if ((rc = launch_rows_from_soa(data, stride, dim, n, ws, dev))) return rc;
+			data = ws->rows_copy; layout = KMX_AOS; stride = dim;
+		}
+	}
 	if ((rc = profile_begin(1))) return rc;
 	exec->block_count = chunks;
 	if (chunks > 0) {
@@ -289,10 +427,7 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 		}
 		KMX_LAUNCH_CHECK("ordered_histogram_kernel");
 	}
-	const uint32_t scan_blocks = (uint32_t)((range_words + 255) / 256);
-	KMX_LAUNCH_KERNEL(ordered_range_sums_kernel, dim3(scan_blocks), dim3(256), 0, stream(), hist, range_sums, k, chunks, ranges, per);
-	KMX_LAUNCH_CHECK("ordered_range_sums_kernel");
-	KMX_LAUNCH_KERNEL(ordered_offsets_kernel, dim3(scan_blocks), dim3(256), 0, stream(), hist, range_sums, cluster_sizes, k, chunks, ranges, per);
+	KMX_LAUNCH_KERNEL(ordered_offsets_kernel, dim3((k + SCAN_COLUMNS - 1) / SCAN_COLUMNS), dim3(SCAN_COLUMNS * SCAN_SHARES), 0, stream(), hist, cluster_sizes, k, chunks);
 	KMX_LAUNCH_CHECK("ordered_offsets_kernel");
 	KMX_LAUNCH_KERNEL(ordered_starts_kernel, dim3(1), dim3(1024), 0, stream(), cluster_sizes, starts, k);
 	KMX_LAUNCH_CHECK("ordered_starts_kernel");
@@ -305,10 +440,10 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 			KMX_LAUNCH_KERNEL((ordered_scatter_kernel<false>), dim3(chunks), dim3(WAVE), 0, stream(), assignment, hist, starts, sorted, k, n, chunk_points);
 		KMX_LAUNCH_CHECK("ordered_scatter_kernel");
 	}
-	if (layout == KMX_AOS && layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, divide, dev);
-	else if (layout == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, divide, dev);
-	else if (layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_SOA, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, divide, dev);
-	else rc = launch_ordered_sum<F, KMX_SOA, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, divide, dev);
+	if (layout == KMX_AOS && layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
+	else if (layout == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
+	else if (layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_SOA, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
+	else rc = launch_ordered_sum<F, KMX_SOA, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
 	if (rc) return rc;
 	return profile_end(1);
 }

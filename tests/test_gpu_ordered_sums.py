@@ -1,0 +1,44 @@
+"""The serial-order update for clusters of many members (ordered_staged_sum_kernel, csrc/update_ordered.hip): the bits of one
+addition after the other, at the edges of its blocks of coordinates, pieces and fetches (-m gpu)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dim,k", [(1, 3), (2, 40), (3, 20), (4, 9), (5, 33), (16, 2), (17, 12), (31, 5), (33, 7), (35, 6), (64, 4), (65, 3), (130, 2)])
+def test_staged_sums_have_the_bits_of_the_serial_loop(km, gpu, dim, k, dtype):
+    rng = np.random.default_rng(dim + 100 * k)
+    sizes = [0, 1, 3, 4, 15, 16, 17, 255, 256, 257, 1024, 4097, 9000][:k] + [90] * max(0, k - 13)
+    sizes[-1] += max(0, 600 * k - sum(sizes))  # well over 512 members on average, most of them in one cluster
+    which = rng.permutation(np.repeat(np.arange(k), sizes)).astype(np.uint32)
+    n = len(which)
+    which[5:n:97] = k  # not a cluster: left out
+    rows = (rng.normal(size=(n, dim)) * np.exp(rng.normal(size=(n, 1)) * 4)).astype(dtype)
+    want = np.zeros((k, dim), dtype)
+    counts = np.zeros(k, np.uint32)
+    for c in range(k):
+        members = rows[which == c]
+        counts[c] = len(members)
+        if len(members):  # cumsum adds one after the other (numpy's sum does not)
+            want[c] = np.cumsum(np.concatenate([np.zeros((1, dim), dtype), members]), axis=0, dtype=dtype)[-1] / dtype(len(members))
+    size = np.dtype(dtype).itemsize
+    a = km.DeviceBuffer(4 * n); a.write(which)
+    m = km.DeviceBuffer(size * k * dim); s = km.DeviceBuffer(4 * k)
+    for layout, pad in [(0, 0), (0, 3), (1, 0)]:
+        stride = dim + pad if layout == 0 else n
+        data = np.full((n, stride), np.nan, dtype) if layout == 0 else rows.T
+        if layout == 0:
+            data[:, :dim] = rows
+        data = np.ascontiguousarray(data).ravel()
+        d = km.DeviceBuffer(data.nbytes); d.write(data)
+        for layout_means in (0, 1):
+            km.update(km.UPDATE_SERIAL_ORDER, d, layout, stride, a, m, layout_means, km.layout_stride(layout_means, k, dim), s, dim, k, n, dtype=dtype)
+            km.sync()
+            got = m.read(dtype, k * dim)
+            got = got.reshape(k, dim) if layout_means == 0 else got.reshape(dim, k).T
+            assert np.array_equal(s.read(np.uint32, k), counts)
+            assert np.array_equal(got, want), "layouts %d/%d: %d differ" % (layout, layout_means, int((got != want).sum()))
+        d.free()
+    a.free(); m.free(); s.free()
