@@ -5,9 +5,9 @@
  * share them: every wavefront owns centroid tiles of its own, whose packed operands it reads straight from the caches (no two
  * wavefronts of a work-group want the same ones, so LDS would only add a copy).
  *
- * Ranking, split operands and certificates are those of assign_bf16.hip: a[j] = |c_j|^2 - 2 c_j . x by
- * v_mfma_f32_32x32x16_bf16, either the hi parts alone (the first level: all points) or three products (the second level: the
- * points the first could not settle; the only level of small inputs). What three products cannot settle goes to the exact pass.
+ * Ranking, operands and certificates are those of rank16.hip, one product per dimension in half precision, and the points it lists get
+ * their serial result from the exact pass of that file (rank16_exact_impl.h). Rows of more than 2304 dimensions, whose operands that
+ * pass cannot keep in LDS, and kmx_set_two_level_sweep(0) take the three bf16 products of assign_bf16.hip and its exact pass.
  *
  * Split of the work. Per block of 16 dimensions a wavefront reads the operands of its NT centroid tiles (1 KB each, global)
  * and of the PT point tiles (1 KB each, LDS) for NT * PT MFMAs of 32 cycles; with NT = 2, PT = 4 the four SIMDs of a compute
@@ -16,9 +16,10 @@
  * The rows of a unit are read from memory once while 512 centroids go by; with more centroids the converted rows stay in LDS
  * if they fit (d <= 512 in the first level), otherwise they are staged again per group of 512.
  *
- * N = 131071, d = 512, k = 400, one iteration: the lane-per-point kernel that took these rows before needed 147 ms.
+ * N = 131071, d = 512, k = 400, one iteration: the lane-per-point kernel that took these rows before needed 147 ms, two levels of bf16
+ * products and a pass over the slices of the queued points (234 us of the assignment) 0.29 ms.
  */
-#include "assign_bf16_impl.h"
+#include "rank16_exact_impl.h"
 
 namespace kmx {
 
@@ -37,9 +38,12 @@ __host__ __device__ __forceinline__ size_t wide_plane_units(uint32_t kp, uint32_
 
 struct WideArgs {
 	const float* data; size_t stride;
-	const bf16x8* packed; const float* norms;
+	const bf16x8* packed;   /* bf16 parts, or half-precision values of S (c - m) */
+	const float* norms;     /* tiles of |c - m|^2 (S^2 |c - m|^2) */
+	const float* part_norms; /* per row the squared norm of the mid parts, then of the rest (of what half precision leaves out) */
+	const float* frame;     /* dp floats: m; bf16: then |m|^2 and an upper bound of |m| */
+	float* scale;           /* half precision: S (rank16_leave_bounds) */
 	uint32_t* assignment; uint32_t* queue; uint32_t* counters;
-	const uint32_t* list; const uint32_t* list_length;
 	uint32_t dim, dp, k, kp, n, buffers;
 	float kd, kd_unmoved;
 };
@@ -116,9 +120,100 @@ pack_means_wide_kernel(const float* __restrict__ means, size_t stride_means, __b
 	}
 }
 
+/* ws->norms16 of wide rows: tiles of S^2 |c - m|^2; per row the squared norms of what half precision leaves out and of the bf16 mid
+ * and rest parts (all of S (c - m)); m; S, 1 / S^2 and (rank16_leave_bounds) three maxima */
+__host__ __device__ __forceinline__ size_t wide16_part_offset(uint32_t kp) { return (size_t)(kp / TILE) * NORM_TILE; }
+__host__ __device__ __forceinline__ size_t wide16_frame_offset(uint32_t kp) { return wide16_part_offset(kp) + 3 * (size_t)kp; }
+__host__ __device__ __forceinline__ size_t wide16_scale_offset(uint32_t kp, uint32_t dp) { return wide16_frame_offset(kp) + dp; }
+static size_t wide16_norms_floats(uint32_t kp, uint32_t dp) { return wide16_scale_offset(kp, dp) + 8; }
+
+/* groups of 32 listed points whose operands fit the LDS of the exact pass (0: none) */
+static uint32_t wide16_groups(uint32_t dp, uint32_t lds_budget)
+{
+	for (uint32_t groups : { 4u, 2u, 1u })
+		if (exact_dynamic_bytes(dp / KBLOCK, groups) + EXACT_STATIC_BYTES <= lds_budget) return groups;
+	return 0;
+}
+
+/* pack_means16_kernel (rank16.hip) for any row length: one wavefront per (padded) centroid row */
+template <int LM>
+__global__ void __launch_bounds__(256)
+pack_means16_wide_kernel(const float* __restrict__ means, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
+                         uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters)
+{
+	extern __shared__ float m[]; /* dp floats */
+	__shared__ float wave_far[4];
+	constexpr uint32_t SAMPLE = 16;
+	const uint32_t lane = threadIdx.x & (WAVE - 1);
+	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; }
+	const uint32_t sample = min(k, SAMPLE);
+	float far = 0.0f;
+	for (uint32_t q = threadIdx.x; q < dp; q += 256) {
+		float sum = 0.0f;
+		if (q < dim) {
+			float v[SAMPLE];
+#pragma unroll
+			for (uint32_t r = 0; r < SAMPLE; ++r) v[r] = r < sample ? means[elem<LM>(stride_means, r, q)] : 0.0f;
+#pragma unroll
+			for (uint32_t r = 0; r < SAMPLE; ++r) sum += __builtin_fabsf(v[r]) < __builtin_inff() ? v[r] : 0.0f;
+			sum = sum / (float)sample;
+			sum = __builtin_fabsf(sum) < __builtin_inff() ? sum : 0.0f;
+#pragma unroll
+			for (uint32_t r = 0; r < SAMPLE; ++r) {
+				const float d = __builtin_fabsf(v[r] - sum);
+				if (r < sample && d < __builtin_inff()) far = fmaxf(far, d);
+			}
+		}
+		m[q] = sum;
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) far = fmaxf(far, __shfl_xor(far, off));
+	if (lane == 0) wave_far[threadIdx.x / WAVE] = far;
+	__syncthreads();
+	const float scale = rank16_scale(fmaxf(fmaxf(wave_far[0], wave_far[1]), fmaxf(wave_far[2], wave_far[3])));
+	if (blockIdx.x == 0) {
+		for (uint32_t q = threadIdx.x; q < dp; q += 256) norms[wide16_frame_offset(kp) + q] = m[q];
+		if (threadIdx.x == 0) {
+			norms[wide16_scale_offset(kp, dp)] = scale;
+			norms[wide16_scale_offset(kp, dp) + 1] = 1.0f / (scale * scale);
+		}
+	}
+	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+	if (j >= kp) return;
+	float c2 = 0.0f, low2 = 0.0f, mid2 = 0.0f, rest2 = 0.0f;
+	for (uint32_t q = lane; q < dp; q += WAVE) {
+		const bool there = j < k && q < dim;
+		const float exact = there ? means[elem<LM>(stride_means, j, q)] : 0.0f;
+		const float v = there ? __builtin_fmaf(exact, scale, -(m[q] * scale)) : 0.0f;
+		c2 += v * v;
+		const float cv = -2.0f * v;
+		const _Float16 half = (_Float16)cv;
+		const float low = cv - (float)half;
+		low2 += low * low;
+		__bf16 hi, mid;
+		const float rest = split_bf16(cv, hi, mid);
+		mid2 += (float)mid * (float)mid;
+		rest2 += rest * rest;
+		rows[(size_t)j * dp + q] = exact;
+		packed[(((size_t)(j / TILE) * (dp / KBLOCK) + q / KBLOCK) * WAVE + (q % KBLOCK) / 8 * TILE + j % TILE) * 8 + q % 8] = half;
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) {
+		c2 += __shfl_xor(c2, off);
+		low2 += __shfl_xor(low2, off);
+		mid2 += __shfl_xor(mid2, off);
+		rest2 += __shfl_xor(rest2, off);
+	}
+	if (lane == 0) {
+		norms[norm_at(j)] = j < k ? c2 : 1.7e38f;
+		norms[wide16_part_offset(kp) + j] = low2;
+		norms[wide16_part_offset(kp) + kp + j] = mid2;
+		norms[wide16_part_offset(kp) + 2 * kp + j] = rest2;
+	}
+	if (lane < NORM_TILE - TILE && j % TILE == 0) norms[(j / TILE) * NORM_TILE + TILE + lane] = 1.7e38f;
+}
+
 /*
  * PT point tiles of 32 per unit, NT centroid tiles per wavefront and group (a group: the WIDE_WAVES * NT tiles that go by together),
- * X3: three products instead of the hi parts alone. LISTED: the points of a list (entries of two words, the first the point number).
+ * X3: three bf16 products instead of one in half precision.
  *
  * Order of a step (one chunk of 64 dimensions against one group): the operands of the chunk's four blocks are in registers,
  * each block's are replaced by those of the next step as soon as its MFMAs have been issued; the B operands of block b + 1
@@ -130,7 +225,7 @@ pack_means_wide_kernel(const float* __restrict__ means, size_t stride_means, __b
  * (cert_kd_keyed): three operations per value for the two smallest and the place of the smallest. A NaN anywhere makes the smallest
  * NaN (v_minimum3_f32 passes it on), which certifies nothing.
  */
-template <int PT, int NT, bool X3, int LD, bool VEC, bool LISTED>
+template <int PT, int NT, bool X3, int LD, bool VEC>
 __global__ void __launch_bounds__(WIDE_THREADS)
 wide_sweep_kernel(const WideArgs w)
 {
@@ -158,7 +253,8 @@ wide_sweep_kernel(const WideArgs w)
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 	const uint32_t col = lane & 31, h = lane >> 5;
-	const uint32_t n = LISTED ? min(w.list_length[0], w.n) : w.n;
+	const uint32_t n = w.n;
+	const float scale = X3 ? 1.0f : w.scale[0];
 	const uint32_t units = (n + ROWS - 1) / ROWS;
 	const uint32_t tiles = w.kp / TILE;
 	const uint32_t groups = (tiles + GROUP_TILES - 1) / GROUP_TILES;
@@ -171,16 +267,15 @@ wide_sweep_kernel(const WideArgs w)
 
 	/* the certificate's maxima over the centroids (bit patterns: NaN and infinity win) and the frame */
 	if (tid == 0) flag_count = 0u;
-	for (uint32_t q = tid; q < w.dp; q += WIDE_THREADS) frame[q] = w.norms[frame_offset(w.kp) + q];
-	const float m2 = w.norms[frame_offset(w.kp) + w.dp], mnorm = w.norms[frame_offset(w.kp) + w.dp + 1];
+	for (uint32_t q = tid; q < w.dp; q += WIDE_THREADS) frame[q] = w.frame[q] * scale; /* S m */
+	const float m2 = X3 ? w.frame[w.dp] : 0.0f, mnorm = X3 ? w.frame[w.dp + 1] : 0.0f;
 	CertCoeffs cert;
 	{
-		const float* part_norms = w.norms + split_norms_offset(w.kp);
 		uint32_t most[3] = { 0u, 0u, 0u };
 		for (uint32_t j = tid; j < w.k; j += WIDE_THREADS) {
 			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
-			most[1] = max(most[1], __float_as_uint(part_norms[j]));
-			most[2] = max(most[2], __float_as_uint(part_norms[w.kp + j]));
+			most[1] = max(most[1], __float_as_uint(w.part_norms[j]));
+			if (X3) most[2] = max(most[2], __float_as_uint(w.part_norms[w.kp + j]));
 		}
 #pragma unroll
 		for (int q = 0; q < 3; ++q) {
@@ -194,6 +289,7 @@ wide_sweep_kernel(const WideArgs w)
 			for (uint32_t v = 0; v < WIDE_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
 		}
 		const CentroidBounds cb{ __uint_as_float(most[0]), __uint_as_float(most[1]), __uint_as_float(most[2]) };
+		if (!X3 && blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], w.part_norms, w.k, w.kp);
 		cert = X3 ? cert_coeffs_split(cb) : cert_coeffs_level1(cb);
 	}
 
@@ -203,7 +299,7 @@ wide_sweep_kernel(const WideArgs w)
 	f32x4 piece[VECS];
 	auto point_of = [&](uint32_t unit) -> uint32_t { /* rows beyond the end repeat the last one */
 		const uint32_t slot = min(unit * ROWS + row, n - 1);
-		return LISTED ? w.list[2 * (size_t)slot] : slot;
+		return slot;
 	};
 	auto request_rows = [&](uint32_t pt, uint32_t chunk) {
 #pragma unroll
@@ -247,15 +343,25 @@ wide_sweep_kernel(const WideArgs w)
 			float a = 0.0f, b = 0.0f, c = 0.0f;
 #pragma unroll
 			for (int e = 0; e < 4; ++e) {
-				const float v = chunk * WIDE_CHUNK + f * 4 + e < w.dim ? piece[i][e] - mv[e] : 0.0f;
-				__bf16 vh, vm;
-				split_bf16(v, vh, vm);
-				hi[e] = vh;
-				mid[e] = vm;
-				const float low = X3 ? (float)vm : v - (float)vh;
-				a += v * v;
-				b += low * low;
-				c += v * mv[e];
+				const bool there = chunk * WIDE_CHUNK + f * 4 + e < w.dim;
+				if constexpr (X3) {
+					const float v = there ? piece[i][e] - mv[e] : 0.0f;
+					__bf16 vh, vm;
+					split_bf16(v, vh, vm);
+					hi[e] = vh;
+					mid[e] = vm;
+					a += v * v;
+					b += (float)vm * (float)vm;
+					c += v * mv[e];
+				}
+				else {
+					const float v = there ? __builtin_fmaf(piece[i][e], scale, -mv[e]) : 0.0f;
+					const _Float16 half = (_Float16)v;
+					const float low = v - (float)half;
+					hi[e] = __builtin_bit_cast(__bf16, half);
+					a += v * v;
+					b += low * low;
+				}
 			}
 			if (first_pass) { xx += a; xpart += b; xalong += c; }
 			char* at = base + ((f / 2) * UNIT_STRIDE + row) * 16 + (f % 2) * 8;
@@ -374,7 +480,10 @@ wide_sweep_kernel(const WideArgs w)
 							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(amid[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
 						}
 #pragma unroll
-						for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
+						for (int p = 0; p < PT; ++p) {
+							if constexpr (X3) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
+							else acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ahi[b][nt]), __builtin_bit_cast(f16x8, bhi[b & 1][p]), acc[nt][p], 0, 0, 0);
+						}
 					}
 					__builtin_amdgcn_sched_barrier(0);
 					fetch_ops(b);
@@ -467,13 +576,15 @@ wide_sweep_kernel(const WideArgs w)
 			const float tau = cert_tau(w.kd, x2, row_info[1][tid], cert);
 			const uint32_t slot = unit * ROWS + tid;
 			const bool mine = slot < uniform_n;
-			const uint32_t point = LISTED ? w.list[2 * (size_t)min(slot, uniform_n - 1)] : slot;
-			const bool decided = (next - first > tau) && (x2 + cert.c2max > 1e-30f) && idx < w.k;
-			if (mine) w.assignment[point] = idx < w.k ? idx : 0u;
+			/* squares of the data as given underflow or overflow: no ranking says anything about the serial sums (in the frame of the
+			 * data as it is, an overflow makes the values infinite or NaN) */
+			const bool extreme = !(x2 + cert.c2max > 1e-30f * (scale * scale)) || (!X3 && !(x2 + cert.c2max < 1e37f * (scale * scale)));
+			const bool decided = (next - first > tau) && !extreme && idx < w.k;
+			if (mine) w.assignment[slot] = idx < w.k ? idx : 0u;
 			if (mine && !decided) {
 				const uint32_t at = atomicAdd(&flag_count, 1u);
-				flags[2 * at] = point;
-				flags[2 * at + 1] = w.kd_unmoved > 0.0f
+				flags[2 * at] = slot;
+				flags[2 * at + 1] = !X3 ? screening_threshold(extreme ? __builtin_inff() : first, tau) : w.kd_unmoved > 0.0f
 					? screening_threshold(cert_unmoved_threshold(first, tau, x2, along, cert.c2max, m2, mnorm, w.kd_unmoved), 0.0f)
 					: screening_threshold(first, tau);
 			}
@@ -499,12 +610,12 @@ bool wide_supports(const AssignArgs& a, const DeviceInfo& dev)
 	return a.dim > 256 && a.dim <= WIDE_MAX_DIM && dp * 4 + 2 * wide_buffer_bytes(4, true) + wide_static_bytes(4, 2) <= dev.lds_bytes;
 }
 
-template <int PT, int NT, bool X3, bool LISTED>
+template <int PT, int NT, bool X3>
 static int launch_wide_sweep(const AssignArgs& a, WideArgs w, const DeviceInfo& dev, kmx_exec_params* exec)
 {
 	const bool vec = a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data & 15) == 0;
-	void (*kernel)(WideArgs) = a.layout == KMX_SOA ? wide_sweep_kernel<PT, NT, X3, KMX_SOA, false, LISTED>
-	                           : vec ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, true, LISTED> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, false, LISTED>;
+	void (*kernel)(WideArgs) = a.layout == KMX_SOA ? wide_sweep_kernel<PT, NT, X3, KMX_SOA, false>
+	                           : vec ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, true> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, false>;
 	const uint32_t chunks = w.dp / WIDE_CHUNK, groups = (w.kp / TILE + WIDE_WAVES * NT - 1) / (WIDE_WAVES * NT);
 	const uint32_t buffer = wide_buffer_bytes(PT, X3);
 	const uint32_t room = dev.lds_bytes - wide_static_bytes(PT, NT) - w.dp * 4;
@@ -521,57 +632,75 @@ static int launch_wide_sweep(const AssignArgs& a, WideArgs w, const DeviceInfo& 
 }
 
 /* every offset the kernels form must lie inside its allocation (see check_sweep_plan) */
-static int check_wide_plan(const AssignArgs& a, const WideArgs& w, const Workspace* ws, bool two_level)
+static int check_wide_plan(const AssignArgs& a, const WideArgs& w, const Workspace* ws, bool half)
 {
 #define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (wide rows): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u)", #cond, a.dim, a.k, w.kp, a.n); } while (0)
 	KMX_PLAN(w.dp % WIDE_CHUNK == 0 && w.dp >= a.dim && w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1);
+	if (half) {
+		KMX_PLAN(ws->packed16 && wide_plane_units(w.kp, w.dp) * 4 + (size_t)w.kp * w.dp <= ws->packed16_cap);
+		KMX_PLAN(ws->norms16 && wide16_norms_floats(w.kp, w.dp) <= ws->norms16_cap);
+		KMX_PLAN(ws->listed && 2 * (size_t)a.n <= ws->listed_cap && ws->counters);
+		return KMX_OK;
+	}
 	KMX_PLAN(ws->packed_means && wide_plane_units(w.kp, w.dp) * 2 * 4 <= ws->packed_cap);
 	KMX_PLAN(ws->norms && wide_norms_floats(w.kp, w.dp) <= ws->norms_cap);
 	KMX_PLAN(ws->means_t && (size_t)w.kp * a.dim <= ws->means_t_cap);
 	KMX_PLAN(ws->queue && 2 * (size_t)a.n <= ws->queue_cap && ws->counters);
-	KMX_PLAN(!two_level || (ws->listed && 2 * (size_t)a.n <= ws->listed_cap));
 #undef KMX_PLAN
 	return KMX_OK;
 }
 
-/* Two levels pay from about a hundred units of 128 points and two centroid tiles on: below that the second launch costs more
- * than the products it saves. Few points are swept in units of 32, so that they reach more compute units. */
-constexpr uint32_t WIDE_TWO_LEVEL_POINTS = 1u << 14;
+/* one half-precision product per dimension, then the exact pass for what that lists */
+static int launch_assign_wide16(const AssignArgs& a, uint32_t dp, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	const uint32_t kp = round_up(a.k, TILE);
+	const size_t operand_floats = wide_plane_units(kp, dp) * 4;
+	int rc = reserve_packed16(ws, operand_floats + (size_t)kp * dp, wide16_norms_floats(kp, dp));
+	if (rc) return rc;
+	if ((rc = reserve_listed(ws, 2 * (size_t)a.n))) return rc;
+	float* rows = ws->packed16 + operand_floats;
+	auto pack = a.layout_means == KMX_AOS ? pack_means16_wide_kernel<KMX_AOS> : pack_means16_wide_kernel<KMX_SOA>;
+	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), dp * 4, stream(),
+	                   a.means, a.stride_means, (_Float16*)ws->packed16, rows, ws->norms16, a.dim, a.k, kp, dp, ws->counters);
+	KMX_LAUNCH_CHECK("pack_means16_wide_kernel");
+	const float* norms = ws->norms16;
+	const WideArgs w = { a.data, a.stride, (const bf16x8*)ws->packed16, norms, norms + wide16_part_offset(kp), norms + wide16_frame_offset(kp), ws->norms16 + wide16_scale_offset(kp, dp),
+	                     a.assignment, ws->listed, ws->counters + LISTED_COUNTER, a.dim, dp, a.k, kp, a.n, 0,
+	                     cert_kd_level1(a.dim) + cert_kd_keyed(5) + 8.0f * CERT_UNIT + a.kd_extra, 0.0f };
+	if (!sizing_only() && (rc = check_wide_plan(a, w, ws, true))) return rc;
+	if ((rc = profile_begin(0))) return rc;
+	/* units of 128 points, or, where those do not reach half of the compute units, of 32 */
+	rc = a.n >= 64 * dev.compute_units ? launch_wide_sweep<4, 2, false>(a, w, dev, exec) : launch_wide_sweep<1, 1, false>(a, w, dev, exec);
+	if (rc) return rc;
+	if ((rc = profile_end(0))) return rc;
+	const bool aos = a.layout == KMX_AOS;
+	const ExactArgs e = { a.data, aos ? a.stride : 1, aos ? 1 : a.stride, a.dim, rows, (const f16x8*)ws->packed16, norms,
+	                      norms + wide16_frame_offset(kp), norms + wide16_scale_offset(kp, dp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
+	                      a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, dp / KBLOCK, wide16_groups(dp, lds_budget_of(exec, dev)) };
+	return launch_listed_exact_kb<0>(a, e, dev);
+}
 
 int launch_assign_wide(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	AssignArgs a = args;
 	const uint32_t dp = round_up(a.dim, WIDE_CHUNK), kp = round_up(a.k, TILE);
+	if (a.two_level && two_level_mode() != 0 && !a.ranking_only && a.k < (1u << 25) && wide16_groups(dp, lds_budget_of(exec, dev)) > 0)
+		return launch_assign_wide16(a, dp, exec, ws, dev);
 	const bool moved = !a.ranking_only; /* (the double path hands over copies it has moved itself) */
-	const int mode = two_level_mode();
-	const bool two_level = a.two_level && mode != 0 && (mode == 2 || (a.n >= WIDE_TWO_LEVEL_POINTS && kp > 2 * TILE));
 	int rc = reserve_packed(ws, wide_plane_units(kp, dp) * 2 * 4, wide_norms_floats(kp, dp), (size_t)kp * a.dim);
 	if (rc) return rc;
 	if ((rc = reserve_queue(ws, 2 * (size_t)a.n))) return rc;
-	if (two_level && (rc = reserve_listed(ws, 2 * (size_t)a.n))) return rc;
 	auto pack = a.layout_means == KMX_AOS ? pack_means_wide_kernel<KMX_AOS> : pack_means_wide_kernel<KMX_SOA>;
 	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), dp * 4, stream(),
 	                   a.means, a.stride_means, (__bf16*)ws->packed_means, ws->norms, ws->means_t, a.dim, a.k, kp, dp, moved ? 1u : 0u, ws->counters);
 	KMX_LAUNCH_CHECK("pack_means_wide_kernel");
 
-	const float extra = (moved ? 8.0f * CERT_UNIT : 0.0f) + a.kd_extra;
-	WideArgs w = { a.data, a.stride, (const bf16x8*)ws->packed_means, ws->norms, a.assignment, ws->queue, ws->counters, nullptr, nullptr,
-	               a.dim, dp, a.k, kp, a.n, 0, 0.0f, moved ? cert_kd_unmoved(a.dim) : 0.0f };
-	if (!sizing_only() && (rc = check_wide_plan(a, w, ws, two_level))) return rc;
+	const WideArgs w = { a.data, a.stride, (const bf16x8*)ws->packed_means, ws->norms, ws->norms + split_norms_offset(kp), ws->norms + frame_offset(kp), nullptr,
+	                     a.assignment, ws->queue, ws->counters, a.dim, dp, a.k, kp, a.n, 0,
+	                     cert_kd_split(a.dim) + cert_kd_keyed(4) + (moved ? 8.0f * CERT_UNIT : 0.0f) + a.kd_extra, moved ? cert_kd_unmoved(a.dim) : 0.0f };
+	if (!sizing_only() && (rc = check_wide_plan(a, w, ws, false))) return rc;
 	if ((rc = profile_begin(0))) return rc;
-	if (two_level) {
-		WideArgs first = w;
-		first.queue = ws->listed;
-		first.counters = ws->counters + LISTED_COUNTER;
-		first.kd = cert_kd_level1(a.dim) + cert_kd_keyed(5) + extra;
-		if ((rc = launch_wide_sweep<4, 2, false, false>(a, first, dev, exec))) return rc;
-		w.list = ws->listed;
-		w.list_length = ws->counters + LISTED_COUNTER;
-	}
-	w.kd = cert_kd_split(a.dim) + cert_kd_keyed(4) + extra;
-	const bool large = a.n >= 128 * dev.compute_units;
-	if (two_level) rc = a.n >= (1u << 18) ? launch_wide_sweep<4, 1, true, true>(a, w, dev, nullptr) : launch_wide_sweep<1, 1, true, true>(a, w, dev, nullptr);
-	else rc = large ? launch_wide_sweep<4, 1, true, false>(a, w, dev, exec) : launch_wide_sweep<1, 1, true, false>(a, w, dev, exec);
+	rc = a.n >= 128 * dev.compute_units ? launch_wide_sweep<4, 1, true>(a, w, dev, exec) : launch_wide_sweep<1, 1, true>(a, w, dev, exec);
 	if (rc) return rc;
 	if ((rc = profile_end(0))) return rc;
 	if (a.ranking_only) return KMX_OK; /* the caller resolves the queued points */

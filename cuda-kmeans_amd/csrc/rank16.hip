@@ -15,7 +15,7 @@
  *
  * What bounds it: the sweep by the matrix instructions and the tracking of the minima that shares the issue slots with them
  * (N = 1M, d = 256, k = 1024: 630 us, 0.87 PFLOP/s; d = 32, k = 1024, N = 2M: 185 us); the exact pass by reading centroid operands
- * and rows (12 % of N = 1M, d = 256 listed: 131 us). Whole calls, two bf16 levels before -> now: N = 1M, d = 256, k = 1024 1713 ->
+ * and rows (12 % of N = 1M, d = 256 listed: 131 us; 1 %: 40 us, the latency of one unit). Whole calls, two bf16 levels before -> now: N = 1M, d = 256, k = 1024 1713 ->
  * 743 us; N = 2M, d = 128, k = 1024 1443 -> 683 (SoA 1629 -> 940); N = 2M, d = 32, k = 1024 332 -> 230; N = 1M, d = 64, k = 512 203 -> 122;
  * N = 100k, d = 256, k = 32 92 -> 51.
  */
@@ -46,12 +46,12 @@ KMX_DECLARE_EXACT16(6) KMX_DECLARE_EXACT16(8) KMX_DECLARE_EXACT16(12) KMX_DECLAR
  * One wavefront per (padded) centroid row: its half-precision operands, S^2 |c|^2, the squared norms of what half precision and the
  * bf16 parts leave out. Every work-group computes the frame m (sweep_frame) and S from the first 16 centroids: S max |c - m| over them
  * is in [16, 32), so that a coordinate may be 2000 times larger before it overflows.
- * norms: tiles of S^2 |c - m|^2, then per row low2, mid2, rest2, then the frame (sweep_frame), S and 1 / S^2.
+ * norms: tiles of S^2 |c - m|^2, then per row low2, mid2, rest2, then the frame (sweep_frame), S, 1 / S^2 and (rank16_leave_bounds) three maxima.
  */
 __host__ __device__ __forceinline__ size_t rank16_low_offset(uint32_t kp) { return (size_t)(kp / TILE) * NORM_TILE; }
 __host__ __device__ __forceinline__ size_t rank16_frame_offset(uint32_t kp) { return rank16_low_offset(kp) + 3 * (size_t)kp; }
 __host__ __device__ __forceinline__ size_t rank16_scale_offset(uint32_t kp) { return rank16_frame_offset(kp) + FRAME_FLOATS; }
-static size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) + 4; }
+static size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) + 8; }
 
 template <int LM>
 __global__ void __launch_bounds__(256)
@@ -86,13 +86,10 @@ pack_means16_kernel(const float* __restrict__ means, size_t stride_means, _Float
 	if (lane == 0) wave_far[threadIdx.x / WAVE] = far;
 	__syncthreads();
 	far = fmaxf(fmaxf(wave_far[0], wave_far[1]), fmaxf(wave_far[2], wave_far[3]));
-	/* 2^(131 - exponent) puts the largest into [16, 32); kept inside what S and 1 / S^2 can be as normal numbers */
-	const int exponent = (int)(__float_as_uint(far) >> 23);
-	const int shift = far > 0.0f ? min(max(131 - exponent, -60), 60) : 0;
-	const float scale = __uint_as_float((uint32_t)(127 + shift) << 23);
+	const float scale = rank16_scale(far);
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		norms[rank16_scale_offset(kp)] = scale;
-		norms[rank16_scale_offset(kp) + 1] = __uint_as_float((uint32_t)(127 - 2 * shift) << 23);
+		norms[rank16_scale_offset(kp) + 1] = 1.0f / (scale * scale);
 	}
 	if (j >= kp) return;
 	float c2 = 0.0f, low2 = 0.0f, mid2 = 0.0f, rest2 = 0.0f;
@@ -133,7 +130,7 @@ bool rank16_supports(const AssignArgs& a, uint32_t lds_budget)
 	const uint32_t kb = rank16_kb(a.dim);
 	if (a.dim <= 4 || kb == 0 || a.k >= (1u << 25) || a.n > (1u << 31)) return false;
 	const uint32_t sweep = (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + kb * KBLOCK) * 4 + 64 + 2 * (kb * WAVE * 4 + NORM_TILE) * 4; /* two tiles */
-	return sweep <= lds_budget && std::max<uint32_t>(EXACT_GROUPS * kb * WAVE * 16, EXACT_SQUARES * 4) + EXACT_STATIC_BYTES <= lds_budget;
+	return sweep <= lds_budget && exact_dynamic_bytes(kb, EXACT_GROUPS) + EXACT_STATIC_BYTES <= lds_budget;
 }
 
 /* the centroids for launch_rank16_sweep */
@@ -157,7 +154,7 @@ static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Works
 	if (rc) return rc;
 	if (a.layout == KMX_SOA && (rc = reserve_queued_rows(ws, a.n, copy_stride, 0))) return rc;
 	const float* norms = ws->norms16;
-	const Rank16Args w = { a.data, a.stride, (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp), norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp),
+	const Rank16Args w = { a.data, a.stride, (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp), norms + rank16_frame_offset(kp), ws->norms16 + rank16_scale_offset(kp),
 	                       a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->queued_rows, copy_stride, a.dim, a.k, kp, a.n, 0,
 	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + (a.ranking_only ? 0.0f : 8.0f * CERT_UNIT) + a.kd_extra };
 	switch (kb) {
@@ -180,10 +177,10 @@ static int launch_listed_exact(const AssignArgs& a, Workspace* ws, const DeviceI
 	const float* norms = ws->norms16;
 	const bool aos = a.layout == KMX_AOS;
 	const uint32_t row_dim = aos ? a.dim : round_up(a.dim, 8);
-	const ExactArgs w = { aos ? a.data : ws->queued_rows, aos ? a.stride : row_dim, row_dim,
-	                      ws->packed16 + rank16_rows_offset(kp, dp), (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp),
+	const ExactArgs w = { aos ? a.data : ws->queued_rows, aos ? a.stride : row_dim, 1, row_dim,
+	                      ws->packed16 + rank16_rows_offset(kp, dp), (const f16x8*)ws->packed16, norms,
 	                      norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
-	                      a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT };
+	                      a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, kb, EXACT_GROUPS };
 	switch (kb) {
 	case 1: return launch_listed_exact_1(a, w, dev);
 	case 2: return launch_listed_exact_2(a, w, dev);

@@ -17,15 +17,18 @@ constexpr uint32_t EXACT_HITS = 256;                       /* pairs per wavefron
 constexpr uint32_t EXACT_PAIR_FLOATS = KBLOCK + 4;         /* a pair's squares of one block of 16 dimensions; the padding spreads 16 lanes' reads over all banks */
 constexpr uint32_t EXACT_SQUARES = EXACT_WAVES * WAVE * EXACT_PAIR_FLOATS;
 
-constexpr uint32_t EXACT_STATIC_BYTES = (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + 3 * EXACT_WAVES) * 4 + 64;
+constexpr uint32_t EXACT_STATIC_BYTES = (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + EXACT_WAVES) * 4 + 64;
 
 struct ExactArgs {
-	const float* data; size_t stride; uint32_t row_dim; /* AoS, row_dim coordinates (zeros behind the first dim) */
+	/* coordinate d of point p: data[p * stride + d * step]; step 1: rows of row_dim coordinates (zeros behind the first dim). Other
+	 * steps (SoA points) are for KB = 0 only. */
+	const float* data; size_t stride, step; uint32_t row_dim;
 	const float* means;                     /* rows of KB * 16 floats, zeros behind the coordinates */
-	const f16x8* packed; const float* norms; const float* low; const float* frame; const float* scale;
+	const f16x8* packed; const float* norms; const float* frame; const float* scale;
 	uint32_t* assignment; const uint32_t* list; const uint32_t* length; uint32_t* undecided;
 	uint32_t dim, k, kp;
 	float kd_split;
+	uint32_t blocks, most_groups; /* KB = 0: blocks of 16 dimensions per row; groups whose operands fit LDS */
 };
 
 __device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
@@ -35,6 +38,7 @@ __device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
 }
 
 /*
+ * KB: blocks of 16 dimensions per row, 0: any number (their operands do not stay in registers, the accumulators of the groups do).
  * A unit is 32, 64 or 128 listed points of a work-group of eight wavefronts: as many as leave every work-group something to do, since
  * all of a unit's points share one reading of the centroids' operands (512 KB at k = 1024, d = 256).
  *   1. The rows, moved, scaled and rounded as in the sweep, go to LDS as operands of the ranking.
@@ -52,19 +56,19 @@ template <int KB>
 __global__ void __launch_bounds__(EXACT_THREADS, 4)
 listed_exact_kernel(const ExactArgs w)
 {
-	constexpr uint32_t DP = KB * KBLOCK;
+	const uint32_t blocks = KB ? KB : w.blocks, DP = blocks * KBLOCK;
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	f16x8* ops = (f16x8*)lds;                                   /* groups x KB x 64 lanes; the squares afterwards */
 	__shared__ unsigned long long best[EXACT_ROWS], second[EXACT_ROWS];
 	__shared__ float threshold[EXACT_ROWS], tau3[EXACT_ROWS];
 	__shared__ uint32_t point[EXACT_ROWS];
 	__shared__ uint32_t hits[EXACT_WAVES][EXACT_HITS];          /* row << 25 | centroid (supports: k < 2^25) */
-	__shared__ uint32_t wave_max[3][EXACT_WAVES];
+	__shared__ uint32_t noted_by[EXACT_WAVES];
 	constexpr uint32_t CENTROID = (1u << 25) - 1u;
 	const uint32_t count = w.length[0];
 	if (count == 0) return;
 	uint32_t groups = 1;
-	while (groups < EXACT_GROUPS && groups * TILE * gridDim.x < count) groups *= 2;
+	while (2 * groups <= w.most_groups && groups * TILE * gridDim.x < count) groups *= 2;
 	const uint32_t unit_rows = groups * TILE, units = (count + unit_rows - 1) / unit_rows;
 	if (blockIdx.x >= units) return;
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
@@ -72,44 +76,31 @@ listed_exact_kernel(const ExactArgs w)
 	const uint32_t col = lane & 31, h = lane >> 5;
 	const float scale = w.scale[0], unscale = w.scale[1];
 	const uint32_t tiles = w.kp / TILE;
-	const bool ragged = w.row_dim < DP;
+	const bool strided = KB == 0 && w.step != 1, ragged = w.row_dim < DP && !strided;
 
-	CertCoeffs cert; /* of the three-product ranking: only what is counted depends on it */
-	{
-		uint32_t most[3] = { 0u, 0u, 0u };
-		for (uint32_t j = tid; j < w.k; j += EXACT_THREADS) {
-			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
-			most[1] = max(most[1], __float_as_uint(w.low[w.kp + j]));
-			most[2] = max(most[2], __float_as_uint(w.low[2 * w.kp + j]));
-		}
-#pragma unroll
-		for (int q = 0; q < 3; ++q) {
-			for (int off = WAVE / 2; off > 0; off >>= 1) most[q] = max(most[q], (uint32_t)__shfl_xor((int)most[q], off));
-			if (lane == 0) wave_max[q][wave] = most[q];
-		}
-		__syncthreads();
-#pragma unroll
-		for (int q = 0; q < 3; ++q) {
-			most[q] = 0;
-			for (uint32_t v = 0; v < EXACT_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
-		}
-		cert = cert_coeffs_split(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), __uint_as_float(most[2]) });
-	}
+	/* of the three-product ranking: only what is counted depends on it (the sweep left the maxima behind the scale) */
+	const CertCoeffs cert = cert_coeffs_split(CentroidBounds{ w.scale[2], w.scale[3], w.scale[4] });
 
 	/* four coordinates of a row at its coordinate d, as they come from memory (d brought inside the row) ... */
 	auto source = [&](uint32_t row) -> const float* { return w.data + (size_t)point[row] * w.stride; };
 	auto request = [&](f32x4& v, const float* src, uint32_t d) {
 		typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-		v = *(const f32x4_any*)(src + min(d, w.row_dim - 4));
+		if (strided) {
+#pragma unroll
+			for (uint32_t e = 0; e < 4; ++e) v[e] = d + e < w.dim ? src[(size_t)(d + e) * w.step] : 0.0f;
+		}
+		else v = *(const f32x4_any*)(src + min(d, w.row_dim - 4));
 	};
 	/* ... and in their places, zeros beyond the row */
 	auto place = [&](f32x4& v, uint32_t d) {
-		const int shift = (int)(d + 4) - (int)w.row_dim;
-		const f32x4 t = v;
-		v.x = shift <= 0 ? t.x : shift == 1 ? t.y : shift == 2 ? t.z : shift == 3 ? t.w : 0.0f;
-		v.y = shift <= 0 ? t.y : shift == 1 ? t.z : shift == 2 ? t.w : 0.0f;
-		v.z = shift <= 0 ? t.z : shift == 1 ? t.w : 0.0f;
-		v.w = shift <= 0 ? t.w : 0.0f;
+		/* (masks: the compiler makes branches of the selections) */
+		const uint32_t shift = d + 4 > w.row_dim ? d + 4 - w.row_dim : 0;
+		const uint32_t m0 = 0u - (uint32_t)(shift == 0), m1 = 0u - (uint32_t)(shift == 1), m2 = 0u - (uint32_t)(shift == 2), m3 = 0u - (uint32_t)(shift == 3);
+		const uint32_t x = __float_as_uint(v.x), y = __float_as_uint(v.y), z = __float_as_uint(v.z), t = __float_as_uint(v.w);
+		v.x = __uint_as_float((x & m0) | (y & m1) | (z & m2) | (t & m3));
+		v.y = __uint_as_float((y & m0) | (z & m1) | (t & m2));
+		v.z = __uint_as_float((z & m0) | (t & m1));
+		v.w = __uint_as_float(t & m0);
 	};
 	uint32_t close_here = 0;
 	for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
@@ -130,7 +121,7 @@ listed_exact_kernel(const ExactArgs w)
 			const uint32_t lanes = EXACT_THREADS / unit_rows; /* per row: 16, 8 or 4, a piece of four coordinates each */
 			const uint32_t row = me / lanes, sub = me % lanes;
 			const float* src = source(row);
-			f16x8* dst = ops + (row / TILE) * (KB * WAVE) + row % TILE;
+			f16x8* dst = ops + (row / TILE) * (blocks * WAVE) + row % TILE;
 			float x2 = 0.0f, xmid2 = 0.0f;
 #pragma unroll 1
 			for (uint32_t f0 = sub; f0 < DP / 4; f0 += 4 * lanes) {
@@ -179,7 +170,7 @@ listed_exact_kernel(const ExactArgs w)
 				float sum = 0.0f;
 #pragma unroll 1
 				for (uint32_t d = 0; d < w.dim; ++d) {
-					const float diff = src[d] - mean[d];
+					const float diff = src[strided ? (size_t)d * w.step : (size_t)d] - mean[d];
 					const float sq = diff * diff;
 					sum = sum + sq;
 				}
@@ -189,62 +180,93 @@ listed_exact_kernel(const ExactArgs w)
 			__builtin_amdgcn_wave_barrier();
 			noted = 0;
 		};
+		auto screen = [&](const f32x16& a, uint32_t t, uint32_t g) {
+			const float limit = threshold[g * TILE + col];
+			float low = a[0]; /* NaN-propagating minimum */
+#pragma unroll
+			for (int r = 1; r < 16; ++r) low = __builtin_elementwise_minimum(low, a[r]);
+			const bool near = !(low > limit);
+			if (__builtin_amdgcn_ballot_w64(near) == 0) return;
+			uint32_t passed = 0; /* bit r: result r */
+#pragma unroll
+			for (int r = 0; r < 16; ++r) passed |= !(a[r] > limit) ? 1u << r : 0u;
+			if (t + 1 == tiles) { /* rows that do not exist */
+#pragma unroll
+				for (int r = 0; r < 16; ++r)
+					if (t * TILE + 8 * (r / 4) + 4 * h + (r % 4) >= w.k) passed &= ~(1u << r);
+			}
+			for (;;) { /* the lanes' next results */
+				const unsigned long long mask = __builtin_amdgcn_ballot_w64(passed != 0);
+				if (mask == 0) break;
+				const uint32_t more = (uint32_t)__popcll(mask);
+				if (noted + more > EXACT_HITS) evaluate_alone();
+				if (passed) {
+					const uint32_t r = (uint32_t)__builtin_ctz(passed);
+					hits[wave][noted + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (g * TILE + col) << 25 | (t * TILE + 8 * (r / 4) + 4 * h + r % 4);
+					passed &= passed - 1;
+				}
+				noted += more;
+			}
+		};
+		auto start_of = [&](uint32_t t) {
+			f32x16 start;
+#pragma unroll
+			for (int q = 0; q < 4; ++q) {
+				const f32x4 n0 = *(const f32x4*)(w.norms + t * NORM_TILE + 8 * q + 4 * h);
+				start[4 * q] = n0.x; start[4 * q + 1] = n0.y; start[4 * q + 2] = n0.z; start[4 * q + 3] = n0.w;
+			}
+			return start;
+		};
 		/* few tiles: the wavefronts share out the groups of points as well */
 		const uint32_t parts = tiles < EXACT_WAVES ? groups : 1;
 #pragma unroll 1
 		for (uint32_t t = wave / parts; t < tiles; t += EXACT_WAVES / parts) {
-			f32x16 start;
+			const f16x8* operand = w.packed + (size_t)t * (blocks * WAVE) + lane;
+			if constexpr (KB > 0) {
+				const f32x16 start = start_of(t);
+				f16x8 c[KB];
 #pragma unroll
-			for (int g = 0; g < 4; ++g) {
-				const f32x4 n0 = *(const f32x4*)(w.norms + t * NORM_TILE + 8 * g + 4 * h);
-				start[4 * g] = n0.x; start[4 * g + 1] = n0.y; start[4 * g + 2] = n0.z; start[4 * g + 3] = n0.w;
-			}
-			const f16x8* operand = w.packed + (size_t)t * (KB * WAVE) + lane;
-			f16x8 c[KB];
-#pragma unroll
-			for (int kb = 0; kb < KB; ++kb) c[kb] = operand[kb * WAVE];
+				for (int kb = 0; kb < KB; ++kb) c[kb] = operand[kb * WAVE];
 #pragma unroll 1
-			for (uint32_t g = wave % parts; g < groups; g += parts) {
-				f32x16 a = start;
-				const f16x8* x = ops + g * (KB * WAVE) + lane;
+				for (uint32_t g = wave % parts; g < groups; g += parts) {
+					f32x16 a = start;
+					const f16x8* x = ops + g * (KB * WAVE) + lane;
 #pragma unroll
-				for (int kb = 0; kb < KB; ++kb) a = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], x[kb * WAVE], a, 0, 0, 0);
-				const float limit = threshold[g * TILE + col];
-				float low = a[0]; /* NaN-propagating minimum */
-#pragma unroll
-				for (int r = 1; r < 16; ++r) low = __builtin_elementwise_minimum(low, a[r]);
-				const bool near = !(low > limit);
-				if (__builtin_amdgcn_ballot_w64(near) == 0) continue;
-				uint32_t passed = 0; /* bit r: result r */
-#pragma unroll
-				for (int r = 0; r < 16; ++r) passed |= !(a[r] > limit) ? 1u << r : 0u;
-				if (t + 1 == tiles) { /* rows that do not exist */
-#pragma unroll
-					for (int r = 0; r < 16; ++r)
-						if (t * TILE + 8 * (r / 4) + 4 * h + (r % 4) >= w.k) passed &= ~(1u << r);
+					for (int kb = 0; kb < KB; ++kb) a = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], x[kb * WAVE], a, 0, 0, 0);
+					screen(a, t, g);
 				}
-				for (;;) { /* the lanes' next results */
-					const unsigned long long mask = __builtin_amdgcn_ballot_w64(passed != 0);
-					if (mask == 0) break;
-					const uint32_t more = (uint32_t)__popcll(mask);
-					if (noted + more > EXACT_HITS) evaluate_alone();
-					if (passed) {
-						const uint32_t r = (uint32_t)__builtin_ctz(passed);
-						hits[wave][noted + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (g * TILE + col) << 25 | (t * TILE + 8 * (r / 4) + 4 * h + r % 4);
-						passed &= passed - 1;
-					}
-					noted += more;
+			}
+			else {
+				const uint32_t g0 = wave % parts;
+				f32x16 a[EXACT_GROUPS];
+				a[0] = start_of(t);
+#pragma unroll
+				for (uint32_t q = 1; q < EXACT_GROUPS; ++q) a[q] = a[0];
+				for (uint32_t kb = 0; kb < blocks; kb += 4) { /* (rows are padded to whole chunks of four blocks) */
+					f16x8 four[4];
+#pragma unroll
+					for (uint32_t i = 0; i < 4; ++i) four[i] = operand[(kb + i) * WAVE];
+#pragma unroll
+					for (uint32_t q = 0; q < EXACT_GROUPS; ++q)
+						if (g0 + q * parts < groups) {
+							const f16x8* x = ops + ((g0 + q * parts) * blocks + kb) * WAVE + lane;
+#pragma unroll
+							for (uint32_t i = 0; i < 4; ++i) a[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(four[i], x[i * WAVE], a[q], 0, 0, 0);
+						}
 				}
+#pragma unroll
+				for (uint32_t q = 0; q < EXACT_GROUPS; ++q)
+					if (g0 + q * parts < groups) screen(a[q], t, g0 + q * parts);
 			}
 		}
-		if (lane == 0) wave_max[0][wave] = noted;
+		if (lane == 0) noted_by[wave] = noted;
 		__syncthreads(); /* all pairs are listed, the operands are no longer needed */
 
 		{
 #pragma clang fp contract(off)
 			uint32_t total = 0;
 #pragma unroll
-			for (uint32_t v = 0; v < EXACT_WAVES; ++v) total += wave_max[0][v];
+			for (uint32_t v = 0; v < EXACT_WAVES; ++v) total += noted_by[v];
 			/* equal shares of the pairs, in groups of 16 */
 			const uint32_t share = ((total + 15) / 16 + EXACT_WAVES - 1) / EXACT_WAVES * 16;
 			const uint32_t end = min((wave + 1) * share, total);
@@ -253,59 +275,68 @@ listed_exact_kernel(const ExactArgs w)
 			for (uint32_t p0 = wave * share; p0 < end; p0 += WAVE) {
 				/* this lane's pair (the last one again behind the end), and the four it fetches for */
 				uint32_t at = min(p0 + lane, end - 1), list = 0;
-				while (at >= wave_max[0][list]) at -= wave_max[0][list++];
+				while (at >= noted_by[list]) at -= noted_by[list++];
 				const uint32_t hit = hits[list][at];
-				const uint32_t fours = min((end - p0 + 15) / 16, 4u);
-				const float* x[4]; const float* m[4];
-#pragma unroll
-				for (uint32_t g = 0; g < 4; ++g) {
-					const uint32_t other = (uint32_t)__shfl((int)hit, (int)(16 * g + lane / 4));
-					x[g] = source(other >> 25);
-					m[g] = w.means + (size_t)(other & CENTROID) * DP + lane % 4 * 4;
-				}
-				f32x4 xv[4], mv[4];
-#pragma unroll
-				for (int g = 0; g < 4; ++g) asm volatile("" : "=v"(xv[g]), "=v"(mv[g])); /* no values yet */
-				auto fetch = [&](uint32_t kb) {
-#pragma unroll
-					for (uint32_t g = 0; g < 4; ++g)
-						if (g < fours) {
-							request(xv[g], x[g], kb * KBLOCK + lane % 4 * 4);
-							mv[g] = *(const f32x4*)(m[g] + kb * KBLOCK);
-						}
-				};
-				fetch(0);
 				float sum = 0.0f;
-#pragma unroll 1
-				for (uint32_t kb = 0; kb < KB; ++kb) {
+				/* GROUPS of 16 pairs (those beyond the last repeat it), DEPTH blocks on their way while one is squared and added */
+				auto evaluate = [&](auto groups_tag, auto depth_tag) {
+					constexpr uint32_t GROUPS = decltype(groups_tag)::value, DEPTH = decltype(depth_tag)::value;
+					const float* x[GROUPS]; const float* m[GROUPS];
 #pragma unroll
-					for (uint32_t g = 0; g < 4; ++g)
-						if (g < fours) {
-							if (ragged && (kb + 1) * KBLOCK > w.row_dim) place(xv[g], kb * KBLOCK + lane % 4 * 4);
-							f32x4 sq;
-#pragma unroll
-							for (int e = 0; e < 4; ++e) {
-								const float diff = xv[g][e] - mv[g][e];
-								sq[e] = diff * diff;
-							}
-							*(f32x4*)(squares + (16 * g + lane / 4) * EXACT_PAIR_FLOATS + lane % 4 * 4) = sq;
-						}
-					if (kb + 1 < KB) fetch(kb + 1);
-					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-					__builtin_amdgcn_wave_barrier();
-					const float* mine = squares + lane * EXACT_PAIR_FLOATS;
-					if (lane < 16 * fours) {
-						f32x4 s[4];
-#pragma unroll
-						for (int q = 0; q < 4; ++q) s[q] = *(const f32x4*)(mine + 4 * q);
-#pragma unroll
-						for (int q = 0; q < 4; ++q)
-#pragma unroll
-							for (int e = 0; e < 4; ++e) sum = sum + s[q][e]; /* (zeros behind the row change nothing) */
+					for (uint32_t g = 0; g < GROUPS; ++g) {
+						const uint32_t other = (uint32_t)__shfl((int)hit, (int)(16 * g + lane / 4));
+						x[g] = source(other >> 25);
+						m[g] = w.means + (size_t)(other & CENTROID) * DP + lane % 4 * 4;
 					}
-					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-					__builtin_amdgcn_wave_barrier();
-				}
+					f32x4 xv[DEPTH][GROUPS], mv[DEPTH][GROUPS];
+					auto fetch = [&](uint32_t u, uint32_t kb) {
+						kb = min(kb, blocks - 1);
+#pragma unroll
+						for (uint32_t g = 0; g < GROUPS; ++g) {
+							request(xv[u][g], x[g], kb * KBLOCK + lane % 4 * 4);
+							mv[u][g] = *(const f32x4*)(m[g] + kb * KBLOCK);
+						}
+					};
+#pragma unroll
+					for (uint32_t u = 0; u < DEPTH; ++u) fetch(u, u);
+#pragma unroll 1
+					for (uint32_t kb0 = 0; kb0 < blocks; kb0 += DEPTH) {
+#pragma unroll
+						for (uint32_t u = 0; u < DEPTH; ++u) {
+							const uint32_t kb = kb0 + u;
+							if (DEPTH > 1 && kb >= blocks) break;
+							if (ragged && (kb + 1) * KBLOCK > w.row_dim) {
+#pragma unroll
+								for (uint32_t g = 0; g < GROUPS; ++g) place(xv[u][g], kb * KBLOCK + lane % 4 * 4);
+							}
+#pragma unroll
+							for (uint32_t g = 0; g < GROUPS; ++g) {
+								f32x4 sq;
+#pragma unroll
+								for (int e = 0; e < 4; ++e) {
+									const float diff = xv[u][g][e] - mv[u][g][e];
+									sq[e] = diff * diff;
+								}
+								*(f32x4*)(squares + (16 * g + lane / 4) * EXACT_PAIR_FLOATS + lane % 4 * 4) = sq;
+							}
+							fetch(u, kb + DEPTH);
+							__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+							__builtin_amdgcn_wave_barrier();
+							const float* mine = squares + (GROUPS == 4 ? lane : lane % 16) * EXACT_PAIR_FLOATS;
+							f32x4 s[4];
+#pragma unroll
+							for (int q = 0; q < 4; ++q) s[q] = *(const f32x4*)(mine + 4 * q);
+#pragma unroll
+							for (int q = 0; q < 4; ++q)
+#pragma unroll
+								for (int e = 0; e < 4; ++e) sum = sum + s[q][e]; /* (zeros behind the row change nothing) */
+							__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+							__builtin_amdgcn_wave_barrier();
+						}
+					}
+				};
+				if (end - p0 <= 16) evaluate(std::integral_constant<uint32_t, 1>{}, std::integral_constant<uint32_t, 4>{});
+				else evaluate(std::integral_constant<uint32_t, 4>{}, std::integral_constant<uint32_t, 1>{});
 				if (p0 + lane < end) merge(hit >> 25, exact_key(sum, hit & CENTROID));
 			}
 		}
@@ -323,13 +354,14 @@ listed_exact_kernel(const ExactArgs w)
 	}
 }
 
-template <int KB> constexpr uint32_t exact_dynamic_bytes() { return std::max<uint32_t>(EXACT_GROUPS * KB * WAVE * 16, EXACT_SQUARES * 4); }
+/* operands of the groups; the squares take their place */
+constexpr uint32_t exact_dynamic_bytes(uint32_t blocks, uint32_t groups) { return std::max<uint32_t>(groups * blocks * WAVE * 16, EXACT_SQUARES * 4); }
 
 template <int KB>
 static int launch_listed_exact_kb(const AssignArgs& a, const ExactArgs& w, const DeviceInfo& dev)
 {
 	void (*kernel)(ExactArgs) = listed_exact_kernel<KB>;
-	const uint32_t lds = exact_dynamic_bytes<KB>();
+	const uint32_t lds = exact_dynamic_bytes(KB ? KB : w.blocks, w.most_groups);
 	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 	const uint32_t grid = std::min<uint32_t>((a.n + TILE - 1) / TILE, 2 * dev.compute_units);
 	KMX_LAUNCH_KERNEL(kernel, dim3(grid), dim3(EXACT_THREADS), lds, stream(), w);

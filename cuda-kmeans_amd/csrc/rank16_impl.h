@@ -24,7 +24,7 @@ struct Rank16Args {
 	const float* norms;    /* tiles of S^2 |c - m|^2 */
 	const float* low2;     /* per padded row the squared norm of what the half-precision parts leave out */
 	const float* frame;    /* m */
-	const float* scale;    /* S, 1 / S^2 */
+	float* scale;          /* S, 1 / S^2; the first work-group puts the maxima of the norms and of the bf16 mid and rest parts behind them */
 	uint32_t* assignment; uint32_t* list; uint32_t* length;
 	float* copies; uint32_t copy_stride; /* SoA: the rows as AoS, zeros behind the coordinates */
 	uint32_t dim, k, kp, n, chunk_tiles;
@@ -34,6 +34,30 @@ struct Rank16Args {
 /* 16 tile bytes per block of 16 dimensions and lane, then the tile's norms */
 template <int KB> constexpr uint32_t rank16_tile_floats() { return KB * WAVE * 4; }
 template <int KB> constexpr uint32_t rank16_static_bytes() { return (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + KB * KBLOCK) * 4 + 64; }
+
+/* S for centroids whose coordinates are up to `far` from the frame: the power of two that puts far into [16, 32), kept inside what S and
+ * 1 / S^2 can be as normal numbers */
+__device__ __forceinline__ float rank16_scale(float far)
+{
+	const int shift = far > 0.0f ? min(max(131 - (int)(__float_as_uint(far) >> 23), -60), 60) : 0;
+	return __uint_as_float((uint32_t)(127 + shift) << 23);
+}
+
+/* the exact pass's certificate, by one work-group (first wavefront): max |c|^2, max |mid|^2, max |rest|^2 to scale[2 .. 4] */
+__device__ __forceinline__ void rank16_leave_bounds(float* scale, uint32_t c2max, const float* part_norms, uint32_t k, uint32_t kp)
+{
+	if (threadIdx.x >= WAVE) return;
+	uint32_t mid = 0, rest = 0; /* (bit patterns: NaN and infinity win) */
+	for (uint32_t j = threadIdx.x; j < k; j += WAVE) {
+		mid = max(mid, __float_as_uint(part_norms[kp + j]));
+		rest = max(rest, __float_as_uint(part_norms[2 * kp + j]));
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) {
+		mid = max(mid, (uint32_t)__shfl_xor((int)mid, off));
+		rest = max(rest, (uint32_t)__shfl_xor((int)rest, off));
+	}
+	if (threadIdx.x == 0) { scale[2] = __uint_as_float(c2max); scale[3] = __uint_as_float(mid); scale[4] = __uint_as_float(rest); }
+}
 
 /* the 8 coordinates of a half-wave of block kb as they come from memory, zeros beyond the row. Blocks inside the row (the same
  * for all lanes) are loaded without guards. */
@@ -146,6 +170,7 @@ rank16_kernel(const Rank16Args w)
 			most[q] = 0;
 			for (uint32_t v = 0; v < RANK16_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
 		}
+		if (blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], w.low2, w.k, w.kp);
 		cert = cert_coeffs_level1(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), 0.0f });
 		cert.c2max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(cert.c2max)));
 		cert.a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(cert.a)));

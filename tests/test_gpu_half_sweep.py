@@ -75,7 +75,7 @@ def test_half_precision_products_accumulate_as_the_certificate_assumes(km, gpu, 
     assert (alone == np.float32(2.0 ** -14)).all()             # subnormal operands are not flushed
 
 
-@pytest.mark.parametrize("dim,k,n,mode", [(8, 130, 40001, 1), (50, 300, 70007, 1), (50, 60, 40003, 1), (9, 40, 33000, 1), (256, 129, 33001, 1), (300, 20, 33003, 1), (50, 300, 40000, 0)])
+@pytest.mark.parametrize("dim,k,n,mode", [(8, 130, 40001, 1), (50, 300, 70007, 1), (50, 60, 40003, 1), (9, 40, 33000, 1), (256, 129, 33001, 1), (300, 20, 33003, 1), (50, 300, 40000, 0), (390, 70, 33001, 0)])
 def test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, mode):
     """The assignment's copy of the rows, or the one made ahead of it, is what the update adds up."""
     rng = np.random.default_rng(dim + k)
