@@ -53,7 +53,7 @@ static bool rank16_pays(const AssignArgs& a)
 static bool takes_rank16(const AssignArgs& a, uint32_t lds_budget)
 {
 	const int mode = two_level_mode(); /* kmx_set_two_level_sweep: 0 never, 1 where it pays, 2 wherever the kernels allow it */
-	return a.dim <= 256 && !a.ranking_only && a.two_level && mode != 0 && (mode == 2 || rank16_pays(a)) && rank16_supports(a, lds_budget);
+	return a.dim <= 256 && (!a.ranking_only || a.points64) && a.two_level && mode != 0 && (mode == 2 || rank16_pays(a)) && rank16_supports(a, lds_budget);
 }
 
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
@@ -186,7 +186,7 @@ pack_means_bf16_kernel(const float* __restrict__ means, size_t stride_means, flo
 bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev)
 {
 	const uint32_t kb = pick_kb(a.dim);
-	if (kb == 0) return !a.ranking_only && wide_supports(a, dev);
+	if (kb == 0) return wide_supports(a, dev) && (!a.ranking_only || wide16_supports(a, dev)); /* (the caller's pass over a queue takes no such rows) */
 	/* two tiles (the double-buffered stream of the centroid block) plus the static flag lists must fit */
 	return (size_t)(tile_floats(KBLOCK * kb + ROW_PAD) + NORM_TILE) * 4 * 2 + 2 * FLAG_CAP * MFMA_WAVES * 4 + 1024 <= dev.lds_bytes;
 }

@@ -128,17 +128,17 @@ __host__ __device__ __forceinline__ size_t wide16_scale_offset(uint32_t kp, uint
 static size_t wide16_norms_floats(uint32_t kp, uint32_t dp) { return wide16_scale_offset(kp, dp) + 8; }
 
 /* groups of 32 listed points whose operands fit the LDS of the exact pass (0: none) */
-static uint32_t wide16_groups(uint32_t dp, uint32_t lds_budget)
+static uint32_t wide16_groups(uint32_t dp, bool doubles, uint32_t lds_budget)
 {
 	for (uint32_t groups : { 4u, 2u, 1u })
-		if (exact_dynamic_bytes(dp / KBLOCK, groups) + EXACT_STATIC_BYTES <= lds_budget) return groups;
+		if (exact_dynamic_bytes(dp / KBLOCK, groups) + exact_static_bytes(doubles) <= lds_budget) return groups;
 	return 0;
 }
 
 /* pack_means16_kernel (rank16.hip) for any row length: one wavefront per (padded) centroid row */
 template <int LM>
 __global__ void __launch_bounds__(256)
-pack_means16_wide_kernel(const float* __restrict__ means, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
+pack_means16_wide_kernel(const float* __restrict__ means, const double* __restrict__ means64, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
                          uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters)
 {
 	extern __shared__ float m[]; /* dp floats */
@@ -193,7 +193,8 @@ pack_means16_wide_kernel(const float* __restrict__ means, size_t stride_means, _
 		const float rest = split_bf16(cv, hi, mid);
 		mid2 += (float)mid * (float)mid;
 		rest2 += rest * rest;
-		rows[(size_t)j * dp + q] = exact;
+		if (means64) ((double*)rows)[(size_t)j * dp + q] = there ? means64[elem<LM>(stride_means, j, q)] : 0.0;
+		else rows[(size_t)j * dp + q] = exact;
 		packed[(((size_t)(j / TILE) * (dp / KBLOCK) + q / KBLOCK) * WAVE + (q % KBLOCK) / 8 * TILE + j % TILE) * 8 + q % 8] = half;
 	}
 	for (int off = WAVE / 2; off > 0; off >>= 1) {
@@ -637,7 +638,7 @@ static int check_wide_plan(const AssignArgs& a, const WideArgs& w, const Workspa
 #define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (wide rows): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u)", #cond, a.dim, a.k, w.kp, a.n); } while (0)
 	KMX_PLAN(w.dp % WIDE_CHUNK == 0 && w.dp >= a.dim && w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1);
 	if (half) {
-		KMX_PLAN(ws->packed16 && wide_plane_units(w.kp, w.dp) * 4 + (size_t)w.kp * w.dp <= ws->packed16_cap);
+		KMX_PLAN(ws->packed16 && wide_plane_units(w.kp, w.dp) * 4 + (size_t)w.kp * w.dp * (a.points64 ? 2 : 1) <= ws->packed16_cap);
 		KMX_PLAN(ws->norms16 && wide16_norms_floats(w.kp, w.dp) <= ws->norms16_cap);
 		KMX_PLAN(ws->listed && 2 * (size_t)a.n <= ws->listed_cap && ws->counters);
 		return KMX_OK;
@@ -655,13 +656,13 @@ static int launch_assign_wide16(const AssignArgs& a, uint32_t dp, kmx_exec_param
 {
 	const uint32_t kp = round_up(a.k, TILE);
 	const size_t operand_floats = wide_plane_units(kp, dp) * 4;
-	int rc = reserve_packed16(ws, operand_floats + (size_t)kp * dp, wide16_norms_floats(kp, dp));
+	int rc = reserve_packed16(ws, operand_floats + (size_t)kp * dp * (a.points64 ? 2 : 1), wide16_norms_floats(kp, dp));
 	if (rc) return rc;
 	if ((rc = reserve_listed(ws, 2 * (size_t)a.n))) return rc;
 	float* rows = ws->packed16 + operand_floats;
 	auto pack = a.layout_means == KMX_AOS ? pack_means16_wide_kernel<KMX_AOS> : pack_means16_wide_kernel<KMX_SOA>;
 	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), dp * 4, stream(),
-	                   a.means, a.stride_means, (_Float16*)ws->packed16, rows, ws->norms16, a.dim, a.k, kp, dp, ws->counters);
+	                   a.means, a.means64, a.stride_means, (_Float16*)ws->packed16, rows, ws->norms16, a.dim, a.k, kp, dp, ws->counters);
 	KMX_LAUNCH_CHECK("pack_means16_wide_kernel");
 	const float* norms = ws->norms16;
 	const WideArgs w = { a.data, a.stride, (const bf16x8*)ws->packed16, norms, norms + wide16_part_offset(kp), norms + wide16_frame_offset(kp), ws->norms16 + wide16_scale_offset(kp, dp),
@@ -673,18 +674,31 @@ static int launch_assign_wide16(const AssignArgs& a, uint32_t dp, kmx_exec_param
 	rc = a.n >= 64 * dev.compute_units ? launch_wide_sweep<4, 2, false>(a, w, dev, exec) : launch_wide_sweep<1, 1, false>(a, w, dev, exec);
 	if (rc) return rc;
 	if ((rc = profile_end(0))) return rc;
-	const bool aos = a.layout == KMX_AOS;
-	const ExactArgs e = { a.data, aos ? a.stride : 1, aos ? 1 : a.stride, a.dim, rows, (const f16x8*)ws->packed16, norms,
-	                      norms + wide16_frame_offset(kp), norms + wide16_scale_offset(kp, dp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
-	                      a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, dp / KBLOCK, wide16_groups(dp, lds_budget_of(exec, dev)) };
-	return launch_listed_exact_kb<0>(a, e, dev);
+	const size_t stride = a.layout == KMX_AOS ? a.stride : 1, step = a.layout == KMX_AOS ? 1 : a.stride;
+	const uint32_t groups = wide16_groups(dp, a.points64 != nullptr, dev.lds_bytes);
+	auto exact = [&](auto* points, auto* centroids) -> int {
+		typedef typename std::remove_const<typename std::remove_pointer<decltype(points)>::type>::type F;
+		const ExactArgs<F> e = { a.data, stride, step, a.dim, points, stride, step, a.dim, centroids, (const f16x8*)ws->packed16, norms,
+		                         norms + wide16_frame_offset(kp), norms + wide16_scale_offset(kp, dp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
+		                         a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, dp / KBLOCK, groups };
+		return launch_listed_exact_kb<0, F>(a, e, dev);
+	};
+	rc = a.points64 ? exact(a.points64, (const double*)rows) : exact(a.data, (const float*)rows);
+	if (rc) return rc;
+	if (a.settled) *a.settled = true;
+	return KMX_OK;
+}
+
+bool wide16_supports(const AssignArgs& a, const DeviceInfo& dev)
+{
+	return a.two_level && two_level_mode() != 0 && a.k < (1u << 25) && (!a.ranking_only || a.points64) && wide16_groups(round_up(a.dim, WIDE_CHUNK), a.points64 != nullptr, dev.lds_bytes) > 0;
 }
 
 int launch_assign_wide(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	AssignArgs a = args;
 	const uint32_t dp = round_up(a.dim, WIDE_CHUNK), kp = round_up(a.k, TILE);
-	if (a.two_level && two_level_mode() != 0 && !a.ranking_only && a.k < (1u << 25) && wide16_groups(dp, lds_budget_of(exec, dev)) > 0)
+	if (wide16_supports(a, dev))
 		return launch_assign_wide16(a, dp, exec, ws, dev);
 	const bool moved = !a.ranking_only; /* (the double path hands over copies it has moved itself) */
 	int rc = reserve_packed(ws, wide_plane_units(kp, dp) * 2 * 4, wide_norms_floats(kp, dp), (size_t)kp * a.dim);

@@ -1301,25 +1301,6 @@ extern "C" int kmx_assign_f64(int variant,
 	}
 	const bool float_ranking = variant == KMX_ASSIGN_MFMA || variant == KMX_ASSIGN_MFMA_BF16X3 || variant == KMX_ASSIGN_BEST;
 
-	const uint32_t kp = round_up_u32(k, WIDE_GROUP);
-	rc = reserve_f64(&g_means_t, &g_means_t_cap, (size_t)kp * dim);
-	if (rc) return rc;
-	rc = reserve_f64(&g_norms, &g_norms_cap, kp);
-	if (rc) return rc;
-	rc = reserve_f64(&g_queue, &g_queue_cap, float_ranking ? 1 : (size_t)n / 2 + 1);
-	if (rc) return rc;
-	rc = reserve_f64(&g_misc, &g_misc_cap, 4);
-	if (rc) return rc;
-	unsigned long long* misc = (unsigned long long*)g_misc;
-	KMX_LAUNCH_KERNEL(reset_f64_kernel, dim3(1), dim3(64), 0, stream(), misc);
-	KMX_LAUNCH_CHECK("reset_f64_kernel");
-	const dim3 pgrid((kp + 255) / 256);
-	if (layout_means == KMX_AOS)
-		KMX_LAUNCH_KERNEL(prepare_rows_f64_kernel, dim3((kp + 31) / 32), dim3(256), 0, stream(), means, stride_means, g_means_t, g_norms, misc, dim, k, kp);
-	else
-		KMX_LAUNCH_KERNEL((prepare_means_f64_kernel<KMX_SOA>), pgrid, dim3(256), 0, stream(), means, stride_means, g_means_t, g_norms, misc, dim, k, kp);
-	KMX_LAUNCH_CHECK("prepare_means_f64_kernel");
-
 	const uint32_t* float_queue = nullptr;
 	const uint32_t* float_queue_length = nullptr;
 	if (float_ranking) {
@@ -1345,9 +1326,13 @@ extern "C" int kmx_assign_f64(int variant,
 		AssignArgs a{ (const float*)g_data32, layout, stride, (const float*)g_means32, layout_means, stride_means, assignment, dim, k, n };
 		a.kd_extra = 6.0f * 1.1920929e-07f;
 		a.ranking_only = true;
+		bool settled = false;
+		if (dim <= 256 || variant == KMX_ASSIGN_BEST) { /* (asked for by name, the matrix-core variants take doubles of up to 256 dimensions) */
+			a.points64 = data; a.means64 = means; a.settled = &settled;
+		}
 		int chosen = -1;
 		rc = dispatch_assign(variant, a, exec, ws, *dev, &chosen); /* brackets its sweep for the profile itself */
-		if (rc) return rc;
+		if (rc || settled) return rc;
 		if (chosen == KMX_ASSIGN_BASE) /* no float sweep fits the shape: evaluate everything on the doubles */
 			variant = KMX_ASSIGN_BASE;
 		else {
@@ -1355,6 +1340,25 @@ extern "C" int kmx_assign_f64(int variant,
 			float_queue_length = ws->counters;
 		}
 	}
+
+	const uint32_t kp = round_up_u32(k, WIDE_GROUP);
+	rc = reserve_f64(&g_means_t, &g_means_t_cap, (size_t)kp * dim);
+	if (rc) return rc;
+	rc = reserve_f64(&g_norms, &g_norms_cap, kp);
+	if (rc) return rc;
+	rc = reserve_f64(&g_queue, &g_queue_cap, float_ranking ? 1 : (size_t)n / 2 + 1);
+	if (rc) return rc;
+	rc = reserve_f64(&g_misc, &g_misc_cap, 4);
+	if (rc) return rc;
+	unsigned long long* misc = (unsigned long long*)g_misc;
+	KMX_LAUNCH_KERNEL(reset_f64_kernel, dim3(1), dim3(64), 0, stream(), misc);
+	KMX_LAUNCH_CHECK("reset_f64_kernel");
+	const dim3 pgrid((kp + 255) / 256);
+	if (layout_means == KMX_AOS)
+		KMX_LAUNCH_KERNEL(prepare_rows_f64_kernel, dim3((kp + 31) / 32), dim3(256), 0, stream(), means, stride_means, g_means_t, g_norms, misc, dim, k, kp);
+	else
+		KMX_LAUNCH_KERNEL((prepare_means_f64_kernel<KMX_SOA>), pgrid, dim3(256), 0, stream(), means, stride_means, g_means_t, g_norms, misc, dim, k, kp);
+	KMX_LAUNCH_CHECK("prepare_means_f64_kernel");
 
 	if (!float_queue) {
 		rc = profile_begin(0);

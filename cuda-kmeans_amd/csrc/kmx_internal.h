@@ -141,6 +141,9 @@ struct AssignArgs {
 	bool two_level = true;
 	/* the single-pass fused kernel: write the result of every point to `assignment`, not only those of the exact pass */
 	bool emit_assignment = false;
+	/* ranking_only: the doubles behind the float copies (layouts and strides of the copies). A sweep whose exact pass takes doubles leaves
+	 * nothing to the caller and says so in *settled. */
+	const double* points64 = nullptr; const double* means64 = nullptr; bool* settled = nullptr;
 	/* SoA points: filled in by a sweep that wrote all rows as AoS on the way (left alone by the others) */
 	AosRows* rows_out = nullptr;
 };
@@ -188,6 +191,7 @@ bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const D
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */
 bool wide_supports(const AssignArgs& a, const DeviceInfo& dev);
+bool wide16_supports(const AssignArgs& a, const DeviceInfo& dev); /* ... in half precision, nothing left to the caller */
 int launch_assign_wide(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 bool lds_fma_supports(const AssignArgs& a, const DeviceInfo& dev);
 bool lds_fma_reads_through_scalar_cache(const AssignArgs& a); /* a handful of centroids: no LDS staging */

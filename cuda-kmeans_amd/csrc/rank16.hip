@@ -38,7 +38,8 @@ static uint32_t rank16_kb(uint32_t dim)
 #define KMX_DECLARE_RANK16(W) int launch_rank16_##W(const AssignArgs& a, const Rank16Args& w, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 KMX_DECLARE_RANK16(1) KMX_DECLARE_RANK16(2) KMX_DECLARE_RANK16(3) KMX_DECLARE_RANK16(4)
 KMX_DECLARE_RANK16(6) KMX_DECLARE_RANK16(8) KMX_DECLARE_RANK16(12) KMX_DECLARE_RANK16(16)
-#define KMX_DECLARE_EXACT16(W) int launch_listed_exact_##W(const AssignArgs& a, const ExactArgs& w, const DeviceInfo& dev);
+#define KMX_DECLARE_EXACT16(W) int launch_listed_exact_##W(const AssignArgs& a, const ExactArgs<float>& w, const DeviceInfo& dev); \
+	int launch_listed_exact_##W(const AssignArgs& a, const ExactArgs<double>& w, const DeviceInfo& dev);
 KMX_DECLARE_EXACT16(1) KMX_DECLARE_EXACT16(2) KMX_DECLARE_EXACT16(3) KMX_DECLARE_EXACT16(4)
 KMX_DECLARE_EXACT16(6) KMX_DECLARE_EXACT16(8) KMX_DECLARE_EXACT16(12) KMX_DECLARE_EXACT16(16)
 
@@ -55,8 +56,8 @@ static size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) 
 
 template <int LM>
 __global__ void __launch_bounds__(256)
-pack_means16_kernel(const float* __restrict__ means, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
-                    uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t moved, uint32_t* __restrict__ counters)
+pack_means16_kernel(const float* __restrict__ means, const double* __restrict__ means64, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
+                    uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters)
 {
 	__shared__ float frame[FRAME_DIMS];
 	__shared__ float wave_far[4];
@@ -70,7 +71,7 @@ pack_means16_kernel(const float* __restrict__ means, size_t stride_means, _Float
 		const uint32_t q = lane + i * WAVE;
 		exact[i] = (j < k && q < dim) ? means[elem<LM>(stride_means, j, q)] : 0.0f;
 	}
-	sweep_frame<LM>(means, stride_means, dim, k, dp, moved ? FRAME_MOVED : FRAME_KEPT, frame, norms + rank16_frame_offset(kp));
+	sweep_frame<LM>(means, stride_means, dim, k, dp, FRAME_MOVED, frame, norms + rank16_frame_offset(kp));
 	float far = 0.0f;
 	for (uint32_t q = threadIdx.x; q < dim; q += 256) {
 		float v[16];
@@ -107,7 +108,8 @@ pack_means16_kernel(const float* __restrict__ means, size_t stride_means, _Float
 		const float rest = split_bf16(cv, hi, mid);
 		mid2 += (float)mid * (float)mid;
 		rest2 += rest * rest;
-		rows[(size_t)j * dp + q] = exact[i];
+		if (means64) ((double*)rows)[(size_t)j * dp + q] = (j < k && q < dim) ? means64[elem<LM>(stride_means, j, q)] : 0.0;
+		else rows[(size_t)j * dp + q] = exact[i];
 		packed[(((size_t)(j / TILE) * (dp / KBLOCK) + q / KBLOCK) * WAVE + (q % KBLOCK) / 8 * TILE + j % TILE) * 8 + q % 8] = half;
 	}
 	for (int off = WAVE / 2; off > 0; off >>= 1) {
@@ -130,18 +132,18 @@ bool rank16_supports(const AssignArgs& a, uint32_t lds_budget)
 	const uint32_t kb = rank16_kb(a.dim);
 	if (a.dim <= 4 || kb == 0 || a.k >= (1u << 25) || a.n > (1u << 31)) return false;
 	const uint32_t sweep = (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + kb * KBLOCK) * 4 + 64 + 2 * (kb * WAVE * 4 + NORM_TILE) * 4; /* two tiles */
-	return sweep <= lds_budget && exact_dynamic_bytes(kb, EXACT_GROUPS) + EXACT_STATIC_BYTES <= lds_budget;
+	return sweep <= lds_budget && exact_dynamic_bytes(kb, EXACT_GROUPS) + exact_static_bytes(a.points64 != nullptr) <= lds_budget;
 }
 
 /* the centroids for launch_rank16_sweep */
 static int launch_pack16(const AssignArgs& a, Workspace* ws)
 {
 	const uint32_t dp = rank16_kb(a.dim) * KBLOCK, kp = round_up(a.k, TILE);
-	const int rc = reserve_packed16(ws, rank16_rows_offset(kp, dp) + (size_t)kp * dp, rank16_norms_floats(kp));
+	const int rc = reserve_packed16(ws, rank16_rows_offset(kp, dp) + (size_t)kp * dp * (a.points64 ? 2 : 1), rank16_norms_floats(kp));
 	if (rc) return rc;
 	auto pack = a.layout_means == KMX_AOS ? pack_means16_kernel<KMX_AOS> : pack_means16_kernel<KMX_SOA>;
 	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), 0, stream(),
-	                   a.means, a.stride_means, (_Float16*)ws->packed16, ws->packed16 + rank16_rows_offset(kp, dp), ws->norms16, a.dim, a.k, kp, dp, a.ranking_only ? 0u : 1u, ws->counters);
+	                   a.means, a.means64, a.stride_means, (_Float16*)ws->packed16, ws->packed16 + rank16_rows_offset(kp, dp), ws->norms16, a.dim, a.k, kp, dp, ws->counters);
 	KMX_LAUNCH_CHECK("pack_means16_kernel");
 	return KMX_OK;
 }
@@ -156,7 +158,7 @@ static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Works
 	const float* norms = ws->norms16;
 	const Rank16Args w = { a.data, a.stride, (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp), norms + rank16_frame_offset(kp), ws->norms16 + rank16_scale_offset(kp),
 	                       a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->queued_rows, copy_stride, a.dim, a.k, kp, a.n, 0,
-	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + (a.ranking_only ? 0.0f : 8.0f * CERT_UNIT) + a.kd_extra };
+	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + 8.0f * CERT_UNIT + a.kd_extra };
 	switch (kb) {
 	case 1: return launch_rank16_1(a, w, exec, ws, dev);
 	case 2: return launch_rank16_2(a, w, exec, ws, dev);
@@ -170,17 +172,18 @@ static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Works
 	}
 }
 
-/* the serial result for the points in ws->listed, after launch_rank16_sweep */
-static int launch_listed_exact(const AssignArgs& a, Workspace* ws, const DeviceInfo& dev)
+/* the serial result for the points in ws->listed, after launch_rank16_sweep; F: what the serial arithmetic is done in */
+template <typename F>
+static int launch_listed_exact(const AssignArgs& a, const F* points, size_t points_stride, size_t points_step, uint32_t points_dim, Workspace* ws, const DeviceInfo& dev)
 {
 	const uint32_t kb = rank16_kb(a.dim), dp = kb * KBLOCK, kp = round_up(a.k, TILE);
 	const float* norms = ws->norms16;
 	const bool aos = a.layout == KMX_AOS;
 	const uint32_t row_dim = aos ? a.dim : round_up(a.dim, 8);
-	const ExactArgs w = { aos ? a.data : ws->queued_rows, aos ? a.stride : row_dim, 1, row_dim,
-	                      ws->packed16 + rank16_rows_offset(kp, dp), (const f16x8*)ws->packed16, norms,
-	                      norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
-	                      a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, kb, EXACT_GROUPS };
+	const ExactArgs<F> w = { aos ? a.data : ws->queued_rows, aos ? a.stride : row_dim, 1, row_dim, points, points_stride, points_step, points_dim,
+	                         (const F*)(ws->packed16 + rank16_rows_offset(kp, dp)), (const f16x8*)ws->packed16, norms,
+	                         norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
+	                         a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, kb, EXACT_GROUPS };
 	switch (kb) {
 	case 1: return launch_listed_exact_1(a, w, dev);
 	case 2: return launch_listed_exact_2(a, w, dev);
@@ -215,8 +218,13 @@ int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 		if (first == 0 && (rc = profile_begin(0))) return rc;
 		if ((rc = launch_rank16_sweep(p, exec, ws, dev))) return rc;
 		if (first == 0 && (rc = profile_end(0))) return rc;
-		if ((rc = launch_listed_exact(p, ws, dev))) return rc;
+		const bool aos = a.layout == KMX_AOS;
+		if (a.points64) rc = launch_listed_exact<double>(p, a.points64 + first, aos ? a.stride : 1, aos ? 1 : a.stride, a.dim, ws, dev);
+		else if (aos) rc = launch_listed_exact<float>(p, p.data, p.stride, 1, p.dim, ws, dev);
+		else rc = launch_listed_exact<float>(p, ws->queued_rows, round_up(a.dim, 8), 1, round_up(a.dim, 8), ws, dev);
+		if (rc) return rc;
 	}
+	if (a.settled) *a.settled = true;
 	if (a.rows_out && a.layout == KMX_SOA && part == a.n) *a.rows_out = AosRows{ ws->queued_rows, round_up(a.dim, 8) };
 	return KMX_OK;
 }

@@ -14,22 +14,59 @@ constexpr uint32_t EXACT_WAVES = EXACT_THREADS / WAVE;
 constexpr uint32_t EXACT_GROUPS = 4;                       /* most groups of 32 points per unit */
 constexpr uint32_t EXACT_ROWS = EXACT_GROUPS * TILE;
 constexpr uint32_t EXACT_HITS = 256;                       /* pairs per wavefront and unit that wait for the common evaluation */
-constexpr uint32_t EXACT_PAIR_FLOATS = KBLOCK + 4;         /* a pair's squares of one block of 16 dimensions; the padding spreads 16 lanes' reads over all banks */
-constexpr uint32_t EXACT_SQUARES = EXACT_WAVES * WAVE * EXACT_PAIR_FLOATS;
+constexpr uint32_t EXACT_SQUARES_BYTES = EXACT_WAVES * WAVE * (KBLOCK + 4) * 4; /* (doubles: half as many pairs) */
+constexpr uint32_t exact_static_bytes(bool doubles)
+{
+	return (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + EXACT_WAVES) * 4 + 96 + (doubles ? EXACT_WAVES * EXACT_HITS * 8 + 2 * EXACT_ROWS * 4 : 0);
+}
 
-constexpr uint32_t EXACT_STATIC_BYTES = (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + EXACT_WAVES) * 4 + 64;
-
+template <typename F>
 struct ExactArgs {
 	/* coordinate d of point p: data[p * stride + d * step]; step 1: rows of row_dim coordinates (zeros behind the first dim). Other
 	 * steps (SoA points) are for KB = 0 only. */
 	const float* data; size_t stride, step; uint32_t row_dim;
-	const float* means;                     /* rows of KB * 16 floats, zeros behind the coordinates */
+	/* the same of the points the serial arithmetic is for (doubles: data is their float copy) */
+	const F* points; size_t points_stride, points_step; uint32_t points_dim;
+	const F* means;                         /* rows of KB * 16 values, zeros behind the coordinates */
 	const f16x8* packed; const float* norms; const float* frame; const float* scale;
 	uint32_t* assignment; const uint32_t* list; const uint32_t* length; uint32_t* undecided;
 	uint32_t dim, k, kp;
 	float kd_split;
 	uint32_t blocks, most_groups; /* KB = 0: blocks of 16 dimensions per row; groups whose operands fit LDS */
 };
+
+/* four coordinates of a row at its coordinate d, as they come from memory: d brought inside the row (row_dim >= 4), or, strided, zeros beyond it */
+template <typename F>
+__device__ __forceinline__ void exact_request(F __attribute__((ext_vector_type(4)))& v, const F* src, uint32_t d, uint32_t dim, uint32_t row_dim, size_t step, bool strided)
+{
+	typedef F F4_any __attribute__((ext_vector_type(4), aligned(sizeof(F))));
+	if (strided) {
+#pragma unroll
+		for (uint32_t e = 0; e < 4; ++e) v[e] = d + e < dim ? src[(size_t)(d + e) * step] : (F)0;
+	}
+	else v = *(const F4_any*)(src + min(d, row_dim - 4));
+}
+
+/* ... and in their places, zeros beyond the row (masks: the compiler makes branches of selections) */
+template <typename F>
+__device__ __forceinline__ void exact_place(F __attribute__((ext_vector_type(4)))& v, uint32_t d, uint32_t row_dim)
+{
+	typedef typename std::conditional<sizeof(F) == 8, unsigned long long, uint32_t>::type bits_t;
+	const uint32_t shift = d + 4 > row_dim ? d + 4 - row_dim : 0;
+	const bits_t m0 = (bits_t)0 - (bits_t)(shift == 0), m1 = (bits_t)0 - (bits_t)(shift == 1), m2 = (bits_t)0 - (bits_t)(shift == 2), m3 = (bits_t)0 - (bits_t)(shift == 3);
+	const bits_t x = __builtin_bit_cast(bits_t, (F)v.x), y = __builtin_bit_cast(bits_t, (F)v.y), z = __builtin_bit_cast(bits_t, (F)v.z), t = __builtin_bit_cast(bits_t, (F)v.w);
+	v.x = __builtin_bit_cast(F, (x & m0) | (y & m1) | (z & m2) | (t & m3));
+	v.y = __builtin_bit_cast(F, (y & m0) | (z & m1) | (t & m2));
+	v.z = __builtin_bit_cast(F, (z & m0) | (t & m1));
+	v.w = __builtin_bit_cast(F, t & m0);
+}
+
+/* doubles: the bits of a serial distance as they are compared, like exact_key without the centroid */
+__device__ __forceinline__ unsigned long long exact_bits(double sum, uint32_t c)
+{
+	const double dist = __builtin_sqrt(sum);
+	return (c == 0 && dist != dist) ? 0ull : (unsigned long long)__double_as_longlong(dist);
+}
 
 __device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
 {
@@ -48,13 +85,14 @@ __device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
  *      bytes each of point and centroid and square the differences (64 consecutive bytes per row: a lane of its own per row would
  *      touch 64 lines per load), the squares go through LDS to the pair's lane, which adds them in order. The results merge into
  *      the point's two smallest keys (distance bits << 32 | centroid, see evaluate_pair) in LDS.
+ * F: the type of the serial arithmetic; doubles are ranked by float copies.
  * A wavefront whose list fills up (data that the thresholds tell nothing about) evaluates it on the spot, one lane per pair.
  *
  * counters[0] receives the number of points whose two smallest serial distances are closer than the three-product certificate.
  */
-template <int KB>
+template <int KB, typename F>
 __global__ void __launch_bounds__(EXACT_THREADS, 4)
-listed_exact_kernel(const ExactArgs w)
+listed_exact_kernel(const ExactArgs<F> w)
 {
 	const uint32_t blocks = KB ? KB : w.blocks, DP = blocks * KBLOCK;
 	extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -64,6 +102,12 @@ listed_exact_kernel(const ExactArgs w)
 	__shared__ uint32_t point[EXACT_ROWS];
 	__shared__ uint32_t hits[EXACT_WAVES][EXACT_HITS];          /* row << 25 | centroid (supports: k < 2^25) */
 	__shared__ uint32_t noted_by[EXACT_WAVES];
+	constexpr bool DOUBLES = sizeof(F) == 8; /* keys of 96 bits: the smallest distances first, then who has them */
+	__shared__ unsigned long long pair_bits[DOUBLES ? EXACT_WAVES * EXACT_HITS : 1];
+	__shared__ uint32_t winner[DOUBLES ? EXACT_ROWS : 1], redo[DOUBLES ? EXACT_ROWS : 1];
+	constexpr uint32_t PASS = DOUBLES ? 32 : 64; /* pairs a wavefront evaluates at a time */
+	typedef F F4 __attribute__((ext_vector_type(4)));
+	constexpr uint32_t PAIR = KBLOCK + 16 / sizeof(F); /* a pair's squares of a block in LDS; the padding spreads 16 lanes' reads over all banks */
 	constexpr uint32_t CENTROID = (1u << 25) - 1u;
 	const uint32_t count = w.length[0];
 	if (count == 0) return;
@@ -77,31 +121,15 @@ listed_exact_kernel(const ExactArgs w)
 	const float scale = w.scale[0], unscale = w.scale[1];
 	const uint32_t tiles = w.kp / TILE;
 	const bool strided = KB == 0 && w.step != 1, ragged = w.row_dim < DP && !strided;
+	const bool points_strided = (KB == 0 || DOUBLES) && w.points_step != 1, points_ragged = w.points_dim < DP && !points_strided;
 
 	/* of the three-product ranking: only what is counted depends on it (the sweep left the maxima behind the scale) */
 	const CertCoeffs cert = cert_coeffs_split(CentroidBounds{ w.scale[2], w.scale[3], w.scale[4] });
 
-	/* four coordinates of a row at its coordinate d, as they come from memory (d brought inside the row) ... */
+	/* four coordinates of a row at its coordinate d, as they come from memory (d brought inside the row), see exact_place */
 	auto source = [&](uint32_t row) -> const float* { return w.data + (size_t)point[row] * w.stride; };
-	auto request = [&](f32x4& v, const float* src, uint32_t d) {
-		typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-		if (strided) {
-#pragma unroll
-			for (uint32_t e = 0; e < 4; ++e) v[e] = d + e < w.dim ? src[(size_t)(d + e) * w.step] : 0.0f;
-		}
-		else v = *(const f32x4_any*)(src + min(d, w.row_dim - 4));
-	};
-	/* ... and in their places, zeros beyond the row */
-	auto place = [&](f32x4& v, uint32_t d) {
-		/* (masks: the compiler makes branches of the selections) */
-		const uint32_t shift = d + 4 > w.row_dim ? d + 4 - w.row_dim : 0;
-		const uint32_t m0 = 0u - (uint32_t)(shift == 0), m1 = 0u - (uint32_t)(shift == 1), m2 = 0u - (uint32_t)(shift == 2), m3 = 0u - (uint32_t)(shift == 3);
-		const uint32_t x = __float_as_uint(v.x), y = __float_as_uint(v.y), z = __float_as_uint(v.z), t = __float_as_uint(v.w);
-		v.x = __uint_as_float((x & m0) | (y & m1) | (z & m2) | (t & m3));
-		v.y = __uint_as_float((y & m0) | (z & m1) | (t & m2));
-		v.z = __uint_as_float((z & m0) | (t & m1));
-		v.w = __uint_as_float(t & m0);
-	};
+	auto serial_source = [&](uint32_t row) -> const F* { return w.points + (size_t)point[row] * w.points_stride; };
+	auto request = [&](f32x4& v, const float* src, uint32_t d) { exact_request<float>(v, src, d, w.dim, w.row_dim, w.step, strided); };
 	uint32_t close_here = 0;
 	for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
 		const uint32_t first = unit * unit_rows;
@@ -111,6 +139,7 @@ listed_exact_kernel(const ExactArgs w)
 			point[tid] = w.list[2 * (size_t)e];
 			threshold[tid] = first + tid < count ? __uint_as_float(w.list[2 * (size_t)e + 1]) : -__builtin_inff(); /* rows beyond the list pass nothing */
 			best[tid] = ~0ull;
+			if constexpr (DOUBLES) { winner[tid] = ~0u; redo[tid] = 0u; }
 			second[tid] = ~0ull;
 		}
 		__syncthreads();
@@ -132,7 +161,7 @@ listed_exact_kernel(const ExactArgs w)
 				for (int i = 0; i < 4; ++i) {
 					const uint32_t d = (f0 + i * lanes) * 4;
 					if (d >= DP) break;
-					if (ragged) place(v[i], d);
+					if (ragged) exact_place<float>(v[i], d, w.row_dim);
 					const f32x4 m = *(const f32x4*)(w.frame + d);
 					typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 					f16x4 half;
@@ -154,27 +183,40 @@ listed_exact_kernel(const ExactArgs w)
 		}
 		__syncthreads();
 
-		auto merge = [&](uint32_t row, unsigned long long key) {
-			const unsigned long long before = atomicMin(&best[row], key);
-			atomicMin(&second[row], before < key ? key : before);
+		/* the serial sum of a point and a centroid, by one lane */
+		auto serial_sum = [&](uint32_t row, uint32_t c) -> F {
+#pragma clang fp contract(off)
+			const F* src = serial_source(row);
+			const F* mean = w.means + (size_t)c * DP;
+			F sum = (F)0;
+#pragma unroll 1
+			for (uint32_t d = 0; d < w.dim; ++d) {
+				const F diff = src[points_strided ? (size_t)d * w.points_step : (size_t)d] - mean[d];
+				const F sq = diff * diff;
+				sum = sum + sq;
+			}
+			return sum;
+		};
+		/* doubles: who has the smallest distance is settled when it is known (in_list), or by another look at all centroids (redo) */
+		auto merge = [&](uint32_t row, uint32_t c, F sum, uint32_t in_list) {
+			if constexpr (DOUBLES) {
+				const unsigned long long bits = exact_bits(sum, c);
+				atomicMin(&best[row], bits);
+				if (in_list == ~0u) redo[row] = 1u;
+				else pair_bits[in_list] = bits;
+			}
+			else {
+				const unsigned long long key = exact_key(sum, c), before = atomicMin(&best[row], key);
+				atomicMin(&second[row], before < key ? key : before);
+			}
 		};
 		uint32_t noted = 0; /* wave-uniform */
 		auto evaluate_alone = [&]() {
-#pragma clang fp contract(off)
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 			__builtin_amdgcn_wave_barrier();
 			for (uint32_t i = lane; i < noted; i += WAVE) {
 				const uint32_t hit = hits[wave][i], row = hit >> 25, c = hit & CENTROID;
-				const float* src = source(row);
-				const float* mean = w.means + (size_t)c * DP;
-				float sum = 0.0f;
-#pragma unroll 1
-				for (uint32_t d = 0; d < w.dim; ++d) {
-					const float diff = src[strided ? (size_t)d * w.step : (size_t)d] - mean[d];
-					const float sq = diff * diff;
-					sum = sum + sq;
-				}
-				merge(row, exact_key(sum, c));
+				merge(row, c, serial_sum(row, c), ~0u);
 			}
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 			__builtin_amdgcn_wave_barrier();
@@ -267,34 +309,37 @@ listed_exact_kernel(const ExactArgs w)
 			uint32_t total = 0;
 #pragma unroll
 			for (uint32_t v = 0; v < EXACT_WAVES; ++v) total += noted_by[v];
+			auto pair_of = [&](uint32_t at) -> uint32_t { /* pair `at` of all the lists */
+				uint32_t list = 0;
+				while (at >= noted_by[list]) at -= noted_by[list++];
+				return hits[list][at];
+			};
 			/* equal shares of the pairs, in groups of 16 */
 			const uint32_t share = ((total + 15) / 16 + EXACT_WAVES - 1) / EXACT_WAVES * 16;
 			const uint32_t end = min((wave + 1) * share, total);
-			float* squares = lds + wave * (WAVE * EXACT_PAIR_FLOATS);
+			F* squares = (F*)lds + wave * (PASS * PAIR);
 #pragma unroll 1
-			for (uint32_t p0 = wave * share; p0 < end; p0 += WAVE) {
-				/* this lane's pair (the last one again behind the end), and the four it fetches for */
-				uint32_t at = min(p0 + lane, end - 1), list = 0;
-				while (at >= noted_by[list]) at -= noted_by[list++];
-				const uint32_t hit = hits[list][at];
-				float sum = 0.0f;
+			for (uint32_t p0 = wave * share; p0 < end; p0 += PASS) {
+				/* this lane's pair (the last one again behind the end), and those it fetches for */
+				const uint32_t hit = pair_of(min(p0 + lane % PASS, end - 1));
+				F sum = (F)0;
 				/* GROUPS of 16 pairs (those beyond the last repeat it), DEPTH blocks on their way while one is squared and added */
 				auto evaluate = [&](auto groups_tag, auto depth_tag) {
 					constexpr uint32_t GROUPS = decltype(groups_tag)::value, DEPTH = decltype(depth_tag)::value;
-					const float* x[GROUPS]; const float* m[GROUPS];
+					const F* x[GROUPS]; const F* m[GROUPS];
 #pragma unroll
 					for (uint32_t g = 0; g < GROUPS; ++g) {
 						const uint32_t other = (uint32_t)__shfl((int)hit, (int)(16 * g + lane / 4));
-						x[g] = source(other >> 25);
+						x[g] = serial_source(other >> 25);
 						m[g] = w.means + (size_t)(other & CENTROID) * DP + lane % 4 * 4;
 					}
-					f32x4 xv[DEPTH][GROUPS], mv[DEPTH][GROUPS];
+					F4 xv[DEPTH][GROUPS], mv[DEPTH][GROUPS];
 					auto fetch = [&](uint32_t u, uint32_t kb) {
 						kb = min(kb, blocks - 1);
 #pragma unroll
 						for (uint32_t g = 0; g < GROUPS; ++g) {
-							request(xv[u][g], x[g], kb * KBLOCK + lane % 4 * 4);
-							mv[u][g] = *(const f32x4*)(m[g] + kb * KBLOCK);
+							exact_request<F>(xv[u][g], x[g], kb * KBLOCK + lane % 4 * 4, w.dim, w.points_dim, w.points_step, points_strided);
+							mv[u][g] = *(const F4*)(m[g] + kb * KBLOCK);
 						}
 					};
 #pragma unroll
@@ -305,27 +350,27 @@ listed_exact_kernel(const ExactArgs w)
 						for (uint32_t u = 0; u < DEPTH; ++u) {
 							const uint32_t kb = kb0 + u;
 							if (DEPTH > 1 && kb >= blocks) break;
-							if (ragged && (kb + 1) * KBLOCK > w.row_dim) {
+							if (points_ragged && (kb + 1) * KBLOCK > w.points_dim) {
 #pragma unroll
-								for (uint32_t g = 0; g < GROUPS; ++g) place(xv[u][g], kb * KBLOCK + lane % 4 * 4);
+								for (uint32_t g = 0; g < GROUPS; ++g) exact_place<F>(xv[u][g], kb * KBLOCK + lane % 4 * 4, w.points_dim);
 							}
 #pragma unroll
 							for (uint32_t g = 0; g < GROUPS; ++g) {
-								f32x4 sq;
+								F4 sq;
 #pragma unroll
 								for (int e = 0; e < 4; ++e) {
-									const float diff = xv[u][g][e] - mv[u][g][e];
+									const F diff = xv[u][g][e] - mv[u][g][e];
 									sq[e] = diff * diff;
 								}
-								*(f32x4*)(squares + (16 * g + lane / 4) * EXACT_PAIR_FLOATS + lane % 4 * 4) = sq;
+								*(F4*)(squares + (16 * g + lane / 4) * PAIR + lane % 4 * 4) = sq;
 							}
 							fetch(u, kb + DEPTH);
 							__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 							__builtin_amdgcn_wave_barrier();
-							const float* mine = squares + (GROUPS == 4 ? lane : lane % 16) * EXACT_PAIR_FLOATS;
-							f32x4 s[4];
+							const F* mine = squares + lane % (16 * GROUPS) * PAIR;
+							F4 s[4];
 #pragma unroll
-							for (int q = 0; q < 4; ++q) s[q] = *(const f32x4*)(mine + 4 * q);
+							for (int q = 0; q < 4; ++q) s[q] = *(const F4*)(mine + 4 * q);
 #pragma unroll
 							for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -335,17 +380,40 @@ listed_exact_kernel(const ExactArgs w)
 						}
 					}
 				};
-				if (end - p0 <= 16) evaluate(std::integral_constant<uint32_t, 1>{}, std::integral_constant<uint32_t, 4>{});
-				else evaluate(std::integral_constant<uint32_t, 4>{}, std::integral_constant<uint32_t, 1>{});
-				if (p0 + lane < end) merge(hit >> 25, exact_key(sum, hit & CENTROID));
+				if (end - p0 <= 16) evaluate(std::integral_constant<uint32_t, 1>{}, std::integral_constant<uint32_t, DOUBLES ? 2 : 4>{});
+				else evaluate(std::integral_constant<uint32_t, PASS / 16>{}, std::integral_constant<uint32_t, 1>{});
+				if (lane < PASS && p0 + lane < end) merge(hit >> 25, hit & CENTROID, sum, p0 + lane);
+			}
+			if constexpr (DOUBLES) {
+				__syncthreads();
+				auto settle = [&](uint32_t row, uint32_t c, unsigned long long bits) {
+					if (bits != best[row]) atomicMin(&second[row], bits);
+					else if (atomicMin(&winner[row], c) != ~0u) atomicMin(&second[row], bits);
+				};
+				for (uint32_t i = tid; i < total; i += EXACT_THREADS) {
+					const uint32_t hit = pair_of(i), row = hit >> 25;
+					if (!redo[row]) settle(row, hit & CENTROID, pair_bits[i]);
+				}
+				for (uint32_t row = wave; row < unit_rows; row += EXACT_WAVES)
+					if (redo[row])
+						for (uint32_t c = lane; c < w.k; c += WAVE) settle(row, c, exact_bits(serial_sum(row, c), c));
 			}
 		}
 		__syncthreads();
 		if (tid < unit_rows && first + tid < count) {
 			const unsigned long long key = best[tid], next = second[tid];
-			w.assignment[point[tid]] = key == ~0ull ? 0u : (uint32_t)key;
-			const float d1 = __uint_as_float((uint32_t)(key >> 32)), d2 = __uint_as_float((uint32_t)(next >> 32));
-			if (next != ~0ull && !((d2 * d2 - d1 * d1) / unscale > tau3[tid])) ++close_here;
+			uint32_t c;
+			double d1, d2;
+			if constexpr (DOUBLES) {
+				c = winner[tid];
+				d1 = __longlong_as_double((long long)key); d2 = __longlong_as_double((long long)next);
+			}
+			else {
+				c = (uint32_t)key;
+				d1 = __uint_as_float((uint32_t)(key >> 32)); d2 = __uint_as_float((uint32_t)(next >> 32));
+			}
+			w.assignment[point[tid]] = key == ~0ull ? 0u : c;
+			if (next != ~0ull && !((float)(d2 * d2 - d1 * d1) / unscale > tau3[tid])) ++close_here;
 		}
 	}
 	if (wave < EXACT_ROWS / WAVE) {
@@ -355,12 +423,12 @@ listed_exact_kernel(const ExactArgs w)
 }
 
 /* operands of the groups; the squares take their place */
-constexpr uint32_t exact_dynamic_bytes(uint32_t blocks, uint32_t groups) { return std::max<uint32_t>(groups * blocks * WAVE * 16, EXACT_SQUARES * 4); }
+constexpr uint32_t exact_dynamic_bytes(uint32_t blocks, uint32_t groups) { return std::max<uint32_t>(groups * blocks * WAVE * 16, EXACT_SQUARES_BYTES); }
 
-template <int KB>
-static int launch_listed_exact_kb(const AssignArgs& a, const ExactArgs& w, const DeviceInfo& dev)
+template <int KB, typename F>
+static int launch_listed_exact_kb(const AssignArgs& a, const ExactArgs<F>& w, const DeviceInfo& dev)
 {
-	void (*kernel)(ExactArgs) = listed_exact_kernel<KB>;
+	void (*kernel)(ExactArgs<F>) = listed_exact_kernel<KB, F>;
 	const uint32_t lds = exact_dynamic_bytes(KB ? KB : w.blocks, w.most_groups);
 	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 	const uint32_t grid = std::min<uint32_t>((a.n + TILE - 1) / TILE, 2 * dev.compute_units);

@@ -15,9 +15,14 @@ int KMX_CAT(launch_rank16_, KMX_KB)(const AssignArgs& a, const Rank16Args& w, km
 	return launch_rank16_kb<KMX_KB>(a, w, exec, ws, dev);
 }
 
-int KMX_CAT(launch_listed_exact_, KMX_KB)(const AssignArgs& a, const ExactArgs& w, const DeviceInfo& dev)
+int KMX_CAT(launch_listed_exact_, KMX_KB)(const AssignArgs& a, const ExactArgs<float>& w, const DeviceInfo& dev)
 {
-	return launch_listed_exact_kb<KMX_KB>(a, w, dev);
+	return launch_listed_exact_kb<KMX_KB, float>(a, w, dev);
+}
+
+int KMX_CAT(launch_listed_exact_, KMX_KB)(const AssignArgs& a, const ExactArgs<double>& w, const DeviceInfo& dev)
+{
+	return launch_listed_exact_kb<KMX_KB, double>(a, w, dev);
 }
 
 } // namespace kmx
