@@ -53,7 +53,7 @@ static bool rank16_pays(const AssignArgs& a)
 static bool takes_rank16(const AssignArgs& a, uint32_t lds_budget)
 {
 	const int mode = two_level_mode(); /* kmx_set_two_level_sweep: 0 never, 1 where it pays, 2 wherever the kernels allow it */
-	return a.dim <= 256 && (!a.ranking_only || a.points64) && a.two_level && mode != 0 && (mode == 2 || rank16_pays(a)) && rank16_supports(a, lds_budget);
+	return a.dim <= 256 && (!a.ranking_only || a.points64) && mode != 0 && (mode == 2 || rank16_pays(a)) && rank16_supports(a, lds_budget);
 }
 
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
@@ -84,10 +84,7 @@ pack_means_bf16_kernel(const float* __restrict__ means, size_t stride_means, flo
 {
 	const uint32_t lane = threadIdx.x & (WAVE - 1);
 	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-	if (blockIdx.x == 0 && threadIdx.x == 0) {
-		counters[0] = 0u; /* the recheck queue of this call starts empty */
-		counters[LISTED_COUNTER] = 0u; /* and so does the list of points the first level of a two-level sweep passes on */
-	}
+	if (blockIdx.x == 0 && threadIdx.x == 0) counters[0] = 0u; /* the recheck queue of this call starts empty */
 	/* packed rows: the frame of the sweep, the mean of the first centroids (up to 256 of them, one per lane; the finite
 	 * coordinates; any vector would do, this one is near the middle of the data). Every work-group computes it, in the same order. */
 	__shared__ float frame_parts[4][4];

@@ -14,7 +14,7 @@
  * unit ask the LDS for 64 and the vector cache for 32 of their 128 / 64 bytes per cycle, and all centroids pass by 128 points
  * at a time. The alternatives: PT = 2 doubles the cache traffic (at its limit), NT = 4 does not fit the registers.
  * The rows of a unit are read from memory once while 512 centroids go by; with more centroids the converted rows stay in LDS
- * if they fit (d <= 512 in the first level), otherwise they are staged again per group of 512.
+ * if they fit (d <= 512), otherwise they are staged again per group of 512.
  *
  * N = 131071, d = 512, k = 400, one iteration: the lane-per-point kernel that took these rows before needed 147 ms, two levels of bf16
  * products and a pass over the slices of the queued points (234 us of the assignment) 0.29 ms.
@@ -220,7 +220,7 @@ pack_means16_wide_kernel(const float* __restrict__ means, const double* __restri
  * each block's are replaced by those of the next step as soon as its MFMAs have been issued; the B operands of block b + 1
  * are requested from LDS before the MFMAs of block b. After the step the rows requested a step ago are converted and written to the next
  * buffer, and the chunk after them is requested: every load has a whole step (NT * PT * 4 MFMAs per wavefront, two wavefronts
- * on a SIMD: about a microsecond in the first level) to arrive. Loads retire in order, hence the rows are requested after all of
+ * on a SIMD: about a microsecond) to arrive. Loads retire in order, hence the rows are requested after all of
  * the step's operand loads.
  * Ranking values carry the number of their result (4 or 5 bits) in the lowest mantissa bits, as in the single-pass kernels
  * (cert_kd_keyed): three operations per value for the two smallest and the place of the smallest. A NaN anywhere makes the smallest
@@ -691,7 +691,7 @@ static int launch_assign_wide16(const AssignArgs& a, uint32_t dp, kmx_exec_param
 
 bool wide16_supports(const AssignArgs& a, const DeviceInfo& dev)
 {
-	return a.two_level && two_level_mode() != 0 && a.k < (1u << 25) && (!a.ranking_only || a.points64) && wide16_groups(round_up(a.dim, WIDE_CHUNK), a.points64 != nullptr, dev.lds_bytes) > 0;
+	return two_level_mode() != 0 && a.k < (1u << 25) && (!a.ranking_only || a.points64) && wide16_groups(round_up(a.dim, WIDE_CHUNK), a.points64 != nullptr, dev.lds_bytes) > 0;
 }
 
 int launch_assign_wide(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)

@@ -39,13 +39,13 @@
  *     small for data far from the origin, and the two roundings move a distance by at most 2 u (|x'| + |c'|)^2 <= 2 u' S,
  *     a difference of two distances by 4 u' S: 8 u' more in kd (part of the packed form's kd; the launcher adds it to
  *     the three-product form's when that sweep moves its frame).
- *   - one-product form (the first level of the two-level sweep: hi*hi only, d products and the norm):
+ *   - one-product form (the half-precision sweep, rank16.hip: hi is the half-precision value; d products and the norm):
  *        accumulation <= (d + 2) u' 2 S
  *        dropped = sum_i c'hi_i (x_i - xhi_i) + (c'_i - c'hi_i) x_i <= |c'hi| |xlo| + |c'lo| |x|
- *     with xlo = x - xhi, whose norm the lane computes when it splits the point (the subtraction is exact in fp32),
- *     |c'hi| <= (1 + 2^-8) |c'| and |c'lo| <= |c'mid| + |c'rest| from the packing kernel. The bound is about 2^-8 |c'||x|,
- *     two hundred times the three-product one: this level settles the points whose two nearest centroids are far apart
- *     (86 % at the headline configuration) with a third of the matrix work, the others are swept again with three products.
+ *     with xlo = x - xhi, whose norm the lane computes when it rounds the point (the subtraction is exact in fp32),
+ *     |c'hi| <= (1 + 2^-8) |c'| and |c'lo| from the packing kernel (up to its two arguments). The bound is about
+ *     2^-11 |c'||x|, thirty times the three-product one, for a third of the matrix work: it settles 90 to 99.5 % of the
+ *     points, the others get their serial result.
  * tau = kd S + TRUNC_FACTOR * (bound of the dropped products); kd = (12 d + 8 + 2 d + 12 + slack) u' and
  * (16 d + 8 + 2 d + 12 + 8 + slack) u'; TRUNC_FACTOR = 2 plus 1/16 for the fp32 roundings in the norms and square roots.
  * Values the bound does not cover (NaN, infinities, sums that overflow) make tau NaN or infinite, and the

@@ -341,10 +341,9 @@ int kmx_last_kernel_ms(int which, float* ms);
 int kmx_set_queued_rows_limit(size_t bytes);
 
 /*
- * Where KMX_ASSIGN_MFMA_BF16X3 takes one product per dimension for all points (no counterpart in the reference): rows of up to
- * 256 dimensions in half precision, a third of the matrix work of the three bf16 products, followed by the exact pass for what
- * its wider certificate leaves; wider rows, and the float ranking of double rows, with a second level of three products for
- * those points in between. The results are the same at every setting. mode 0: three products for all points always; 1
+ * Where KMX_ASSIGN_MFMA_BF16X3 takes one product per dimension for all points (no counterpart in the reference): one
+ * product in half precision is a third of the matrix work of the three bf16 products and leaves more points to the exact pass
+ * behind it. The results are the same at every setting. mode 0: three products for all points always; 1
  * (default): one product where it pays (by size, see rank16_pays in csrc/assign_bf16.hip); 2: wherever the kernels allow it
  * (for tests and measurements on small inputs).
  */
@@ -362,7 +361,7 @@ int kmx_set_two_level_sweep(int mode);
  *           number of replaced bits, 4 (up to 16 centroids) or 5
  *   form 1: split-bf16 sweep, three products per dimension         xpart2 = sum_i xmid_i^2
  *   form 2: split-bf16 sweep, packed rows (dim <= 4, four products) xpart2 = sum_i xrest_i^2
- *   form 4: first level of the two-level split-bf16 sweep (one product per dimension, hi * hi) xpart2 = sum_i (x_i - xhi_i)^2
+ *   form 4: half-precision sweep (one product per dimension)       xpart2 = sum_i (x_i - xhi_i)^2
  * x2 = |x|^2, c2max = max_j |c_j|^2, cmid2max / crest2max = max_j of the squared norms of the mid / rest parts of -2 c_j;
  * all of them in the frame the sweep works in: the float sweeps subtract a vector m from points and centroids (the mean
  * of the first 16 centroids; for packed rows, with 128 centroids or more, of the first 256; the single-pass fused kernel
