@@ -56,6 +56,18 @@ static bool takes_rank16(const AssignArgs& a, uint32_t lds_budget)
 	return a.dim <= 256 && (!a.ranking_only || a.points64) && mode != 0 && (mode == 2 || rank16_pays(a)) && rank16_supports(a, lds_budget);
 }
 
+/*
+ * Where the grid of cells (assign_cells.hip) beats the sweeps: its lists take 20 to 55 us to build, so there have to be comparisons to
+ * save (us, sweep -> cells: N = 4M, d = 2: k = 30 61 -> 71, k = 100 126 -> 73, k = 1000 345 -> 75; N = 4M, d = 4: k = 64 79 -> 68, k = 4096
+ * 700 -> 200; N = 500k: d = 3, k = 64 24 -> 38, d = 4, k = 300 44 -> 41; N = 250k, d = 4, k = 128 31 -> 33; N = 30k, k = 4000 65 -> 123).
+ */
+bool takes_cells(const AssignArgs& a, uint32_t lds_budget)
+{
+	const int mode = two_level_mode();
+	const bool pays = a.n >= (1u << 18) && a.k >= 64 && (uint64_t)a.n * a.k >= 150000000u;
+	return a.dim <= 4 && mode != 0 && (mode == 2 || pays) && cells_support(a, lds_budget);
+}
+
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
 {
 	return a.layout == KMX_SOA && bf16_supports(a, dev) && takes_rank16(a, lds_budget_of(exec, dev)) &&
@@ -218,6 +230,7 @@ int launch_screen_bf16(const float* rows, const Workspace* ws, const uint32_t* r
 int launch_assign_bf16(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	if (args.dim > 256) return launch_assign_wide(args, exec, ws, dev);
+	if (takes_cells(args, lds_budget_of(exec, dev))) return launch_assign_cells(args, exec, ws, dev);
 	if (takes_rank16(args, lds_budget_of(exec, dev))) return launch_assign_rank16(args, exec, ws, dev);
 	AssignArgs a = args;
 	/* wide rows and many centroids: a second sweep screens the queued points (narrow rows fit the registers of the

@@ -1,0 +1,530 @@
+/*
+ * Assignment of rows of 2 to 4 dimensions through a grid of cells.
+ *
+ * The sweeps compare every point with every centroid; with so few dimensions what they spend is not the products but the search for
+ * the smallest of k results (N = 4M, d = 4, k = 4096: 710 us, 0.04 ns per pair, four fifths of it vector instructions). Here the box around the
+ * centroids (and some way beyond) is divided into 2^15 or 2^16 cells, every cell gets the list of the centroids that can be the
+ * nearest of a point in it, and a point is compared with the twenty or so of its cell's list, in the serial arithmetic and in
+ * ascending order: the result is the serial scan's, no certificate needed.
+ *
+ * A centroid stays off a cell's list if its smallest distance to the cell's box, squared, exceeds the smallest of all centroids'
+ * largest ones by more than CELL_SLACK: the serial distances of any point of the box then compare the same way (they are off by at
+ * most (d + 4) 2^-24 each). Boxes and centroids are taken relative to the grid's corner, where all coordinates are small, and a box
+ * reaches CELL_MARGIN of its width beyond its edges, which covers the roundings of a point's coordinates there and of its cell.
+ *
+ * Points outside the grid, and those of cells without a list of their own (the lists take CELL_POOL_UNITS x 16 bytes; coordinates that
+ * are not finite, squares that would overflow or underflow make the whole grid one of those), get a bound from the
+ * list of the nearest cell, or a sample of the centroids, and go to the exact pass of rank16_exact_impl.h with it as their threshold.
+ */
+#include "rank16_exact_impl.h"
+
+namespace kmx {
+
+constexpr float CELL_SLACK = 1e-5f;
+constexpr float CELL_MARGIN = 1e-3f;
+constexpr uint32_t CELL_MAX_K = 6144;              /* what the building kernel's LDS holds */
+constexpr uint32_t CELL_UNIT = 8;                  /* entries (16 bits) of a list that are read together */
+constexpr uint32_t CELL_POOL_UNITS = 1u << 20;
+constexpr uint32_t CELL_SAMPLE = 64;               /* centroids of the list for points without one, at the start of the pool */
+constexpr uint32_t CELL_TRUNCATED = 1u << 31;      /* table entry: list start in units (20 bits), length in units (11), this flag */
+constexpr uint32_t CELL_MOST_UNITS = (1u << 11) - 1;
+constexpr uint32_t BUILD_THREADS = 1024;
+constexpr uint32_t BUILD_WAVES = BUILD_THREADS / WAVE;
+constexpr uint32_t BUILD_SHORT = 1024;             /* most centroids on the list of a second-level cell */
+
+/* cells per dimension: TOP of the first level (a work-group each), times MID (a wavefront each), times LOW */
+template <int D> struct CellShape;
+template <> struct CellShape<2> { static constexpr uint32_t TOP = 16, MID = 4, LOW = 4; };
+template <> struct CellShape<3> { static constexpr uint32_t TOP = 8, MID = 2, LOW = 2; };
+template <> struct CellShape<4> { static constexpr uint32_t TOP = 4, MID = 2, LOW = 2; };
+template <int D> constexpr uint32_t cells_per_dim() { return CellShape<D>::TOP * CellShape<D>::MID * CellShape<D>::LOW; }
+constexpr uint32_t power(uint32_t b, int e) { return e == 0 ? 1 : b * power(b, e - 1); }
+template <int D> constexpr uint32_t cell_count() { return power(cells_per_dim<D>(), D); }
+
+/* the grid: corner, cells per unit of length, cell widths (four floats each) */
+struct Grid {
+	float corner[4], inverse[4], width[4];
+};
+
+struct CellArgs {
+	const float* means; size_t stride_means;
+	Grid* grid; uint32_t* table; uint16_t* pool; uint32_t* used;
+	uint32_t k, pool_units;
+};
+
+template <int D>
+__device__ __forceinline__ void cell_distances(const float (&c)[D], const float (&lo)[D], const float (&hi)[D], float& least, float& most)
+{
+	least = 0.0f;
+	most = 0.0f;
+#pragma unroll
+	for (int q = 0; q < D; ++q) {
+		const float below = lo[q] - c[q], above = c[q] - hi[q]; /* (hi > lo) */
+		const float out = fmaxf(fmaxf(below, above), 0.0f), far = fmaxf(-below, -above);
+		least = __builtin_fmaf(out, out, least);
+		most = __builtin_fmaf(far, far, most);
+	}
+}
+
+/*
+ * One work-group per first-level cell. All of them find the box of the centroids (they have to read them anyway), then three levels of
+ * lists, each filtered from the one above: the work-group's, one per wavefront, one per cell.
+ * What bounds it: the latency of its dozen barriers and of the pass over all centroids (12 us at k = 4096, d = 4; one level
+ * of lists, every cell from all centroids, would be 65536 x k boxes, a millisecond).
+ */
+template <int D, int LM>
+__global__ void __launch_bounds__(BUILD_THREADS)
+build_cells_kernel(const CellArgs w)
+{
+	constexpr uint32_t TOP = CellShape<D>::TOP, MID = CellShape<D>::MID, LOW = CellShape<D>::LOW, N = cells_per_dim<D>();
+	constexpr uint32_t MIDS = power(MID, D), LOWS = power(LOW, D), LANES = WAVE / LOWS; /* second-level cells, cells of one, lanes per cell */
+	static_assert(MIDS <= BUILD_WAVES && LOWS * LANES == WAVE, "shape");
+	extern __shared__ __attribute__((aligned(16))) float lds[];
+	float* coords = lds;                                        /* k x D, relative to the corner */
+	uint16_t* first_list = (uint16_t*)(lds + w.k * D);          /* k */
+	uint16_t* second_lists = first_list + (w.k + 1) / 2 * 2;    /* BUILD_WAVES x BUILD_SHORT */
+	__shared__ float reduce[2 * D][BUILD_WAVES];
+	__shared__ uint32_t wave_count[BUILD_WAVES], wave_units[BUILD_WAVES], pool_start;
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
+	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+
+	/* the box of the centroids; anything that is not finite shows in it */
+	float low[D], high[D];
+#pragma unroll
+	for (int q = 0; q < D; ++q) { low[q] = __builtin_inff(); high[q] = -__builtin_inff(); }
+	bool odd = false;
+	for (uint32_t j = tid; j < w.k; j += BUILD_THREADS)
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			const float v = w.means[elem<LM>(w.stride_means, j, q)];
+			coords[j * D + q] = v;
+			low[q] = fminf(low[q], v);
+			high[q] = fmaxf(high[q], v);
+			odd = odd || !(__builtin_fabsf(v) < __builtin_inff());
+		}
+#pragma unroll
+	for (int q = 0; q < D; ++q) {
+		for (int off = WAVE / 2; off > 0; off >>= 1) { low[q] = fminf(low[q], __shfl_xor(low[q], off)); high[q] = fmaxf(high[q], __shfl_xor(high[q], off)); }
+		if (lane == 0) { reduce[q][wave] = low[q]; reduce[D + q][wave] = high[q]; }
+	}
+	if (tid == 0) pool_start = 0;
+	bool usable = !__syncthreads_or(odd ? 1 : 0);
+	float corner[D], width[D], inverse[D];
+	{
+		const float share = fmaxf(0.75f * __builtin_powf((float)w.k, -1.0f / D), 0.05f); /* of the extent, added on either side */
+		float extent2 = 0.0f;
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			float lo = reduce[q][0], hi = reduce[D + q][0];
+			for (uint32_t v = 1; v < BUILD_WAVES; ++v) { lo = fminf(lo, reduce[q][v]); hi = fmaxf(hi, reduce[D + q][v]); }
+			const float half = fmaxf(0.5f * (hi - lo) * (1.0f + 2.0f * share), 1e-6f * (__builtin_fabsf(lo) + __builtin_fabsf(hi)) + 1e-16f);
+			corner[q] = 0.5f * lo + 0.5f * hi - half;
+			width[q] = 2.0f * half / (float)N;
+			inverse[q] = (float)N / (2.0f * half);
+			extent2 += half * half;
+			usable = usable && width[q] * width[q] > 1e-30f;
+		}
+		usable = usable && extent2 < 1e36f;
+	}
+	if (blockIdx.x == 0 && tid < D) {
+		float c = corner[0], i = inverse[0], s = width[0];
+#pragma unroll
+		for (int q = 1; q < D; ++q) {
+			c = tid == (uint32_t)q ? corner[q] : c;
+			i = tid == (uint32_t)q ? inverse[q] : i;
+			s = tid == (uint32_t)q ? width[q] : s;
+		}
+		w.grid->corner[tid] = c; w.grid->inverse[tid] = i; w.grid->width[tid] = s;
+	}
+	if (blockIdx.x == 0 && tid < CELL_SAMPLE) w.pool[tid] = (uint16_t)((uint64_t)tid * w.k / CELL_SAMPLE);
+	const uint32_t nothing = CELL_TRUNCATED | (CELL_SAMPLE / CELL_UNIT) << 20; /* the sample */
+
+	/* this lane's cell */
+	uint32_t top[D], mid[D], at[D];
+	{
+		uint32_t t = blockIdx.x, m = min(wave, MIDS - 1), l = lane / LANES;
+#pragma unroll
+		for (int q = D - 1; q >= 0; --q) {
+			top[q] = t % TOP; t /= TOP;
+			mid[q] = m % MID; m /= MID;
+			at[q] = (top[q] * MID + mid[q]) * LOW + l % LOW; l /= LOW;
+		}
+	}
+	uint32_t cell = 0;
+#pragma unroll
+	for (int q = 0; q < D; ++q) cell = cell * N + at[q];
+	const bool writes = wave < MIDS && lane % LANES == 0;
+	if (!usable) {
+		if (writes) w.table[cell] = nothing;
+		return; /* (the whole work-group) */
+	}
+	for (uint32_t j = tid; j < w.k; j += BUILD_THREADS)
+#pragma unroll
+		for (int q = 0; q < D; ++q) coords[j * D + q] -= corner[q]; /* (this lane's own entries) */
+	__syncthreads();
+
+	auto box = [&](float (&lo)[D], float (&hi)[D], const uint32_t (&first)[D], uint32_t cells) {
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			lo[q] = ((float)first[q] - CELL_MARGIN) * width[q];
+			hi[q] = ((float)(first[q] + cells) + CELL_MARGIN) * width[q];
+		}
+	};
+	auto measure = [&](uint32_t j, const float (&lo)[D], const float (&hi)[D], float& least, float& most) {
+		float c[D];
+#pragma unroll
+		for (int q = 0; q < D; ++q) c[q] = coords[j * D + q];
+		cell_distances<D>(c, lo, hi, least, most);
+	};
+	auto enough = [](float bound) { return bound * (1.0f + CELL_SLACK); };
+	float lo[D], hi[D];
+
+	/* the work-group's list */
+	uint32_t first_count = 0;
+	{
+		uint32_t start[D];
+#pragma unroll
+		for (int q = 0; q < D; ++q) start[q] = top[q] * MID * LOW;
+		box(lo, hi, start, MID * LOW);
+		float bound = __builtin_inff();
+#pragma unroll 2
+		for (uint32_t j = tid; j < w.k; j += BUILD_THREADS) {
+			float least, most;
+			measure(j, lo, hi, least, most);
+			bound = fminf(bound, most);
+		}
+		for (int off = WAVE / 2; off > 0; off >>= 1) bound = fminf(bound, __shfl_xor(bound, off));
+		if (lane == 0) reduce[0][wave] = bound;
+		__syncthreads();
+		bound = reduce[0][0];
+		for (uint32_t v = 1; v < BUILD_WAVES; ++v) bound = fminf(bound, reduce[0][v]);
+		for (uint32_t base = 0; base < w.k; base += BUILD_THREADS) {
+			const uint32_t j = base + tid;
+			float least = __builtin_inff(), most;
+			if (j < w.k) measure(j, lo, hi, least, most);
+			const bool keep = j < w.k && least <= enough(bound);
+			const unsigned long long mask = __ballot(keep);
+			if (lane == 0) wave_count[wave] = (uint32_t)__popcll(mask);
+			__syncthreads();
+			uint32_t before = first_count;
+			for (uint32_t v = 0; v < BUILD_WAVES; ++v) {
+				before += v < wave ? wave_count[v] : 0u;
+				first_count += wave_count[v];
+			}
+			if (keep) first_list[before + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)j;
+			__syncthreads();
+		}
+	}
+
+	/* the wavefront's list */
+	uint16_t* second_list = second_lists + wave * BUILD_SHORT;
+	uint32_t second_count = 0;
+	if (wave < MIDS) {
+		uint32_t start[D];
+#pragma unroll
+		for (int q = 0; q < D; ++q) start[q] = (top[q] * MID + mid[q]) * LOW;
+		box(lo, hi, start, LOW);
+		float bound = __builtin_inff();
+#pragma unroll 4
+		for (uint32_t i = lane; i < first_count; i += WAVE) {
+			float least, most;
+			measure(first_list[i], lo, hi, least, most);
+			bound = fminf(bound, most);
+		}
+		for (int off = WAVE / 2; off > 0; off >>= 1) bound = fminf(bound, __shfl_xor(bound, off));
+#pragma unroll 4
+		for (uint32_t base = 0; base < first_count; base += WAVE) {
+			const uint32_t i = base + lane;
+			const uint16_t j = first_list[min(i, first_count - 1)];
+			float least, most;
+			measure(j, lo, hi, least, most);
+			const bool keep = i < first_count && least <= enough(bound);
+			const unsigned long long mask = __ballot(keep);
+			const uint32_t to = second_count + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+			if (keep && to < BUILD_SHORT) second_list[to] = j;
+			second_count += (uint32_t)__popcll(mask);
+		}
+	}
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	const bool too_long = second_count > BUILD_SHORT;
+
+	/* the cells' lists: LANES lanes share a cell, a contiguous part of the wavefront's list each */
+	const uint32_t part = lane % LANES;
+	const uint32_t i0 = too_long ? 0u : part * second_count / LANES, i1 = too_long ? 0u : (part + 1) * second_count / LANES;
+	box(lo, hi, at, 1);
+	float bound = __builtin_inff();
+#pragma unroll 4
+	for (uint32_t i = i0; i < i1; ++i) {
+		float least, most;
+		measure(second_list[i], lo, hi, least, most);
+		bound = fminf(bound, most);
+	}
+	for (uint32_t off = LANES / 2; off > 0; off >>= 1) bound = fminf(bound, __shfl_xor(bound, (int)off));
+	bound = enough(bound);
+	uint32_t count = 0;
+	unsigned long long kept = 0; /* which of this lane's first 63 */
+#pragma unroll 4
+	for (uint32_t i = i0; i < i1; ++i) {
+		float least, most;
+		measure(second_list[i], lo, hi, least, most);
+		const bool keep = least <= bound;
+		count += keep ? 1u : 0u;
+		kept |= (unsigned long long)(keep ? 1u : 0u) << min(i - i0, 63u);
+	}
+	uint32_t before = 0, total = 0; /* entries of the lanes before this one, of the cell */
+#pragma unroll
+	for (uint32_t v = 0; v < LANES; ++v) {
+		const uint32_t c = (uint32_t)__shfl((int)count, (int)(lane - part + v));
+		before += v < part ? c : 0u;
+		total += c;
+	}
+	uint32_t units = wave < MIDS ? (total + CELL_UNIT - 1) / CELL_UNIT : 0u;
+	const bool fits = units <= CELL_MOST_UNITS && !too_long;
+	if (!fits) units = 0;
+	uint32_t upto = part == 0 ? units : 0u; /* inclusive over the wavefront's cells */
+#pragma unroll
+	for (uint32_t off = 1; off < WAVE; off <<= 1) {
+		const uint32_t v = (uint32_t)__shfl_up((int)upto, off);
+		if (lane >= off) upto += v;
+	}
+	if (lane == WAVE - 1) wave_units[wave] = upto;
+	__syncthreads();
+	if (tid == 0) {
+		uint32_t all = 0;
+		for (uint32_t v = 0; v < BUILD_WAVES; ++v) { const uint32_t u = wave_units[v]; wave_units[v] = all; all += u; }
+		pool_start = CELL_SAMPLE / CELL_UNIT + atomicAdd(w.used, all);
+	}
+	__syncthreads();
+	const uint32_t start = pool_start + wave_units[wave] + upto - units; /* (lanes of a cell behind its first: upto counts the cell already) */
+	const bool listed = fits && units > 0 && (uint64_t)start + units <= w.pool_units;
+	if (writes) w.table[cell] = listed ? start | units << 20 : nothing;
+	if (listed && wave < MIDS) {
+		uint16_t* out = w.pool + (size_t)start * CELL_UNIT;
+		uint32_t to = before;
+		uint16_t last = 0;
+		kept &= ~(1ull << 63);
+		while (kept) {
+			last = second_list[i0 + (uint32_t)__builtin_ctzll(kept)];
+			out[to++] = last;
+			kept &= kept - 1;
+		}
+		for (uint32_t i = i0 + 63; i < i1; ++i) {
+			const uint16_t j = second_list[i];
+			float least, most;
+			measure(j, lo, hi, least, most);
+			if (least <= bound) { out[to++] = j; last = j; }
+		}
+		/* the lane with the cell's last entry fills the last unit up with it */
+		if (count > 0 && to == total)
+			for (; to < units * CELL_UNIT; ++to) out[to] = last;
+	}
+}
+
+struct CellAssignArgs {
+	const float* data; size_t stride;
+	const float* means; size_t stride_means;
+	const Grid* grid; const uint32_t* table; const uint16_t* pool;
+	const float* norms; const float* low2; const float* frame; float* scale; /* of the exact pass (pack_means16_kernel) */
+	uint32_t* assignment; uint32_t* list; uint32_t* length;
+	uint32_t k, kp, n;
+	float kd;
+};
+
+constexpr uint32_t CELL_THREADS = 1024;
+constexpr uint32_t CELL_WAVES = CELL_THREADS / WAVE;
+constexpr uint32_t CELL_LIST = 64; /* points per wavefront that wait for the list */
+
+/*
+ * A lane per point, the centroids in LDS. What bounds it: the gathers, 16 bytes of centroid per comparison from LDS and 16 bytes of list per
+ * eight of them from the caches, and the longest list among a wavefront's points.
+ */
+template <int D, int LD, int LM>
+__global__ void __launch_bounds__(CELL_THREADS)
+assign_cells_kernel(const CellAssignArgs w)
+{
+	constexpr uint32_t N = cells_per_dim<D>();
+	extern __shared__ __attribute__((aligned(16))) float lds[]; /* k x 4 */
+	__shared__ uint32_t wave_max[2][CELL_WAVES];
+	__shared__ uint32_t flag_list[CELL_WAVES][2 * CELL_LIST];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
+	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	for (uint32_t j = tid; j < w.k; j += CELL_THREADS) {
+		f32x4 c = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+		for (int q = 0; q < D; ++q) c[q] = w.means[elem<LM>(w.stride_means, j, q)];
+		*(f32x4*)(lds + 4 * j) = c;
+	}
+	CertCoeffs cert;
+	{
+		uint32_t most[2] = { 0u, 0u };
+		for (uint32_t j = tid; j < w.k; j += CELL_THREADS) {
+			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
+			most[1] = max(most[1], __float_as_uint(w.low2[j]));
+		}
+#pragma unroll
+		for (int q = 0; q < 2; ++q) {
+			for (int off = WAVE / 2; off > 0; off >>= 1) most[q] = max(most[q], (uint32_t)__shfl_xor((int)most[q], off));
+			if (lane == 0) wave_max[q][wave] = most[q];
+		}
+		__syncthreads();
+#pragma unroll
+		for (int q = 0; q < 2; ++q) {
+			most[q] = 0;
+			for (uint32_t v = 0; v < CELL_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
+		}
+		if (blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], w.low2, w.k, w.kp);
+		cert = cert_coeffs_level1(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), 0.0f });
+	}
+	const float scale = w.scale[0];
+	float corner[D], inverse[D];
+#pragma unroll
+	for (int q = 0; q < D; ++q) { corner[q] = w.grid->corner[q]; inverse[q] = w.grid->inverse[q]; }
+
+	uint32_t flagged = 0; /* wave-uniform */
+	for (uint32_t base = blockIdx.x * CELL_THREADS; base < w.n; base += gridDim.x * CELL_THREADS) {
+		const uint32_t pt = base + tid;
+		const bool mine = pt < w.n;
+		float x[D];
+#pragma unroll
+		for (int q = 0; q < D; ++q) x[q] = w.data[elem<LD>(w.stride, min(pt, w.n - 1), q)];
+		bool inside = true;
+		uint32_t cell = 0;
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			const float y = (x[q] - corner[q]) * inverse[q];
+			inside = inside && y >= 0.0f && y < (float)N;
+			cell = cell * N + (uint32_t)fminf(fmaxf(y, 0.0f), (float)(N - 1)); /* (NaN: 0) */
+		}
+		const uint32_t entry = w.table[cell];
+		const uint32_t units = (entry >> 20) & CELL_MOST_UNITS;
+		const uint4* list = (const uint4*)w.pool + (entry & 0xFFFFFu);
+		float best = __builtin_inff();
+		uint32_t winner = 0;
+		auto compare = [&](uint32_t j) {
+#pragma clang fp contract(off)
+			const f32x4 c = *(const f32x4*)(lds + 4 * j);
+			float sum = 0.0f;
+#pragma unroll
+			for (int q = 0; q < D; ++q) {
+				const float diff = x[q] - c[q];
+				const float sq = diff * diff;
+				sum = sum + sq;
+			}
+			/* the serial scan compares square roots: a smaller square may have the same one */
+			if (sum < best && (sum < best * 0.9999995f || __builtin_sqrtf(sum) < __builtin_sqrtf(best))) { best = sum; winner = j; }
+		};
+		uint4 next = list[0];
+		for (uint32_t u = 0; u < units; ++u) {
+			const uint4 now = next;
+			next = list[min(u + 1, units - 1)];
+			compare(now.x & 0xFFFFu); compare(now.x >> 16);
+			compare(now.y & 0xFFFFu); compare(now.y >> 16);
+			compare(now.z & 0xFFFFu); compare(now.z >> 16);
+			compare(now.w & 0xFFFFu); compare(now.w >> 16);
+		}
+		if (mine) w.assignment[pt] = winner;
+		const bool flag = mine && (!inside || (entry & CELL_TRUNCATED));
+		const unsigned long long mask = __ballot(flag);
+		if (mask) {
+			const uint32_t add = (uint32_t)__popcll(mask);
+			if (flagged + add > CELL_LIST) {
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+				__builtin_amdgcn_wave_barrier();
+				uint32_t slot = 0;
+				if (lane == 0) slot = atomicAdd(w.length, flagged);
+				slot = (uint32_t)__shfl((int)slot, 0);
+				for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[2 * (size_t)slot + i] = flag_list[wave][i];
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+				__builtin_amdgcn_wave_barrier();
+				flagged = 0;
+			}
+			if (flag) {
+				/* every centroid as near as the winner ranks at or below its distance, within the certificate of the ranking */
+				float x2 = 0.0f, low2 = 0.0f;
+#pragma unroll
+				for (int q = 0; q < D; ++q) {
+					const float v = __builtin_fmaf(x[q], scale, -(w.frame[q] * scale));
+					const float r = v - (float)(_Float16)v;
+					x2 = __builtin_fmaf(v, v, x2);
+					low2 = __builtin_fmaf(r, r, low2);
+				}
+				const float nearest2 = best * (scale * scale);
+				const bool extreme = !(best > 1e-30f && best < 1e37f && nearest2 < 1e37f && x2 < 1e37f);
+				const float tau = cert_tau(w.kd, x2, low2, cert) + 64.0f * CERT_UNIT * nearest2;
+				const uint32_t at = 2 * (flagged + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)));
+				flag_list[wave][at] = pt;
+				flag_list[wave][at + 1] = screening_threshold(extreme ? __builtin_inff() : nearest2 - x2, tau);
+			}
+			flagged += add;
+		}
+	}
+	/* what is left in the lists: one addition per work-group */
+	__syncthreads();
+	if (lane == 0) wave_max[0][wave] = flagged;
+	__syncthreads();
+	uint32_t before = 0, all = 0;
+#pragma unroll
+	for (uint32_t v = 0; v < CELL_WAVES; ++v) {
+		before += v < wave ? wave_max[0][v] : 0u;
+		all += wave_max[0][v];
+	}
+	if (all == 0) return;
+	if (tid == 0) wave_max[1][0] = atomicAdd(w.length, all);
+	__syncthreads();
+	const size_t slot = 2 * (size_t)(wave_max[1][0] + before);
+	for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[slot + i] = flag_list[wave][i];
+}
+
+template <int D>
+static int launch_cells_d(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half)
+{
+	constexpr uint32_t CELLS = cell_count<D>();
+	const size_t table_words = sizeof(Grid) / 4 + CELLS;
+	int rc = reserve_cells(ws, table_words + (size_t)CELL_POOL_UNITS * CELL_UNIT / 2);
+	if (rc) return rc;
+	if ((rc = reserve_listed(ws, 2 * (size_t)a.n))) return rc;
+	Grid* grid = (Grid*)ws->cells;
+	uint32_t* table = ws->cells + sizeof(Grid) / 4;
+	uint16_t* pool = (uint16_t*)(ws->cells + table_words);
+	static_assert(sizeof(Grid) % 16 == 0 && CELLS % 4 == 0, "the pool is read in units of 16 bytes");
+	const uint32_t build_lds = a.k * D * 4 + (a.k + 1) / 2 * 4 + BUILD_WAVES * BUILD_SHORT * 2;
+	const CellArgs b = { a.means, a.stride_means, grid, table, pool, ws->counters + CELLS_COUNTER, a.k, CELL_POOL_UNITS };
+	void (*build)(CellArgs) = a.layout_means == KMX_AOS ? build_cells_kernel<D, KMX_AOS> : build_cells_kernel<D, KMX_SOA>;
+	KMX_HIP(hipFuncSetAttribute((const void*)build, hipFuncAttributeMaxDynamicSharedMemorySize, (int)build_lds));
+	KMX_LAUNCH_KERNEL(build, dim3(power(CellShape<D>::TOP, D)), dim3(BUILD_THREADS), build_lds, stream(), b);
+	KMX_LAUNCH_CHECK("build_cells_kernel");
+
+	const CellAssignArgs w = { a.data, a.stride, a.means, a.stride_means, grid, table, pool, half.norms, half.low2, half.frame, half.scale,
+	                           a.assignment, ws->listed, ws->counters + LISTED_COUNTER, a.k, half.kp, a.n, half.kd };
+	void (*assign)(CellAssignArgs) = a.layout == KMX_AOS ? (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_AOS, KMX_AOS> : assign_cells_kernel<D, KMX_AOS, KMX_SOA>)
+	                                                     : (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_SOA, KMX_AOS> : assign_cells_kernel<D, KMX_SOA, KMX_SOA>);
+	const uint32_t lds = a.k * 16, per_cu = std::max<uint32_t>(1, std::min<uint32_t>(2, dev.lds_bytes / (lds + CELL_WAVES * 2 * CELL_LIST * 4 + 256)));
+	const uint32_t blocks = std::min((a.n + CELL_THREADS - 1) / CELL_THREADS, per_cu * dev.compute_units);
+	exec->block_count = blocks;
+	if ((rc = profile_begin(0))) return rc;
+	KMX_HIP(hipFuncSetAttribute((const void*)assign, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+	KMX_LAUNCH_KERNEL(assign, dim3(blocks), dim3(CELL_THREADS), lds, stream(), w);
+	KMX_LAUNCH_CHECK("assign_cells_kernel");
+	return profile_end(0);
+}
+
+bool cells_support(const AssignArgs& a, uint32_t lds_budget)
+{
+	if (a.dim < 2 || a.dim > 4 || a.k > CELL_MAX_K || a.k < 2 || a.n > (1u << 31) || a.ranking_only) return false;
+	const uint32_t build_lds = a.k * a.dim * 4 + (a.k + 1) / 2 * 4 + BUILD_WAVES * BUILD_SHORT * 2 + 1024;
+	const uint32_t assign_lds = a.k * 16 + CELL_WAVES * 2 * CELL_LIST * 4 + 256;
+	return std::max(build_lds, assign_lds) <= lds_budget && exact_dynamic_bytes(1, EXACT_GROUPS) + exact_static_bytes(false) <= lds_budget;
+}
+
+int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half)
+{
+	switch (a.dim) {
+	case 2: return launch_cells_d<2>(a, exec, ws, dev, half);
+	case 3: return launch_cells_d<3>(a, exec, ws, dev, half);
+	case 4: return launch_cells_d<4>(a, exec, ws, dev, half);
+	default: return fail(KMX_ERR_UNSUPPORTED, "assign (cells): dim %u is not supported", a.dim);
+	}
+}
+
+} // namespace kmx

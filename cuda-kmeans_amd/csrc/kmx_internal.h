@@ -57,6 +57,7 @@ struct Workspace {
 	float* packed_means = nullptr;  size_t packed_cap = 0;     /* floats  */
 	float* packed16 = nullptr;      size_t packed16_cap = 0;   /* floats: half-precision operands of the centroids (rank16.hip) */
 	float* norms = nullptr;         size_t norms_cap = 0;      /* floats  */
+	uint32_t* cells = nullptr;      size_t cells_cap = 0;      /* words: grid, table and lists of assign_cells.hip */
 	float* norms16 = nullptr;       size_t norms16_cap = 0;    /* floats: norms, frame and scale of the half-precision sweep */
 	float* means_t = nullptr;       size_t means_t_cap = 0;    /* floats: exact transposed centroids [dim][kp] */
 	float* partials = nullptr;      size_t partials_cap = 0;   /* floats  */
@@ -73,6 +74,7 @@ struct Workspace {
 int workspace(Workspace** ws);
 int reserve_queue(Workspace* ws, size_t entries);
 int reserve_packed(Workspace* ws, size_t packed_floats, size_t norm_floats, size_t transposed_floats);
+int reserve_cells(Workspace* ws, size_t words);
 int reserve_packed16(Workspace* ws, size_t packed_floats, size_t norm_floats);
 int reserve_partials(Workspace* ws, size_t floats);
 int reserve_fused_assignment(Workspace* ws, size_t entries);
@@ -82,6 +84,7 @@ int reserve_queued_rows(Workspace* ws, size_t rows, size_t dim, size_t extra_wor
 int reserve_carried(Workspace* ws, size_t words);
 int reserve_listed(Workspace* ws, size_t words);
 int two_level_mode(); /* kmx_set_two_level_sweep */
+constexpr uint32_t CELLS_COUNTER = 5;  /* word of Workspace::counters that counts the list units handed out by build_cells_kernel */
 constexpr uint32_t LISTED_COUNTER = 4; /* word of Workspace::counters that holds the length of Workspace::listed */
 
 #define KMX_HIP(call)                                                                                         \
@@ -184,6 +187,15 @@ bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_bf16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* rank16.hip: one half-precision product per dimension for all points, the serial result for what that leaves */
 bool rank16_supports(const AssignArgs& a, uint32_t lds_budget);
+/* assign_cells.hip: rows of 2 to 4 dimensions through a grid; half: what pack_means16_kernel left for the exact pass */
+struct Cells16 {
+	const float* norms; const float* low2; const float* frame; float* scale;
+	uint32_t kp; float kd;
+};
+bool takes_cells(const AssignArgs& a, uint32_t lds_budget); /* KMX_ASSIGN_MFMA_BF16X3 runs as cells (assign_bf16.hip) */
+bool cells_support(const AssignArgs& a, uint32_t lds_budget);
+int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half);
+int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev); /* rank16.hip: all of it */
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST would write a.rows_out */
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */

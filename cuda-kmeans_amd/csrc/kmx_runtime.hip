@@ -120,6 +120,7 @@ int reserve_packed(Workspace* ws, size_t packed_floats, size_t norm_floats, size
 	return grow(&ws->means_t, &ws->means_t_cap, transposed_floats);
 }
 
+int reserve_cells(Workspace* ws, size_t words) { return grow(&ws->cells, &ws->cells_cap, words); }
 int reserve_packed16(Workspace* ws, size_t packed_floats, size_t norm_floats)
 {
 	int rc = grow(&ws->packed16, &ws->packed16_cap, packed_floats);
@@ -158,6 +159,7 @@ static int release_workspace()
 	if (g_ws.packed_means) KMX_HIP(hipFree(g_ws.packed_means));
 	if (g_ws.norms) KMX_HIP(hipFree(g_ws.norms));
 	if (g_ws.packed16) KMX_HIP(hipFree(g_ws.packed16));
+	if (g_ws.cells) KMX_HIP(hipFree(g_ws.cells));
 	if (g_ws.norms16) KMX_HIP(hipFree(g_ws.norms16));
 	if (g_ws.means_t) KMX_HIP(hipFree(g_ws.means_t));
 	if (g_ws.partials) KMX_HIP(hipFree(g_ws.partials));
@@ -212,6 +214,7 @@ int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Wor
 		 * The plain-VALU variant, which reads a small centroid block through the scalar cache, wins with at most 16
 		 * centroids of at most 16 dimensions (d = 16, k = 16: 0.086 against 0.105 ms; d = 8, k = 8: 0.049 against 0.080 ms)
 		 * and loses from there on (d = 16, k = 32: 0.128 against 0.110 ms; d = 32, k = 16: 0.183 against 0.161 ms).
+		 * Rows of 2 to 4 dimensions and many points: a grid of cells, under the same name (takes_cells).
 		 * The double path, which pays more per queued point: the packed form from 256 centroids on, where its exact pass
 		 * works in batches (N = 4M doubles, d = 4, k = 4096: 1.09 against 1.64 ms per call; d = 3, k = 1024: 0.40 against
 		 * 0.52 ms; d = 4, k = 256: 0.25 against 0.29 ms; d = 2, k = 1024: level); the plain-VALU variant
@@ -222,7 +225,7 @@ int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Wor
 		const bool split_wins = a.dim >= 16 || (a.dim >= 5 && a.k > 64);
 		const bool few = a.ranking_only ? a.k <= 32 : (a.k <= 16 && a.dim <= 16);
 		if (few && lds_fma_supports(a, dev) && lds_fma_reads_through_scalar_cache(a)) variant = KMX_ASSIGN_LDS_FMA;
-		else if (bf16_supports(a, dev) && (split_wins || packed_wins)) variant = KMX_ASSIGN_MFMA_BF16X3;
+		else if (bf16_supports(a, dev) && (split_wins || packed_wins || takes_cells(a, lds_budget_of(exec, dev)))) variant = KMX_ASSIGN_MFMA_BF16X3;
 		else if (mfma_supports(a, dev)) variant = KMX_ASSIGN_MFMA;
 		else if (lds_fma_supports(a, dev)) variant = KMX_ASSIGN_LDS_FMA;
 		else variant = KMX_ASSIGN_BASE;

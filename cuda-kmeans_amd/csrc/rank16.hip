@@ -62,7 +62,7 @@ pack_means16_kernel(const float* __restrict__ means, const double* __restrict__ 
 	__shared__ float frame[FRAME_DIMS];
 	__shared__ float wave_far[4];
 	const uint32_t lane = threadIdx.x & (WAVE - 1);
-	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; }
+	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; counters[CELLS_COUNTER] = 0u; }
 	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
 	/* this row's coordinates are requested ahead of the frame they will be moved to */
 	float exact[FRAME_DIMS / WAVE];
@@ -178,9 +178,9 @@ static int launch_listed_exact(const AssignArgs& a, const F* points, size_t poin
 {
 	const uint32_t kb = rank16_kb(a.dim), dp = kb * KBLOCK, kp = round_up(a.k, TILE);
 	const float* norms = ws->norms16;
-	const bool aos = a.layout == KMX_AOS;
-	const uint32_t row_dim = aos ? a.dim : round_up(a.dim, 8);
-	const ExactArgs<F> w = { aos ? a.data : ws->queued_rows, aos ? a.stride : row_dim, 1, row_dim, points, points_stride, points_step, points_dim,
+	const bool aos = a.layout == KMX_AOS, copied = !aos && a.dim > 4; /* (narrow rows have not been copied) */
+	const uint32_t row_dim = copied ? round_up(a.dim, 8) : a.dim;
+	const ExactArgs<F> w = { copied ? ws->queued_rows : a.data, aos ? a.stride : copied ? row_dim : 1, aos || copied ? 1 : a.stride, row_dim, points, points_stride, points_step, points_dim,
 	                         (const F*)(ws->packed16 + rank16_rows_offset(kp, dp)), (const f16x8*)ws->packed16, norms,
 	                         norms + rank16_frame_offset(kp), norms + rank16_scale_offset(kp), a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->counters,
 	                         a.dim, a.k, kp, cert_kd_split(a.dim) + 8.0f * CERT_UNIT, kb, EXACT_GROUPS };
@@ -227,6 +227,18 @@ int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 	if (a.settled) *a.settled = true;
 	if (a.rows_out && a.layout == KMX_SOA && part == a.n) *a.rows_out = AosRows{ ws->queued_rows, round_up(a.dim, 8) };
 	return KMX_OK;
+}
+
+int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	int rc = launch_pack16(a, ws);
+	if (rc) return rc;
+	const uint32_t kp = round_up(a.k, TILE);
+	const Cells16 half = { ws->norms16, ws->norms16 + rank16_low_offset(kp), ws->norms16 + rank16_frame_offset(kp), ws->norms16 + rank16_scale_offset(kp), kp,
+	                       cert_kd_level1(a.dim) + 8.0f * CERT_UNIT };
+	if ((rc = launch_cells(a, exec, ws, dev, half))) return rc;
+	const bool aos = a.layout == KMX_AOS;
+	return launch_listed_exact<float>(a, a.data, aos ? a.stride : 1, aos ? 1 : a.stride, a.dim, ws, dev);
 }
 
 } // namespace kmx

@@ -23,7 +23,7 @@ constexpr uint32_t exact_static_bytes(bool doubles)
 template <typename F>
 struct ExactArgs {
 	/* coordinate d of point p: data[p * stride + d * step]; step 1: rows of row_dim coordinates (zeros behind the first dim). Other
-	 * steps (SoA points) are for KB = 0 only. */
+	 * steps (SoA points) are for KB <= 1 only. */
 	const float* data; size_t stride, step; uint32_t row_dim;
 	/* the same of the points the serial arithmetic is for (doubles: data is their float copy) */
 	const F* points; size_t points_stride, points_step; uint32_t points_dim;
@@ -120,8 +120,9 @@ listed_exact_kernel(const ExactArgs<F> w)
 	const uint32_t col = lane & 31, h = lane >> 5;
 	const float scale = w.scale[0], unscale = w.scale[1];
 	const uint32_t tiles = w.kp / TILE;
-	const bool strided = KB == 0 && w.step != 1, ragged = w.row_dim < DP && !strided;
-	const bool points_strided = (KB == 0 || DOUBLES) && w.points_step != 1, points_ragged = w.points_dim < DP && !points_strided;
+	/* (rows of fewer than four coordinates are read one by one, like those of SoA points) */
+	const bool strided = KB <= 1 && (w.step != 1 || w.row_dim < 4), ragged = w.row_dim < DP && !strided;
+	const bool points_strided = (KB <= 1 || DOUBLES) && (w.points_step != 1 || w.points_dim < 4), points_ragged = w.points_dim < DP && !points_strided;
 
 	/* of the three-product ranking: only what is counted depends on it (the sweep left the maxima behind the scale) */
 	const CertCoeffs cert = cert_coeffs_split(CentroidBounds{ w.scale[2], w.scale[3], w.scale[4] });

@@ -1,0 +1,62 @@
+"""Rows of 2 to 4 dimensions through the grid of cells (csrc/assign_cells.hip) against the serial oracle, bit for bit: points inside and
+outside the grid, on its edges, exact ties, degenerate boxes, lists that do not fit, values that are not finite (-m gpu)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def flat(rows, layout):
+    return np.ascontiguousarray(rows if layout == 0 else rows.T).ravel()
+
+
+@pytest.mark.parametrize("kind", ["uniform", "clustered", "lattice", "offset", "line", "same", "dense", "nan", "huge", "tiny"])
+@pytest.mark.parametrize("dim,k,n", [(2, 2, 1), (2, 129, 2049), (2, 6000, 20000), (3, 7, 1025), (3, 1000, 9000), (3, 4097, 12000), (4, 33, 1000), (4, 512, 5000), (4, 4096, 20001)])
+def test_cells_match_the_oracle(km, orc, gpu, dim, k, n, kind):
+    rng = np.random.default_rng(dim * 41 + k)
+    means = rng.uniform(0, 1, size=(k, dim)).astype(np.float32)
+    rows = rng.uniform(-0.05, 1.05, size=(n, dim)).astype(np.float32)
+    if kind == "clustered":
+        centres = rng.uniform(-10, 10, size=(20, dim))
+        means = (centres[rng.integers(0, 20, k)] + rng.normal(size=(k, dim))).astype(np.float32)
+        rows = (centres[rng.integers(0, 20, n)] + rng.normal(size=(n, dim))).astype(np.float32)
+    elif kind == "lattice":   # ties everywhere, points on the edges of cells
+        means = np.round(means * 8).astype(np.float32); rows = (np.round(rows * 32) / 4).astype(np.float32)
+    elif kind == "offset":
+        means += np.float32(1000); rows += np.float32(1000)
+    elif kind == "line":      # no extent in one dimension
+        means[:, dim - 1] = 0.5; rows[::2, dim - 1] = 0.5
+    elif kind == "same":
+        means[:] = means[0]
+    elif kind == "dense":     # almost all centroids and points in one cell
+        means[1:] = (0.5 + means[1:] * 1e-3).astype(np.float32); rows[1:] = (0.5 + rows[1:] * 1e-3).astype(np.float32)
+        means[0] = 30
+    elif kind == "nan":
+        means[k // 2] = np.nan
+    elif kind == "huge":
+        means *= np.float32(1e19); rows *= np.float32(1e19)
+    elif kind == "tiny":
+        means *= np.float32(1e-22); rows *= np.float32(1e-22)
+    if n > 20:
+        rows[3] = means[min(3, k - 1)]
+        rows[7, 0] = np.nan; rows[11, dim - 1] = np.inf; rows[13] = -1e30; rows[17] = 1e6
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    a = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for layout, layout_means, pad in [(0, 0, 0), (0, 1, 3), (1, 1, 0)]:
+            stride = dim + pad if layout == 0 else n
+            padded = rows
+            if pad:
+                padded = np.full((n, stride), np.float32(np.nan)); padded[:, :dim] = rows
+            d = km.DeviceBuffer(padded.nbytes); d.write(flat(padded, layout))
+            m = km.DeviceBuffer(4 * k * dim); m.write(flat(means, layout_means))
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, layout, stride, m, layout_means, km.layout_stride(layout_means, k, dim), a, dim, k, n)
+            km.sync()
+            got = a.read(np.uint32, n)
+            d.free(); m.free()
+            assert np.array_equal(got, want), "layouts %d/%d: %d mismatches" % (layout, layout_means, int((got != want).sum()))
+    finally:
+        km.set_two_level_sweep(1)
+    a.free()
