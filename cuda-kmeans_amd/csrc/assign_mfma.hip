@@ -58,11 +58,16 @@ static uint32_t pick_dph(uint32_t dim)
 template <int LM>
 __global__ void __launch_bounds__(256)
 pack_means_kernel(const float* __restrict__ means, size_t stride_means, float* __restrict__ packed, float* __restrict__ norms,
-                  float* __restrict__ means_t, uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t moved, uint32_t* __restrict__ counters)
+                  float* __restrict__ means_t, uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t moved, uint32_t* __restrict__ counters, const ClearOutputs clear)
 {
 	const uint32_t lane = threadIdx.x & (WAVE - 1);
 	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-	if (blockIdx.x == 0 && threadIdx.x == 0) counters[0] = 0u; /* the recheck queue of this call starts empty */
+	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[FINISH_COUNTER] = 0u; } /* the recheck queue of this call starts empty */
+	if (clear.means) { /* the outputs the single-pass kernel adds to */
+		for (size_t i = threadIdx.x + (size_t)blockIdx.x * blockDim.x; i < clear.words; i += (size_t)blockDim.x * gridDim.x) clear.means[i] = 0.0f;
+		if (blockIdx.x == 0)
+			for (uint32_t c = threadIdx.x; c < k; c += blockDim.x) clear.sizes[c] = 0u;
+	}
 	/* the frame of the sweep (zeros unless `moved`): the rows are those of c - m, with their norms; the exact pass gets
 	 * the centroids and their norms as given */
 	__shared__ float frame[FRAME_DIMS];
@@ -110,7 +115,7 @@ KMX_DECLARE_MFMA_LAUNCHER(16) KMX_DECLARE_MFMA_LAUNCHER(24) KMX_DECLARE_MFMA_LAU
 KMX_DECLARE_MFMA_LAUNCHER(128)
 
 /* packs the centroids of this call into the work space (rows of dp floats, kp rows) and empties the recheck queue */
-int launch_pack_means(const AssignArgs& a, Workspace* ws, uint32_t dp, uint32_t kp, uint32_t moved)
+int launch_pack_means(const AssignArgs& a, Workspace* ws, uint32_t dp, uint32_t kp, uint32_t moved, const ClearOutputs& clear)
 {
 	int rc = reserve_packed(ws, (size_t)(kp / TILE) * tile_floats(dp + ROW_PAD), plain_norms_floats(kp), (size_t)kp * a.dim);
 	if (rc) return rc;
@@ -119,10 +124,10 @@ int launch_pack_means(const AssignArgs& a, Workspace* ws, uint32_t dp, uint32_t 
 	const uint32_t pack_blocks = (kp * WAVE + 255) / 256;
 	if (a.layout_means == KMX_AOS)
 		KMX_LAUNCH_KERNEL((pack_means_kernel<KMX_AOS>), dim3(pack_blocks), dim3(256), 0, stream(),
-		                   a.means, a.stride_means, ws->packed_means, ws->norms, ws->means_t, a.dim, a.k, kp, dp, moved, ws->counters);
+		                   a.means, a.stride_means, ws->packed_means, ws->norms, ws->means_t, a.dim, a.k, kp, dp, moved, ws->counters, clear);
 	else
 		KMX_LAUNCH_KERNEL((pack_means_kernel<KMX_SOA>), dim3(pack_blocks), dim3(256), 0, stream(),
-		                   a.means, a.stride_means, ws->packed_means, ws->norms, ws->means_t, a.dim, a.k, kp, dp, moved, ws->counters);
+		                   a.means, a.stride_means, ws->packed_means, ws->norms, ws->means_t, a.dim, a.k, kp, dp, moved, ws->counters, clear);
 	KMX_LAUNCH_CHECK("pack_means_kernel");
 	return KMX_OK;
 }

@@ -17,7 +17,7 @@
  *      Such points (a few in a hundred) are not settled where they turn up: the wavefront notes them in a list in
  *      LDS and, once half a wavefront of them waits, reads their rows again and settles them together, one per
  *      lane. Only a point with three or more centroids within tau, or with data the bound does not cover (NaN,
- *      overflow), stays unresolved: it goes to the recheck queue and a fix-up kernel adds it to the sums afterwards.
+ *      overflow), stays unresolved: it goes to the recheck queue, and fused_finish_kernel adds it to the sums afterwards.
  *   3. Accumulation on the matrix cores: the sums of a wavefront's 64 points are the product of the k x 64 indicator
  *      matrix (1 where the point belongs to the cluster) with the 64 x dim block of coordinates. The wavefront parks
  *      its rows and results in LDS (that transposes them: the MFMA wants one lane per dimension) and issues
@@ -800,35 +800,130 @@ fused_matrix_kernel(const float* __restrict__ data, size_t stride, const float* 
 	if (threadIdx.x < k && members[threadIdx.x]) atomicAdd(&sizes[threadIdx.x], members[threadIdx.x]);
 }
 
-/* adds the points the exact pass has just resolved (the queue of the fused kernel) to the sums and counts: every
- * work-group gathers its share in LDS first, so the few hundred result words see one global atomic per work-group */
+/*
+ * What the single pass leaves: the serial scan over all centroids for the points in the queue, 32 lanes per point (a centroid each),
+ * their rows added up in LDS; the work-group that finishes last adds the sums and counts of all of them to those of the single pass
+ * and divides (the guarded divide of the reference's divideMeansKernel, kernels.cu:149-163). Global atomics instead, a few hundred
+ * per address, took 44 to 80 us for 29000 points; the three launches before this one (exact pass, additions, division) took 44 us.
+ * Bound by latency: a dozen trips to memory.
+ */
+constexpr uint32_t FINISH_THREADS = 1024;
+constexpr uint32_t FINISH_GROUP = 32;                             /* lanes per point: k, dim <= 32 */
+constexpr uint32_t FINISH_POINTS = FINISH_THREADS / FINISH_GROUP; /* points of a work-group at a time */
+constexpr uint32_t FINISH_SHARE = 128;                            /* points that are worth a work-group */
+
 template <int LD, int LM>
-__global__ void __launch_bounds__(256)
-fused_fixup_kernel(const float* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment,
-                   float* __restrict__ means_out, size_t stride_means, uint32_t* __restrict__ sizes,
-                   const uint32_t* __restrict__ queue, const uint32_t* __restrict__ counters, uint32_t dim, uint32_t k)
+__global__ void __launch_bounds__(FINISH_THREADS)
+fused_finish_kernel(const float* __restrict__ data, size_t stride, const float* __restrict__ means_in, uint32_t* __restrict__ assignment,
+                    float* __restrict__ means_out, size_t stride_means, uint32_t* __restrict__ sizes,
+                    const uint32_t* __restrict__ queue, uint32_t* __restrict__ counters, float* __restrict__ partials, uint32_t dim, uint32_t k)
 {
-	__shared__ float sums[32 * 32];
+	__shared__ float centroids[32 * 33]; /* odd rows: consecutive centroids in different banks */
+	__shared__ float sums[32 * 32], rows[FINISH_POINTS][32];
 	__shared__ uint32_t members[32];
-	const uint32_t count = counters[0];
-	if ((uint64_t)blockIdx.x * blockDim.x >= (uint64_t)count * dim) return; /* nothing for this work-group */
-	for (uint32_t i = threadIdx.x; i < k * dim; i += blockDim.x) sums[i] = 0.0f;
-	if (threadIdx.x < 32) members[threadIdx.x] = 0u;
+	__shared__ bool last;
+	const uint32_t count = counters[0], tid = threadIdx.x;
+	const uint32_t working = min(gridDim.x, max(1u, (count + FINISH_SHARE - 1) / FINISH_SHARE));
+	if (blockIdx.x >= working) return;
+	for (uint32_t i = tid; i < k * dim; i += FINISH_THREADS) {
+		centroids[i / dim * 33 + i % dim] = means_in[elem<LM>(stride_means, i / dim, i % dim)];
+		sums[i] = 0.0f;
+	}
+	if (tid < 32) members[tid] = 0u;
 	__syncthreads();
-	const uint64_t total = (uint64_t)count * dim;
-	for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (uint64_t)gridDim.x * blockDim.x) {
-		const uint32_t entry = (uint32_t)(i / dim), d = (uint32_t)(i - (uint64_t)entry * dim);
-		const uint32_t pt = queue[2 * (size_t)entry];
-		const uint32_t t = assignment[pt];
-		unsafeAtomicAdd(&sums[t * dim + d], data[elem<LD>(stride, pt, d)]);
-		if (d == 0) atomicAdd(&members[t], 1u);
+	const uint32_t group = tid / FINISH_GROUP, lane = tid % FINISH_GROUP;
+	const float* mine = centroids + min(lane, k - 1) * 33;
+	float* x = rows[group];
+	/* (the two groups of a wavefront go round together: one without a point of its own repeats the last one and adds nothing) */
+	for (uint32_t base = blockIdx.x * FINISH_POINTS; base < count; base += working * FINISH_POINTS) {
+		const bool valid = base + group < count;
+		const uint32_t pt = queue[2 * (size_t)min(base + group, count - 1)];
+		const float coordinate = data[elem<LD>(stride, pt, min(lane, dim - 1))];
+		x[lane] = coordinate;
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		float sum = 0.0f;
+#pragma unroll 4
+		for (uint32_t d = 0; d < dim; ++d) {
+			const float diff = x[d] - mine[d];
+			const float sq = diff * diff;
+			sum = sum + sq;
+		}
+		const float dist = __builtin_sqrtf(sum);
+		/* distance bits, then the number: the first centroid's NaN beats everything, like in the scan (see evaluate_pair) */
+		unsigned long long key = lane >= k ? ~0ull : (lane == 0 && dist != dist) ? 0ull : (((unsigned long long)__float_as_uint(dist) << 32) | lane);
+#pragma unroll
+		for (int off = FINISH_GROUP / 2; off > 0; off >>= 1) {
+			const unsigned long long other = __shfl_xor(key, off);
+			key = other < key ? other : key;
+		}
+		const uint32_t winner = (uint32_t)key;
+		if (valid && lane == 0) { assignment[pt] = winner; atomicAdd(&members[winner], 1u); }
+		if (valid && lane < dim) unsafeAtomicAdd(&sums[winner * dim + lane], coordinate);
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
 	}
 	__syncthreads();
-	for (uint32_t e = threadIdx.x; e < k * dim; e += blockDim.x) {
-		const uint32_t c = e / dim, d = e - c * dim;
-		if (sums[e] != 0.0f) unsafeAtomicAdd(&means_out[elem<LM>(stride_means, c, d)], sums[e]);
+	/* this work-group's sums and counts: element e of all work-groups side by side would be written one word per line */
+	const uint32_t words = k * dim + k;
+	if (working > 1) {
+		for (uint32_t e = tid; e < words; e += FINISH_THREADS) {
+			const float v = e < k * dim ? sums[e] : __uint_as_float(members[e - k * dim]);
+			__hip_atomic_store(&partials[(size_t)blockIdx.x * words + e], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		}
+		/* They are there before the work-group counts as finished: stores of device scope pass the L2 by, so that having completed is
+		 * enough. (A fence of device scope writes the L2 back, per wavefront: 45 us for 230 work-groups.) */
+		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+		__syncthreads();
+		if (tid == 0) last = atomicAdd(&counters[FINISH_COUNTER], 1u) == working - 1;
+		__syncthreads();
+		if (!last) return;
 	}
-	if (threadIdx.x < k && members[threadIdx.x]) atomicAdd(&sizes[threadIdx.x], members[threadIdx.x]);
+	const uint32_t shares = FINISH_THREADS / 256; /* lanes per element, in passes of 256 elements */
+	float* share_sums = rows[0]; /* 1024 floats */
+	for (uint32_t e0 = 0; e0 < words; e0 += 256) {
+		const uint32_t e = e0 + tid % 256, share = tid / 256;
+		float sum = 0.0f;
+		uint32_t size = 0;
+		if (working > 1 && e < words) {
+			constexpr uint32_t BATCH = 16;
+			for (uint32_t g = share; g < working; g += BATCH * shares) {
+				float v[BATCH];
+#pragma unroll
+				for (uint32_t u = 0; u < BATCH; ++u)
+					v[u] = __hip_atomic_load(&partials[(size_t)min(g + u * shares, working - 1) * words + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+				for (uint32_t u = 0; u < BATCH; ++u)
+					if (g + u * shares < working) {
+						if (e < k * dim) sum += v[u];
+						else size += __float_as_uint(v[u]);
+					}
+			}
+		}
+		else if (share == 0 && e < words) {
+			if (e < k * dim) sum = sums[e];
+			else size = members[e - k * dim];
+		}
+		__syncthreads(); /* (rows, then the shares of the pass before, have been read) */
+		share_sums[tid] = e < k * dim ? sum : __uint_as_float(size);
+		__syncthreads();
+		if (share == 0 && e < words) {
+			for (uint32_t v = 1; v < shares; ++v) {
+				if (e < k * dim) sum += share_sums[v * 256 + tid];
+				else size += __float_as_uint(share_sums[v * 256 + tid]);
+			}
+			/* the sums of the queue; the counts first have to be complete */
+			if (e < k * dim) sums[e] = sum;
+			else { members[e - k * dim] = sizes[e - k * dim] + size; sizes[e - k * dim] = members[e - k * dim]; }
+		}
+	}
+	__syncthreads();
+	for (uint32_t e = tid; e < k * dim; e += FINISH_THREADS) {
+		float* mean = &means_out[elem<LM>(stride_means, e / dim, e % dim)];
+		const float sum = *mean + sums[e];
+		const uint32_t size = members[e / dim];
+		*mean = size > 0 ? sum / (float)size : sum;
+	}
 }
 
 /* the padded row widths whose ranking runs on the matrix cores (fused_matrix_kernel): measured against the lane-per-point
@@ -894,12 +989,12 @@ static int launch_fused_t(const AssignArgs& a, float* means_out, uint32_t* sizes
 }
 
 template <int LD, int LM>
-static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t* sizes, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t* sizes, const ClearOutputs& clear, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	const uint32_t dp = fused_dp(a.dim);
 	const uint32_t kp = round_up(a.k, TILE);
 	/* the ranking works in a frame moved to the middle of the centroids when they lie far from the origin */
-	int rc = launch_pack_means(a, ws, dp, kp, FRAME_MOVED_IF_FAR);
+	int rc = launch_pack_means(a, ws, dp, kp, FRAME_MOVED_IF_FAR, clear);
 	if (rc) return rc;
 	/* the bound of a ranking by chains of fused multiply-adds, or by the fp32 matrix instruction, see certificate.h;
 	 * 8 * 2^-23 for the roundings of x - m, c - m; the low bits of the values carry the centroid's number */
@@ -913,26 +1008,24 @@ static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t*
 	default: return fail(KMX_ERR_UNSUPPORTED, "fused iteration: dim %u is not supported by the single-pass kernel", a.dim);
 	}
 	if (rc) return rc;
-	/* the unresolved points: exact pass into the work-space assignment vector, then their share of the sums */
-	ws->exact_norms = ws->norms + plain_exact_norms_offset(kp);
-	rc = launch_recheck(a, ws, kp);
-	ws->exact_norms = nullptr;
-	if (rc) return rc;
-	KMX_LAUNCH_KERNEL((fused_fixup_kernel<LD, LM>), dim3(64), dim3(256), 0, stream(),
-	                   a.data, a.stride, a.assignment, means_out, a.stride_means, sizes, ws->queue, ws->counters, a.dim, a.k);
-	KMX_LAUNCH_CHECK("fused_fixup_kernel");
+	const uint32_t blocks = std::min(dev.compute_units, (a.n + FINISH_SHARE - 1) / FINISH_SHARE);
+	if ((rc = reserve_partials(ws, (size_t)blocks * (a.k * a.dim + a.k)))) return rc;
+	KMX_LAUNCH_KERNEL((fused_finish_kernel<LD, LM>), dim3(blocks), dim3(FINISH_THREADS), 0, stream(),
+	                   a.data, a.stride, a.means, a.assignment, means_out, a.stride_means, sizes, ws->queue, ws->counters, ws->partials, a.dim, a.k);
+	KMX_LAUNCH_CHECK("fused_finish_kernel");
 	return KMX_OK;
 }
 
 /* a.assignment: a vector of n entries -- the work-space vector (only the entries of the points left to the exact pass are
  * written), or with a.emit_assignment the caller's, which then receives every point's result; means_out and sizes are zero
- * on entry; the caller divides */
-int launch_fused_small(const AssignArgs& a, float* means_out, uint32_t* sizes, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+ * on entry unless clear_words says how many words of means_out (and the sizes) to clear first */
+int launch_fused_small(const AssignArgs& a, float* means_out, uint32_t* sizes, size_t clear_words, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
-	if (a.layout == KMX_AOS && a.layout_means == KMX_AOS) return launch_fused_layouts<KMX_AOS, KMX_AOS>(a, means_out, sizes, exec, ws, dev);
-	if (a.layout == KMX_AOS && a.layout_means == KMX_SOA) return launch_fused_layouts<KMX_AOS, KMX_SOA>(a, means_out, sizes, exec, ws, dev);
-	if (a.layout == KMX_SOA && a.layout_means == KMX_AOS) return launch_fused_layouts<KMX_SOA, KMX_AOS>(a, means_out, sizes, exec, ws, dev);
-	return launch_fused_layouts<KMX_SOA, KMX_SOA>(a, means_out, sizes, exec, ws, dev);
+	const ClearOutputs clear = { clear_words ? means_out : nullptr, clear_words, sizes };
+	if (a.layout == KMX_AOS && a.layout_means == KMX_AOS) return launch_fused_layouts<KMX_AOS, KMX_AOS>(a, means_out, sizes, clear, exec, ws, dev);
+	if (a.layout == KMX_AOS && a.layout_means == KMX_SOA) return launch_fused_layouts<KMX_AOS, KMX_SOA>(a, means_out, sizes, clear, exec, ws, dev);
+	if (a.layout == KMX_SOA && a.layout_means == KMX_AOS) return launch_fused_layouts<KMX_SOA, KMX_AOS>(a, means_out, sizes, clear, exec, ws, dev);
+	return launch_fused_layouts<KMX_SOA, KMX_SOA>(a, means_out, sizes, clear, exec, ws, dev);
 }
 
 } // namespace kmx

@@ -85,6 +85,7 @@ int reserve_carried(Workspace* ws, size_t words);
 int reserve_listed(Workspace* ws, size_t words);
 int two_level_mode(); /* kmx_set_two_level_sweep */
 constexpr uint32_t CELLS_COUNTER = 5;  /* word of Workspace::counters that counts the list units handed out by build_cells_kernel */
+constexpr uint32_t FINISH_COUNTER = 6; /* and the one that counts the work-groups fused_finish_kernel has behind it */
 constexpr uint32_t LISTED_COUNTER = 4; /* word of Workspace::counters that holds the length of Workspace::listed */
 
 #define KMX_HIP(call)                                                                                         \
@@ -180,7 +181,8 @@ uint32_t screen_unit_rows(uint32_t dim);
 /* assign_mfma.hip / assign_lds_fma.hip: return KMX_ERR_UNSUPPORTED (without message side effects
  * beyond kmx_last_error) when the shape does not fit the variant. */
 /* shared by both fast variants: packed centroids (-2c rows of dp floats, kp rows), norms, transposed copy, empty queue */
-int launch_pack_means(const AssignArgs& a, Workspace* ws, uint32_t dp, uint32_t kp, uint32_t moved); /* FRAME_KEPT, FRAME_MOVED, FRAME_MOVED_IF_FAR (assign_mfma_impl.h) */
+struct ClearOutputs { float* means; size_t words; uint32_t* sizes; }; /* outputs to clear on the way (means: nullptr: none) */
+int launch_pack_means(const AssignArgs& a, Workspace* ws, uint32_t dp, uint32_t kp, uint32_t moved, const ClearOutputs& clear = {}); /* FRAME_KEPT, FRAME_MOVED, FRAME_MOVED_IF_FAR (assign_mfma_impl.h) */
 bool mfma_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_mfma(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev);
@@ -235,8 +237,6 @@ int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Works
 /* whether launch_update would copy the SoA points of u into AoS rows first, and that copy: ws->rows_copy, rows of dim floats */
 bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev);
 int launch_rows_from_soa(const float* data, size_t stride, uint32_t dim, uint32_t n, Workspace* ws, const DeviceInfo& dev);
-int launch_divide_means(const UpdateArgs& u);
-int clear_update_outputs(const UpdateArgs& u); /* means (replica 0) and cluster sizes := 0 in one launch */
 
 /* update_ordered.hip: KMX_UPDATE_SERIAL_ORDER for floats and doubles -- stable counting sort of the point numbers by
  * cluster, then one lane per (cluster, coordinate) adds the members in ascending point order and divides: the bits of
@@ -259,7 +259,7 @@ void forget_prepared_points_f64(const void* dst, size_t bytes);
  * (only the entries of the points left to the exact pass are written); means_out and sizes are zero on entry and hold
  * sums and counts on return (the caller divides). */
 bool fused_small_supports(uint32_t dim, uint32_t k, int layout, size_t stride, uint32_t n);
-int launch_fused_small(const AssignArgs& a, float* means_out, uint32_t* sizes, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
+int launch_fused_small(const AssignArgs& a, float* means_out, uint32_t* sizes, size_t clear_words, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 
 } // namespace kmx
 

@@ -690,10 +690,7 @@ int kmx_fused_f32(int variant,
 		AssignArgs a{ data, layout, stride, means_in, layout_means, stride_means, ws->fused_assignment, dim, k, n };
 		UpdateArgs small{ data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
 		if (small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) return launch_iteration_small(a, small, exec, ws, *dev);
-		rc = launch_fused_small(a, means_out, cluster_sizes, exec, ws, *dev);
-		if (rc) return rc;
-		UpdateArgs u{ data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
-		return launch_divide_means(u);
+		return launch_fused_small(a, means_out, cluster_sizes, 0, exec, ws, *dev);
 	}
 	return two_passes(data, layout, stride, means_in, means_out, layout_means, stride_means, ws->fused_assignment, cluster_sizes, dim, k, n, exec);
 }
@@ -729,15 +726,11 @@ int kmx_iteration_f32(const float* data, int layout, size_t stride,
 			g_last_iteration_passes = 1;
 			return launch_iteration_small(small, u, exec, ws, *dev);
 		}
-		rc = clear_update_outputs(u); /* the single-pass kernel accumulates into them */
-		if (rc) return rc;
 		AssignArgs a{ data, layout, stride, means_in, layout_means, stride_means, assignment, dim, k, n };
 		a.emit_assignment = true;
 		g_last_assign_variant = KMX_ASSIGN_LDS_FMA; /* the ranking of the single-pass kernel: fused multiply-adds on scalar operands */
-		rc = launch_fused_small(a, means_out, cluster_sizes, exec, ws, *dev);
-		if (rc) return rc;
 		g_last_iteration_passes = 1;
-		return launch_divide_means(u);
+		return launch_fused_small(a, means_out, cluster_sizes, layout_means == KMX_AOS ? (size_t)k * stride_means : (size_t)dim * stride_means, exec, ws, *dev);
 	}
 	const DeviceInfo* dev = nullptr;
 	int rc = device_info(&dev);

@@ -1182,19 +1182,6 @@ static int launch_update_t(int variant, const UpdateArgs& u, kmx_exec_params* ex
 	return KMX_OK;
 }
 
-/* means[c][d] /= count[c] for the non-empty clusters (divideMeansKernel of the reference, kernels.cu:149-171) */
-int launch_divide_means(const UpdateArgs& u)
-{
-	const uint32_t total = u.k * u.dim;
-	const uint32_t blocks = std::min<uint32_t>((total + 255) / 256, 1024);
-	if (u.layout_means == KMX_AOS)
-		KMX_LAUNCH_KERNEL((divide_means_kernel<KMX_AOS>), dim3(blocks), dim3(256), 0, stream(), u.means, u.stride_means, u.cluster_sizes, u.dim, u.k);
-	else
-		KMX_LAUNCH_KERNEL((divide_means_kernel<KMX_SOA>), dim3(blocks), dim3(256), 0, stream(), u.means, u.stride_means, u.cluster_sizes, u.dim, u.k);
-	KMX_LAUNCH_CHECK("divide_means_kernel");
-	return KMX_OK;
-}
-
 /*
  * SoA points and the tuned variant: the kernels that read whole rows (sorted chunks, private copies) are 5 to 10 times
  * faster than anything that adds element by element (measured at N = 2M, d = 32, k = 1024: 0.07 ms against 0.68 ms for the
@@ -1257,8 +1244,6 @@ int noalloc_workspace(Workspace** ws)
 	*ws = &w;
 	return KMX_OK;
 }
-
-int clear_update_outputs(const UpdateArgs& u) { return clear_outputs(u); }
 
 bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev)
 {
