@@ -177,7 +177,7 @@ def double_main(km, args, spec, data, means0):
     update_bytes = 8.0 * (n * dim + k * dim) + 4.0 * (n + k)
     update_gbs = update_bytes / (k_update * 1e-3) / 1e9
     if ran_variant == km.ASSIGN_MFMA_BF16X3:
-        roofline = {"kernel": "ranking sweep on float copies (split-bf16 MFMA)", "bound": "mfma", "achieved": round(algorithmic, 1),
+        roofline = {"kernel": "ranking sweep on float copies (half-precision MFMA)", "bound": "mfma", "achieved": round(algorithmic, 1),
                     "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(algorithmic / PEAK_BF16_TFLOPS, 4), "traffic": None,
                     "flops_counted": "algorithmic: 2 N k d per launch"}
     elif k >= 64:
@@ -269,7 +269,7 @@ def main():
                     help="replay a recorded pair of iterations (HIP graph) instead of launching every kernel of the timed "
                          "iterations one by one (measured: no gain on this runtime, 0.042 vs 0.035 ms at configuration 1)")
     ap.add_argument("--two-level", type=int, default=1, choices=[0, 1, 2],
-                    help="the split-bf16 sweep in two levels: 0 never, 1 where it pays (default), 2 wherever the kernels allow it")
+                    help="one half-precision product per dimension: 0 never (three bf16 products), 1 where it pays (default), 2 wherever the kernels allow it")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="one device-to-device copy of the point array before the timed region (a copy kernel of known "
                          "size, to scale FETCH_SIZE / WRITE_SIZE counter readings)")
@@ -350,10 +350,10 @@ def main():
     assign_gbs = assign_bytes / (k_assign * 1e-3) / 1e9
     # the dominant kernel is the assignment sweep; it is compute-bound unless k is tiny (flop/byte = k/2)
     if k >= 64 and ran_variant == km.ASSIGN_MFMA_BF16X3:
-        # The sweep runs on the bf16 matrix pipeline: the fraction is the ALGORITHMIC work (one multiply-add per point x
-        # centroid x dim) against that pipeline's peak. Each algorithmic multiply-add is executed as three bf16 products
-        # (split operands); the executed rate is reported beside it, not as the roofline fraction.
-        roofline = {"kernel": "assignment sweep (split-bf16 MFMA)", "bound": "mfma", "achieved": round(assign_tflops, 1),
+        # The sweep runs on the 16-bit matrix pipeline: the fraction is the ALGORITHMIC work (one multiply-add per point x
+        # centroid x dim) against that pipeline's peak. With --two-level 0 each algorithmic multiply-add is executed as three
+        # bf16 products (split operands); the executed rate is reported beside it, not as the roofline fraction.
+        roofline = {"kernel": "assignment sweep (%s MFMA)" % ("split-bf16" if args.two_level == 0 else "half-precision"), "bound": "mfma", "achieved": round(assign_tflops, 1),
                     "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(assign_tflops / PEAK_BF16_TFLOPS, 4),
                     "traffic": None, "flops_counted": "algorithmic: 2 N k d per launch",
                     "frac_of_fp32_peak": round(assign_tflops / PEAK_FP32_TFLOPS, 4)}
@@ -362,8 +362,9 @@ def main():
             roofline.update({"executed_tflops": round(3.0 * assign_tflops, 1), "executed_frac": round(3.0 * assign_tflops / PEAK_BF16_TFLOPS, 4),
                              "executed_note": "3 bf16 products per point x centroid x dim on the bf16 matrix pipeline"})
         else:
-            roofline["executed_note"] = ("two levels where they pay: one bf16 product per point x centroid x dim for every point, three more "
-                                         "for the points the first level cannot settle; packed rows (dim <= 4): one instruction per tile")
+            roofline["executed_note"] = ("one half-precision product per point x centroid x dim where it pays (three bf16 products elsewhere); rows "
+                                         "of 2 to 4 dimensions and many points go through a grid of cells, which executes a small part of the "
+                                         "counted work")
     elif k >= 64:
         roofline = {"kernel": "assignment sweep", "bound": "mfma", "achieved": round(assign_tflops, 2),
                     "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": round(assign_tflops / PEAK_FP32_TFLOPS, 4),
@@ -389,7 +390,7 @@ def main():
         "vs_baseline": round(ms_per_step / PUBLISHED_MS[args.config], 4) if args.config in PUBLISHED_MS else None,
         "baseline_note": "published: 25.45 ms on V100 SXM2 for this shape (reference results/README.md:20); lower is better"
                          if args.config in PUBLISHED_MS else None,
-        "dtype": "f32 (sweep on bf16x3 split operands, f32 accumulate; exact f32 re-evaluation of uncertified points)"
+        "dtype": "f32 (sweep on half-precision or bf16x3 split operands, f32 accumulate; exact f32 re-evaluation of uncertified points)"
                  if ran_variant == km.ASSIGN_MFMA_BF16X3 else "f32",
         "data": "synthetic",
         "config": {"workload": "benchmark configuration %d: N=%d d=%d k=%d, %s, initial centroids = first k points, seed %d"

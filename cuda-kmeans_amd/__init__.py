@@ -443,7 +443,7 @@ def set_queued_rows_limit(nbytes):
 
 
 def set_two_level_sweep(mode):
-    """kmx_set_two_level_sweep: 0 = one level always, 1 = two levels where they pay (default), 2 = wherever the kernels allow."""
+    """kmx_set_two_level_sweep: 0 = three products always, 1 = one product where it pays (default), 2 = wherever the kernels allow."""
     check(hip_lib().kmx_set_two_level_sweep(mode))
 
 
