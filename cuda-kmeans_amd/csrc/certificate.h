@@ -43,9 +43,10 @@
  *        accumulation <= (d + 2) u' 2 S
  *        dropped = sum_i c'hi_i (x_i - xhi_i) + (c'_i - c'hi_i) x_i <= |c'hi| |xlo| + |c'lo| |x|
  *     with xlo = x - xhi, whose norm the lane computes when it rounds the point (the subtraction is exact in fp32),
- *     |c'hi| <= (1 + 2^-8) |c'| and |c'lo| from the packing kernel (up to its two arguments). The bound is about
- *     2^-11 |c'||x|, thirty times the three-product one, for a third of the matrix work: it settles 90 to 99.5 % of the
- *     points, the others get their serial result.
+ *     |c'lo| from the packing kernel (up to its two arguments) and |c'hi| <= |c'| + |c'lo|: below the smallest normal
+ *     half-precision number the part rounded away can be as large as the value itself, so no factor of |c'| would do.
+ *     The bound is about 2^-11 |c'||x|, thirty times the three-product one, for a third of the matrix work: it settles
+ *     90 to 99.5 % of the points, the others get their serial result.
  * tau = kd S + TRUNC_FACTOR * (bound of the dropped products); kd = (12 d + 8 + 2 d + 12 + slack) u' and
  * (16 d + 8 + 2 d + 12 + 8 + slack) u'; TRUNC_FACTOR = 2 plus 1/16 for the fp32 roundings in the norms and square roots.
  * Values the bound does not cover (NaN, infinities, sums that overflow) make tau NaN or infinite, and the
@@ -99,7 +100,7 @@ KMX_HD CertCoeffs cert_coeffs_level1(const CentroidBounds& c)
 {
 	const float cnorm = 2.0f * __builtin_sqrtf(c.c2max); /* |c'| */
 	const float clo = __builtin_sqrtf(c.mid2max) + __builtin_sqrtf(c.rest2max); /* >= |c' - c'hi| */
-	return CertCoeffs{ c.c2max, CERT_TRUNC_FACTOR * (cnorm * (1.0f + CERT_BF16_UNIT)), CERT_TRUNC_FACTOR * clo };
+	return CertCoeffs{ c.c2max, CERT_TRUNC_FACTOR * (cnorm + clo), CERT_TRUNC_FACTOR * clo };
 }
 
 KMX_HD CertCoeffs cert_coeffs_packed(const CentroidBounds& c)

@@ -224,6 +224,26 @@ def test_tau_of_the_first_level_covers_one_product_per_dimension(km, dim, kind):
     assert not wrong.any(), "%d certified pairs contradict the serial comparison" % int(wrong.sum())
 
 
+@pytest.mark.parametrize("dim", [5, 16, 64, 256])
+@pytest.mark.parametrize("exponent", [-25, -24, -20, -14, 3])
+def test_tau_of_one_half_precision_product_covers_values_below_the_smallest_normal_one(km, dim, exponent):
+    """Coordinates just above 2^-25 round up to the smallest half-precision number, 2^-24: the rounded centroid is twice as long as
+    the centroid, and what is dropped of both operands is as large as they are. tau (form 4) must cover twice the dropped sum of every
+    pair; nothing is allowed for here but the dropped products (squares of such numbers are exact in fp32)."""
+    rng = np.random.default_rng(100 * dim + exponent)
+    size = np.float32(2.0 ** exponent)
+    x = (size * (1 + rng.integers(1, 512, (64, dim)) * 2.0 ** -14)).astype(np.float32)
+    c = (size * (1 + rng.integers(1, 512, (8, dim)) * 2.0 ** -14)).astype(np.float32)     # c' = -2c, as the packing kernel has it
+    xh, ch = x.astype(np.float16).astype(np.float32), c.astype(np.float16).astype(np.float32)
+    kept = ch.astype(np.float64) @ xh.astype(np.float64).T
+    exact = c.astype(np.float64) @ x.astype(np.float64).T
+    x2, xlo2 = (x.astype(np.float64) ** 2).sum(1), ((x - xh).astype(np.float64) ** 2).sum(1)
+    c2max, clo2 = float((c.astype(np.float64) ** 2).sum(1).max() / 4), float(((c - ch).astype(np.float64) ** 2).sum(1).max())
+    tau = np.array([km.certificate_tau(4, dim, float(x2[i]), float(xlo2[i]), c2max, clo2, 0.0) for i in range(len(x))])
+    need = 2 * np.abs(kept - exact).max(0)
+    assert np.all(need <= tau), "tau misses %d points (worst ratio %.3f)" % (int((need > tau).sum()), float((need / tau).max()))
+
+
 @pytest.mark.parametrize("dim", [2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("kind", ["adversarial", "ties0", "ties100", "ties10000"])
 def test_tau_of_the_vector_alu_sweeps_covers_a_chain_of_fused_multiply_adds(km, dim, kind):
