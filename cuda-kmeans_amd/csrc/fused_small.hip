@@ -993,8 +993,11 @@ static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t*
 {
 	const uint32_t dp = fused_dp(a.dim);
 	const uint32_t kp = round_up(a.k, TILE);
+	const uint32_t blocks = std::min(dev.compute_units, (a.n + FINISH_SHARE - 1) / FINISH_SHARE);
+	int rc = reserve_partials(ws, (size_t)blocks * (a.k * a.dim + a.k)); /* (ahead of the launches: a recording that cannot have it is refused whole) */
+	if (rc) return rc;
 	/* the ranking works in a frame moved to the middle of the centroids when they lie far from the origin */
-	int rc = launch_pack_means(a, ws, dp, kp, FRAME_MOVED_IF_FAR, clear);
+	rc = launch_pack_means(a, ws, dp, kp, FRAME_MOVED_IF_FAR, clear);
 	if (rc) return rc;
 	/* the bound of a ranking by chains of fused multiply-adds, or by the fp32 matrix instruction, see certificate.h;
 	 * 8 * 2^-23 for the roundings of x - m, c - m; the low bits of the values carry the centroid's number */
@@ -1008,8 +1011,6 @@ static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t*
 	default: return fail(KMX_ERR_UNSUPPORTED, "fused iteration: dim %u is not supported by the single-pass kernel", a.dim);
 	}
 	if (rc) return rc;
-	const uint32_t blocks = std::min(dev.compute_units, (a.n + FINISH_SHARE - 1) / FINISH_SHARE);
-	if ((rc = reserve_partials(ws, (size_t)blocks * (a.k * a.dim + a.k)))) return rc;
 	KMX_LAUNCH_KERNEL((fused_finish_kernel<LD, LM>), dim3(blocks), dim3(FINISH_THREADS), 0, stream(),
 	                   a.data, a.stride, a.means, a.assignment, means_out, a.stride_means, sizes, ws->queue, ws->counters, ws->partials, a.dim, a.k);
 	KMX_LAUNCH_CHECK("fused_finish_kernel");

@@ -296,6 +296,8 @@ extern "C" {
 static int two_passes(const float* data, int layout, size_t stride, const float* means_in, float* means_out, int layout_means, size_t stride_means,
                       uint32_t* assignment, uint32_t* cluster_sizes, uint32_t dim, uint32_t k, uint32_t n, kmx_exec_params* exec);
 
+static int g_last_iteration_passes = 0;
+
 const char* kmx_last_error(void) { return g_error; }
 
 int kmx_device_count(int* count)
@@ -509,26 +511,25 @@ int kmx_reserve_f32(int assign_variant, int update_variant, int layout, int layo
 	/* the launchers themselves say what they need: they are walked with the launches switched off, on pointers that are
 	 * never followed (16-byte aligned, like buffers from kmx_malloc) */
 	float* const points = (float*)(uintptr_t)4096;
+	float* const other = (float*)(uintptr_t)8192; /* (means_in and means_out must differ) */
 	uint32_t* const words = (uint32_t*)(uintptr_t)4096;
 	const size_t stride = layout == KMX_AOS ? dim : n, stride_means = layout_means == KMX_AOS ? dim : k;
 	kmx_exec_params exec = { 256, 0, 0, 1, 1, 1 };
-	const int last_variant = g_last_assign_variant;
+	const int last_variant = g_last_assign_variant, last_passes = g_last_iteration_passes;
 	g_sizing = true;
 	int rc = kmx_assign_f32(assign_variant, points, layout, stride, points, layout_means, stride_means, nullptr, words, dim, k, n, &exec);
 	if (rc == KMX_OK) rc = kmx_update_f32(update_variant, points, layout, stride, words, points, layout_means, stride_means, words, dim, k, n, &exec);
-	/* an iteration on SoA points may run on an AoS copy of them */
-	if (rc == KMX_OK && layout == KMX_SOA) rc = two_passes(points, layout, stride, points, points, layout_means, stride_means, words, words, dim, k, n, &exec);
-	if (rc == KMX_OK) {
-		Workspace* ws = nullptr;
-		rc = workspace(&ws);
-		if (rc == KMX_OK) rc = reserve_fused_assignment(ws, n); /* kmx_fused_f32 keeps its assignment vector in the work space */
-	}
+	/* the calls that do both choose kernels of their own: small inputs and single passes keep partial sums, SoA points an AoS copy */
+	if (rc == KMX_OK) rc = kmx_iteration_f32(points, layout, stride, points, other, layout_means, stride_means, words, words, dim, k, n, &exec);
+	for (int variant : { KMX_FUSED_TWO_PASS, KMX_FUSED_BEST })
+		if (rc == KMX_OK) rc = kmx_fused_f32(variant, points, layout, stride, points, other, layout_means, stride_means, words, dim, k, n, &exec);
 	if (rc == KMX_OK) {
 		Workspace* scratch = nullptr;
 		rc = noalloc_workspace(&scratch); /* kmx_update_f32_noalloc: the address of its scratch array on this device */
 	}
 	g_sizing = false;
 	g_last_assign_variant = last_variant;
+	g_last_iteration_passes = last_passes;
 	return rc;
 }
 
@@ -694,8 +695,6 @@ int kmx_fused_f32(int variant,
 	}
 	return two_passes(data, layout, stride, means_in, means_out, layout_means, stride_means, ws->fused_assignment, cluster_sizes, dim, k, n, exec);
 }
-
-static int g_last_iteration_passes = 0;
 
 int kmx_iteration_f32(const float* data, int layout, size_t stride,
                       const float* means_in, float* means_out, int layout_means, size_t stride_means,

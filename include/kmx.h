@@ -147,7 +147,8 @@ int kmx_assign_f32(int variant,
 /*
  * Sizes the library's work space (packed centroids, recheck queue, copied rows, partial sums, the values carried between
  * the sweeps of slices of centroids) for kmx_assign_f32 /
- * kmx_update_f32 / kmx_fused_f32 calls of this shape and these variants, so that those calls allocate nothing afterwards
+ * kmx_update_f32 calls of this shape and these variants and for kmx_iteration_f32 and kmx_fused_f32 calls of this shape, so that
+ * those calls allocate nothing afterwards
  * (no counterpart in the reference, whose runners allocate nothing: cuda.hpp:54-64 allocates everything in initialize()).
  * Without it the first call of a shape grows the work space itself, which waits for the stream and calls hipMalloc; a
  * call with a different LDS budget (shared_mem_bytes) than the default may still grow it. Not while a graph is recorded.

@@ -1040,3 +1040,39 @@ def test_reserved_work_space_is_enough(km, orc, gpu, dim, k, n, layout):
     assert rel_err(out.read(np.float32, k * dim), om) < CENTROID_RTOL
     for b in (d, m, a, out, sizes):
         b.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,k,n,layout", [(16, 16, 1 << 20, AOS), (20, 128, 10240, AOS), (8, 64, 65536, SOA), (4, 8, 300001, SOA), (50, 300, 40000, SOA)])
+def test_reserved_work_space_is_enough_for_whole_iterations(km, orc, gpu, dim, k, n, layout):
+    """The same for the calls that assign and update in one: single passes and small inputs keep partial sums of their own. Every replay
+    (with eager work in between) gives the oracle's assignment and counts, and its centroids."""
+    rng = np.random.default_rng(dim * 7 + k)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    cents = rows[rng.choice(n, k, replace=False)].copy()
+    stride = dim if layout == AOS else n
+    d = km.DeviceBuffer(4 * n * dim); d.write(rows.ravel() if layout == AOS else rows.T.copy().ravel())
+    m = km.DeviceBuffer(4 * k * dim); m.write(cents.ravel())
+    a = km.DeviceBuffer(4 * n); out = km.DeviceBuffer(4 * k * dim); sizes = km.DeviceBuffer(4 * k)
+    oa = orc.assign(rows.ravel(), cents.ravel(), dim, k, n, threads=0, fast=True)
+    om, osz = orc.update(rows.ravel(), oa, dim, k, n, threads=0)
+    for fused in (False, True):
+        km.sync()
+        km.check(km.hip_lib().kmx_shutdown())
+        km.reserve(km.ASSIGN_BEST, km.UPDATE_ATOMIC_SHM, layout, AOS, dim, k, n)
+        with km.Graph() as g:
+            if fused:
+                out.zero(); sizes.zero()
+                km.fused(km.FUSED_BEST, d, layout, stride, m, out, AOS, dim, sizes, dim, k, n)
+            else:
+                km.iteration(d, layout, stride, m, out, AOS, dim, a, sizes, dim, k, n)
+        for _ in range(3):
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32)); out.write(np.full(k * dim, np.nan, np.float32)); sizes.write(np.full(k, 7, np.uint32))
+            g.launch()
+            km.sync()
+            assert fused or np.array_equal(a.read(np.uint32, n), oa)
+            assert np.array_equal(sizes.read(np.uint32, k), osz)
+            assert rel_err(out.read(np.float32, k * dim), om) < CENTROID_RTOL
+        g.destroy()
+    for b in (d, m, a, out, sizes):
+        b.free()
