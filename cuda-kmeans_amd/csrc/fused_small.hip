@@ -878,6 +878,8 @@ fused_finish_kernel(const float* __restrict__ data, size_t stride, const float* 
 		if (tid == 0) last = atomicAdd(&counters[FINISH_COUNTER], 1u) == working - 1;
 		__syncthreads();
 		if (!last) return;
+		/* the counter said that all partial sums are there; nothing below is read ahead of it (one fence per call: only the last work-group gets here) */
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 	}
 	const uint32_t shares = FINISH_THREADS / 256; /* lanes per element, in passes of 256 elements */
 	float* share_sums = rows[0]; /* 1024 floats */
