@@ -70,7 +70,7 @@ bool takes_cells(const AssignArgs& a, uint32_t lds_budget)
 
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
 {
-	return a.layout == KMX_SOA && bf16_supports(a, dev) && takes_rank16(a, lds_budget_of(exec, dev)) &&
+	return a.layout == KMX_SOA && bf16_supports(a, lds_budget_of(exec, dev), dev) && takes_rank16(a, lds_budget_of(exec, dev)) &&
 	       (size_t)a.n * round_up(a.dim, 8) * sizeof(float) <= queued_rows_limit();
 }
 
@@ -192,10 +192,10 @@ pack_means_bf16_kernel(const float* __restrict__ means, size_t stride_means, flo
 	}
 }
 
-bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev)
+bool bf16_supports(const AssignArgs& a, uint32_t lds_budget, const DeviceInfo& dev)
 {
 	const uint32_t kb = pick_kb(a.dim);
-	if (kb == 0) return wide_supports(a, dev) && (!a.ranking_only || wide16_supports(a, dev)); /* (the caller's pass over a queue takes no such rows) */
+	if (kb == 0) return wide_supports(a, lds_budget) && (!a.ranking_only || wide16_supports(a, lds_budget)); /* (the caller's pass over a queue takes no such rows) */
 	/* two tiles (the double-buffered stream of the centroid block) plus the static flag lists must fit */
 	return (size_t)(tile_floats(KBLOCK * kb + ROW_PAD) + NORM_TILE) * 4 * 2 + 2 * FLAG_CAP * MFMA_WAVES * 4 + 1024 <= dev.lds_bytes;
 }

@@ -605,27 +605,29 @@ constexpr uint32_t WIDE_MAX_DIM = 2560; /* what the exact pass takes */
 static uint32_t wide_buffer_bytes(uint32_t pt, bool x3) { return (x3 ? 2u : 1u) * 2 * WIDE_BLOCKS * (pt * TILE + WIDE_ROW_PAD) * 16; }
 static uint32_t wide_static_bytes(uint32_t pt, uint32_t nt) { return (3 * WIDE_WAVES * pt * TILE + 3 * pt * TILE + WIDE_WAVES * nt * TILE + 2 * WIDE_LIST + 3 * WIDE_WAVES + 64) * 4; }
 
-bool wide_supports(const AssignArgs& a, const DeviceInfo& dev)
+/* LDS of a sweep with units of 32 pt points, nt tiles per wavefront, two buffers */
+static uint32_t wide_sweep_bytes(uint32_t dp, uint32_t pt, uint32_t nt, bool x3) { return dp * 4 + 2 * wide_buffer_bytes(pt, x3) + wide_static_bytes(pt, nt); }
+
+bool wide_supports(const AssignArgs& a, uint32_t lds_budget)
 {
-	const uint32_t dp = round_up(a.dim, WIDE_CHUNK);
-	return a.dim > 256 && a.dim <= WIDE_MAX_DIM && dp * 4 + 2 * wide_buffer_bytes(4, true) + wide_static_bytes(4, 2) <= dev.lds_bytes;
+	return a.dim > 256 && a.dim <= WIDE_MAX_DIM && (wide16_supports(a, lds_budget) || wide_sweep_bytes(round_up(a.dim, WIDE_CHUNK), 1, 1, true) <= lds_budget);
 }
 
 template <int PT, int NT, bool X3>
-static int launch_wide_sweep(const AssignArgs& a, WideArgs w, const DeviceInfo& dev, kmx_exec_params* exec)
+static int launch_wide_sweep(const AssignArgs& a, WideArgs w, uint32_t lds_budget, const DeviceInfo& dev, kmx_exec_params* exec)
 {
 	const bool vec = a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data & 15) == 0;
 	void (*kernel)(WideArgs) = a.layout == KMX_SOA ? wide_sweep_kernel<PT, NT, X3, KMX_SOA, false>
 	                           : vec ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, true> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, false>;
 	const uint32_t chunks = w.dp / WIDE_CHUNK, groups = (w.kp / TILE + WIDE_WAVES * NT - 1) / (WIDE_WAVES * NT);
 	const uint32_t buffer = wide_buffer_bytes(PT, X3);
-	const uint32_t room = dev.lds_bytes - wide_static_bytes(PT, NT) - w.dp * 4;
+	const uint32_t room = lds_budget - wide_static_bytes(PT, NT) - w.dp * 4; /* (wide_sweep_bytes fits) */
 	/* all chunks of a unit stay in LDS where another group of centroids wants them again */
 	w.buffers = std::min(chunks, (groups > 1 && (uint64_t)chunks * buffer <= room) ? chunks : 2u);
 	const uint32_t lds_bytes = w.dp * 4 + w.buffers * buffer;
 	const uint32_t units = (a.n + PT * TILE - 1) / (PT * TILE);
 	const uint32_t grid = std::min(units, dev.compute_units);
-	if (exec) exec->block_count = grid;
+	exec->block_count = grid;
 	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
 	KMX_LAUNCH_KERNEL(kernel, dim3(grid), dim3(WIDE_THREADS), lds_bytes, stream(), w);
 	KMX_LAUNCH_CHECK("wide_sweep_kernel");
@@ -670,12 +672,14 @@ static int launch_assign_wide16(const AssignArgs& a, uint32_t dp, kmx_exec_param
 	                     cert_kd_level1(a.dim) + cert_kd_keyed(5) + 8.0f * CERT_UNIT + a.kd_extra, 0.0f };
 	if (!sizing_only() && (rc = check_wide_plan(a, w, ws, true))) return rc;
 	if ((rc = profile_begin(0))) return rc;
-	/* units of 128 points, or, where those do not reach half of the compute units, of 32 */
-	rc = a.n >= 64 * dev.compute_units ? launch_wide_sweep<4, 2, false>(a, w, dev, exec) : launch_wide_sweep<1, 1, false>(a, w, dev, exec);
+	/* units of 128 points, or, where those do not reach half of the compute units or do not fit, of 32 */
+	const uint32_t budget = lds_budget_of(exec, dev);
+	const bool large = a.n >= 64 * dev.compute_units && wide_sweep_bytes(dp, 4, 2, false) <= budget;
+	rc = large ? launch_wide_sweep<4, 2, false>(a, w, budget, dev, exec) : launch_wide_sweep<1, 1, false>(a, w, budget, dev, exec);
 	if (rc) return rc;
 	if ((rc = profile_end(0))) return rc;
 	const size_t stride = a.layout == KMX_AOS ? a.stride : 1, step = a.layout == KMX_AOS ? 1 : a.stride;
-	const uint32_t groups = wide16_groups(dp, a.points64 != nullptr, dev.lds_bytes);
+	const uint32_t groups = wide16_groups(dp, a.points64 != nullptr, budget);
 	auto exact = [&](auto* points, auto* centroids) -> int {
 		typedef typename std::remove_const<typename std::remove_pointer<decltype(points)>::type>::type F;
 		const ExactArgs<F> e = { a.data, stride, step, a.dim, points, stride, step, a.dim, centroids, (const f16x8*)ws->packed16, norms,
@@ -689,16 +693,19 @@ static int launch_assign_wide16(const AssignArgs& a, uint32_t dp, kmx_exec_param
 	return KMX_OK;
 }
 
-bool wide16_supports(const AssignArgs& a, const DeviceInfo& dev)
+bool wide16_supports(const AssignArgs& a, uint32_t lds_budget)
 {
-	return two_level_mode() != 0 && a.k < (1u << 25) && (!a.ranking_only || a.points64) && wide16_groups(round_up(a.dim, WIDE_CHUNK), a.points64 != nullptr, dev.lds_bytes) > 0;
+	const uint32_t dp = round_up(a.dim, WIDE_CHUNK);
+	return two_level_mode() != 0 && a.k < (1u << 25) && (!a.ranking_only || a.points64) && wide_sweep_bytes(dp, 1, 1, false) <= lds_budget &&
+	       wide16_groups(dp, a.points64 != nullptr, lds_budget) > 0;
 }
 
 int launch_assign_wide(const AssignArgs& args, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	AssignArgs a = args;
 	const uint32_t dp = round_up(a.dim, WIDE_CHUNK), kp = round_up(a.k, TILE);
-	if (wide16_supports(a, dev))
+	const uint32_t budget = lds_budget_of(exec, dev);
+	if (wide16_supports(a, budget))
 		return launch_assign_wide16(a, dp, exec, ws, dev);
 	const bool moved = !a.ranking_only; /* (the double path hands over copies it has moved itself) */
 	int rc = reserve_packed(ws, wide_plane_units(kp, dp) * 2 * 4, wide_norms_floats(kp, dp), (size_t)kp * a.dim);
@@ -714,7 +721,8 @@ int launch_assign_wide(const AssignArgs& args, kmx_exec_params* exec, Workspace*
 	                     cert_kd_split(a.dim) + cert_kd_keyed(4) + (moved ? 8.0f * CERT_UNIT : 0.0f) + a.kd_extra, moved ? cert_kd_unmoved(a.dim) : 0.0f };
 	if (!sizing_only() && (rc = check_wide_plan(a, w, ws, false))) return rc;
 	if ((rc = profile_begin(0))) return rc;
-	rc = a.n >= 128 * dev.compute_units ? launch_wide_sweep<4, 1, true>(a, w, dev, exec) : launch_wide_sweep<1, 1, true>(a, w, dev, exec);
+	const bool large = a.n >= 128 * dev.compute_units && wide_sweep_bytes(dp, 4, 1, true) <= budget;
+	rc = large ? launch_wide_sweep<4, 1, true>(a, w, budget, dev, exec) : launch_wide_sweep<1, 1, true>(a, w, budget, dev, exec);
 	if (rc) return rc;
 	if ((rc = profile_end(0))) return rc;
 	if (a.ranking_only) return KMX_OK; /* the caller resolves the queued points */

@@ -185,7 +185,7 @@ struct ClearOutputs { float* means; size_t words; uint32_t* sizes; }; /* outputs
 int launch_pack_means(const AssignArgs& a, Workspace* ws, uint32_t dp, uint32_t kp, uint32_t moved, const ClearOutputs& clear = {}); /* FRAME_KEPT, FRAME_MOVED, FRAME_MOVED_IF_FAR (assign_mfma_impl.h) */
 bool mfma_supports(const AssignArgs& a, const DeviceInfo& dev);
 int launch_assign_mfma(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
-bool bf16_supports(const AssignArgs& a, const DeviceInfo& dev);
+bool bf16_supports(const AssignArgs& a, uint32_t lds_budget, const DeviceInfo& dev); /* (the budget decides for rows of more than 256 dimensions; the launchers of narrower ones say what they need) */
 int launch_assign_bf16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* rank16.hip: one half-precision product per dimension for all points, the serial result for what that leaves */
 bool rank16_supports(const AssignArgs& a, uint32_t lds_budget);
@@ -201,8 +201,8 @@ int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* w
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST would write a.rows_out */
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */
-bool wide_supports(const AssignArgs& a, const DeviceInfo& dev);
-bool wide16_supports(const AssignArgs& a, const DeviceInfo& dev); /* ... in half precision, nothing left to the caller */
+bool wide_supports(const AssignArgs& a, uint32_t lds_budget);
+bool wide16_supports(const AssignArgs& a, uint32_t lds_budget); /* ... in half precision, nothing left to the caller */
 int launch_assign_wide(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 bool lds_fma_supports(const AssignArgs& a, const DeviceInfo& dev);
 bool lds_fma_reads_through_scalar_cache(const AssignArgs& a); /* a handful of centroids: no LDS staging */

@@ -225,7 +225,7 @@ int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Wor
 		const bool split_wins = a.dim >= 16 || (a.dim >= 5 && a.k > 64);
 		const bool few = a.ranking_only ? a.k <= 32 : (a.k <= 16 && a.dim <= 16);
 		if (few && lds_fma_supports(a, dev) && lds_fma_reads_through_scalar_cache(a)) variant = KMX_ASSIGN_LDS_FMA;
-		else if (bf16_supports(a, dev) && (split_wins || packed_wins || takes_cells(a, lds_budget_of(exec, dev)))) variant = KMX_ASSIGN_MFMA_BF16X3;
+		else if (bf16_supports(a, lds_budget_of(exec, dev), dev) && (split_wins || packed_wins || takes_cells(a, lds_budget_of(exec, dev)))) variant = KMX_ASSIGN_MFMA_BF16X3;
 		else if (mfma_supports(a, dev)) variant = KMX_ASSIGN_MFMA;
 		else if (lds_fma_supports(a, dev)) variant = KMX_ASSIGN_LDS_FMA;
 		else variant = KMX_ASSIGN_BASE;
@@ -244,8 +244,8 @@ int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Wor
 			return fail(KMX_ERR_UNSUPPORTED, "kmx_assign_f32: shape dim=%u k=%u is not supported by the MFMA variant", a.dim, a.k);
 		return launch_assign_mfma(a, exec, ws, dev);
 	case KMX_ASSIGN_MFMA_BF16X3:
-		if (!bf16_supports(a, dev))
-			return fail(KMX_ERR_UNSUPPORTED, "kmx_assign_f32: shape dim=%u k=%u is not supported by the split-bf16 MFMA variant", a.dim, a.k);
+		if (!bf16_supports(a, lds_budget_of(exec, dev), dev))
+			return fail(KMX_ERR_UNSUPPORTED, "kmx_assign_f32: shape dim=%u k=%u is not supported by the split-bf16 MFMA variant (LDS budget %u bytes)", a.dim, a.k, lds_budget_of(exec, dev));
 		return launch_assign_bf16(a, exec, ws, dev);
 	default:
 		return fail(KMX_ERR_INVALID_ARGUMENT, "kmx_assign_f32: unknown variant %d", variant);

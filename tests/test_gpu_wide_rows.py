@@ -53,3 +53,31 @@ def test_wide_rows_match_the_oracle(km, orc, gpu, dim, k, n, kind):
             assert np.array_equal(got, want), "layouts %d/%d, mode %d: %d mismatches" % (layout, layout_means, mode, int((got != want).sum()))
         d.free(); m.free()
     a.free()
+
+
+@pytest.mark.parametrize("budget,variant,blocks", [
+    (0, "MFMA_BF16X3", 129),           # 129 units of 128 points
+    (54 * 1024, "MFMA_BF16X3", 256),   # too little for those: units of 32
+    (31 * 1024, "MFMA_BF16X3", 256),   # too little for the half-precision exact pass: three products
+    (16 * 1024, "BASE", None),         # no sweep fits
+])
+def test_wide_rows_keep_to_the_lds_budget(km, orc, gpu, budget, variant, blocks):
+    dim, k, n = 512, 40, 16400
+    rng = np.random.default_rng(budget)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    means = np.ascontiguousarray(rows[rng.choice(n, k, replace=False)])
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, 0))
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 0))
+    a = km.DeviceBuffer(4 * n); a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+    ex = km.ExecParams(shared_mem_bytes=budget)
+    km.assign(km.ASSIGN_BEST, d, 0, dim, m, 0, dim, a, dim, k, n, ex)
+    km.sync()
+    assert km.last_assign_variant() == getattr(km, "ASSIGN_" + variant)
+    assert blocks is None or ex.block_count == min(blocks, gpu.compute_units)
+    assert np.array_equal(a.read(np.uint32, n), want)
+    if variant == "BASE":
+        with pytest.raises(km.KmxError, match="LDS budget"):
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, 0, dim, m, 0, dim, a, dim, k, n, km.ExecParams(shared_mem_bytes=budget))
+    for b in (d, m, a):
+        b.free()
