@@ -431,15 +431,13 @@ constexpr uint32_t SMALL_FEW_CENTROIDS = 12; /* up to here a tile of one point t
  * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
  */
 constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
-#ifndef KMX_SMALL_EFFORT
-#define KMX_SMALL_EFFORT 450000000ull
-#endif
+constexpr uint64_t SMALL_EFFORT = 450000000;
 template <typename F>
 bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
 	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
 	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
-	const uint64_t limit = KMX_SMALL_EFFORT * (dim > 32 ? 3 : 2) / 2 * (sizeof(F) / 4);
+	const uint64_t limit = SMALL_EFFORT * (dim > 32 ? 3 : 2) / 2 * (sizeof(F) / 4);
 	return effort <= limit && assign_small_lds<F>(dim, k) + assign_small_static<F>() <= lds_budget;
 }
 
