@@ -17,7 +17,7 @@ constexpr uint32_t EXACT_HITS = 256;                       /* pairs per wavefron
 constexpr uint32_t EXACT_SQUARES_BYTES = EXACT_WAVES * WAVE * (KBLOCK + 4) * 4; /* (doubles: half as many pairs) */
 constexpr uint32_t exact_static_bytes(bool doubles)
 {
-	return (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + EXACT_WAVES) * 4 + 96 + (doubles ? EXACT_WAVES * EXACT_HITS * 8 + 2 * EXACT_ROWS * 4 : 0);
+	return (7 * EXACT_ROWS + EXACT_WAVES * EXACT_HITS + EXACT_WAVES) * 4 + 96 + (doubles ? EXACT_WAVES * EXACT_HITS * 8 + EXACT_ROWS * 4 : 0);
 }
 
 template <typename F>
@@ -61,6 +61,19 @@ __device__ __forceinline__ void exact_place(F __attribute__((ext_vector_type(4))
 	v.w = __builtin_bit_cast(F, t & m0);
 }
 
+/* the value of lane Q (0..3) of this lane's four */
+template <int Q> __device__ __forceinline__ float lane_of_four(float v)
+{
+	return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), Q * 0x55, 0xF, 0xF, true)); /* quad_perm [Q Q Q Q] */
+}
+template <int Q> __device__ __forceinline__ double lane_of_four(double v)
+{
+	const unsigned long long bits = __builtin_bit_cast(unsigned long long, v);
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)bits, Q * 0x55, 0xF, 0xF, true);
+	const uint32_t up = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(bits >> 32), Q * 0x55, 0xF, 0xF, true);
+	return __builtin_bit_cast(double, (unsigned long long)up << 32 | lo);
+}
+
 /* doubles: the bits of a serial distance as they are compared, like exact_key without the centroid */
 __device__ __forceinline__ unsigned long long exact_bits(double sum, uint32_t c)
 {
@@ -86,7 +99,8 @@ __device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
  *      touch 64 lines per load), the squares go through LDS to the pair's lane, which adds them in order. The results merge into
  *      the point's two smallest keys (distance bits << 32 | centroid, see evaluate_pair) in LDS.
  * F: the type of the serial arithmetic; doubles are ranked by float copies.
- * A wavefront whose list fills up (data that the thresholds tell nothing about) evaluates it on the spot, one lane per pair.
+ * A wavefront whose list fills up (ties, duplicated centroids, data that the thresholds tell nothing about) evaluates it on the spot, 16
+ * pairs at a time (N = 262144, d = 256, k = 1024, 32 copies each of 32 centroids: 1.15 ms a call, with a lane per pair 6.85).
  *
  * counters[0] receives the number of points whose two smallest serial distances are closer than the three-product certificate.
  */
@@ -104,7 +118,7 @@ listed_exact_kernel(const ExactArgs<F> w)
 	__shared__ uint32_t noted_by[EXACT_WAVES];
 	constexpr bool DOUBLES = sizeof(F) == 8; /* keys of 96 bits: the smallest distances first, then who has them */
 	__shared__ unsigned long long pair_bits[DOUBLES ? EXACT_WAVES * EXACT_HITS : 1];
-	__shared__ uint32_t winner[DOUBLES ? EXACT_ROWS : 1], redo[DOUBLES ? EXACT_ROWS : 1];
+	__shared__ uint32_t winner[DOUBLES ? EXACT_ROWS : 1];
 	constexpr uint32_t PASS = DOUBLES ? 32 : 64; /* pairs a wavefront evaluates at a time */
 	typedef F F4 __attribute__((ext_vector_type(4)));
 	constexpr uint32_t PAIR = KBLOCK + 16 / sizeof(F); /* a pair's squares of a block in LDS; the padding spreads 16 lanes' reads over all banks */
@@ -140,7 +154,7 @@ listed_exact_kernel(const ExactArgs<F> w)
 			point[tid] = w.list[2 * (size_t)e];
 			threshold[tid] = first + tid < count ? __uint_as_float(w.list[2 * (size_t)e + 1]) : -__builtin_inff(); /* rows beyond the list pass nothing */
 			best[tid] = ~0ull;
-			if constexpr (DOUBLES) { winner[tid] = ~0u; redo[tid] = 0u; }
+			if constexpr (DOUBLES) winner[tid] = ~0u;
 			second[tid] = ~0ull;
 		}
 		__syncthreads();
@@ -184,52 +198,140 @@ listed_exact_kernel(const ExactArgs<F> w)
 		}
 		__syncthreads();
 
-		/* the serial sum of a point and a centroid, by one lane */
-		auto serial_sum = [&](uint32_t row, uint32_t c) -> F {
+		/*
+		 * The serial sum of a point and a centroid, by four lanes (the same pair in all of them; all lanes of the wavefront call): each
+		 * fetches and squares four of a block's 16 differences, then the running sum goes round the four, which add their squares in order.
+		 */
+		auto serial_sum = [&](uint32_t row, uint32_t c, uint32_t lane) -> F {
 #pragma clang fp contract(off)
 			const F* src = serial_source(row);
-			const F* mean = w.means + (size_t)c * DP;
+			const F* mean = w.means + (size_t)c * DP + lane % 4 * 4;
+			constexpr uint32_t AT_ONCE = KB == 0 ? 2 : 1; /* blocks requested together (wide rows come from the L2 and are whole chunks of four blocks) */
 			F sum = (F)0;
 #pragma unroll 1
-			for (uint32_t d = 0; d < w.dim; ++d) {
-				const F diff = src[points_strided ? (size_t)d * w.points_step : (size_t)d] - mean[d];
-				const F sq = diff * diff;
-				sum = sum + sq;
+			for (uint32_t kb = 0; kb < blocks; kb += AT_ONCE) {
+				F4 x[AT_ONCE], m[AT_ONCE];
+#pragma unroll
+				for (uint32_t u = 0; u < AT_ONCE; ++u) {
+					exact_request<F>(x[u], src, (kb + u) * KBLOCK + lane % 4 * 4, w.dim, w.points_dim, w.points_step, points_strided);
+					m[u] = *(const F4*)(mean + (kb + u) * KBLOCK);
+				}
+#pragma unroll
+				for (uint32_t u = 0; u < AT_ONCE; ++u) {
+					if (points_ragged && (kb + u + 1) * KBLOCK > w.points_dim) exact_place<F>(x[u], (kb + u) * KBLOCK + lane % 4 * 4, w.points_dim);
+					F4 sq;
+#pragma unroll
+					for (int e = 0; e < 4; ++e) {
+						const F diff = x[u][e] - m[u][e];
+						sq[e] = diff * diff;
+					}
+					auto add = [&]() { return (((sum + sq[0]) + sq[1]) + sq[2]) + sq[3]; };
+					sum = lane_of_four<0>(add()); /* (zeros behind the row change nothing) */
+					sum = lane_of_four<1>(add());
+					sum = lane_of_four<2>(add());
+					sum = lane_of_four<3>(add());
+				}
 			}
 			return sum;
 		};
-		/* doubles: who has the smallest distance is settled when it is known (in_list), or by another look at all centroids (redo) */
-		auto merge = [&](uint32_t row, uint32_t c, F sum, uint32_t in_list) {
+		/* doubles: who has the smallest distance is settled when it is known; `at`: where the pair's distance waits for that */
+		auto merge = [&](uint32_t row, uint32_t c, F sum, uint32_t at) {
 			if constexpr (DOUBLES) {
-				const unsigned long long bits = exact_bits(sum, c);
-				atomicMin(&best[row], bits);
-				if (in_list == ~0u) redo[row] = 1u;
-				else pair_bits[in_list] = bits;
+				pair_bits[at] = exact_bits(sum, c);
+				atomicMin(&best[row], pair_bits[at]);
 			}
 			else {
 				const unsigned long long key = exact_key(sum, c), before = atomicMin(&best[row], key);
 				atomicMin(&second[row], before < key ? key : before);
 			}
 		};
-		uint32_t noted = 0; /* wave-uniform */
-		auto evaluate_alone = [&]() {
+		uint32_t noted = 0;                      /* wave-uniform */
+		[[maybe_unused]] uint32_t kept = 0;      /* doubles: of those, evaluated before and kept */
+		/* a list that is full: 16 pairs at a time (their rows and the tile's centroids are in the caches), or, rows of up to four floats, one per lane */
+		auto evaluate_here = [&]() {
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 			__builtin_amdgcn_wave_barrier();
-			for (uint32_t i = lane; i < noted; i += WAVE) {
-				const uint32_t hit = hits[wave][i], row = hit >> 25, c = hit & CENTROID;
-				merge(row, c, serial_sum(row, c), ~0u);
+			[[maybe_unused]] const uint32_t full = noted;
+			if (KB == 1 && w.dim <= 4) {
+#pragma clang fp contract(off)
+				for (uint32_t i = kept + lane; i < noted; i += WAVE) {
+					const uint32_t hit = hits[wave][i], row = hit >> 25, c = hit & CENTROID;
+					F4 x;
+					exact_request<F>(x, serial_source(row), 0, w.dim, w.points_dim, w.points_step, points_strided);
+					const F4 m = *(const F4*)(w.means + (size_t)c * DP);
+					F sum = (F)0;
+#pragma unroll
+					for (int e = 0; e < 4; ++e) {
+						const F diff = x[e] - m[e];
+						const F sq = diff * diff;
+						sum = sum + sq;
+					}
+					merge(row, c, sum, wave * EXACT_HITS + i);
+				}
 			}
-			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-			__builtin_amdgcn_wave_barrier();
+			else
+			{
+				uint32_t me = lane;
+				asm volatile("" : "+v"(me)); /* (rare: nothing of this is worth keeping in registers meanwhile) */
+#pragma unroll 1
+				for (uint32_t i = kept; i < noted; i += WAVE / 4) {
+					const uint32_t hit = hits[wave][min(i + me / 4, noted - 1)], row = hit >> 25, c = hit & CENTROID;
+					const F sum = serial_sum(row, c, me);
+					if (i + me / 4 < noted && me % 4 == 0) merge(row, c, sum, wave * EXACT_HITS + i + me / 4);
+				}
+			}
+			auto in_order = [&]() {
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+				__builtin_amdgcn_wave_barrier();
+			};
+			in_order();
 			noted = 0;
+			if constexpr (DOUBLES) {
+				/* what stays in the list is, per row, the first centroid of those at the row's smallest distance so far: at most one per row */
+				constexpr uint32_t EACH = EXACT_HITS / WAVE;
+				uint32_t hit[EACH];
+				unsigned long long bits[EACH];
+#pragma unroll
+				for (uint32_t q = 0; q < EACH; ++q) {
+					hit[q] = hits[wave][lane + q * WAVE];
+					bits[q] = pair_bits[wave * EXACT_HITS + lane + q * WAVE];
+				}
+				in_order();
+				uint32_t* lowest = (uint32_t*)&pair_bits[wave * EXACT_HITS]; /* per row; the distances are in registers */
+				for (uint32_t row = lane; row < EXACT_ROWS; row += WAVE) lowest[row] = ~0u;
+				in_order();
+				bool keep[EACH];
+#pragma unroll
+				for (uint32_t q = 0; q < EACH; ++q) {
+					keep[q] = lane + q * WAVE < full && bits[q] == best[hit[q] >> 25];
+					if (keep[q]) atomicMin(&lowest[hit[q] >> 25], hit[q] & CENTROID);
+				}
+				in_order();
+#pragma unroll
+				for (uint32_t q = 0; q < EACH; ++q) {
+					keep[q] = keep[q] && lowest[hit[q] >> 25] == (hit[q] & CENTROID);
+					if (lane + q * WAVE < full && !keep[q]) atomicMin(&second[hit[q] >> 25], bits[q]);
+				}
+				in_order();
+#pragma unroll
+				for (uint32_t q = 0; q < EACH; ++q) {
+					const unsigned long long mask = __builtin_amdgcn_ballot_w64(keep[q]);
+					const uint32_t to = noted + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+					if (keep[q]) { hits[wave][to] = hit[q]; pair_bits[wave * EXACT_HITS + to] = bits[q]; }
+					noted += (uint32_t)__popcll(mask);
+				}
+				kept = noted;
+				in_order();
+			}
 		};
-		auto screen = [&](const f32x16& a, uint32_t t, uint32_t g) {
+		uint32_t rounds = 0; /* of the tile and group at hand, noted before the list was full */
+		auto screen = [&](const f32x16& a, uint32_t t, uint32_t g) -> bool { /* false: the list is full */
 			const float limit = threshold[g * TILE + col];
 			float low = a[0]; /* NaN-propagating minimum */
 #pragma unroll
 			for (int r = 1; r < 16; ++r) low = __builtin_elementwise_minimum(low, a[r]);
 			const bool near = !(low > limit);
-			if (__builtin_amdgcn_ballot_w64(near) == 0) return;
+			if (__builtin_amdgcn_ballot_w64(near) == 0) return true;
 			uint32_t passed = 0; /* bit r: result r */
 #pragma unroll
 			for (int r = 0; r < 16; ++r) passed |= !(a[r] > limit) ? 1u << r : 0u;
@@ -238,18 +340,22 @@ listed_exact_kernel(const ExactArgs<F> w)
 				for (int r = 0; r < 16; ++r)
 					if (t * TILE + 8 * (r / 4) + 4 * h + (r % 4) >= w.k) passed &= ~(1u << r);
 			}
+			for (uint32_t r = 0; r < rounds; ++r) passed &= passed - 1;
 			for (;;) { /* the lanes' next results */
 				const unsigned long long mask = __builtin_amdgcn_ballot_w64(passed != 0);
 				if (mask == 0) break;
 				const uint32_t more = (uint32_t)__popcll(mask);
-				if (noted + more > EXACT_HITS) evaluate_alone();
+				if (noted + more > EXACT_HITS) return false;
 				if (passed) {
 					const uint32_t r = (uint32_t)__builtin_ctz(passed);
 					hits[wave][noted + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (g * TILE + col) << 25 | (t * TILE + 8 * (r / 4) + 4 * h + r % 4);
 					passed &= passed - 1;
 				}
 				noted += more;
+				++rounds;
 			}
+			rounds = 0;
+			return true;
 		};
 		auto start_of = [&](uint32_t t) {
 			f32x16 start;
@@ -262,45 +368,58 @@ listed_exact_kernel(const ExactArgs<F> w)
 		};
 		/* few tiles: the wavefronts share out the groups of points as well */
 		const uint32_t parts = tiles < EXACT_WAVES ? groups : 1;
+		uint32_t t = wave / parts, g = wave % parts;
+		for (;;) {
+			bool room = true;
 #pragma unroll 1
-		for (uint32_t t = wave / parts; t < tiles; t += EXACT_WAVES / parts) {
-			const f16x8* operand = w.packed + (size_t)t * (blocks * WAVE) + lane;
-			if constexpr (KB > 0) {
-				const f32x16 start = start_of(t);
-				f16x8 c[KB];
+			while (t < tiles) {
+				const f16x8* operand = w.packed + (size_t)t * (blocks * WAVE) + lane;
+				if constexpr (KB > 0) {
+					const f32x16 start = start_of(t);
+					f16x8 c[KB];
 #pragma unroll
-				for (int kb = 0; kb < KB; ++kb) c[kb] = operand[kb * WAVE];
+					for (int kb = 0; kb < KB; ++kb) c[kb] = operand[kb * WAVE];
 #pragma unroll 1
-				for (uint32_t g = wave % parts; g < groups; g += parts) {
-					f32x16 a = start;
-					const f16x8* x = ops + g * (KB * WAVE) + lane;
+					for (; g < groups; g += parts) {
+						f32x16 a = start;
+						const f16x8* x = ops + g * (KB * WAVE) + lane;
 #pragma unroll
-					for (int kb = 0; kb < KB; ++kb) a = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], x[kb * WAVE], a, 0, 0, 0);
-					screen(a, t, g);
+						for (int kb = 0; kb < KB; ++kb) a = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], x[kb * WAVE], a, 0, 0, 0);
+						room = screen(a, t, g);
+						if (!room) break;
+					}
 				}
-			}
-			else {
-				const uint32_t g0 = wave % parts;
-				f32x16 a[EXACT_GROUPS];
-				a[0] = start_of(t);
+				else {
+					const uint32_t g0 = wave % parts;
+					f32x16 a[EXACT_GROUPS];
+					a[0] = start_of(t);
 #pragma unroll
-				for (uint32_t q = 1; q < EXACT_GROUPS; ++q) a[q] = a[0];
-				for (uint32_t kb = 0; kb < blocks; kb += 4) { /* (rows are padded to whole chunks of four blocks) */
-					f16x8 four[4];
+					for (uint32_t q = 1; q < EXACT_GROUPS; ++q) a[q] = a[0];
+					for (uint32_t kb = 0; kb < blocks; kb += 4) { /* (rows are padded to whole chunks of four blocks) */
+						f16x8 four[4];
 #pragma unroll
-					for (uint32_t i = 0; i < 4; ++i) four[i] = operand[(kb + i) * WAVE];
+						for (uint32_t i = 0; i < 4; ++i) four[i] = operand[(kb + i) * WAVE];
+#pragma unroll
+						for (uint32_t q = 0; q < EXACT_GROUPS; ++q)
+							if (g0 + q * parts < groups) {
+								const f16x8* x = ops + ((g0 + q * parts) * blocks + kb) * WAVE + lane;
+#pragma unroll
+								for (uint32_t i = 0; i < 4; ++i) a[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(four[i], x[i * WAVE], a[q], 0, 0, 0);
+							}
+					}
 #pragma unroll
 					for (uint32_t q = 0; q < EXACT_GROUPS; ++q)
-						if (g0 + q * parts < groups) {
-							const f16x8* x = ops + ((g0 + q * parts) * blocks + kb) * WAVE + lane;
-#pragma unroll
-							for (uint32_t i = 0; i < 4; ++i) a[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(four[i], x[i * WAVE], a[q], 0, 0, 0);
+						if (room && g0 + q * parts == g && g < groups) {
+							room = screen(a[q], t, g);
+							if (room) g += parts;
 						}
 				}
-#pragma unroll
-				for (uint32_t q = 0; q < EXACT_GROUPS; ++q)
-					if (g0 + q * parts < groups) screen(a[q], t, g0 + q * parts);
+				if (!room) break;
+				t += EXACT_WAVES / parts;
+				g = wave % parts;
 			}
+			if (room) break;
+			evaluate_here(); /* then this tile and group again, from where the list was full */
 		}
 		if (lane == 0) noted_by[wave] = noted;
 		__syncthreads(); /* all pairs are listed, the operands are no longer needed */
@@ -393,11 +512,8 @@ listed_exact_kernel(const ExactArgs<F> w)
 				};
 				for (uint32_t i = tid; i < total; i += EXACT_THREADS) {
 					const uint32_t hit = pair_of(i), row = hit >> 25;
-					if (!redo[row]) settle(row, hit & CENTROID, pair_bits[i]);
+					settle(row, hit & CENTROID, pair_bits[i]);
 				}
-				for (uint32_t row = wave; row < unit_rows; row += EXACT_WAVES)
-					if (redo[row])
-						for (uint32_t c = lane; c < w.k; c += WAVE) settle(row, c, exact_bits(serial_sum(row, c), c));
 			}
 		}
 		__syncthreads();

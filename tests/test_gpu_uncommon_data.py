@@ -1,0 +1,64 @@
+"""Inputs whose distribution is unlike the usual mixture: the default assignment must not collapse on them. Each is timed beside
+kmx_set_two_level_sweep(0), the sweeps that make no assumption about the data beyond their own; same results, and no slower than 1.3
+times that (the margin is what runs and boxes differ by; what these tests are for was 2 to 90 times) (-m gpu)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+MARGIN = 1.3
+
+
+def assign_timed(km, rows, means):
+    """(median time of a call in ms, assignment) per mode of kmx_set_two_level_sweep"""
+    (n, dim), k = rows.shape, len(means)
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    m = km.DeviceBuffer(means.nbytes); m.write(means.ravel())
+    a = km.DeviceBuffer(4 * n)
+    start, stop = km.Event(), km.Event()
+    out = {}
+    try:
+        for mode in (0, 1):
+            km.set_two_level_sweep(mode)
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            times = []
+            for call in range(9):
+                start.record()
+                km.assign(km.ASSIGN_BEST, d, 0, dim, m, 0, dim, a, dim, k, n, None, rows.dtype)
+                stop.record()
+                km.sync()
+                if call > 1:
+                    times.append(start.elapsed_ms(stop))
+            out[mode] = float(np.median(times)), a.read(np.uint32, n)
+    finally:
+        km.set_two_level_sweep(1)
+        for b in (d, m, a):
+            b.free()
+    return out
+
+
+def check(km, orc, rows, means):
+    out = assign_timed(km, rows, means)
+    (off, want), (default, got) = out[0], out[1]
+    assert np.array_equal(got, want)
+    sample = np.random.default_rng(1).choice(len(rows), 500, replace=False)
+    fn = orc.assign if rows.dtype == np.float32 else orc.assign_f64
+    some = np.ascontiguousarray(rows[sample])
+    assert np.array_equal(got[sample], fn(some.ravel(), means.ravel(), rows.shape[1], len(means), 500, threads=0))
+    print("off %.3f ms, default %.3f ms" % (off, default))
+    assert default <= MARGIN * off, "default %.3f ms, switched off %.3f ms" % (default, off)
+
+
+def mixture(rng, n, dim, k, spread, noise=1.0):
+    centres = rng.uniform(-spread, spread, size=(k, dim)).astype(np.float32)
+    return (centres[rng.integers(0, k, n)] + rng.normal(size=(n, dim)).astype(np.float32) * np.float32(noise)).astype(np.float32)
+
+
+@pytest.mark.parametrize("dtype,dim,k,n,distinct", [(np.float32, 32, 1024, 1 << 18, 32), (np.float32, 32, 1024, 1 << 17, 1), (np.float32, 256, 1024, 1 << 16, 32),
+                                                    (np.float64, 32, 1024, 1 << 17, 32)])
+def test_duplicated_centroids(km, orc, gpu, dtype, dim, k, n, distinct):
+    """Every point ties between k / distinct centroids: the lists of candidates overflow."""
+    rng = np.random.default_rng(dim + distinct)
+    rows = mixture(rng, n, dim, k, 10).astype(dtype)
+    means = np.tile(rows[:distinct], (k // distinct, 1))
+    check(km, orc, rows, means)
