@@ -142,18 +142,18 @@ pack_means16_wide_kernel(const float* __restrict__ means, const double* __restri
                          uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters)
 {
 	extern __shared__ float m[]; /* dp floats */
-	__shared__ float wave_far[4];
+	__shared__ float wave_far[2][4];
 	constexpr uint32_t SAMPLE = 16;
 	const uint32_t lane = threadIdx.x & (WAVE - 1);
 	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; }
 	const uint32_t sample = min(k, SAMPLE);
-	float far = 0.0f;
+	float far = 0.0f, size = 0.0f;
 	for (uint32_t q = threadIdx.x; q < dp; q += 256) {
 		float sum = 0.0f;
 		if (q < dim) {
 			float v[SAMPLE];
 #pragma unroll
-			for (uint32_t r = 0; r < SAMPLE; ++r) v[r] = r < sample ? means[elem<LM>(stride_means, r, q)] : 0.0f;
+			for (uint32_t r = 0; r < SAMPLE; ++r) v[r] = r < sample ? means[elem<LM>(stride_means, even_row(r, 4, k), q)] : 0.0f;
 #pragma unroll
 			for (uint32_t r = 0; r < SAMPLE; ++r) sum += __builtin_fabsf(v[r]) < __builtin_inff() ? v[r] : 0.0f;
 			sum = sum / (float)sample;
@@ -161,15 +161,16 @@ pack_means16_wide_kernel(const float* __restrict__ means, const double* __restri
 #pragma unroll
 			for (uint32_t r = 0; r < SAMPLE; ++r) {
 				const float d = __builtin_fabsf(v[r] - sum);
-				if (r < sample && d < __builtin_inff()) far = fmaxf(far, d);
+				if (r < sample && d < __builtin_inff()) { far = fmaxf(far, d); size = fmaxf(size, __builtin_fabsf(v[r])); }
 			}
 		}
 		m[q] = sum;
 	}
-	for (int off = WAVE / 2; off > 0; off >>= 1) far = fmaxf(far, __shfl_xor(far, off));
-	if (lane == 0) wave_far[threadIdx.x / WAVE] = far;
+	for (int off = WAVE / 2; off > 0; off >>= 1) { far = fmaxf(far, __shfl_xor(far, off)); size = fmaxf(size, __shfl_xor(size, off)); }
+	if (lane == 0) { wave_far[0][threadIdx.x / WAVE] = far; wave_far[1][threadIdx.x / WAVE] = size; }
 	__syncthreads();
-	const float scale = rank16_scale(fmaxf(fmaxf(wave_far[0], wave_far[1]), fmaxf(wave_far[2], wave_far[3])));
+	const float scale = rank16_scale(fmaxf(fmaxf(wave_far[0][0], wave_far[0][1]), fmaxf(wave_far[0][2], wave_far[0][3])),
+	                                 fmaxf(fmaxf(wave_far[1][0], wave_far[1][1]), fmaxf(wave_far[1][2], wave_far[1][3])));
 	if (blockIdx.x == 0) {
 		for (uint32_t q = threadIdx.x; q < dp; q += 256) norms[wide16_frame_offset(kp) + q] = m[q];
 		if (threadIdx.x == 0) {

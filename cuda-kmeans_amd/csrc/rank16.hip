@@ -2,7 +2,7 @@
  * Assignment of rows of 5 to 256 dimensions by one half-precision product per dimension, and the exact pass behind it.
  *
  * Ranking. Points and centroids are moved to the middle of the centroids and scaled by a power of two S that brings the centroids'
- * coordinates to about 16..32, then rounded to half precision (11 significant bits): a[j] = S^2 (|c_j|^2 - 2 c_j . x) is one
+ * coordinates to about 2^-5 (rank16_scale), then rounded to half precision (11 significant bits): a[j] = S^2 (|c_j|^2 - 2 c_j . x) is one
  * v_mfma_f32_32x32x16_f16 per 16 dimensions, a third of what three bf16 products cost. The certificate is the one-product form of
  * certificate.h with the norms of what the roundings actually dropped, |x - x_half| of the point and max_j |c'_j - c'_half| of the
  * centroids; overflow to infinity and values lost below the smallest half-precision number are covered by the same norms (an
@@ -45,9 +45,10 @@ KMX_DECLARE_EXACT16(6) KMX_DECLARE_EXACT16(8) KMX_DECLARE_EXACT16(12) KMX_DECLAR
 
 /*
  * One wavefront per (padded) centroid row: its half-precision operands, S^2 |c|^2, the squared norms of what half precision and the
- * bf16 parts leave out. Every work-group computes the frame m (sweep_frame) and S from the first 16 centroids: S max |c - m| over them
- * is in [16, 32), so that a coordinate may be 2000 times larger before it overflows.
- * norms: tiles of S^2 |c - m|^2, then per row low2, mid2, rest2, then the frame (sweep_frame), S, 1 / S^2 and (rank16_leave_bounds) three maxima.
+ * bf16 parts leave out. Every work-group computes the frame m and S (rank16_scale) from centroids spread evenly over
+ * all of them: the first ones are often the first points, and those may be unlike the rest (blank rows ahead of an image, the quiet start
+ * of a recording).
+ * norms: tiles of S^2 |c - m|^2, then per row low2, mid2, rest2, then the frame, S, 1 / S^2 and (rank16_leave_bounds) three maxima.
  */
 __host__ __device__ __forceinline__ size_t rank16_low_offset(uint32_t kp) { return (size_t)(kp / TILE) * NORM_TILE; }
 __host__ __device__ __forceinline__ size_t rank16_frame_offset(uint32_t kp) { return rank16_low_offset(kp) + 3 * (size_t)kp; }
@@ -60,7 +61,7 @@ pack_means16_kernel(const float* __restrict__ means, const double* __restrict__ 
                     uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters)
 {
 	__shared__ float frame[FRAME_DIMS];
-	__shared__ float wave_far[4];
+	__shared__ float wave_far[2][4];
 	const uint32_t lane = threadIdx.x & (WAVE - 1);
 	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; counters[CELLS_COUNTER] = 0u; }
 	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
@@ -71,23 +72,34 @@ pack_means16_kernel(const float* __restrict__ means, const double* __restrict__ 
 		const uint32_t q = lane + i * WAVE;
 		exact[i] = (j < k && q < dim) ? means[elem<LM>(stride_means, j, q)] : 0.0f;
 	}
-	sweep_frame<LM>(means, stride_means, dim, k, dp, FRAME_MOVED, frame, norms + rank16_frame_offset(kp));
-	float far = 0.0f;
-	for (uint32_t q = threadIdx.x; q < dim; q += 256) {
-		float v[16];
+	/* 16 coordinates per lane, of as many rows spread evenly over the centroids: 16 rows of 129 to 256 dimensions, 128 of 17 to 32 */
+	const uint32_t log_columns = 32 - __builtin_clz(max(dim, 2u) - 1), log_groups = 8 - log_columns; /* (dim <= 256) */
+	const uint32_t column = min(threadIdx.x & ((1u << log_columns) - 1u), dim - 1), group = threadIdx.x >> log_columns;
+	float sample[16];
 #pragma unroll
-		for (uint32_t r = 0; r < 16; ++r) v[r] = means[elem<LM>(stride_means, min(r, k - 1), q)];
+	for (uint32_t i = 0; i < 16; ++i) sample[i] = means[elem<LM>(stride_means, even_row(group * 16 + i, 4 + log_groups, k), column)];
+	/* the frame m: the mean of the first lanes' 16 rows, finite coordinates only (any vector would do; this one lies inside the data) */
+	if (group == 0 && threadIdx.x < dim) {
+		float sum = 0.0f;
 #pragma unroll
-		for (uint32_t r = 0; r < 16; ++r) {
-			const float d = __builtin_fabsf(v[r] - frame[q]);
-			if (d < __builtin_inff()) far = fmaxf(far, d);
-		}
+		for (uint32_t i = 0; i < 16; ++i) sum += __builtin_fabsf(sample[i]) < __builtin_inff() ? sample[i] : 0.0f;
+		sum = sum / 16.0f;
+		frame[column] = __builtin_fabsf(sum) < __builtin_inff() ? sum : 0.0f; /* (the sum of finite values may overflow) */
 	}
-	for (int off = WAVE / 2; off > 0; off >>= 1) far = fmaxf(far, __shfl_xor(far, off));
-	if (lane == 0) wave_far[threadIdx.x / WAVE] = far;
+	if (threadIdx.x >= dim && threadIdx.x < dp) frame[threadIdx.x] = 0.0f;
 	__syncthreads();
-	far = fmaxf(fmaxf(wave_far[0], wave_far[1]), fmaxf(wave_far[2], wave_far[3]));
-	const float scale = rank16_scale(far);
+	if (blockIdx.x == 0 && threadIdx.x < dp) norms[rank16_frame_offset(kp) + threadIdx.x] = frame[threadIdx.x];
+	float far = 0.0f, size = 0.0f; /* (infinities and NaN drop out) */
+#pragma unroll
+	for (uint32_t i = 0; i < 16; ++i) {
+		const float d = __builtin_fabsf(sample[i] - frame[column]);
+		if (d < __builtin_inff()) { far = fmaxf(far, d); size = fmaxf(size, __builtin_fabsf(sample[i])); }
+	}
+	for (int off = WAVE / 2; off > 0; off >>= 1) { far = fmaxf(far, __shfl_xor(far, off)); size = fmaxf(size, __shfl_xor(size, off)); }
+	if (lane == 0) { wave_far[0][threadIdx.x / WAVE] = far; wave_far[1][threadIdx.x / WAVE] = size; }
+	__syncthreads();
+	const float scale = rank16_scale(fmaxf(fmaxf(wave_far[0][0], wave_far[0][1]), fmaxf(wave_far[0][2], wave_far[0][3])),
+	                                 fmaxf(fmaxf(wave_far[1][0], wave_far[1][1]), fmaxf(wave_far[1][2], wave_far[1][3])));
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		norms[rank16_scale_offset(kp)] = scale;
 		norms[rank16_scale_offset(kp) + 1] = 1.0f / (scale * scale);

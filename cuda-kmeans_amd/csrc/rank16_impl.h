@@ -35,12 +35,26 @@ struct Rank16Args {
 template <int KB> constexpr uint32_t rank16_tile_floats() { return KB * WAVE * 4; }
 template <int KB> constexpr uint32_t rank16_static_bytes() { return (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + KB * KBLOCK) * 4 + 64; }
 
-/* S for centroids whose coordinates are up to `far` from the frame: the power of two that puts far into [16, 32), kept inside what S and
- * 1 / S^2 can be as normal numbers */
-__device__ __forceinline__ float rank16_scale(float far)
+/*
+ * S for centroids whose coordinates are up to `far` from the frame and up to `size` from the origin, both of a sample: the power of two
+ * that puts far into [2^-5, 2^-4), kept inside what S and 1 / S^2 can be as normal numbers. A coordinate may then be half a million
+ * times larger before it overflows (which would certify nothing any more), and what half precision loses below its smallest normal
+ * number, 2^-25 at most, is a 256th of the rounding of a coordinate as large as far. Less than 2^-12 of `size` is taken for that: a
+ * sample of equal rows differs from their mean by its roundings only. (With far in [16, 32) from the first 16 centroids a quiet start of
+ * 5e-3 before centroids of 20 overflowed: N = 1M, d = 32, k = 512 in 29 ms; now 0.36.)
+ */
+__device__ __forceinline__ float rank16_scale(float far, float size)
 {
-	const int shift = far > 0.0f ? min(max(131 - (int)(__float_as_uint(far) >> 23), -60), 60) : 0;
+	far = fmaxf(far, size * 0x1p-12f);
+	const int shift = far > 0.0f ? min(max(122 - (int)(__float_as_uint(far) >> 23), -60), 60) : 0;
 	return __uint_as_float((uint32_t)(127 + shift) << 23);
+}
+
+/* row r of 2^log >= 4 rows spread evenly over k: four neighbours (of SoA centroids, in one line) at each place, the places multiples of the
+ * golden ratio (equal steps would meet the same row again and again where rows repeat) */
+__device__ __forceinline__ uint32_t even_row(uint32_t r, uint32_t log, uint32_t k)
+{
+	return min(k <= (1u << log) ? r : __umulhi(r / 4 * 0x9E3779B9u, k) + r % 4, k - 1);
 }
 
 /* the exact pass's certificate, by one work-group (first wavefront): max |c|^2, max |mid|^2, max |rest|^2 to scale[2 .. 4] */
