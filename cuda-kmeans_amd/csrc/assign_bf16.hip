@@ -134,23 +134,13 @@ pack_means_bf16_kernel(const float* __restrict__ means, size_t stride_means, flo
 	float c2 = 0.0f, mid2 = 0.0f, rest2 = 0.0f; /* |c|^2 (of the moved centroid) and, for the certificate, sum_i c'mid_i^2, sum_i c'rest_i^2 */
 	float exact2 = 0.0f; /* unpacked rows: |c|^2 of the centroid as given */
 	if (packed_form) {
-		/* rows of at most 4 dimensions: slots 0..3 = hi, 4..7 = mid, 8..11 = hi, 12..15 = mid of -2c; inside the tile
-		 * the first halves of all rows, then the second halves (packed_half; load_packed_points has the matching order
-		 * of the point's parts) */
 		if (lane < KBLOCK) {
 			const uint32_t q = lane % 4;
 			const float exact = (j < k && q < dim) ? means[elem<LM>(stride_means, j, q)] : 0.0f;
 			const float v = (j < k && q < dim) ? exact - (q == 0 ? frame[0] : q == 1 ? frame[1] : q == 2 ? frame[2] : frame[3]) : 0.0f;
-			__bf16 hi, mid;
-			const float rest = split_bf16(-2.0f * v, hi, mid);
-			float* tile = packed + (size_t)(j / TILE) * tile_floats(rs);
-			((__bf16*)(tile + packed_half(j % TILE, lane / 8)))[lane % 8] = (lane / 4) % 2 == 1 ? mid : hi;
-			if (j % TILE == TILE - 1 && lane < TILE_PAD) tile[TILE * rs + lane] = 0.0f;
+			pack_packed_row(packed, j, lane, v, c2, mid2, rest2);
 			if (lane < 4) {
-				c2 = v * v;
 				exact2 = exact * exact;
-				mid2 = (float)mid * (float)mid;
-				rest2 = rest * rest;
 				if (q < dim) means_t[(size_t)q * kp + j] = exact; /* exact copy for the recheck pass */
 			}
 		}

@@ -56,6 +56,37 @@ __host__ __device__ __forceinline__ size_t exact_norms_offset(uint32_t kp) { ret
 __host__ __device__ __forceinline__ size_t split_norms_floats(uint32_t kp) { return exact_norms_offset(kp) + split_norms_offset(kp); }
 struct Frame { float m[4]; };
 
+/* The packed form of centroid row j, by lanes 0 to 15 of a wavefront; v: this lane's coordinate lane % 4 in the frame of the sweep. Slots
+ * 0..3 = hi, 4..7 = mid, 8..11 = hi, 12..15 = mid of -2c; inside the tile the first halves of all rows, then the second halves (packed_half;
+ * load_packed_points has the matching order of the point's parts). Lanes 0 to 3 get their shares of the norms. */
+__device__ __forceinline__ void pack_packed_row(float* packed, uint32_t j, uint32_t lane, float v, float& c2, float& mid2, float& rest2)
+{
+	constexpr uint32_t RS = row_floats<1, true>();
+	__bf16 hi, mid;
+	const float rest = split_bf16(-2.0f * v, hi, mid);
+	float* tile = packed + (size_t)(j / TILE) * tile_floats(RS);
+	((__bf16*)(tile + packed_half(j % TILE, lane / 8)))[lane % 8] = (lane / 4) % 2 == 1 ? mid : hi;
+	if (j % TILE == TILE - 1 && lane < TILE_PAD) tile[TILE * RS + lane] = 0.0f;
+	if (lane < 4) {
+		c2 = v * v;
+		mid2 = (float)mid * (float)mid;
+		rest2 = rest * rest;
+	}
+}
+
+/*
+ * The packed sweep behind the grid of cells (assign_cells.hip): it runs if the search left a word for it, and hands what it cannot certify
+ * to the exact pass of rank16_exact_impl.h, with thresholds for that pass's ranking (the same frame, scaled by S, one half-precision
+ * product per dimension).
+ */
+struct WayBack {
+	const uint32_t* wanted;
+	const float* scale; /* S, 1 / S^2, then (rank16_leave_bounds) the maxima of |c|^2, of the squared bf16 mid and rest parts, of what half precision leaves out */
+	float kd16;
+};
+__device__ __forceinline__ WayBack way_back_of() { return WayBack{ nullptr, nullptr, 0.0f }; }
+__device__ __forceinline__ WayBack way_back_of(const WayBack& w) { return w; }
+
 /* One tile of 32 points as B operands: per block of 16 dimensions the lane holds the 8 dimensions of its
  * half-wave (lanes 0-31: the first 8, lanes 32-63: the second 8) of ONE point, as hi and mid parts. */
 template <int KB> struct SplitPoints {
@@ -602,8 +633,10 @@ constexpr uint32_t CARRY_IN = 1u, CARRY_OUT = 2u;
 template <class T, class... Extra> constexpr bool extra_is() { return sizeof...(Extra) == 1 && (std::is_same<T, Extra>::value || ...); }
 __device__ __forceinline__ CentroidSlice slice_of() { return CentroidSlice{ nullptr, nullptr, 0u, 0u, 0u, 0u }; }
 __device__ __forceinline__ CentroidSlice slice_of(const CentroidSlice& s) { return s; }
+__device__ __forceinline__ CentroidSlice slice_of(const WayBack&) { return slice_of(); }
+__device__ __forceinline__ WayBack way_back_of(const CentroidSlice&) { return way_back_of(); }
 
-/* (Slice: nothing; CentroidSlice for the instances that sweep slices) */
+/* (Slice: nothing; CentroidSlice for the instances that sweep slices, WayBack for those behind the cells) */
 template <int KB, int P, int LD, bool VEC, bool STREAM, bool COARSE, bool PREFETCH, bool PACKED = false, class... Slice>
 __global__ void __launch_bounds__(MFMA_WAVES * WAVE)
 assign_bf16_kernel(const float* __restrict__ data, size_t stride, const float* __restrict__ packed, const float* __restrict__ norms,
@@ -613,7 +646,12 @@ assign_bf16_kernel(const float* __restrict__ data, size_t stride, const float* _
 {
 	static_assert(sizeof...(Slice) <= 1, "at most one slice");
 	constexpr bool SLICED = extra_is<CentroidSlice, Slice...>();
+	constexpr bool BEHIND_CELLS = extra_is<WayBack, Slice...>();
 	[[maybe_unused]] const CentroidSlice slice = slice_of(slice_argument...);
+	[[maybe_unused]] const WayBack way = way_back_of(slice_argument...);
+	if constexpr (BEHIND_CELLS) {
+		if (way.wanted[0] == 0u) return;
+	}
 	const float* __restrict__ all_norms = SLICED ? slice.all_norms : norms;
 	const uint32_t all_k = SLICED ? slice.all_k : k, all_kp = SLICED ? slice.all_kp : kp;
 	constexpr uint32_t RS = row_floats<KB, PACKED>();
@@ -1245,6 +1283,16 @@ assign_bf16_kernel(const float* __restrict__ data, size_t stride, const float* _
 					const uint32_t at = 2 * (flagged + __builtin_popcountll(mask & ((1ull << lane) - 1ull)));
 					flag_list[wave][at] = pt;
 					/* kd_unmoved > 0: for kernels that evaluate in the frame of the data (certificate.h) */
+					if constexpr (BEHIND_CELLS) {
+						/* a centroid that can win is at A' <= first + tau, so at S^2 A' plus the error of the other ranking there. What half
+						 * precision leaves out of a coordinate: 2^-11 of it, or 2^-25; none of it holds beyond its largest number. */
+						const float s2 = way.scale[0] * way.scale[0], scaled = s2 * xsq;
+						const float low = 0x1p-11f * cert_sqrt_upper(scaled) + 0x1p-24f;
+						const CertCoeffs cert16 = cert_coeffs_level1(CentroidBounds{ way.scale[2], way.scale[5], 0.0f });
+						const bool covered = xsq + c2max > 1e-30f && scaled < 4e9f && s2 * c2max < 1e37f;
+						flag_list[wave][at + 1] = screening_threshold(covered ? s2 * (first + tau) : __builtin_inff(), cert_tau(way.kd16, scaled, low * low, cert16));
+					}
+					else
 					flag_list[wave][at + 1] = kd_unmoved > 0.0f
 						? screening_threshold(cert_unmoved_threshold(first, tau, xsq, along, c2max, frame_m2, frame_norm, kd_unmoved), 0.0f)
 						: screening_threshold(first, tau);
@@ -1618,7 +1666,7 @@ template <int KB> struct SplitSweepShape {
 };
 
 template <int KB, int LD, bool VEC, bool PACKED = false>
-static int launch_bf16_t(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd)
+static int launch_bf16_t(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd, [[maybe_unused]] const WayBack* way = nullptr)
 {
 	constexpr uint32_t RS = row_floats<KB, PACKED>();
 	constexpr int P = PACKED ? 4 : SplitSweepShape<KB>::P; /* one MFMA per tile: four point tiles share the centroid operand and the norms */
@@ -1690,7 +1738,13 @@ static int launch_bf16_t(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 	else {
 		kernel = assign_bf16_kernel<KB, P, LD, VEC, true, false, PF>;
 	}
-	const void* launched = slices > 1 ? (const void*)sliced_kernel : (const void*)kernel;
+	void (*way_kernel)(const float*, size_t, const float*, const float*, uint32_t*, uint32_t*, uint32_t*,
+	                   uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, float, float, uint32_t, float, WayBack) = nullptr;
+	if constexpr (PACKED) {
+		if (way && stream_mode) way_kernel = coarse ? assign_bf16_kernel<KB, P, LD, VEC, true, true, PF, PACKED, WayBack> : assign_bf16_kernel<KB, P, LD, VEC, true, false, PF, PACKED, WayBack>;
+		else if (way) way_kernel = coarse ? assign_bf16_kernel<KB, PR, LD, VEC, false, true, PF, PACKED, WayBack> : assign_bf16_kernel<KB, PR, LD, VEC, false, false, PF, PACKED, WayBack>;
+	}
+	const void* launched = way_kernel ? (const void*)way_kernel : slices > 1 ? (const void*)sliced_kernel : (const void*)kernel;
 	KMX_HIP(hipFuncSetAttribute(launched, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
 	int per_cu = 1;
 	KMX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, launched, (int)(MFMA_WAVES * WAVE), lds_bytes));
@@ -1703,6 +1757,13 @@ static int launch_bf16_t(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 		const SweepPlan plan = { (uint32_t)KB, RS, kp, a.k, a.n, chunk_rows, slices, lds_bytes, static_bytes, grid, stream_mode, PACKED, wide_rows_sweep<KB>() };
 		if ((rc = check_sweep_plan(plan, ws, dev, a.data, VEC))) return rc;
 		if (slices > 1 ? !sliced_kernel : !kernel) return fail(KMX_ERR_DEVICE, "assign (split-bf16 MFMA): no kernel instance for this plan");
+	}
+	if (way_kernel) { /* (the search ahead of it has begun the profile) */
+		KMX_LAUNCH_KERNEL(way_kernel, dim3(grid), dim3(MFMA_WAVES * WAVE), lds_bytes, stream(),
+		                   a.data, a.stride, ws->packed_means, ws->norms, a.assignment, ws->queue, ws->counters,
+		                   a.dim, a.k, kp, a.n, chunk_rows, kd, -__builtin_inff(), a.shifted_cap, kd_unmoved, *way);
+		KMX_LAUNCH_CHECK("assign_bf16_kernel (behind the cells)");
+		return KMX_OK;
 	}
 	if ((rc = profile_begin(0))) return rc;
 	if (slices == 1) {
@@ -1728,16 +1789,21 @@ static int launch_bf16_t(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 	return profile_end(0);
 }
 
+inline bool aligned_rows(const AssignArgs& a) { return a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data % 16) == 0; }
+
+inline int launch_bf16_packed(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd, const WayBack* way)
+{
+	if (a.layout == KMX_SOA) return launch_bf16_t<1, KMX_SOA, false, true>(a, exec, ws, dev, kp, kd, way);
+	if (aligned_rows(a)) return launch_bf16_t<1, KMX_AOS, true, true>(a, exec, ws, dev, kp, kd, way);
+	return launch_bf16_t<1, KMX_AOS, false, true>(a, exec, ws, dev, kp, kd, way);
+}
+
 template <int KB>
 static int launch_bf16_kb(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd)
 {
-	const bool aligned = a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data % 16) == 0;
+	const bool aligned = aligned_rows(a);
 	if constexpr (KB == 1) {
-		if (packed_rows(a.dim)) {
-			if (a.layout == KMX_SOA) return launch_bf16_t<KB, KMX_SOA, false, true>(a, exec, ws, dev, kp, kd);
-			if (aligned) return launch_bf16_t<KB, KMX_AOS, true, true>(a, exec, ws, dev, kp, kd);
-			return launch_bf16_t<KB, KMX_AOS, false, true>(a, exec, ws, dev, kp, kd);
-		}
+		if (packed_rows(a.dim)) return launch_bf16_packed(a, exec, ws, dev, kp, kd, nullptr);
 	}
 	if (a.layout == KMX_SOA) return launch_bf16_t<KB, KMX_SOA, false>(a, exec, ws, dev, kp, kd);
 	if (aligned) return launch_bf16_t<KB, KMX_AOS, true>(a, exec, ws, dev, kp, kd);

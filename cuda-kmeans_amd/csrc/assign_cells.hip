@@ -327,13 +327,16 @@ struct CellAssignArgs {
 	const Grid* grid; const uint32_t* table; const uint16_t* pool;
 	const float* norms; const float* low2; const float* frame; float* scale; /* of the exact pass (pack_means16_kernel) */
 	uint32_t* assignment; uint32_t* list; uint32_t* length;
+	uint32_t* way_back; /* nullptr: no choice; otherwise 0 or 1 is left there */
 	uint32_t k, kp, n;
 	float kd;
 };
 
 constexpr uint32_t CELL_THREADS = 1024;
 constexpr uint32_t CELL_WAVES = CELL_THREADS / WAVE;
+constexpr uint32_t CHOICE_EACH = 2, CHOICE_GROUPS = CHOICE_EACH * CELL_WAVES; /* groups of 64 points that the choice between cells and sweep looks at */
 constexpr uint32_t CELL_LIST = 64; /* points per wavefront that wait for the list */
+constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* LDS of assign_cells_kernel beside the centroids */
 
 /*
  * A lane per point, the centroids in LDS. What bounds it: the gathers, 16 bytes of centroid per comparison from LDS and 16 bytes of list per
@@ -345,41 +348,100 @@ assign_cells_kernel(const CellAssignArgs w)
 {
 	constexpr uint32_t N = cells_per_dim<D>();
 	extern __shared__ __attribute__((aligned(16))) float lds[]; /* k x 4 */
-	__shared__ uint32_t wave_max[2][CELL_WAVES];
+	__shared__ uint32_t wave_max[6][CELL_WAVES];
 	__shared__ uint32_t flag_list[CELL_WAVES][2 * CELL_LIST];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	const float scale = w.scale[0];
+	float corner[D], inverse[D];
+#pragma unroll
+	for (int q = 0; q < D; ++q) { corner[q] = w.grid->corner[q]; inverse[q] = w.grid->inverse[q]; }
+	auto locate = [&](const float (&x)[D], bool& inside) -> uint32_t {
+		inside = true;
+		uint32_t cell = 0;
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			const float y = (x[q] - corner[q]) * inverse[q];
+			inside = inside && y >= 0.0f && y < (float)N;
+			cell = cell * N + (uint32_t)fminf(fmaxf(y, 0.0f), (float)(N - 1)); /* (NaN: 0) */
+		}
+		return cell;
+	};
+
+	/* the sample of the choice below is on its way while the centroids are */
+	const bool choose = w.way_back != nullptr;
+	float sample[CHOICE_EACH][D];
+	if (choose) {
+#pragma unroll
+		for (uint32_t i = 0; i < CHOICE_EACH; ++i) {
+			const uint32_t pt = min((uint32_t)((uint64_t)(w.n / WAVE) * (wave * CHOICE_EACH + i) / CHOICE_GROUPS) * WAVE + lane, w.n - 1);
+#pragma unroll
+			for (int q = 0; q < D; ++q) sample[i][q] = w.data[elem<LD>(w.stride, pt, q)];
+		}
+	}
 	for (uint32_t j = tid; j < w.k; j += CELL_THREADS) {
 		f32x4 c = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
 		for (int q = 0; q < D; ++q) c[q] = w.means[elem<LM>(w.stride_means, j, q)];
 		*(f32x4*)(lds + 4 * j) = c;
 	}
-	CertCoeffs cert;
-	{
-		uint32_t most[2] = { 0u, 0u };
-		for (uint32_t j = tid; j < w.k; j += CELL_THREADS) {
-			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
-			most[1] = max(most[1], __float_as_uint(w.low2[j]));
+	/* the maxima of the certificate; the first work-group leaves them and those of the exact pass's own (rank16_leave_bounds) */
+	uint32_t most[6] = { 0u, 0u, 0u, 0u, 0u, 0u }; /* of |c|^2, low^2, mid^2, rest^2; then two sums: entries, points without a list */
+	for (uint32_t j = tid; j < w.k; j += CELL_THREADS) {
+		most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
+		most[1] = max(most[1], __float_as_uint(w.low2[j]));
+		if (blockIdx.x == 0) {
+			most[2] = max(most[2], __float_as_uint(w.low2[w.kp + j]));
+			most[3] = max(most[3], __float_as_uint(w.low2[2 * w.kp + j]));
 		}
-#pragma unroll
-		for (int q = 0; q < 2; ++q) {
-			for (int off = WAVE / 2; off > 0; off >>= 1) most[q] = max(most[q], (uint32_t)__shfl_xor((int)most[q], off));
-			if (lane == 0) wave_max[q][wave] = most[q];
-		}
-		__syncthreads();
-#pragma unroll
-		for (int q = 0; q < 2; ++q) {
-			most[q] = 0;
-			for (uint32_t v = 0; v < CELL_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
-		}
-		if (blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], w.low2, w.k, w.kp);
-		cert = cert_coeffs_level1(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), 0.0f });
 	}
-	const float scale = w.scale[0];
-	float corner[D], inverse[D];
+	if (choose) {
 #pragma unroll
-	for (int q = 0; q < D; ++q) { corner[q] = w.grid->corner[q]; inverse[q] = w.grid->inverse[q]; }
+		for (uint32_t i = 0; i < CHOICE_EACH; ++i) {
+			bool inside;
+			const uint32_t entry = w.table[locate(sample[i], inside)];
+			uint32_t units = (entry >> 20) & CELL_MOST_UNITS;
+			for (int off = WAVE / 2; off > 0; off >>= 1) units = max(units, (uint32_t)__shfl_xor((int)units, off));
+			most[4] += units * CELL_UNIT;
+			most[5] += (uint32_t)__popcll(__ballot(!inside || (entry & CELL_TRUNCATED)));
+		}
+	}
+#pragma unroll
+	for (int q = 0; q < 6; ++q) {
+		if (q < 4)
+			for (int off = WAVE / 2; off > 0; off >>= 1) most[q] = max(most[q], (uint32_t)__shfl_xor((int)most[q], off));
+		if (lane == 0) wave_max[q][wave] = most[q];
+	}
+	__syncthreads();
+#pragma unroll
+	for (int q = 0; q < 6; ++q) {
+		most[q] = 0;
+		for (uint32_t v = 0; v < CELL_WAVES; ++v) most[q] = q < 4 ? max(most[q], wave_max[q][v]) : most[q] + wave_max[q][v];
+	}
+	if (blockIdx.x == 0 && tid == 0) {
+		w.scale[2] = __uint_as_float(most[0]); w.scale[3] = __uint_as_float(most[2]);
+		w.scale[4] = __uint_as_float(most[3]); w.scale[5] = __uint_as_float(most[1]);
+	}
+	const CertCoeffs cert = cert_coeffs_level1(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), 0.0f });
+
+	/*
+	 * Are the cells any good for these points? The sample (CHOICE_GROUPS wavefronts' worth, spread evenly over the points) says what
+	 * they would cost: a wavefront its longest list, N = 4M points 75 us and 1.1 (d = 3) to 1.45 us (d = 4) per entry; a point without a list
+	 * as much as k to 2 k entries in the exact pass. The packed sweep costs those points 110 us + 0.14 per centroid, its exact pass what the
+	 * data make of it, and the lists have been built by then. So it is left to that sweep (all work-groups come to the same answer) if
+	 *   - the lists are longer than k / 8 + 70 (d = 4; normal points, k = 1000: 168 entries, 340 against 322 us; exponential 474: 766
+	 *     against 404; points along a line 189: 450 against 2490, the sweep certifies few of those) or k / 8 + 320 (d = 2, 3: skewed data, which
+	 *     has such lists, costs the sweep more too: lognormal, k = 1000: 423 entries, 549 against 1044 us);
+	 *   - or the points without a list cost more than half of the first of these (normal, d = 4, k = 4096: 65 % of the points, 4329
+	 *     against 825 us; all outside the grid, d = 4, k = 1000: 1690 against 287).
+	 */
+	if (choose) {
+		const uint32_t entries = most[4], unlisted = most[5];
+		const bool sweep = 8 * entries > CHOICE_GROUPS * (w.k + 8 * (D == 4 ? 70 : 320)) ||
+		                   3 * w.k * unlisted * 8 > CHOICE_GROUPS * WAVE * (w.k + 8 * 70);
+		if (blockIdx.x == 0 && tid == 0) w.way_back[0] = sweep ? 1u : 0u;
+		if (sweep) return; /* the whole grid */
+	}
 
 	uint32_t flagged = 0; /* wave-uniform */
 	for (uint32_t base = blockIdx.x * CELL_THREADS; base < w.n; base += gridDim.x * CELL_THREADS) {
@@ -388,15 +450,8 @@ assign_cells_kernel(const CellAssignArgs w)
 		float x[D];
 #pragma unroll
 		for (int q = 0; q < D; ++q) x[q] = w.data[elem<LD>(w.stride, min(pt, w.n - 1), q)];
-		bool inside = true;
-		uint32_t cell = 0;
-#pragma unroll
-		for (int q = 0; q < D; ++q) {
-			const float y = (x[q] - corner[q]) * inverse[q];
-			inside = inside && y >= 0.0f && y < (float)N;
-			cell = cell * N + (uint32_t)fminf(fmaxf(y, 0.0f), (float)(N - 1)); /* (NaN: 0) */
-		}
-		const uint32_t entry = w.table[cell];
+		bool inside;
+		const uint32_t entry = w.table[locate(x, inside)];
 		const uint32_t units = (entry >> 20) & CELL_MOST_UNITS;
 		const uint4* list = (const uint4*)w.pool + (entry & 0xFFFFFu);
 		float best = __builtin_inff();
@@ -477,7 +532,7 @@ assign_cells_kernel(const CellAssignArgs w)
 }
 
 template <int D>
-static int launch_cells_d(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half)
+static int launch_cells_d(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half, bool choose)
 {
 	constexpr uint32_t CELLS = cell_count<D>();
 	const size_t table_words = sizeof(Grid) / 4 + CELLS;
@@ -496,33 +551,33 @@ static int launch_cells_d(const AssignArgs& a, kmx_exec_params* exec, Workspace*
 	KMX_LAUNCH_CHECK("build_cells_kernel");
 
 	const CellAssignArgs w = { a.data, a.stride, a.means, a.stride_means, grid, table, pool, half.norms, half.low2, half.frame, half.scale,
-	                           a.assignment, ws->listed, ws->counters + LISTED_COUNTER, a.k, half.kp, a.n, half.kd };
+	                           a.assignment, ws->listed, ws->counters + LISTED_COUNTER, choose ? ws->counters + WAY_BACK_COUNTER : nullptr, a.k, half.kp, a.n, half.kd };
 	void (*assign)(CellAssignArgs) = a.layout == KMX_AOS ? (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_AOS, KMX_AOS> : assign_cells_kernel<D, KMX_AOS, KMX_SOA>)
 	                                                     : (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_SOA, KMX_AOS> : assign_cells_kernel<D, KMX_SOA, KMX_SOA>);
-	const uint32_t lds = a.k * 16, per_cu = std::max<uint32_t>(1, std::min<uint32_t>(2, dev.lds_bytes / (lds + CELL_WAVES * 2 * CELL_LIST * 4 + 256)));
+	const uint32_t lds = a.k * 16, per_cu = std::max<uint32_t>(1, std::min<uint32_t>(2, dev.lds_bytes / (lds + CELL_STATIC)));
 	const uint32_t blocks = std::min((a.n + CELL_THREADS - 1) / CELL_THREADS, per_cu * dev.compute_units);
 	exec->block_count = blocks;
-	if ((rc = profile_begin(0))) return rc;
+	if ((rc = profile_begin(0))) return rc; /* (ended behind the packed sweep: one of the two does the work) */
 	KMX_HIP(hipFuncSetAttribute((const void*)assign, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 	KMX_LAUNCH_KERNEL(assign, dim3(blocks), dim3(CELL_THREADS), lds, stream(), w);
 	KMX_LAUNCH_CHECK("assign_cells_kernel");
-	return profile_end(0);
+	return KMX_OK;
 }
 
 bool cells_support(const AssignArgs& a, uint32_t lds_budget)
 {
 	if (a.dim < 2 || a.dim > 4 || a.k > CELL_MAX_K || a.k < 2 || a.n > (1u << 31) || a.ranking_only) return false;
 	const uint32_t build_lds = a.k * a.dim * 4 + (a.k + 1) / 2 * 4 + BUILD_WAVES * BUILD_SHORT * 2 + 1024;
-	const uint32_t assign_lds = a.k * 16 + CELL_WAVES * 2 * CELL_LIST * 4 + 256;
+	const uint32_t assign_lds = a.k * 16 + CELL_STATIC;
 	return std::max(build_lds, assign_lds) <= lds_budget && exact_dynamic_bytes(1, EXACT_GROUPS) + exact_static_bytes(false) <= lds_budget;
 }
 
-int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half)
+int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half, bool choose)
 {
 	switch (a.dim) {
-	case 2: return launch_cells_d<2>(a, exec, ws, dev, half);
-	case 3: return launch_cells_d<3>(a, exec, ws, dev, half);
-	case 4: return launch_cells_d<4>(a, exec, ws, dev, half);
+	case 2: return launch_cells_d<2>(a, exec, ws, dev, half, choose);
+	case 3: return launch_cells_d<3>(a, exec, ws, dev, half, choose);
+	case 4: return launch_cells_d<4>(a, exec, ws, dev, half, choose);
 	default: return fail(KMX_ERR_UNSUPPORTED, "assign (cells): dim %u is not supported", a.dim);
 	}
 }

@@ -291,7 +291,7 @@ wide_sweep_kernel(const WideArgs w)
 			for (uint32_t v = 0; v < WIDE_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
 		}
 		const CentroidBounds cb{ __uint_as_float(most[0]), __uint_as_float(most[1]), __uint_as_float(most[2]) };
-		if (!X3 && blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], w.part_norms, w.k, w.kp);
+		if (!X3 && blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], most[1], w.part_norms, w.k, w.kp);
 		cert = X3 ? cert_coeffs_split(cb) : cert_coeffs_level1(cb);
 	}
 

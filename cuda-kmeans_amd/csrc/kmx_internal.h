@@ -86,6 +86,7 @@ int reserve_listed(Workspace* ws, size_t words);
 int two_level_mode(); /* kmx_set_two_level_sweep */
 constexpr uint32_t CELLS_COUNTER = 5;  /* word of Workspace::counters that counts the list units handed out by build_cells_kernel */
 constexpr uint32_t FINISH_COUNTER = 6; /* and the one that counts the work-groups fused_finish_kernel has behind it */
+constexpr uint32_t WAY_BACK_COUNTER = 7; /* not zero: the points are left to the packed sweep (assign_cells_kernel) */
 constexpr uint32_t LISTED_COUNTER = 4; /* word of Workspace::counters that holds the length of Workspace::listed */
 
 #define KMX_HIP(call)                                                                                         \
@@ -196,7 +197,7 @@ struct Cells16 {
 };
 bool takes_cells(const AssignArgs& a, uint32_t lds_budget); /* KMX_ASSIGN_MFMA_BF16X3 runs as cells (assign_bf16.hip) */
 bool cells_support(const AssignArgs& a, uint32_t lds_budget);
-int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half);
+int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half, bool choose); /* choose: may leave all points to the packed sweep (WAY_BACK_COUNTER) */
 int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev); /* rank16.hip: all of it */
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST would write a.rows_out */
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);

@@ -57,8 +57,8 @@ __device__ __forceinline__ uint32_t even_row(uint32_t r, uint32_t log, uint32_t 
 	return min(k <= (1u << log) ? r : __umulhi(r / 4 * 0x9E3779B9u, k) + r % 4, k - 1);
 }
 
-/* the exact pass's certificate, by one work-group (first wavefront): max |c|^2, max |mid|^2, max |rest|^2 to scale[2 .. 4] */
-__device__ __forceinline__ void rank16_leave_bounds(float* scale, uint32_t c2max, const float* part_norms, uint32_t k, uint32_t kp)
+/* the exact pass's certificate, by one work-group (first wavefront): max |c|^2, max |mid|^2, max |rest|^2 and max |low|^2 to scale[2 .. 5] */
+__device__ __forceinline__ void rank16_leave_bounds(float* scale, uint32_t c2max, uint32_t low2max, const float* part_norms, uint32_t k, uint32_t kp)
 {
 	if (threadIdx.x >= WAVE) return;
 	uint32_t mid = 0, rest = 0; /* (bit patterns: NaN and infinity win) */
@@ -70,7 +70,7 @@ __device__ __forceinline__ void rank16_leave_bounds(float* scale, uint32_t c2max
 		mid = max(mid, (uint32_t)__shfl_xor((int)mid, off));
 		rest = max(rest, (uint32_t)__shfl_xor((int)rest, off));
 	}
-	if (threadIdx.x == 0) { scale[2] = __uint_as_float(c2max); scale[3] = __uint_as_float(mid); scale[4] = __uint_as_float(rest); }
+	if (threadIdx.x == 0) { scale[2] = __uint_as_float(c2max); scale[3] = __uint_as_float(mid); scale[4] = __uint_as_float(rest); scale[5] = __uint_as_float(low2max); }
 }
 
 /* the 8 coordinates of a half-wave of block kb as they come from memory, zeros beyond the row. Blocks inside the row (the same
@@ -184,7 +184,7 @@ rank16_kernel(const Rank16Args w)
 			most[q] = 0;
 			for (uint32_t v = 0; v < RANK16_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
 		}
-		if (blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], w.low2, w.k, w.kp);
+		if (blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], most[1], w.low2, w.k, w.kp);
 		cert = cert_coeffs_level1(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), 0.0f });
 		cert.c2max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(cert.c2max)));
 		cert.a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(cert.a)));

@@ -60,3 +60,42 @@ def test_cells_match_the_oracle(km, orc, gpu, dim, k, n, kind):
     finally:
         km.set_two_level_sweep(1)
     a.free()
+
+
+@pytest.mark.parametrize("kind", ["planar", "outside", "lattice", "tiny", "huge", "nan"])
+@pytest.mark.parametrize("dim,k", [(2, 600), (3, 6100), (4, 601), (4, 700)])   # (6100: streamed centroids; 600 and more: tracked per tile)
+@pytest.mark.parametrize("layout,pad", [(0, 0), (0, 3), (1, 0)])
+def test_points_the_cells_are_no_good_for_match_the_oracle(km, orc, gpu, dim, k, kind, layout, pad):
+    """In the default mode such points are left to the packed sweep, whose queue goes to the exact pass of the cells."""
+    n = (1 << 18) + 17
+    rng = np.random.default_rng(dim * 41 + k)
+    means = rng.normal(size=(k, dim)).astype(np.float32)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    if kind == "planar":      # no extent in one dimension: no grid
+        means[:, dim - 1] = 0; rows[:, dim - 1] = 0
+    else:                     # all points outside the grid
+        rows[:, 0] += np.float32(20)
+    if kind == "lattice":     # ties
+        means, rows = (np.round(means * 4) / 4).astype(np.float32), (np.round(rows * 8) / 8).astype(np.float32)
+    elif kind in ("tiny", "huge"):
+        factor = np.float32(1e-17 if kind == "tiny" else 3e16)
+        means *= factor; rows *= factor
+    elif kind == "nan":
+        means[k // 2, 0] = np.nan
+    rows[3] = means[3]; rows[7, 0] = np.nan; rows[11, dim - 1] = np.inf; rows[13] = -1e30; rows[17] = 1e6; rows[19] = 1e-30
+    sample = np.concatenate([np.arange(40), rng.choice(n, 30000, replace=False)])
+    stride = dim + pad if layout == 0 else n
+    padded = rows
+    if pad:
+        padded = np.full((n, stride), np.float32(np.nan)); padded[:, :dim] = rows
+    d = km.DeviceBuffer(padded.nbytes); d.write(flat(padded, layout))
+    m = km.DeviceBuffer(4 * k * dim); m.write(flat(means, 0))
+    a = km.DeviceBuffer(4 * n); a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+    km.assign(km.ASSIGN_BEST, d, layout, stride, m, 0, dim, a, dim, k, n)
+    km.sync()
+    got = a.read(np.uint32, n)
+    for b in (d, m, a):
+        b.free()
+    want = orc.assign(np.ascontiguousarray(rows[sample]).ravel(), means.ravel(), dim, k, len(sample), threads=0, fast=True)
+    assert got.max() < k
+    assert np.array_equal(got[sample], want), "%d of %d differ" % (int((got[sample] != want).sum()), len(sample))

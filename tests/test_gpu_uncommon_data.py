@@ -81,3 +81,17 @@ def test_first_centroids_unlike_the_rest(km, orc, gpu, dtype, dim, k, n, kind):
     if kind == "outlier":
         means[k // 2] = 30000
     check(km, orc, rows, means)
+
+
+@pytest.mark.parametrize("kind,dim,k", [("normal", 4, 4096), ("exponential", 4, 1000), ("planar", 4, 1000), ("planar", 3, 4096), ("sorted", 3, 1000), ("sorted", 4, 4096)])
+def test_points_a_regular_grid_is_no_good_for(km, orc, gpu, kind, dim, k):
+    """Rows of few dimensions: a dense middle, no extent in one dimension, first points all at one end."""
+    n = 1 << 22
+    rng = np.random.default_rng(dim + k)
+    rows = rng.exponential(size=(n, dim)).astype(np.float32) if kind == "exponential" else rng.normal(size=(n, dim)).astype(np.float32)
+    if kind == "planar":
+        rows[:, dim - 1] = 0
+    elif kind == "sorted":
+        rows = rng.random((n, dim), dtype=np.float32)
+        rows = np.ascontiguousarray(rows[np.argsort(rows[:, 0])])
+    check(km, orc, rows, rows[:k].copy())
