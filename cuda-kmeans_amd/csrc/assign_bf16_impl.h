@@ -1791,11 +1791,12 @@ static int launch_bf16_t(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 
 inline bool aligned_rows(const AssignArgs& a) { return a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data % 16) == 0; }
 
-inline int launch_bf16_packed(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd, const WayBack* way)
+template <int KB> /* (1; a template, so that only the files that launch it hold its kernels) */
+static int launch_bf16_packed(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd, const WayBack* way)
 {
-	if (a.layout == KMX_SOA) return launch_bf16_t<1, KMX_SOA, false, true>(a, exec, ws, dev, kp, kd, way);
-	if (aligned_rows(a)) return launch_bf16_t<1, KMX_AOS, true, true>(a, exec, ws, dev, kp, kd, way);
-	return launch_bf16_t<1, KMX_AOS, false, true>(a, exec, ws, dev, kp, kd, way);
+	if (a.layout == KMX_SOA) return launch_bf16_t<KB, KMX_SOA, false, true>(a, exec, ws, dev, kp, kd, way);
+	if (aligned_rows(a)) return launch_bf16_t<KB, KMX_AOS, true, true>(a, exec, ws, dev, kp, kd, way);
+	return launch_bf16_t<KB, KMX_AOS, false, true>(a, exec, ws, dev, kp, kd, way);
 }
 
 template <int KB>
@@ -1803,7 +1804,7 @@ static int launch_bf16_kb(const AssignArgs& a, kmx_exec_params* exec, Workspace*
 {
 	const bool aligned = aligned_rows(a);
 	if constexpr (KB == 1) {
-		if (packed_rows(a.dim)) return launch_bf16_packed(a, exec, ws, dev, kp, kd, nullptr);
+		if (packed_rows(a.dim)) return launch_bf16_packed<KB>(a, exec, ws, dev, kp, kd, nullptr);
 	}
 	if (a.layout == KMX_SOA) return launch_bf16_t<KB, KMX_SOA, false>(a, exec, ws, dev, kp, kd);
 	if (aligned) return launch_bf16_t<KB, KMX_AOS, true>(a, exec, ws, dev, kp, kd);

@@ -21,7 +21,7 @@ int KMX_CAT(launch_bf16_, KMX_KB)(const AssignArgs& a, kmx_exec_params* exec, Wo
 #if KMX_KB == 1
 int launch_bf16_behind_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, uint32_t kp, float kd, const WayBack& way)
 {
-	return launch_bf16_packed(a, exec, ws, dev, kp, kd, &way);
+	return launch_bf16_packed<KMX_KB>(a, exec, ws, dev, kp, kd, &way);
 }
 #endif
 

@@ -48,8 +48,10 @@ struct Grid {
 
 struct CellArgs {
 	const float* means; size_t stride_means;
-	Grid* grid; uint32_t* table; uint16_t* pool; uint32_t* used;
-	uint32_t k, pool_units;
+	Grid* grid; uint32_t* table; uint16_t* pool; uint32_t* counters;
+	_Float16* packed; float* rows; float* norms;  /* operands, rows and norms of the exact pass (rank16_impl.h) */
+	float* packed_form; float* form_norms;        /* of the packed sweep (assign_bf16_impl.h) */
+	uint32_t k, kp, pool_units;
 };
 
 template <int D>
@@ -68,7 +70,8 @@ __device__ __forceinline__ void cell_distances(const float (&c)[D], const float 
 
 /*
  * One work-group per first-level cell. All of them find the box of the centroids (they have to read them anyway), then three levels of
- * lists, each filtered from the one above: the work-group's, one per wavefront, one per cell.
+ * lists, each filtered from the one above: the work-group's, one per wavefront, one per cell. On the way a wavefront packs a row for
+ * the exact pass and the packed sweep (as a kernel of its own ahead of this one that took 5 to 7 us and a launch).
  * What bounds it: the latency of its dozen barriers and of the pass over all centroids (12 us at k = 4096, d = 4; one level
  * of lists, every cell from all centroids, would be 65536 x k boxes, a millisecond).
  */
@@ -88,7 +91,17 @@ build_cells_kernel(const CellArgs w)
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 
-	/* the box of the centroids; anything that is not finite shows in it */
+	/* the frame of the packed rows: the mean of 16 centroids spread evenly; and this wavefront's (first) row, a coordinate per lane */
+	float frame[D], member[D];
+	{
+		const uint32_t r = even_row(lane % 16, 4, w.k);
+#pragma unroll
+		for (int q = 0; q < D; ++q) member[q] = w.means[elem<LM>(w.stride_means, r, q)];
+	}
+	const uint32_t first_row = blockIdx.x * BUILD_WAVES + wave;
+	float exact = w.means[elem<LM>(w.stride_means, min(first_row, w.k - 1), min(lane, (uint32_t)D - 1))];
+
+	/* the box of the centroids (of their finite coordinates) */
 	float low[D], high[D];
 #pragma unroll
 	for (int q = 0; q < D; ++q) { low[q] = __builtin_inff(); high[q] = -__builtin_inff(); }
@@ -98,18 +111,26 @@ build_cells_kernel(const CellArgs w)
 		for (int q = 0; q < D; ++q) {
 			const float v = w.means[elem<LM>(w.stride_means, j, q)];
 			coords[j * D + q] = v;
-			low[q] = fminf(low[q], v);
-			high[q] = fmaxf(high[q], v);
-			odd = odd || !(__builtin_fabsf(v) < __builtin_inff());
+			const bool finite = __builtin_fabsf(v) < __builtin_inff();
+			low[q] = finite ? fminf(low[q], v) : low[q];
+			high[q] = finite ? fmaxf(high[q], v) : high[q];
+			odd = odd || !finite;
 		}
 #pragma unroll
 	for (int q = 0; q < D; ++q) {
 		for (int off = WAVE / 2; off > 0; off >>= 1) { low[q] = fminf(low[q], __shfl_xor(low[q], off)); high[q] = fmaxf(high[q], __shfl_xor(high[q], off)); }
 		if (lane == 0) { reduce[q][wave] = low[q]; reduce[D + q][wave] = high[q]; }
 	}
+#pragma unroll
+	for (int q = 0; q < D; ++q) {
+		float sum = __builtin_fabsf(member[q]) < __builtin_inff() ? member[q] : 0.0f;
+		for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+		sum = sum / 16.0f;
+		frame[q] = __builtin_fabsf(sum) < __builtin_inff() ? sum : 0.0f; /* (the sum of finite values may overflow) */
+	}
 	if (tid == 0) pool_start = 0;
 	bool usable = !__syncthreads_or(odd ? 1 : 0);
-	float corner[D], width[D], inverse[D];
+	float corner[D], width[D], inverse[D], far = 0.0f, size = 0.0f;
 	{
 		const float share = fmaxf(0.75f * __builtin_powf((float)w.k, -1.0f / D), 0.05f); /* of the extent, added on either side */
 		float extent2 = 0.0f;
@@ -117,6 +138,8 @@ build_cells_kernel(const CellArgs w)
 		for (int q = 0; q < D; ++q) {
 			float lo = reduce[q][0], hi = reduce[D + q][0];
 			for (uint32_t v = 1; v < BUILD_WAVES; ++v) { lo = fminf(lo, reduce[q][v]); hi = fmaxf(hi, reduce[D + q][v]); }
+			far = fmaxf(far, fmaxf(hi - frame[q], frame[q] - lo));
+			size = fmaxf(size, fmaxf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
 			const float half = fmaxf(0.5f * (hi - lo) * (1.0f + 2.0f * share), 1e-6f * (__builtin_fabsf(lo) + __builtin_fabsf(hi)) + 1e-16f);
 			corner[q] = 0.5f * lo + 0.5f * hi - half;
 			width[q] = 2.0f * half / (float)N;
@@ -138,6 +161,55 @@ build_cells_kernel(const CellArgs w)
 	}
 	if (blockIdx.x == 0 && tid < CELL_SAMPLE) w.pool[tid] = (uint16_t)((uint64_t)tid * w.k / CELL_SAMPLE);
 	const uint32_t nothing = CELL_TRUNCATED | (CELL_SAMPLE / CELL_UNIT) << 20; /* the sample */
+
+	/* the packed rows, as pack_means16_kernel and pack_means_bf16_kernel make them */
+	{
+		const bool any = size < __builtin_inff(); /* (of finite coordinates) */
+		const float scale = rank16_scale(any ? far : 0.0f, any ? size : 0.0f);
+		float m = 0.0f;
+#pragma unroll
+		for (int q = 0; q < D; ++q) m = lane == (uint32_t)q ? frame[q] : m;
+		for (uint32_t j = first_row; j < w.kp; j += gridDim.x * BUILD_WAVES) {
+			if (j != first_row) exact = w.means[elem<LM>(w.stride_means, min(j, w.k - 1), min(lane, (uint32_t)D - 1))];
+			const bool there = j < w.k && lane < (uint32_t)D;
+			const float v = there ? __builtin_fmaf(exact, scale, -(m * scale)) : 0.0f;
+			const float cv = -2.0f * v;
+			const _Float16 half = (_Float16)cv;
+			const float low_part = cv - (float)half;
+			__bf16 hi, mid;
+			const float rest = split_bf16(cv, hi, mid);
+			float sums[7] = { v * v, low_part * low_part, (float)mid * (float)mid, rest * rest, 0.0f, 0.0f, 0.0f };
+			const float moved = __shfl(there ? exact - m : 0.0f, (int)(lane % 4)); /* (by all lanes; zeros behind the row) */
+			if (lane < KBLOCK) {
+				w.rows[(size_t)j * KBLOCK + lane] = there ? exact : 0.0f;
+				w.packed[((size_t)(j / TILE) * WAVE + lane / 8 * TILE + j % TILE) * 8 + lane % 8] = half;
+				pack_packed_row(w.packed_form, j, lane, moved, sums[4], sums[5], sums[6]);
+			}
+#pragma unroll
+			for (int u = 0; u < 7; ++u) { sums[u] += __shfl_xor(sums[u], 2); sums[u] += __shfl_xor(sums[u], 1); }
+			if (lane == 0) {
+				w.norms[norm_at(j)] = j < w.k ? sums[0] : 1.7e38f;
+				w.form_norms[norm_at(j)] = j < w.k ? sums[4] : __builtin_inff();
+#pragma unroll
+				for (int u = 0; u < 3; ++u) w.norms[rank16_low_offset(w.kp) + u * w.kp + j] = sums[1 + u];
+#pragma unroll
+				for (int u = 0; u < 2; ++u) w.form_norms[split_norms_offset(w.kp) + u * w.kp + j] = sums[5 + u];
+			}
+			if (lane < NORM_TILE - TILE && j % TILE == 0) {
+				w.norms[(j / TILE) * NORM_TILE + TILE + lane] = 1.7e38f;
+				w.form_norms[(j / TILE) * NORM_TILE + TILE + lane] = __builtin_inff();
+			}
+		}
+		if (blockIdx.x == 0 && wave == 0) {
+			if (lane < KBLOCK) w.norms[rank16_frame_offset(w.kp) + lane] = m; /* (zeros behind the row) */
+			if (lane < 4) w.form_norms[frame_offset(w.kp) + lane] = m;
+			if (lane == 0) {
+				w.norms[rank16_scale_offset(w.kp)] = scale;
+				w.norms[rank16_scale_offset(w.kp) + 1] = 1.0f / (scale * scale);
+				w.counters[0] = 0u; w.counters[LISTED_COUNTER] = 0u; /* (CELLS_COUNTER: cleared by the last search) */
+			}
+		}
+	}
 
 	/* this lane's cell */
 	uint32_t top[D], mid[D], at[D];
@@ -293,7 +365,7 @@ build_cells_kernel(const CellArgs w)
 	if (tid == 0) {
 		uint32_t all = 0;
 		for (uint32_t v = 0; v < BUILD_WAVES; ++v) { const uint32_t u = wave_units[v]; wave_units[v] = all; all += u; }
-		pool_start = CELL_SAMPLE / CELL_UNIT + atomicAdd(w.used, all);
+		pool_start = CELL_SAMPLE / CELL_UNIT + atomicAdd(w.counters + CELLS_COUNTER, all);
 	}
 	__syncthreads();
 	const uint32_t start = pool_start + wave_units[wave] + upto - units; /* (lanes of a cell behind its first: upto counts the cell already) */
@@ -325,10 +397,10 @@ struct CellAssignArgs {
 	const float* data; size_t stride;
 	const float* means; size_t stride_means;
 	const Grid* grid; const uint32_t* table; const uint16_t* pool;
-	const float* norms; const float* low2; const float* frame; float* scale; /* of the exact pass (pack_means16_kernel) */
-	uint32_t* assignment; uint32_t* list; uint32_t* length;
-	uint32_t* way_back; /* nullptr: no choice; otherwise 0 or 1 is left there */
-	uint32_t k, kp, n;
+	const float* norms; const float* low2; const float* frame; float* scale; /* of the exact pass */
+	uint32_t* assignment; uint32_t* list;
+	uint32_t* counters; /* LISTED_COUNTER: the list's length; CELLS_COUNTER: cleared for the next call; WAY_BACK_COUNTER: 0 or 1 is left there */
+	uint32_t k, kp, n, choose;
 	float kd;
 };
 
@@ -340,10 +412,12 @@ constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* 
 
 /*
  * A lane per point, the centroids in LDS. What bounds it: the gathers, 16 bytes of centroid per comparison from LDS and 16 bytes of list per
- * eight of them from the caches, and the longest list among a wavefront's points.
+ * eight of them from the caches, and the longest list among a wavefront's points. Two work-groups share a compute unit, eight wavefronts
+ * a SIMD: with more than 80 scalar registers (and the 16 the hardware adds) only seven fit, which is one work-group (d = 3, k = 4096,
+ * normal points: 162 -> 220 us).
  */
 template <int D, int LD, int LM>
-__global__ void __launch_bounds__(CELL_THREADS)
+__global__ void __launch_bounds__(CELL_THREADS) __attribute__((amdgpu_num_sgpr(80)))
 assign_cells_kernel(const CellAssignArgs w)
 {
 	constexpr uint32_t N = cells_per_dim<D>();
@@ -369,7 +443,7 @@ assign_cells_kernel(const CellAssignArgs w)
 	};
 
 	/* the sample of the choice below is on its way while the centroids are */
-	const bool choose = w.way_back != nullptr;
+	const bool choose = w.choose != 0;
 	float sample[CHOICE_EACH][D];
 	if (choose) {
 #pragma unroll
@@ -419,6 +493,7 @@ assign_cells_kernel(const CellAssignArgs w)
 		for (uint32_t v = 0; v < CELL_WAVES; ++v) most[q] = q < 4 ? max(most[q], wave_max[q][v]) : most[q] + wave_max[q][v];
 	}
 	if (blockIdx.x == 0 && tid == 0) {
+		w.counters[CELLS_COUNTER] = 0u;
 		w.scale[2] = __uint_as_float(most[0]); w.scale[3] = __uint_as_float(most[2]);
 		w.scale[4] = __uint_as_float(most[3]); w.scale[5] = __uint_as_float(most[1]);
 	}
@@ -439,7 +514,7 @@ assign_cells_kernel(const CellAssignArgs w)
 		const uint32_t entries = most[4], unlisted = most[5];
 		const bool sweep = 8 * entries > CHOICE_GROUPS * (w.k + 8 * (D == 4 ? 70 : 320)) ||
 		                   3 * w.k * unlisted * 8 > CHOICE_GROUPS * WAVE * (w.k + 8 * 70);
-		if (blockIdx.x == 0 && tid == 0) w.way_back[0] = sweep ? 1u : 0u;
+		if (blockIdx.x == 0 && tid == 0) w.counters[WAY_BACK_COUNTER] = sweep ? 1u : 0u;
 		if (sweep) return; /* the whole grid */
 	}
 
@@ -487,7 +562,7 @@ assign_cells_kernel(const CellAssignArgs w)
 				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 				__builtin_amdgcn_wave_barrier();
 				uint32_t slot = 0;
-				if (lane == 0) slot = atomicAdd(w.length, flagged);
+				if (lane == 0) slot = atomicAdd(w.counters + LISTED_COUNTER, flagged);
 				slot = (uint32_t)__shfl((int)slot, 0);
 				for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[2 * (size_t)slot + i] = flag_list[wave][i];
 				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -525,7 +600,7 @@ assign_cells_kernel(const CellAssignArgs w)
 		all += wave_max[0][v];
 	}
 	if (all == 0) return;
-	if (tid == 0) wave_max[1][0] = atomicAdd(w.length, all);
+	if (tid == 0) wave_max[1][0] = atomicAdd(w.counters + LISTED_COUNTER, all);
 	__syncthreads();
 	const size_t slot = 2 * (size_t)(wave_max[1][0] + before);
 	for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[slot + i] = flag_list[wave][i];
@@ -544,14 +619,18 @@ static int launch_cells_d(const AssignArgs& a, kmx_exec_params* exec, Workspace*
 	uint16_t* pool = (uint16_t*)(ws->cells + table_words);
 	static_assert(sizeof(Grid) % 16 == 0 && CELLS % 4 == 0, "the pool is read in units of 16 bytes");
 	const uint32_t build_lds = a.k * D * 4 + (a.k + 1) / 2 * 4 + BUILD_WAVES * BUILD_SHORT * 2;
-	const CellArgs b = { a.means, a.stride_means, grid, table, pool, ws->counters + CELLS_COUNTER, a.k, CELL_POOL_UNITS };
+	const CellArgs b = { a.means, a.stride_means, grid, table, pool, ws->counters, (_Float16*)ws->packed16, ws->packed16 + rank16_rows_offset(half.kp, KBLOCK), ws->norms16,
+	                     ws->packed_means, ws->norms, a.k, half.kp, CELL_POOL_UNITS };
+	if (!sizing_only() && ((size_t)half.kp * KBLOCK * 3 / 2 > ws->packed16_cap || rank16_norms_floats(half.kp) > ws->norms16_cap ||
+	                       (size_t)half.kp / TILE * tile_floats(row_floats<1, true>()) > ws->packed_cap || split_norms_floats(half.kp) > ws->norms_cap))
+		return fail(KMX_ERR_DEVICE, "assign (cells): launch refused, the packed rows of k %u do not fit their buffers", a.k);
 	void (*build)(CellArgs) = a.layout_means == KMX_AOS ? build_cells_kernel<D, KMX_AOS> : build_cells_kernel<D, KMX_SOA>;
 	KMX_HIP(hipFuncSetAttribute((const void*)build, hipFuncAttributeMaxDynamicSharedMemorySize, (int)build_lds));
 	KMX_LAUNCH_KERNEL(build, dim3(power(CellShape<D>::TOP, D)), dim3(BUILD_THREADS), build_lds, stream(), b);
 	KMX_LAUNCH_CHECK("build_cells_kernel");
 
 	const CellAssignArgs w = { a.data, a.stride, a.means, a.stride_means, grid, table, pool, half.norms, half.low2, half.frame, half.scale,
-	                           a.assignment, ws->listed, ws->counters + LISTED_COUNTER, choose ? ws->counters + WAY_BACK_COUNTER : nullptr, a.k, half.kp, a.n, half.kd };
+	                           a.assignment, ws->listed, ws->counters, a.k, half.kp, a.n, choose ? 1u : 0u, half.kd };
 	void (*assign)(CellAssignArgs) = a.layout == KMX_AOS ? (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_AOS, KMX_AOS> : assign_cells_kernel<D, KMX_AOS, KMX_SOA>)
 	                                                     : (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_SOA, KMX_AOS> : assign_cells_kernel<D, KMX_SOA, KMX_SOA>);
 	const uint32_t lds = a.k * 16, per_cu = std::max<uint32_t>(1, std::min<uint32_t>(2, dev.lds_bytes / (lds + CELL_STATIC)));

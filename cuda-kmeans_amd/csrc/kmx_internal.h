@@ -190,7 +190,7 @@ bool bf16_supports(const AssignArgs& a, uint32_t lds_budget, const DeviceInfo& d
 int launch_assign_bf16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* rank16.hip: one half-precision product per dimension for all points, the serial result for what that leaves */
 bool rank16_supports(const AssignArgs& a, uint32_t lds_budget);
-/* assign_cells.hip: rows of 2 to 4 dimensions through a grid; half: what pack_means16_kernel left for the exact pass */
+/* assign_cells.hip: rows of 2 to 4 dimensions through a grid; half: where the exact pass finds its norms, frame and scale */
 struct Cells16 {
 	const float* norms; const float* low2; const float* frame; float* scale;
 	uint32_t kp; float kd;

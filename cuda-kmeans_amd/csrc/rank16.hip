@@ -23,9 +23,6 @@
 
 namespace kmx {
 
-/* ws->packed16: the operands, then the centroids' rows as they are, padded with zeros to whole blocks */
-static size_t rank16_rows_offset(uint32_t kp, uint32_t dp) { return (size_t)kp * dp / 2; }
-
 /* blocks of 16 dimensions the sweep is built for */
 static uint32_t rank16_kb(uint32_t dim)
 {
@@ -48,22 +45,16 @@ KMX_DECLARE_EXACT16(6) KMX_DECLARE_EXACT16(8) KMX_DECLARE_EXACT16(12) KMX_DECLAR
  * bf16 parts leave out. Every work-group computes the frame m and S (rank16_scale) from centroids spread evenly over
  * all of them: the first ones are often the first points, and those may be unlike the rest (blank rows ahead of an image, the quiet start
  * of a recording).
- * norms: tiles of S^2 |c - m|^2, then per row low2, mid2, rest2, then the frame, S, 1 / S^2 and (rank16_leave_bounds) three maxima.
  */
-__host__ __device__ __forceinline__ size_t rank16_low_offset(uint32_t kp) { return (size_t)(kp / TILE) * NORM_TILE; }
-__host__ __device__ __forceinline__ size_t rank16_frame_offset(uint32_t kp) { return rank16_low_offset(kp) + 3 * (size_t)kp; }
-__host__ __device__ __forceinline__ size_t rank16_scale_offset(uint32_t kp) { return rank16_frame_offset(kp) + FRAME_FLOATS; }
-static size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) + 8; }
-
 template <int LM>
 __global__ void __launch_bounds__(256)
 pack_means16_kernel(const float* __restrict__ means, const double* __restrict__ means64, size_t stride_means, _Float16* __restrict__ packed, float* __restrict__ rows, float* __restrict__ norms,
-                    uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters, float* __restrict__ packed_form, float* __restrict__ form_norms)
+                    uint32_t dim, uint32_t k, uint32_t kp, uint32_t dp, uint32_t* __restrict__ counters)
 {
 	__shared__ float frame[FRAME_DIMS];
 	__shared__ float wave_far[2][4];
 	const uint32_t lane = threadIdx.x & (WAVE - 1);
-	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; counters[CELLS_COUNTER] = 0u; }
+	if (blockIdx.x == 0 && threadIdx.x == 0) { counters[0] = 0u; counters[LISTED_COUNTER] = 0u; }
 	const uint32_t j = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
 	/* this row's coordinates are requested ahead of the frame they will be moved to */
 	float exact[FRAME_DIMS / WAVE];
@@ -137,26 +128,6 @@ pack_means16_kernel(const float* __restrict__ means, const double* __restrict__ 
 		norms[rank16_low_offset(kp) + 2 * kp + j] = rest2;
 	}
 	if (lane < NORM_TILE - TILE && j % TILE == 0) norms[(j / TILE) * NORM_TILE + TILE + lane] = 1.7e38f;
-
-	/* rows of up to four dimensions: also the operands of the packed sweep, in the same frame (pack_means_bf16_kernel) */
-	if (packed_form) {
-		const uint32_t q = lane % 4;
-		const float mine = __shfl(exact[0], (int)q);
-		c2 = mid2 = rest2 = 0.0f;
-		if (lane < KBLOCK) pack_packed_row(packed_form, j, lane, (j < k && q < dim) ? mine - frame[q] : 0.0f, c2, mid2, rest2);
-		for (int off = 2; off > 0; off >>= 1) {
-			c2 += __shfl_xor(c2, off);
-			mid2 += __shfl_xor(mid2, off);
-			rest2 += __shfl_xor(rest2, off);
-		}
-		if (lane == 0) {
-			form_norms[norm_at(j)] = j < k ? c2 : __builtin_inff();
-			form_norms[split_norms_offset(kp) + j] = mid2;
-			form_norms[split_norms_offset(kp) + kp + j] = rest2;
-		}
-		if (lane < NORM_TILE - TILE && j % TILE == 0) form_norms[(j / TILE) * NORM_TILE + TILE + lane] = __builtin_inff();
-		if (j == 0 && lane < 4) form_norms[frame_offset(kp) + lane] = frame[lane]; /* (zeros behind the row) */
-	}
 }
 
 bool rank16_supports(const AssignArgs& a, uint32_t lds_budget)
@@ -168,16 +139,14 @@ bool rank16_supports(const AssignArgs& a, uint32_t lds_budget)
 }
 
 /* the centroids for launch_rank16_sweep */
-static int launch_pack16(const AssignArgs& a, Workspace* ws, bool packed_form = false)
+static int launch_pack16(const AssignArgs& a, Workspace* ws)
 {
 	const uint32_t dp = rank16_kb(a.dim) * KBLOCK, kp = round_up(a.k, TILE);
-	int rc = reserve_packed16(ws, rank16_rows_offset(kp, dp) + (size_t)kp * dp * (a.points64 ? 2 : 1), rank16_norms_floats(kp));
+	const int rc = reserve_packed16(ws, rank16_rows_offset(kp, dp) + (size_t)kp * dp * (a.points64 ? 2 : 1), rank16_norms_floats(kp));
 	if (rc) return rc;
-	if (packed_form && (rc = reserve_packed(ws, (size_t)(kp / TILE) * tile_floats(row_floats<1, true>()), split_norms_floats(kp), 0))) return rc;
 	auto pack = a.layout_means == KMX_AOS ? pack_means16_kernel<KMX_AOS> : pack_means16_kernel<KMX_SOA>;
 	KMX_LAUNCH_KERNEL(pack, dim3((kp * WAVE + 255) / 256), dim3(256), 0, stream(),
-	                   a.means, a.means64, a.stride_means, (_Float16*)ws->packed16, ws->packed16 + rank16_rows_offset(kp, dp), ws->norms16, a.dim, a.k, kp, dp, ws->counters,
-	                   packed_form ? ws->packed_means : nullptr, packed_form ? ws->norms : nullptr);
+	                   a.means, a.means64, a.stride_means, (_Float16*)ws->packed16, ws->packed16 + rank16_rows_offset(kp, dp), ws->norms16, a.dim, a.k, kp, dp, ws->counters);
 	KMX_LAUNCH_CHECK("pack_means16_kernel");
 	return KMX_OK;
 }
@@ -268,9 +237,10 @@ int launch_bf16_behind_cells(const AssignArgs& a, kmx_exec_params* exec, Workspa
 int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	const bool choose = two_level_mode() != 2; /* (tests of the cells take them whatever the points) */
-	int rc = launch_pack16(a, ws, choose);
-	if (rc) return rc;
 	const uint32_t kp = round_up(a.k, TILE);
+	int rc = reserve_packed16(ws, rank16_rows_offset(kp, KBLOCK) + (size_t)kp * KBLOCK, rank16_norms_floats(kp));
+	if (rc) return rc;
+	if ((rc = reserve_packed(ws, (size_t)(kp / TILE) * tile_floats(row_floats<1, true>()), split_norms_floats(kp), 0))) return rc;
 	const Cells16 half = { ws->norms16, ws->norms16 + rank16_low_offset(kp), ws->norms16 + rank16_frame_offset(kp), ws->norms16 + rank16_scale_offset(kp), kp,
 	                       cert_kd_level1(a.dim) + 8.0f * CERT_UNIT };
 	if ((rc = launch_cells(a, exec, ws, dev, half, choose))) return rc;

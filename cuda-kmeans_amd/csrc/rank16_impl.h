@@ -31,6 +31,15 @@ struct Rank16Args {
 	float kd;
 };
 
+/* ws->packed16: the operands, then the centroids' rows as they are, padded with zeros to whole blocks */
+inline size_t rank16_rows_offset(uint32_t kp, uint32_t dp) { return (size_t)kp * dp / 2; }
+/* ws->norms16: tiles of S^2 |c - m|^2, then per row the squared norms of what half precision leaves out, of the bf16 mid and of the rest
+ * parts, then the frame m, S, 1 / S^2 and (rank16_leave_bounds) four maxima */
+__host__ __device__ __forceinline__ size_t rank16_low_offset(uint32_t kp) { return (size_t)(kp / TILE) * NORM_TILE; }
+__host__ __device__ __forceinline__ size_t rank16_frame_offset(uint32_t kp) { return rank16_low_offset(kp) + 3 * (size_t)kp; }
+__host__ __device__ __forceinline__ size_t rank16_scale_offset(uint32_t kp) { return rank16_frame_offset(kp) + FRAME_FLOATS; }
+inline size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) + 8; }
+
 /* 16 tile bytes per block of 16 dimensions and lane, then the tile's norms */
 template <int KB> constexpr uint32_t rank16_tile_floats() { return KB * WAVE * 4; }
 template <int KB> constexpr uint32_t rank16_static_bytes() { return (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + KB * KBLOCK) * 4 + 64; }
