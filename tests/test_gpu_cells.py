@@ -99,3 +99,36 @@ def test_points_the_cells_are_no_good_for_match_the_oracle(km, orc, gpu, dim, k,
     want = orc.assign(np.ascontiguousarray(rows[sample]).ravel(), means.ravel(), dim, k, len(sample), threads=0, fast=True)
     assert got.max() < k
     assert np.array_equal(got[sample], want), "%d of %d differ" % (int((got[sample] != want).sum()), len(sample))
+
+
+@pytest.mark.parametrize("kind", ["inside", "outside"])
+def test_recorded_cells_replay(km, orc, gpu, kind):
+    """Recorded right after a reservation, replayed with eager calls of another shape in between: the choice between cells and sweep is
+    made anew in every replay, and no counter is left over."""
+    dim, k, n = 4, 700, (1 << 18) + 5
+    rng = np.random.default_rng(7)
+    means = rng.random((k, dim), dtype=np.float32)
+    rows = rng.random((n, dim), dtype=np.float32)
+    far = (rows + np.float32(3)).astype(np.float32)
+    d = km.DeviceBuffer(rows.nbytes); m = km.DeviceBuffer(means.nbytes); m.write(means.ravel())
+    a = km.DeviceBuffer(4 * n)
+    km.sync()
+    km.check(km.hip_lib().kmx_shutdown())
+    km.reserve(km.ASSIGN_BEST, km.UPDATE_ATOMIC_SHM, 0, 0, dim, k, n)
+    with km.Graph() as g:
+        km.assign(km.ASSIGN_BEST, d, 0, dim, m, 0, dim, a, dim, k, n)
+    sample = rng.choice(n, 20000, replace=False)
+    for turn in range(4):
+        points = rows if (turn + (kind == "outside")) % 2 == 0 else far
+        d.write(points.ravel())
+        a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+        g.launch()
+        km.sync()
+        got = a.read(np.uint32, n)
+        want = orc.assign(np.ascontiguousarray(points[sample]).ravel(), means.ravel(), dim, k, len(sample), threads=0, fast=True)
+        assert got.max() < k and np.array_equal(got[sample], want), turn
+        km.assign(km.ASSIGN_BEST, d, 0, 3, m, 0, 3, a, 3, 600, n)     # eager, another grid in the same buffers
+        km.sync()
+    g.destroy()
+    for b in (d, m, a):
+        b.free()
