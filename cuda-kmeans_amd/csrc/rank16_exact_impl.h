@@ -247,24 +247,30 @@ listed_exact_kernel(const ExactArgs<F> w)
 		};
 		uint32_t noted = 0;                      /* wave-uniform */
 		[[maybe_unused]] uint32_t kept = 0;      /* doubles: of those, evaluated before and kept */
-		/* a list that is full: 16 pairs at a time (their rows and the tile's centroids are in the caches), or, rows of up to four floats, one per lane */
+		/* a list that is full: 16 pairs at a time (their rows and the tile's centroids are in the caches), or, rows of one block, a pair per lane */
 		auto evaluate_here = [&]() {
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 			__builtin_amdgcn_wave_barrier();
 			[[maybe_unused]] const uint32_t full = noted;
-			if (KB == 1 && w.dim <= 4) {
+			if constexpr (KB == 1) {
 #pragma clang fp contract(off)
 				for (uint32_t i = kept + lane; i < noted; i += WAVE) {
 					const uint32_t hit = hits[wave][i], row = hit >> 25, c = hit & CENTROID;
-					F4 x;
-					exact_request<F>(x, serial_source(row), 0, w.dim, w.points_dim, w.points_step, points_strided);
-					const F4 m = *(const F4*)(w.means + (size_t)c * DP);
+					const F* src = serial_source(row);
+					const F* mean = w.means + (size_t)c * DP;
 					F sum = (F)0;
+#pragma unroll 1
+					for (uint32_t d = 0; d < w.dim; d += 4) {
+						F4 x;
+						exact_request<F>(x, src, d, w.dim, w.points_dim, w.points_step, points_strided);
+						const F4 m = *(const F4*)(mean + d);
+						if (points_ragged && d + 4 > w.points_dim) exact_place<F>(x, d, w.points_dim);
 #pragma unroll
-					for (int e = 0; e < 4; ++e) {
-						const F diff = x[e] - m[e];
-						const F sq = diff * diff;
-						sum = sum + sq;
+						for (int e = 0; e < 4; ++e) {
+							const F diff = x[e] - m[e];
+							const F sq = diff * diff;
+							sum = sum + sq; /* (zeros behind the row change nothing) */
+						}
 					}
 					merge(row, c, sum, wave * EXACT_HITS + i);
 				}
@@ -345,7 +351,12 @@ listed_exact_kernel(const ExactArgs<F> w)
 				const unsigned long long mask = __builtin_amdgcn_ballot_w64(passed != 0);
 				if (mask == 0) break;
 				const uint32_t more = (uint32_t)__popcll(mask);
-				if (noted + more > EXACT_HITS) return false;
+				if (noted + more > EXACT_HITS) {
+					/* (evaluated here it takes registers from the loops over tiles and groups, which rows of one block have to spare; taking those
+					 * loops up again costs them 7 %: N = 1M, d = 16, k = 1024, coordinates of 0 and 1: 249 against 233 us) */
+					if constexpr (KB == 1) evaluate_here();
+					else return false;
+				}
 				if (passed) {
 					const uint32_t r = (uint32_t)__builtin_ctz(passed);
 					hits[wave][noted + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (g * TILE + col) << 25 | (t * TILE + 8 * (r / 4) + 4 * h + r % 4);
