@@ -206,7 +206,9 @@ listed_exact_kernel(const ExactArgs<F> w)
 #pragma clang fp contract(off)
 			const F* src = serial_source(row);
 			const F* mean = w.means + (size_t)c * DP + lane % 4 * 4;
-			constexpr uint32_t AT_ONCE = KB == 0 ? 2 : 1; /* blocks requested together (wide rows come from the L2 and are whole chunks of four blocks) */
+			/* blocks requested together: often one wavefront has all the pairs and nobody to wait beside (wide rows are whole chunks of four blocks) */
+			constexpr uint32_t AT_ONCE = KB == 1 ? 1 : KB == 3 || KB == 6 ? 3 : KB == 2 || DOUBLES ? 2 : 4;
+			static_assert(KB % AT_ONCE == 0, "whole steps");
 			F sum = (F)0;
 #pragma unroll 1
 			for (uint32_t kb = 0; kb < blocks; kb += AT_ONCE) {
