@@ -249,6 +249,7 @@ listed_exact_kernel(const ExactArgs<F> w)
 		};
 		uint32_t noted = 0;                      /* wave-uniform */
 		[[maybe_unused]] uint32_t kept = 0;      /* doubles: of those, evaluated before and kept */
+		constexpr bool INSIDE = KB <= (DOUBLES ? 2 : 4); /* full lists are evaluated where they are found full */
 		/* a list that is full: 16 pairs at a time (their rows and the tile's centroids are in the caches), or, rows of one block, a pair per lane */
 		auto evaluate_here = [&]() {
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -354,9 +355,11 @@ listed_exact_kernel(const ExactArgs<F> w)
 				if (mask == 0) break;
 				const uint32_t more = (uint32_t)__popcll(mask);
 				if (noted + more > EXACT_HITS) {
-					/* (evaluated here it takes registers from the loops over tiles and groups, which rows of one block have to spare; taking those
-					 * loops up again costs them 7 %: N = 1M, d = 16, k = 1024, coordinates of 0 and 1: 249 against 233 us) */
-					if constexpr (KB == 1) evaluate_here();
+					/* (evaluated here it takes registers from the loops over tiles and groups, which narrow rows have to spare; being able to take
+					 * those loops up again costs them more: N = 1M, d = 16, k = 1024, coordinates of 0 and 1: 249 against 233 us a call; N = 2M,
+					 * d = 32, k = 1024: this kernel 64 against 60; N = 1M, d = 64, k = 512, small whole numbers: 1.6 % of a call. Doubles of 3 and 4
+					 * blocks would spill 72 registers instead of 31) */
+					if constexpr (INSIDE) evaluate_here();
 					else return false;
 				}
 				if (passed) {
