@@ -249,7 +249,7 @@ listed_exact_kernel(const ExactArgs<F> w)
 		};
 		uint32_t noted = 0;                      /* wave-uniform */
 		[[maybe_unused]] uint32_t kept = 0;      /* doubles: of those, evaluated before and kept */
-		constexpr bool INSIDE = KB <= (DOUBLES ? 2 : 4); /* full lists are evaluated where they are found full */
+		constexpr bool INSIDE = KB >= 1 && KB <= (DOUBLES ? 2 : 4); /* full lists are evaluated where they are found full */
 		/* a list that is full: 16 pairs at a time (their rows and the tile's centroids are in the caches), or, rows of one block, a pair per lane */
 		auto evaluate_here = [&]() {
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
