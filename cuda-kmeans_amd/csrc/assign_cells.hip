@@ -72,7 +72,7 @@ __device__ __forceinline__ void cell_distances(const float (&c)[D], const float 
  * One work-group per first-level cell. All of them find the box of the centroids (they have to read them anyway), then three levels of
  * lists, each filtered from the one above: the work-group's, one per wavefront, one per cell. On the way a wavefront packs a row for
  * the exact pass and the packed sweep (as a kernel of its own ahead of this one that took 5 to 7 us and a launch).
- * What bounds it: the latency of its dozen barriers and of the pass over all centroids (12 us at k = 4096, d = 4; one level
+ * What bounds it: the box distances (the vector ALU is busy three quarters of the 42 to 46 us at k = 4096, d = 4), then its dozen barriers (one level
  * of lists, every cell from all centroids, would be 65536 x k boxes, a millisecond).
  */
 template <int D, int LM>
@@ -411,8 +411,9 @@ constexpr uint32_t CELL_LIST = 64; /* points per wavefront that wait for the lis
 constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* LDS of assign_cells_kernel beside the centroids */
 
 /*
- * A lane per point, the centroids in LDS. What bounds it: the gathers, 16 bytes of centroid per comparison from LDS and 16 bytes of list per
- * eight of them from the caches, and the longest list among a wavefront's points. Two work-groups share a compute unit, eight wavefronts
+ * A lane per point, the centroids in LDS. What bounds it: the vector ALU, which takes a wavefront through the longest list of its 64 points (N = 4M,
+ * d = 4, k = 4096, uniform points: 77 M vector instructions fill the issue slots of the 104 to 114 us; lists of 29 entries on average, the longest
+ * of a wavefront 70, so more than half of the lanes idle). Two work-groups share a compute unit, eight wavefronts
  * a SIMD: with more than 80 scalar registers (and the 16 the hardware adds) only seven fit, which is one work-group (d = 3, k = 4096,
  * normal points: 162 -> 220 us).
  */

@@ -100,7 +100,7 @@ __device__ __forceinline__ unsigned long long exact_key(float sum, uint32_t c)
  *      the point's two smallest keys (distance bits << 32 | centroid, see evaluate_pair) in LDS.
  * F: the type of the serial arithmetic; doubles are ranked by float copies.
  * A wavefront whose list fills up (ties, duplicated centroids, data that the thresholds tell nothing about) evaluates it on the spot, 16
- * pairs at a time (N = 262144, d = 256, k = 1024, 32 copies each of 32 centroids: 1.15 ms a call, with a lane per pair 6.85).
+ * pairs at a time (N = 262144, d = 256, k = 1024, 32 copies each of 32 centroids: 1.00 ms a call, with a lane per pair 6.85).
  *
  * counters[0] receives the number of points whose two smallest serial distances are closer than the three-product certificate.
  */

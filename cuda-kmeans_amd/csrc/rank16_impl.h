@@ -50,7 +50,7 @@ template <int KB> constexpr uint32_t rank16_static_bytes() { return (2 * RANK16_
  * times larger before it overflows (which would certify nothing any more), and what half precision loses below its smallest normal
  * number, 2^-25 at most, is a 256th of the rounding of a coordinate as large as far. Less than 2^-12 of `size` is taken for that: a
  * sample of equal rows differs from their mean by its roundings only. (With far in [16, 32) from the first 16 centroids a quiet start of
- * 5e-3 before centroids of 20 overflowed: N = 1M, d = 32, k = 512 in 29 ms; now 0.36.)
+ * 5e-3 before centroids of 20 overflowed: N = 1M, d = 32, k = 512 in 29 ms; now 0.31.)
  */
 __device__ __forceinline__ float rank16_scale(float far, float size)
 {

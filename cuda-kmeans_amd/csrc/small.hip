@@ -45,7 +45,8 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  * (192 ALU cycles against 128 of the LDS that four SIMDs share) the vector ALU sets the pace, T = 1 (48 against 64) is for a
  * dozen centroids at most, which would leave most of the larger tile empty. (A lane per point with the centroids broadcast is
  * bound by the LDS; with the centroids as scalar operands every scalar load waits for all earlier ones: N = 2588, d = 60, k = 1288
- * 135 us.) The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
+ * 135 us.) A few dozen centroids leave most of the time to the trips to memory and the barriers in front of that (N = 65536, d = 8, k = 64: 3 us
+ * of vector instructions in 14 us). The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
  * ascending dimension, every operation rounded separately. Global loads are issued in batches of eight per lane: one after the
  * other they cost a microsecond each.
  *

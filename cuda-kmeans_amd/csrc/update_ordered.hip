@@ -257,8 +257,9 @@ ordered_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __
  * The same for clusters of many members: a work-group per cluster and block of up to 32 coordinates. All eight wavefronts fetch the
  * members' pieces (16 bytes each, STAGED_PIECES per lane) of the next few hundred rows into registers while the first one adds
  * the last fetch from LDS, a lane per coordinate, four members per LDS read. The chain then runs at the latency of an addition and an LDS read
- * instead of a trip to memory per 32 rows; what bounds it is that chain for the largest cluster, or the gathering of the rows
- * (N = 2M, d = 32, k = 1024: 389 -> 125 us, 2.1 TB/s; N = 4M, d = 16, k = 16, all of it 33 -> 7.5 ms).
+ * instead of a trip to memory per 32 rows. What bounds it: with clusters far larger than a fetch that chain (N = 4M, d = 16, k = 16, all of
+ * it 33 -> 7.5 ms); with clusters of a few fetches the trips to memory, which nothing hides then (N = 2M, d = 32, k = 1024: 389 -> 125 us, 2.1 TB/s;
+ * 2048 work-groups, two per compute unit and so four rounds, of two fetches each: 36 cycles per addition, with 16 of 512 lanes adding).
  * ELEMENTS: SoA points, rows shorter than a piece: single coordinates, consecutive lanes take consecutive members.
  */
 constexpr uint32_t STAGED_THREADS = 512, STAGED_PIECES = 8;

@@ -344,8 +344,10 @@ int kmx_set_queued_rows_limit(size_t bytes);
 /*
  * Where KMX_ASSIGN_MFMA_BF16X3 takes one product per dimension for all points (no counterpart in the reference): one
  * product in half precision is a third of the matrix work of the three bf16 products and leaves more points to the exact pass
- * behind it. The results are the same at every setting. mode 0: three products for all points always; 1
- * (default): one product where it pays (by size, see rank16_pays in csrc/assign_bf16.hip); 2: wherever the kernels allow it
+ * behind it. Rows of 2 to 4 dimensions are compared with the centroids listed for their cell of a grid instead of all. The results are
+ * the same at every setting. mode 0: three products for all points (all pairs at 2 to 4 dimensions) always; 1 (default): one product, or
+ * the cells, where they pay (by size, see rank16_pays and takes_cells in csrc/assign_bf16.hip); the cells look at a sample of the points
+ * first and leave points that a regular grid is no good for to the sweep; 2: wherever the kernels allow it, the cells whatever the points
  * (for tests and measurements on small inputs).
  */
 int kmx_set_two_level_sweep(int mode);

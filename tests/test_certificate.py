@@ -182,7 +182,7 @@ def test_tau_covers_the_split_and_the_serial_margin(km, dim, packed, kind):
 @pytest.mark.parametrize("dim", [17, 20, 32])
 @pytest.mark.parametrize("kind", ["adversarial", "pairs", "ties0", "ties100", "ties10000"])
 def test_tau_of_the_first_level_covers_one_product_per_dimension(km, dim, kind):
-    """The first level of the two-level sweep keeps hi * hi only: a1[j] = |c_j|^2 + sum_i c'hi_i xhi_i. Its tau (form 4, with
+    """A sweep of one product keeps hi * hi only: a1[j] = |c_j|^2 + sum_i c'hi_i xhi_i. Its tau (form 4, here with bf16 parts, with
     sum_i (x_i - xhi_i)^2 of the point) must cover twice what that drops plus the accumulation allowance of d products
     plus the serial margin, and every pair it would certify must be a strict win of the serial comparison."""
     rng = np.random.default_rng(dim * 17)

@@ -1,7 +1,7 @@
-"""The two-level split-bf16 sweep (rows of 17 to 32 and of 129 to 256 dimensions): one product per dimension for all points, three for those the
-first level cannot settle, the exact pass for the rest. By default it runs from 2^18 points on; here it is forced
-(kmx_set_two_level_sweep(2)) so that the inputs aimed at the certificates and the hard inputs of the other modules, which are
-smaller, pass through both levels. Every result must be the serial scan's index, as with one level."""
+"""The half-precision sweep (rows of 17 to 32 and of 129 to 256 dimensions here): one product per dimension for all points, its exact pass for those
+the certificate cannot settle. By default it runs where it pays; here it is forced (kmx_set_two_level_sweep(2)) so that the inputs
+aimed at the certificates and the hard inputs of the other modules, which are smaller, pass through it. Every result must be the
+serial scan's index, as with three bf16 products."""
 import numpy as np
 import pytest
 
@@ -40,8 +40,8 @@ def test_assignment_is_bit_exact(km, orc, gpu, two_levels, dim, k, n, layout, la
 
 
 def test_both_settings_return_the_same_and_the_first_level_settles_most_points(km, orc, gpu):
-    """Configuration 2 (its first 2^18 points): the same assignment with one level and with two; the exact pass sees the
-    same order of magnitude of points either way (what the second level cannot settle is what one level could not)."""
+    """Configuration 2 (its first 2^18 points): the same assignment with three products (mode 0) and with one. What the call counts as
+    re-evaluated are the points that three products could not settle either, so the counts are of the same order."""
     spec = km.baseline_config(2)
     n, dim, k = 1 << 18, spec.dim, spec.k
     data, means0 = km.generate_points(spec, n), km.first_k_means(spec)

@@ -1,5 +1,6 @@
-"""Rows of more than 256 dimensions (csrc/assign_wide.hip) against the serial oracle, bit for bit: both levels, both unit sizes,
-one and several groups of centroids, rows kept in LDS and rows staged again, ragged ends everywhere (-m gpu)."""
+"""Rows of more than 256 dimensions (csrc/assign_wide.hip) against the serial oracle, bit for bit: one half-precision product and
+three bf16 products, both unit sizes, one and several groups of centroids, rows kept in LDS and rows staged again, ragged ends
+everywhere (-m gpu)."""
 import numpy as np
 import pytest
 
@@ -12,10 +13,10 @@ def flat(rows, layout):
 
 @pytest.mark.parametrize("kind", ["clustered", "grid", "offset"])
 @pytest.mark.parametrize("dim,k,n", [
-    (257, 1, 1), (300, 5, 31), (320, 33, 130), (511, 400, 700), (257, 290, 1500),   # units of 32 points, one level
-    (384, 520, 16500), (512, 545, 16384), (515, 100, 16421),                         # two levels; groups of 512; resident rows
+    (257, 1, 1), (300, 5, 31), (320, 33, 130), (511, 400, 700), (257, 290, 1500),   # units of 32 points
+    (384, 520, 16500), (512, 545, 16384), (515, 100, 16421),                         # units of 128; groups of 512; resident rows
     (1030, 600, 16400), (2560, 40, 300),                                             # rows staged again per group; the widest
-    (300, 40, 33000),                                                                # units of 128 points, one level (two tiles)
+    (300, 40, 33000),                                                                # units of 128 points, two tiles
 ])
 def test_wide_rows_match_the_oracle(km, orc, gpu, dim, k, n, kind):
     rng = np.random.default_rng(dim * 31 + k)
@@ -40,7 +41,7 @@ def test_wide_rows_match_the_oracle(km, orc, gpu, dim, k, n, kind):
             padded = rows
         d = km.DeviceBuffer(padded.nbytes); d.write(flat(padded, layout))
         m = km.DeviceBuffer(4 * k * dim); m.write(flat(means, layout_means))
-        for mode in (1, 2):  # two levels where they pay, two levels always
+        for mode in (0, 1, 2):  # three bf16 products; one half-precision product (rows of up to 2304 dimensions), the same
             km.set_two_level_sweep(mode)
             try:
                 a.write(np.full(n, 0xFFFFFFF1, np.uint32))
