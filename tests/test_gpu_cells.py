@@ -101,6 +101,31 @@ def test_points_the_cells_are_no_good_for_match_the_oracle(km, orc, gpu, dim, k,
     assert np.array_equal(got[sample], want), "%d of %d differ" % (int((got[sample] != want).sum()), len(sample))
 
 
+@pytest.mark.parametrize("budget,limit", [(0, 1 << 20), (46 * 1024, 0), (64 * 1024, 1 << 20), (100 * 1024, 0)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_the_way_back_keeps_to_the_limits_of_the_caller(km, orc, gpu, budget, limit, layout):
+    """Little LDS (centroids streamed behind the cells, or no cells at all) and a small block for copied rows."""
+    dim, k, n = 4, 1500, (1 << 18) + 5
+    rng = np.random.default_rng(budget + layout)
+    means, rows = rng.normal(size=(k, dim)).astype(np.float32), rng.normal(size=(n, dim)).astype(np.float32)
+    means[:, 3] = 0; rows[:, 3] = 0
+    d, m, a = km.DeviceBuffer(rows.nbytes), km.DeviceBuffer(means.nbytes), km.DeviceBuffer(4 * n)
+    d.write(flat(rows, layout)); m.write(flat(means, 0)); a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+    if limit:
+        km.set_queued_rows_limit(limit)
+    try:
+        km.assign(km.ASSIGN_BEST, d, layout, dim if layout == 0 else n, m, 0, dim, a, dim, k, n, km.ExecParams(shared_mem_bytes=budget))
+        km.sync()
+    finally:
+        km.set_queued_rows_limit(1 << 30)
+    got = a.read(np.uint32, n)
+    for b in (d, m, a):
+        b.free()
+    sample = rng.choice(n, 30000, replace=False)
+    want = orc.assign(np.ascontiguousarray(rows[sample]).ravel(), means.ravel(), dim, k, len(sample), threads=0, fast=True)
+    assert np.array_equal(got[sample], want), "%d of %d differ" % (int((got[sample] != want).sum()), len(sample))
+
+
 @pytest.mark.parametrize("kind", ["inside", "outside"])
 def test_recorded_cells_replay(km, orc, gpu, kind):
     """Recorded right after a reservation, replayed with eager calls of another shape in between: the choice between cells and sweep is
