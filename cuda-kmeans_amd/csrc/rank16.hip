@@ -134,8 +134,7 @@ bool rank16_supports(const AssignArgs& a, uint32_t lds_budget)
 {
 	const uint32_t kb = rank16_kb(a.dim);
 	if (a.dim <= 4 || kb == 0 || a.k >= (1u << 25) || a.n > (1u << 31)) return false;
-	const uint32_t sweep = (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + kb * KBLOCK) * 4 + 64 + 2 * (kb * WAVE * 4 + NORM_TILE) * 4; /* two tiles */
-	return sweep <= lds_budget && exact_dynamic_bytes(kb, EXACT_GROUPS) + exact_static_bytes(a.points64 != nullptr) <= lds_budget;
+	return rank16_least_bytes(kb, a.layout) <= lds_budget && exact_dynamic_bytes(kb, EXACT_GROUPS) + exact_static_bytes(a.points64 != nullptr) <= lds_budget;
 }
 
 /* the centroids for launch_rank16_sweep */

@@ -13,10 +13,18 @@ namespace kmx {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-constexpr uint32_t RANK16_WAVES = 8;
-constexpr uint32_t RANK16_THREADS = RANK16_WAVES * WAVE;
+/*
+ * Wavefronts of a work-group: eight around centroids in LDS. Where the centroids stream by (slots of a chunk of tiles that go round, filled by
+ * requests straight to LDS, a barrier per chunk), rows of up to 128 dimensions keep that form with two chunks as large as fit, since the
+ * barriers are what costs (us per assignment, two work-groups of four wavefronts with four slots of 32 matrix instructions -> this: N = 2M,
+ * d = 128, k = 1024 659 -> 627; N = 1M, d = 96, k = 2000 493 -> 440; d = 64, k = 3000 473 -> 424). Wider rows have a barrier's worth of matrix
+ * instructions in a single tile: two work-groups of four wavefronts on a compute unit, one of which reads its points while the other has
+ * the matrix cores, and four slots of a tile (N = 1M, d = 256, k = 1024: 549, with eight wavefronts and two chunks of four tiles 569).
+ * With chunks through registers and eight wavefronts for all widths: 656, 655, 480, 464.
+ */
+constexpr uint32_t rank16_waves(uint32_t kb, bool stream) { return stream && kb >= 12 ? 4 : 8; }
 constexpr int RANK16_P = 2; /* point tiles per wavefront: an operand read serves two instructions */
-constexpr uint32_t RANK16_LIST = 128;
+constexpr uint32_t RANK16_LIST = 120;
 
 struct Rank16Args {
 	const float* data; size_t stride;
@@ -42,7 +50,15 @@ inline size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) 
 
 /* 16 tile bytes per block of 16 dimensions and lane, then the tile's norms */
 template <int KB> constexpr uint32_t rank16_tile_floats() { return KB * WAVE * 4; }
-template <int KB> constexpr uint32_t rank16_static_bytes() { return (2 * RANK16_LIST * RANK16_WAVES + 4 * RANK16_WAVES + KB * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_slots(uint32_t kb) { return kb >= 12 ? 4 : 2; }
+__host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { return (tiles * NORM_TILE + WAVE - 1) / WAVE; }
+/* what a chunk takes in LDS, its norms behind its operands as whole requests of 64 words */
+__host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t tiles) { return tiles * kb * WAVE * 16 + rank16_norm_blocks(tiles) * WAVE * 4; }
+constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
+constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
+constexpr uint32_t rank16_exchange(uint32_t kb, int layout) { return rank16_shared_rows(kb, layout) || layout == KMX_SOA ? RANK16_EXCHANGE : 0; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream) { return ((2 * RANK16_LIST + rank16_exchange(kb, layout) + 4) * rank16_waves(kb, stream) + kb * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
  * S for centroids whose coordinates are up to `far` from the frame and up to `size` from the origin, both of a sample: the power of two
@@ -82,72 +98,194 @@ __device__ __forceinline__ void rank16_leave_bounds(float* scale, uint32_t c2max
 	if (threadIdx.x == 0) { scale[2] = __uint_as_float(c2max); scale[3] = __uint_as_float(mid); scale[4] = __uint_as_float(rest); scale[5] = __uint_as_float(low2max); }
 }
 
-/* the 8 coordinates of a half-wave of block kb as they come from memory, zeros beyond the row. Blocks inside the row (the same
- * for all lanes) are loaded without guards. */
-template <int LD>
-__device__ __forceinline__ void rank16_request(float (&v)[8], const float* __restrict__ data, size_t stride, uint32_t pt, uint32_t kb, uint32_t h, uint32_t dim)
+/*
+ * How the coordinates come from memory. AoS: four lanes take 64 consecutive bytes of a row, lane 4 r + q the piece q (four coordinates) of
+ * rows r and 16 + r of the tile, and the rounded values go through LDS to the lanes that hold them as operands: a lane per row would make
+ * every 16 bytes an access of their own to the vector cache, 64 a load instead of 16 (N = 1M, d = 256, k = 1024: 104 M accesses a launch,
+ * the cache busy for half of it). SoA: lane (col, h) takes eight coordinates of point col, which are its operand.
+ * Without branches, so that many blocks travel together: blocks that the row does not fill (ragged rows only) read what lies inside it, and
+ * rank16_place puts that into its places. WHOLE: no such blocks.
+ */
+struct Rank16Source { const float* row[2]; }; /* AoS: the lane's two rows; SoA: row[0], the lane's point at coordinate 0 */
+
+template <int LD, bool SHARED>
+__device__ __forceinline__ Rank16Source rank16_source(const float* __restrict__ data, size_t stride, uint32_t tile_first, uint32_t n, uint32_t lane)
+{
+	if (!SHARED) return Rank16Source{ { data + (size_t)min(tile_first + lane % TILE, n - 1) * (LD == KMX_AOS ? stride : 1), nullptr } }; /* rows beyond the points repeat the last one */
+	return Rank16Source{ { data + (size_t)min(tile_first + lane / 4, n - 1) * stride, data + (size_t)min(tile_first + 16 + lane / 4, n - 1) * stride } };
+}
+
+template <int LD, bool SHARED, bool WHOLE>
+__device__ __forceinline__ void rank16_request(float (&v)[8], const Rank16Source& from, size_t stride, uint32_t kb, uint32_t lane, uint32_t dim)
 {
 	typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-	const uint32_t d0 = kb * KBLOCK + h * 8;
 	if (LD == KMX_AOS) {
-		const float* src = data + (size_t)pt * stride + d0;
-		if ((kb + 1) * KBLOCK <= dim) {
-			const f32x4 lo = *(const f32x4_any*)src, up = *(const f32x4_any*)(src + 4);
-			v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = up.x; v[5] = up.y; v[6] = up.z; v[7] = up.w;
+		const uint32_t d = kb * KBLOCK + (SHARED ? lane % 4 * 4 : lane / TILE * 8), at = WHOLE ? d : min(d, dim - 4), at2 = SHARED ? at : WHOLE ? d + 4 : min(d + 4, dim - 4);
+		const f32x4 lo = *(const f32x4_any*)(from.row[0] + at), up = *(const f32x4_any*)(from.row[SHARED] + at2);
+		v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = up.x; v[5] = up.y; v[6] = up.z; v[7] = up.w;
+	}
+	else {
+		asm volatile("" : "+v"(lane)); /* (addresses are formed here: 64 of them kept for the next tile of points would be spilled) */
+		const uint32_t d0 = kb * KBLOCK + lane / TILE * 8;
+		const float* src = from.row[0] + (size_t)(WHOLE ? d0 : min(d0, dim - 1)) * stride;
+#pragma unroll
+		for (uint32_t j = 0; j < 8; ++j) {
+			v[j] = *src;
+			src += WHOLE || d0 + j + 1 < dim ? stride : 0;
 		}
-		else {
-			load_piece_any(v, src, true, d0, dim);
-			load_piece_any(v + 4, src + 4, true, d0 + 4, dim);
+	}
+}
+
+/* ragged rows: zeros behind the row (AoS: rows of at least 4 coordinates, pieces that end behind the row have been read up to its end) */
+template <int LD, bool SHARED>
+__device__ __forceinline__ void rank16_place(float (&v)[8], uint32_t kb, uint32_t lane, uint32_t dim)
+{
+	if ((kb + 1) * KBLOCK <= dim) return; /* (the same for all lanes) */
+	if (LD == KMX_AOS) {
+#pragma unroll
+		for (uint32_t q = 0; q < 8; q += 4) {
+			const uint32_t beyond = max(kb * KBLOCK + (SHARED ? lane % 4 * 4 : lane / TILE * 8 + q) + 4, dim) - dim; /* coordinates of the piece behind the row */
+			const float x = v[q], y = v[q + 1], z = v[q + 2], t = v[q + 3];
+			v[q] = beyond == 0 ? x : beyond == 1 ? y : beyond == 2 ? z : beyond == 3 ? t : 0.0f;
+			v[q + 1] = beyond == 0 ? y : beyond == 1 ? z : beyond == 2 ? t : 0.0f;
+			v[q + 2] = beyond == 0 ? z : beyond == 1 ? t : 0.0f;
+			v[q + 3] = beyond == 0 ? t : 0.0f;
 		}
 	}
 	else {
-		const float* src = data + (size_t)d0 * stride + pt;
-		if ((kb + 1) * KBLOCK <= dim) {
+		const uint32_t d0 = kb * KBLOCK + lane / TILE * 8;
 #pragma unroll
-			for (int j = 0; j < 8; ++j) { v[j] = *src; src += stride; }
-		}
-		else {
-#pragma unroll
-			for (int j = 0; j < 8; ++j) { v[j] = d0 + j < dim ? *src : 0.0f; src += stride; }
-		}
+		for (uint32_t j = 0; j < 8; ++j) v[j] = d0 + j < dim ? v[j] : 0.0f;
 	}
+}
+
+__device__ __forceinline__ void rank16_exchanged() /* LDS keeps the order of a wavefront's requests; the compiler has to as well */
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
 }
 
 /*
  * SoA: the rows go out as AoS on the way, for the exact pass and whatever else reads single rows (coordinates of a listed point lie a
  * cache line each apart; with 9 % of N = 2M, d = 128 listed, gathering them read all data again, 430 us, and was no cheaper right
- * behind the sweep of the point, 360 us. The stores travel behind the matrix instructions).
+ * behind the sweep of the point, 360 us. The stores travel behind the matrix instructions). Through LDS, so that four lanes store 64
+ * consecutive bytes of a row. `exchange`: RANK16_EXCHANGE words of this wavefront's.
  */
-template <int LD>
-__device__ __forceinline__ void rank16_copy(const Rank16Args& w, const float (&v)[8], uint32_t pt, uint32_t d0)
+__device__ __forceinline__ void rank16_copy(const Rank16Args& w, const float (&v)[8], uint32_t tile_first, uint32_t kb, uint32_t lane, float* exchange)
 {
-	if (LD == KMX_AOS || pt >= w.n || d0 >= w.copy_stride) return;
-	float* dst = w.copies + (size_t)pt * w.copy_stride + d0;
-	*(f32x4*)dst = f32x4{ v[0], v[1], v[2], v[3] };
-	*(f32x4*)(dst + 4) = f32x4{ v[4], v[5], v[6], v[7] };
-}
-
-/* v = S (x - m) rounded once (S is a power of two), its half-precision part, and the shares of |v|^2 and of the squared norm of the rest */
-__device__ __forceinline__ void rank16_convert(f16x8& b, const float (&raw)[8], const float* frame, float scale, float& part, float& low)
-{
-	const f32x4 m0 = *(const f32x4*)frame, m1 = *(const f32x4*)(frame + 4); /* S m */
-	const float m[8] = { m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w };
+	/* half of the tile at a time, 16 words a row in pieces of four; row r's piece q lies in the place q ^ (r / 2 % 4) of the row, which spreads a
+	 * column over the banks */
+	const uint32_t col = lane % TILE, h = lane / TILE, turn = col / 2 % 4, row = lane / 4, d = kb * KBLOCK + lane % 4 * 4;
 #pragma unroll
-	for (int j = 0; j < 8; ++j) {
-		const float v = __builtin_fmaf(raw[j], scale, -m[j]);
-		part = __builtin_fmaf(v, v, part);
-		const _Float16 h = (_Float16)v;
-		const float r = v - (float)h;
-		low = __builtin_fmaf(r, r, low);
-		b[j] = h;
+	for (uint32_t half = 0; half < 2; ++half) {
+		rank16_exchanged();
+		if (col / 16 == half) {
+			float* to = exchange + col % 16 * 16;
+			*(f32x4*)(to + ((2 * h) ^ turn) * 4) = f32x4{ v[0], v[1], v[2], v[3] };
+			*(f32x4*)(to + ((2 * h + 1) ^ turn) * 4) = f32x4{ v[4], v[5], v[6], v[7] };
+		}
+		rank16_exchanged();
+		const f32x4 piece = *(const f32x4*)(exchange + row * 16 + ((lane % 4) ^ (row / 2 % 4)) * 4);
+		const uint32_t pt = tile_first + half * 16 + row;
+		if (pt < w.n && d < w.copy_stride) *(f32x4*)(w.copies + (size_t)pt * w.copy_stride + d) = piece;
 	}
 }
 
+/* four coordinates v = S (x - m) rounded once (S is a power of two), in half precision, and their shares of |v|^2 and of the squared norm of
+ * what half precision leaves out; m: S times the frame */
+__device__ __forceinline__ void rank16_round(f16x2 (&out)[2], const float* raw, const f32x4& m, float scale, float& part, float& low)
+{
+	float minus_one = -1.0f;
+	asm("" : "+s"(minus_one));
+#pragma unroll
+	for (int j = 0; j < 4; j += 2) {
+		const float v0 = __builtin_fmaf(raw[j], scale, -m[j]), v1 = __builtin_fmaf(raw[j + 1], scale, -m[j + 1]);
+		f16x2 pair = { (_Float16)v0, (_Float16)v1 };
+		asm("" : "+v"(pair)); /* (the halves are read from the pair from here on: left alone the compiler rounds again for each use) */
+		const float r0 = __builtin_fmaf((float)pair.x, minus_one, v0), r1 = __builtin_fmaf((float)pair.y, minus_one, v1); /* (one instruction each) */
+		part = __builtin_fmaf(v0, v0, part);
+		part = __builtin_fmaf(v1, v1, part);
+		low = __builtin_fmaf(r0, r0, low);
+		low = __builtin_fmaf(r1, r1, low);
+		out[j / 2] = pair;
+	}
+}
+
+/* what a lane sums up while it converts: AoS: of its two rows; SoA: of its eight coordinates of each block (the second entry stays zero) */
+struct Rank16Sums { float part[2], low[2]; };
+
+/* block kb of a tile of points as this lane's operand; frame: S m, in LDS */
+template <bool SHARED>
+__device__ __forceinline__ void rank16_convert(f16x8& b, const float (&raw)[8], const float* frame, float scale, uint32_t kb, uint32_t lane, Rank16Sums& sums, float* exchange)
+{
+	union { f16x8 all; f16x2 two[4]; } h;
+	if (SHARED) {
+		const f32x4 m = *(const f32x4*)(frame + kb * KBLOCK + lane % 4 * 4);
+		f16x2* to = (f16x2*)exchange + 2 * lane;
+		rank16_exchanged();
+#pragma unroll
+		for (int half = 0; half < 2; ++half) {
+			union { f16x2 two[2]; uint2 all; } piece;
+			rank16_round(piece.two, raw + 4 * half, m, scale, sums.part[half], sums.low[half]);
+			*(uint2*)(to + 2 * WAVE * half) = piece.all; /* row 16 half + lane / 4, 32 bytes a row */
+		}
+		rank16_exchanged();
+		b = *(const f16x8*)((const f16x2*)exchange + lane % TILE * 8 + lane / TILE * 4);
+	}
+	else {
+#pragma unroll
+		for (int half = 0; half < 2; ++half) {
+			f16x2 two[2];
+			rank16_round(two, raw + 4 * half, *(const f32x4*)(frame + kb * KBLOCK + lane / TILE * 8 + 4 * half), scale, sums.part[0], sums.low[0]);
+			h.two[2 * half] = two[0]; h.two[2 * half + 1] = two[1];
+		}
+		b = h.all;
+	}
+}
+
+/* SHARED: the sums of point lane % 32 of the tile, from the lanes that share its row; otherwise the two half-waves have a part each, which
+ * rank16_whole adds up (at the end of a sweep, where nothing waits for it) */
+template <bool SHARED>
+__device__ __forceinline__ void rank16_total(float& x2, float& low2, const Rank16Sums& sums, uint32_t lane)
+{
+	if (!SHARED) { x2 = sums.part[0]; low2 = sums.low[0]; return; }
+	float all[2];
+#pragma unroll
+	for (int q = 0; q < 2; ++q) {
+		float a = q ? sums.low[0] : sums.part[0], c = q ? sums.low[1] : sums.part[1];
+		a += __shfl_xor(a, 1); c += __shfl_xor(c, 1);
+		a += __shfl_xor(a, 2); c += __shfl_xor(c, 2);
+		const float first = __shfl(a, (int)(lane % 16 * 4)), second = __shfl(c, (int)(lane % 16 * 4));
+		all[q] = lane % TILE < 16 ? first : second;
+	}
+	x2 = all[0]; low2 = all[1];
+}
+template <bool SHARED> __device__ __forceinline__ float rank16_whole(float sum) { return SHARED ? sum : sum + __shfl_xor(sum, 32); }
+
+__device__ __forceinline__ uint32_t rank16_uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ const void* rank16_uniform(const void* p)
+{
+	const uint64_t v = (uint64_t)p;
+	return (const void*)((uint64_t)rank16_uniform((uint32_t)(v >> 32)) << 32 | rank16_uniform((uint32_t)v));
+}
+__device__ __forceinline__ void stage_block(const void* from, uint32_t lane, uint32_t to)
+{
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(rank16_uniform(to)), "v"(lane * 16), "s"(rank16_uniform(from)) : "m0");
+}
+__device__ __forceinline__ void stage_words(const void* from, uint32_t lane, uint32_t to)
+{
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(rank16_uniform(to)), "v"(lane * 4), "s"(rank16_uniform(from)) : "m0");
+}
+/* all but the last LATER requests of this wavefront have arrived (requests of other kinds among them make it wait longer, never shorter) */
+template <uint32_t LATER> __device__ __forceinline__ void staged_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LATER) : "memory"); }
+
 /*
- * A work-group of eight wavefronts around centroids in LDS: all of them (STREAM = false), or two buffers of chunk_tiles tiles that
- * go round (a barrier per chunk, all wavefronts sweep together). A wavefront sweeps 64 points at a time. With resident centroids the
- * wavefronts take items of 64 points from a counter in LDS (a SIMD serves its older wavefront first: equal shares leave the
- * younger ones sweeping alone at the end).
+ * A work-group around centroids in LDS: all of them (STREAM = false), or slots that go round (rank16_waves), all its wavefronts sweeping
+ * together. A wavefront sweeps 64 points at a time. With resident centroids the wavefronts take items of 64 points from a counter in
+ * LDS (a SIMD serves its older wavefront first: equal shares leave the younger ones sweeping alone at the end).
+ *
+ * What bounds the sweep of wide rows (N = 1M, d = 256, k = 1024: 505 us, 1.09 PFLOP/s): the power the matrix cores may take -- at 58 % of their
+ * cycles the clock has come down to 1.73 GHz, without the points' fetches they reach 76 % at 1.51 -- and the fetches and conversions themselves.
  *
  * Tracking is the snapshot of assign_bf16_impl.h: the minimum of a lane's 16 results per tile, the two smallest minima, and the 16
  * results of the leading tile, from which the winner and the runner-up inside that tile come at the end.
@@ -155,30 +293,32 @@ __device__ __forceinline__ void rank16_convert(f16x8& b, const float (&raw)[8], 
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
 template <int KB, int LD, bool STREAM>
-__global__ void __launch_bounds__(RANK16_THREADS)
+__global__ void __launch_bounds__(rank16_waves(KB, STREAM) * WAVE, 2)
 rank16_kernel(const Rank16Args w)
 {
+	constexpr uint32_t WAVES = rank16_waves(KB, STREAM), THREADS = WAVES * WAVE;
 	constexpr int P = RANK16_P;
 	constexpr uint32_t TF = rank16_tile_floats<KB>();
 	constexpr bool PIPE = !STREAM && KB <= 4;
-	constexpr bool SNAP = KB < 12;          /* wider rows: their operands leave no registers for the snapshot, their instructions hide row-by-row tracking */
+	constexpr bool SHARED = rank16_shared_rows(KB, LD);
 	constexpr bool PREFETCH = PIPE && KB <= 2; /* the next item's coordinates travel while the current one is swept */
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
-	__shared__ uint32_t wave_max[4][RANK16_WAVES];
-	__shared__ uint32_t flag_list[RANK16_WAVES][2 * RANK16_LIST];
+	__shared__ uint32_t wave_max[4][WAVES];
+	__shared__ uint32_t flag_list[WAVES][2 * RANK16_LIST];
+	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD) ? RANK16_EXCHANGE : 1];
 	uint32_t& claimed = wave_max[3][0];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 	const uint32_t col = lane & 31, h = lane >> 5;
 	const float scale = w.scale[0], smallest = 1e-30f * (scale * scale), largest = 1e37f * (scale * scale);
 	if (tid == 0) claimed = 0u;
-	for (uint32_t i = tid; i < KB * KBLOCK; i += RANK16_THREADS) frame[i] = w.frame[i] * scale;
+	for (uint32_t i = tid; i < KB * KBLOCK; i += THREADS) frame[i] = w.frame[i] * scale;
 
 	CertCoeffs cert;
 	{
 		uint32_t most[2] = { 0u, 0u };
-		for (uint32_t j = tid; j < w.k; j += RANK16_THREADS) {
+		for (uint32_t j = tid; j < w.k; j += THREADS) {
 			most[0] = max(most[0], __float_as_uint(w.norms[norm_at(j)]));
 			most[1] = max(most[1], __float_as_uint(w.low2[j]));
 		}
@@ -191,7 +331,7 @@ rank16_kernel(const Rank16Args w)
 #pragma unroll
 		for (int q = 0; q < 2; ++q) {
 			most[q] = 0;
-			for (uint32_t v = 0; v < RANK16_WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
+			for (uint32_t v = 0; v < WAVES; ++v) most[q] = max(most[q], wave_max[q][v]);
 		}
 		if (blockIdx.x == 0) rank16_leave_bounds(w.scale, most[0], most[1], w.low2, w.k, w.kp);
 		cert = cert_coeffs_level1(CentroidBounds{ __uint_as_float(most[0]), __uint_as_float(most[1]), 0.0f });
@@ -201,17 +341,14 @@ rank16_kernel(const Rank16Args w)
 	}
 
 	const uint32_t all_tiles = w.kp / TILE;
-	const uint32_t buffer_floats = w.chunk_tiles * (TF + NORM_TILE); /* chunk_tiles tiles of operands, then their norms */
-	const uint32_t chunks = (all_tiles + w.chunk_tiles - 1) / w.chunk_tiles;
-	uint32_t cur = 0;
-	{
-		const uint32_t tiles = min(w.chunk_tiles, all_tiles);
+	if constexpr (!STREAM) {
+		const uint32_t tiles = all_tiles;
 		f32x4* dst = (f32x4*)lds;
 		const f32x4* src = (const f32x4*)w.packed;
-		for (uint32_t i = tid; i < tiles * (TF / 4); i += RANK16_THREADS) dst[i] = src[i];
+		for (uint32_t i = tid; i < tiles * (TF / 4); i += THREADS) dst[i] = src[i];
 		f32x4* ndst = (f32x4*)(lds + (size_t)w.chunk_tiles * TF);
 		const f32x4* nsrc = (const f32x4*)w.norms;
-		for (uint32_t i = tid; i < tiles * (NORM_TILE / 4); i += RANK16_THREADS) ndst[i] = nsrc[i];
+		for (uint32_t i = tid; i < tiles * (NORM_TILE / 4); i += THREADS) ndst[i] = nsrc[i];
 	}
 	__syncthreads();
 
@@ -232,40 +369,52 @@ rank16_kernel(const Rank16Args w)
 	auto operand = [&](const float* tiles, uint32_t tile, int kb) -> f16x8 { return ((const f16x8*)(tiles + (size_t)tile * TF))[kb * WAVE + lane]; };
 
 	f16x8 b[P][KB];
-	float xx[P], xl[P]; /* this half-wave's shares of |v|^2 and of the squared norm of the rest */
+	float xx[P], xl[P]; /* of this lane's point: |v|^2 and the squared norm of what half precision leaves out (rank16_whole) */
+	float* const exchange = exchanges[wave];
 	float m1[P], m2[P];
 	uint32_t leader[P];
-	float snap[P][SNAP ? SNAP_ROWS : 1];
+	float snap[P][SNAP_ROWS];
 
-	auto load_points = [&](uint32_t first) {
+	/* A block is converted while the next DEPTH ones are on their way. (Requesting the first of them while the unit before is swept was no gain:
+	 * N = 2M, d = 128, k = 1024: 653 against 618 us, d = 96 440 against 442.) */
+	constexpr int BLOCKS = P * KB, DEPTH = BLOCKS < 8 ? BLOCKS : 8;
+	auto load_points_of = [&](auto whole, uint32_t first, uint32_t dim) {
+		constexpr bool WHOLE = decltype(whole)::value;
+		float raw[DEPTH][8];
+		Rank16Source from[P];
+		Rank16Sums sums[P];
 #pragma unroll
-		for (int p = 0; p < P; ++p) { xx[p] = 0.0f; xl[p] = 0.0f; }
-		constexpr int GROUP = KB <= 2 ? KB : KB <= 12 ? 4 : 2; /* blocks whose coordinates are in registers at a time */
-		uint32_t dim = w.dim;
-		asm volatile("" : "+s"(dim)); /* (the comparisons with it are not kept from one item to the next: they are as many as scalar registers) */
-#pragma unroll
-		for (int g = 0; g < KB; g += GROUP) {
-#pragma unroll
-			for (int p = 0; p < P; ++p) {
-				float raw[GROUP][8];
-				const uint32_t pt = min(first + p * TILE + col, w.n - 1); /* rows beyond the points repeat the last one */
-#pragma unroll
-				for (int i = 0; i < GROUP; ++i)
-					if (g + i < KB) rank16_request<LD>(raw[i], w.data, w.stride, pt, g + i, h, dim);
-#pragma unroll
-				for (int i = 0; i < GROUP; ++i)
-					if (g + i < KB) {
-						rank16_copy<LD>(w, raw[i], first + p * TILE + col, (g + i) * KBLOCK + h * 8);
-						rank16_convert(b[p][g + i], raw[i], frame + (g + i) * KBLOCK + h * 8, scale, xx[p], xl[p]);
-						if constexpr (KB > 2) asm volatile("" : "+v"(b[p][g + i]));
-					}
-				if constexpr (KB > 2) {
-					/* the sums exist here: left alone the compiler moves them behind the sweep and keeps the coordinates alive */
-					asm volatile("" : "+v"(xx[p]), "+v"(xl[p]));
-					__builtin_amdgcn_sched_barrier(0);
-				}
-			}
+		for (int p = 0; p < P; ++p) {
+			from[p] = rank16_source<LD, SHARED>(w.data, w.stride, first + p * TILE, w.n, lane);
+			sums[p] = Rank16Sums{ { 0.0f, 0.0f }, { 0.0f, 0.0f } };
 		}
+		auto request = [&](int at) { rank16_request<LD, SHARED, WHOLE>(raw[at % DEPTH], from[at / KB], w.stride, at % KB, lane, dim); };
+#pragma unroll
+		for (int at = 0; at < DEPTH; ++at) request(at);
+#pragma unroll
+		for (int at = 0; at < BLOCKS; ++at) {
+			const int p = at / KB, kb = at % KB;
+			__builtin_amdgcn_sched_barrier(0);
+			float (&v)[8] = raw[at % DEPTH];
+			if (!WHOLE) rank16_place<LD, SHARED>(v, kb, lane, dim);
+			if (LD == KMX_SOA) rank16_copy(w, v, first + p * TILE, kb, lane, exchange);
+			rank16_convert<SHARED>(b[p][kb], v, frame, scale, kb, lane, sums[p], exchange);
+			if (!SHARED) asm volatile("" : "+v"(b[p][kb]));
+			/* the sums exist here: left alone the compiler moves them behind the sweep and keeps the coordinates alive */
+			asm volatile("" : "+v"(sums[p].part[0]), "+v"(sums[p].part[1]), "+v"(sums[p].low[0]), "+v"(sums[p].low[1]));
+			__builtin_amdgcn_sched_barrier(0);
+			if (at + DEPTH < BLOCKS) request(at + DEPTH);
+		}
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int p = 0; p < P; ++p) rank16_total<SHARED>(xx[p], xl[p], sums[p], lane);
+	};
+	auto load_points = [&](uint32_t first) {
+		uint32_t dim = w.dim;
+		asm volatile("" : "+v"(dim)); /* (the comparisons with it are not kept from one item to the next: they are as many as scalar registers) */
+		dim = (uint32_t)__builtin_amdgcn_readfirstlane((int)dim);
+		if (dim == KB * KBLOCK) load_points_of(std::true_type{}, first, dim);
+		else load_points_of(std::false_type{}, first, dim);
 	};
 
 	auto finish = [&](uint32_t first_pt) {
@@ -273,8 +422,6 @@ rank16_kernel(const Rank16Args w)
 		for (int p = 0; p < P; ++p) {
 			/* the two smallest of the leading tile's 16 results, the number of a result in its lowest four bits (cert_kd_keyed) */
 			float v1 = __builtin_inff(), v2 = __builtin_inff();
-			if constexpr (!SNAP) { v1 = m1[p]; v2 = m2[p]; }
-			else
 #pragma unroll
 			for (int r = 0; r < SNAP_ROWS; ++r) {
 				const float v = __uint_as_float((__float_as_uint(snap[p][r]) & ~15u) | (uint32_t)r);
@@ -290,9 +437,8 @@ rank16_kernel(const Rank16Args w)
 			const float others = win ? fminf(o1, m2[p]) : fminf(m1[p], o2); /* everything outside the leading 16 rows */
 			const uint32_t idx = win ? mine_idx : oi;
 			const float lowest = win ? v1 : ov1;
-			const float next = fminf(win ? v2 : ov2, others); /* (!SNAP: v2 is m2) */
-			const float x2 = xx[p] + __shfl_xor(xx[p], 32), low = xl[p] + __shfl_xor(xl[p], 32);
-			const float tau = cert_tau(w.kd, x2, low, cert);
+			const float next = fminf(win ? v2 : ov2, others);
+			const float x2 = rank16_whole<SHARED>(xx[p]), tau = cert_tau(w.kd, x2, rank16_whole<SHARED>(xl[p]), cert);
 			const uint32_t pt = first_pt + p * TILE + col;
 			const bool mine = h == 0 && pt < w.n;
 			/* squares of the data as given underflow or overflow: no ranking says anything about the serial sums */
@@ -319,25 +465,12 @@ rank16_kernel(const Rank16Args w)
 		for (int p = 0; p < P; ++p) {
 			m1[p] = __builtin_inff(); m2[p] = __builtin_inff(); leader[p] = 0;
 #pragma unroll
-			for (int i = 0; i < (SNAP ? SNAP_ROWS : 0); ++i) asm volatile("" : "=v"(snap[p][i])); /* no value yet: tile 0 always takes the lead */
+			for (int i = 0; i < SNAP_ROWS; ++i) asm volatile("" : "=v"(snap[p][i])); /* no value yet: tile 0 always takes the lead */
 		}
 	};
 
 	auto lowest_of = [](float a, float c) { return __builtin_elementwise_minimum(a, c); };
 	auto track = [&](const f32x16& acc, int p, uint32_t tile) {
-		if constexpr (!SNAP) { /* every result keyed with its number: the two smallest so far, the tile of the smallest */
-			const float before = m1[p];
-#pragma unroll
-			for (int r = 0; r < 16; ++r) {
-				const float v = __uint_as_float((__float_as_uint(acc[r]) & ~15u) | (uint32_t)r);
-				m2[p] = __builtin_amdgcn_fmed3f(m1[p], m2[p], v);
-				m1[p] = __builtin_elementwise_minimum(m1[p], v);
-				asm volatile("" : "+v"(m1[p]), "+v"(m2[p])); /* value by value (see wide_sweep_kernel) */
-			}
-			leader[p] = m1[p] < before ? tile : leader[p];
-			return;
-		}
-		else {
 		float t = acc[0];
 #pragma unroll
 		for (int i = 1; i < 16; ++i) t = lowest_of(t, acc[i]);
@@ -345,7 +478,6 @@ rank16_kernel(const Rank16Args w)
 		const uint64_t leads = settled_mask(tile == 0 ? ~0ull : __builtin_amdgcn_ballot_w64(t < m1[p]));
 		take_lead_where(leads, m1[p], leader[p], t, tile, snap[p], acc);
 		copy_second_half_where(leads, snap[p], acc);
-		}
 	};
 
 	if constexpr (PIPE) {
@@ -442,21 +574,23 @@ rank16_kernel(const Rank16Args w)
 			float raw[P][KB][8];
 			auto request = [&](uint32_t first) {
 #pragma unroll
-				for (int p = 0; p < P; ++p)
+				for (int p = 0; p < P; ++p) {
+					const Rank16Source from = rank16_source<LD, SHARED>(w.data, w.stride, first + p * TILE, w.n, lane);
 #pragma unroll
-					for (int kb = 0; kb < KB; ++kb) {
-						rank16_request<LD>(raw[p][kb], w.data, w.stride, min(first + p * TILE + col, w.n - 1), kb, h, w.dim);
-					}
+					for (int kb = 0; kb < KB; ++kb) rank16_request<LD, SHARED, false>(raw[p][kb], from, w.stride, kb, lane, w.dim);
+				}
 			};
 			auto convert = [&](uint32_t first) {
 #pragma unroll
 				for (int p = 0; p < P; ++p) {
-					xx[p] = 0.0f; xl[p] = 0.0f;
+					Rank16Sums sums = { { 0.0f, 0.0f }, { 0.0f, 0.0f } };
 #pragma unroll
 					for (int kb = 0; kb < KB; ++kb) {
-						rank16_copy<LD>(w, raw[p][kb], first + p * TILE + col, kb * KBLOCK + h * 8);
-						rank16_convert(b[p][kb], raw[p][kb], frame + kb * KBLOCK + h * 8, scale, xx[p], xl[p]);
+						rank16_place<LD, SHARED>(raw[p][kb], kb, lane, w.dim);
+						if (LD == KMX_SOA) rank16_copy(w, raw[p][kb], first + p * TILE, kb, lane, exchange);
+						rank16_convert<SHARED>(b[p][kb], raw[p][kb], frame, scale, kb, lane, sums, exchange);
 					}
+					rank16_total<SHARED>(xx[p], xl[p], sums, lane);
 				}
 			};
 			uint32_t next = uniform(claim());
@@ -482,84 +616,86 @@ rank16_kernel(const Rank16Args w)
 		}
 	}
 	else {
-		/* one chain of KB instructions per tile and point tile; the operands of block kb + AHEAD are requested before the instructions of block kb */
-		constexpr int AHEAD = 2;
-		constexpr uint32_t PIECES = (TF / 4 + RANK16_THREADS - 1) / RANK16_THREADS; /* 16-byte pieces per lane that cover one tile */
-		const uint32_t units = (w.n + RANK16_WAVES * P * TILE - 1) / (RANK16_WAVES * P * TILE);
+		/* one chain of KB instructions per tile and point tile; the operands of block kb + OPERANDS are requested before the instructions of block kb */
+		constexpr int OPERANDS = 2;
+		auto sweep_tile = [&](const float* operands, const float* norms, uint32_t t, uint32_t tile) {
+			f32x16 acc[P];
+			fetch_norms(acc[0], norms, t, h);
+#pragma unroll
+			for (int p = 1; p < P; ++p) acc[p] = acc[0];
+			f16x8 c[KB];
+#pragma unroll
+			for (int kb = 0; kb < OPERANDS && kb < KB; ++kb) c[kb] = operand(operands, t, kb);
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb) {
+				if (kb + OPERANDS < KB) c[kb + OPERANDS] = operand(operands, t, kb + OPERANDS);
+#pragma unroll
+				for (int p = 0; p < P; ++p) acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], b[p][kb], acc[p], 0, 0, 0);
+			}
+			__builtin_amdgcn_sched_group_barrier(0x100, 4 + (OPERANDS < KB ? OPERANDS : KB), 0);
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb) {
+				__builtin_amdgcn_sched_group_barrier(0x008, P, 0);
+				if (kb + OPERANDS < KB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+			}
+#pragma unroll
+			for (int p = 0; p < P; ++p) track(acc[p], p, tile);
+		};
+		/* the ring of chunks: the one whose turn it is has arrived, the others are on their way */
+		constexpr uint32_t SLOTS = rank16_slots(KB), EACH = (KB + WAVES - 1) / WAVES + (rank16_norm_blocks(1) + WAVES - 1) / WAVES; /* a wavefront's requests for a chunk of one tile (more than two slots) */
+		const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)lds;
+		const uint32_t slot_bytes = rank16_slot_bytes(KB, w.chunk_tiles), norm_blocks = rank16_norm_blocks(w.chunk_tiles);
+		const uint32_t chunks = STREAM ? (all_tiles + w.chunk_tiles - 1) / w.chunk_tiles : 1;
+		uint32_t coming = 0, into = 0, from = 0; /* the chunk requested next, the slot it goes to, and the slot whose turn it is */
+		auto request_chunk = [&]() { /* as many requests each time: a short last chunk repeats its last block */
+			const uint32_t tile0 = coming * w.chunk_tiles, blocks = min(w.chunk_tiles, all_tiles - tile0) * KB, to = lds_base + into * slot_bytes;
+			const char* src = (const char*)(w.packed + (size_t)tile0 * (KB * WAVE));
+			for (uint32_t i = wave; i < w.chunk_tiles * KB + wave; i += WAVES) {
+				const uint32_t block = min(i, blocks - 1);
+				stage_block(src + (size_t)block * (WAVE * 16), lane, to + block * (WAVE * 16));
+			}
+			for (uint32_t i = wave; i < norm_blocks + wave; i += WAVES) {
+				const uint32_t block = min(i, norm_blocks - 1);
+				stage_words(w.norms + (size_t)tile0 * NORM_TILE + block * WAVE, lane, to + w.chunk_tiles * (KB * WAVE * 16) + block * (WAVE * 4));
+			}
+			coming = coming + 1 < chunks ? coming + 1 : 0;
+			into = into + 1 < SLOTS ? into + 1 : 0;
+		};
+		if constexpr (STREAM)
+			for (uint32_t i = 0; i + 1 < SLOTS; ++i) request_chunk();
+		auto sweep_chunk = [&](uint32_t chunk) {
+			if constexpr (!STREAM) {
+				for (uint32_t t = 0; t < all_tiles; ++t) sweep_tile(lds, lds + (size_t)all_tiles * TF, t, t);
+				return;
+			}
+			const uint32_t tile0 = chunk * w.chunk_tiles, tiles = min(w.chunk_tiles, all_tiles - tile0);
+			const float* here = lds + (size_t)from * (slot_bytes / 4);
+			for (uint32_t t = 0; t < tiles; ++t) sweep_tile(here, here + w.chunk_tiles * TF, t, tile0 + t);
+			from = from + 1 < SLOTS ? from + 1 : 0;
+		};
+		auto next_chunk = [&]() {
+			if constexpr (!STREAM) return;
+			staged_but<(SLOTS - 2) * EACH>();
+			__syncthreads(); /* everybody's part of this chunk is here, and nobody reads the one before it any more */
+			request_chunk();
+		};
+		const uint32_t units = (w.n + WAVES * P * TILE - 1) / (WAVES * P * TILE);
 		for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
-			const uint32_t first = (unit * RANK16_WAVES + wave) * (P * TILE);
+			const uint32_t first = (unit * WAVES + wave) * (P * TILE);
 			load_points(first);
 			start();
-			for (uint32_t chunk = 0; chunk < chunks; ++chunk) {
-				const uint32_t tile0 = chunk * w.chunk_tiles, tiles = min(w.chunk_tiles, all_tiles - tile0);
-				const uint32_t next_tile0 = chunk + 1 < chunks ? tile0 + w.chunk_tiles : 0, next_tiles = min(w.chunk_tiles, all_tiles - next_tile0);
-				const float* here = lds + (size_t)cur * buffer_floats;
-				const float* norms = here + (size_t)w.chunk_tiles * TF;
-				const f32x4* src = (const f32x4*)w.packed + (size_t)next_tile0 * (TF / 4);
-				const f32x4* nsrc = (const f32x4*)(w.norms + (size_t)next_tile0 * NORM_TILE);
-				f32x4* dst = (f32x4*)(lds + (size_t)(cur ^ 1u) * buffer_floats);
-				f32x4* ndst = (f32x4*)(lds + (size_t)(cur ^ 1u) * buffer_floats + (size_t)w.chunk_tiles * TF);
-				const uint32_t last_vec = next_tiles * (TF / 4) - 1, norm_vec = min(tid, next_tiles * (NORM_TILE / 4) - 1);
-				uint32_t piece = tid;
-				for (uint32_t t = 0; t < tiles; ++t) {
-					f32x4 pv[PIECES], nv;
-					if constexpr (STREAM) {
-#pragma unroll
-						for (uint32_t i = 0; i < PIECES; ++i) pv[i] = src[min(piece + i * RANK16_THREADS, last_vec)];
-						nv = nsrc[norm_vec];
-					}
-					f32x16 acc[P];
-					fetch_norms(acc[0], norms, t, h);
-#pragma unroll
-					for (int p = 1; p < P; ++p) acc[p] = acc[0];
-					f16x8 c[KB];
-#pragma unroll
-					for (int kb = 0; kb < AHEAD && kb < KB; ++kb) c[kb] = operand(here, t, kb);
-#pragma unroll
-					for (int kb = 0; kb < KB; ++kb) {
-						if (kb + AHEAD < KB) c[kb + AHEAD] = operand(here, t, kb + AHEAD);
-#pragma unroll
-						for (int p = 0; p < P; ++p) acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(c[kb], b[p][kb], acc[p], 0, 0, 0);
-					}
-					__builtin_amdgcn_sched_group_barrier(0x020, STREAM ? PIECES + 1 : 0, 0);
-					__builtin_amdgcn_sched_group_barrier(0x100, 4 + (AHEAD < KB ? AHEAD : KB), 0);
-#pragma unroll
-					for (int kb = 0; kb < KB; ++kb) {
-						__builtin_amdgcn_sched_group_barrier(0x008, P, 0);
-						if (kb + AHEAD < KB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-					}
-#pragma unroll
-					for (int p = 0; p < P; ++p) track(acc[p], p, tile0 + t);
-					if constexpr (STREAM) {
-#pragma unroll
-						for (uint32_t i = 0; i < PIECES; ++i) dst[min(piece + i * RANK16_THREADS, last_vec)] = pv[i];
-						ndst[norm_vec] = nv;
-						piece += PIECES * RANK16_THREADS;
-					}
-				}
-				if constexpr (STREAM) {
-					/* a short chunk has fewer steps than the next one has tiles: the remaining pieces */
-					for (; piece - tid <= last_vec; piece += PIECES * RANK16_THREADS) {
-#pragma unroll
-						for (uint32_t i = 0; i < PIECES; ++i) {
-							const uint32_t at = min(piece + i * RANK16_THREADS, last_vec);
-							dst[at] = src[at];
-						}
-					}
-					__syncthreads();
-					cur ^= 1u;
-				}
-			}
+			for (uint32_t chunk = 0; chunk < chunks; ++chunk) { next_chunk(); sweep_chunk(chunk); }
 			finish(first);
 		}
 	}
+	if constexpr (STREAM) staged_but<0>(); /* (nothing may arrive in LDS that is no longer this work-group's) */
 	/* what is left in the lists: one addition per work-group (one per wavefront took 12 us of a launch: 2048 of them to one address) */
 	__syncthreads();
 	if (lane == 0) wave_max[0][wave] = flagged;
 	__syncthreads();
 	uint32_t before = 0, all = 0;
 #pragma unroll
-	for (uint32_t v = 0; v < RANK16_WAVES; ++v) {
+	for (uint32_t v = 0; v < WAVES; ++v) {
 		before += v < wave ? wave_max[0][v] : 0u;
 		all += wave_max[0][v];
 	}
@@ -573,18 +709,21 @@ rank16_kernel(const Rank16Args w)
 template <int KB>
 static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
-	const uint32_t budget = lds_budget_of(exec, dev), static_bytes = rank16_static_bytes<KB>();
-	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4;
-	if (budget < static_bytes + 2 * tile_bytes) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
-	const uint32_t tiles = w.kp / TILE, fit = (budget - static_bytes) / tile_bytes;
-	const bool stream_mode = tiles > fit;
-	w.chunk_tiles = stream_mode ? std::min(fit / 2, RANK16_THREADS * 4 / NORM_TILE) : tiles;
-	const uint32_t lds_bytes = (stream_mode ? 2 : 1) * w.chunk_tiles * tile_bytes;
+	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4, tiles = w.kp / TILE, budget = lds_budget_of(exec, dev);
+	if (budget < rank16_least_bytes(KB, a.layout)) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
+	const bool stream_mode = (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false) > budget;
+	w.chunk_tiles = tiles;
+	uint32_t lds_bytes = tiles * tile_bytes;
+	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode);
+	if (stream_mode) {
+		w.chunk_tiles = 1;
+		while (rank16_slots(KB) == 2 && w.chunk_tiles < tiles && static_bytes + 2 * rank16_slot_bytes(KB, w.chunk_tiles + 1) <= budget) ++w.chunk_tiles;
+		lds_bytes = rank16_slots(KB) * rank16_slot_bytes(KB, w.chunk_tiles);
+	}
 	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true> : rank16_kernel<KB, KMX_AOS, false>)
 	                                                 : (stream_mode ? rank16_kernel<KB, KMX_SOA, true> : rank16_kernel<KB, KMX_SOA, false>);
-	const bool pipe = !stream_mode && KB <= 4;
-	const uint32_t unit = (pipe ? 1 : RANK16_WAVES) * RANK16_P * TILE;
-	const uint32_t grid = std::min((a.n + unit - 1) / unit, dev.compute_units);
+	const uint32_t waves = rank16_waves(KB, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
+	const uint32_t grid = std::min((a.n + unit - 1) / unit, RANK16_P * 4 / waves * dev.compute_units);
 	exec->block_count = grid;
 #define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (half-precision sweep): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u, chunk tiles %u, LDS %u)", \
 	#cond, a.dim, a.k, w.kp, a.n, w.chunk_tiles, lds_bytes); } while (0)
@@ -592,12 +731,14 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 		KMX_PLAN(w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1 && KB * KBLOCK >= a.dim);
 		KMX_PLAN(w.chunk_tiles >= 1 && (uint64_t)lds_bytes + static_bytes <= dev.lds_bytes && rank16_tile_floats<KB>() % 4 == 0);
 		KMX_PLAN(ws->packed16 && (size_t)tiles * KB * WAVE * 4 <= ws->packed16_cap);
+		KMX_PLAN(!stream_mode || ((rank16_slots(KB) == 2 || w.chunk_tiles == 1) && /* whole requests of norms, the last chunk's too */
+		                          (size_t)(tiles - 1) / w.chunk_tiles * w.chunk_tiles * NORM_TILE + rank16_norm_blocks(w.chunk_tiles) * WAVE <= ws->norms16_cap));
 		KMX_PLAN(a.layout == KMX_AOS || (w.copies && w.copy_stride % 8 == 0 && w.copy_stride >= a.dim && w.copy_stride <= KB * KBLOCK && (size_t)a.n * w.copy_stride <= ws->queued_rows_cap));
 		KMX_PLAN(w.list && w.length && w.norms && w.low2 && w.frame && w.scale);
 	}
 #undef KMX_PLAN
 	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-	KMX_LAUNCH_KERNEL(kernel, dim3(grid), dim3(RANK16_THREADS), lds_bytes, stream(), w);
+	KMX_LAUNCH_KERNEL(kernel, dim3(grid), dim3(waves * WAVE), lds_bytes, stream(), w);
 	KMX_LAUNCH_CHECK("rank16_kernel");
 	return KMX_OK;
 }

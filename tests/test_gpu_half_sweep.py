@@ -99,3 +99,32 @@ def test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, mode
     assert np.allclose(got, sums / counts[:, None], rtol=1e-5, atol=1e-6)
     for b in (d, m, o, a, s):
         b.free()
+
+
+@pytest.mark.parametrize("dim,k,n,budget", [
+    (100, 700, 263003, 0), (60, 1250, 263003, 0), (20, 2300, 140001, 0),   # two chunks as large as fit, several units per work-group
+    (250, 330, 263003, 0), (177, 290, 140001, 0),                           # slots of a tile, two work-groups per compute unit
+    (16, 3000, 700, 56 * 1024), (96, 90, 700, 56 * 1024), (256, 65, 700, 78 * 1024),  # as little LDS as the exact pass runs in
+])
+def test_centroids_that_stream_by(km, orc, gpu, dim, k, n, budget):
+    rng = np.random.default_rng(dim + n)
+    means = rng.normal(size=(k, dim)).astype(np.float32)
+    rows = (means[rng.integers(0, k, n)] + rng.normal(size=(n, dim)) * 0.5).astype(np.float32)
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 0))
+    a = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for layout in (0, 1):
+            d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, layout))
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            ex = km.ExecParams(shared_mem_bytes=budget)
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, layout, km.layout_stride(layout, n, dim), m, 0, dim, a, dim, k, n, ex)
+            km.sync()
+            got = a.read(np.uint32, n)
+            d.free()
+            assert ex.block_count <= 2 * gpu.compute_units
+            assert np.array_equal(got, want), "layout %d: %d mismatches" % (layout, int((got != want).sum()))
+    finally:
+        km.set_two_level_sweep(1)
+    m.free(); a.free()
