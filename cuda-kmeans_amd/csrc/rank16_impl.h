@@ -14,7 +14,14 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 /*
- * Wavefronts of a work-group: eight around centroids in LDS. Where the centroids stream by (slots of a chunk of tiles that go round, filled by
+ * Rows of up to 32 dimensions around resident centroids: three wavefronts on a SIMD, of which the third also covers the ends of the others'
+ * sweeps. That takes tracking in fewer registers (RANK16_GROUPS). us per assignment, two wavefronts with the snapshot -> three: N = 2M, d = 32,
+ * k = 1024 201 -> 191; d = 16 155 -> 137; d = 10, k = 100 69 -> 63. The same tracking with two: 208, 152, 72 against 211, 159, 70. Wider rows would
+ * spill (N = 1M, d = 64, k = 512: 103 -> 114), and so does the copying of SoA points (d = 24, k = 256: 68.6 -> 69.6).
+ */
+constexpr bool rank16_grouped(uint32_t kb, int layout) { return kb == 1 || (kb == 2 && layout == KMX_AOS); }
+/*
+ * Wavefronts of a work-group: otherwise eight around centroids in LDS. Where the centroids stream by (slots of a chunk of tiles that go round, filled by
  * requests straight to LDS, a barrier per chunk), rows of up to 128 dimensions keep that form with two chunks as large as fit, since the
  * barriers are what costs (us per assignment, two work-groups of four wavefronts with four slots of 32 matrix instructions -> this: N = 2M,
  * d = 128, k = 1024 659 -> 627; N = 1M, d = 96, k = 2000 493 -> 440; d = 64, k = 3000 473 -> 424). Wider rows have a barrier's worth of matrix
@@ -22,9 +29,8 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
  * the matrix cores, and four slots of a tile (N = 1M, d = 256, k = 1024: 549, with eight wavefronts and two chunks of four tiles 569).
  * With chunks through registers and eight wavefronts for all widths: 656, 655, 480, 464.
  */
-constexpr uint32_t rank16_waves(uint32_t kb, bool stream) { return stream && kb >= 12 ? 4 : 8; }
+constexpr uint32_t rank16_waves(uint32_t kb, int layout, bool stream) { return stream && kb >= 12 ? 4 : !stream && rank16_grouped(kb, layout) ? 12 : 8; }
 constexpr int RANK16_P = 2; /* point tiles per wavefront: an operand read serves two instructions */
-constexpr uint32_t RANK16_LIST = 120;
 
 struct Rank16Args {
 	const float* data; size_t stride;
@@ -50,6 +56,8 @@ inline size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) 
 
 /* 16 tile bytes per block of 16 dimensions and lane, then the tile's norms */
 template <int KB> constexpr uint32_t rank16_tile_floats() { return KB * WAVE * 4; }
+/* listed points a wavefront keeps in LDS before they go out */
+constexpr uint32_t rank16_list(uint32_t kb, int layout, bool stream) { return rank16_waves(kb, layout, stream) == 12 ? 80 : 120; }
 constexpr uint32_t rank16_slots(uint32_t kb) { return kb >= 12 ? 4 : 2; }
 __host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { return (tiles * NORM_TILE + WAVE - 1) / WAVE; }
 /* what a chunk takes in LDS, its norms behind its operands as whole requests of 64 words */
@@ -57,7 +65,7 @@ __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t t
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
 constexpr uint32_t rank16_exchange(uint32_t kb, int layout) { return rank16_shared_rows(kb, layout) || layout == KMX_SOA ? RANK16_EXCHANGE : 0; }
-constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream) { return ((2 * RANK16_LIST + rank16_exchange(kb, layout) + 4) * rank16_waves(kb, stream) + kb * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream) { return ((2 * rank16_list(kb, layout, stream) + rank16_exchange(kb, layout) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
 constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
@@ -280,6 +288,42 @@ __device__ __forceinline__ void stage_words(const void* from, uint32_t lane, uin
 template <uint32_t LATER> __device__ __forceinline__ void staged_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LATER) : "memory"); }
 
 /*
+ * rank16_grouped: of the leading tile's 16 results only the minima of six groups are kept (the instructions that find the tile's minimum
+ * produce them on the way), and the winning group's three centroids are looked at again at the end. Results of groups 0 to 3: 4 i, 4 i + 1, 4 i + 2; of group 4: 3, 7, 11; of group 5: 15. As rows of a tile: */
+constexpr int RANK16_GROUPS = 6;
+__device__ __forceinline__ uint32_t rank16_group_row(uint32_t group) { return group < 4 ? 8 * group : group == 4 ? 3 : 27; } /* + 4 h: the first */
+__device__ __forceinline__ uint32_t rank16_group_step(uint32_t group) { return group < 4 ? 1 : 8; }
+
+/* In the lanes of `mask` (settled_mask; see take_lead_where): the smallest value so far becomes `lowest`, its tile `tile`, and the minima of the
+ * tile's groups replace those kept */
+__device__ __forceinline__ void take_groups_where(uint64_t mask, float& m1, uint32_t& leader, float lowest, uint32_t tile, f32x2 (&kept)[3], const f32x2 (&now)[2], float g4, float g5)
+{
+	uint64_t saved;
+	float k4 = kept[2].x, k5 = kept[2].y;
+	asm volatile("s_and_saveexec_b64 %[saved], %[mask]\n\tv_mov_b32 %[m1], %[lowest]\n\tv_mov_b32 %[leader], %[tile]\n\t"
+	             "v_mov_b64 %[d0], %[s0]\n\tv_mov_b64 %[d1], %[s1]\n\tv_mov_b32 %[d4], %[s4]\n\tv_mov_b32 %[d5], %[s5]\n\ts_mov_b64 exec, %[saved]"
+	             : [m1] "+v"(m1), [leader] "+v"(leader), [d0] "+v"(kept[0]), [d1] "+v"(kept[1]), [d4] "+v"(k4), [d5] "+v"(k5), [saved] "=&s"(saved)
+	             : [lowest] "v"(lowest), [tile] "s"(tile), [s0] "v"(now[0]), [s1] "v"(now[1]), [s4] "v"(g4), [s5] "v"(g5), [mask] "s"(mask)
+	             : "scc");
+	kept[2] = f32x2{ k4, k5 };
+}
+
+/* sum + the products of eight half-precision values, one rounding each */
+__device__ __forceinline__ float rank16_dot(const f16x8& c, const f16x8& x, float sum)
+{
+#pragma unroll
+	for (int e = 0; e < 8; ++e) sum = __builtin_fmaf((float)c[e], (float)x[e], sum);
+	return sum;
+}
+
+/* the sum of the two half-waves' values, without a trip through LDS */
+__device__ __forceinline__ float rank16_both(float v)
+{
+	const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+	return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+/*
  * A work-group around centroids in LDS: all of them (STREAM = false), or slots that go round (rank16_waves), all its wavefronts sweeping
  * together. A wavefront sweeps 64 points at a time. With resident centroids the wavefronts take items of 64 points from a counter in
  * LDS (a SIMD serves its older wavefront first: equal shares leave the younger ones sweeping alone at the end).
@@ -293,19 +337,20 @@ template <uint32_t LATER> __device__ __forceinline__ void staged_but() { asm vol
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
 template <int KB, int LD, bool STREAM>
-__global__ void __launch_bounds__(rank16_waves(KB, STREAM) * WAVE, 2)
+__global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM) * WAVE, rank16_waves(KB, LD, STREAM) == 12 ? 3 : 2)
 rank16_kernel(const Rank16Args w)
 {
-	constexpr uint32_t WAVES = rank16_waves(KB, STREAM), THREADS = WAVES * WAVE;
+	constexpr uint32_t WAVES = rank16_waves(KB, LD, STREAM), THREADS = WAVES * WAVE, LIST = rank16_list(KB, LD, STREAM);
 	constexpr int P = RANK16_P;
 	constexpr uint32_t TF = rank16_tile_floats<KB>();
 	constexpr bool PIPE = !STREAM && KB <= 4;
 	constexpr bool SHARED = rank16_shared_rows(KB, LD);
-	constexpr bool PREFETCH = PIPE && KB <= 2; /* the next item's coordinates travel while the current one is swept */
+	constexpr bool GROUPED = PIPE && rank16_grouped(KB, LD);
+	constexpr bool PREFETCH = PIPE && (KB == 1 || (KB == 2 && !GROUPED)); /* the next item's coordinates travel while the current one is swept */
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
 	__shared__ uint32_t wave_max[4][WAVES];
-	__shared__ uint32_t flag_list[WAVES][2 * RANK16_LIST];
+	__shared__ uint32_t flag_list[WAVES][2 * LIST];
 	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD) ? RANK16_EXCHANGE : 1];
 	uint32_t& claimed = wave_max[3][0];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
@@ -373,7 +418,8 @@ rank16_kernel(const Rank16Args w)
 	float* const exchange = exchanges[wave];
 	float m1[P], m2[P];
 	uint32_t leader[P];
-	float snap[P][SNAP_ROWS];
+	float snap[P][GROUPED ? 1 : SNAP_ROWS];
+	f32x2 kept[P][RANK16_GROUPS / 2]; /* GROUPED: the minima of the leading tile's groups */
 
 	/* A block is converted while the next DEPTH ones are on their way. (Requesting the first of them while the unit before is swept was no gain:
 	 * N = 2M, d = 128, k = 1024: 653 against 618 us, d = 96 440 against 442.) */
@@ -422,22 +468,51 @@ rank16_kernel(const Rank16Args w)
 		for (int p = 0; p < P; ++p) {
 			/* the two smallest of the leading tile's 16 results, the number of a result in its lowest four bits (cert_kd_keyed) */
 			float v1 = __builtin_inff(), v2 = __builtin_inff();
+			constexpr int VALUES = GROUPED ? RANK16_GROUPS : SNAP_ROWS;
+			constexpr uint32_t NUMBER = GROUPED ? 7u : 15u;
 #pragma unroll
-			for (int r = 0; r < SNAP_ROWS; ++r) {
-				const float v = __uint_as_float((__float_as_uint(snap[p][r]) & ~15u) | (uint32_t)r);
+			for (int r = 0; r < VALUES; ++r) {
+				const float v = __uint_as_float((__float_as_uint(GROUPED ? kept[p][r / 2 % (RANK16_GROUPS / 2)][r % 2] : snap[p][GROUPED ? 0 : r]) & ~NUMBER) | (uint32_t)r);
 				v2 = __builtin_amdgcn_fmed3f(v1, v2, v);
 				v1 = __builtin_elementwise_minimum(v1, v);
 			}
-			const uint32_t r = __float_as_uint(v1) & 15u;
-			const uint32_t mine_idx = leader[p] * TILE + 8 * (r / 4) + 4 * h + r % 4;
+			const uint32_t r = __float_as_uint(v1) & NUMBER;
+			/* GROUPED: the first centroid of the group, and the group */
+			const uint32_t mine_idx = GROUPED ? (leader[p] * TILE + rank16_group_row(r) + 4 * h) * 8 + r : leader[p] * TILE + 8 * (r / 4) + 4 * h + r % 4;
 			const float o1 = __shfl_xor(m1[p], 32), o2 = __shfl_xor(m2[p], 32);
 			const float ov1 = __shfl_xor(v1, 32), ov2 = __shfl_xor(v2, 32);
 			const uint32_t oi = (uint32_t)__shfl_xor((int)mine_idx, 32);
 			const bool win = m1[p] < o1 || (m1[p] == o1 && h == 0);
 			const float others = win ? fminf(o1, m2[p]) : fminf(m1[p], o2); /* everything outside the leading 16 rows */
-			const uint32_t idx = win ? mine_idx : oi;
-			const float lowest = win ? v1 : ov1;
-			const float next = fminf(win ? v2 : ov2, others);
+			uint32_t idx = win ? mine_idx : oi;
+			float lowest = win ? v1 : ov1;
+			float next = fminf(win ? v2 : ov2, others);
+			if constexpr (GROUPED) {
+				/* the group's centroids again, on the vector ALU: half of the dimensions in each half-wave, chains of half as many roundings as the
+				 * matrix instructions' (cert_kd_level1 covers them) */
+				const uint32_t group = idx % 8, first = idx / 8, tile = first / TILE, row = first % TILE, step = rank16_group_step(group);
+				const f16x8* at = (const f16x8*)(lds + (size_t)tile * TF) + h * TILE + row;
+				const float* norms = lds + (size_t)w.chunk_tiles * TF + tile * NORM_TILE + row;
+				float r1 = __builtin_inff(), r2 = __builtin_inff();
+#pragma unroll
+				for (uint32_t q = 0; q < 3; ++q) {
+					const uint32_t on = group == 5 ? 0 : q * step;
+					float sum = 0.0f;
+#pragma unroll
+					for (int kb = 0; kb < KB; ++kb) {
+						const f16x8 c = at[kb * WAVE + on];
+						sum = rank16_dot(c, b[p][kb], sum);
+					}
+					float a = norms[on] + rank16_both(sum);
+					if (q > 0) a = group == 5 ? 1.7e38f : a;
+					const float v = __uint_as_float((__float_as_uint(a) & ~3u) | q);
+					r2 = __builtin_amdgcn_fmed3f(r1, r2, v);
+					r1 = __builtin_elementwise_minimum(r1, v);
+				}
+				idx = first + (__float_as_uint(r1) & 3u) * step;
+				lowest = r1;
+				next = fminf(next, r2);
+			}
 			const float x2 = rank16_whole<SHARED>(xx[p]), tau = cert_tau(w.kd, x2, rank16_whole<SHARED>(xl[p]), cert);
 			const uint32_t pt = first_pt + p * TILE + col;
 			const bool mine = h == 0 && pt < w.n;
@@ -449,7 +524,7 @@ rank16_kernel(const Rank16Args w)
 			const unsigned long long mask = __ballot(flag);
 			if (mask) {
 				const uint32_t add = (uint32_t)__builtin_popcountll(mask);
-				if (flagged + add > RANK16_LIST) flush_flags();
+				if (flagged + add > LIST) flush_flags();
 				if (flag) {
 					const uint32_t at = 2 * (flagged + (uint32_t)__builtin_popcountll(mask & ((1ull << lane) - 1ull)));
 					flag_list[wave][at] = pt;
@@ -465,21 +540,13 @@ rank16_kernel(const Rank16Args w)
 		for (int p = 0; p < P; ++p) {
 			m1[p] = __builtin_inff(); m2[p] = __builtin_inff(); leader[p] = 0;
 #pragma unroll
-			for (int i = 0; i < SNAP_ROWS; ++i) asm volatile("" : "=v"(snap[p][i])); /* no value yet: tile 0 always takes the lead */
+			for (int i = 0; i < (GROUPED ? 0 : SNAP_ROWS); ++i) asm volatile("" : "=v"(snap[p][i])); /* no value yet: tile 0 always takes the lead */
+#pragma unroll
+			for (int i = 0; i < (GROUPED ? RANK16_GROUPS / 2 : 0); ++i) asm volatile("" : "=v"(kept[p][i]));
 		}
 	};
 
 	auto lowest_of = [](float a, float c) { return __builtin_elementwise_minimum(a, c); };
-	auto track = [&](const f32x16& acc, int p, uint32_t tile) {
-		float t = acc[0];
-#pragma unroll
-		for (int i = 1; i < 16; ++i) t = lowest_of(t, acc[i]);
-		m2[p] = __builtin_amdgcn_fmed3f(m1[p], m2[p], t);
-		const uint64_t leads = settled_mask(tile == 0 ? ~0ull : __builtin_amdgcn_ballot_w64(t < m1[p]));
-		take_lead_where(leads, m1[p], leader[p], t, tile, snap[p], acc);
-		copy_second_half_where(leads, snap[p], acc);
-	};
-
 	if constexpr (PIPE) {
 		const float* norms = lds + (size_t)w.chunk_tiles * TF;
 		const uint32_t tiles = all_tiles;
@@ -498,24 +565,42 @@ rank16_kernel(const Rank16Args w)
 			start();
 			f32x16 acc0[P], acc1[P];
 			constexpr int MFMAS = KB * P, SLOTS = KB;
-			constexpr int SNAP_OPS = 12 + SNAP_ROWS / 2;
-			constexpr int OPS_PER_SLOT = (SNAP_OPS + SLOTS - 1) / SLOTS;
+			constexpr int TRACK_OPS = GROUPED ? 11 : 20, OPS_PER_SLOT = (TRACK_OPS + SLOTS - 1) / SLOTS;
+			f32x2 group[P][2];
+			float group4[P], lowest[P];
+			uint64_t leads[P];
+			auto track = [&](const f32x16& a, int p, uint32_t tile, int u) {
+				auto lowest_of_three = [&](float x, float y, float z) { return lowest_of(lowest_of(x, y), z); };
+				const int minima = 8;
+				if (u >= minima) {
+					if (u == minima) m2[p] = __builtin_amdgcn_fmed3f(m1[p], m2[p], lowest[p]);
+					else if (u == minima + 1) leads[p] = settled_mask(tile == 0 ? ~0ull : __builtin_amdgcn_ballot_w64(lowest[p] < m1[p]));
+					else if constexpr (GROUPED) {
+						if (u == minima + 2) take_groups_where(leads[p], m1[p], leader[p], lowest[p], tile, kept[p], group[p], group4[p], a[15]);
+					}
+					else if (u == 12) take_lead_where(leads[p], m1[p], leader[p], lowest[p], tile, snap[p], a);
+					else if (u == 16) copy_second_half_where(leads[p], snap[p], a);
+				}
+				else if constexpr (GROUPED) {
+					if (u < 4) group[p][u / 2][u % 2] = lowest_of_three(a[4 * u], a[4 * u + 1], a[4 * u + 2]);
+					else if (u == 4) group4[p] = lowest_of_three(a[3], a[7], a[11]);
+					else if (u == 5) lowest[p] = lowest_of_three(group[p][0].x, group[p][0].y, group[p][1].x);
+					else if (u == 6) lowest[p] = lowest_of_three(lowest[p], group[p][1].y, group4[p]);
+					else lowest[p] = lowest_of(lowest[p], a[15]);
+				}
+				else lowest[p] = u == 0 ? lowest_of(a[0], a[1]) : lowest_of_three(lowest[p], a[2 * u], a[2 * u + 1]);
+			};
+			auto track_all = [&](const f32x16 (&a)[P], uint32_t tile) {
+#pragma unroll
+				for (int p = 0; p < P; ++p)
+#pragma unroll
+					for (int u = 0; u < TRACK_OPS; ++u) track(a[p], p, tile, u);
+			};
 			/* one step: tile t_new into acc_new (which holds its norms), the tile after it requested, the tile in acc_old tracked in
 			 * pieces behind the matrix instructions, then the norms of the tile after next into acc_old */
 			auto step = [&](Ops& fetch_into, uint32_t t_new, f32x16 (&acc_new)[P], const Ops& use, f32x16 (&acc_old)[P], uint32_t tile_old) {
 				fetch(fetch_into, min(t_new + 1, tiles - 1));
 				__builtin_amdgcn_sched_barrier(0);
-				float lowest[P];
-				uint64_t leads[P];
-				auto op = [&](int p, int u) {
-					const f32x16& a = acc_old[p];
-					if (u == 0) lowest[p] = lowest_of(a[0], a[1]);
-					else if (u < 8) lowest[p] = lowest_of(lowest_of(lowest[p], a[2 * u]), a[2 * u + 1]);
-					else if (u == 8) m2[p] = __builtin_amdgcn_fmed3f(m1[p], m2[p], lowest[p]);
-					else if (u == 9) leads[p] = settled_mask(tile_old == 0 ? ~0ull : __builtin_amdgcn_ballot_w64(lowest[p] < m1[p]));
-					else if (u == 12) take_lead_where(leads[p], m1[p], leader[p], lowest[p], tile_old, snap[p], a);
-					else if (u == 16) copy_second_half_where(leads[p], snap[p], a);
-				};
 				int issued = 0;
 #pragma unroll
 				for (int kb = 0; kb < KB; ++kb)
@@ -526,7 +611,7 @@ rank16_kernel(const Rank16Args w)
 						const int tp = issued / SLOTS, first_op = (issued % SLOTS) * OPS_PER_SLOT;
 #pragma unroll
 						for (int u = first_op; u < first_op + OPS_PER_SLOT; ++u)
-							if (u < SNAP_OPS) op(tp, u);
+							if (u < TRACK_OPS) track(acc_old[tp], tp, tile_old, u);
 						__builtin_amdgcn_sched_barrier(0);
 						if (issued == SLOTS - 1 || MFMAS == 1) { /* acc_old[0] has been tracked */
 							fetch_norms(acc_old[0], norms, min(t_new + 1, tiles - 1), h);
@@ -549,15 +634,10 @@ rank16_kernel(const Rank16Args w)
 			}
 			if (t + 1 < tiles) {
 				multiply(acc1, o1);
-#pragma unroll
-				for (int p = 0; p < P; ++p) track(acc0[p], p, t);
-#pragma unroll
-				for (int p = 0; p < P; ++p) track(acc1[p], p, t + 1);
+				track_all(acc0, t);
+				track_all(acc1, t + 1);
 			}
-			else {
-#pragma unroll
-				for (int p = 0; p < P; ++p) track(acc0[p], p, t);
-			}
+			else track_all(acc0, t);
 		};
 		const uint32_t items_all = (w.n + P * TILE - 1) / (P * TILE);
 		const uint32_t item0 = (uint32_t)((uint64_t)blockIdx.x * items_all / gridDim.x), item1 = (uint32_t)((uint64_t)(blockIdx.x + 1) * items_all / gridDim.x);
@@ -618,6 +698,15 @@ rank16_kernel(const Rank16Args w)
 	else {
 		/* one chain of KB instructions per tile and point tile; the operands of block kb + OPERANDS are requested before the instructions of block kb */
 		constexpr int OPERANDS = 2;
+		auto track = [&](const f32x16& acc, int p, uint32_t tile) {
+			float t = acc[0];
+#pragma unroll
+			for (int i = 1; i < 16; ++i) t = lowest_of(t, acc[i]);
+			m2[p] = __builtin_amdgcn_fmed3f(m1[p], m2[p], t);
+			const uint64_t leads = settled_mask(tile == 0 ? ~0ull : __builtin_amdgcn_ballot_w64(t < m1[p]));
+			take_lead_where(leads, m1[p], leader[p], t, tile, snap[p], acc);
+			copy_second_half_where(leads, snap[p], acc);
+		};
 		auto sweep_tile = [&](const float* operands, const float* norms, uint32_t t, uint32_t tile) {
 			f32x16 acc[P];
 			fetch_norms(acc[0], norms, t, h);
@@ -722,8 +811,8 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 	}
 	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true> : rank16_kernel<KB, KMX_AOS, false>)
 	                                                 : (stream_mode ? rank16_kernel<KB, KMX_SOA, true> : rank16_kernel<KB, KMX_SOA, false>);
-	const uint32_t waves = rank16_waves(KB, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
-	const uint32_t grid = std::min((a.n + unit - 1) / unit, RANK16_P * 4 / waves * dev.compute_units);
+	const uint32_t waves = rank16_waves(KB, a.layout, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
+	const uint32_t grid = std::min((a.n + unit - 1) / unit, (waves == 4 ? 2 : 1) * dev.compute_units);
 	exec->block_count = grid;
 #define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (half-precision sweep): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u, chunk tiles %u, LDS %u)", \
 	#cond, a.dim, a.k, w.kp, a.n, w.chunk_tiles, lds_bytes); } while (0)

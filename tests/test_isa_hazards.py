@@ -68,3 +68,21 @@ def test_masked_copies_read_a_settled_mask(tmp_path, blocks):
     assert any(w is not None for _, w in waits), "masks written by vector compares are expected"
     close = [(i, code[i]) for i, w in waits if w is not None and w < 2]
     assert not close, "%d masked statements within two wait states of the compare that wrote their mask, first: %s" % (len(close), close[0][1])
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 3])
+def test_masked_copies_of_the_half_precision_sweep_read_a_settled_mask(tmp_path, blocks):
+    hipcc = "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    asm = tmp_path / ("rank16_kb%d.s" % blocks)
+    subprocess.check_call([hipcc] + FLAGS + ["-DKMX_KB=%d" % blocks, "-S", "--cuda-device-only",
+                                             os.path.join(CSRC, "rank16_inst.hip"), "-o", str(asm)],
+                          stderr=subprocess.DEVNULL)
+    code = instructions(str(asm))
+    statements = list(masked_statements(code))
+    assert {moves for _, _, moves in statements} >= {6}, "a leader with its groups, or with the first half of its results"
+    waits = [(i, wait_states_since_compare(code, i, reg)) for i, reg, _ in statements]
+    assert any(w is not None for _, w in waits), "masks written by vector compares are expected"
+    close = [(i, code[i]) for i, w in waits if w is not None and w < 2]
+    assert not close, "%d masked statements within two wait states of the compare that wrote their mask, first: %s" % (len(close), close[0][1])
