@@ -16,7 +16,7 @@
  * additions, whatever the machine.
  *
  * Kernels: ordered_histogram_kernel, ordered_offsets_kernel, ordered_starts_kernel, ordered_scatter_kernel,
- * ordered_staged_sum_kernel / ordered_sum_kernel.
+ * ordered_stream_sum_kernel / ordered_staged_sum_kernel / ordered_sum_kernel.
  */
 #include "kmx_internal.h"
 
@@ -342,6 +342,137 @@ ordered_staged_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
 	if (tid < width) means[elem<LM>(stride_means, c, d0 + tid)] = !divide ? sum : (members ? sum / (F)members : (F)0);
 }
 
+/*
+ * The same for AoS rows of whole 16-byte pieces: a work-group per cluster and block of 128 bytes of the row. One wavefront requests the members'
+ * rows straight to LDS, AHEAD batches of eight requests before they are added, and the members' numbers AHEAD batches before that; the other one
+ * adds, a lane per coordinate, two members per LDS read, and waits for nothing but the batch's barrier. What bounds it is the longest
+ * cluster's chain, at 1.5 instructions a member (N = 100k, d = 36, k = 2: 4.9 ns a member; with one wavefront that requests and adds 7.8), then the memory
+ * (N = 2M, d = 32, k = 1024: 80 us, 3.4 TB/s; one wavefront 107, the staged kernel above 169). AHEAD of 1, 2, 3, 4 with one wavefront: 133, 106,
+ * 107, 122 us (four work-groups fit a compute unit with up to 3).
+ */
+constexpr uint32_t STREAM_BLOCK_BYTES = 128, STREAM_REQUESTS = 8, STREAM_SLOT_BYTES = STREAM_REQUESTS * WAVE * 16;
+constexpr uint32_t stream_rows(uint32_t pieces) { return WAVE / pieces; }                     /* per request */
+constexpr uint32_t stream_batch(uint32_t pieces) { return STREAM_REQUESTS * stream_rows(pieces); }
+constexpr uint32_t stream_names(uint32_t pieces) { return (stream_batch(pieces) + WAVE - 1) / WAVE; } /* requests for a batch's numbers */
+/* (a wavefront's wait can leave up to 63 requests on their way) */
+constexpr uint32_t stream_ahead(uint32_t pieces, bool deep) { return !deep ? 3 : std::min(6u, 63 / (STREAM_REQUESTS + stream_names(pieces)) + 1); }
+constexpr uint32_t stream_lds_bytes(uint32_t pieces, bool deep) { return (stream_ahead(pieces, deep) + 1) * (STREAM_SLOT_BYTES + stream_names(pieces) * WAVE * 4); }
+
+/* straight to LDS: 16 (4) bytes per lane, lane by lane behind `to`, a uniform byte offset. Waits are the caller's (vmcnt) */
+__device__ __forceinline__ void stream_request16(const void* from, uint32_t to)
+{
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(from) : "m0", "memory");
+}
+__device__ __forceinline__ void stream_request4(const void* from, uint32_t to)
+{
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(to), "v"(from) : "m0", "memory");
+}
+
+template <typename F, int LM, uint32_t P, bool DEEP>
+__global__ void __launch_bounds__(2 * WAVE)
+ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ starts,
+                          const uint32_t* __restrict__ sizes, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t blocks, uint32_t divide)
+{
+	constexpr uint32_t PIECE = 16 / sizeof(F), BLOCK = STREAM_BLOCK_BYTES / sizeof(F), ROWS = stream_rows(P), BATCH = stream_batch(P), NAMES = stream_names(P);
+	constexpr uint32_t AHEAD = stream_ahead(P, DEEP), SLOTS = AHEAD + 1, EACH = STREAM_REQUESTS + NAMES;
+	extern __shared__ __attribute__((aligned(16))) char stream_lds[];
+	const uint32_t c = blockIdx.x / blocks, d0 = blockIdx.x % blocks * BLOCK, width = min(BLOCK, dim - d0); /* (whole pieces, no more than P) */
+	const uint32_t members = sizes[c], begin = starts[c], lane = threadIdx.x % WAVE;
+	if (__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) != 0) { /* requests */
+		if (members == 0) return;
+		const uint32_t rows_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)stream_lds, names_at = rows_at + SLOTS * STREAM_SLOT_BYTES;
+		/* this lane's row of a request (lanes without one repeat the last) and its piece (a narrower last block repeats its last one) */
+		const uint32_t row = min(lane / P, ROWS - 1);
+		const F* piece = data + d0 + min(lane % P * PIECE, width - PIECE);
+		const uint32_t row_bytes = (uint32_t)(stride * sizeof(F)); /* (below 2^32, see the launcher) */
+		uint32_t named = 0, name_slot = 0, row_slot = 0; /* the next batch to be named, and the slots names and rows go to (rows: by the names of that slot) */
+		auto request_names = [&]() {
+#pragma unroll
+			for (uint32_t i = 0; i < NAMES; ++i) /* (behind the last member, the last again: as many requests each time) */
+				stream_request4(sorted + begin + min(named + i * WAVE + lane, members - 1), names_at + (name_slot * NAMES + i) * (WAVE * 4));
+			named += BATCH;
+			name_slot = name_slot + 1 < SLOTS ? name_slot + 1 : 0;
+		};
+		auto request_rows = [&]() {
+			const uint32_t* names = (const uint32_t*)(stream_lds + SLOTS * STREAM_SLOT_BYTES) + row_slot * (NAMES * WAVE) + row;
+			uint32_t point[STREAM_REQUESTS];
+#pragma unroll
+			for (uint32_t j = 0; j < STREAM_REQUESTS; ++j) point[j] = names[j * ROWS];
+#pragma unroll
+			for (uint32_t j = 0; j < STREAM_REQUESTS; ++j) stream_request16((const char*)piece + (uint64_t)point[j] * row_bytes, rows_at + row_slot * STREAM_SLOT_BYTES + j * (WAVE * 16));
+			row_slot = row_slot + 1 < SLOTS ? row_slot + 1 : 0;
+		};
+		if (members <= AHEAD * BATCH) { /* all of it at once, and no more requests than there are members for */
+			for (uint32_t i = 0; i * WAVE < members; ++i) stream_request4(sorted + begin + min(i * WAVE + lane, members - 1), names_at + i * (WAVE * 4));
+			asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+			const uint32_t* names = (const uint32_t*)(stream_lds + SLOTS * STREAM_SLOT_BYTES);
+			for (uint32_t j = 0; j * ROWS < members; ++j)
+				stream_request16((const char*)piece + (uint64_t)names[min(j * ROWS + row, members - 1)] * row_bytes, rows_at + j * (WAVE * 16));
+			asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+			for (uint32_t first = 0; first < members; first += BATCH) __syncthreads();
+			return;
+		}
+#pragma unroll
+		for (uint32_t i = 0; i < AHEAD; ++i) request_names();
+		asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+#pragma unroll
+		for (uint32_t i = 0; i < AHEAD; ++i) { request_names(); request_rows(); }
+#pragma unroll 1
+		for (uint32_t first = 0; first < members; first += BATCH) {
+			/* the rows of this batch and the names of the one requested now are here (what was requested after them may not be) */
+			asm volatile("s_waitcnt vmcnt(%0)" : : "n"((AHEAD - 1) * EACH) : "memory");
+			__syncthreads(); /* the rows may be added, and those of the batch before have been */
+			request_names();
+			request_rows();
+		}
+		asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); /* (nothing may arrive in LDS that is no longer this work-group's) */
+		return;
+	}
+	F sum = (F)0;
+	const uint32_t own = min(lane, width - 1); /* this lane's coordinate */
+	uint32_t from = 0;
+#pragma unroll 1
+	for (uint32_t first = 0; first < members; first += BATCH) {
+		__syncthreads();
+		const F* mine = (const F*)(stream_lds + from * STREAM_SLOT_BYTES) + own;
+		from = from + 1 < SLOTS ? from + 1 : 0;
+		/* parts of a request's rows, the next part read while one is added (a part behind the last row is read, not added) */
+		constexpr uint32_t PART = ROWS <= 16 ? ROWS : ROWS % 16 == 0 ? 16 : 7, PARTS = ROWS / PART;
+		static_assert(ROWS % PART == 0, "whole parts");
+		F x[2][PART];
+		auto read = [&](F (&into)[PART], uint32_t at) {
+#pragma unroll
+			for (uint32_t r = 0; r < PART; ++r) into[r] = mine[at / PARTS * (WAVE * PIECE) + (at % PARTS * PART + r) * (P * PIECE)];
+		};
+		read(x[0], 0);
+		if (first + BATCH <= members) {
+#pragma unroll
+			for (uint32_t at = 0; at < STREAM_REQUESTS * PARTS; ++at) {
+				if (at + 1 < STREAM_REQUESTS * PARTS) read(x[(at + 1) % 2], at + 1);
+				__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+				for (uint32_t r = 0; r < PART; ++r) sum = sum + x[at % 2][r];
+				__builtin_amdgcn_sched_barrier(0);
+			}
+		}
+		else {
+			const uint32_t here = members - first;
+#pragma unroll 1
+			for (uint32_t at = 0; at * PART < here; at += 2) {
+#pragma unroll
+				for (uint32_t u = 0; u < 2; ++u) {
+					read(x[(u + 1) % 2], min(at + u + 1, STREAM_REQUESTS * PARTS - 1));
+					__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+					for (uint32_t r = 0; r < PART; ++r) sum = (at + u) * PART + r < here ? sum + x[u][r] : sum;
+					__builtin_amdgcn_sched_barrier(0);
+				}
+			}
+		}
+	}
+	if (lane < width) means[elem<LM>(stride_means, c, d0 + lane)] = !divide ? sum : (members ? sum / (F)members : (F)0);
+}
+
 /* Work-groups of one wavefront: what bounds this kernel is the number of cache lines a compute unit keeps in flight, so
  * the chains are spread over as many compute units as there are wavefronts (measured at N = 2M, d = 32, k = 1024: 32
  * work-groups of four wavefronts with 16-byte pieces 0.85 ms). The 16-byte pieces, which need a quarter of the lanes, are
@@ -351,6 +482,30 @@ static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sort
                               F* means, size_t stride_means, uint32_t dim, uint32_t k, uint32_t n, bool divide, const DeviceInfo& dev)
 {
 	constexpr int WIDE = 16 / sizeof(F);
+	/* (all of an iteration, us, the kernels below -> this: N = 2M, d = 32, k = 1024 421 -> 332; d = 16, k = 16, half of the points in one cluster 2669 -> 1504; N = 30k,
+	 * d = 512, k = 512 167 -> 109; N = 40k, d = 32, k = 1024 57 -> 51; N = 10240, d = 20, k = 128 29.8 -> 29.4; N = 20k, d = 100, k = 1000 75 -> 79; rows of
+	 * a piece or two: N = 1M, d = 4, k = 4096 194 -> 191, N = 270k 127 -> 131) */
+	if constexpr (LD == KMX_AOS) {
+		const uint32_t stream_dims = STREAM_BLOCK_BYTES / sizeof(F), stream_blocks = (dim + stream_dims - 1) / stream_dims;
+		if (dim % WIDE == 0 && stride % WIDE == 0 && stride <= 0xFFFFFFFFu / sizeof(F) && ((uintptr_t)data & 15) == 0 && n / k >= (dim / WIDE <= 2 ? 128u : 32u) && (uint64_t)k * stream_blocks <= 0x7FFFFFFFu) {
+			const uint32_t pieces = std::min<uint32_t>(dim / WIDE, STREAM_BLOCK_BYTES / 16);
+			const bool deep = (uint64_t)k * stream_blocks <= 2 * dev.compute_units;
+			void (*kernel)(const F*, size_t, const uint32_t*, const uint32_t*, const uint32_t*, F*, size_t, uint32_t, uint32_t, uint32_t) = nullptr;
+			uint32_t lds = 0;
+			auto take = [&](auto tag) {
+				constexpr uint32_t P = decltype(tag)::value;
+				if (pieces != P) return;
+				kernel = deep ? ordered_stream_sum_kernel<F, LM, P, true> : ordered_stream_sum_kernel<F, LM, P, false>;
+				lds = stream_lds_bytes(P, deep);
+			};
+			take(std::integral_constant<uint32_t, 1>{}); take(std::integral_constant<uint32_t, 2>{}); take(std::integral_constant<uint32_t, 3>{}); take(std::integral_constant<uint32_t, 4>{});
+			take(std::integral_constant<uint32_t, 5>{}); take(std::integral_constant<uint32_t, 6>{}); take(std::integral_constant<uint32_t, 7>{}); take(std::integral_constant<uint32_t, 8>{});
+			KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+			KMX_LAUNCH_KERNEL(kernel, dim3(k * stream_blocks), dim3(2 * WAVE), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, stream_blocks, divide ? 1u : 0u);
+			KMX_LAUNCH_CHECK("ordered_stream_sum_kernel");
+			return KMX_OK;
+		}
+	}
 	/* Clusters of a few dozen members leave a work-group of eight wavefronts nothing to overlap, the more so the more clusters there are
 	 * (all of the update, us, staged and not: N = 80k, d = 32, k = 1024 31, 37; N = 40k 31, 30; d = 4, k = 4096: N = 1M 114, 116; N = 270k 77, 64).
 	 * Blocks of 32 coordinates are whole cache lines; of 16, twice as many work-groups and half the pieces per member, which long

@@ -42,3 +42,41 @@ def test_staged_sums_have_the_bits_of_the_serial_loop(km, gpu, dim, k, dtype):
             assert np.array_equal(got, want), "layouts %d/%d: %d differ" % (layout, layout_means, int((got != want).sum()))
         d.free()
     a.free(); m.free(); s.free()
+
+
+@pytest.mark.parametrize("dtype,dim", [(np.float32, d) for d in (4, 8, 12, 16, 20, 24, 28, 32, 36, 64, 100)] + [(np.float64, d) for d in (2, 6, 10, 14, 16, 18, 50)])
+@pytest.mark.parametrize("k", [5, 600])
+def test_streamed_sums_have_the_bits_of_the_serial_loop(km, gpu, dim, k, dtype):
+    """Rows of whole 16-byte pieces (ordered_stream_sum_kernel): clusters at the edges of requests, of batches and of what is requested
+    at once, few chains (more of them ahead) and many."""
+    rng = np.random.default_rng(dim + k)
+    rows_of = 64 // min(8, dim * np.dtype(dtype).itemsize // 16)  # of a request; a batch is eight, three to six batches travel ahead
+    edges = [0, 1, rows_of - 1, rows_of, rows_of + 1] + [8 * rows_of * b + o for b in (1, 3, 4, 6, 7) for o in (-1, 0, 1)]
+    sizes = (edges if k > 5 else [0, 3 * rows_of + 1, 24 * rows_of, 48 * rows_of + 1, 130 * rows_of + 7])
+    sizes = sizes + [140] * (k - len(sizes))
+    which = rng.permutation(np.repeat(np.arange(k), sizes)).astype(np.uint32)
+    n = len(which)
+    which[5:n:97] = k  # not a cluster: left out
+    rows = (rng.normal(size=(n, dim)) * np.exp(rng.normal(size=(n, 1)) * 4)).astype(dtype)
+    want = np.zeros((k, dim), dtype)
+    order = np.argsort(which, kind="stable")
+    ends = np.cumsum(np.bincount(which, minlength=k + 1))
+    for c in range(k):
+        members = rows[order[ends[c - 1] if c else 0:ends[c]]]
+        if len(members):
+            want[c] = np.cumsum(np.concatenate([np.zeros((1, dim), dtype), members]), axis=0, dtype=dtype)[-1] / dtype(len(members))
+    size = np.dtype(dtype).itemsize
+    a = km.DeviceBuffer(4 * n); a.write(which)
+    m = km.DeviceBuffer(size * k * dim); s = km.DeviceBuffer(4 * k)
+    for pad, layout_means in [(0, 0), (16 // size, 1)]:
+        data = np.full((n, dim + pad), np.nan, dtype)
+        data[:, :dim] = rows
+        d = km.DeviceBuffer(data.nbytes); d.write(data.ravel())
+        km.update(km.UPDATE_SERIAL_ORDER, d, 0, dim + pad, a, m, layout_means, km.layout_stride(layout_means, k, dim), s, dim, k, n, dtype=dtype)
+        km.sync()
+        got = m.read(dtype, k * dim)
+        got = got.reshape(k, dim) if layout_means == 0 else got.reshape(dim, k).T
+        d.free()
+        assert np.array_equal(s.read(np.uint32, k), np.bincount(which[which < k], minlength=k))
+        assert np.array_equal(got, want), "pad %d: %d differ" % (pad, int((got != want).sum()))
+    a.free(); m.free(); s.free()
