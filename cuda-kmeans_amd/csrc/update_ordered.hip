@@ -6,7 +6,7 @@
  * addition is not associative, so only that very order gives those very bits -- but the order only matters INSIDE a
  * cluster and coordinate: the k x dim chains are independent. This variant therefore
  *   1. sorts the point numbers by cluster with a STABLE counting sort (points of one cluster stay in ascending order):
- *      per-chunk histograms -> exclusive scan over (cluster, chunk) -> every chunk, one wavefront, walks its points in
+ *      per-chunk histograms -> exclusive scan over (cluster, chunk) -> a wavefront per chunk (or part of one) walks its points in
  *      order, 64 at a time, and ranks the lanes that share a cluster by their lane number (ballots, no returning
  *      atomics, whose order would be arbitrary);
  *   2. gives every (cluster, coordinate) chain to one lane, which adds the rows of the sorted list one after the other
@@ -15,7 +15,7 @@
  * reference's serial run. The price is the length of the longest chain: a cluster of m members is m dependent
  * additions, whatever the machine.
  *
- * Kernels: ordered_histogram_kernel, ordered_offsets_kernel, ordered_starts_kernel, ordered_scatter_kernel,
+ * Kernels: ordered_histogram_kernel, ordered_offsets_kernel, ordered_starts_kernel, ordered_scatter_kernel / ordered_scatter_group_kernel,
  * ordered_stream_sum_kernel / ordered_staged_sum_kernel / ordered_sum_kernel.
  */
 #include "kmx_internal.h"
@@ -28,35 +28,43 @@ namespace kmx {
 constexpr uint32_t ORDERED_LDS_CLUSTERS = 16384; /* up to here a chunk's counters live in LDS (64 KB per wavefront-sized work-group) */
 constexpr uint32_t ORDERED_HIST_WORDS = 1u << 21; /* bound of chunks x k */
 constexpr uint32_t ORDERED_MAX_CHUNKS = 4096;
+/* wavefronts that share a chunk's row of the histogram, each with counters of its own in LDS while it scatters: 64 KB of them at most */
+constexpr uint32_t ordered_group(uint32_t k) { return k <= 2048 ? 8 : k <= 4096 ? 4 : 1; }
 
 /*
- * Histogram of one chunk of points: hist[chunk][cluster]. One wavefront per chunk, the same chunks as the scatter.
- * IN_LDS: counters in LDS, the row is written out whole (nothing to clear beforehand); otherwise the row in global
+ * Histogram of one chunk of points: hist[chunk][cluster]. One work-group per chunk, the same chunks as the scatter.
+ * IN_LDS: counters in LDS, the row is written out whole (nothing to clear beforehand); otherwise (one wavefront) the row in global
  * memory is the counter array (cleared by the launcher) and takes the atomics directly -- it belongs to this wavefront,
  * but two lanes may hold the same cluster.
  */
 template <bool IN_LDS>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(512)
 ordered_histogram_kernel(const uint32_t* __restrict__ assignment, uint32_t* __restrict__ hist, uint32_t k, uint32_t n, uint32_t chunk_points)
 {
 	extern __shared__ uint32_t counters[];
-	const uint32_t lane = threadIdx.x;
+	const uint32_t tid = threadIdx.x, threads = blockDim.x;
 	uint32_t* row = hist + (size_t)blockIdx.x * k;
-	if (IN_LDS) {
-		for (uint32_t c = lane; c < k; c += WAVE) counters[c] = 0u;
-		__syncthreads();
-	}
 	const uint32_t begin = blockIdx.x * chunk_points;          /* chunks * chunk_points < 2^32: the launcher keeps n below 2^32 - 2^20 */
 	const uint32_t end = min(n, begin + chunk_points);
-	for (uint32_t i = begin + lane; i < end; i += WAVE) {
-		const uint32_t c = assignment[i];
-		if (c >= k) continue; /* not a cluster: the point is left out, as by the scatter */
-		if (IN_LDS) atomicAdd(&counters[c], 1u);
-		else atomicAdd(&row[c], 1u);
+	if (IN_LDS) {
+		for (uint32_t c = tid; c < k; c += threads) counters[c] = 0u;
+		__syncthreads();
+	}
+	constexpr uint32_t BATCH = 8; /* loads in flight */
+	for (uint32_t i0 = begin + tid; i0 < end; i0 += BATCH * threads) {
+		uint32_t c[BATCH];
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u) c[u] = i0 + u * threads < end ? assignment[i0 + u * threads] : 0xFFFFFFFFu;
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u) {
+			if (c[u] >= k) continue; /* not a cluster: the point is left out, as by the scatter */
+			if (IN_LDS) atomicAdd(&counters[c[u]], 1u);
+			else atomicAdd(&row[c[u]], 1u);
+		}
 	}
 	if (IN_LDS) {
 		__syncthreads();
-		for (uint32_t c = lane; c < k; c += WAVE) row[c] = counters[c];
+		for (uint32_t c = tid; c < k; c += threads) row[c] = counters[c];
 	}
 }
 
@@ -200,6 +208,84 @@ ordered_scatter_kernel(const uint32_t* __restrict__ assignment, uint32_t* __rest
 			}
 		}
 		if (!IN_LDS) __threadfence();
+	}
+}
+
+/*
+ * The same by work-groups of GROUP wavefronts, which share a row of the histogram: each counts its part of the chunk first (so there is an
+ * eighth of the rows to write, scan and read; N = 2M, k = 1024, us, a row per wavefront -> this: counting 11 -> 4.6, scanning 13 -> 4.9, starts 4.7 -> 0, scattering
+ * 29 -> 18) and starts behind the wavefronts before it. Every work-group finds the clusters' starts for itself from their sizes, the first one leaves them for the sums.
+ * Neighbouring chunks go to the same XCD, whose L2 then holds whole lines of the sorted list before they are written back.
+ */
+template <uint32_t GROUP>
+__global__ void __launch_bounds__(GROUP * WAVE)
+ordered_scatter_group_kernel(const uint32_t* __restrict__ assignment, const uint32_t* __restrict__ hist, const uint32_t* __restrict__ sizes, uint32_t* __restrict__ starts,
+                             uint32_t* __restrict__ sorted, uint32_t k, uint32_t n, uint32_t chunk_points)
+{
+	constexpr uint32_t THREADS = GROUP * WAVE, XCDS = 8;
+	extern __shared__ uint32_t counters[]; /* GROUP rows of k */
+	__shared__ uint32_t wave_sum[GROUP];
+	const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	const uint32_t xcd = blockIdx.x % XCDS, chunk = xcd * (gridDim.x / XCDS) + min(xcd, gridDim.x % XCDS) + blockIdx.x / XCDS;
+	const uint32_t* row = hist + (size_t)chunk * k;
+	const uint32_t part = chunk_points / GROUP; /* (whole steps of 64 points) */
+	const uint32_t begin = min(n, chunk * chunk_points + wave * part), end = min(n, begin + part);
+	/* this lane's share of the clusters: neighbours */
+	const uint32_t each = (k + THREADS - 1) / THREADS, c0 = min(k, tid * each), c1 = min(k, c0 + each);
+	uint32_t members = 0;
+	for (uint32_t c = c0; c < c1; ++c) members += sizes[c];
+	for (uint32_t c = tid; c < GROUP * k; c += THREADS) counters[c] = 0u;
+	uint32_t upto = members; /* inclusive within the wavefront */
+#pragma unroll
+	for (uint32_t off = 1; off < WAVE; off <<= 1) {
+		const uint32_t below = (uint32_t)__shfl_up((int)upto, off);
+		if (lane >= off) upto += below;
+	}
+	if (lane == WAVE - 1) wave_sum[wave] = upto;
+	__syncthreads();
+	uint32_t* next = counters + wave * k;
+	constexpr uint32_t BATCH = 8; /* loads in flight */
+	for (uint32_t i0 = begin + lane; i0 < end; i0 += BATCH * WAVE) {
+		uint32_t c[BATCH];
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u) c[u] = i0 + u * WAVE < end ? assignment[i0 + u * WAVE] : 0xFFFFFFFFu;
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u)
+			if (c[u] < k) atomicAdd(&next[c[u]], 1u);
+	}
+	__syncthreads();
+	uint32_t start = upto - members;
+	for (uint32_t v = 0; v < wave; ++v) start += wave_sum[v];
+	for (uint32_t c = c0; c < c1; ++c) {
+		if (chunk == 0) starts[c] = start;
+		uint32_t running = start + row[c];
+		start += sizes[c];
+#pragma unroll
+		for (uint32_t v = 0; v < GROUP; ++v) {
+			const uint32_t count = counters[v * k + c];
+			counters[v * k + c] = running;
+			running += count;
+		}
+	}
+	__syncthreads();
+	const unsigned long long below = (1ull << lane) - 1ull;
+	const uint32_t bits = 32 - (uint32_t)__builtin_clz(k - 1 | 1u);
+	uint32_t cluster = begin + lane < end ? assignment[begin + lane] : 0xFFFFFFFFu;
+	for (uint32_t base = begin; base < end; base += WAVE) {
+		const uint32_t i = base + lane, c = cluster;
+		if (base + WAVE < end) cluster = i + WAVE < end ? assignment[i + WAVE] : 0xFFFFFFFFu; /* of the next step */
+		unsigned long long same = __ballot(c < k);
+		for (uint32_t bit = 0; bit < bits; ++bit) {
+			const bool set = (c >> bit) & 1u;
+			const unsigned long long with = __ballot(set);
+			same &= set ? with : ~with;
+		}
+		const uint32_t rank = (uint32_t)__popcll(same & below), group = (uint32_t)__popcll(same);
+		if (c < k) {
+			const uint32_t slot = next[c] + rank;
+			sorted[slot] = i;
+			if (rank + 1 == group) next[c] = slot + 1;
+		}
 	}
 }
 
@@ -544,12 +630,13 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 {
 	if (n > 0xFFFFFFFFu - (1u << 20)) return fail(KMX_ERR_UNSUPPORTED, "the serial-order update takes fewer than 2^32 - 2^20 points");
 	if ((uint64_t)k * dim > 0xFFFFFFFFull * WAVE) return fail(KMX_ERR_UNSUPPORTED, "the serial-order update: k * dim is too large for one launch");
-	/* chunks: one wavefront each, a multiple of 64 points, few enough that chunks x k counters stay small */
+	/* chunks: `group` wavefronts each, a multiple of 64 points per wavefront, few enough that chunks x k counters stay small */
+	const uint32_t group = ordered_group(k);
 	uint32_t chunks = 0, chunk_points = WAVE;
 	if (n > 0) {
 		const uint32_t by_memory = std::max<uint32_t>(1, ORDERED_HIST_WORDS / k);
-		chunks = std::min<uint32_t>({ by_memory, ORDERED_MAX_CHUNKS, (n + 255) / 256 });
-		chunk_points = ((n + chunks - 1) / chunks + WAVE - 1) / WAVE * WAVE;
+		chunks = (std::min<uint32_t>({ by_memory, ORDERED_MAX_CHUNKS, (n + 255) / 256 }) + group - 1) / group;
+		chunk_points = ((n + chunks - 1) / chunks + group * WAVE - 1) / (group * WAVE) * (group * WAVE);
 		chunks = (n + chunk_points - 1) / chunk_points;
 	}
 	const size_t hist_words = (size_t)std::max(chunks, 1u) * k;
@@ -574,7 +661,7 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 	if (chunks > 0) {
 		if (in_lds) {
 			KMX_HIP(hipFuncSetAttribute((const void*)ordered_histogram_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-			KMX_LAUNCH_KERNEL((ordered_histogram_kernel<true>), dim3(chunks), dim3(WAVE), lds_bytes, stream(), assignment, hist, k, n, chunk_points);
+			KMX_LAUNCH_KERNEL((ordered_histogram_kernel<true>), dim3(chunks), dim3(group * WAVE), lds_bytes, stream(), assignment, hist, k, n, chunk_points);
 		}
 		else {
 			rc = kmx_fill_zero_u32(hist, hist_words);
@@ -585,10 +672,17 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 	}
 	KMX_LAUNCH_KERNEL(ordered_offsets_kernel, dim3((k + SCAN_COLUMNS - 1) / SCAN_COLUMNS), dim3(SCAN_COLUMNS * SCAN_SHARES), 0, stream(), hist, cluster_sizes, k, chunks);
 	KMX_LAUNCH_CHECK("ordered_offsets_kernel");
-	KMX_LAUNCH_KERNEL(ordered_starts_kernel, dim3(1), dim3(1024), 0, stream(), cluster_sizes, starts, k);
-	KMX_LAUNCH_CHECK("ordered_starts_kernel");
+	if (group == 1 || chunks == 0) {
+		KMX_LAUNCH_KERNEL(ordered_starts_kernel, dim3(1), dim3(1024), 0, stream(), cluster_sizes, starts, k);
+		KMX_LAUNCH_CHECK("ordered_starts_kernel");
+	}
 	if (chunks > 0) {
-		if (in_lds) {
+		if (group > 1) {
+			auto kernel = group == 8 ? ordered_scatter_group_kernel<8> : ordered_scatter_group_kernel<4>;
+			KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(group * lds_bytes)));
+			KMX_LAUNCH_KERNEL(kernel, dim3(chunks), dim3(group * WAVE), group * lds_bytes, stream(), assignment, hist, cluster_sizes, starts, sorted, k, n, chunk_points);
+		}
+		else if (in_lds) {
 			KMX_HIP(hipFuncSetAttribute((const void*)ordered_scatter_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
 			KMX_LAUNCH_KERNEL((ordered_scatter_kernel<true>), dim3(chunks), dim3(WAVE), lds_bytes, stream(), assignment, hist, starts, sorted, k, n, chunk_points);
 		}

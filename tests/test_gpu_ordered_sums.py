@@ -80,3 +80,28 @@ def test_streamed_sums_have_the_bits_of_the_serial_loop(km, gpu, dim, k, dtype):
         assert np.array_equal(s.read(np.uint32, k), np.bincount(which[which < k], minlength=k))
         assert np.array_equal(got, want), "pad %d: %d differ" % (pad, int((got != want).sum()))
     a.free(); m.free(); s.free()
+
+
+@pytest.mark.parametrize("k,n", [(1, 1), (1, 5000), (2, 63), (7, 513), (2048, 9001), (2049, 9001), (4096, 20003), (4097, 20003), (16384, 40001), (16385, 40001), (1000, 300007)])
+def test_members_are_added_in_point_order(km, gpu, k, n):
+    """The stable sort by work-groups of eight, four and one wavefronts, counters in LDS and in memory."""
+    rng = np.random.default_rng(k + n)
+    which = np.minimum(rng.integers(0, k + 1, n), rng.integers(0, k + 1, n)).astype(np.uint32)  # (k: not a cluster)
+    rows = (rng.normal(size=(n, 4)) * np.exp(rng.normal(size=(n, 1)) * 4)).astype(np.float32)
+    want = np.zeros((k, 4), np.float32)
+    for i in np.flatnonzero(which < k) if n < 50000 else []:
+        want[which[i]] += rows[i]
+    if n >= 50000:
+        for c in range(k):
+            want[c] = np.cumsum(np.concatenate([np.zeros((1, 4), np.float32), rows[which == c]]), axis=0, dtype=np.float32)[-1]
+    counts = np.bincount(which[which < k], minlength=k)
+    want = np.where(counts[:, None] > 0, want / np.maximum(counts, 1)[:, None].astype(np.float32), np.float32(0))
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * n); a.write(which)
+    m = km.DeviceBuffer(16 * k); s = km.DeviceBuffer(4 * k)
+    km.update(km.UPDATE_SERIAL_ORDER, d, 0, 4, a, m, 0, 4, s, 4, k, n)
+    km.sync()
+    assert np.array_equal(s.read(np.uint32, k), counts)
+    assert np.array_equal(m.read(np.float32, 4 * k).reshape(k, 4), want)
+    for b in (d, a, m, s):
+        b.free()
