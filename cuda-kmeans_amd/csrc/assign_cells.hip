@@ -22,6 +22,12 @@ namespace kmx {
 
 constexpr float CELL_SLACK = 1e-5f;
 constexpr float CELL_MARGIN = 1e-3f;
+/*
+ * A centroid whose square, by fused multiply-adds, is less than 1 / CELL_CLEAR of all the others' is the serial scan's: both sums of squares are of the
+ * same differences and off by at most 4 x 2^-24 each, so the serial ones differ by more than (33 - 4 x 4) 2^-24 of themselves, and their
+ * square roots by more than a rounding (2 x 2^-24 of the square).
+ */
+constexpr float CELL_CLEAR = 1.000002f;
 constexpr uint32_t CELL_MAX_K = 6144;              /* what the building kernel's LDS holds */
 constexpr uint32_t CELL_UNIT = 8;                  /* entries (16 bits) of a list that are read together */
 constexpr uint32_t CELL_POOL_UNITS = 1u << 20;
@@ -374,22 +380,20 @@ build_cells_kernel(const CellArgs w)
 	if (listed && wave < MIDS) {
 		uint16_t* out = w.pool + (size_t)start * CELL_UNIT;
 		uint32_t to = before;
-		uint16_t last = 0;
 		kept &= ~(1ull << 63);
 		while (kept) {
-			last = second_list[i0 + (uint32_t)__builtin_ctzll(kept)];
-			out[to++] = last;
+			out[to++] = second_list[i0 + (uint32_t)__builtin_ctzll(kept)];
 			kept &= kept - 1;
 		}
 		for (uint32_t i = i0 + 63; i < i1; ++i) {
 			const uint16_t j = second_list[i];
 			float least, most;
 			measure(j, lo, hi, least, most);
-			if (least <= bound) { out[to++] = j; last = j; }
+			if (least <= bound) out[to++] = j;
 		}
-		/* the lane with the cell's last entry fills the last unit up with it */
+		/* the lane with the cell's last entry fills the last unit up, with the row behind the last centroid (which is infinitely far) */
 		if (count > 0 && to == total)
-			for (; to < units * CELL_UNIT; ++to) out[to] = last;
+			for (; to < units * CELL_UNIT; ++to) out[to] = (uint16_t)w.k;
 	}
 }
 
@@ -408,23 +412,29 @@ constexpr uint32_t CELL_THREADS = 1024;
 constexpr uint32_t CELL_WAVES = CELL_THREADS / WAVE;
 constexpr uint32_t CHOICE_EACH = 2, CHOICE_GROUPS = CHOICE_EACH * CELL_WAVES; /* groups of 64 points that the choice between cells and sweep looks at */
 constexpr uint32_t CELL_LIST = 64; /* points per wavefront that wait for the list */
-constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* LDS of assign_cells_kernel beside the centroids */
+constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* LDS of assign_cells_kernel beside the centroids: the infinite row, flag_list, wave_max */
 
 /*
- * A lane per point, the centroids in LDS. What bounds it: the vector ALU, which takes a wavefront through the longest list of its 64 points (N = 4M,
- * d = 4, k = 4096, uniform points: 77 M vector instructions fill the issue slots of the 104 to 114 us; lists of 29 entries on average, the longest
- * of a wavefront 70, so more than half of the lanes idle). Two work-groups share a compute unit, eight wavefronts
- * a SIMD: with more than 80 scalar registers (and the 16 the hardware adds) only seven fit, which is one work-group (d = 3, k = 4096,
- * normal points: 162 -> 220 us).
+ * A lane per point, the centroids in LDS. What bounds it: the gathers from LDS (N = 4M, d = 4, k = 4096, uniform points: a wavefront goes through
+ * the longest list of its 64 points, 70 entries of 29 on average, and 16 bytes at 64 unrelated addresses take 11 cycles with their bank conflicts:
+ * 179 000 of the 227 000 cycles of a compute unit), then the vector ALU. A comparison is 13 instructions and no branch: the sums are fused, the
+ * two smallest are kept (one v_med3), and the few points whose two smallest are not CELL_CLEAR of each other go through their list again in the
+ * serial arithmetic. Against that arithmetic for all, with its branches (17 instructions, and each row waited for by itself): 122 -> 112 us;
+ * normal points, d = 4, k = 1000: 246 -> 216 us per call; d = 3, k = 6000: 119 -> 108 us; points and centroids on a lattice of 16^4 places, nearly
+ * all of them ties: 178 -> 228 us. Sorting a wavefront's 256 points by the length of their lists takes a quarter of the instructions out, but
+ * fuller wavefronts have more bank conflicts: 122 -> 136 us. Two work-groups share a compute unit, eight wavefronts
+ * a SIMD, which takes 64 vector registers; with more than 80 scalar registers (and the 16 the hardware adds) only seven fit, which is one
+ * work-group (d = 3, k = 4096, normal points: 162 -> 220 us).
  */
 template <int D, int LD, int LM>
-__global__ void __launch_bounds__(CELL_THREADS) __attribute__((amdgpu_num_sgpr(80)))
+__global__ void __launch_bounds__(CELL_THREADS) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8)))
 assign_cells_kernel(const CellAssignArgs w)
 {
 	constexpr uint32_t N = cells_per_dim<D>();
-	extern __shared__ __attribute__((aligned(16))) float lds[]; /* k x 4 */
-	__shared__ uint32_t wave_max[6][CELL_WAVES];
-	__shared__ uint32_t flag_list[CELL_WAVES][2 * CELL_LIST];
+	extern __shared__ __attribute__((aligned(16))) float lds[]; /* (k + 1) x 4 */
+	/* (all of it is dynamic, so a row's address is 16 times its number) */
+	uint32_t (*const wave_max)[CELL_WAVES] = (uint32_t (*)[CELL_WAVES])(lds + 4 * (w.k + 1));
+	uint32_t (*const flag_list)[2 * CELL_LIST] = (uint32_t (*)[2 * CELL_LIST])(wave_max + 6);
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 	const float scale = w.scale[0];
@@ -460,6 +470,7 @@ assign_cells_kernel(const CellAssignArgs w)
 		for (int q = 0; q < D; ++q) c[q] = w.means[elem<LM>(w.stride_means, j, q)];
 		*(f32x4*)(lds + 4 * j) = c;
 	}
+	if (tid < 4) lds[4 * w.k + tid] = __builtin_inff();
 	/* the maxima of the certificate; the first work-group leaves them and those of the exact pass's own (rank16_leave_bounds) */
 	uint32_t most[6] = { 0u, 0u, 0u, 0u, 0u, 0u }; /* of |c|^2, low^2, mid^2, rest^2; then two sums: entries, points without a list */
 	for (uint32_t j = tid; j < w.k; j += CELL_THREADS) {
@@ -531,10 +542,9 @@ assign_cells_kernel(const CellAssignArgs w)
 		const uint32_t units = (entry >> 20) & CELL_MOST_UNITS;
 		const uint4* list = (const uint4*)w.pool + (entry & 0xFFFFFu);
 		float best = __builtin_inff();
-		uint32_t winner = 0;
-		auto compare = [&](uint32_t j) {
+		uint32_t winner = 0; /* as an LDS address */
+		auto compare = [&](const f32x4& c, uint32_t at) {
 #pragma clang fp contract(off)
-			const f32x4 c = *(const f32x4*)(lds + 4 * j);
 			float sum = 0.0f;
 #pragma unroll
 			for (int q = 0; q < D; ++q) {
@@ -543,19 +553,52 @@ assign_cells_kernel(const CellAssignArgs w)
 				sum = sum + sq;
 			}
 			/* the serial scan compares square roots: a smaller square may have the same one */
-			if (sum < best && (sum < best * 0.9999995f || __builtin_sqrtf(sum) < __builtin_sqrtf(best))) { best = sum; winner = j; }
+			if (sum < best && (sum < best * 0.9999995f || __builtin_sqrtf(sum) < __builtin_sqrtf(best))) { best = sum; winner = at; }
 		};
-		uint4 next = list[0];
-		for (uint32_t u = 0; u < units; ++u) {
-			const uint4 now = next;
-			next = list[min(u + 1, units - 1)];
-			compare(now.x & 0xFFFFu); compare(now.x >> 16);
-			compare(now.y & 0xFFFFu); compare(now.y >> 16);
-			compare(now.z & 0xFFFFu); compare(now.z >> 16);
-			compare(now.w & 0xFFFFu); compare(now.w >> 16);
-		}
-		if (mine) w.assignment[pt] = winner;
+		auto walk = [&](auto&& take) {
+			uint4 next = list[0];
+			for (uint32_t u = 0; u < units; ++u) {
+				const uint4 now = next;
+				next = list[min(u + 1, units - 1)];
+				asm volatile("" ::: "memory"); /* (the next unit is requested here, not where it is used) */
+				const uint32_t word[4] = { now.x, now.y, now.z, now.w };
+#pragma unroll
+				for (uint32_t h = 0; h < 4; h += 2) {
+					uint32_t at[4]; /* LDS addresses: 16 times an entry */
+					f32x4 c[4];
+#pragma unroll
+					for (uint32_t i = 0; i < 4; ++i) {
+						if (i % 2) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=v"(at[i]) : "v"(4u), "v"(word[h + i / 2]));
+						else asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(at[i]) : "v"(4u), "v"(word[h + i / 2]));
+						c[i] = *(const __attribute__((address_space(3))) f32x4*)at[i];
+					}
+					asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])); /* (all four are on their way before the first is used) */
+#pragma unroll
+					for (uint32_t i = 0; i < 4; ++i) take(c[i], at[i]);
+				}
+			}
+		};
+		float second = __builtin_inff();
+		walk([&](const f32x4& c, uint32_t at) {
+			float sum = 0.0f;
+#pragma unroll
+			for (int q = 0; q < D; ++q) {
+				const float diff = x[q] - c[q];
+				sum = q ? __builtin_fmaf(diff, diff, sum) : diff * diff;
+			}
+			second = __builtin_amdgcn_fmed3f(sum, best, second);
+			const bool less = sum < best;
+			best = less ? sum : best;
+			winner = less ? at : winner;
+		});
 		const bool flag = mine && (!inside || (entry & CELL_TRUNCATED));
+		/* (a flagged point's distance becomes its threshold: the serial one, as ever; smaller squares may have lost bits) */
+		if (flag || !(best > 1e-30f && second > best * CELL_CLEAR)) {
+			best = __builtin_inff();
+			winner = 0;
+			walk(compare);
+		}
+		if (mine) w.assignment[pt] = winner / 16;
 		const unsigned long long mask = __ballot(flag);
 		if (mask) {
 			const uint32_t add = (uint32_t)__popcll(mask);
@@ -634,7 +677,7 @@ static int launch_cells_d(const AssignArgs& a, kmx_exec_params* exec, Workspace*
 	                           a.assignment, ws->listed, ws->counters, a.k, half.kp, a.n, choose ? 1u : 0u, half.kd };
 	void (*assign)(CellAssignArgs) = a.layout == KMX_AOS ? (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_AOS, KMX_AOS> : assign_cells_kernel<D, KMX_AOS, KMX_SOA>)
 	                                                     : (a.layout_means == KMX_AOS ? assign_cells_kernel<D, KMX_SOA, KMX_AOS> : assign_cells_kernel<D, KMX_SOA, KMX_SOA>);
-	const uint32_t lds = a.k * 16, per_cu = std::max<uint32_t>(1, std::min<uint32_t>(2, dev.lds_bytes / (lds + CELL_STATIC)));
+	const uint32_t lds = a.k * 16 + CELL_STATIC, per_cu = std::max<uint32_t>(1, std::min<uint32_t>(2, dev.lds_bytes / lds));
 	const uint32_t blocks = std::min((a.n + CELL_THREADS - 1) / CELL_THREADS, per_cu * dev.compute_units);
 	exec->block_count = blocks;
 	if ((rc = profile_begin(0))) return rc; /* (ended behind the packed sweep: one of the two does the work) */

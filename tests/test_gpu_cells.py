@@ -62,6 +62,35 @@ def test_cells_match_the_oracle(km, orc, gpu, dim, k, n, kind):
     a.free()
 
 
+@pytest.mark.parametrize("dim,k", [(2, 2), (2, 130), (2, 4094), (3, 130), (3, 2000), (4, 64), (4, 4096)])
+def test_near_ties_are_told_apart_as_the_serial_scan_does(km, orc, gpu, dim, k):
+    """Pairs of centroids, and points whose squared distances to both differ by 0 to some 1e-5 of themselves: on either side of what the
+    fused sums decide by themselves."""
+    rng = np.random.default_rng(dim * 7 + k)
+    first = rng.uniform(0, 1, size=(k // 2, dim))
+    apart = rng.normal(size=(k // 2, dim))
+    apart *= 0.3 / k ** (1 / dim) / np.linalg.norm(apart, axis=1, keepdims=True)
+    means = np.concatenate([first, first + apart]).astype(np.float32)
+    n = 20001
+    pair = rng.integers(0, k // 2, n)
+    a, b = means[pair].astype(np.float64), means[pair + k // 2].astype(np.float64)
+    off = rng.choice([0, 1e-7, 2e-7, 5e-7, 1e-6, 2e-6], n) * rng.uniform(-1, 1, n)
+    rows = ((a + b) / 2 + (b - a) * off[:, None]).astype(np.float32)
+    want = orc.assign(rows.ravel(), means.ravel(), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    m = km.DeviceBuffer(means.nbytes); m.write(means.ravel())
+    out = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        km.assign(km.ASSIGN_MFMA_BF16X3, d, km.AOS, dim, m, km.AOS, dim, out, dim, k, n)
+        km.sync()
+    finally:
+        km.set_two_level_sweep(1)
+    got = out.read(np.uint32, n)
+    d.free(); m.free(); out.free()
+    assert np.array_equal(got, want), "%d mismatches" % int((got != want).sum())
+
+
 @pytest.mark.parametrize("kind", ["planar", "outside", "lattice", "tiny", "huge", "nan"])
 @pytest.mark.parametrize("dim,k", [(2, 600), (3, 6100), (4, 601), (4, 700)])   # (6100: streamed centroids; 600 and more: tracked per tile)
 @pytest.mark.parametrize("layout,pad", [(0, 0), (0, 3), (1, 0)])
