@@ -16,10 +16,15 @@
  * The rows of a unit are read from memory once while 512 centroids go by; with more centroids the converted rows stay in LDS
  * if they fit (d <= 512), otherwise they are staged again per group of 512.
  *
- * What bounds it: one work-group of eight wavefronts per compute unit with a barrier per 64 dimensions, the conversion of the next 64 behind
- * the matrix instructions of these (N = 131071, d = 512, k = 400: 106 us, half of the rate of a large matrix product; 13 tiles for eight wavefronts).
+ * What bounds it: latencies, between one barrier per 64 dimensions and the next, of one work-group of eight wavefronts per compute unit
+ * (N = 131071, d = 512, k = 400: 85 us; the matrix cores are busy 32 % of the time, 13 tiles for eight wavefronts; the vector ALU 46 %, half of it the
+ * search for the smallest results; the rows alone take 44 us to read). A wavefront converts its share of the next 64 dimensions piece by piece between
+ * its matrix instructions of a block, while the SIMD's other wavefront has its own under way, and the last 64 of a unit bring the first of the next one
+ * with them, so six of the eight wavefronts go on while two decide over the unit's points. With the conversion behind the 64
+ * dimensions' products, and each unit started with a conversion of its own and a barrier: 111 us; columns of points, N = 65536: 175 -> 135 us per
+ * call; k = 8, d = 257: 120 -> 101 us.
  * N = 131071, d = 512, k = 400, one iteration: the lane-per-point kernel that took these rows before needed 147 ms, two levels of bf16
- * products and a pass over the slices of the queued points (234 us of the assignment) 0.29 ms, this one 0.21 ms.
+ * products and a pass over the slices of the queued points (234 us of the assignment) 0.29 ms, this one 0.18 ms.
  */
 #include "rank16_exact_impl.h"
 
@@ -229,7 +234,7 @@ pack_means16_wide_kernel(const float* __restrict__ means, const double* __restri
  * (cert_kd_keyed): three operations per value for the two smallest and the place of the smallest. A NaN anywhere makes the smallest
  * NaN (v_minimum3_f32 passes it on), which certifies nothing.
  */
-template <int PT, int NT, bool X3, int LD, bool VEC>
+template <int PT, int NT, bool X3, int LD, bool VEC, bool RESIDENT>
 __global__ void __launch_bounds__(WIDE_THREADS)
 wide_sweep_kernel(const WideArgs w)
 {
@@ -241,7 +246,8 @@ wide_sweep_kernel(const WideArgs w)
 	constexpr uint32_t BUFFER_UNITS = (X3 ? 2 : 1) * PART_UNITS;
 	constexpr uint32_t GROUP_TILES = WIDE_WAVES * NT;
 	constexpr uint32_t KEY_MASK = NT * 16 - 1;
-	static_assert(VECS * SUBS * 4 == WIDE_CHUNK && NT <= 2, "shape");
+	constexpr uint32_t SUMS = X3 ? 3 : 2;                   /* of a row: |x|^2, the part left out; X3: (x - m) . m */
+	static_assert(VECS * SUBS * 4 == WIDE_CHUNK && NT <= 2 && SUMS * WIDE_THREADS <= BUFFER_UNITS * 4, "shape");
 
 	extern __shared__ __attribute__((aligned(16))) float dyn[];
 	float* frame = dyn;                            /* dp floats (a multiple of 64) */
@@ -264,9 +270,8 @@ wide_sweep_kernel(const WideArgs w)
 	const uint32_t groups = (tiles + GROUP_TILES - 1) / GROUP_TILES;
 	const uint32_t chunks = w.dp / WIDE_CHUNK;
 	const uint32_t blocks = w.dp / KBLOCK;
-	const bool resident = w.buffers >= chunks;
 	const uint32_t steps = groups * chunks;
-	const uint32_t staged_steps = resident ? chunks : steps;
+	const uint32_t staged_steps = RESIDENT ? chunks : steps;
 	if (blockIdx.x >= units) return; /* the whole work-group */
 
 	/* the certificate's maxima over the centroids (bit patterns: NaN and infinity win) and the frame */
@@ -305,73 +310,69 @@ wide_sweep_kernel(const WideArgs w)
 		const uint32_t slot = min(unit * ROWS + row, n - 1);
 		return slot;
 	};
-	auto request_rows = [&](uint32_t pt, uint32_t chunk) {
-#pragma unroll
-		for (uint32_t i = 0; i < VECS; ++i) {
-			const uint32_t d = chunk * WIDE_CHUNK + (i * SUBS + sub) * 4;
-			f32x4 v = { 0.0f, 0.0f, 0.0f, 0.0f };
-			/* (pieces beyond the row repeat its end: no branches around the loads; store_rows puts zeros there) */
-			if (LD == KMX_AOS) {
-				typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4))); /* 16-byte loads need no more than 4-byte alignment */
-				const float* at = w.data + (size_t)pt * w.stride + min(d, w.dim - 4);
-				if constexpr (VEC) v = *(const f32x4*)at;
-				else v = *(const f32x4_any*)at;
-			}
-			else {
-#pragma unroll
-				for (uint32_t e = 0; e < 4; ++e) v[e] = w.data[elem<LD>(w.stride, pt, min(d + e, w.dim - 1))];
-			}
-			piece[i] = v;
+	auto request_piece = [&](uint32_t i, uint32_t pt, uint32_t chunk) {
+		const uint32_t d = chunk * WIDE_CHUNK + (i * SUBS + sub) * 4;
+		f32x4 v = { 0.0f, 0.0f, 0.0f, 0.0f };
+		/* (pieces beyond the row repeat its end: no branches around the loads; store_piece puts zeros there) */
+		if (LD == KMX_AOS) {
+			typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4))); /* 16-byte loads need no more than 4-byte alignment */
+			const float* at = w.data + (size_t)pt * w.stride + min(d, w.dim - 4);
+			if constexpr (VEC) v = *(const f32x4*)at;
+			else v = *(const f32x4_any*)at;
 		}
+		else {
+#pragma unroll
+			for (uint32_t e = 0; e < 4; ++e) v[e] = w.data[elem<LD>(w.stride, pt, min(d + e, w.dim - 1))];
+		}
+		piece[i] = v;
 	};
 	float xx = 0.0f, xpart = 0.0f, xalong = 0.0f;
-	auto store_rows = [&](uint32_t buffer, uint32_t chunk, bool first_pass) {
+	auto store_piece = [&](uint32_t i, uint32_t buffer, uint32_t chunk, bool first_pass) {
 		typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 		char* base = (char*)(rows_lds + (size_t)buffer * BUFFER_UNITS);
-#pragma unroll
-		for (uint32_t i = 0; i < VECS; ++i) {
-			const uint32_t f = i * SUBS + sub;
-			const f32x4 mv = *(const f32x4*)(frame + chunk * WIDE_CHUNK + f * 4);
-			if constexpr (LD == KMX_AOS && !VEC) {
-				/* the piece that holds the end of a row whose length is no multiple of four came from up to three places before */
-				const uint32_t d = chunk * WIDE_CHUNK + f * 4;
-				if ((chunk + 1) * WIDE_CHUNK > w.dim && d + 4 > w.dim && d < w.dim) {
-					const f32x4 p = piece[i];
-					const uint32_t s = d + 4 - w.dim;
-					piece[i].x = s == 1 ? p.y : s == 2 ? p.z : p.w;
-					piece[i].y = s == 1 ? p.z : p.w;
-					piece[i].z = p.w;
-				}
+		const uint32_t f = i * SUBS + sub, d = chunk * WIDE_CHUNK + f * 4;
+		const f32x4 mv = *(const f32x4*)(frame + d);
+		if constexpr (LD == KMX_AOS && !VEC) {
+			/* the piece that holds the end of a row whose length is no multiple of four came from up to three places before */
+			if ((chunk + 1) * WIDE_CHUNK > w.dim && d + 4 > w.dim && d < w.dim) {
+				const f32x4 p = piece[i];
+				const uint32_t s = d + 4 - w.dim;
+				piece[i].x = s == 1 ? p.y : s == 2 ? p.z : p.w;
+				piece[i].y = s == 1 ? p.z : p.w;
+				piece[i].z = p.w;
 			}
-			bf16x4 hi, mid;
-			float a = 0.0f, b = 0.0f, c = 0.0f;
-#pragma unroll
-			for (int e = 0; e < 4; ++e) {
-				const bool there = chunk * WIDE_CHUNK + f * 4 + e < w.dim;
-				if constexpr (X3) {
-					const float v = there ? piece[i][e] - mv[e] : 0.0f;
-					__bf16 vh, vm;
-					split_bf16(v, vh, vm);
-					hi[e] = vh;
-					mid[e] = vm;
-					a += v * v;
-					b += (float)vm * (float)vm;
-					c += v * mv[e];
-				}
-				else {
-					const float v = there ? __builtin_fmaf(piece[i][e], scale, -mv[e]) : 0.0f;
-					const _Float16 half = (_Float16)v;
-					const float low = v - (float)half;
-					hi[e] = __builtin_bit_cast(__bf16, half);
-					a += v * v;
-					b += low * low;
-				}
-			}
-			if (first_pass) { xx += a; xpart += b; xalong += c; }
-			char* at = base + ((f / 2) * UNIT_STRIDE + row) * 16 + (f % 2) * 8;
-			*(bf16x4*)at = hi;
-			if constexpr (X3) *(bf16x4*)(at + PART_UNITS * 16) = mid;
 		}
+		bf16x4 hi, mid;
+		float a = 0.0f, b = 0.0f, c = 0.0f;
+#pragma unroll
+		for (uint32_t e = 0; e < 4; ++e) {
+			const bool there = d + (VEC ? 0 : e) < w.dim;
+			if constexpr (X3) {
+				const float v = there ? piece[i][e] - mv[e] : 0.0f;
+				__bf16 vh, vm;
+				split_bf16(v, vh, vm);
+				hi[e] = vh;
+				mid[e] = vm;
+				a += v * v;
+				b += (float)vm * (float)vm;
+				c += v * mv[e];
+			}
+			else {
+				const float v = there ? __builtin_fmaf(piece[i][e], scale, -mv[e]) : 0.0f;
+				const _Float16 half = (_Float16)v;
+				const float low = v - (float)half;
+				hi[e] = __builtin_bit_cast(__bf16, half);
+				a += v * v;
+				b += low * low;
+			}
+		}
+		xx += first_pass ? a : 0.0f;
+		xpart += first_pass ? b : 0.0f;
+		if constexpr (X3) xalong += first_pass ? c : 0.0f;
+		asm volatile("" : "+v"(xx), "+v"(xpart)); /* (summed here: left alone the compiler keeps all pieces' values until after the matrix instructions) */
+		char* at = base + ((f / 2) * UNIT_STRIDE + row) * 16 + (f % 2) * 8;
+		*(bf16x4*)at = hi;
+		if constexpr (X3) *(bf16x4*)(at + PART_UNITS * 16) = mid;
 	};
 
 	/* this wavefront's tile of a group (beyond the last tile: the last one again, with infinite norms) */
@@ -391,12 +392,15 @@ wide_sweep_kernel(const WideArgs w)
 		}
 		seek();
 	};
-	bf16x8 ahi[WIDE_BLOCKS][NT], amid[X3 ? WIDE_BLOCKS : 1][NT];
-	auto fetch_ops = [&](int b) {
+	/* Blocks that a centroid tile's operands are requested ahead, and buffers of the points'. Units of 128 points have no registers left for more (4 blocks
+	 * ahead: 88 -> 98 us at N = 131071, d = 512, k = 400); units of 32 are all latency (n = 3000, k = 300: 45 us with these, 49 with the others). */
+	constexpr int RING = PT == 1 ? WIDE_BLOCKS : 2, SLOTS = PT == 1 ? 2 : 1;
+	bf16x8 ahi[RING][NT], amid[X3 ? RING : 1][NT];
+	auto fetch_ops = [&](int slot, int b) {
 #pragma unroll
 		for (int nt = 0; nt < NT; ++nt) {
-			ahi[b][nt] = next_ops[nt][b * WAVE + lane];
-			if constexpr (X3) amid[b][nt] = (next_ops[nt] + plane)[b * WAVE + lane];
+			ahi[slot][nt] = next_ops[nt][b * WAVE + lane];
+			if constexpr (X3) amid[slot][nt] = (next_ops[nt] + plane)[b * WAVE + lane];
 		}
 	};
 	/* |c|^2 of this wavefront's tiles of a group, one per lane; requested a group ahead */
@@ -412,10 +416,17 @@ wide_sweep_kernel(const WideArgs w)
 	request_norms(0);
 	seek();
 #pragma unroll
-	for (int b = 0; b < (int)WIDE_BLOCKS; ++b) fetch_ops(b);
-	advance();
-	request_rows(pt, 0);
+	for (int b = 0; b < RING; ++b) fetch_ops(b, b);
+#pragma unroll
+	for (uint32_t i = 0; i < VECS; ++i) request_piece(i, pt, 0);
 	const uint32_t uniform_n = n;
+#pragma unroll
+	for (uint32_t i = 0; i < VECS; ++i) {
+		store_piece(i, 0, 0, true);
+		request_piece(i, pt, 1);
+	}
+	uint32_t write_chunk = 1, write_buffer = 1, read_buffer = 0;
+	__syncthreads();
 
 	for (; unit < units; unit += gridDim.x) {
 		const uint32_t next_pt = unit + gridDim.x < units ? point_of(unit + gridDim.x) : pt;
@@ -423,22 +434,9 @@ wide_sweep_kernel(const WideArgs w)
 		uint32_t best_idx[PT];
 #pragma unroll
 		for (int p = 0; p < PT; ++p) { best[p] = __builtin_inff(); second[p] = __builtin_inff(); best_idx[p] = 0; }
-		xx = xpart = xalong = 0.0f;
-		store_rows(0, 0, true);
-		if (staged_steps > 1) request_rows(pt, 1 % chunks);
-		else request_rows(next_pt, 0);
-		__syncthreads();
-		if (flag_count + ROWS > WIDE_LIST) { /* (the same in every lane: the barrier above) */
-			__syncthreads();
-			if (tid == 0) { flag_base = atomicAdd(&w.counters[0], flag_count); }
-			__syncthreads();
-			for (uint32_t i = tid; i < 2 * flag_count; i += WIDE_THREADS) w.queue[2 * (size_t)flag_base + i] = flags[i];
-			__syncthreads();
-			if (tid == 0) flag_count = 0u;
-			/* (the next lane to add to the list does so behind at least one more barrier) */
-		}
+		float unit_xx = 0.0f, unit_xpart = 0.0f, unit_xalong = 0.0f;
 
-		uint32_t step = 0, write_chunk = 1 % chunks, write_buffer = 1, read_buffer = 0;
+		uint32_t step = 0;
 		for (uint32_t group = 0; group < groups; ++group) {
 			f32x16 acc[NT][PT];
 			norm_stage[wave][NT == 2 ? lane : col] = norm_reg;
@@ -461,43 +459,71 @@ wide_sweep_kernel(const WideArgs w)
 
 			for (uint32_t chunk = 0; chunk < chunks; ++chunk, ++step) {
 				const bf16x8* rows_at = rows_lds + (size_t)read_buffer * BUFFER_UNITS + h * UNIT_STRIDE + col;
-				bf16x8 bhi[2][PT], bmid[2][X3 ? PT : 1];
-				auto fetch_points = [&](int b) {
-#pragma unroll
-					for (int p = 0; p < PT; ++p) {
-						bhi[b & 1][p] = rows_at[2 * b * UNIT_STRIDE + p * TILE];
-						if constexpr (X3) bmid[b & 1][p] = rows_at[PART_UNITS + 2 * b * UNIT_STRIDE + p * TILE];
-					}
+				bf16x8 bhi[SLOTS][PT], bmid[SLOTS][X3 ? PT : 1];
+				auto fetch_point = [&](int b, int p) {
+					bhi[b % SLOTS][p] = rows_at[2 * b * UNIT_STRIDE + p * TILE];
+					if constexpr (X3) bmid[b % SLOTS][p] = rows_at[PART_UNITS + 2 * b * UNIT_STRIDE + p * TILE];
 				};
-				fetch_points(0);
+				/* the last step stages the first chunk of the next unit, so that its products follow without a wait */
+				const bool last_step = step + 1 == steps;
+				const bool stages = (!RESIDENT && PT > 1) || step + 1 < staged_steps || (last_step && (PT > 1 || unit + gridDim.x < units)), first_pass = step + 1 < chunks || last_step;
+				const uint32_t request_pt = step + 2 < staged_steps ? pt : next_pt, request_chunk = write_chunk + 1 < chunks ? write_chunk + 1 : 0;
+				if (last_step) {
+					if (RESIDENT) __syncthreads(); /* (all are past the unit's first chunk) */
+					unit_xx = xx; unit_xpart = xpart; unit_xalong = xalong;
+					xx = xpart = xalong = 0.0f;
+				}
+#pragma unroll
+				for (int p = 0; p < PT; ++p) fetch_point(0, p);
 #pragma unroll
 				for (int b = 0; b < (int)WIDE_BLOCKS; ++b) {
-					if (b + 1 < (int)WIDE_BLOCKS) fetch_points(b + 1);
-					__builtin_amdgcn_sched_barrier(0);
+					if constexpr (SLOTS > 1)
+						if (b + 1 < (int)WIDE_BLOCKS)
 #pragma unroll
-					for (int nt = 0; nt < NT; ++nt) {
-						if (!busy[nt]) continue;
+							for (int p = 0; p < PT; ++p) fetch_point(b + 1, p);
+					__builtin_amdgcn_sched_barrier(0);
+					auto products = [&](int nt) {
+						const bool ahead = SLOTS == 1 && nt == NT - 1 && b + 1 < (int)WIDE_BLOCKS;
+						if (!busy[nt]) {
+							if (ahead)
+#pragma unroll
+								for (int p = 0; p < PT; ++p) fetch_point(b + 1, p);
+							return;
+						}
 						if constexpr (X3) {
 #pragma unroll
-							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b][nt], bmid[b & 1][p], acc[nt][p], 0, 0, 0);
+							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b % RING][nt], bmid[b % SLOTS][p], acc[nt][p], 0, 0, 0);
 #pragma unroll
-							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(amid[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
+							for (int p = 0; p < PT; ++p) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(amid[X3 ? b % RING : 0][nt], bhi[b % SLOTS][p], acc[nt][p], 0, 0, 0);
 						}
 #pragma unroll
 						for (int p = 0; p < PT; ++p) {
-							if constexpr (X3) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b][nt], bhi[b & 1][p], acc[nt][p], 0, 0, 0);
-							else acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ahi[b][nt]), __builtin_bit_cast(f16x8, bhi[b & 1][p]), acc[nt][p], 0, 0, 0);
+							if constexpr (X3) acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[b % RING][nt], bhi[b % SLOTS][p], acc[nt][p], 0, 0, 0);
+							else acc[nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ahi[b % RING][nt]), __builtin_bit_cast(f16x8, bhi[b % SLOTS][p]), acc[nt][p], 0, 0, 0);
+							if (ahead) {
+								fetch_point(b + 1, p);
+								__builtin_amdgcn_sched_barrier(0);
+							}
 						}
+					};
+					products(0);
+					__builtin_amdgcn_sched_barrier(0);
+					if (stages) {
+#pragma unroll
+						for (uint32_t i = 0; i < VECS; ++i)
+							if ((int)((i + 1) * WIDE_BLOCKS / VECS) == b + 1) {
+								store_piece(i, write_buffer, write_chunk, first_pass);
+								request_piece(i, request_pt, request_chunk);
+							}
 					}
 					__builtin_amdgcn_sched_barrier(0);
-					fetch_ops(b);
+					if constexpr (NT == 2) products(NT - 1);
+					__builtin_amdgcn_sched_barrier(0);
+					if ((b + RING) % (int)WIDE_BLOCKS == 0) advance();
+					fetch_ops(b % RING, (b + RING) % (int)WIDE_BLOCKS);
 					__builtin_amdgcn_sched_barrier(0);
 				}
-				advance();
-				if (step + 1 < staged_steps) {
-					store_rows(write_buffer, write_chunk, step + 1 < chunks);
-					if (step + 2 < staged_steps) request_rows(pt, write_chunk + 1 == chunks ? 0 : write_chunk + 1);
-					else request_rows(next_pt, 0);
+				if (stages) {
 					write_chunk = write_chunk + 1 == chunks ? 0 : write_chunk + 1;
 					write_buffer = write_buffer + 1 == w.buffers ? 0 : write_buffer + 1;
 					__syncthreads();
@@ -543,29 +569,39 @@ wide_sweep_kernel(const WideArgs w)
 		}
 		if (LD == KMX_AOS) {
 			for (int off = SUBS / 2; off > 0; off >>= 1) {
-				xx += __shfl_xor(xx, off);
-				xpart += __shfl_xor(xpart, off);
-				xalong += __shfl_xor(xalong, off);
+				unit_xx += __shfl_xor(unit_xx, off);
+				unit_xpart += __shfl_xor(unit_xpart, off);
+				unit_xalong += __shfl_xor(unit_xalong, off);
 			}
-			if (sub == 0) { row_info[0][row] = xx; row_info[1][row] = xpart; row_info[2][row] = xalong; }
+			if (sub == 0) { row_info[0][row] = unit_xx; row_info[1][row] = unit_xpart; if constexpr (X3) row_info[2][row] = unit_xalong; }
 		}
 		else {
-			/* the lanes of a row sit in different wavefronts: their shares meet in LDS, in a fixed order */
-			float* share = (float*)rows_lds; /* (all wavefronts are past their last read after the barrier) */
-			__syncthreads();
-			share[(0 * SUBS + sub) * ROWS + row] = xx;
-			share[(1 * SUBS + sub) * ROWS + row] = xpart;
-			share[(2 * SUBS + sub) * ROWS + row] = xalong;
+			/* the lanes of a row sit in different wavefronts: their shares meet in LDS, in a fixed order, where the unit's last chunk was */
+			if (PT == 1) __syncthreads(); /* (its last step need not have ended with a barrier) */
+			float* share = (float*)(rows_lds + (size_t)(read_buffer ? read_buffer - 1 : w.buffers - 1) * BUFFER_UNITS);
+			share[(0 * SUBS + sub) * ROWS + row] = unit_xx;
+			share[(1 * SUBS + sub) * ROWS + row] = unit_xpart;
+			if constexpr (X3) share[(2 * SUBS + sub) * ROWS + row] = unit_xalong;
 			__syncthreads();
 			if (tid < ROWS) {
-				for (int q = 0; q < 3; ++q) {
+				for (uint32_t q = 0; q < SUMS; ++q) {
 					float s = 0.0f;
 					for (uint32_t i = 0; i < SUBS; ++i) s += share[(q * SUBS + i) * ROWS + tid];
 					row_info[q][tid] = s;
 				}
 			}
 		}
+		const bool full = flag_count + ROWS > WIDE_LIST; /* (the same in every lane: no one adds to the list between the last step's barrier and the next one) */
 		__syncthreads();
+		if (full) {
+			if (tid == 0) { flag_base = atomicAdd(&w.counters[0], flag_count); }
+			__syncthreads();
+			for (uint32_t i = tid; i < 2 * flag_count; i += WIDE_THREADS) w.queue[2 * (size_t)flag_base + i] = flags[i];
+			__syncthreads();
+			if (tid == 0) flag_count = 0u;
+			__syncthreads();
+		}
+		/* the other wavefronts go on with the next unit */
 		if (tid < ROWS) {
 			float first = cand_first[0][tid], next = cand_second[0][tid];
 			uint32_t idx = cand_idx[0][tid];
@@ -576,7 +612,7 @@ wide_sweep_kernel(const WideArgs w)
 				idx = cf < first ? cand_idx[v][tid] : idx;
 				first = __builtin_elementwise_minimum(first, cf);
 			}
-			const float x2 = row_info[0][tid], along = row_info[2][tid];
+			const float x2 = row_info[0][tid], along = X3 ? row_info[2][tid] : 0.0f;
 			const float tau = cert_tau(w.kd, x2, row_info[1][tid], cert);
 			const uint32_t slot = unit * ROWS + tid;
 			const bool mine = slot < uniform_n;
@@ -620,13 +656,15 @@ template <int PT, int NT, bool X3>
 static int launch_wide_sweep(const AssignArgs& a, WideArgs w, uint32_t lds_budget, const DeviceInfo& dev, kmx_exec_params* exec)
 {
 	const bool vec = a.dim % 4 == 0 && a.stride % 4 == 0 && ((uintptr_t)a.data & 15) == 0;
-	void (*kernel)(WideArgs) = a.layout == KMX_SOA ? wide_sweep_kernel<PT, NT, X3, KMX_SOA, false>
-	                           : vec ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, true> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, false>;
 	const uint32_t chunks = w.dp / WIDE_CHUNK, groups = (w.kp / TILE + WIDE_WAVES * NT - 1) / (WIDE_WAVES * NT);
 	const uint32_t buffer = wide_buffer_bytes(PT, X3);
 	const uint32_t room = lds_budget - wide_static_bytes(PT, NT) - w.dp * 4; /* (wide_sweep_bytes fits) */
 	/* all chunks of a unit stay in LDS where another group of centroids wants them again */
-	w.buffers = std::min(chunks, (groups > 1 && (uint64_t)chunks * buffer <= room) ? chunks : 2u);
+	const bool resident = groups > 1 && (uint64_t)chunks * buffer <= room;
+	w.buffers = resident ? chunks : 2u;
+	void (*kernel)(WideArgs) = a.layout == KMX_SOA ? (resident ? wide_sweep_kernel<PT, NT, X3, KMX_SOA, false, true> : wide_sweep_kernel<PT, NT, X3, KMX_SOA, false, false>)
+	                           : vec ? (resident ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, true, true> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, true, false>)
+	                                 : (resident ? wide_sweep_kernel<PT, NT, X3, KMX_AOS, false, true> : wide_sweep_kernel<PT, NT, X3, KMX_AOS, false, false>);
 	const uint32_t lds_bytes = w.dp * 4 + w.buffers * buffer;
 	const uint32_t units = (a.n + PT * TILE - 1) / (PT * TILE);
 	const uint32_t grid = std::min(units, dev.compute_units);

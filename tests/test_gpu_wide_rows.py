@@ -56,6 +56,30 @@ def test_wide_rows_match_the_oracle(km, orc, gpu, dim, k, n, kind):
     a.free()
 
 
+@pytest.mark.parametrize("dim,k,n", [(300, 40, 9000), (257, 300, 8225),    # units of 32 points, one and several groups
+                                     (320, 520, 33000), (1030, 600, 32800), (300, 3, 66000)])   # of 128: resident, staged again, one tile
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_units_that_follow_one_another_match_the_oracle(km, orc, gpu, dim, k, n, mode, layout):
+    """More units than work-groups: the first chunk of a work-group's next unit is staged during the last step of the one before."""
+    rng = np.random.default_rng(dim + k)
+    centres = rng.uniform(-3, 3, size=(k, dim)).astype(np.float32)
+    rows = (centres[rng.integers(0, k, n)] + rng.normal(size=(n, dim))).astype(np.float32)
+    want = orc.assign(flat(rows, 0), flat(centres, 0), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, layout))
+    m = km.DeviceBuffer(centres.nbytes); m.write(flat(centres, layout))
+    a = km.DeviceBuffer(4 * n); a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+    km.set_two_level_sweep(mode)
+    try:
+        km.assign(km.ASSIGN_BEST, d, layout, km.layout_stride(layout, n, dim), m, layout, km.layout_stride(layout, k, dim), a, dim, k, n)
+        km.sync()
+    finally:
+        km.set_two_level_sweep(1)
+    got = a.read(np.uint32, n)
+    d.free(); m.free(); a.free()
+    assert np.array_equal(got, want), "%d mismatches" % int((got != want).sum())
+
+
 @pytest.mark.parametrize("budget,variant,blocks", [
     (0, "MFMA_BF16X3", 129),           # 129 units of 128 points
     (54 * 1024, "MFMA_BF16X3", 256),   # too little for those: units of 32
