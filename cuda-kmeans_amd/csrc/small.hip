@@ -46,7 +46,10 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  * dozen centroids at most, which would leave most of the larger tile empty. (A lane per point with the centroids broadcast is
  * bound by the LDS; with the centroids as scalar operands every scalar load waits for all earlier ones: N = 2588, d = 60, k = 1288
  * 135 us.) A few dozen centroids leave most of the time to the trips to memory and the barriers in front of that (N = 65536, d = 8, k = 64: 3 us
- * of vector instructions in 14 us). The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
+ * of vector instructions in 11 us): points and centroids are requested together, and no lane asks for more than there is. With one after the other, each
+ * in eight loads a lane whatever there was to load, that call was 25.0 instead of 22.0 us; d = 100, k = 40, N = 30000: 17.2 against 15.6; N = 10240,
+ * d = 20, k = 128: 19.5 against 18.9. (76 vector registers leave three of the four work-groups that a compute unit could hold; with 64 the sums spill:
+ * 23.1 us.) The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
  * ascending dimension, every operation rounded separately. Global loads are issued in batches of eight per lane: one after the
  * other they cost a microsecond each.
  *
@@ -59,58 +62,64 @@ constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading t
 constexpr uint32_t SMALL_POINTS = WAVE;
 constexpr int SMALL_BATCH = 8;
 
-/* count rows of dim elements into LDS rows of row_stride: AoS rows `stride` apart, or columns (row r of column q at src[q * stride + r]).
- * magic = ceil(2^32 / dim): i / dim = umulhi(i, magic) for the few ten thousand elements of a work-group. */
-template <typename F, int L>
-__device__ __forceinline__ void stage_rows(F* __restrict__ to, const F* __restrict__ src, size_t stride, uint32_t count, uint32_t last, uint32_t dim,
-                                           uint32_t row_stride, uint32_t magic, uint32_t vec4)
+/*
+ * `count` rows of dim elements on their way to LDS rows of row_stride: AoS rows `stride` apart, or columns (row r of column q at src[q * stride + r];
+ * a wavefront takes 64 rows of one column at a time). vec4: rows of whole, aligned pieces of four. Rows behind `last` repeat it.
+ * magic = ceil(2^32 / dim): i / dim = umulhi(i, magic) for the few ten thousand elements of a work-group.
+ */
+template <typename F>
+struct SmallRows {
+	F* to; const F* src; size_t stride;
+	uint32_t count, last, dim, row_stride, magic; bool vec4;
+};
+template <typename F, int L> __device__ __forceinline__ uint32_t small_items(const SmallRows<F>& s)
 {
+	return L == KMX_SOA ? (s.count + WAVE - 1) / WAVE * s.dim : s.vec4 ? s.count * (s.dim / 4) : s.count * s.dim;
+}
+
+/* items base, base + 1, .. of every lane (SoA: wavefront): all of them are requested before the first is placed. Lanes without an item ask for nothing:
+ * a repeated one costs the caches as much as any (N = 65536, d = 8, k = 64: seven of eight were). */
+template <typename F, int L, int B>
+struct SmallBatch {
 	typedef typename SmallVec<F>::type F4;
-	if (L == KMX_AOS && vec4) { /* rows of whole, aligned pieces of four */
-		const uint32_t pieces = dim / 4, total = count * pieces;
-		for (uint32_t i0 = threadIdx.x; i0 < total; i0 += SMALL_THREADS * SMALL_BATCH) {
-			F4 v[SMALL_BATCH];
-			uint32_t at[SMALL_BATCH];
+	F4 v[B];
+	uint32_t at[B];
+	static __device__ __forceinline__ uint32_t item(uint32_t i)
+	{
+		return L == KMX_SOA ? i * SMALL_WAVES + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) : i * SMALL_THREADS + threadIdx.x;
+	}
+	__device__ __forceinline__ void request(const SmallRows<F>& s, uint32_t base, uint32_t items)
+	{
 #pragma unroll
-			for (int u = 0; u < SMALL_BATCH; ++u) {
-				const uint32_t i = min(i0 + u * SMALL_THREADS, total - 1);
-				const uint32_t r = __umulhi(i * 4, magic), q = i * 4 - r * dim;
-				at[u] = r * row_stride + q;
-				v[u] = *(const F4*)(src + (size_t)min(r, last) * stride + q);
-			}
-#pragma unroll
-			for (int u = 0; u < SMALL_BATCH; ++u) *(F4*)(to + at[u]) = v[u];
+		for (int u = 0; u < B; ++u) {
+			const uint32_t i = item(base + u);
+			if (i >= items) continue;
+			const uint32_t e = L == KMX_AOS && s.vec4 ? i * 4 : i, whole = s.dim == 1 ? e : __umulhi(e, s.magic), q = e - whole * s.dim;
+			const uint32_t r = L == KMX_SOA ? min(whole * WAVE + threadIdx.x % WAVE, s.count - 1) : whole;
+			const F* from = s.src + elem<L>(s.stride, min(r, s.last), q);
+			at[u] = r * s.row_stride + q;
+			if (L == KMX_AOS && s.vec4) v[u] = *(const F4*)from;
+			else v[u].x = *from;
 		}
 	}
-	else if (L == KMX_AOS) {
-		const uint32_t total = count * dim;
-		for (uint32_t i0 = threadIdx.x; i0 < total; i0 += SMALL_THREADS * SMALL_BATCH) {
-			F v[SMALL_BATCH];
-			uint32_t at[SMALL_BATCH];
+	__device__ __forceinline__ void place(const SmallRows<F>& s, uint32_t base, uint32_t items) const
+	{
 #pragma unroll
-			for (int u = 0; u < SMALL_BATCH; ++u) {
-				const uint32_t i = min(i0 + u * SMALL_THREADS, total - 1);
-				const uint32_t r = dim == 1 ? i : __umulhi(i, magic), q = i - r * dim;
-				at[u] = r * row_stride + q;
-				v[u] = src[(size_t)min(r, last) * stride + q];
-			}
-#pragma unroll
-			for (int u = 0; u < SMALL_BATCH; ++u) to[at[u]] = v[u];
+		for (int u = 0; u < B; ++u) {
+			if (item(base + u) >= items) continue;
+			if (L == KMX_AOS && s.vec4) *(F4*)(s.to + at[u]) = v[u];
+			else s.to[at[u]] = v[u].x;
 		}
 	}
-	else {
-		/* a wavefront takes 64 rows of one column at a time */
-		const uint32_t lane = threadIdx.x & (WAVE - 1);
-		for (uint32_t r0 = 0; r0 < count; r0 += WAVE) {
-			const uint32_t r = min(r0 + lane, count - 1);
-			for (uint32_t q0 = threadIdx.x / WAVE; q0 < dim; q0 += SMALL_WAVES * SMALL_BATCH) {
-				F v[SMALL_BATCH];
-#pragma unroll
-				for (int u = 0; u < SMALL_BATCH; ++u) v[u] = src[(size_t)min(q0 + u * SMALL_WAVES, dim - 1) * stride + min(r, last)];
-#pragma unroll
-				for (int u = 0; u < SMALL_BATCH; ++u) to[r * row_stride + min(q0 + u * SMALL_WAVES, dim - 1)] = v[u];
-			}
-		}
+};
+template <typename F, int L>
+__device__ __forceinline__ void stage_rows(const SmallRows<F>& s, uint32_t base, uint32_t items)
+{
+	constexpr uint32_t STEP = L == KMX_SOA ? SMALL_WAVES : SMALL_THREADS;
+	for (; base * STEP < items; base += SMALL_BATCH) {
+		SmallBatch<F, L, SMALL_BATCH> batch;
+		batch.request(s, base, items);
+		batch.place(s, base, items);
 	}
 }
 
@@ -137,7 +146,25 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 	const uint32_t here = min(POINTS, n - first);
 	if (blockIdx.x == 0 && tid == 0) counters[0] = 0u; /* nothing is left to an exact pass */
 
-	stage_rows<F, LD>(rows, LD == KMX_AOS ? data + (size_t)first * stride : data + first, stride, POINTS, here - 1, dim, row_stride, magic, vec4 & 1u);
+	auto centroids = [&](uint32_t base) -> SmallRows<F> {
+		const uint32_t count = min(chunk, k - base);
+		return SmallRows<F>{ cents, LM == KMX_AOS ? means + (size_t)base * stride_means : means + base, stride_means, count, count - 1, dim, row_stride, magic, (vec4 & 2u) != 0 };
+	};
+	{
+		/* points and centroids travel together, up to 4 items a lane of each: one trip to memory where there were two */
+		const SmallRows<F> points = { rows, LD == KMX_AOS ? data + (size_t)first * stride : data + first, stride, POINTS, here - 1, dim, row_stride, magic, (vec4 & 1u) != 0 };
+		const SmallRows<F> start = centroids(0);
+		const uint32_t point_items = small_items<F, LD>(points), start_items = small_items<F, LM>(start);
+		constexpr int TOGETHER = 4;
+		SmallBatch<F, LD, TOGETHER> some;
+		SmallBatch<F, LM, TOGETHER> others;
+		some.request(points, 0, point_items);
+		others.request(start, 0, start_items);
+		some.place(points, 0, point_items);
+		others.place(start, 0, start_items);
+		stage_rows<F, LD>(points, TOGETHER, point_items);
+		stage_rows<F, LM>(start, TOGETHER, start_items);
+	}
 
 	F low[T];
 	uint32_t at[T];
@@ -146,8 +173,11 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 	const F* mine = rows + (pg * (16 * T) + lp) * row_stride;
 	for (uint32_t base = 0; base < k; base += chunk) {
 		const uint32_t count = min(chunk, k - base);
-		if (base) __syncthreads(); /* the previous chunk is no longer needed */
-		stage_rows<F, LM>(cents, LM == KMX_AOS ? means + (size_t)base * stride_means : means + base, stride_means, count, count - 1, dim, row_stride, magic, vec4 & 2u);
+		if (base) {
+			__syncthreads(); /* the previous chunk is no longer needed */
+			const SmallRows<F> next = centroids(base);
+			stage_rows<F, LM>(next, 0, small_items<F, LM>(next));
+		}
 		__syncthreads();
 		for (uint32_t c0 = cw * (4 * T); c0 < count; c0 += CW * (4 * T)) {
 			F sum[T][T];

@@ -56,6 +56,14 @@ def test_small_assignment_and_iteration(km, orc, gpu, dtype, dim, k, n, layout, 
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dim,k,n", [(128, 64, 64), (132, 62, 65), (64, 128, 100), (64, 129, 100),   # 2048 pieces of four coordinates travel together, then more
+                                     (31, 66, 70), (32, 64, 64), (33, 65, 70), (127, 17, 64)])       # 2048 coordinates, or 32 columns of 64 rows
+@pytest.mark.parametrize("layout,layout_means", [(0, 0), (1, 1), (0, 1)])
+def test_small_staging_at_the_edges_of_its_batches(km, orc, gpu, dtype, dim, k, n, layout, layout_means):
+    test_small_assignment_and_iteration(km, orc, gpu, dtype, dim, k, n, layout, layout_means)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("dim,k,n", [(1, 1, 1), (3, 2, 4095), (4, 256, 4096), (5, 257, 4097), (20, 128, 12288), (9, 600, 12289), (2, 4096, 32768), (300, 40, 700)])
 @pytest.mark.parametrize("layout,layout_means", [(0, 0), (1, 1)])
 @pytest.mark.parametrize("kind", ["uniform", "hot"])
