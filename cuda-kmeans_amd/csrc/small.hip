@@ -48,19 +48,19 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  * 135 us.) A few dozen centroids leave most of the time to the trips to memory and the barriers in front of that (N = 65536, d = 8, k = 64: 3 us
  * of vector instructions in 11 us): points and centroids are requested together, and no lane asks for more than there is. With one after the other, each
  * in eight loads a lane whatever there was to load, that call was 25.0 instead of 22.0 us; d = 100, k = 40, N = 30000: 17.2 against 15.6; N = 10240,
- * d = 20, k = 128: 19.5 against 18.9. (76 vector registers leave three of the four work-groups that a compute unit could hold; with 64 the sums spill:
- * 23.1 us.) The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
+ * d = 20, k = 128: 19.5 against 18.9. Floats are held to 64 vector registers, so that a compute unit
+ * takes four work-groups (with 76 three: N = 50000, d = 2, k = 10 14.0 against 13.4 us, N = 65000, d = 5, k = 50 10.0 against 9.5). The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
  * ascending dimension, every operation rounded separately. Global loads are issued in batches of eight per lane: one after the
  * other they cost a microsecond each.
  *
  * SUMS: membership (clusters x 64 points) times rows (64 points x coordinates) on v_mfma_f32_16x16x4_f32: 1.0 times a coordinate is
- * exact, the accumulators add in fp32. A wavefront keeps the memberships of 16 clusters in registers and goes over the coordinates 16
- * at a time. 0.0 times an infinity or a NaN would reach every cluster: a work-group that sees one adds its points up again, an
+ * exact, the accumulators add in fp32. A wavefront has 16 clusters and goes over the coordinates 16 at a time; where that leaves
+ * wavefronts over, they share out the coordinates (N = 5000, d = 200, k = 20: 24.4 -> 20.7 us). 0.0 times an infinity or a NaN would reach every cluster: a work-group that sees one adds its points up again, an
  * element of the sums per lane.
  */
 constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading the memberships again (update_small_kernel) is cheaper than as many partial sums */
 constexpr uint32_t SMALL_POINTS = WAVE;
-constexpr int SMALL_BATCH = 8;
+constexpr int SMALL_BATCH = 4;
 
 /*
  * `count` rows of dim elements on their way to LDS rows of row_stride: AoS rows `stride` apart, or columns (row r of column q at src[q * stride + r];
@@ -124,7 +124,7 @@ __device__ __forceinline__ void stage_rows(const SmallRows<F>& s, uint32_t base,
 }
 
 template <typename F, int T, int LD, int LM, bool SUMS>
-__global__ void __launch_bounds__(SMALL_THREADS)
+__global__ void __launch_bounds__(SMALL_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(F) == 4 ? 8 : 4)))
 assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restrict__ means, size_t stride_means,
                     uint32_t* __restrict__ assignment, uint32_t dim, uint32_t k, uint32_t n, uint32_t row_stride, uint32_t chunk,
                     uint32_t magic, uint32_t vec4, uint32_t* __restrict__ counters, F* __restrict__ partial, uint32_t* __restrict__ partial_counts)
@@ -278,18 +278,27 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 		F* out = partial + (size_t)blockIdx.x * k * dim;
 		const uint32_t l16 = lane & 15, quad = lane >> 4;
 		bool bad = false;
-		for (uint32_t cluster = wave * 16; cluster < k; cluster += SMALL_WAVES * 16) {
-			float in[POINTS / 4]; /* point 4 i + quad belongs to cluster + l16 */
-#pragma unroll
-			for (uint32_t i = 0; i < POINTS / 4; ++i) in[i] = member[4 * i + quad] == cluster + l16 ? 1.0f : 0.0f;
-			for (uint32_t d0 = 0; d0 < dim; d0 += 16) {
+		/* wavefronts beyond one per 16 clusters share out the coordinates */
+		const uint32_t across = min((k + 15) / 16, SMALL_WAVES);
+		uint32_t column = wave, share = 0, shares = 1;
+		while (column >= across) { column -= across; ++share; }
+		while ((shares + 1) * across <= SMALL_WAVES) ++shares;
+		for (uint32_t cluster = column * 16; cluster < k && share < shares; cluster += across * 16) {
+			for (uint32_t d0 = share * 16; d0 < dim; d0 += shares * 16) {
 				const F* at_row = rows + quad * row_stride + min(d0 + l16, dim - 1);
+				const uint32_t* whose = member + quad;
 				f32x4 sum = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll 1
+				for (uint32_t i = 0; i < POINTS / 4; i += 8) { /* (all 16 at once take more registers than eight wavefronts of a SIMD have) */
 #pragma unroll
-				for (uint32_t i = 0; i < POINTS / 4; ++i) {
-					const float x = at_row[4 * i * row_stride];
-					bad = bad || !(__builtin_fabsf(x) < __builtin_inff());
-					sum = __builtin_amdgcn_mfma_f32_16x16x4f32(in[i], x, sum, 0, 0, 0);
+					for (uint32_t j = 0; j < 8; ++j) {
+						const float in = whose[4 * j] == cluster + l16 ? 1.0f : 0.0f; /* point 4 (i + j) + quad belongs to cluster + l16 */
+						const float x = at_row[4 * j * row_stride];
+						bad = bad || !(__builtin_fabsf(x) < __builtin_inff());
+						sum = __builtin_amdgcn_mfma_f32_16x16x4f32(in, x, sum, 0, 0, 0);
+					}
+					whose += 32;
+					at_row += 32 * row_stride;
 				}
 #pragma unroll
 				for (uint32_t r = 0; r < 4; ++r)
@@ -303,6 +312,7 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 			for (uint32_t e = tid; e < k * dim; e += SMALL_THREADS) {
 				const uint32_t cl = e / dim, d = e - cl * dim;
 				F s = (F)0;
+#pragma unroll 1 /* (rare, and not worth the registers) */
 				for (uint32_t p = 0; p < POINTS; p += 4) {
 					const u4 m = *(const u4*)(member + p);
 #pragma unroll
