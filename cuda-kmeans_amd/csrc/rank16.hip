@@ -13,11 +13,11 @@
  * operands, notes the centroids within the point's threshold (two or three of k) and evaluates the serial arithmetic for those.
  * Gather, screen, evaluate and scatter were four launches (63 us at N = 1M, d = 256, k = 1024, behind a second sweep of 188).
  *
- * What bounds it: the sweep by the matrix instructions and the tracking of the minima that shares the issue slots with them
- * (N = 1M, d = 256, k = 1024: 630 us, 0.87 PFLOP/s; d = 32, k = 1024, N = 2M: 185 us); the exact pass by reading centroid operands
- * and rows (12 % of N = 1M, d = 256 listed: 131 us; 1 %: 40 us, the latency of one unit). Whole calls, two bf16 levels before -> now: N = 1M, d = 256, k = 1024 1713 ->
- * 743 us; N = 2M, d = 128, k = 1024 1443 -> 683 (SoA 1629 -> 940); N = 2M, d = 32, k = 1024 332 -> 230; N = 1M, d = 64, k = 512 203 -> 122;
- * N = 100k, d = 256, k = 32 92 -> 51.
+ * What bounds it: the sweep by the matrix instructions and the tracking of the minima that shares the issue slots with them, at a clock that
+ * gives way to the power they take (N = 1M, d = 256, k = 1024: 475 to 505 us, 1.09 to 1.16 PFLOP/s; d = 32, k = 1024, N = 2M: 151 to 169 us); the
+ * exact pass by the latencies of one unit, list, rows, ranking and pairs in turn (1 to 4 % listed: 26 to 35 us; 9 % of N = 2M, d = 128: 110).
+ * Whole calls, two bf16 levels -> this kernel at first -> now: N = 1M, d = 256, k = 1024 1713 -> 743 -> 520 us; N = 2M, d = 128, k = 1024, SoA
+ * 1629 -> 940 -> 845; N = 2M, d = 32, k = 1024 332 -> 230 -> 185.
  */
 #include "rank16_exact_impl.h"
 
