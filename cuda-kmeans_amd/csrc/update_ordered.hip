@@ -19,6 +19,7 @@
  * ordered_stream_sum_kernel / ordered_staged_sum_kernel / ordered_sum_kernel.
  */
 #include "kmx_internal.h"
+#include "update_ordered_route.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -348,7 +349,7 @@ ordered_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __
  * 2048 work-groups, two per compute unit and so four rounds, of two fetches each: 36 cycles per addition, with 16 of 512 lanes adding).
  * ELEMENTS: SoA points, rows shorter than a piece: single coordinates, consecutive lanes take consecutive members.
  */
-constexpr uint32_t STAGED_THREADS = 512, STAGED_PIECES = 8;
+constexpr uint32_t STAGED_PIECES = 8;
 
 template <typename F, int LD, int LM, bool ELEMENTS>
 __global__ void __launch_bounds__(STAGED_THREADS, 4)
@@ -436,7 +437,8 @@ ordered_staged_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
  * (N = 2M, d = 32, k = 1024: 80 us, 3.4 TB/s; one wavefront 107, the staged kernel above 169). AHEAD of 1, 2, 3, 4 with one wavefront: 133, 106,
  * 107, 122 us (four work-groups fit a compute unit with up to 3).
  */
-constexpr uint32_t STREAM_BLOCK_BYTES = 128, STREAM_REQUESTS = 8, STREAM_SLOT_BYTES = STREAM_REQUESTS * WAVE * 16;
+constexpr uint32_t STREAM_REQUESTS = 8, STREAM_SLOT_BYTES = STREAM_REQUESTS * WAVE * 16;
+static_assert(STREAM_THREADS == 2 * WAVE, "one wavefront requests, one adds");
 constexpr uint32_t stream_rows(uint32_t pieces) { return WAVE / pieces; }                     /* per request */
 constexpr uint32_t stream_batch(uint32_t pieces) { return STREAM_REQUESTS * stream_rows(pieces); }
 constexpr uint32_t stream_names(uint32_t pieces) { return (stream_batch(pieces) + WAVE - 1) / WAVE; } /* requests for a batch's numbers */
@@ -455,7 +457,7 @@ __device__ __forceinline__ void stream_request4(const void* from, uint32_t to)
 }
 
 template <typename F, int LM, uint32_t P, bool DEEP>
-__global__ void __launch_bounds__(2 * WAVE)
+__global__ void __launch_bounds__(STREAM_THREADS)
 ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ starts,
                           const uint32_t* __restrict__ sizes, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t blocks, uint32_t divide)
 {
@@ -568,14 +570,13 @@ static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sort
                               F* means, size_t stride_means, uint32_t dim, uint32_t k, uint32_t n, bool divide, const DeviceInfo& dev)
 {
 	constexpr int WIDE = 16 / sizeof(F);
-	/* (all of an iteration, us, the kernels below -> this: N = 2M, d = 32, k = 1024 421 -> 332; d = 16, k = 16, half of the points in one cluster 2669 -> 1504; N = 30k,
-	 * d = 512, k = 512 167 -> 109; N = 40k, d = 32, k = 1024 57 -> 51; N = 10240, d = 20, k = 128 29.8 -> 29.4; N = 20k, d = 100, k = 1000 75 -> 79; rows of
-	 * a piece or two: N = 1M, d = 4, k = 4096 194 -> 191, N = 270k 127 -> 131) */
+	const bool fits = LD == KMX_AOS && dim % WIDE == 0 && stride % WIDE == 0 && ((uintptr_t)data & 15) == 0;
+	const OrderedSumRoute route = ordered_sum_route(sizeof(F), fits && stride <= 0xFFFFFFFFu / sizeof(F), dim, k, n);
+	const uint32_t groups = k * route.blocks;
 	if constexpr (LD == KMX_AOS) {
-		const uint32_t stream_dims = STREAM_BLOCK_BYTES / sizeof(F), stream_blocks = (dim + stream_dims - 1) / stream_dims;
-		if (dim % WIDE == 0 && stride % WIDE == 0 && stride <= 0xFFFFFFFFu / sizeof(F) && ((uintptr_t)data & 15) == 0 && n / k >= (dim / WIDE <= 2 ? 128u : 32u) && (uint64_t)k * stream_blocks <= 0x7FFFFFFFu) {
+		if (route.kernel == ORDERED_STREAM) {
 			const uint32_t pieces = std::min<uint32_t>(dim / WIDE, STREAM_BLOCK_BYTES / 16);
-			const bool deep = (uint64_t)k * stream_blocks <= 2 * dev.compute_units;
+			const bool deep = groups <= 2 * dev.compute_units;
 			void (*kernel)(const F*, size_t, const uint32_t*, const uint32_t*, const uint32_t*, F*, size_t, uint32_t, uint32_t, uint32_t) = nullptr;
 			uint32_t lds = 0;
 			auto take = [&](auto tag) {
@@ -587,29 +588,21 @@ static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sort
 			take(std::integral_constant<uint32_t, 1>{}); take(std::integral_constant<uint32_t, 2>{}); take(std::integral_constant<uint32_t, 3>{}); take(std::integral_constant<uint32_t, 4>{});
 			take(std::integral_constant<uint32_t, 5>{}); take(std::integral_constant<uint32_t, 6>{}); take(std::integral_constant<uint32_t, 7>{}); take(std::integral_constant<uint32_t, 8>{});
 			KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-			KMX_LAUNCH_KERNEL(kernel, dim3(k * stream_blocks), dim3(2 * WAVE), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, stream_blocks, divide ? 1u : 0u);
+			KMX_LAUNCH_KERNEL(kernel, dim3(groups), dim3(STREAM_THREADS), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, route.blocks, divide ? 1u : 0u);
 			KMX_LAUNCH_CHECK("ordered_stream_sum_kernel");
 			return KMX_OK;
 		}
 	}
-	/* Clusters of a few dozen members leave a work-group of eight wavefronts nothing to overlap, the more so the more clusters there are
-	 * (all of the update, us, staged and not: N = 80k, d = 32, k = 1024 31, 37; N = 40k 31, 30; d = 4, k = 4096: N = 1M 114, 116; N = 270k 77, 64).
-	 * Blocks of 32 coordinates are whole cache lines; of 16, twice as many work-groups and half the pieces per member, which long
-	 * chains want (N = 2M, d = 32, k = 1024 261 -> 231; N = 1M, d = 64, k = 100 388 -> 274) and the others do not (N = 500k, d = 500,
-	 * k = 200 432 -> 479; N = 100k, d = 32, k = 1024 34 -> 38). */
-	const uint32_t members = n / k;
-	const uint32_t block_dims = members >= 512 && (uint64_t)k * ((dim + 31) / 32) <= 1024 ? 16 : 32;
-	const uint32_t blocks = (dim + block_dims - 1) / block_dims;
-	if (members >= ((uint64_t)k * blocks <= 2048 ? 64u : 256u) && (uint64_t)k * blocks <= 0x7FFFFFFFu) {
+	if (route.kernel == ORDERED_STAGED) {
+		const uint32_t block_dims = route.block_dims;
 		const bool elements = LD == KMX_SOA || dim < (uint32_t)WIDE || (dim % block_dims != 0 && dim % block_dims < (uint32_t)WIDE);
 		const uint32_t lds = STAGED_THREADS * STAGED_PIECES * (elements ? sizeof(F) : 16) + std::min(dim, block_dims) * 16;
 		auto kernel = elements ? ordered_staged_sum_kernel<F, LD, LM, true> : ordered_staged_sum_kernel<F, KMX_AOS, LM, false>;
 		KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-		KMX_LAUNCH_KERNEL(kernel, dim3(k * blocks), dim3(STAGED_THREADS), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, blocks, block_dims, divide ? 1u : 0u);
+		KMX_LAUNCH_KERNEL(kernel, dim3(groups), dim3(STAGED_THREADS), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, route.blocks, block_dims, divide ? 1u : 0u);
 		KMX_LAUNCH_CHECK("ordered_staged_sum_kernel");
 		return KMX_OK;
 	}
-	const bool fits = LD == KMX_AOS && dim % WIDE == 0 && stride % WIDE == 0 && ((uintptr_t)data & 15) == 0;
 	const bool wide = fits && (size_t)k * (dim / WIDE) >= (size_t)2 * WAVE * dev.compute_units;
 	const size_t total = (size_t)k * (wide ? dim / WIDE : dim);
 	const dim3 grid((uint32_t)((total + WAVE - 1) / WAVE));
