@@ -28,6 +28,15 @@ constexpr float CELL_MARGIN = 1e-3f;
  * square roots by more than a rounding (2 x 2^-24 of the square).
  */
 constexpr float CELL_CLEAR = 1.000002f;
+/*
+ * A wavefront that has met this many points whose two smallest squares are not clear of each other stays with the serial arithmetic. On a raster (whole
+ * numbers, colours, quantised measurements) every batch has some, and going through the lists twice costs more than the fused sums save (N = 4M, us
+ * per call, the serial arithmetic alone, both for such points' wavefronts, this: d = 3, k = 4096, 16 places a dimension: 107, 142, 109; d = 4: 185, 237,
+ * 189; 64 places 193, 215, 194; normal points rounded to 1/40 of their deviation, d = 3: 248, 300, 255). Other data have a dozen such points in all of
+ * N = 4M: with 1 their wavefronts, which the others wait for at the end, cost half of what the fused sums save (normal points, d = 3, k = 4096: 254, 231, 248;
+ * with 2 level with 231); with 4 the rounded normal points take 265.
+ */
+constexpr uint32_t CELL_TIES = 2;
 constexpr uint32_t CELL_MAX_K = 6144;              /* what the building kernel's LDS holds */
 constexpr uint32_t CELL_UNIT = 8;                  /* entries (16 bits) of a list that are read together */
 constexpr uint32_t CELL_POOL_UNITS = 1u << 20;
@@ -419,9 +428,9 @@ constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* 
  * the longest list of its 64 points, 70 entries of 29 on average, and 16 bytes at 64 unrelated addresses take 11 cycles with their bank conflicts:
  * 179 000 of the 242 000 cycles of a compute unit), then the vector ALU. A comparison is 13 instructions and no branch: the sums are fused, the
  * two smallest are kept (one v_med3), and the few points whose two smallest are not CELL_CLEAR of each other go through their list again in the
- * serial arithmetic. Against that arithmetic for all, with its branches (17 instructions, and each row waited for by itself): 122 -> 112 us;
- * normal points, d = 4, k = 1000: 246 -> 216 us per call; d = 3, k = 6000: 119 -> 108 us; points and centroids on a lattice of 16^4 places, nearly
- * all of them ties: 178 -> 228 us. Sorting a wavefront's 256 points by the length of their lists takes a quarter of the instructions out, but
+ * serial arithmetic (see CELL_TIES). Against that arithmetic for all, with its branches (17 instructions, and each row waited for by itself): 122 -> 112 us;
+ * normal points, d = 4, k = 1000: 246 -> 216 us per call; d = 3, k = 6000: 119 -> 108 us. Sorting a wavefront's 256 points by the length of their
+ * lists takes a quarter of the instructions out, but
  * fuller wavefronts have more bank conflicts: 122 -> 136 us. Two work-groups share a compute unit, eight wavefronts
  * a SIMD, which takes 64 vector registers; with more than 80 scalar registers (and the 16 the hardware adds) only seven fit, which is one
  * work-group (d = 3, k = 4096, normal points: 162 -> 220 us).
@@ -531,6 +540,7 @@ assign_cells_kernel(const CellAssignArgs w)
 	}
 
 	uint32_t flagged = 0; /* wave-uniform */
+	uint32_t ties = 0;    /* wave-uniform: points whose nearest two were not clear of each other */
 	for (uint32_t base = blockIdx.x * CELL_THREADS; base < w.n; base += gridDim.x * CELL_THREADS) {
 		const uint32_t pt = base + tid;
 		const bool mine = pt < w.n;
@@ -578,22 +588,28 @@ assign_cells_kernel(const CellAssignArgs w)
 				}
 			}
 		};
-		float second = __builtin_inff();
-		walk([&](const f32x4& c, uint32_t at) {
-			float sum = 0.0f;
-#pragma unroll
-			for (int q = 0; q < D; ++q) {
-				const float diff = x[q] - c[q];
-				sum = q ? __builtin_fmaf(diff, diff, sum) : diff * diff;
-			}
-			second = __builtin_amdgcn_fmed3f(sum, best, second);
-			const bool less = sum < best;
-			best = less ? sum : best;
-			winner = less ? at : winner;
-		});
 		const bool flag = mine && (!inside || (entry & CELL_TRUNCATED));
-		/* (a flagged point's distance becomes its threshold: the serial one, as ever; smaller squares may have lost bits) */
-		if (flag || !(best > 1e-30f && second > best * CELL_CLEAR)) {
+		bool open = true;
+		if (ties < CELL_TIES) {
+			float second = __builtin_inff();
+			walk([&](const f32x4& c, uint32_t at) {
+				float sum = 0.0f;
+#pragma unroll
+				for (int q = 0; q < D; ++q) {
+					const float diff = x[q] - c[q];
+					sum = q ? __builtin_fmaf(diff, diff, sum) : diff * diff;
+				}
+				second = __builtin_amdgcn_fmed3f(sum, best, second);
+				const bool less = sum < best;
+				best = less ? sum : best;
+				winner = less ? at : winner;
+			});
+			/* (smaller squares may have lost bits; a sum of 0 is 0 in either arithmetic, and the first one wins) */
+			const bool clear = best == 0.0f || (best > 1e-30f && second > best * CELL_CLEAR);
+			ties += (uint32_t)__popcll(__ballot(!clear && !flag));
+			open = flag || !clear; /* (a flagged point's distance becomes its threshold: the serial one) */
+		}
+		if (open) {
 			best = __builtin_inff();
 			winner = 0;
 			walk(compare);

@@ -95,3 +95,23 @@ def test_points_a_regular_grid_is_no_good_for(km, orc, gpu, kind, dim, k):
         rows = rng.random((n, dim), dtype=np.float32)
         rows = np.ascontiguousarray(rows[np.argsort(rows[:, 0])])
     check(km, orc, rows, rows[:k].copy())
+
+
+@pytest.mark.parametrize("dim,k", [(3, 4096), (4, 4096)])
+def test_points_on_a_raster(km, orc, gpu, dim, k):
+    """Whole numbers as colours and quantised measurements are: most points are as near to one centroid as to another, in every wavefront's
+    every batch. Timed beside the same points spread evenly around their places, where hardly one is: settling ties costs no
+    more than 1.1 times that (0.97 to 1; it was 1.16 to 1.2 where every tie sent its wavefront through the lists a second time)."""
+    n = 1 << 22
+    rng = np.random.default_rng(dim + k)
+    rows = rng.integers(0, 16, size=(n, dim)).astype(np.float32)
+    means = rows[rng.permutation(n)[:k]].copy()
+    spread = rows + rng.uniform(-0.5, 0.5, size=(n, dim)).astype(np.float32)
+    out = assign_timed(km, rows, means)
+    (_, want), (raster, got) = out[0], out[1]
+    assert np.array_equal(got, want)
+    sample = rng.choice(n, 3000, replace=False)
+    assert np.array_equal(got[sample], orc.assign(np.ascontiguousarray(rows[sample]).ravel(), means.ravel(), dim, k, len(sample), threads=0))
+    even = assign_timed(km, spread, means)[1][0]
+    print("raster %.3f ms, spread %.3f ms" % (raster, even))
+    assert raster <= 1.1 * even, "raster %.3f ms, spread %.3f ms" % (raster, even)
