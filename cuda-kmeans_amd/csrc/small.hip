@@ -46,12 +46,12 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  * dozen centroids at most, which would leave most of the larger tile empty. (A lane per point with the centroids broadcast is
  * bound by the LDS; with the centroids as scalar operands every scalar load waits for all earlier ones: N = 2588, d = 60, k = 1288
  * 135 us.) A few dozen centroids leave most of the time to the trips to memory and the barriers in front of that (N = 65536, d = 8, k = 64: 3 us
- * of vector instructions in 11 us): points and centroids are requested together, and no lane asks for more than there is. With one after the other, each
- * in eight loads a lane whatever there was to load, that call was 25.0 instead of 22.0 us; d = 100, k = 40, N = 30000: 17.2 against 15.6; N = 10240,
- * d = 20, k = 128: 19.5 against 18.9. Floats are held to 64 vector registers, so that a compute unit
- * takes four work-groups (with 76 three: N = 50000, d = 2, k = 10 14.0 against 13.4 us, N = 65000, d = 5, k = 50 10.0 against 9.5). The row stride is an odd number of 16-byte pieces: rows read together start in different banks. Every sum runs in
- * ascending dimension, every operation rounded separately. Global loads are issued in batches of eight per lane: one after the
- * other they cost a microsecond each.
+ * of vector instructions in 11 us): the first four pieces a lane has of points and of centroids are requested together, and no lane asks for more than there
+ * is. With one after the other, each in eight loads a lane whatever there was to load, that call was 25.0 instead of 22.0 us; d = 100, k = 40, N = 30000:
+ * 17.2 against 15.6; N = 10240, d = 20, k = 128: 19.5 against 18.9. Floats are held to 64 vector registers, so that a compute unit takes four work-groups
+ * where their LDS lets it (40 KB each: up to 20 dimensions with a full chunk of centroids, 120 with a dozen; with 76 registers three: N = 50000, d = 2,
+ * k = 10 14.0 against 13.4 us, N = 65000, d = 5, k = 50 10.0 against 9.5). The row stride is an odd number of 16-byte pieces: rows read together start in
+ * different banks. Every sum runs in ascending dimension, every operation rounded separately.
  *
  * SUMS: membership (clusters x 64 points) times rows (64 points x coordinates) on v_mfma_f32_16x16x4_f32: 1.0 times a coordinate is
  * exact, the accumulators add in fp32. A wavefront has 16 clusters and goes over the coordinates 16 at a time; where that leaves
@@ -60,7 +60,6 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  */
 constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading the memberships again (update_small_kernel) is cheaper than as many partial sums */
 constexpr uint32_t SMALL_POINTS = WAVE;
-constexpr int SMALL_BATCH = 4;
 
 /*
  * `count` rows of dim elements on their way to LDS rows of row_stride: AoS rows `stride` apart, or columns (row r of column q at src[q * stride + r];
@@ -72,55 +71,129 @@ struct SmallRows {
 	F* to; const F* src; size_t stride;
 	uint32_t count, last, dim, row_stride, magic; bool vec4;
 };
-template <typename F, int L> __device__ __forceinline__ uint32_t small_items(const SmallRows<F>& s)
-{
-	return L == KMX_SOA ? (s.count + WAVE - 1) / WAVE * s.dim : s.vec4 ? s.count * (s.dim / 4) : s.count * s.dim;
-}
+/* AoS: pieces of four or single coordinates */
+template <typename F> __device__ __forceinline__ uint32_t small_items(const SmallRows<F>& s) { return s.vec4 ? s.count * (s.dim / 4) : s.count * s.dim; }
 
-/* items base, base + 1, .. of every lane (SoA: wavefront): all of them are requested before the first is placed. Lanes without an item ask for nothing:
- * a repeated one costs the caches as much as any (N = 65536, d = 8, k = 64: seven of eight were). */
-template <typename F, int L, int B>
+/* AoS: up to B items of every lane, all of them requested before the first is placed. Lanes without an item ask for nothing: a repeated one costs the
+ * caches as much as any (N = 65536, d = 8, k = 64: seven of eight were). For the first items only: with any number of them in such batches and their
+ * branches N = 94 doubles, d = 186, k = 3 took 9.3 us, with stage_items 7.9; N = 675 doubles, d = 195, k = 108: 58.6, 53.8. */
+template <typename F, int B>
 struct SmallBatch {
 	typedef typename SmallVec<F>::type F4;
 	F4 v[B];
 	uint32_t at[B];
-	static __device__ __forceinline__ uint32_t item(uint32_t i)
+	static __device__ __forceinline__ bool holds(const SmallRows<F>& s) { return small_items(s) <= B * SMALL_THREADS; }
+	__device__ __forceinline__ void request(const SmallRows<F>& s)
 	{
-		return L == KMX_SOA ? i * SMALL_WAVES + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) : i * SMALL_THREADS + threadIdx.x;
-	}
-	__device__ __forceinline__ void request(const SmallRows<F>& s, uint32_t base, uint32_t items)
-	{
+		const uint32_t items = small_items(s);
 #pragma unroll
 		for (int u = 0; u < B; ++u) {
-			const uint32_t i = item(base + u);
+			const uint32_t i = u * SMALL_THREADS + threadIdx.x;
 			if (i >= items) continue;
-			const uint32_t e = L == KMX_AOS && s.vec4 ? i * 4 : i, whole = s.dim == 1 ? e : __umulhi(e, s.magic), q = e - whole * s.dim;
-			const uint32_t r = L == KMX_SOA ? min(whole * WAVE + threadIdx.x % WAVE, s.count - 1) : whole;
-			const F* from = s.src + elem<L>(s.stride, min(r, s.last), q);
+			const uint32_t e = s.vec4 ? i * 4 : i, r = s.dim == 1 ? e : __umulhi(e, s.magic), q = e - r * s.dim;
+			const F* from = s.src + (size_t)min(r, s.last) * s.stride + q;
 			at[u] = r * s.row_stride + q;
-			if (L == KMX_AOS && s.vec4) v[u] = *(const F4*)from;
+			if (s.vec4) v[u] = *(const F4*)from;
 			else v[u].x = *from;
 		}
 	}
-	__device__ __forceinline__ void place(const SmallRows<F>& s, uint32_t base, uint32_t items) const
+	__device__ __forceinline__ void place(const SmallRows<F>& s) const
 	{
+		const uint32_t items = small_items(s);
 #pragma unroll
 		for (int u = 0; u < B; ++u) {
-			if (item(base + u) >= items) continue;
-			if (L == KMX_AOS && s.vec4) *(F4*)(s.to + at[u]) = v[u];
+			if (u * SMALL_THREADS + threadIdx.x >= items) continue;
+			if (s.vec4) *(F4*)(s.to + at[u]) = v[u];
 			else s.to[at[u]] = v[u].x;
 		}
 	}
 };
-template <typename F, int L>
-__device__ __forceinline__ void stage_rows(const SmallRows<F>& s, uint32_t base, uint32_t items)
+
+/*
+ * AoS: the items from the one of that number per lane on, any number of them. A lane's pieces of four: four at a time, none beyond the last (the second and
+ * later chunks of centroids have a piece or two for a lane: N = 8000 doubles, d = 48, k = 300 42.8 us, with repeated ones 44.7). Single coordinates: six at a
+ * time, which is what 64 registers hold, the last one again behind the end: no branches between the loads.
+ */
+template <typename F, bool VEC>
+__device__ __forceinline__ void stage_items(const SmallRows<F>& s, uint32_t from)
 {
-	constexpr uint32_t STEP = L == KMX_SOA ? SMALL_WAVES : SMALL_THREADS;
-	for (; base * STEP < items; base += SMALL_BATCH) {
-		SmallBatch<F, L, SMALL_BATCH> batch;
-		batch.request(s, base, items);
-		batch.place(s, base, items);
+	typedef typename std::conditional<VEC, typename SmallVec<F>::type, F>::type V;
+	constexpr int BATCH = VEC ? 4 : 6;
+	const uint32_t last = small_items(s) - 1, one = s.dim == 1 ? 1u : 0u; /* (magic is 0 for rows of one) */
+	for (uint32_t i0 = from * SMALL_THREADS + threadIdx.x; i0 <= last; i0 += SMALL_THREADS * BATCH) {
+		V v[BATCH];
+		uint32_t at[BATCH];
+#pragma unroll
+		for (int u = 0; u < BATCH; ++u) {
+			const uint32_t i = i0 + u * SMALL_THREADS;
+			if (VEC && i > last) continue;
+			const uint32_t e = min(i, last) * (VEC ? 4 : 1), r = __umulhi(e, s.magic) + e * one, q = e - r * s.dim;
+			at[u] = r * s.row_stride + q;
+			v[u] = *(const V*)(s.src + (size_t)min(r, s.last) * s.stride + q);
+		}
+#pragma unroll
+		for (int u = 0; u < BATCH; ++u)
+			if (!VEC || i0 + u * SMALL_THREADS <= last) *(V*)(s.to + at[u]) = v[u];
 	}
+}
+
+/*
+ * Columns: a wavefront takes 64 rows of one at a time. Wide rows: eight columns under way, the last one again behind the end. Rows of fewer than two columns per
+ * wavefront: blocks of 64 rows follow one another without a pause, and wavefronts beyond the columns take blocks of their own (the first way and this,
+ * us: N = 21376, d = 2, k = 287 18.7, 17.6; N = 2550, d = 8, k = 284 15.0, 13.6; N = 43539, d = 9, k = 111 14.5, 13.6; but N = 53567, d = 42, k = 32 12.4, 13.3;
+ * N = 3895, d = 252, k = 2 10.0, and 15.7 in batches of four).
+ */
+template <typename F>
+__device__ __forceinline__ void stage_columns(const SmallRows<F>& s)
+{
+	constexpr uint32_t BATCH = 8;
+	const uint32_t lane = threadIdx.x % WAVE, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+	if (s.dim >= 2 * SMALL_WAVES) {
+		for (uint32_t r0 = 0; r0 < s.count; r0 += WAVE) {
+			const uint32_t r = min(r0 + lane, s.count - 1);
+			const F* src = s.src + min(r, s.last);
+			for (uint32_t q0 = wave; q0 < s.dim; q0 += SMALL_WAVES * BATCH) {
+				F v[BATCH];
+#pragma unroll
+				for (uint32_t u = 0; u < BATCH; ++u) v[u] = src[(size_t)min(q0 + u * SMALL_WAVES, s.dim - 1) * s.stride];
+#pragma unroll
+				for (uint32_t u = 0; u < BATCH; ++u) s.to[r * s.row_stride + min(q0 + u * SMALL_WAVES, s.dim - 1)] = v[u];
+			}
+		}
+		return;
+	}
+	/* groups of wavefronts, each with all columns of its blocks (one group where the columns are as many as wavefronts) */
+	const bool few = s.dim < SMALL_WAVES;
+	const uint32_t group = !few ? 0 : s.dim == 1 ? wave : __umulhi(wave, s.magic), groups = !few ? 1 : s.dim == 1 ? SMALL_WAVES : __umulhi(SMALL_WAVES, s.magic);
+	const uint32_t first = wave - group * s.dim;
+	uint32_t q = first, r0 = group < groups ? group * WAVE : s.count;
+	while (r0 < s.count) {
+		F v[BATCH];
+		uint32_t at[BATCH], got = 0;
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u) {
+			if (r0 >= s.count) continue;
+			const uint32_t r = min(r0 + lane, s.count - 1);
+			at[u] = r * s.row_stride + q;
+			v[u] = s.src[(size_t)q * s.stride + min(r, s.last)];
+			got = u + 1;
+			q += SMALL_WAVES;
+			const bool wrap = q >= s.dim;
+			q = wrap ? first : q;
+			r0 += wrap ? groups * WAVE : 0u;
+		}
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u)
+			if (u < got) s.to[at[u]] = v[u];
+	}
+}
+
+template <typename F, int L>
+__device__ __forceinline__ void stage_rows(const SmallRows<F>& s, uint32_t from)
+{
+	if (L == KMX_SOA) stage_columns(s);
+	else if (s.vec4) stage_items<F, true>(s, from);
+	else stage_items<F, false>(s, from);
 }
 
 template <typename F, int T, int LD, int LM, bool SUMS>
@@ -151,19 +224,27 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 		return SmallRows<F>{ cents, LM == KMX_AOS ? means + (size_t)base * stride_means : means + base, stride_means, count, count - 1, dim, row_stride, magic, (vec4 & 2u) != 0 };
 	};
 	{
-		/* points and centroids travel together, up to 4 items a lane of each: one trip to memory where there were two */
 		const SmallRows<F> points = { rows, LD == KMX_AOS ? data + (size_t)first * stride : data + first, stride, POINTS, here - 1, dim, row_stride, magic, (vec4 & 1u) != 0 };
 		const SmallRows<F> start = centroids(0);
-		const uint32_t point_items = small_items<F, LD>(points), start_items = small_items<F, LM>(start);
-		constexpr int TOGETHER = 4;
-		SmallBatch<F, LD, TOGETHER> some;
-		SmallBatch<F, LM, TOGETHER> others;
-		some.request(points, 0, point_items);
-		others.request(start, 0, start_items);
-		some.place(points, 0, point_items);
-		others.place(start, 0, start_items);
-		stage_rows<F, LD>(points, TOGETHER, point_items);
-		stage_rows<F, LM>(start, TOGETHER, start_items);
+		uint32_t staged = 0; /* items of a lane */
+		bool rest = true;
+		if constexpr (LD == KMX_AOS && LM == KMX_AOS) {
+			/* points and centroids travel together where all of them do, or where both are whole pieces: one trip to memory instead of two */
+			typedef SmallBatch<F, 4> Batch;
+			rest = !(Batch::holds(points) && Batch::holds(start));
+			if (!rest || (points.vec4 && start.vec4)) {
+				Batch some, others;
+				some.request(points);
+				others.request(start);
+				some.place(points);
+				others.place(start);
+				staged = 4;
+			}
+		}
+		if (rest) {
+			stage_rows<F, LD>(points, staged);
+			stage_rows<F, LM>(start, staged);
+		}
 	}
 
 	F low[T];
@@ -175,8 +256,7 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 		const uint32_t count = min(chunk, k - base);
 		if (base) {
 			__syncthreads(); /* the previous chunk is no longer needed */
-			const SmallRows<F> next = centroids(base);
-			stage_rows<F, LM>(next, 0, small_items<F, LM>(next));
+			stage_rows<F, LM>(centroids(base), 0);
 		}
 		__syncthreads();
 		for (uint32_t c0 = cw * (4 * T); c0 < count; c0 += CW * (4 * T)) {

@@ -91,3 +91,38 @@ def test_small_update(km, gpu, dtype, dim, k, n, layout, layout_means, kind):
     assert np.abs(got - truth).max() < (1e-5 if dtype == np.float32 else 1e-13) * max(1.0, np.abs(truth).max())
     for b in (d, a, m, sizes):
         b.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dim,k,n", [(1, 600, 700), (3, 130, 140), (7, 200, 210), (8, 129, 140), (9, 128, 140), (15, 193, 200), (16, 193, 200), (17, 65, 70),   # blocks of 64 rows
+                                     (49, 130, 140), (50, 63, 70)])   # six single coordinates a lane at a time, eight columns a wavefront
+@pytest.mark.parametrize("layout,layout_means", [(0, 0), (1, 1), (1, 0)])
+def test_small_staging_of_columns_and_single_coordinates(km, orc, gpu, dtype, dim, k, n, layout, layout_means):
+    test_small_assignment_and_iteration(km, orc, gpu, dtype, dim, k, n, layout, layout_means)
+
+
+@pytest.mark.parametrize("dim,k,n", [(252, 2, 3895), (100, 5, 3750)])
+def test_columns_cost_little_more_than_rows(km, gpu, dim, k, n):
+    """Points and centroids in columns beside the same in rows: staging them costs the same number of trips to memory (1.1 to 1.2
+    times the rows' call; it was 1.5 to 1.9 times while columns went in batches of four with branches between the loads)."""
+    rng = np.random.default_rng(dim)
+    rows, means = rng.normal(size=(n, dim)).astype(np.float32), rng.normal(size=(k, dim)).astype(np.float32)
+    a = km.DeviceBuffer(4 * n)
+    start, stop = km.Event(), km.Event()
+    took = []
+    for layout in (0, 1):
+        d = km.DeviceBuffer(rows.nbytes); d.write(np.ascontiguousarray(rows if layout == 0 else rows.T).ravel())
+        m = km.DeviceBuffer(means.nbytes); m.write(np.ascontiguousarray(means if layout == 0 else means.T).ravel())
+        times = []
+        for series in range(9):
+            start.record()
+            for _ in range(100):
+                km.assign(km.ASSIGN_BEST, d, layout, km.layout_stride(layout, n, dim), m, layout, km.layout_stride(layout, k, dim), a, dim, k, n)
+            stop.record()
+            km.sync()
+            times.append(start.elapsed_ms(stop) * 10)
+        took.append(float(np.median(times[1:])))
+        d.free(); m.free()
+    a.free()
+    print("rows %.2f us, columns %.2f us" % tuple(took))
+    assert took[1] <= 1.4 * took[0], "rows %.2f us, columns %.2f us" % tuple(took)
