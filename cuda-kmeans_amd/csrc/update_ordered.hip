@@ -15,7 +15,7 @@
  * reference's serial run. The price is the length of the longest chain: a cluster of m members is m dependent
  * additions, whatever the machine.
  *
- * Kernels: ordered_histogram_kernel, ordered_offsets_kernel, ordered_starts_kernel, ordered_scatter_kernel / ordered_scatter_group_kernel,
+ * Kernels: ordered_histogram_kernel, ordered_offsets_kernel, ordered_starts_kernel, ordered_scatter_kernel / ordered_scatter_group_kernel, ordered_large_kernel,
  * ordered_stream_sum_kernel / ordered_staged_sum_kernel / ordered_sum_kernel.
  */
 #include "kmx_internal.h"
@@ -290,20 +290,41 @@ ordered_scatter_group_kernel(const uint32_t* __restrict__ assignment, const uint
 	}
 }
 
+/* large[0] = how many clusters have at least `least` members, then their numbers in no particular order: one work-group, 1024 clusters per step */
+__global__ void __launch_bounds__(1024)
+ordered_large_kernel(const uint32_t* __restrict__ sizes, uint32_t* __restrict__ large, uint32_t k, uint32_t least)
+{
+	__shared__ uint32_t count;
+	if (threadIdx.x == 0) count = 0u;
+	__syncthreads();
+	constexpr uint32_t BATCH = 4; /* loads in flight */
+	for (uint32_t c0 = threadIdx.x; c0 < k; c0 += BATCH * 1024) {
+		uint32_t members[BATCH];
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u) members[u] = c0 + u * 1024 < k ? sizes[c0 + u * 1024] : 0u;
+#pragma unroll
+		for (uint32_t u = 0; u < BATCH; ++u)
+			if (members[u] >= least) large[1 + atomicAdd(&count, 1u)] = c0 + u * 1024;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) large[0] = count;
+}
+
 /*
  * One lane per cluster and piece of VEC consecutive coordinates (VEC = 1, or a 16-byte piece of an AoS row): the members'
  * coordinates added one after the other in the order of the sorted list, i.e. in ascending point number, starting from
  * zero like the serial loop (serial.hpp:57-63), then the guarded divide (serial.hpp:65-71). The additions of a
  * coordinate are a chain; what can overlap are the loads: the pieces of UNROLL rows are in flight together, and the
  * point numbers of the next UNROLL rows are requested before the current ones are added (a chain is as many sums as
- * the machine runs at once here, so the time is the latency of a load divided by the loads in flight).
+ * the machine runs at once here, so the time is the latency of a load divided by the loads in flight). Clusters of `most` members and more
+ * are left out.
  */
 template <typename F, int VEC> struct alignas(sizeof(F) * VEC) OrderedPiece { F v[VEC]; };
 
 template <typename F, int LD, int LM, int VEC, int UNROLL>
 __global__ void __launch_bounds__(64)
 ordered_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ starts,
-                   const uint32_t* __restrict__ sizes, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t k, uint32_t divide)
+                   const uint32_t* __restrict__ sizes, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t k, uint32_t divide, uint32_t most)
 {
 	static_assert(VEC == 1 || LD == KMX_AOS, "pieces of several coordinates are pieces of AoS rows");
 	typedef OrderedPiece<F, VEC> piece_t;
@@ -312,6 +333,7 @@ ordered_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __
 	if (e >= (size_t)k * pieces) return;
 	const uint32_t c = (uint32_t)(e / pieces), d = (uint32_t)(e % pieces) * VEC;
 	const uint32_t members = sizes[c];
+	if (members >= most) return; /* left to ordered_stream_sum_kernel */
 	const uint32_t begin = starts[c], end = begin + members;
 	piece_t sum;
 #pragma unroll
@@ -430,7 +452,7 @@ ordered_staged_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
 }
 
 /*
- * The same for AoS rows of whole 16-byte pieces: a work-group per cluster and block of 128 bytes of the row. One wavefront requests the members'
+ * The same for AoS rows of whole 16-byte pieces: a work-group per cluster (`large`: of that list only) and block of 128 bytes of the row. One wavefront requests the members'
  * rows straight to LDS, AHEAD batches of eight requests before they are added, and the members' numbers AHEAD batches before that; the other one
  * adds, a lane per coordinate, two members per LDS read, and waits for nothing but the batch's barrier. What bounds it is the longest
  * cluster's chain, at 1.5 instructions a member (N = 100k, d = 36, k = 2: 4.9 ns a member; with one wavefront that requests and adds 7.8), then the memory
@@ -459,12 +481,13 @@ __device__ __forceinline__ void stream_request4(const void* from, uint32_t to)
 template <typename F, int LM, uint32_t P, bool DEEP>
 __global__ void __launch_bounds__(STREAM_THREADS)
 ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ starts,
-                          const uint32_t* __restrict__ sizes, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t blocks, uint32_t divide)
+                          const uint32_t* __restrict__ sizes, const uint32_t* __restrict__ large, F* __restrict__ means, size_t stride_means, uint32_t dim, uint32_t blocks, uint32_t divide)
 {
 	constexpr uint32_t PIECE = 16 / sizeof(F), BLOCK = STREAM_BLOCK_BYTES / sizeof(F), ROWS = stream_rows(P), BATCH = stream_batch(P), NAMES = stream_names(P);
 	constexpr uint32_t AHEAD = stream_ahead(P, DEEP), SLOTS = AHEAD + 1, EACH = STREAM_REQUESTS + NAMES;
 	extern __shared__ __attribute__((aligned(16))) char stream_lds[];
-	const uint32_t c = blockIdx.x / blocks, d0 = blockIdx.x % blocks * BLOCK, width = min(BLOCK, dim - d0); /* (whole pieces, no more than P) */
+	if (large && blockIdx.x / blocks >= large[0]) return;
+	const uint32_t c = large ? large[1 + blockIdx.x / blocks] : blockIdx.x / blocks, d0 = blockIdx.x % blocks * BLOCK, width = min(BLOCK, dim - d0); /* (whole pieces, no more than P) */
 	const uint32_t members = sizes[c], begin = starts[c], lane = threadIdx.x % WAVE;
 	if (__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) != 0) { /* requests */
 		if (members == 0) return;
@@ -566,18 +589,24 @@ ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
  * work-groups of four wavefronts with 16-byte pieces 0.85 ms). The 16-byte pieces, which need a quarter of the lanes, are
  * taken only where they still leave two wavefronts per compute unit. */
 template <typename F, int LD, int LM>
-static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sorted, const uint32_t* starts, const uint32_t* sizes,
+static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sorted, const uint32_t* starts, const uint32_t* sizes, uint32_t* large,
                               F* means, size_t stride_means, uint32_t dim, uint32_t k, uint32_t n, bool divide, const DeviceInfo& dev)
 {
 	constexpr int WIDE = 16 / sizeof(F);
 	const bool fits = LD == KMX_AOS && dim % WIDE == 0 && stride % WIDE == 0 && ((uintptr_t)data & 15) == 0;
 	const OrderedSumRoute route = ordered_sum_route(sizeof(F), fits && stride <= 0xFFFFFFFFu / sizeof(F), dim, k, n);
-	const uint32_t groups = k * route.blocks;
+	uint32_t most = 0xFFFFFFFFu; /* members of a cluster that ordered_sum_kernel does not take */
 	if constexpr (LD == KMX_AOS) {
-		if (route.kernel == ORDERED_STREAM) {
-			const uint32_t pieces = std::min<uint32_t>(dim / WIDE, STREAM_BLOCK_BYTES / 16);
+		if (route.kernel == ORDERED_STREAM || route.kernel == ORDERED_SPLIT) {
+			const bool split = route.kernel == ORDERED_SPLIT;
+			if (split) {
+				most = ORDERED_LARGE;
+				KMX_LAUNCH_KERNEL(ordered_large_kernel, dim3(1), dim3(1024), 0, stream(), sizes, large, k, most);
+				KMX_LAUNCH_CHECK("ordered_large_kernel");
+			}
+			const uint32_t pieces = std::min<uint32_t>(dim / WIDE, STREAM_BLOCK_BYTES / 16), groups = (split ? ordered_most_large(n) : k) * route.blocks;
 			const bool deep = groups <= 2 * dev.compute_units;
-			void (*kernel)(const F*, size_t, const uint32_t*, const uint32_t*, const uint32_t*, F*, size_t, uint32_t, uint32_t, uint32_t) = nullptr;
+			void (*kernel)(const F*, size_t, const uint32_t*, const uint32_t*, const uint32_t*, const uint32_t*, F*, size_t, uint32_t, uint32_t, uint32_t) = nullptr;
 			uint32_t lds = 0;
 			auto take = [&](auto tag) {
 				constexpr uint32_t P = decltype(tag)::value;
@@ -588,13 +617,13 @@ static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sort
 			take(std::integral_constant<uint32_t, 1>{}); take(std::integral_constant<uint32_t, 2>{}); take(std::integral_constant<uint32_t, 3>{}); take(std::integral_constant<uint32_t, 4>{});
 			take(std::integral_constant<uint32_t, 5>{}); take(std::integral_constant<uint32_t, 6>{}); take(std::integral_constant<uint32_t, 7>{}); take(std::integral_constant<uint32_t, 8>{});
 			KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-			KMX_LAUNCH_KERNEL(kernel, dim3(groups), dim3(STREAM_THREADS), lds, stream(), data, stride, sorted, starts, sizes, means, stride_means, dim, route.blocks, divide ? 1u : 0u);
+			KMX_LAUNCH_KERNEL(kernel, dim3(groups), dim3(STREAM_THREADS), lds, stream(), data, stride, sorted, starts, sizes, split ? (const uint32_t*)large : nullptr, means, stride_means, dim, route.blocks, divide ? 1u : 0u);
 			KMX_LAUNCH_CHECK("ordered_stream_sum_kernel");
-			return KMX_OK;
+			if (!split) return KMX_OK;
 		}
 	}
 	if (route.kernel == ORDERED_STAGED) {
-		const uint32_t block_dims = route.block_dims;
+		const uint32_t block_dims = route.block_dims, groups = k * route.blocks;
 		const bool elements = LD == KMX_SOA || dim < (uint32_t)WIDE || (dim % block_dims != 0 && dim % block_dims < (uint32_t)WIDE);
 		const uint32_t lds = STAGED_THREADS * STAGED_PIECES * (elements ? sizeof(F) : 16) + std::min(dim, block_dims) * 16;
 		auto kernel = elements ? ordered_staged_sum_kernel<F, LD, LM, true> : ordered_staged_sum_kernel<F, KMX_AOS, LM, false>;
@@ -608,10 +637,10 @@ static int launch_ordered_sum(const F* data, size_t stride, const uint32_t* sort
 	const dim3 grid((uint32_t)((total + WAVE - 1) / WAVE));
 	if (wide)
 		KMX_LAUNCH_KERNEL((ordered_sum_kernel<F, KMX_AOS, LM, WIDE, 32>), grid, dim3(WAVE), 0, stream(),
-		                   data, stride, sorted, starts, sizes, means, stride_means, dim, k, divide ? 1u : 0u);
+		                   data, stride, sorted, starts, sizes, means, stride_means, dim, k, divide ? 1u : 0u, most);
 	else
 		KMX_LAUNCH_KERNEL((ordered_sum_kernel<F, LD, LM, 1, 32>), grid, dim3(WAVE), 0, stream(),
-		                   data, stride, sorted, starts, sizes, means, stride_means, dim, k, divide ? 1u : 0u);
+		                   data, stride, sorted, starts, sizes, means, stride_means, dim, k, divide ? 1u : 0u, most);
 	KMX_LAUNCH_CHECK("ordered_sum_kernel");
 	return KMX_OK;
 }
@@ -683,10 +712,11 @@ int launch_update_serial_order(const F* data, int layout, size_t stride, const u
 			KMX_LAUNCH_KERNEL((ordered_scatter_kernel<false>), dim3(chunks), dim3(WAVE), 0, stream(), assignment, hist, starts, sorted, k, n, chunk_points);
 		KMX_LAUNCH_CHECK("ordered_scatter_kernel");
 	}
-	if (layout == KMX_AOS && layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
-	else if (layout == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
-	else if (layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_SOA, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
-	else rc = launch_ordered_sum<F, KMX_SOA, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, means, stride_means, dim, k, n, divide, dev);
+	/* (the histograms are no longer needed: their first words take the list of the large clusters) */
+	if (layout == KMX_AOS && layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, hist, means, stride_means, dim, k, n, divide, dev);
+	else if (layout == KMX_AOS) rc = launch_ordered_sum<F, KMX_AOS, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, hist, means, stride_means, dim, k, n, divide, dev);
+	else if (layout_means == KMX_AOS) rc = launch_ordered_sum<F, KMX_SOA, KMX_AOS>(data, stride, sorted, starts, cluster_sizes, hist, means, stride_means, dim, k, n, divide, dev);
+	else rc = launch_ordered_sum<F, KMX_SOA, KMX_SOA>(data, stride, sorted, starts, cluster_sizes, hist, means, stride_means, dim, k, n, divide, dev);
 	if (rc) return rc;
 	return profile_end(1);
 }
