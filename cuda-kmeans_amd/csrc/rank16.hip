@@ -160,7 +160,7 @@ static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Works
 	const float* norms = ws->norms16;
 	const Rank16Args w = { a.data, a.stride, (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp), norms + rank16_frame_offset(kp), ws->norms16 + rank16_scale_offset(kp),
 	                       a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->queued_rows, copy_stride, a.dim, a.k, kp, a.n, 0,
-	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + 8.0f * CERT_UNIT + a.kd_extra };
+	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + 8.0f * CERT_UNIT + a.kd_extra, 0 };
 	switch (kb) {
 	case 1: return launch_rank16_1(a, w, exec, ws, dev);
 	case 2: return launch_rank16_2(a, w, exec, ws, dev);

@@ -43,6 +43,7 @@ struct Rank16Args {
 	float* copies; uint32_t copy_stride; /* SoA: the rows as AoS, zeros behind the coordinates */
 	uint32_t dim, k, kp, n, chunk_tiles;
 	float kd;
+	uint32_t list_entries; /* of a wavefront's list, resident centroids */
 };
 
 /* ws->packed16: the operands, then the centroids' rows as they are, padded with zeros to whole blocks */
@@ -56,8 +57,15 @@ inline size_t rank16_norms_floats(uint32_t kp) { return rank16_scale_offset(kp) 
 
 /* 16 tile bytes per block of 16 dimensions and lane, then the tile's norms */
 template <int KB> constexpr uint32_t rank16_tile_floats() { return KB * WAVE * 4; }
-/* listed points a wavefront keeps in LDS before they go out */
-constexpr uint32_t rank16_list(uint32_t kb, int layout, bool stream) { return rank16_waves(kb, layout, stream) == 12 ? 80 : 120; }
+/*
+ * Listed points a wavefront keeps in LDS before they go out, 32 of a tile at most at a time. Going out is an addition to one word in memory, of which
+ * the card makes one in 5.3 ns: where nearly every point is listed (coordinates that are all 0 or 1) that bounds the launch (N = 1M, d = 16, k = 256:
+ * 156 us a call with lists of 80, which go out at 64; 125 with 128). Around resident centroids the lists take what the centroids leave of LDS, up to 128.
+ */
+constexpr uint32_t RANK16_LIST_STREAMED = 120, RANK16_LIST_MOST = 128;
+/* the least, before the centroids stream by instead. Rows of more than 128 dimensions are no slower that way (N = 262144, d = 256, k = 285, SoA: 177
+ * streamed, 193 resident, where the registers do not hold everything), rows of up to 128 are (d = 40, k = 1500, SoA: 86, 79) */
+constexpr uint32_t rank16_list_least(uint32_t kb) { return kb >= 12 ? 120 : 64; }
 constexpr uint32_t rank16_slots(uint32_t kb) { return kb >= 12 ? 4 : 2; }
 __host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { return (tiles * NORM_TILE + WAVE - 1) / WAVE; }
 /* what a chunk takes in LDS, its norms behind its operands as whole requests of 64 words */
@@ -65,7 +73,9 @@ __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t t
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
 constexpr uint32_t rank16_exchange(uint32_t kb, int layout) { return rank16_shared_rows(kb, layout) || layout == KMX_SOA ? RANK16_EXCHANGE : 0; }
-constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream) { return ((2 * rank16_list(kb, layout, stream) + rank16_exchange(kb, layout) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
+/* the lists of a work-group around resident centroids, lying behind them */
+constexpr uint32_t rank16_list_bytes(uint32_t kb, int layout, uint32_t entries) { return rank16_waves(kb, layout, false) * entries * 8; }
 constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
@@ -340,7 +350,7 @@ template <int KB, int LD, bool STREAM>
 __global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM) * WAVE, rank16_waves(KB, LD, STREAM) == 12 ? 3 : 2)
 rank16_kernel(const Rank16Args w)
 {
-	constexpr uint32_t WAVES = rank16_waves(KB, LD, STREAM), THREADS = WAVES * WAVE, LIST = rank16_list(KB, LD, STREAM);
+	constexpr uint32_t WAVES = rank16_waves(KB, LD, STREAM), THREADS = WAVES * WAVE;
 	constexpr int P = RANK16_P;
 	constexpr uint32_t TF = rank16_tile_floats<KB>();
 	constexpr bool PIPE = !STREAM && KB <= 4;
@@ -350,7 +360,7 @@ rank16_kernel(const Rank16Args w)
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
 	__shared__ uint32_t wave_max[4][WAVES];
-	__shared__ uint32_t flag_list[WAVES][2 * LIST];
+	__shared__ uint32_t streamed_lists[STREAM ? WAVES : 1][STREAM ? 2 * RANK16_LIST_STREAMED : 1];
 	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD) ? RANK16_EXCHANGE : 1];
 	uint32_t& claimed = wave_max[3][0];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
@@ -397,6 +407,8 @@ rank16_kernel(const Rank16Args w)
 	}
 	__syncthreads();
 
+	const uint32_t list_entries = STREAM ? RANK16_LIST_STREAMED : w.list_entries;
+	uint32_t* const flag_list = STREAM ? streamed_lists[wave] : (uint32_t*)lds + (size_t)w.chunk_tiles * (TF + NORM_TILE) + wave * 2 * list_entries;
 	uint32_t flagged = 0; /* wave-uniform */
 	auto flush_flags = [&]() {
 		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -404,7 +416,7 @@ rank16_kernel(const Rank16Args w)
 		uint32_t slot = 0;
 		if (lane == 0) slot = atomicAdd(w.length, flagged);
 		slot = (uint32_t)__shfl((int)slot, 0);
-		for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[2 * (size_t)slot + i] = flag_list[wave][i];
+		for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[2 * (size_t)slot + i] = flag_list[i];
 		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 		__builtin_amdgcn_wave_barrier();
 		flagged = 0;
@@ -524,11 +536,11 @@ rank16_kernel(const Rank16Args w)
 			const unsigned long long mask = __ballot(flag);
 			if (mask) {
 				const uint32_t add = (uint32_t)__builtin_popcountll(mask);
-				if (flagged + add > LIST) flush_flags();
+				if (flagged + add > list_entries) flush_flags();
 				if (flag) {
 					const uint32_t at = 2 * (flagged + (uint32_t)__builtin_popcountll(mask & ((1ull << lane) - 1ull)));
-					flag_list[wave][at] = pt;
-					flag_list[wave][at + 1] = screening_threshold(extreme ? __builtin_inff() : lowest, tau); /* (scaled, like the values) */
+					flag_list[at] = pt;
+					flag_list[at + 1] = screening_threshold(extreme ? __builtin_inff() : lowest, tau); /* (scaled, like the values) */
 				}
 				flagged += add;
 			}
@@ -792,7 +804,7 @@ rank16_kernel(const Rank16Args w)
 	if (tid == 0) wave_max[1][0] = atomicAdd(w.length, all);
 	__syncthreads();
 	const size_t slot = 2 * (size_t)(wave_max[1][0] + before);
-	for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[slot + i] = flag_list[wave][i];
+	for (uint32_t i = lane; i < 2 * flagged; i += WAVE) w.list[slot + i] = flag_list[i];
 }
 
 template <int KB>
@@ -800,9 +812,12 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 {
 	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4, tiles = w.kp / TILE, budget = lds_budget_of(exec, dev);
 	if (budget < rank16_least_bytes(KB, a.layout)) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
-	const bool stream_mode = (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false) > budget;
+	const uint64_t resident = (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false);
+	const bool stream_mode = resident + rank16_list_bytes(KB, a.layout, rank16_list_least(KB)) > budget;
 	w.chunk_tiles = tiles;
-	uint32_t lds_bytes = tiles * tile_bytes;
+	w.list_entries = RANK16_LIST_MOST;
+	while (!stream_mode && resident + rank16_list_bytes(KB, a.layout, w.list_entries) > budget) --w.list_entries;
+	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, a.layout, w.list_entries);
 	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode);
 	if (stream_mode) {
 		w.chunk_tiles = 1;
@@ -819,6 +834,7 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 	if (!sizing_only()) {
 		KMX_PLAN(w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1 && KB * KBLOCK >= a.dim);
 		KMX_PLAN(w.chunk_tiles >= 1 && (uint64_t)lds_bytes + static_bytes <= dev.lds_bytes && rank16_tile_floats<KB>() % 4 == 0);
+		KMX_PLAN(stream_mode || (w.list_entries >= RANK16_P * TILE / 2 && rank16_waves(KB, a.layout, false) * 2 * w.list_entries + tiles * (tile_bytes / 4) <= lds_bytes / 4));
 		KMX_PLAN(ws->packed16 && (size_t)tiles * KB * WAVE * 4 <= ws->packed16_cap);
 		KMX_PLAN(!stream_mode || ((rank16_slots(KB) == 2 || w.chunk_tiles == 1) && /* whole requests of norms, the last chunk's too */
 		                          (size_t)(tiles - 1) / w.chunk_tiles * w.chunk_tiles * NORM_TILE + rank16_norm_blocks(w.chunk_tiles) * WAVE <= ws->norms16_cap));

@@ -128,3 +128,32 @@ def test_centroids_that_stream_by(km, orc, gpu, dim, k, n, budget):
     finally:
         km.set_two_level_sweep(1)
     m.free(); a.free()
+
+
+@pytest.mark.parametrize("dim,k,budget", [
+    (16, 1184, 56 * 1024), (16, 1344, 56 * 1024), (16, 1345, 56 * 1024),   # the longest lists, shorter ones, centroids that stream by instead
+    (32, 640, 56 * 1024), (30, 704, 56 * 1024), (48, 470, 56 * 1024), (61, 350, 56 * 1024), (96, 230, 56 * 1024), (128, 160, 56 * 1024),
+    (200, 60, 78 * 1024), (16, 64, 0),
+])
+def test_lists_that_share_lds_with_the_centroids(km, orc, gpu, dim, k, budget):
+    """Every centroid twice: all points are listed, more of them per wavefront than its list holds, whatever the centroids leave for it."""
+    n = 263003
+    rng = np.random.default_rng(dim + k)
+    means = np.repeat(rng.normal(size=((k + 1) // 2, dim)), 2, axis=0)[:k].astype(np.float32)
+    rows = (means[rng.integers(0, k, n)] + rng.normal(size=(n, dim)) * 0.5).astype(np.float32)
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 0))
+    a = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for layout in (0, 1):
+            d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, layout))
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, layout, km.layout_stride(layout, n, dim), m, 0, dim, a, dim, k, n, km.ExecParams(shared_mem_bytes=budget))
+            km.sync()
+            got = a.read(np.uint32, n)
+            d.free()
+            assert np.array_equal(got, want), "layout %d: %d mismatches" % (layout, int((got != want).sum()))
+    finally:
+        km.set_two_level_sweep(1)
+    m.free(); a.free()
