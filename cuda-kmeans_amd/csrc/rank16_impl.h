@@ -72,11 +72,12 @@ __host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { retu
 __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t tiles) { return tiles * kb * WAVE * 16 + rank16_norm_blocks(tiles) * WAVE * 4; }
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
-constexpr uint32_t rank16_exchange(uint32_t kb, int layout) { return rank16_shared_rows(kb, layout) || layout == KMX_SOA ? RANK16_EXCHANGE : 0; }
-constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
+/* direct: SoA rows are not exchanged (rank16_copy) */
+constexpr uint32_t rank16_exchange(uint32_t kb, int layout, bool direct) { return rank16_shared_rows(kb, layout) || (layout == KMX_SOA && !direct) ? RANK16_EXCHANGE : 0; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, bool direct) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, direct) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
 /* the lists of a work-group around resident centroids, lying behind them */
 constexpr uint32_t rank16_list_bytes(uint32_t kb, int layout, uint32_t entries) { return rank16_waves(kb, layout, false) * entries * 8; }
-constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
+constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true, false) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
  * S for centroids whose coordinates are up to `far` from the frame and up to `size` from the origin, both of a sample: the power of two
@@ -187,10 +188,21 @@ __device__ __forceinline__ void rank16_exchanged() /* LDS keeps the order of a w
  * SoA: the rows go out as AoS on the way, for the exact pass and whatever else reads single rows (coordinates of a listed point lie a
  * cache line each apart; with 9 % of N = 2M, d = 128 listed, gathering them read all data again, 430 us, and was no cheaper right
  * behind the sweep of the point, 360 us. The stores travel behind the matrix instructions). Through LDS, so that four lanes store 64
- * consecutive bytes of a row. `exchange`: RANK16_EXCHANGE words of this wavefront's.
+ * consecutive bytes of a row. `exchange`: RANK16_EXCHANGE words of this wavefront's. Where resident centroids leave no room for it a lane stores
+ * its 32 bytes as they are (DIRECT): the centroids would have to stream by otherwise (N = 1M, d = 12, k = 4000 262 us, streamed 368; d = 40,
+ * k = 1536 249, 283; d = 64, k = 1150 255, 295; with room for it, d = 64, k = 256, 170 through LDS, 183 without).
  */
+template <bool DIRECT>
 __device__ __forceinline__ void rank16_copy(const Rank16Args& w, const float (&v)[8], uint32_t tile_first, uint32_t kb, uint32_t lane, float* exchange)
 {
+	if (DIRECT) {
+		const uint32_t pt = tile_first + lane % TILE, d = kb * KBLOCK + lane / TILE * 8;
+		if (pt >= w.n || d >= w.copy_stride) return;
+		float* to = w.copies + (size_t)pt * w.copy_stride + d;
+		*(f32x4*)to = f32x4{ v[0], v[1], v[2], v[3] };
+		*(f32x4*)(to + 4) = f32x4{ v[4], v[5], v[6], v[7] };
+		return;
+	}
 	/* half of the tile at a time, 16 words a row in pieces of four; row r's piece q lies in the place q ^ (r / 2 % 4) of the row, which spreads a
 	 * column over the banks */
 	const uint32_t col = lane % TILE, h = lane / TILE, turn = col / 2 % 4, row = lane / 4, d = kb * KBLOCK + lane % 4 * 4;
@@ -346,7 +358,7 @@ __device__ __forceinline__ float rank16_both(float v)
  * Rows of up to 64 dimensions and resident centroids: two accumulator sets, the tracking of one tile in pieces behind the matrix
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
-template <int KB, int LD, bool STREAM>
+template <int KB, int LD, bool STREAM, bool DIRECT>
 __global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM) * WAVE, rank16_waves(KB, LD, STREAM) == 12 ? 3 : 2)
 rank16_kernel(const Rank16Args w)
 {
@@ -361,7 +373,7 @@ rank16_kernel(const Rank16Args w)
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
 	__shared__ uint32_t wave_max[4][WAVES];
 	__shared__ uint32_t streamed_lists[STREAM ? WAVES : 1][STREAM ? 2 * RANK16_LIST_STREAMED : 1];
-	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD) ? RANK16_EXCHANGE : 1];
+	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD, DIRECT) ? RANK16_EXCHANGE : 1];
 	uint32_t& claimed = wave_max[3][0];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
@@ -455,7 +467,7 @@ rank16_kernel(const Rank16Args w)
 			__builtin_amdgcn_sched_barrier(0);
 			float (&v)[8] = raw[at % DEPTH];
 			if (!WHOLE) rank16_place<LD, SHARED>(v, kb, lane, dim);
-			if (LD == KMX_SOA) rank16_copy(w, v, first + p * TILE, kb, lane, exchange);
+			if (LD == KMX_SOA) rank16_copy<DIRECT>(w, v, first + p * TILE, kb, lane, exchange);
 			rank16_convert<SHARED>(b[p][kb], v, frame, scale, kb, lane, sums[p], exchange);
 			if (!SHARED) asm volatile("" : "+v"(b[p][kb]));
 			/* the sums exist here: left alone the compiler moves them behind the sweep and keeps the coordinates alive */
@@ -679,7 +691,7 @@ rank16_kernel(const Rank16Args w)
 #pragma unroll
 					for (int kb = 0; kb < KB; ++kb) {
 						rank16_place<LD, SHARED>(raw[p][kb], kb, lane, w.dim);
-						if (LD == KMX_SOA) rank16_copy(w, raw[p][kb], first + p * TILE, kb, lane, exchange);
+						if (LD == KMX_SOA) rank16_copy<DIRECT>(w, raw[p][kb], first + p * TILE, kb, lane, exchange);
 						rank16_convert<SHARED>(b[p][kb], raw[p][kb], frame, scale, kb, lane, sums, exchange);
 					}
 					rank16_total<SHARED>(xx[p], xl[p], sums, lane);
@@ -812,20 +824,23 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 {
 	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4, tiles = w.kp / TILE, budget = lds_budget_of(exec, dev);
 	if (budget < rank16_least_bytes(KB, a.layout)) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
-	const uint64_t resident = (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false);
-	const bool stream_mode = resident + rank16_list_bytes(KB, a.layout, rank16_list_least(KB)) > budget;
+	auto resident = [&](bool direct, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, direct) + rank16_list_bytes(KB, a.layout, entries) <= budget; };
+	const bool direct = KB < 12 && a.layout == KMX_SOA && !resident(false, rank16_list_least(KB)) && resident(true, rank16_list_least(KB));
+	const bool stream_mode = !resident(direct, rank16_list_least(KB));
 	w.chunk_tiles = tiles;
 	w.list_entries = RANK16_LIST_MOST;
-	while (!stream_mode && resident + rank16_list_bytes(KB, a.layout, w.list_entries) > budget) --w.list_entries;
+	while (!stream_mode && !resident(direct, w.list_entries)) --w.list_entries;
 	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, a.layout, w.list_entries);
-	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode);
+	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode, direct);
 	if (stream_mode) {
 		w.chunk_tiles = 1;
 		while (rank16_slots(KB) == 2 && w.chunk_tiles < tiles && static_bytes + 2 * rank16_slot_bytes(KB, w.chunk_tiles + 1) <= budget) ++w.chunk_tiles;
 		lds_bytes = rank16_slots(KB) * rank16_slot_bytes(KB, w.chunk_tiles);
 	}
-	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true> : rank16_kernel<KB, KMX_AOS, false>)
-	                                                 : (stream_mode ? rank16_kernel<KB, KMX_SOA, true> : rank16_kernel<KB, KMX_SOA, false>);
+	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true, false> : rank16_kernel<KB, KMX_AOS, false, false>)
+	                                                 : (stream_mode ? rank16_kernel<KB, KMX_SOA, true, false> : rank16_kernel<KB, KMX_SOA, false, false>);
+	if constexpr (KB < 12)
+		if (direct) kernel = rank16_kernel<KB, KMX_SOA, false, true>;
 	const uint32_t waves = rank16_waves(KB, a.layout, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
 	const uint32_t grid = std::min((a.n + unit - 1) / unit, (waves == 4 ? 2 : 1) * dev.compute_units);
 	exec->block_count = grid;

@@ -157,3 +157,31 @@ def test_lists_that_share_lds_with_the_centroids(km, orc, gpu, dim, k, budget):
     finally:
         km.set_two_level_sweep(1)
     m.free(); a.free()
+
+
+@pytest.mark.parametrize("dim,k,more,bound", [(12, 3600, 4000, 1.3), (64, 1050, 1150, 1.19)])
+def test_soa_points_around_as_many_centroids_as_fit(km, gpu, dim, k, more, bound):
+    """The room in which SoA rows are exchanged does not push the centroids out of LDS: a tenth more of them takes 1.08 and 1.05 to 1.11 times
+    as long (1.53 and 1.27 where they streamed by instead)."""
+    n = 1 << 20
+    rng = np.random.default_rng(dim)
+    rows = rng.standard_normal((n, dim), dtype=np.float32)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, 1))
+    a = km.DeviceBuffer(4 * n)
+    start, stop = km.Event(), km.Event()
+    ms = []
+    for count in (k, more):
+        m = km.DeviceBuffer(4 * count * dim); m.write(flat(rows[:count], 1))
+        times = []
+        for call in range(12):
+            start.record()
+            km.assign(km.ASSIGN_BEST, d, 1, n, m, 1, count, a, dim, count, n)
+            stop.record()
+            km.sync()
+            if call > 2:
+                times.append(start.elapsed_ms(stop))
+        ms.append(float(np.median(times)))
+        m.free()
+    d.free(); a.free()
+    print("%d: %.3f ms, %d: %.3f ms" % (k, ms[0], more, ms[1]))
+    assert ms[1] <= bound * ms[0]
