@@ -173,15 +173,58 @@ def test_soa_points_around_as_many_centroids_as_fit(km, gpu, dim, k, more, bound
     for count in (k, more):
         m = km.DeviceBuffer(4 * count * dim); m.write(flat(rows[:count], 1))
         times = []
-        for call in range(12):
+        for call in range(30):
             start.record()
             km.assign(km.ASSIGN_BEST, d, 1, n, m, 1, count, a, dim, count, n)
             stop.record()
             km.sync()
-            if call > 2:
+            if call > 9:
                 times.append(start.elapsed_ms(stop))
         ms.append(float(np.median(times)))
         m.free()
     d.free(); a.free()
     print("%d: %.3f ms, %d: %.3f ms" % (k, ms[0], more, ms[1]))
     assert ms[1] <= bound * ms[0]
+
+
+def group_of(row):
+    """Of a centroid's row in its tile: the half-wave that holds its result, and the group of that lane's 16 results (rank16_impl.h)."""
+    result, half = row // 8 * 4 + row % 4, row // 4 % 2
+    return half * 6 + (5 if result == 15 else 4 if result % 4 == 3 else result // 4)
+
+
+@pytest.mark.parametrize("dim,k", [(5, 32), (16, 70), (16, 96), (20, 64), (32, 129)])
+def test_every_place_of_the_runner_up(km, orc, gpu, dim, k):
+    """Points on the line between every two centroids, next to the middle: the nearest two lie in one group of a tile's results, in two
+    groups, in the two half-waves and in two tiles, in every combination, with margins from nothing to what the sweep settles by itself."""
+    rng = np.random.default_rng(dim + k)
+    means = rng.normal(size=(k, dim)).astype(np.float32)
+    a, b = (i.ravel() for i in np.meshgrid(np.arange(k), np.arange(k), indexing="ij"))
+    a, b = a[a != b], b[a != b]
+    shift = np.array([0, 1e-7, 1e-6, 1e-5, 1e-4, 1e-3, 1e-2, 0.1])
+    at = (0.5 - shift)[:, None, None]  # (b, a as well as a, b: to either side of the middle)
+    rows = (means[a] * (1 - at) + means[b] * at).astype(np.float32).reshape(-1, dim)
+    n = len(rows)
+    if 16 <= dim <= 20:  # the tile's groups as winner and runner-up, each with each
+        far = ((rows[:, None, :].astype(np.float64) - means[None]) ** 2).sum(2)
+        first, second = np.argsort(far, axis=1)[:, :2].T
+        same = first // 32 == second // 32
+        met = {(group_of(i % 32), group_of(j % 32)) for i, j in zip(first[same], second[same])}
+        alone = {5, 11}  # (groups of one result)
+        assert met >= {(i, j) for i in range(12) for j in range(12) if i != j or i not in alone}
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0)
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 0))
+    out = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for layout in (0, 1):
+            d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, layout))
+            out.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, layout, km.layout_stride(layout, n, dim), m, 0, dim, out, dim, k, n)
+            km.sync()
+            got = out.read(np.uint32, n)
+            d.free()
+            assert np.array_equal(got, want), "layout %d: %d mismatches" % (layout, int((got != want).sum()))
+    finally:
+        km.set_two_level_sweep(1)
+    m.free(); out.free()
