@@ -424,9 +424,10 @@ constexpr uint32_t CELL_LIST = 64; /* points per wavefront that wait for the lis
 constexpr uint32_t CELL_STATIC = CELL_WAVES * (2 * CELL_LIST + 6) * 4 + 128; /* LDS of assign_cells_kernel beside the centroids: the infinite row, flag_list, wave_max */
 
 /*
- * A lane per point, the centroids in LDS. What bounds it: the gathers from LDS (N = 4M, d = 4, k = 4096, uniform points: a wavefront goes through
- * the longest list of its 64 points, 70 entries of 29 on average, and 16 bytes at 64 unrelated addresses take 11 cycles with their bank conflicts:
- * 179 000 of the 242 000 cycles of a compute unit), then the vector ALU. A comparison is 13 instructions and no branch: the sums are fused, the
+ * A lane per point, the centroids in LDS. What bounds it: the gathers from LDS and the vector ALU, which are both close to full (N = 4M, d = 4, k = 4096,
+ * uniform points: a wavefront goes through the longest list of its 64 points, 70 entries of 29 on average, and 16 bytes at 64 unrelated addresses take
+ * 11 cycles with their bank conflicts: 179 000 of the 242 000 cycles of a compute unit; 61 600 vector instructions on a SIMD, one in 3.9 cycles: minima and
+ * medians take 4.4 of them, fused sums two). A comparison is 13 instructions and no branch: the sums are fused, the
  * two smallest are kept (one v_med3), and the few points whose two smallest are not CELL_CLEAR of each other go through their list again in the
  * serial arithmetic (see CELL_TIES). Against that arithmetic for all, with its branches (17 instructions, and each row waited for by itself): 122 -> 112 us;
  * normal points, d = 4, k = 1000: 246 -> 216 us per call; d = 3, k = 6000: 119 -> 108 us. Sorting a wavefront's 256 points by the length of their
@@ -522,11 +523,13 @@ assign_cells_kernel(const CellAssignArgs w)
 
 	/*
 	 * Are the cells any good for these points? The sample (CHOICE_GROUPS wavefronts' worth, spread evenly over the points) says what
-	 * they would cost: a wavefront its longest list, N = 4M points 75 us and 1.1 (d = 3) to 1.45 us (d = 4) per entry; a point without a list
-	 * as much as k to 2 k entries in the exact pass. (A fifth less per entry since the fused comparisons: the line lies on the cells' safe side.) The packed sweep costs those points 110 us + 0.14 per centroid, its exact pass what the
-	 * data make of it, and the lists have been built by then. So it is left to that sweep (all work-groups come to the same answer) if
-	 *   - the lists are longer than k / 8 + 70 (d = 4; normal points, k = 1000: 168 entries, 340 against 322 us; exponential 474: 766
-	 *     against 404; points along a line 189: 450 against 2490, the sweep certifies few of those) or k / 8 + 320 (d = 2, 3: skewed data, which
+	 * they would cost: a wavefront its longest list, N = 4M points 60 us and 1 us per entry (d = 4; 75 and 1.45 in the serial arithmetic alone, which
+	 * rasters keep to: CELL_TIES); a point without a list as much as k to 2 k entries in the exact pass. The packed sweep costs those points 110 us + 0.14
+	 * per centroid, its exact pass what the data make of it, and the lists have been built by then. So it is left to that sweep (all work-groups
+	 * come to the same answer) if
+	 *   - the lists are longer than k / 8 + 70 (d = 4, k = 1000: normal points, 168 entries, 261 us through the cells, 340 after all by the sweep; exponential,
+	 *     474, 661 and 397: level at some 280, the line lies below since rasters cost the cells half as much again; points along a line 189, 450 and 2490 in the
+	 *     serial arithmetic, the sweep certifies few of those) or k / 8 + 320 (d = 2, 3: skewed data, which
 	 *     has such lists, costs the sweep more too: lognormal, k = 1000: 423 entries, 549 against 1044 us);
 	 *   - or the points without a list cost more than half of the first of these (normal, d = 4, k = 4096: 65 % of the points, 4329
 	 *     against 825 us; all outside the grid, d = 4, k = 1000: 1690 against 287).

@@ -17,7 +17,7 @@
  * gives way to the power they take (N = 1M, d = 256, k = 1024: 475 to 505 us, 1.09 to 1.16 PFLOP/s; d = 32, k = 1024, N = 2M: 151 to 169 us); the
  * exact pass by the latencies of one unit, list, rows, ranking and pairs in turn (1 to 4 % listed: 26 to 35 us; 9 % of N = 2M, d = 128: 110).
  * Whole calls, two bf16 levels -> this kernel at first -> now: N = 1M, d = 256, k = 1024 1713 -> 743 -> 520 us; N = 2M, d = 128, k = 1024, SoA
- * 1629 -> 940 -> 845; N = 2M, d = 32, k = 1024 332 -> 230 -> 185.
+ * 1629 -> 940 -> 845; N = 2M, d = 32, k = 1024 332 -> 230 -> 204 (Gaussian mixture, centroids after two rounds; 218 around its first points).
  */
 #include "rank16_exact_impl.h"
 

@@ -346,15 +346,16 @@ __device__ __forceinline__ float rank16_both(float v)
 }
 
 /*
- * A work-group around centroids in LDS: all of them (STREAM = false), or slots that go round (rank16_waves), all its wavefronts sweeping
- * together. A wavefront sweeps 64 points at a time. With resident centroids the wavefronts take items of 64 points from a counter in
- * LDS (a SIMD serves its older wavefront first: equal shares leave the younger ones sweeping alone at the end).
+ * A work-group around centroids in LDS: all of them (STREAM = false), or slots that go round (rank16_waves). A wavefront sweeps 64 points at
+ * a time. Rows of up to 64 dimensions around resident centroids: the wavefronts take items of 64 points from a counter in LDS (a SIMD
+ * serves its older wavefront first: equal shares leave the younger ones sweeping alone at the end). Otherwise a work-group takes units of
+ * 64 points per wavefront, its wavefronts side by side, every gridDim.x-th unit.
  *
  * What bounds the sweep of wide rows (N = 1M, d = 256, k = 1024: 505 us, 1.09 PFLOP/s): the power the matrix cores may take -- at 58 % of their
  * cycles the clock has come down to 1.73 GHz, without the points' fetches they reach 76 % at 1.51 -- and the fetches and conversions themselves.
  *
  * Tracking is the snapshot of assign_bf16_impl.h: the minimum of a lane's 16 results per tile, the two smallest minima, and the 16
- * results of the leading tile, from which the winner and the runner-up inside that tile come at the end.
+ * results of the leading tile, from which the winner and the runner-up inside that tile come at the end; rank16_grouped: six minima of those.
  * Rows of up to 64 dimensions and resident centroids: two accumulator sets, the tracking of one tile in pieces behind the matrix
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
