@@ -15,9 +15,9 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 /*
  * Rows of up to 32 dimensions around resident centroids: three wavefronts on a SIMD, of which the third also covers the ends of the others'
- * sweeps. That takes tracking in fewer registers (RANK16_GROUPS). us per assignment, two wavefronts with the snapshot -> three: N = 2M, d = 32,
- * k = 1024 201 -> 191; d = 16 155 -> 137; d = 10, k = 100 69 -> 63. The same tracking with two: 208, 152, 72 against 211, 159, 70. Wider rows would
- * spill (N = 1M, d = 64, k = 512: 103 -> 114), and so does the copying of SoA points (d = 24, k = 256: 68.6 -> 69.6).
+ * sweeps. That takes tracking in fewer registers (RANK16_GROUPS). us per assignment (N = 2M, Gaussian mixture, centroids after two rounds), two wavefronts with
+ * the snapshot -> three: d = 32, k = 1024 219 -> 204; d = 16 174 -> 150; d = 10, k = 100 74 -> 70. The same tracking with two: 220, 165, 78. Wider rows
+ * would spill (N = 1M, d = 64, k = 512: 103 -> 114), and so does the copying of SoA points (d = 24, k = 256: 68.6 -> 69.6).
  */
 constexpr bool rank16_grouped(uint32_t kb, int layout) { return kb == 1 || (kb == 2 && layout == KMX_AOS); }
 /*
