@@ -903,9 +903,8 @@ update_ranges_rows_f64_kernel(const double* __restrict__ data, size_t stride, co
  * listing pass takes each point's rank inside its cluster from the atomic that counts it), the sorted list is cut into
  * equal segments, one per group of G lanes (lane = dimension), and a group adds the rows of its segment in a register,
  * eight row loads in flight, and hands the sum over to the LDS copy -- with an atomic, as a cluster may span segments --
- * only where the cluster changes: one LDS atomic per run of a cluster instead of one per row (an LDS floating-point
- * atomic of a wavefront takes about 70 cycles; they bounded update_ranges_f64_kernel): N = 2M doubles, d = 32, k = 1024:
- * 0.147 -> 0.115 ms (4.4 TB/s with the clearing and the division).
+ * only where the cluster changes: one LDS atomic per run of a cluster instead of one per row: N = 2M doubles, d = 32, k = 1024:
+ * 0.147 -> 0.115 ms (4.4 TB/s with the clearing and the division). For what update_sums64.hip leaves: sums too large for its slices, few points.
  */
 constexpr uint32_t SORTED_PIECE_POINTS = 8192;             /* 13 bits of position in a list entry, the cluster above */
 constexpr uint32_t SORTED_RANGE_BYTES = 30 * 1024 - 64;    /* sums of a range: with the sorted list and the counts just below 64 KB */
@@ -1413,6 +1412,13 @@ static int update_f64_call(const char* who, bool divide, int variant,
 	if (variant == KMX_UPDATE_ATOMIC_SHM && small_update_fits<double>(dim, k, n, lds_budget_of(exec, *dev), *dev)) {
 		rc = launch_update_small<double>(data, layout, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n, divide, &exec->block_count, *dev);
 		return rc ? rc : profile_end(1);
+	}
+	if (variant == KMX_UPDATE_ATOMIC_SHM && layout == KMX_AOS && (!recording_graph() || workspace_exists())) {
+		Workspace* ws = nullptr;
+		if ((rc = workspace(&ws))) return rc;
+		Sums64Result result = SUMS64_OTHERS;
+		rc = launch_update_sums64<double>(data, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n, divide, exec, ws, *dev, &result);
+		if (rc || result == SUMS64_DONE) return rc ? rc : profile_end(1);
 	}
 #define KMX_F64_UPDATE(LD, LM) \
 	launch_update_f64_t<LD, LM>(variant, data, stride, assignment, means, stride_means, cluster_sizes, dim, k, n, exec, *dev, divide)

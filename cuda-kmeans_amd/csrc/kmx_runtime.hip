@@ -80,6 +80,8 @@ int device_info(const DeviceInfo** out)
 	return KMX_OK;
 }
 
+bool workspace_exists() { return g_ws.counters != nullptr; }
+
 int workspace(Workspace** ws)
 {
 	if (!g_ws.counters) {
@@ -263,7 +265,7 @@ static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_
 	if ((rc = profile_begin(0))) return rc;
 	if ((rc = launch_assign_small_sums(a, ws->partials, partial_counts, &exec->block_count, ws->counters, dev))) return rc;
 	if ((rc = profile_end(0))) return rc;
-	return launch_reduce_partials(u, ws->partials, partial_counts, exec->block_count);
+	return launch_reduce_partials<float>(ws->partials, partial_counts, exec->block_count, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.divide);
 }
 
 /*

@@ -8,25 +8,23 @@
  *   KMX_UPDATE_ATOMIC_SHM - the tuned variant (counterpart of updateAtomicShmKernel, reference
  *                           kernels.cu:817-858), three kernels chosen by shape. Measured on gfx950: an LDS
  *                           ds_add_f32 costs ~194 cycles per wavefront instruction whatever the address
- *                           pattern (lanes are serialised), ds_add_u32 4.4 cycles, a plain LDS
- *                           read-add-write 8.2 cycles. Floating-point LDS atomics are therefore avoided:
- *       update_private_kernel  small k*dim: every lane group (one lane per dimension) owns a PRIVATE copy
- *                              of the k x dim block in LDS and accumulates with plain read-add-write; the
- *                              copies are merged at the end, one global atomic per element and work-group.
- *                              (update_private_vec_kernel: the same with 16-byte row pieces per lane, for
- *                              millions of points: N = 16.7M, d = 16, k = 16 in 0.205 instead of 0.250 ms.)
- *       update_sorted_kernel   larger k: the work-group counting-sorts its chunk of points by cluster
+ *                           pattern (lanes are serialised), ds_add_u32 4.4 cycles, ds_add_f64 8.2 on rows of
+ *                           16 sums, a plain LDS read-add-write 8.2.
+ *       update_sums64_kernel   (update_sums64.hip) wherever the clusters' sums fit LDS as doubles, in slices of
+ *                              the coordinates if need be: every coordinate one ds_add_f64, the points read in
+ *                              the order they lie in.
+ *       update_sorted_kernel   larger k * dim: the work-group counting-sorts its chunk of points by cluster
  *                              with integer LDS atomics, then lane groups walk the sorted list and sum each
  *                              cluster's rows in registers (no atomics at all); per-chunk sums go to a partial
  *                              buffer with plain coalesced stores and reduce_partials_kernel folds them.
- *       update_lds_kernel      fallback for the shapes/layouts the two above do not take (SoA points):
- *                              LDS-privatised ds_add_f32.
+ *       update_lds_kernel      fallback for the shapes/layouts the two above do not take (SoA points), and while
+ *                              a graph is recorded and nothing can be allocated: LDS-privatised ds_add_f32.
  *     Points are read exactly once in all three.
  *   reduce_copies_kernel / divide_means_kernel
  *                         - counterparts of reducePrivCopiesKernel / divideMeansKernel
  *                           (reference kernels.cu:115-135,149-163); empty clusters keep their zero.
  *
- * Sums are fp32 and their order differs from the serial order, exactly as in the reference's GPU path
+ * Partial sums are fp32 and their order differs from the serial order, exactly as in the reference's GPU path
  * (atomics); counts are integers and exact.
  */
 #include "kmx_internal.h"
@@ -325,151 +323,7 @@ update_lds_kernel(const float* __restrict__ data, size_t stride, const uint32_t*
 	}
 }
 
-/*
- * Small k*dim. Lane group = GW lanes (GW = power of two >= dim), lane gl < dim owns dimension gl. Every group
- * has a private block [k*dim sums | k counts] in LDS; consecutive groups take consecutive points, so a
- * wavefront reads 64/GW consecutive rows per step. LDS operations of one wavefront execute in order, so a
- * plain read-add-write is correct even when consecutive points fall into the same cluster. copy_stride is
- * chosen so that the groups of one wavefront start GW banks apart: equal targets (the hot-cluster case) are
- * conflict-free.
- */
-template <int LM>
-__global__ void __launch_bounds__(256)
-update_private_kernel(const float* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment,
-                      float* __restrict__ means, size_t stride_means, uint32_t* __restrict__ sizes,
-                      uint32_t dim, uint32_t k, uint32_t n, uint32_t gw, uint32_t copy_stride, uint32_t chunk_points)
-{
-	extern __shared__ float lds[];
-	const uint32_t groups = blockDim.x / gw;
-	const uint32_t group = threadIdx.x / gw;
-	const uint32_t gl = threadIdx.x - group * gw;
-	for (uint32_t i = threadIdx.x; i < groups * copy_stride; i += blockDim.x) lds[i] = 0.0f;
-	__syncthreads();
-
-	float* acc = lds + (size_t)group * copy_stride;
-	uint32_t* cnt = (uint32_t*)(acc + (size_t)k * dim);
-	const uint32_t p_begin = (uint32_t)min((uint64_t)blockIdx.x * chunk_points, (uint64_t)n);
-	const uint32_t p_end = (uint32_t)min((uint64_t)p_begin + chunk_points, (uint64_t)n);
-	const bool lane_on = gl < dim;
-	const float* src = data + (lane_on ? gl : 0);
-	uint32_t p = p_begin + group;
-	for (; p + (UPDATE_UNROLL - 1) * groups < p_end; p += UPDATE_UNROLL * groups) {
-		float v[UPDATE_UNROLL];
-		uint32_t t[UPDATE_UNROLL];
-#pragma unroll
-		for (int u = 0; u < UPDATE_UNROLL; ++u) {
-			v[u] = src[(size_t)(p + u * groups) * stride];
-			t[u] = assignment[p + u * groups];
-		}
-#pragma unroll
-		for (int u = 0; u < UPDATE_UNROLL; ++u) {
-			if (lane_on) acc[t[u] * dim + gl] += v[u];
-			if (gl == 0) cnt[t[u]] += 1u;
-		}
-	}
-	for (; p < p_end; p += groups) {
-		float v = src[(size_t)p * stride];
-		uint32_t t = assignment[p];
-		if (lane_on) acc[t * dim + gl] += v;
-		if (gl == 0) cnt[t] += 1u;
-	}
-	__syncthreads();
-
-	for (uint32_t e = threadIdx.x; e < k * dim; e += blockDim.x) {
-		float s = 0.0f;
-		for (uint32_t g = 0; g < groups; ++g) s += lds[(size_t)g * copy_stride + e];
-		const uint32_t c = e / dim, d = e - c * dim;
-		if (s != 0.0f) atomic_add_f32(&means[elem<LM>(stride_means, c, d)], s);
-	}
-	for (uint32_t c = threadIdx.x; c < k; c += blockDim.x) {
-		uint32_t s = 0;
-		for (uint32_t g = 0; g < groups; ++g) s += ((const uint32_t*)lds)[(size_t)g * copy_stride + (size_t)k * dim + c];
-		if (s) atomicAdd(&sizes[c], s);
-	}
-}
-
-/*
- * The same with 16-byte pieces of a row per lane: a group is GW4 = dim / 4 lanes (rounded
- * up to a power of two), so a wavefront reads 64 / GW4 consecutive rows with one instruction -- a quarter of the load
- * instructions, and of the loads of the assignment, that one lane per dimension issues. Every group still needs a copy of its
- * own (lanes of one instruction that met in one copy would lose updates), so a work-group of 256 lanes holds 256 / GW4 copies:
- * more LDS per work-group, fewer work-groups per compute unit, the same bytes in flight.
- */
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-constexpr int UPDATE_UNROLL_VEC = 8; /* row pieces in flight per lane (16 measured the same) */
-
-/*
- * FULL: dim a multiple of 4 and aligned rows. Otherwise the last piece of a row is read so that it ends with the row (16-byte
- * loads need 4-byte alignment only) and shifted into place; the sums in LDS have rows of whole pieces, whose surplus is never read.
- */
-template <int LM, bool FULL>
-__global__ void __launch_bounds__(256)
-update_private_vec_kernel(const float* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment,
-                          float* __restrict__ means, size_t stride_means, uint32_t* __restrict__ sizes,
-                          uint32_t dim, uint32_t k, uint32_t n, uint32_t gw, uint32_t copy_stride, uint32_t chunk_points)
-{
-	extern __shared__ __attribute__((aligned(16))) float lds[];
-	const uint32_t dim4 = (dim + 3) & ~3u;
-	const uint32_t groups = blockDim.x / gw;
-	const uint32_t group = threadIdx.x / gw;
-	const uint32_t gl = threadIdx.x - group * gw;
-	for (uint32_t i = threadIdx.x; i < groups * copy_stride; i += blockDim.x) lds[i] = 0.0f;
-	__syncthreads();
-
-	float* acc = lds + (size_t)group * copy_stride;
-	uint32_t* cnt = (uint32_t*)(acc + (size_t)k * dim4);
-	const uint32_t p_begin = (uint32_t)min((uint64_t)blockIdx.x * chunk_points, (uint64_t)n);
-	const uint32_t p_end = (uint32_t)min((uint64_t)p_begin + chunk_points, (uint64_t)n);
-	const bool lane_on = gl * 4 < dim;
-	const uint32_t d0 = lane_on ? gl * 4 : 0;
-	const uint32_t shift = FULL ? 0u : d0 + 4 > dim ? d0 + 4 - dim : 0u; /* places the piece was read too early */
-	const float* src = data + d0 - shift;
-	auto load = [&](uint32_t p) -> f32x4 {
-		if constexpr (FULL) return *(const f32x4*)(src + (size_t)p * stride);
-		else return *(const f32x4_any*)(src + (size_t)p * stride);
-	};
-	auto add_row = [&](uint32_t target, const f32x4& w) {
-		if (lane_on) {
-			f32x4 v = w;
-			if constexpr (!FULL) {
-				v.x = shift == 0 ? w.x : shift == 1 ? w.y : shift == 2 ? w.z : w.w;
-				v.y = shift == 0 ? w.y : shift == 1 ? w.z : w.w;
-				v.z = shift == 0 ? w.z : w.w;
-			}
-			f32x4* at = (f32x4*)(acc + target * dim4 + gl * 4);
-			f32x4 a = *at;
-			a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
-			*at = a;
-		}
-		if (gl == 0) cnt[target] += 1u;
-	};
-	uint32_t p = p_begin + group;
-	for (; p + (UPDATE_UNROLL_VEC - 1) * groups < p_end; p += UPDATE_UNROLL_VEC * groups) {
-		f32x4 v[UPDATE_UNROLL_VEC];
-		uint32_t t[UPDATE_UNROLL_VEC];
-#pragma unroll
-		for (int u = 0; u < UPDATE_UNROLL_VEC; ++u) {
-			v[u] = load(p + u * groups);
-			t[u] = assignment[p + u * groups];
-		}
-#pragma unroll
-		for (int u = 0; u < UPDATE_UNROLL_VEC; ++u) add_row(t[u], v[u]);
-	}
-	for (; p < p_end; p += groups) add_row(assignment[p], load(p));
-	__syncthreads();
-
-	for (uint32_t e = threadIdx.x; e < k * dim; e += blockDim.x) {
-		const uint32_t c = e / dim, d = e - c * dim;
-		float s = 0.0f;
-		for (uint32_t g = 0; g < groups; ++g) s += lds[(size_t)g * copy_stride + c * dim4 + d];
-		if (s != 0.0f) atomic_add_f32(&means[elem<LM>(stride_means, c, d)], s);
-	}
-	for (uint32_t c = threadIdx.x; c < k; c += blockDim.x) {
-		uint32_t s = 0;
-		for (uint32_t g = 0; g < groups; ++g) s += ((const uint32_t*)lds)[(size_t)g * copy_stride + (size_t)k * dim4 + c];
-		if (s) atomicAdd(&sizes[c], s);
-	}
-}
 
 /*
  * Larger k. Grid = (point chunks, 32-wide dimension slices); work-group = 1024 lanes.
@@ -755,13 +609,13 @@ update_sorted_kernel(const float* __restrict__ data, size_t stride, const uint32
  */
 constexpr uint32_t REDUCE_THREADS = 1024;
 
-template <int LM, uint32_t COLS>
+template <typename F, int LM, uint32_t COLS>
 __global__ void __launch_bounds__(REDUCE_THREADS)
-reduce_partials_kernel(const float* __restrict__ partial, const uint32_t* __restrict__ partial_counts, float* __restrict__ means, size_t stride_means,
+reduce_partials_kernel(const F* __restrict__ partial, const uint32_t* __restrict__ partial_counts, F* __restrict__ means, size_t stride_means,
                        uint32_t* __restrict__ sizes, uint32_t dim, uint32_t k, uint32_t chunks, uint32_t divide)
 {
 	constexpr uint32_t MAX_SHARES = REDUCE_THREADS / COLS;
-	__shared__ float part[MAX_SHARES][COLS];
+	__shared__ F part[MAX_SHARES][COLS];
 	__shared__ uint32_t part_count[MAX_SHARES][COLS];
 	const uint32_t col = threadIdx.x % COLS, share = threadIdx.x / COLS;
 	const uint32_t shares = blockDim.x / COLS; /* the launcher gives every share at least 8 chunks */
@@ -779,20 +633,20 @@ reduce_partials_kernel(const float* __restrict__ partial, const uint32_t* __rest
 	uint32_t cv[16];
 #pragma unroll
 	for (int u = 0; u < 16; ++u) cv[u] = (counting && c0 + u < c1) ? pc[(size_t)(c0 + u) * k] : 0u;
-	float s = 0.0f;
+	F s = (F)0;
 	if (e < kd) {
 		uint32_t c = c0;
 		for (; c + 16 <= c1; c += 16) {
-			float v[16];
+			F v[16];
 #pragma unroll
 			for (int u = 0; u < 16; ++u) v[u] = partial[(size_t)(c + u) * kd + e];
 #pragma unroll
 			for (int u = 0; u < 16; ++u) s += v[u];
 		}
 		if (c < c1) {
-			float v[16];
+			F v[16];
 #pragma unroll
-			for (int u = 0; u < 16; ++u) v[u] = c + u < c1 ? partial[(size_t)(c + u) * kd + e] : 0.0f;
+			for (int u = 0; u < 16; ++u) v[u] = c + u < c1 ? partial[(size_t)(c + u) * kd + e] : (F)0;
 #pragma unroll
 			for (int u = 0; u < 16; ++u) s += v[u];
 		}
@@ -811,13 +665,13 @@ reduce_partials_kernel(const float* __restrict__ partial, const uint32_t* __rest
 	part[share][col] = s;
 	__syncthreads();
 	if (share == 0 && e < kd) {
-		s = 0.0f;
+		s = (F)0;
 		for (uint32_t i = 0; i < shares; ++i) s += part[i][col];
 		const uint32_t cl = e / dim, d = e - cl * dim;
 		uint32_t count = 0;
 		for (uint32_t i = 0; i < shares; ++i) count += part_count[i][cl - cl_lo];
 		if (d == 0) sizes[cl] = count; /* the work-group that holds the cluster's first element publishes its size */
-		means[elem<LM>(stride_means, cl, d)] = !divide ? s : (count ? s / (float)count : 0.0f);
+		means[elem<LM>(stride_means, cl, d)] = !divide ? s : (count ? s / (F)count : (F)0);
 	}
 }
 
@@ -884,18 +738,21 @@ static uint32_t pow2_at_least(uint32_t v)
 	return p;
 }
 
-int launch_reduce_partials(const UpdateArgs& u, const float* partial, const uint32_t* partial_counts, uint32_t chunks)
+template <typename F>
+int launch_reduce_partials(const F* partial, const uint32_t* partial_counts, uint32_t chunks, F* means, int layout_means, size_t stride_means, uint32_t* sizes, uint32_t dim, uint32_t k, bool divide)
 {
-	const uint32_t total = u.k * u.dim;
+	const uint32_t total = k * dim;
 	const uint32_t cols = chunks > 256 && total <= 4096 ? 16 : 64;
 	const uint32_t shares = std::max<uint32_t>(64 / cols, std::min<uint32_t>(REDUCE_THREADS / cols, chunks / 8));
-	auto kernel = u.layout_means == KMX_AOS ? (cols == 16 ? reduce_partials_kernel<KMX_AOS, 16> : reduce_partials_kernel<KMX_AOS, 64>)
-	                                        : (cols == 16 ? reduce_partials_kernel<KMX_SOA, 16> : reduce_partials_kernel<KMX_SOA, 64>);
+	auto kernel = layout_means == KMX_AOS ? (cols == 16 ? reduce_partials_kernel<F, KMX_AOS, 16> : reduce_partials_kernel<F, KMX_AOS, 64>)
+	                                      : (cols == 16 ? reduce_partials_kernel<F, KMX_SOA, 16> : reduce_partials_kernel<F, KMX_SOA, 64>);
 	KMX_LAUNCH_KERNEL(kernel, dim3((total + cols - 1) / cols), dim3(cols * shares), 0, stream(),
-	                   partial, partial_counts, u.means, u.stride_means, u.cluster_sizes, u.dim, u.k, chunks, u.divide ? 1u : 0u);
+	                   partial, partial_counts, means, stride_means, sizes, dim, k, chunks, divide ? 1u : 0u);
 	KMX_LAUNCH_CHECK("reduce_partials_kernel");
 	return KMX_OK;
 }
+template int launch_reduce_partials<float>(const float*, const uint32_t*, uint32_t, float*, int, size_t, uint32_t*, uint32_t, uint32_t, bool);
+template int launch_reduce_partials<double>(const double*, const uint32_t*, uint32_t, double*, int, size_t, uint32_t*, uint32_t, uint32_t, bool);
 
 template <int ITEMS, int LM>
 static int launch_sorted(const UpdateArgs& u, Workspace* ws, uint32_t chunks, uint32_t slices, uint32_t chunk_points, uint32_t gw, uint32_t vec, uint32_t lds_bytes, bool whole_rows)
@@ -928,22 +785,9 @@ static int launch_sorted(const UpdateArgs& u, Workspace* ws, uint32_t chunks, ui
 	KMX_LAUNCH_KERNEL(kernel, dim3(chunks, slices), dim3(1024), lds_bytes, stream(),
 	                   u.data, u.stride, u.assignment, ws->partials, partial_counts, u.dim, u.k, u.n, chunk_points);
 	KMX_LAUNCH_CHECK("update_sorted_kernel");
-	return launch_reduce_partials(u, ws->partials, partial_counts, chunks);
+	return launch_reduce_partials<float>(ws->partials, partial_counts, chunks, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.divide);
 }
 
-/*
- * Private copies or sorted chunks (us per call, private / sorted). Clearing and folding the copies costs a work-group the same
- * whatever its points, so 16-byte pieces pay from here on: d = 16, k = 16: 1 M 29 / 32, 2 M 37 / 50, 4 M 53 / 87; d = 13,
- * k = 20: 1 M 29 / 24, 2 M 42 / 47, 4 M 66 / 94; d = 32, k = 16: 1 M 37 / 34, 2 M 52 / 54; d = 60, k = 3: 1 M 67 / 62, 2 M 100 / 133.
- */
-constexpr uint32_t PRIVATE_VEC_MIN_POINTS = 3u << 19;
-/* Single words per lane are for short rows: d = 4, k = 8 12 us (70 k points) to 62 (12 M) against 18 to 228; d = 8, k = 64:
- * 70 k 14 / 12, 500 k 26 / 15, 2 M 43 / 38, 4 M 66 / 72. From nine dimensions on the sorted chunks are ahead everywhere the
- * pieces above do not fit (d = 32, k = 64: 70 k 22 / 12, 4 M 238 / 99; d = 64, k = 32: 200 k 57 / 19, 4 M 287 / 199). */
-static bool private_words_pay(uint32_t dim, uint32_t k, uint32_t n)
-{
-	return dim <= 4 || (dim <= 8 && (k <= 32 || n >= (3u << 20)));
-}
 /* Picks and launches the kernel of KMX_UPDATE_ATOMIC_SHM. *state: 0 = no LDS variant fits the shape, 1 = sums and
  * counts accumulated (divide still to do), 2 = centroids finished (the sorted path divides while it folds the partials). */
 template <int LD, int LM>
@@ -952,60 +796,14 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 	*state = 1;
 	const uint32_t budget = exec->shared_mem_bytes ? std::min(exec->shared_mem_bytes, dev.lds_bytes) : dev.lds_bytes;
 
-	if (LD == KMX_AOS && u.dim >= 8 && u.dim <= 64 && u.n >= PRIVATE_VEC_MIN_POINTS) {
-		/* private copies for groups of dim / 4 lanes with 16-byte row pieces */
-		const uint32_t gw = pow2_at_least((u.dim + 3) / 4);
-		const bool full = u.dim % 4 == 0 && u.stride % 4 == 0 && ((uintptr_t)u.data & 15) == 0;
-		const uint32_t groups = 256 / gw;
-		const uint64_t copy_words = (uint64_t)u.k * ((u.dim + 3) / 4 * 4 + 1);
-		const uint64_t copy_stride = (copy_words + 31) / 32 * 32 + 4 * gw; /* groups of one 128-byte LDS cycle start 4 gw banks apart */
-		const uint64_t lds_bytes = groups * copy_stride * 4;
-		if (lds_bytes <= std::min<uint32_t>(budget, 96 * 1024)) {
-			const uint32_t wg_per_cu = std::max<uint32_t>(1, std::min<uint32_t>(8, (uint32_t)(dev.lds_bytes / lds_bytes)));
-			uint32_t chunks = dev.compute_units * wg_per_cu;
-			const uint32_t quantum = groups * UPDATE_UNROLL_VEC;
-			uint32_t chunk_points = (u.n + chunks - 1) / chunks;
-			chunk_points = (chunk_points + quantum - 1) / quantum * quantum;
-			chunks = (u.n + chunk_points - 1) / chunk_points;
-			exec->block_count = chunks;
-			int rc = clear_outputs(u);
-			if (rc) return rc;
-			auto kernel = full ? update_private_vec_kernel<LM, true> : update_private_vec_kernel<LM, false>;
-			KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-			KMX_LAUNCH_KERNEL(kernel, dim3(chunks), dim3(256), (uint32_t)lds_bytes, stream(),
-			                   u.data, u.stride, u.assignment, u.means, u.stride_means, u.cluster_sizes,
-			                   u.dim, u.k, u.n, gw, (uint32_t)copy_stride, chunk_points);
-			KMX_LAUNCH_CHECK("update_private_vec_kernel");
-			return KMX_OK;
-		}
+	Sums64Result sums64 = SUMS64_OTHERS;
+	if (LD == KMX_AOS) {
+		const int rc = launch_update_sums64<float>(u.data, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.n, u.divide, exec, ws, dev, &sums64);
+		if (sums64 == SUMS64_DONE) *state = 2;
+		if (rc || sums64 == SUMS64_DONE) return rc;
 	}
 
-	if (LD == KMX_AOS && private_words_pay(u.dim, u.k, u.n)) {
-		/* private copies: 256 / gw groups, each k*dim sums + k counts, padded so that groups start gw banks apart */
-		const uint32_t gw = pow2_at_least(u.dim);
-		const uint32_t groups = 256 / gw;
-		const uint64_t copy_words = (uint64_t)u.k * (u.dim + 1);
-		const uint64_t copy_stride = (copy_words + 63) / 64 * 64 + gw;
-		const uint64_t lds_bytes = groups * copy_stride * 4;
-		if (lds_bytes <= std::min<uint32_t>(budget, 96 * 1024)) {
-			const uint32_t wg_per_cu = std::max<uint32_t>(1, std::min<uint32_t>(8, (uint32_t)(dev.lds_bytes / lds_bytes)));
-			uint32_t chunks = dev.compute_units * wg_per_cu;
-			const uint32_t quantum = groups * UPDATE_UNROLL;
-			uint32_t chunk_points = (u.n + chunks - 1) / chunks;
-			chunk_points = (chunk_points + quantum - 1) / quantum * quantum;
-			chunks = (u.n + chunk_points - 1) / chunk_points;
-			exec->block_count = chunks;
-			int rc = clear_outputs(u);
-			if (rc) return rc;
-			KMX_LAUNCH_KERNEL((update_private_kernel<LM>), dim3(chunks), dim3(256), (uint32_t)lds_bytes, stream(),
-			                   u.data, u.stride, u.assignment, u.means, u.stride_means, u.cluster_sizes,
-			                   u.dim, u.k, u.n, gw, (uint32_t)copy_stride, chunk_points);
-			KMX_LAUNCH_CHECK("update_private_kernel");
-			return KMX_OK;
-		}
-	}
-
-	if (LD == KMX_AOS && u.k < (1u << (32 - SORT_SHIFT)) && (uint64_t)(u.k + 36) * 4 + 1024 * 4 + 1024 * 5 * 4 <= budget) {
+	if (LD == KMX_AOS && sums64 != SUMS64_NO_ROOM && u.k < (1u << (32 - SORT_SHIFT)) && (uint64_t)(u.k + 36) * 4 + 1024 * 4 + 1024 * 5 * 4 <= budget) {
 		const uint32_t slices = (u.dim + 31) / 32;
 		/* rows of 33 to 256 dimensions: the work-groups of a chunk take ranges of clusters and read whole rows (measured at
 		 * N = 1M, d = 256, k = 1024: 0.29 ms in slices of 32 dimensions) */

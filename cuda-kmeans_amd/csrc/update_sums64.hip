@@ -1,0 +1,217 @@
+/*
+ * The update for clusters whose sums fit LDS as doubles: one pass over the rows in the order they lie in, every coordinate one ds_add_f64.
+ *
+ * ds_add_f64 takes 8 cycles for a wavefront on rows of 16 sums (two sums side by side in every bank of 8 bytes), as a plain read, addition and write would;
+ * ds_add_f32 takes 194 whatever the addresses. So the sums are doubles, and nothing has to be sorted, listed or owned: the sorted chunks (update.hip) read rows
+ * in the order of their clusters after a sort during which the memory idles, this kernel as a copy would. us per call, sorted chunks -> this:
+ *   N = 8,388,608, d = 32, k = 1024 239 -> 208; N = 2M, d = 32, k = 1024 63 -> 55; N = 4M, d = 4, k = 4096 59 -> 26; N = 4M, d = 8, k = 1024 77 -> 31;
+ *   N = 4M, d = 16, k = 512 85 -> 50; N = 1M, d = 64, k = 1024 65 -> 57; N = 1M, d = 128, k = 1024 135 -> 126.
+ */
+#include "kmx_internal.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace kmx {
+
+constexpr uint32_t SUMS64_THREADS = 1024, SUMS64_WAVES = SUMS64_THREADS / WAVE;
+constexpr uint32_t SUMS64_LANES = 64;      /* most coordinates of a slice: a lane each */
+constexpr uint32_t SUMS64_XCDS = 8;
+
+template <int LW> struct Sums64 {
+	static constexpr uint32_t ROWS = WAVE / LW;                   /* rows of a request */
+	static constexpr uint32_t SPAN = LW >= 16 ? 16 : LW >= 4 ? 4 : LW; /* consecutive rows of a group of LW lanes, whose memberships lie in the lanes of one register */
+	static constexpr uint32_t REQUESTS = 16;                      /* of a step */
+	static constexpr uint32_t REGS = REQUESTS / SPAN;             /* registers of memberships */
+	static constexpr uint32_t POINTS = REQUESTS * ROWS;           /* of a step */
+	static constexpr int STEPS = LW >= 16 ? 3 : 2;                /* under way */
+};
+
+/* the value that lane U of this lane's 16 (SPAN = 16), 4 or 2 lanes has */
+template <int SPAN, int U> __device__ __forceinline__ uint32_t sums64_member(uint32_t v)
+{
+	if constexpr (SPAN == 1) return v;
+	else return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, SPAN == 16 ? 0x150 + U /* row_newbcast */ : SPAN == 4 ? U * 0x55 : U * 0x05 + (U + 2) * 0x50 /* quad_perm */, 0xF, 0xF, true);
+}
+
+template <int LW, bool FULL, typename F>
+__global__ void __launch_bounds__(SUMS64_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+update_sums64_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment, F* __restrict__ partial, uint32_t* __restrict__ partial_counts,
+                     uint32_t dim, uint32_t k, uint32_t n, uint32_t chunk_points, uint32_t chunks, uint32_t slices, uint32_t width, uint32_t copies)
+{
+	typedef Sums64<LW> S;
+	/* copies of k + 1 rows of `width` sums (the last row takes what is no cluster's), then copies of k + 1 counts */
+	extern __shared__ __attribute__((aligned(16))) double sums64[];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	/* the slices of a chunk share lines of memory: they lie on one XCD, whose second level of cache sees them side by side */
+	const uint32_t at = blockIdx.x / SUMS64_XCDS, slice = at % slices, chunk = blockIdx.x % SUMS64_XCDS + SUMS64_XCDS * (at / slices);
+	if (chunk >= chunks) return;
+	const uint32_t copy = (k + 1) * width;
+	uint32_t* counts = (uint32_t*)(sums64 + copies * copy);
+	const uint32_t d0 = slice * width, mine = min(width, dim - d0);
+	const uint32_t p_begin = (uint32_t)min((uint64_t)chunk * chunk_points, (uint64_t)n), count = min(chunk_points, n - p_begin);
+	for (uint32_t i = tid; i < copies * copy; i += SUMS64_THREADS) sums64[i] = 0.0;
+	for (uint32_t i = tid; i < copies * (k + 1); i += SUMS64_THREADS) counts[i] = 0u;
+	__syncthreads();
+
+	const uint32_t gl = lane % LW, group = lane / LW;
+	const bool lane_on = gl < mine;
+	const F* src = data + (size_t)p_begin * stride + d0 + min(gl, mine - 1);
+	const uint32_t* members = assignment + p_begin;
+	const uint32_t steps = (count + S::POINTS - 1) / S::POINTS;
+	const bool counting = slice == 0 && gl < S::SPAN;
+	const uint32_t which = group % copies;
+	const uint32_t sums_at = (which * copy + gl) * 8, nowhere = (which * copy + k * width + gl % width) * 8;
+	uint32_t* counts_at = counts + which * (k + 1);
+	struct Step { F x[S::REQUESTS]; uint32_t member[S::REGS]; };
+	auto request = [&](Step& s, uint32_t step) {
+		const uint32_t first = step * S::POINTS;
+#pragma unroll
+		for (uint32_t r = 0; r < S::REGS; ++r) {
+			const uint32_t p = first + (r * S::ROWS + group) * S::SPAN + gl % S::SPAN;
+			s.member[r] = p < count ? members[p] : k;
+		}
+#pragma unroll
+		for (uint32_t u = 0; u < S::REQUESTS; ++u) {
+			const uint32_t p = first + (u / S::SPAN * S::ROWS + group) * S::SPAN + u % S::SPAN;
+			s.x[u] = src[(size_t)min(p, count - 1) * stride];
+		}
+	};
+	auto add = [&](Step& s) {
+#pragma unroll
+		for (uint32_t r = 0; r < S::REGS; ++r) {
+			const uint32_t c = min(s.member[r], k);
+			if (counting) atomicAdd(&counts_at[c], 1u);
+			s.member[r] = c * (width * 8);
+		}
+		auto put = [&](auto tag) {
+			constexpr uint32_t U = decltype(tag)::value;
+			const uint32_t row = sums64_member<S::SPAN, U % S::SPAN>(s.member[U / S::SPAN]);
+			unsafeAtomicAdd((double*)((char*)sums64 + (FULL || lane_on ? row + sums_at : nowhere)), (double)s.x[U]);
+		};
+#define KMX_PUT4(U) put(std::integral_constant<uint32_t, U>{}); put(std::integral_constant<uint32_t, U + 1>{}); put(std::integral_constant<uint32_t, U + 2>{}); put(std::integral_constant<uint32_t, U + 3>{});
+		KMX_PUT4(0) KMX_PUT4(4) KMX_PUT4(8) KMX_PUT4(12)
+#undef KMX_PUT4
+	};
+	constexpr int STEPS = S::STEPS;
+	Step ring[STEPS];
+#pragma unroll
+	for (int i = 0; i < STEPS - 1; ++i)
+		if (wave + SUMS64_WAVES * i < steps) request(ring[i], wave + SUMS64_WAVES * i);
+	for (uint32_t step = wave; step < steps; step += SUMS64_WAVES * STEPS) {
+#pragma unroll
+		for (int i = 0; i < STEPS; ++i) {
+			const uint32_t now = step + SUMS64_WAVES * i, then = now + SUMS64_WAVES * (STEPS - 1);
+			if (then < steps) request(ring[(i + STEPS - 1) % STEPS], then);
+			if (now < steps) add(ring[i]);
+		}
+	}
+	__syncthreads();
+	F* out = partial + (size_t)chunk * k * dim + d0 + gl;
+	for (uint32_t c = tid / LW; c < k; c += SUMS64_THREADS / LW)
+		if (lane_on) {
+			double sum = sums64[c * width + gl];
+			for (uint32_t i = 1; i < copies; ++i) sum += sums64[i * copy + c * width + gl];
+			out[(size_t)c * dim] = (F)sum;
+		}
+	if (slice == 0)
+		for (uint32_t c = tid; c < k; c += SUMS64_THREADS) {
+			uint32_t size = counts[c];
+			for (uint32_t i = 1; i < copies; ++i) size += counts[i * (k + 1) + c];
+			partial_counts[(size_t)chunk * k + c] = size;
+		}
+}
+
+/*
+ * A work-group per compute unit: slices of the coordinates x chunks of the points, as few slices as let their sums fit LDS, ten at most (d = 160, k = 600: ten
+ * 139 us, five 129, sorted chunks 158; d = 256, k = 1024: sixteen 277, sorted chunks 242; N = 1M here and below). Slices are equal, or, in floats, of whole 64
+ * bytes up to 32 coordinates (sorted chunks / equal / these: d = 33, k = 1000 54 / 41 / 35; d = 80, k = 1000 86 / 101 / 77; wider ones d = 100, k = 100,
+ * N = 500000: 50 + 50 38, 64 + 36 46). Rows of up to 48 floats go in slices of 16, doubles in slices of 32 or two, even where the whole row fits (d = 40,
+ * k = 300: 34, whole 37; doubles, N = 2M, d = 32, k = 500: 103, 113): the sums to write are fewer. Doubles whose sums do not fit as a whole: 16 at a time (N = 500000,
+ * d = 128, k = 1024: 123, slices of 19 142, sums of ranges of clusters 204), equal where the last would be narrow (N = 1M, d = 33, k = 1000: 73,
+ * 16 + 16 + 1 86, ranges 77), eight at a time where rows are odd multiples of 32 bytes and short (N = 1M, d = 24, k = 1200: 43, 12 + 12 47, ranges 53). Rows of more than 192 floats in slices of 32 and less lose
+ * (N = 500000, d = 256, k = 600: 123 against 121).
+ * As many chunks per XCD as it has compute units for: one more somewhere comes alone at the end (d = 48, k = 1024: 85 chunks of three slices 62, 80 42).
+ * A chunk has as many points as there are clusters, 512 at least: its sums are written and read once more (N = 200000, d = 4, k = 4000: 256 chunks 17 us, 50
+ * 14, sorted chunks 31; N = 50000, d = 32, k = 1000: 17, 14, 16); where that leaves compute units over and a slice is wide, more slices (N = 100000, d = 32,
+ * k = 500: one slice 16, two 13). Sums of doubles are twice as dear: four times as many points, and few points are left to the kernels that add to the means
+ * where they lie (N = 400000, d = 32, k = 1000 33.2, those 34.2; N = 100000, k = 500 17.4, 17.1; N = 200000, d = 4, k = 4000 19.0, 16.2).
+ * Few clusters: the rows of a request mostly meet at the same sums, which costs an LDS cycle each; copies of them, as many as rows (N = 16M, d = 2,
+ * k = 2: 90 us without, 34 with).
+ */
+struct Sums64Plan { uint32_t width, slices, copies, chunks, chunk_points, lds_bytes; };
+constexpr uint32_t SUMS64_SLICES = 10;
+
+static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint32_t budget, uint32_t compute_units, Sums64Plan* plan)
+{
+	auto bytes = [&](uint32_t width) -> uint64_t { return ((uint64_t)k + 1) * (8 * width + 4); };
+	auto slices_of = [&](uint32_t width) -> uint32_t { return (dim - 1) / width + 1; };
+	auto chunks_of = [&](uint32_t width) -> uint32_t { return std::max<uint32_t>(1, compute_units / SUMS64_XCDS / slices_of(width)) * SUMS64_XCDS; };
+	if (dim > SUMS64_SLICES * SUMS64_LANES || (doubles && n / 200 < k && (uint64_t)k * dim > 8192)) return false;
+	const uint64_t least_points = std::max<uint64_t>(512, (uint64_t)k * (doubles ? 4 : 1));
+	/* doubles whose sums do not fit as a whole */
+	const bool parts = doubles && bytes(dim) > budget, eights = parts && dim <= 56 && dim % 4 == 0 && dim % 16 != 0;
+	if (parts && slices_of(16) == 7 && dim % 16 != 0 && dim % 16 <= 8) return false;
+	const uint32_t fewest = dim <= 16 ? 1 : parts ? slices_of(eights ? 8 : 16) : doubles ? std::max<uint32_t>(2, slices_of(32)) : dim <= 48 ? slices_of(16) : slices_of(SUMS64_LANES);
+	uint32_t width = 0;
+	for (uint32_t slices = fewest; slices <= SUMS64_SLICES && (width == 0 || width > 16); ++slices) {
+		const uint32_t equal = (dim - 1) / slices + 1, whole = equal > 8 ? (equal + 15) / 16 * 16 : equal > 4 ? 8 : 4;
+		const bool as_is = doubles ? !eights && !(parts && equal > 8 && (dim - 1) % 16 >= 7) : equal > 32;
+		const uint32_t w = dim <= 16 || as_is ? equal : whole;
+		if (bytes(w) > budget || (dim > 192 && w <= 32 && !doubles)) continue;
+		if (width != 0 && least_points * 2 * chunks_of(width) <= n) break; /* enough points for this many work-groups */
+		width = w;
+	}
+	if (width == 0) return false;
+	uint32_t lanes = 1, copies = 1;
+	while (lanes < width) lanes *= 2;
+	while (copies * 2 <= WAVE / lanes && 2 * copies * bytes(width) <= std::min<uint32_t>(budget, 48 * 1024)) copies *= 2;
+	const uint64_t points = (std::max<uint64_t>(least_points, ((uint64_t)n + chunks_of(width) - 1) / chunks_of(width)) + WAVE - 1) / WAVE * WAVE;
+	const uint32_t chunk_points = (uint32_t)std::min<uint64_t>(points, 1u << 31);
+	*plan = { width, slices_of(width), copies, (uint32_t)(((uint64_t)n + chunk_points - 1) / chunk_points), chunk_points, (uint32_t)(copies * bytes(width)) };
+	return true;
+}
+
+template <int LW, bool FULL, typename F>
+static int launch_sums64(const F* data, size_t stride, const uint32_t* assignment, F* partial, uint32_t* partial_counts, uint32_t dim, uint32_t k, uint32_t n, const Sums64Plan& p)
+{
+	auto kernel = update_sums64_kernel<LW, FULL, F>;
+	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds_bytes));
+	KMX_LAUNCH_KERNEL(kernel, dim3((p.chunks + SUMS64_XCDS - 1) / SUMS64_XCDS * SUMS64_XCDS * p.slices), dim3(SUMS64_THREADS), p.lds_bytes, stream(),
+	                  data, stride, assignment, partial, partial_counts, dim, k, n, p.chunk_points, p.chunks, p.slices, p.width, p.copies);
+	KMX_LAUNCH_CHECK("update_sums64_kernel");
+	return KMX_OK;
+}
+
+template <typename F>
+int launch_update_sums64(const F* data, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
+                         uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, Sums64Result* result)
+{
+	*result = SUMS64_OTHERS;
+	Sums64Plan p;
+	if (n == 0 || !plan_sums64(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p)) return KMX_OK;
+	const size_t sums = (size_t)p.chunks * k * dim, words = sums * (sizeof(F) / sizeof(float)) + (size_t)p.chunks * k;
+	if (recording_graph() && words > ws->partials_cap) {
+		*result = SUMS64_NO_ROOM;
+		return KMX_OK;
+	}
+	int rc = reserve_partials(ws, words);
+	if (rc) return rc;
+	*result = SUMS64_DONE;
+	exec->block_count = p.chunks * p.slices;
+	F* partial = (F*)ws->partials;
+	uint32_t* partial_counts = (uint32_t*)(partial + sums);
+#define KMX_SUMS64(LW) (dim % p.width == 0 && p.width == LW ? launch_sums64<LW, true, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p) \
+	                                                        : launch_sums64<LW, false, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p))
+	rc = p.width <= 1 ? launch_sums64<1, true, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p)
+	   : p.width <= 2 ? KMX_SUMS64(2) : p.width <= 4 ? KMX_SUMS64(4) : p.width <= 8 ? KMX_SUMS64(8) : p.width <= 16 ? KMX_SUMS64(16)
+	   : p.width <= 32 ? KMX_SUMS64(32) : KMX_SUMS64(64);
+#undef KMX_SUMS64
+	if (rc) return rc;
+	return launch_reduce_partials<F>(partial, partial_counts, p.chunks, means, layout_means, stride_means, sizes, dim, k, divide);
+}
+
+template int launch_update_sums64<float>(const float*, size_t, const uint32_t*, float*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
+template int launch_update_sums64<double>(const double*, size_t, const uint32_t*, double*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
+
+} // namespace kmx

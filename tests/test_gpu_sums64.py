@@ -1,0 +1,115 @@
+"""The update whose sums lie in LDS as doubles (csrc/update_sums64.hip): every number of lanes per row, whole and partly filled slices, ends of chunks and
+steps, copies of the sums, members of no cluster, against sums in 64 bits.
+
+The bound: a chunk's sums are exact to a double's rounding and rounded to the result's type once, then at most 256 chunks are added one after the other and the
+sum is divided: 258 roundings of at most the sum of the magnitudes (doubles: one more per member)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+AOS, SOA = 0, 1
+
+
+def check(km, dim, k, n, dtype, stride=None, layout_means=AOS, outside=False, one=False, seed=0):
+    rng = np.random.default_rng(seed + 1000 * dim + k)
+    stride = stride or dim
+    rows = np.full((n, stride), np.nan, dtype)
+    rows[:, :dim] = rng.normal(size=(n, dim)) * np.exp2(rng.integers(-20, 20, size=dim))
+    member = rng.integers(0, k + (2 if outside else 0), size=n).astype(np.uint32)
+    if one:
+        member[:] = k - 1
+    member[-1] = k - 1
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * n); a.write(member)
+    stride_means = dim if layout_means == AOS else k
+    m = km.DeviceBuffer(rows.itemsize * k * dim); s = km.DeviceBuffer(4 * k)
+    m.zero(); s.zero()
+    km.update(km.UPDATE_ATOMIC_SHM, d, AOS, stride, a, m, layout_means, stride_means, s, dim, k, n, None, dtype)
+    got = m.read(dtype, k * dim)
+    got = got.reshape(k, dim) if layout_means == AOS else got.reshape(dim, k).T
+    sizes = s.read(np.uint32, k)
+    for b in (d, a, m, s):
+        b.free()
+    inside = member < k
+    want_sizes = np.bincount(member[inside], minlength=k)
+    assert np.array_equal(sizes, want_sizes)
+    x = rows[inside, :dim].astype(np.longdouble)
+    total, size = np.zeros((k, dim), np.longdouble), np.zeros((k, dim), np.longdouble)
+    np.add.at(total, member[inside], x)
+    np.add.at(size, member[inside], np.abs(x))
+    count = np.maximum(want_sizes, 1)[:, None]
+    unit = np.finfo(dtype).eps / 2
+    roundings = 258 + (count if dtype is np.float64 else 0)
+    assert np.all(np.abs(got - total / count) <= roundings * unit * size / count)
+
+
+# rows of every number of lanes, full and not; 300 clusters of up to 64 coordinates as a whole, 1024 in slices; a chunk is 512 or k points and more
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dim,k", [(1, 70), (2, 70), (3, 70), (4, 70), (5, 70), (8, 70), (9, 70), (16, 70), (17, 70), (32, 70), (33, 70), (63, 70), (64, 70), (65, 70), (100, 70), (128, 70), (300, 20), (640, 20), (641, 20),
+                                   (16, 1200), (24, 1200), (32, 1024), (36, 1200), (48, 1024), (56, 1200), (80, 900), (100, 1000), (36, 2500), (4, 4500), (12, 4200), (13, 13000)])
+def test_sums_of_every_width(km, gpu, dim, k, dtype):
+    for n in (20011, 70003):
+        check(km, dim, k, n, dtype, outside=n == 20011)
+
+
+@pytest.mark.parametrize("dim,k", [(1, 2), (2, 2), (4, 3), (7, 2), (16, 4), (30, 5), (64, 2)])
+@pytest.mark.parametrize("n", [16384, 40961, 262144 + 65])
+def test_few_clusters(km, gpu, dim, k, n):
+    check(km, dim, k, n, np.float32)
+    check(km, dim, k, n, np.float32, one=True, seed=1)
+    check(km, dim, k, n, np.float64, one=True, seed=2)
+
+
+@pytest.mark.parametrize("dim,stride", [(5, 9), (16, 19), (33, 40), (50, 56), (96, 101)])
+def test_padded_rows_and_centroids_by_columns(km, gpu, dim, stride):
+    check(km, dim, 200, 50021, np.float32, stride=stride, layout_means=SOA)
+    check(km, dim, 200, 50021, np.float64, stride=stride, layout_means=SOA)
+
+
+def test_infinities_stay_in_their_cluster(km, gpu):
+    dim, k, n = 20, 300, 60000
+    rng = np.random.default_rng(1)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    member = (np.arange(n) % k).astype(np.uint32)
+    rows[7, 3], rows[8, 19], rows[9, 0], rows[9 + k, 0] = np.inf, np.nan, np.inf, -np.inf
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * n); a.write(member)
+    m = km.DeviceBuffer(4 * k * dim); s = km.DeviceBuffer(4 * k)
+    km.update(km.UPDATE_ATOMIC_SHM, d, AOS, dim, a, m, AOS, dim, s, dim, k, n)
+    got = m.read(np.float32, k * dim).reshape(k, dim)
+    assert np.isinf(got[7, 3]) and np.isnan(got[8, 19]) and np.isnan(got[9, 0])
+    odd = np.zeros((k, dim), bool)
+    odd[7, 3] = odd[8, 19] = odd[9, 0] = True
+    assert np.all(np.isfinite(got[~odd]))
+    for b in (d, a, m, s):
+        b.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_recorded_without_room_for_partial_sums(km, gpu, dtype):
+    """Nothing is allocated while a graph is recorded: kernels without partial sums take the call, and every replay gives their result."""
+    dim, k, n = 16, 16, 1 << 16
+    rng = np.random.default_rng(2)
+    rows = rng.normal(size=(n, dim)).astype(dtype)
+    member = rng.integers(0, k, size=n).astype(np.uint32)
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * n); a.write(member)
+    m = km.DeviceBuffer(rows.itemsize * k * dim); s = km.DeviceBuffer(4 * k)
+    update = lambda n: km.update(km.UPDATE_ATOMIC_SHM, d, AOS, dim, a, m, AOS, dim, s, dim, k, n, None, dtype)
+    km.sync()
+    km.check(km.hip_lib().kmx_shutdown())
+    if dtype == np.float32:
+        update(64)   # the work space as such, without partial sums
+    with km.Graph() as g:
+        m.zero(); s.zero()
+        update(n)
+    want = np.stack([rows[member == c].astype(np.float64).mean(0) for c in range(k)])
+    for _ in range(3):
+        m.write(np.full(k * dim, np.nan, dtype)); s.write(np.full(k, 7, np.uint32))
+        g.launch()
+        km.sync()
+        assert np.array_equal(s.read(np.uint32, k), np.bincount(member, minlength=k))
+        assert np.abs(m.read(dtype, k * dim).reshape(k, dim) - want).max() < 1e-5
+    g.destroy()
+    for b in (d, a, m, s):
+        b.free()
