@@ -31,6 +31,31 @@ template <typename F> __device__ __forceinline__ F small_sqrt(F v);
 template <> __device__ __forceinline__ float small_sqrt<float>(float v) { return __builtin_sqrtf(v); }
 template <> __device__ __forceinline__ double small_sqrt<double>(double v) { return __builtin_sqrt(v); }
 
+/* a root and its centroid's number (0xFFFFFFFF: none), ordered as the serial scan decides */
+template <typename F> struct SmallKey {
+	F root; uint32_t at;
+	SmallKey() = default;
+	__device__ __forceinline__ SmallKey(F root, uint32_t at) : root(root), at(at) {}
+	__device__ __forceinline__ SmallKey of_lane(int off) const { return SmallKey(__shfl_xor(root, off), (uint32_t)__shfl_xor((int)at, off)); }
+	__device__ __forceinline__ uint32_t number() const { return at; }
+	__device__ __forceinline__ void take(const SmallKey& o)
+	{
+		const bool pinned = at == 0 && root != root, other_pinned = o.at == 0 && o.root != o.root;
+		const bool wins = other_pinned || (!pinned && o.at != 0xFFFFFFFFu && (at == 0xFFFFFFFFu || o.root < root || (o.root == root && o.at < at)));
+		root = wins ? o.root : root;
+		at = wins ? o.at : at;
+	}
+};
+template <> struct SmallKey<float> { /* roots are not negative: their bits are in their order, NaN behind infinity */
+	unsigned long long bits;
+	SmallKey() = default;
+	__device__ __forceinline__ SmallKey(float root, uint32_t at)
+	    : bits(at == 0xFFFFFFFFu ? ~0ull : at == 0 && root != root ? 0ull : (unsigned long long)__float_as_uint(root) << 32 | at) {}
+	__device__ __forceinline__ SmallKey of_lane(int off) const { SmallKey o; o.bits = __shfl_xor(bits, off); return o; }
+	__device__ __forceinline__ uint32_t number() const { return (uint32_t)bits; }
+	__device__ __forceinline__ void take(const SmallKey& o) { bits = o.bits < bits ? o.bits : bits; }
+};
+
 /* The serial scan compares correctly rounded square roots. Two sums whose ratio is below this differ in their roots by more
  * than one unit in the last place, so comparing the sums decides; between this and 1 the roots themselves are compared. (Below
  * `tiny` the sums may be subnormal and their ratio means nothing.) */
@@ -39,8 +64,8 @@ template <> struct SqrtMargin<float> { static constexpr float ratio = 0.9999995f
 template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e-15, tiny = 1e-290; };
 
 /*
- * A work-group owns 64 points, whose rows it stages in LDS next to a chunk of the centroids. A wavefront is 16 x 4 lanes with
- * T points times T centroids each, so it covers 16 T points and 4 T centroids at a time; the eight wavefronts are 4 / T groups of
+ * A work-group owns 64 points (or 32, see SMALL_HALF_POINTS), whose rows it stages in LDS next to a chunk of the centroids. A wavefront is 16 x 4 lanes with
+ * T points times T centroids each, so it covers 16 T points and 4 T centroids at a time; of 64 points, the eight wavefronts are 4 / T groups of
  * points times 2 T shares of the centroids. Per four dimensions a lane reads 2 T pieces of 16 bytes for its T^2 pairs: with T = 2
  * (192 ALU cycles against 128 of the LDS that four SIMDs share) the vector ALU sets the pace, T = 1 (48 against 64) is for a
  * dozen centroids at most, which would leave most of the larger tile empty. (A lane per point with the centroids broadcast is
@@ -53,10 +78,9 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  * k = 10 14.0 against 13.4 us, N = 65000, d = 5, k = 50 10.0 against 9.5). The row stride is an odd number of 16-byte pieces: rows read together start in
  * different banks. Every sum runs in ascending dimension, every operation rounded separately.
  *
- * SUMS: membership (clusters x 64 points) times rows (64 points x coordinates) on v_mfma_f32_16x16x4_f32: 1.0 times a coordinate is
- * exact, the accumulators add in fp32. A wavefront has 16 clusters and goes over the coordinates 16 at a time; where that leaves
- * wavefronts over, they share out the coordinates (N = 5000, d = 200, k = 20: 24.4 -> 20.7 us). 0.0 times an infinity or a NaN would reach every cluster: a work-group that sees one adds its points up again, an
- * element of the sums per lane.
+ * SUMS: the rows, which are still in LDS, added up in doubles where the centroids were, one ds_add_f64 per coordinate (8 cycles of a wavefront; memberships
+ * times rows on the fp32 matrix instruction, which keeps the vector ALU, took 2.1 instead of 0.5 us of a work-group: N = 10240, d = 20, k = 128 17.7 -> 16.4 us per
+ * iteration, N = 65536, d = 8, k = 64 20.5 -> 18.4, N = 20000, d = 20, k = 100 22.3 -> 19.4).
  */
 constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading the memberships again (update_small_kernel) is cheaper than as many partial sums */
 constexpr uint32_t SMALL_POINTS = WAVE;
@@ -77,18 +101,18 @@ template <typename F> __device__ __forceinline__ uint32_t small_items(const Smal
 /* AoS: up to B items of every lane, all of them requested before the first is placed. Lanes without an item ask for nothing: a repeated one costs the
  * caches as much as any (N = 65536, d = 8, k = 64: seven of eight were). For the first items only: with any number of them in such batches and their
  * branches N = 94 doubles, d = 186, k = 3 took 9.3 us, with stage_items 7.9; N = 675 doubles, d = 195, k = 108: 58.6, 53.8. */
-template <typename F, int B>
+template <typename F, int B, uint32_t THREADS>
 struct SmallBatch {
 	typedef typename SmallVec<F>::type F4;
 	F4 v[B];
 	uint32_t at[B];
-	static __device__ __forceinline__ bool holds(const SmallRows<F>& s) { return small_items(s) <= B * SMALL_THREADS; }
+	static __device__ __forceinline__ bool holds(const SmallRows<F>& s) { return small_items(s) <= B * THREADS; }
 	__device__ __forceinline__ void request(const SmallRows<F>& s)
 	{
 		const uint32_t items = small_items(s);
 #pragma unroll
 		for (int u = 0; u < B; ++u) {
-			const uint32_t i = u * SMALL_THREADS + threadIdx.x;
+			const uint32_t i = u * THREADS + threadIdx.x;
 			if (i >= items) continue;
 			const uint32_t e = s.vec4 ? i * 4 : i, r = s.dim == 1 ? e : __umulhi(e, s.magic), q = e - r * s.dim;
 			const F* from = s.src + (size_t)min(r, s.last) * s.stride + q;
@@ -102,7 +126,7 @@ struct SmallBatch {
 		const uint32_t items = small_items(s);
 #pragma unroll
 		for (int u = 0; u < B; ++u) {
-			if (u * SMALL_THREADS + threadIdx.x >= items) continue;
+			if (u * THREADS + threadIdx.x >= items) continue;
 			if (s.vec4) *(F4*)(s.to + at[u]) = v[u];
 			else s.to[at[u]] = v[u].x;
 		}
@@ -114,18 +138,18 @@ struct SmallBatch {
  * later chunks of centroids have a piece or two for a lane: N = 8000 doubles, d = 48, k = 300 42.8 us, with repeated ones 44.7). Single coordinates: six at a
  * time, which is what 64 registers hold, the last one again behind the end: no branches between the loads.
  */
-template <typename F, bool VEC>
+template <typename F, bool VEC, uint32_t THREADS>
 __device__ __forceinline__ void stage_items(const SmallRows<F>& s, uint32_t from)
 {
 	typedef typename std::conditional<VEC, typename SmallVec<F>::type, F>::type V;
 	constexpr int BATCH = VEC ? 4 : 6;
 	const uint32_t last = small_items(s) - 1, one = s.dim == 1 ? 1u : 0u; /* (magic is 0 for rows of one) */
-	for (uint32_t i0 = from * SMALL_THREADS + threadIdx.x; i0 <= last; i0 += SMALL_THREADS * BATCH) {
+	for (uint32_t i0 = from * THREADS + threadIdx.x; i0 <= last; i0 += THREADS * BATCH) {
 		V v[BATCH];
 		uint32_t at[BATCH];
 #pragma unroll
 		for (int u = 0; u < BATCH; ++u) {
-			const uint32_t i = i0 + u * SMALL_THREADS;
+			const uint32_t i = i0 + u * THREADS;
 			if (VEC && i > last) continue;
 			const uint32_t e = min(i, last) * (VEC ? 4 : 1), r = __umulhi(e, s.magic) + e * one, q = e - r * s.dim;
 			at[u] = r * s.row_stride + q;
@@ -133,7 +157,7 @@ __device__ __forceinline__ void stage_items(const SmallRows<F>& s, uint32_t from
 		}
 #pragma unroll
 		for (int u = 0; u < BATCH; ++u)
-			if (!VEC || i0 + u * SMALL_THREADS <= last) *(V*)(s.to + at[u]) = v[u];
+			if (!VEC || i0 + u * THREADS <= last) *(V*)(s.to + at[u]) = v[u];
 	}
 }
 
@@ -143,28 +167,28 @@ __device__ __forceinline__ void stage_items(const SmallRows<F>& s, uint32_t from
  * us: N = 21376, d = 2, k = 287 18.7, 17.6; N = 2550, d = 8, k = 284 15.0, 13.6; N = 43539, d = 9, k = 111 14.5, 13.6; but N = 53567, d = 42, k = 32 12.4, 13.3;
  * N = 3895, d = 252, k = 2 10.0, and 15.7 in batches of four).
  */
-template <typename F>
+template <typename F, uint32_t WAVES>
 __device__ __forceinline__ void stage_columns(const SmallRows<F>& s)
 {
 	constexpr uint32_t BATCH = 8;
 	const uint32_t lane = threadIdx.x % WAVE, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
-	if (s.dim >= 2 * SMALL_WAVES) {
+	if (s.dim >= 2 * WAVES) {
 		for (uint32_t r0 = 0; r0 < s.count; r0 += WAVE) {
 			const uint32_t r = min(r0 + lane, s.count - 1);
 			const F* src = s.src + min(r, s.last);
-			for (uint32_t q0 = wave; q0 < s.dim; q0 += SMALL_WAVES * BATCH) {
+			for (uint32_t q0 = wave; q0 < s.dim; q0 += WAVES * BATCH) {
 				F v[BATCH];
 #pragma unroll
-				for (uint32_t u = 0; u < BATCH; ++u) v[u] = src[(size_t)min(q0 + u * SMALL_WAVES, s.dim - 1) * s.stride];
+				for (uint32_t u = 0; u < BATCH; ++u) v[u] = src[(size_t)min(q0 + u * WAVES, s.dim - 1) * s.stride];
 #pragma unroll
-				for (uint32_t u = 0; u < BATCH; ++u) s.to[r * s.row_stride + min(q0 + u * SMALL_WAVES, s.dim - 1)] = v[u];
+				for (uint32_t u = 0; u < BATCH; ++u) s.to[r * s.row_stride + min(q0 + u * WAVES, s.dim - 1)] = v[u];
 			}
 		}
 		return;
 	}
 	/* groups of wavefronts, each with all columns of its blocks (one group where the columns are as many as wavefronts) */
-	const bool few = s.dim < SMALL_WAVES;
-	const uint32_t group = !few ? 0 : s.dim == 1 ? wave : __umulhi(wave, s.magic), groups = !few ? 1 : s.dim == 1 ? SMALL_WAVES : __umulhi(SMALL_WAVES, s.magic);
+	const bool few = s.dim < WAVES;
+	const uint32_t group = !few ? 0 : s.dim == 1 ? wave : __umulhi(wave, s.magic), groups = !few ? 1 : s.dim == 1 ? WAVES : __umulhi(WAVES, s.magic);
 	const uint32_t first = wave - group * s.dim;
 	uint32_t q = first, r0 = group < groups ? group * WAVE : s.count;
 	while (r0 < s.count) {
@@ -177,7 +201,7 @@ __device__ __forceinline__ void stage_columns(const SmallRows<F>& s)
 			at[u] = r * s.row_stride + q;
 			v[u] = s.src[(size_t)q * s.stride + min(r, s.last)];
 			got = u + 1;
-			q += SMALL_WAVES;
+			q += WAVES;
 			const bool wrap = q >= s.dim;
 			q = wrap ? first : q;
 			r0 += wrap ? groups * WAVE : 0u;
@@ -188,35 +212,33 @@ __device__ __forceinline__ void stage_columns(const SmallRows<F>& s)
 	}
 }
 
-template <typename F, int L>
+template <typename F, int L, uint32_t THREADS>
 __device__ __forceinline__ void stage_rows(const SmallRows<F>& s, uint32_t from)
 {
-	if (L == KMX_SOA) stage_columns(s);
-	else if (s.vec4) stage_items<F, true>(s, from);
-	else stage_items<F, false>(s, from);
+	if (L == KMX_SOA) stage_columns<F, THREADS / WAVE>(s);
+	else if (s.vec4) stage_items<F, true, THREADS>(s, from);
+	else stage_items<F, false, THREADS>(s, from);
 }
 
-template <typename F, int T, int LD, int LM, bool SUMS>
-__global__ void __launch_bounds__(SMALL_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(F) == 4 ? 8 : 4)))
+template <typename F, int T, int POINTS, uint32_t THREADS, int LD, int LM, bool SUMS>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(F) == 4 && THREADS == 512 ? 8 : 4)))
 assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restrict__ means, size_t stride_means,
                     uint32_t* __restrict__ assignment, uint32_t dim, uint32_t k, uint32_t n, uint32_t row_stride, uint32_t chunk,
                     uint32_t magic, uint32_t vec4, uint32_t* __restrict__ counters, F* __restrict__ partial, uint32_t* __restrict__ partial_counts)
 {
 	typedef typename SmallVec<F>::type F4;
-	constexpr uint32_t POINTS = SMALL_POINTS;
-	constexpr uint32_t PG = 4 / T, CW = SMALL_WAVES / PG; /* groups of points, shares of the centroids */
+	constexpr uint32_t WAVES = THREADS / WAVE, PG = POINTS / 16 / T, CW = WAVES / PG; /* groups of points, shares of the centroids */
 	extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
 	F* rows = (F*)lds_raw;
-	F* cents = rows + (size_t)POINTS * row_stride; /* chunk rows; with SUMS later k * dim sums and k counts */
-	__shared__ F cand_dist[CW][POINTS];
-	__shared__ uint32_t cand_idx[CW][POINTS];
+	F* cents = rows + (size_t)POINTS * row_stride; /* chunk rows; with SUMS later k * dim doubles and k counts */
+	__shared__ SmallKey<F> cand[CW][POINTS];
 	__shared__ __attribute__((aligned(16))) uint32_t member[POINTS];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 	const uint32_t pg = wave % PG, cw = wave / PG;
 	const uint32_t lp = lane & 15, lc = lane >> 4; /* points lp + 16 p of the group, centroids T lc + u of the wavefront's 4 T */
 	const uint32_t first = blockIdx.x * POINTS;
-	const uint32_t here = min(POINTS, n - first);
+	const uint32_t here = min((uint32_t)POINTS, n - first);
 	if (blockIdx.x == 0 && tid == 0) counters[0] = 0u; /* nothing is left to an exact pass */
 
 	auto centroids = [&](uint32_t base) -> SmallRows<F> {
@@ -230,7 +252,7 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 		bool rest = true;
 		if constexpr (LD == KMX_AOS && LM == KMX_AOS) {
 			/* points and centroids travel together where all of them do, or where both are whole pieces: one trip to memory instead of two */
-			typedef SmallBatch<F, 4> Batch;
+			typedef SmallBatch<F, 4, THREADS> Batch;
 			rest = !(Batch::holds(points) && Batch::holds(start));
 			if (!rest || (points.vec4 && start.vec4)) {
 				Batch some, others;
@@ -242,8 +264,8 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 			}
 		}
 		if (rest) {
-			stage_rows<F, LD>(points, staged);
-			stage_rows<F, LM>(start, staged);
+			stage_rows<F, LD, THREADS>(points, staged);
+			stage_rows<F, LM, THREADS>(start, staged);
 		}
 	}
 
@@ -256,7 +278,7 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 		const uint32_t count = min(chunk, k - base);
 		if (base) {
 			__syncthreads(); /* the previous chunk is no longer needed */
-			stage_rows<F, LM>(centroids(base), 0);
+			stage_rows<F, LM, THREADS>(centroids(base), 0);
 		}
 		__syncthreads();
 		for (uint32_t c0 = cw * (4 * T); c0 < count; c0 += CW * (4 * T)) {
@@ -314,94 +336,43 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 			}
 		}
 	}
-	/* the four lanes of a point, then the wavefronts: the smaller root, then the smaller number. The share that holds centroid 0
-	 * keeps a NaN root of it against everything. */
+	/* the four lanes of a point, then the wavefronts: the smaller root, then the smaller number; centroid 0 keeps a NaN root against everything, any other loses
+	 * with one. Floats: as one comparison of 64 bits (N = 10240, d = 20, k = 128 15.2 -> 14.6 us per iteration, N = 65536, d = 8, k = 64 18.4 -> 17.7). */
+	typedef SmallKey<F> Key;
 #pragma unroll
 	for (int p = 0; p < T; ++p) {
-		F d = small_sqrt(low[p]);
-		uint32_t i = at[p];
+		Key key(small_sqrt(low[p]), at[p]);
 #pragma unroll
-		for (int off = 16; off < WAVE; off <<= 1) {
-			const F od = __shfl_xor(d, off);
-			const uint32_t oi = (uint32_t)__shfl_xor((int)i, off);
-			const bool pinned = i == 0 && d != d, other_pinned = oi == 0 && od != od;
-			const bool wins = other_pinned || (!pinned && oi != 0xFFFFFFFFu && (i == 0xFFFFFFFFu || od < d || (od == d && oi < i)));
-			d = wins ? od : d;
-			i = wins ? oi : i;
-		}
-		if (lc == 0) { cand_dist[cw][pg * (16 * T) + lp + 16 * p] = d; cand_idx[cw][pg * (16 * T) + lp + 16 * p] = i; }
+		for (int off = 16; off < WAVE; off <<= 1) key.take(key.of_lane(off));
+		if (lc == 0) cand[cw][pg * (16 * T) + lp + 16 * p] = key;
 	}
 	__syncthreads();
+	double* sums = (double*)cents; /* SUMS: k * dim of them, then k counts; the centroids are no longer needed */
+	uint32_t* counts = (uint32_t*)(sums + k * dim);
+	if constexpr (SUMS) {
+		for (uint32_t i = tid; i < k * dim; i += THREADS) sums[i] = 0.0;
+		for (uint32_t i = tid; i < k; i += THREADS) counts[i] = 0u;
+	}
 	if (tid < POINTS) {
-		F best = cand_dist[0][tid];
-		uint32_t idx = cand_idx[0][tid];
+		Key best = cand[0][tid];
 #pragma unroll
-		for (uint32_t w = 1; w < CW; ++w) {
-			const F d = cand_dist[w][tid];
-			const uint32_t i = cand_idx[w][tid];
-			const bool wins = i != 0xFFFFFFFFu && (d < best || (d == best && i < idx));
-			best = wins ? d : best;
-			idx = wins ? i : idx;
-		}
+		for (uint32_t w = 1; w < CW; ++w) best.take(cand[w][tid]);
+		const uint32_t idx = best.number();
 		if (tid < here) assignment[first + tid] = idx;
 		if (SUMS) member[tid] = tid < here ? idx : 0xFFFFFFFFu;
 	}
 
 	if constexpr (SUMS) {
-		typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-		uint32_t* counts = (uint32_t*)cents; /* k words; the centroids are no longer needed */
-		__shared__ uint32_t not_finite;
-		if (tid == 0) not_finite = 0u;
-		for (uint32_t i = tid; i < k; i += SMALL_THREADS) counts[i] = 0u;
 		__syncthreads();
+		for (uint32_t e = tid; e < here * dim; e += THREADS) {
+			const uint32_t p = dim == 1 ? e : __umulhi(e, magic), q = e - p * dim;
+			unsafeAtomicAdd(&sums[member[p] * dim + q], (double)rows[p * row_stride + q]);
+		}
 		if (tid < here) atomicAdd(&counts[member[tid]], 1u);
-		F* out = partial + (size_t)blockIdx.x * k * dim;
-		const uint32_t l16 = lane & 15, quad = lane >> 4;
-		bool bad = false;
-		/* wavefronts beyond one per 16 clusters share out the coordinates */
-		const uint32_t across = min((k + 15) / 16, SMALL_WAVES);
-		uint32_t column = wave, share = 0, shares = 1;
-		while (column >= across) { column -= across; ++share; }
-		while ((shares + 1) * across <= SMALL_WAVES) ++shares;
-		for (uint32_t cluster = column * 16; cluster < k && share < shares; cluster += across * 16) {
-			for (uint32_t d0 = share * 16; d0 < dim; d0 += shares * 16) {
-				const F* at_row = rows + quad * row_stride + min(d0 + l16, dim - 1);
-				const uint32_t* whose = member + quad;
-				f32x4 sum = { 0.0f, 0.0f, 0.0f, 0.0f };
-#pragma unroll 1
-				for (uint32_t i = 0; i < POINTS / 4; i += 8) { /* (all 16 at once take more registers than eight wavefronts of a SIMD have) */
-#pragma unroll
-					for (uint32_t j = 0; j < 8; ++j) {
-						const float in = whose[4 * j] == cluster + l16 ? 1.0f : 0.0f; /* point 4 (i + j) + quad belongs to cluster + l16 */
-						const float x = at_row[4 * j * row_stride];
-						bad = bad || !(__builtin_fabsf(x) < __builtin_inff());
-						sum = __builtin_amdgcn_mfma_f32_16x16x4f32(in, x, sum, 0, 0, 0);
-					}
-					whose += 32;
-					at_row += 32 * row_stride;
-				}
-#pragma unroll
-				for (uint32_t r = 0; r < 4; ++r)
-					if (cluster + 4 * quad + r < k && d0 + l16 < dim) out[(size_t)(cluster + 4 * quad + r) * dim + d0 + l16] = sum[r];
-			}
-		}
-		if (bad) not_finite = 1u;
 		__syncthreads();
-		for (uint32_t i = tid; i < k; i += SMALL_THREADS) partial_counts[(size_t)blockIdx.x * k + i] = counts[i];
-		if (not_finite) { /* (the stores above have left before the barrier) */
-			for (uint32_t e = tid; e < k * dim; e += SMALL_THREADS) {
-				const uint32_t cl = e / dim, d = e - cl * dim;
-				F s = (F)0;
-#pragma unroll 1 /* (rare, and not worth the registers) */
-				for (uint32_t p = 0; p < POINTS; p += 4) {
-					const u4 m = *(const u4*)(member + p);
-#pragma unroll
-					for (uint32_t i = 0; i < 4; ++i)
-						if (m[i] == cl) s += rows[(p + i) * row_stride + d];
-				}
-				out[e] = s;
-			}
-		}
+		F* out = partial + (size_t)blockIdx.x * k * dim;
+		for (uint32_t e = tid; e < k * dim; e += THREADS) out[e] = (F)sums[e];
+		for (uint32_t i = tid; i < k; i += THREADS) partial_counts[(size_t)blockIdx.x * k + i] = counts[i];
 	}
 }
 
@@ -537,46 +508,59 @@ template <typename F> static uint32_t assign_small_chunk(uint32_t dim, uint32_t 
 	const uint32_t fit = 32 * 1024 / (small_row_stride(dim) * (uint32_t)sizeof(F)) / 32 * 32;
 	return std::min(k, std::max(32u, fit));
 }
-template <typename F> static uint32_t assign_small_lds(uint32_t dim, uint32_t k)
+template <typename F> static uint32_t assign_small_lds(uint32_t dim, uint32_t k, uint32_t points, bool sums)
 {
-	return (SMALL_POINTS + assign_small_chunk<F>(dim, k)) * small_row_stride(dim) * (uint32_t)sizeof(F);
+	const uint32_t centroids = assign_small_chunk<F>(dim, k) * small_row_stride(dim) * (uint32_t)sizeof(F);
+	return points * small_row_stride(dim) * (uint32_t)sizeof(F) + (sums ? std::max(centroids, k * dim * 8 + k * 4) : centroids);
 }
 
 constexpr uint32_t SMALL_FEW_CENTROIDS = 12; /* up to here a tile of one point times one centroid per lane */
 
 /*
  * Every pair costs 3 dim operations and about 30 to compare and keep, four cycles each on a SIMD; a work-group of 64 points keeps one
- * compute unit, so fewer than 256 of them leave units idle. Fitted: 12 us + effort / 2.6e7 per us. The general path takes 30 to
- * 35 us for rows of up to 32 dimensions, 50 to 75 us for wider ones (N = 30000, d = 32: k = 40 18.5 against 42.8 us, k = 150 31.9
- * against 35.5, k = 600 76 against 46; d = 100: k = 40 30.6 against 55.6, k = 150 54.8 against 65.3), twice that for doubles.
+ * compute unit, so fewer than 256 of them leave units idle. Us per iteration near the line, these kernels / the general path: N = 40000, d = 32, k = 100
+ * (effort 504 million) 28.7 / 40.3; N = 32768, d = 32, k = 128 (528) 27.1 / 31.5; N = 65536, d = 16, k = 100 (511) 27.2 / 32.0; N = 50000, d = 16, k = 128 (499)
+ * 29.9 / 28.3; N = 65536, d = 8, k = 200 (708) 33.8 / 29.3. Wider rows, per assignment: N = 65536, d = 64, k = 50 (727) 20.4 / 22.6; N = 40000, d = 64, k = 80
+ * (710) 20.2 / 21.7; N = 20000, d = 64, k = 200 (888) 32.1 / 22.7. Twice that for doubles.
  * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
  */
 constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
-constexpr uint64_t SMALL_EFFORT = 450000000;
+constexpr uint64_t SMALL_EFFORT = 530000000;
 template <typename F>
 bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
 	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
 	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
 	const uint64_t limit = SMALL_EFFORT * (dim > 32 ? 3 : 2) / 2 * (sizeof(F) / 4);
-	return effort <= limit && assign_small_lds<F>(dim, k) + assign_small_static<F>() <= lds_budget;
+	return effort <= limit && assign_small_lds<F>(dim, k, SMALL_POINTS, false) + assign_small_static<F>() <= lds_budget;
 }
+
+/*
+ * Up to 128 work-groups of 64 points leave half of the compute units idle: 32 points each (us per iteration, 64 / 32 points: N = 1000, d = 20, k = 128 14.4 / 12.0;
+ * N = 5000, d = 32, k = 100 16.5 / 14.5; N = 10240, d = 20, k = 128 16.4 / 16.6: twice the partial sums). Little more than one work-group per compute unit: 16
+ * wavefronts each, whose waits for the LDS others cover (eight / 16: N = 10240, d = 20, k = 128 16.4 / 15.2; N = 16384 15.9 / 15.0; N = 20000, k = 100
+ * 19.4 / 19.3; N = 32768, d = 8, k = 64 13.6 / 14.6).
+ */
+constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 20000;
 
 template <typename F, bool SUMS>
 static int launch_assign_small_t(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
                                  uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, F* partial, uint32_t* partial_counts, uint32_t* blocks, const DeviceInfo& dev)
 {
-	const uint32_t lds = assign_small_lds<F>(dim, k);
-	*blocks = (n + SMALL_POINTS - 1) / SMALL_POINTS;
+	const bool half = n <= SMALL_HALF_POINTS, wide = !half && n <= SMALL_WIDE_POINTS;
+	const uint32_t points = half ? SMALL_POINTS / 2 : SMALL_POINTS;
+	const uint32_t lds = assign_small_lds<F>(dim, k, points, SUMS);
+	*blocks = (n + points - 1) / points;
 	const uint32_t align = 4 * sizeof(F) - 1;
 	const uint32_t vec4 = (dim % 4 == 0 && stride % 4 == 0 && ((uintptr_t)data & align) == 0 ? 1u : 0u) | (dim % 4 == 0 && stride_means % 4 == 0 && ((uintptr_t)means & align) == 0 ? 2u : 0u);
 	void (*kernel)(const F*, size_t, const F*, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t*, F*, uint32_t*) = nullptr;
-#define KMX_PICK(P) (layout == KMX_AOS ? (layout_means == KMX_AOS ? assign_small_kernel<F, P, KMX_AOS, KMX_AOS, SUMS> : assign_small_kernel<F, P, KMX_AOS, KMX_SOA, SUMS>) \
-                                       : (layout_means == KMX_AOS ? assign_small_kernel<F, P, KMX_SOA, KMX_AOS, SUMS> : assign_small_kernel<F, P, KMX_SOA, KMX_SOA, SUMS>))
-	kernel = k > SMALL_FEW_CENTROIDS ? KMX_PICK(2) : KMX_PICK(1);
+#define KMX_PICK(P, Q, W) (layout == KMX_AOS ? (layout_means == KMX_AOS ? assign_small_kernel<F, P, Q, W, KMX_AOS, KMX_AOS, SUMS> : assign_small_kernel<F, P, Q, W, KMX_AOS, KMX_SOA, SUMS>) \
+                                       : (layout_means == KMX_AOS ? assign_small_kernel<F, P, Q, W, KMX_SOA, KMX_AOS, SUMS> : assign_small_kernel<F, P, Q, W, KMX_SOA, KMX_SOA, SUMS>))
+	const bool few = k <= SMALL_FEW_CENTROIDS;
+	kernel = half ? (few ? KMX_PICK(1, 32, 512) : KMX_PICK(2, 32, 512)) : wide ? (few ? KMX_PICK(1, 64, 1024) : KMX_PICK(2, 64, 1024)) : few ? KMX_PICK(1, 64, 512) : KMX_PICK(2, 64, 512);
 #undef KMX_PICK
 	if (lds > 48 * 1024) KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(SMALL_THREADS), lds, stream(), data, stride, means, stride_means, assignment, dim, k, n,
+	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(wide ? 1024 : SMALL_THREADS), lds, stream(), data, stride, means, stride_means, assignment, dim, k, n,
 	                   small_row_stride(dim), assign_small_chunk<F>(dim, k), (uint32_t)((0x100000000ull + dim - 1) / dim), vec4, counters, partial, partial_counts);
 	KMX_LAUNCH_CHECK("assign_small_kernel");
 	return KMX_OK;
@@ -589,17 +573,18 @@ int launch_assign_small(const F* data, int layout, size_t stride, const F* means
 	return launch_assign_small_t<F, false>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, counters, nullptr, nullptr, blocks, dev);
 }
 
-/* the single-pass iteration of small inputs: partial sums and counts of *blocks work-groups, for launch_reduce_partials */
+/* the single-pass iteration of small inputs: partial sums and counts of *blocks work-groups, at most assign_small_max_blocks(n), for launch_reduce_partials */
 int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, const DeviceInfo& dev)
 {
 	return launch_assign_small_t<float, true>(a.data, a.layout, a.stride, a.means, a.layout_means, a.stride_means, a.assignment, a.dim, a.k, a.n,
 	                                          counters, partial, partial_counts, blocks, dev);
 }
-uint32_t assign_small_max_blocks(uint32_t n) { return (n + SMALL_POINTS - 1) / SMALL_POINTS; }
+uint32_t assign_small_max_blocks(uint32_t n) { return n <= SMALL_HALF_POINTS ? (n + SMALL_POINTS / 2 - 1) / (SMALL_POINTS / 2) : (n + SMALL_POINTS - 1) / SMALL_POINTS; }
 /* (the partial sums of all work-groups are written and read once) */
 bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
-	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * assign_small_max_blocks(n) <= (2u << 20) && small_assign_fits<float>(dim, k, n, lds_budget);
+	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * ((n + SMALL_POINTS - 1) / SMALL_POINTS) <= (2u << 20) && small_assign_fits<float>(dim, k, n, lds_budget) &&
+	       assign_small_lds<float>(dim, k, SMALL_POINTS, true) + assign_small_static<float>() <= lds_budget;
 }
 
 /*
