@@ -454,9 +454,10 @@ ordered_staged_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
 /*
  * The same for AoS rows of whole 16-byte pieces: a work-group per cluster (`large`: of that list only) and block of 128 bytes of the row. One wavefront requests the members'
  * rows straight to LDS, AHEAD batches of eight requests before they are added, and the members' numbers AHEAD batches before that; the other one
- * adds, a lane per coordinate, two members per LDS read, and waits for nothing but the batch's barrier. What bounds it is the longest
- * cluster's chain, at 1.5 instructions a member (N = 100k, d = 36, k = 2: 4.9 ns a member; with one wavefront that requests and adds 7.8), then the memory
- * (N = 2M, d = 32, k = 1024: 80 us, 3.4 TB/s; one wavefront 107, the staged kernel above 169). AHEAD of 1, 2, 3, 4 with one wavefront: 133, 106,
+ * adds, a lane per coordinate, two members per LDS read, three parts of eight to 16 members on their way from LDS, across the barrier between two batches too.
+ * What bounds it is the longest cluster's chain, at 1.5 to 1.6 instructions a member, which a wavefront alone issues every five cycles (rows of 16 bytes 2.9 ns a
+ * member, of 128 bytes 4.0; with one part on its way, from anew in every batch, 3.6 and 4.9; with one wavefront that requests and adds 7.8), then the memory
+ * (N = 2M, d = 32, k = 1024: 64 us, with one part 77; one wavefront 107, the staged kernel above 169). AHEAD of 1, 2, 3, 4 with one wavefront: 133, 106,
  * 107, 122 us (four work-groups fit a compute unit with up to 3).
  */
 constexpr uint32_t STREAM_REQUESTS = 8, STREAM_SLOT_BYTES = STREAM_REQUESTS * WAVE * 16;
@@ -504,11 +505,13 @@ ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
 			named += BATCH;
 			name_slot = name_slot + 1 < SLOTS ? name_slot + 1 : 0;
 		};
-		auto request_rows = [&]() {
+		uint32_t point[STREAM_REQUESTS];
+		auto read_names = [&]() {
 			const uint32_t* names = (const uint32_t*)(stream_lds + SLOTS * STREAM_SLOT_BYTES) + row_slot * (NAMES * WAVE) + row;
-			uint32_t point[STREAM_REQUESTS];
 #pragma unroll
 			for (uint32_t j = 0; j < STREAM_REQUESTS; ++j) point[j] = names[j * ROWS];
+		};
+		auto request_rows = [&]() {
 #pragma unroll
 			for (uint32_t j = 0; j < STREAM_REQUESTS; ++j) stream_request16((const char*)piece + (uint64_t)point[j] * row_bytes, rows_at + row_slot * STREAM_SLOT_BYTES + j * (WAVE * 16));
 			row_slot = row_slot + 1 < SLOTS ? row_slot + 1 : 0;
@@ -527,11 +530,12 @@ ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
 		for (uint32_t i = 0; i < AHEAD; ++i) request_names();
 		asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
 #pragma unroll
-		for (uint32_t i = 0; i < AHEAD; ++i) { request_names(); request_rows(); }
+		for (uint32_t i = 0; i < AHEAD; ++i) { request_names(); read_names(); request_rows(); }
 #pragma unroll 1
 		for (uint32_t first = 0; first < members; first += BATCH) {
 			/* the rows of this batch and the names of the one requested now are here (what was requested after them may not be) */
 			asm volatile("s_waitcnt vmcnt(%0)" : : "n"((AHEAD - 1) * EACH) : "memory");
+			read_names();
 			__syncthreads(); /* the rows may be added, and those of the batch before have been */
 			request_names();
 			request_rows();
@@ -542,42 +546,55 @@ ordered_stream_sum_kernel(const F* __restrict__ data, size_t stride, const uint3
 	F sum = (F)0;
 	const uint32_t own = min(lane, width - 1); /* this lane's coordinate */
 	uint32_t from = 0;
+	/* parts of a request's rows (a part behind the last row is read, not added) */
+	constexpr uint32_t PART = ROWS <= 16 ? ROWS : ROWS % 16 == 0 ? 16 : 7, PARTS = ROWS / PART, ALL = STREAM_REQUESTS * PARTS;
+	static_assert(ROWS % PART == 0 && ALL % 4 == 0, "whole parts, whole rounds");
+	/* three parts are on their way while one is added, across the barrier between two batches too (the first time round zeros, which the sum of nothing takes
+	 * without a trace) */
+	F x[4][PART];
+#pragma unroll
+	for (uint32_t u = 1; u < 4; ++u)
+#pragma unroll
+		for (uint32_t r = 0; r < PART; ++r) x[u][r] = (F)0;
+	auto add = [&](const F (&part)[PART]) {
+#pragma unroll
+		for (uint32_t r = 0; r < PART; ++r) sum = sum + part[r];
+	};
+	uint32_t first = 0;
 #pragma unroll 1
-	for (uint32_t first = 0; first < members; first += BATCH) {
+	for (; first + BATCH <= members; first += BATCH) {
 		__syncthreads();
 		const F* mine = (const F*)(stream_lds + from * STREAM_SLOT_BYTES) + own;
 		from = from + 1 < SLOTS ? from + 1 : 0;
-		/* parts of a request's rows, the next part read while one is added (a part behind the last row is read, not added) */
-		constexpr uint32_t PART = ROWS <= 16 ? ROWS : ROWS % 16 == 0 ? 16 : 7, PARTS = ROWS / PART;
-		static_assert(ROWS % PART == 0, "whole parts");
-		F x[2][PART];
+#pragma unroll
+		for (uint32_t at = 0; at < ALL; ++at) {
+#pragma unroll
+			for (uint32_t r = 0; r < PART; ++r) x[at % 4][r] = mine[at / PARTS * (WAVE * PIECE) + (at % PARTS * PART + r) * (P * PIECE)];
+			__builtin_amdgcn_sched_barrier(0);
+			add(x[(at + 1) % 4]);
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	}
+	add(x[1]); add(x[2]); add(x[3]);
+	if (first < members) { /* the last batch, not full */
+		__syncthreads();
+		const F* mine = (const F*)(stream_lds + from * STREAM_SLOT_BYTES) + own;
+		const uint32_t here = members - first;
 		auto read = [&](F (&into)[PART], uint32_t at) {
+			at = min(at, ALL - 1);
 #pragma unroll
 			for (uint32_t r = 0; r < PART; ++r) into[r] = mine[at / PARTS * (WAVE * PIECE) + (at % PARTS * PART + r) * (P * PIECE)];
 		};
 		read(x[0], 0);
-		if (first + BATCH <= members) {
-#pragma unroll
-			for (uint32_t at = 0; at < STREAM_REQUESTS * PARTS; ++at) {
-				if (at + 1 < STREAM_REQUESTS * PARTS) read(x[(at + 1) % 2], at + 1);
-				__builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-				for (uint32_t r = 0; r < PART; ++r) sum = sum + x[at % 2][r];
-				__builtin_amdgcn_sched_barrier(0);
-			}
-		}
-		else {
-			const uint32_t here = members - first;
 #pragma unroll 1
-			for (uint32_t at = 0; at * PART < here; at += 2) {
+		for (uint32_t at = 0; at * PART < here; at += 2) {
 #pragma unroll
-				for (uint32_t u = 0; u < 2; ++u) {
-					read(x[(u + 1) % 2], min(at + u + 1, STREAM_REQUESTS * PARTS - 1));
-					__builtin_amdgcn_sched_barrier(0);
+			for (uint32_t u = 0; u < 2; ++u) {
+				read(x[(u + 1) % 2], at + u + 1);
+				__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-					for (uint32_t r = 0; r < PART; ++r) sum = (at + u) * PART + r < here ? sum + x[u][r] : sum;
-					__builtin_amdgcn_sched_barrier(0);
-				}
+				for (uint32_t r = 0; r < PART; ++r) sum = (at + u) * PART + r < here ? sum + x[u][r] : sum;
+				__builtin_amdgcn_sched_barrier(0);
 			}
 		}
 	}
