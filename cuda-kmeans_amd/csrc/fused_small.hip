@@ -801,45 +801,51 @@ fused_matrix_kernel(const float* __restrict__ data, size_t stride, const float* 
 }
 
 /*
- * What the single pass leaves: the serial scan over all centroids for the points in the queue, 32 lanes per point (a centroid each),
- * their rows added up in LDS; the work-group that finishes last adds the sums and counts of all of them to those of the single pass
- * and divides (the guarded divide of the reference's divideMeansKernel, kernels.cu:149-163). Global atomics instead, a few hundred
- * per address, took 44 to 80 us for 29000 points; the three launches before this one (exact pass, additions, division) took 44 us.
- * Bound by latency: a dozen trips to memory.
+ * What the single pass leaves: the serial scan over all centroids for the points in the queue, 16 or 32 lanes per point (a centroid each),
+ * their rows added up in LDS, in doubles (an LDS addition of floats takes a wavefront 194 cycles, of doubles 8 to 17); the work-group that finishes last adds the
+ * sums and counts of all of them to those of the single pass and divides (the guarded divide of the reference's divideMeansKernel, kernels.cu:149-163). Global
+ * atomics instead, a few hundred per address, took 44 to 80 us for 29000 points; the three launches before this one (exact pass, additions, division) took 44 us.
+ * Bound by latency: a dozen trips to memory, and by what one compute unit gets past the caches at the end. (22000 points, d = 16, k = 16: 26 us with 32 lanes per
+ * point, additions of floats and a word per load at the end, now 20.)
  */
 constexpr uint32_t FINISH_THREADS = 1024;
-constexpr uint32_t FINISH_GROUP = 32;                             /* lanes per point: k, dim <= 32 */
-constexpr uint32_t FINISH_POINTS = FINISH_THREADS / FINISH_GROUP; /* points of a work-group at a time */
 constexpr uint32_t FINISH_SHARE = 128;                            /* points that are worth a work-group */
 
-template <int LD, int LM>
+template <int LD, int LM, uint32_t GROUP> /* lanes per point: k <= GROUP */
 __global__ void __launch_bounds__(FINISH_THREADS)
 fused_finish_kernel(const float* __restrict__ data, size_t stride, const float* __restrict__ means_in, uint32_t* __restrict__ assignment,
                     float* __restrict__ means_out, size_t stride_means, uint32_t* __restrict__ sizes,
-                    const uint32_t* __restrict__ queue, uint32_t* __restrict__ counters, float* __restrict__ partials, uint32_t dim, uint32_t k)
+                    const uint32_t* __restrict__ queue, uint32_t* __restrict__ counters, unsigned long long* __restrict__ partials, uint32_t dim, uint32_t k)
 {
+	constexpr uint32_t POINTS = FINISH_THREADS / GROUP; /* of a work-group at a time */
+	constexpr uint32_t EACH = 32 / GROUP;               /* coordinates of a lane (dim <= 32) */
 	__shared__ float centroids[32 * 33]; /* odd rows: consecutive centroids in different banks */
-	__shared__ float sums[32 * 32], rows[FINISH_POINTS][32];
+	__shared__ double sums[32 * 32];
+	__shared__ float rows[POINTS][32];
 	__shared__ uint32_t members[32];
+	__shared__ unsigned long long shares_of[FINISH_THREADS];
 	__shared__ bool last;
 	const uint32_t count = counters[0], tid = threadIdx.x;
 	const uint32_t working = min(gridDim.x, max(1u, (count + FINISH_SHARE - 1) / FINISH_SHARE));
 	if (blockIdx.x >= working) return;
 	for (uint32_t i = tid; i < k * dim; i += FINISH_THREADS) {
 		centroids[i / dim * 33 + i % dim] = means_in[elem<LM>(stride_means, i / dim, i % dim)];
-		sums[i] = 0.0f;
+		sums[i] = 0.0;
 	}
 	if (tid < 32) members[tid] = 0u;
 	__syncthreads();
-	const uint32_t group = tid / FINISH_GROUP, lane = tid % FINISH_GROUP;
+	const uint32_t group = tid / GROUP, lane = tid % GROUP;
 	const float* mine = centroids + min(lane, k - 1) * 33;
 	float* x = rows[group];
-	/* (the two groups of a wavefront go round together: one without a point of its own repeats the last one and adds nothing) */
-	for (uint32_t base = blockIdx.x * FINISH_POINTS; base < count; base += working * FINISH_POINTS) {
+	/* (the groups of a wavefront go round together: one without a point of its own repeats the last one and adds nothing) */
+	for (uint32_t base = blockIdx.x * POINTS; base < count; base += working * POINTS) {
 		const bool valid = base + group < count;
 		const uint32_t pt = queue[2 * (size_t)min(base + group, count - 1)];
-		const float coordinate = data[elem<LD>(stride, pt, min(lane, dim - 1))];
-		x[lane] = coordinate;
+		float coordinate[EACH];
+#pragma unroll
+		for (uint32_t u = 0; u < EACH; ++u) coordinate[u] = data[elem<LD>(stride, pt, min(lane + u * GROUP, dim - 1))];
+#pragma unroll
+		for (uint32_t u = 0; u < EACH; ++u) x[lane + u * GROUP] = coordinate[u];
 		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 		__builtin_amdgcn_wave_barrier();
 		float sum = 0.0f;
@@ -853,24 +859,25 @@ fused_finish_kernel(const float* __restrict__ data, size_t stride, const float* 
 		/* distance bits, then the number: the first centroid's NaN beats everything, like in the scan (see evaluate_pair) */
 		unsigned long long key = lane >= k ? ~0ull : (lane == 0 && dist != dist) ? 0ull : (((unsigned long long)__float_as_uint(dist) << 32) | lane);
 #pragma unroll
-		for (int off = FINISH_GROUP / 2; off > 0; off >>= 1) {
+		for (int off = GROUP / 2; off > 0; off >>= 1) {
 			const unsigned long long other = __shfl_xor(key, off);
 			key = other < key ? other : key;
 		}
 		const uint32_t winner = (uint32_t)key;
 		if (valid && lane == 0) { assignment[pt] = winner; atomicAdd(&members[winner], 1u); }
-		if (valid && lane < dim) unsafeAtomicAdd(&sums[winner * dim + lane], coordinate);
+#pragma unroll
+		for (uint32_t u = 0; u < EACH; ++u)
+			if (valid && lane + u * GROUP < dim) unsafeAtomicAdd(&sums[winner * dim + lane + u * GROUP], (double)coordinate[u]);
 		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 		__builtin_amdgcn_wave_barrier();
 	}
 	__syncthreads();
-	/* this work-group's sums and counts: element e of all work-groups side by side would be written one word per line */
-	const uint32_t words = k * dim + k;
+	/* this work-group's sums and counts, two words at a time (element e of all work-groups side by side would be written one word per line) */
+	const uint32_t words = k * dim + k, pairs = (words + 1) / 2;
+	auto word = [&](uint32_t e) -> uint32_t { return e < k * dim ? __float_as_uint((float)sums[e]) : e < words ? members[e - k * dim] : 0u; };
 	if (working > 1) {
-		for (uint32_t e = tid; e < words; e += FINISH_THREADS) {
-			const float v = e < k * dim ? sums[e] : __uint_as_float(members[e - k * dim]);
-			__hip_atomic_store(&partials[(size_t)blockIdx.x * words + e], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		}
+		for (uint32_t e = tid; e < pairs; e += FINISH_THREADS)
+			__hip_atomic_store(&partials[(size_t)blockIdx.x * pairs + e], (unsigned long long)word(2 * e + 1) << 32 | word(2 * e), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		/* They are there before the work-group counts as finished: stores of device scope pass the L2 by, so that having completed is
 		 * enough. (A fence of device scope writes the L2 back, per wavefront: 45 us for 230 work-groups.) */
 		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -880,49 +887,55 @@ fused_finish_kernel(const float* __restrict__ data, size_t stride, const float* 
 		if (!last) return;
 		/* the counter said that all partial sums are there; nothing below is read ahead of it (one fence per call: only the last work-group gets here) */
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-	}
-	const uint32_t shares = FINISH_THREADS / 256; /* lanes per element, in passes of 256 elements */
-	float* share_sums = rows[0]; /* 1024 floats */
-	for (uint32_t e0 = 0; e0 < words; e0 += 256) {
-		const uint32_t e = e0 + tid % 256, share = tid / 256;
-		float sum = 0.0f;
-		uint32_t size = 0;
-		if (working > 1 && e < words) {
-			constexpr uint32_t BATCH = 16;
+		/* Several lanes per pair, 16 partial sums of each under way. One compute unit gets some 30 bytes a ns past the caches: their bytes are what this costs */
+		constexpr uint32_t BATCH = 16;
+		const uint32_t across = min(pairs, FINISH_THREADS), shares = FINISH_THREADS / across, share = tid / across, e = tid % across; /* (at most 528 pairs) */
+		double sum[2] = { 0.0, 0.0 };
+		uint32_t size[2] = { 0u, 0u };
+		if (share < shares)
 			for (uint32_t g = share; g < working; g += BATCH * shares) {
-				float v[BATCH];
+				unsigned long long v[BATCH];
 #pragma unroll
 				for (uint32_t u = 0; u < BATCH; ++u)
-					v[u] = __hip_atomic_load(&partials[(size_t)min(g + u * shares, working - 1) * words + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					v[u] = __hip_atomic_load(&partials[(size_t)min(g + u * shares, working - 1) * pairs + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
 				for (uint32_t u = 0; u < BATCH; ++u)
 					if (g + u * shares < working) {
-						if (e < k * dim) sum += v[u];
-						else size += __float_as_uint(v[u]);
+#pragma unroll
+						for (int i = 0; i < 2; ++i) {
+							const uint32_t w = (uint32_t)(v[u] >> (32 * i));
+							if (2 * e + i < k * dim) sum[i] += (double)__uint_as_float(w);
+							else size[i] += w;
+						}
 					}
 			}
-		}
-		else if (share == 0 && e < words) {
-			if (e < k * dim) sum = sums[e];
-			else size = members[e - k * dim];
-		}
-		__syncthreads(); /* (rows, then the shares of the pass before, have been read) */
-		share_sums[tid] = e < k * dim ? sum : __uint_as_float(size);
-		__syncthreads();
-		if (share == 0 && e < words) {
-			for (uint32_t v = 1; v < shares; ++v) {
-				if (e < k * dim) sum += share_sums[v * 256 + tid];
-				else size += __float_as_uint(share_sums[v * 256 + tid]);
+#pragma unroll
+		for (int i = 0; i < 2; ++i) {
+			const bool counts = 2 * e + i >= k * dim;
+			__syncthreads(); /* (all sums have been read, then the shares of the first words) */
+			shares_of[tid] = counts ? size[i] : (unsigned long long)__double_as_longlong(sum[i]);
+			__syncthreads();
+			if (share == 0 && 2 * e + i < words) {
+				for (uint32_t v = 1; v < shares; ++v) {
+					const unsigned long long other = shares_of[v * across + tid];
+					if (counts) size[i] += (uint32_t)other;
+					else sum[i] += __longlong_as_double((long long)other);
+				}
+				if (counts) members[2 * e + i - k * dim] = size[i];
+				else sums[2 * e + i] = sum[i];
 			}
-			/* the sums of the queue; the counts first have to be complete */
-			if (e < k * dim) sums[e] = sum;
-			else { members[e - k * dim] = sizes[e - k * dim] + size; sizes[e - k * dim] = members[e - k * dim]; }
 		}
+		__syncthreads();
+	}
+	/* the counts first have to be complete */
+	if (tid < k) {
+		members[tid] += sizes[tid];
+		sizes[tid] = members[tid];
 	}
 	__syncthreads();
 	for (uint32_t e = tid; e < k * dim; e += FINISH_THREADS) {
 		float* mean = &means_out[elem<LM>(stride_means, e / dim, e % dim)];
-		const float sum = *mean + sums[e];
+		const float sum = (float)((double)*mean + sums[e]);
 		const uint32_t size = members[e / dim];
 		*mean = size > 0 ? sum / (float)size : sum;
 	}
@@ -996,7 +1009,7 @@ static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t*
 	const uint32_t dp = fused_dp(a.dim);
 	const uint32_t kp = round_up(a.k, TILE);
 	const uint32_t blocks = std::min(dev.compute_units, (a.n + FINISH_SHARE - 1) / FINISH_SHARE);
-	int rc = reserve_partials(ws, (size_t)blocks * (a.k * a.dim + a.k)); /* (ahead of the launches: a recording that cannot have it is refused whole) */
+	int rc = reserve_partials(ws, (size_t)blocks * ((a.k * a.dim + a.k + 1) / 2 * 2)); /* (ahead of the launches: a recording that cannot have it is refused whole) */
 	if (rc) return rc;
 	/* the ranking works in a frame moved to the middle of the centroids when they lie far from the origin */
 	rc = launch_pack_means(a, ws, dp, kp, FRAME_MOVED_IF_FAR, clear);
@@ -1013,8 +1026,9 @@ static int launch_fused_layouts(const AssignArgs& a, float* means_out, uint32_t*
 	default: return fail(KMX_ERR_UNSUPPORTED, "fused iteration: dim %u is not supported by the single-pass kernel", a.dim);
 	}
 	if (rc) return rc;
-	KMX_LAUNCH_KERNEL((fused_finish_kernel<LD, LM>), dim3(blocks), dim3(FINISH_THREADS), 0, stream(),
-	                   a.data, a.stride, a.means, a.assignment, means_out, a.stride_means, sizes, ws->queue, ws->counters, ws->partials, a.dim, a.k);
+	auto finish = a.k <= 16 ? fused_finish_kernel<LD, LM, 16> : fused_finish_kernel<LD, LM, 32>;
+	KMX_LAUNCH_KERNEL(finish, dim3(blocks), dim3(FINISH_THREADS), 0, stream(),
+	                   a.data, a.stride, a.means, a.assignment, means_out, a.stride_means, sizes, ws->queue, ws->counters, (unsigned long long*)ws->partials, a.dim, a.k);
 	KMX_LAUNCH_CHECK("fused_finish_kernel");
 	return KMX_OK;
 }
