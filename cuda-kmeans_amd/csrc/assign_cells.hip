@@ -39,13 +39,21 @@ constexpr float CELL_CLEAR = 1.000002f;
 constexpr uint32_t CELL_TIES = 2;
 constexpr uint32_t CELL_MAX_K = 6144;              /* what the building kernel's LDS holds */
 constexpr uint32_t CELL_UNIT = 8;                  /* entries (16 bits) of a list that are read together */
-constexpr uint32_t CELL_POOL_UNITS = 1u << 20;
+/*
+ * A building work-group's lists go to a region of its own if they fit, else to what all share, by an addition to one counter (256 additions that come
+ * together take 2 us or more: all by the counter, d = 2, k = 1000: 67.2 instead of 65.5 us for the call, d = 3: 74.5 instead of 72.1).
+ */
+constexpr uint32_t CELL_SHARED_UNITS = 1u << 20, CELL_OWN_UNITS = 1u << 18;
+constexpr uint32_t CELL_POOL_UNITS = CELL_SHARED_UNITS + CELL_OWN_UNITS;
 constexpr uint32_t CELL_SAMPLE = 64;               /* centroids of the list for points without one, at the start of the pool */
-constexpr uint32_t CELL_TRUNCATED = 1u << 31;      /* table entry: list start in units (20 bits), length in units (11), this flag */
-constexpr uint32_t CELL_MOST_UNITS = (1u << 11) - 1;
+constexpr uint32_t CELL_TRUNCATED = 1u << 31;      /* table entry: list start in units (21 bits), length in units (10), this flag */
+constexpr uint32_t CELL_START_BITS = 21, CELL_MOST_UNITS = (1u << 10) - 1;
+static_assert(CELL_POOL_UNITS <= 1u << CELL_START_BITS, "table entries");
 constexpr uint32_t BUILD_THREADS = 1024;
 constexpr uint32_t BUILD_WAVES = BUILD_THREADS / WAVE;
 constexpr uint32_t BUILD_SHORT = 1024;             /* most centroids on the list of a second-level cell */
+static_assert(BUILD_SHORT <= CELL_MOST_UNITS * CELL_UNIT, "a list's length");
+constexpr uint32_t BUILD_OWN = CELL_MAX_K / BUILD_THREADS; /* most centroids of a thread */
 
 /* cells per dimension: TOP of the first level (a work-group each), times MID (a wavefront each), times LOW */
 template <int D> struct CellShape;
@@ -83,12 +91,77 @@ __device__ __forceinline__ void cell_distances(const float (&c)[D], const float 
 	}
 }
 
+/* all sums of one value per dimension, the last dimension's numbered fastest: sums of both halves of the dimensions first */
+template <int D, uint32_t EACH>
+__device__ __forceinline__ void all_sums(const float (&v)[D][EACH], float (&sums)[power(EACH, D)])
+{
+	constexpr int LEFT = D / 2, RIGHT = D - LEFT;
+	static_assert(D >= 2 && D <= 4, "halves of one or two dimensions");
+	float left[power(EACH, LEFT)], right[power(EACH, RIGHT)];
+#pragma unroll
+	for (uint32_t i = 0; i < power(EACH, LEFT); ++i) left[i] = LEFT == 1 ? v[0][i] : v[0][i / EACH] + v[1][i % EACH];
+#pragma unroll
+	for (uint32_t i = 0; i < power(EACH, RIGHT); ++i) right[i] = RIGHT == 1 ? v[D - 1][i] : v[D - 2][i / EACH] + v[D - 1][i % EACH];
+#pragma unroll
+	for (uint32_t c = 0; c < power(EACH, D); ++c) sums[c] = left[c / power(EACH, RIGHT)] + right[c % power(EACH, RIGHT)];
+}
+
+template <int CONTROL>
+__device__ __forceinline__ float other_lane(float v) { return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CONTROL, 0xF, 0xF, true)); }
+constexpr int ROW_ROR_8 = 0x128, ROW_HALF_MIRROR = 0x141, QUAD_XOR_2 = 0x4E, QUAD_XOR_1 = 0xB1;
+
+/*
+ * M values per lane: the least of number lane / (WAVE / M) over the wavefront. (Not through LDS, as shuffles are; a mirrored half row's lanes pair all of one
+ * half of it with all of the other, which is as good as lanes 4 apart.)
+ */
+template <uint32_t M, uint32_t OFF = WAVE / 2>
+__device__ __forceinline__ float least_of_each(const float (&v)[M], uint32_t lane)
+{
+	constexpr uint32_t H = M > 1 ? M / 2 : 1;
+	float half[H];
+#pragma unroll
+	for (uint32_t i = 0; i < H; ++i) {
+		const float first = v[i], second = v[M > 1 ? i + H : i]; /* for the lanes whose bit OFF is clear, is set */
+		if constexpr (OFF == 32 || OFF == 16) {
+			const auto both = OFF == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(first), __float_as_uint(second), false, false)
+			                            : __builtin_amdgcn_permlane16_swap(__float_as_uint(first), __float_as_uint(second), false, false);
+			half[i] = fminf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+		}
+		else {
+			constexpr int CONTROL = OFF == 8 ? ROW_ROR_8 : OFF == 4 ? ROW_HALF_MIRROR : OFF == 2 ? QUAD_XOR_2 : QUAD_XOR_1;
+			const bool upper = M > 1 && (lane & OFF) != 0;
+			half[i] = fminf(upper ? second : first, other_lane<CONTROL>(upper ? first : second));
+		}
+	}
+	if constexpr (OFF > 1) return least_of_each<H, OFF / 2>(half, lane);
+	else return half[0];
+}
+
+/* the least of 2 OFF neighbouring lanes */
+template <uint32_t OFF = WAVE / 2>
+__device__ __forceinline__ float least_of_lanes(float v)
+{
+	const float one[1] = { v };
+	return least_of_each<1, OFF>(one, 0);
+}
+
+/* lanes of the mask below this one */
+__device__ __forceinline__ uint32_t lanes_before(unsigned long long mask)
+{
+	return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+__device__ __forceinline__ float of_lane(float v, uint32_t lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+
 /*
  * One work-group per first-level cell. All of them find the box of the centroids (they have to read them anyway), then three levels of
  * lists, each filtered from the one above: the work-group's, one per wavefront, one per cell. On the way a wavefront packs a row for
  * the exact pass and the packed sweep (as a kernel of its own ahead of this one that took 5 to 7 us and a launch).
- * What bounds it: the box distances (the vector ALU is busy three quarters of the 42 to 46 us at k = 4096, d = 4), then its dozen barriers (one level
- * of lists, every cell from all centroids, would be 65536 x k boxes, a millisecond).
+ * What bounds it: the slowest work-group (uniform centroids, k = 4096, d = 4: half of the work-groups are done after 22 us, the last one, whose lists are
+ * twice as long, after 31), in it the second level's box distances (9 us) and the writing of the lists (6), then the barriers. One level of lists,
+ * every cell from all centroids, would be 65536 x k boxes, a millisecond. A thread's centroids stay in registers from the box to the first list, and a
+ * wavefront's cells are filtered together (below): 50 -> 31 us; k = 1000, d = 3: the call 79 -> 72 us. (The second level's cells together as well, all
+ * wavefronts on one list: its slowest work-group as slow, the others by 2 us, d = 3, k = 1000: 76 -> 80 us for the call.)
  */
 template <int D, int LM>
 __global__ void __launch_bounds__(BUILD_THREADS)
@@ -101,8 +174,9 @@ build_cells_kernel(const CellArgs w)
 	float* coords = lds;                                        /* k x D, relative to the corner */
 	uint16_t* first_list = (uint16_t*)(lds + w.k * D);          /* k */
 	uint16_t* second_lists = first_list + (w.k + 1) / 2 * 2;    /* BUILD_WAVES x BUILD_SHORT */
-	__shared__ float reduce[2 * D][BUILD_WAVES];
-	__shared__ uint32_t wave_count[BUILD_WAVES], wave_units[BUILD_WAVES], pool_start;
+	__shared__ __attribute__((aligned(16))) float reduce[8][BUILD_WAVES];
+	__shared__ __attribute__((aligned(16))) uint32_t wave_count[BUILD_WAVES];
+	__shared__ uint32_t wave_units[BUILD_WAVES], pool_start;
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 
@@ -116,26 +190,35 @@ build_cells_kernel(const CellArgs w)
 	const uint32_t first_row = blockIdx.x * BUILD_WAVES + wave;
 	float exact = w.means[elem<LM>(w.stride_means, min(first_row, w.k - 1), min(lane, (uint32_t)D - 1))];
 
-	/* the box of the centroids (of their finite coordinates) */
-	float low[D], high[D];
+	/* the box of the centroids (of their finite coordinates); a thread's own stay in registers, a wavefront's are consecutive */
+	const uint32_t rounds = (w.k + BUILD_THREADS - 1) / BUILD_THREADS, first_own = wave * rounds * WAVE + lane;
+	float own[BUILD_OWN][D];
 #pragma unroll
-	for (int q = 0; q < D; ++q) { low[q] = __builtin_inff(); high[q] = -__builtin_inff(); }
-	bool odd = false;
-	for (uint32_t j = tid; j < w.k; j += BUILD_THREADS)
+	for (uint32_t i = 0; i < BUILD_OWN; ++i)
+		if (i < rounds) {
+			const uint32_t j = min(first_own + i * WAVE, w.k - 1);
+			if constexpr (LM == KMX_AOS) __builtin_memcpy(own[i], w.means + elem<LM>(w.stride_means, j, 0), sizeof(own[i])); /* (one load, which need not be aligned) */
+			else
 #pragma unroll
-		for (int q = 0; q < D; ++q) {
-			const float v = w.means[elem<LM>(w.stride_means, j, q)];
-			coords[j * D + q] = v;
-			const bool finite = __builtin_fabsf(v) < __builtin_inff();
-			low[q] = finite ? fminf(low[q], v) : low[q];
-			high[q] = finite ? fmaxf(high[q], v) : high[q];
-			odd = odd || !finite;
+				for (int q = 0; q < D; ++q) own[i][q] = w.means[elem<LM>(w.stride_means, j, q)];
 		}
+	bool odd = false;
+	float ends[8]; /* least coordinates, least negative ones */
 #pragma unroll
-	for (int q = 0; q < D; ++q) {
-		for (int off = WAVE / 2; off > 0; off >>= 1) { low[q] = fminf(low[q], __shfl_xor(low[q], off)); high[q] = fmaxf(high[q], __shfl_xor(high[q], off)); }
-		if (lane == 0) { reduce[q][wave] = low[q]; reduce[D + q][wave] = high[q]; }
-	}
+	for (uint32_t u = 0; u < 8; ++u) ends[u] = __builtin_inff();
+#pragma unroll
+	for (uint32_t i = 0; i < BUILD_OWN; ++i)
+		if (i < rounds)
+#pragma unroll
+			for (int q = 0; q < D; ++q) {
+				const float v = own[i][q];
+				const bool finite = __builtin_fabsf(v) < __builtin_inff();
+				ends[q] = finite ? fminf(ends[q], v) : ends[q];
+				ends[4 + q] = finite ? fminf(ends[4 + q], -v) : ends[4 + q];
+				odd = odd || !finite;
+			}
+	const float end = least_of_each(ends, lane);
+	if (lane % 8 == 0) reduce[lane / 8][wave] = end;
 #pragma unroll
 	for (int q = 0; q < D; ++q) {
 		float sum = __builtin_fabsf(member[q]) < __builtin_inff() ? member[q] : 0.0f;
@@ -143,16 +226,15 @@ build_cells_kernel(const CellArgs w)
 		sum = sum / 16.0f;
 		frame[q] = __builtin_fabsf(sum) < __builtin_inff() ? sum : 0.0f; /* (the sum of finite values may overflow) */
 	}
-	if (tid == 0) pool_start = 0;
 	bool usable = !__syncthreads_or(odd ? 1 : 0);
 	float corner[D], width[D], inverse[D], far = 0.0f, size = 0.0f;
 	{
+		const float all = least_of_lanes<4>(fminf(reduce[lane / 8][lane % 8 * 2], reduce[lane / 8][lane % 8 * 2 + 1]));
 		const float share = fmaxf(0.75f * __builtin_powf((float)w.k, -1.0f / D), 0.05f); /* of the extent, added on either side */
 		float extent2 = 0.0f;
 #pragma unroll
 		for (int q = 0; q < D; ++q) {
-			float lo = reduce[q][0], hi = reduce[D + q][0];
-			for (uint32_t v = 1; v < BUILD_WAVES; ++v) { lo = fminf(lo, reduce[q][v]); hi = fmaxf(hi, reduce[D + q][v]); }
+			const float lo = of_lane(all, 8 * q), hi = -of_lane(all, 8 * (4 + q));
 			far = fmaxf(far, fmaxf(hi - frame[q], frame[q] - lo));
 			size = fmaxf(size, fmaxf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
 			const float half = fmaxf(0.5f * (hi - lo) * (1.0f + 2.0f * share), 1e-6f * (__builtin_fabsf(lo) + __builtin_fabsf(hi)) + 1e-16f);
@@ -175,7 +257,7 @@ build_cells_kernel(const CellArgs w)
 		w.grid->corner[tid] = c; w.grid->inverse[tid] = i; w.grid->width[tid] = s;
 	}
 	if (blockIdx.x == 0 && tid < CELL_SAMPLE) w.pool[tid] = (uint16_t)((uint64_t)tid * w.k / CELL_SAMPLE);
-	const uint32_t nothing = CELL_TRUNCATED | (CELL_SAMPLE / CELL_UNIT) << 20; /* the sample */
+	const uint32_t nothing = CELL_TRUNCATED | (CELL_SAMPLE / CELL_UNIT) << CELL_START_BITS; /* the sample */
 
 	/* the packed rows, as pack_means16_kernel and pack_means_bf16_kernel make them */
 	{
@@ -245,11 +327,6 @@ build_cells_kernel(const CellArgs w)
 		if (writes) w.table[cell] = nothing;
 		return; /* (the whole work-group) */
 	}
-	for (uint32_t j = tid; j < w.k; j += BUILD_THREADS)
-#pragma unroll
-		for (int q = 0; q < D; ++q) coords[j * D + q] -= corner[q]; /* (this lane's own entries) */
-	__syncthreads();
-
 	auto box = [&](float (&lo)[D], float (&hi)[D], const uint32_t (&first)[D], uint32_t cells) {
 #pragma unroll
 		for (int q = 0; q < D; ++q) {
@@ -273,34 +350,49 @@ build_cells_kernel(const CellArgs w)
 #pragma unroll
 		for (int q = 0; q < D; ++q) start[q] = top[q] * MID * LOW;
 		box(lo, hi, start, MID * LOW);
-		float bound = __builtin_inff();
-#pragma unroll 2
-		for (uint32_t j = tid; j < w.k; j += BUILD_THREADS) {
-			float least, most;
-			measure(j, lo, hi, least, most);
-			bound = fminf(bound, most);
-		}
-		for (int off = WAVE / 2; off > 0; off >>= 1) bound = fminf(bound, __shfl_xor(bound, off));
+		float bound = __builtin_inff(), least[BUILD_OWN];
+#pragma unroll
+		for (uint32_t i = 0; i < BUILD_OWN; ++i)
+			if (i < rounds) {
+				const uint32_t j = first_own + i * WAVE;
+				float most;
+#pragma unroll
+				for (int q = 0; q < D; ++q) own[i][q] -= corner[q];
+				cell_distances<D>(own[i], lo, hi, least[i], most);
+				bound = fminf(bound, most); /* (behind the last centroid: that one again) */
+				if (j < w.k)
+#pragma unroll
+					for (int q = 0; q < D; ++q) coords[j * D + q] = own[i][q];
+			}
+		bound = least_of_lanes(bound);
+		__syncthreads(); /* (the box has been read) */
 		if (lane == 0) reduce[0][wave] = bound;
 		__syncthreads();
-		bound = reduce[0][0];
-		for (uint32_t v = 1; v < BUILD_WAVES; ++v) bound = fminf(bound, reduce[0][v]);
-		for (uint32_t base = 0; base < w.k; base += BUILD_THREADS) {
-			const uint32_t j = base + tid;
-			float least = __builtin_inff(), most;
-			if (j < w.k) measure(j, lo, hi, least, most);
-			const bool keep = j < w.k && least <= enough(bound);
-			const unsigned long long mask = __ballot(keep);
-			if (lane == 0) wave_count[wave] = (uint32_t)__popcll(mask);
-			__syncthreads();
-			uint32_t before = first_count;
-			for (uint32_t v = 0; v < BUILD_WAVES; ++v) {
-				before += v < wave ? wave_count[v] : 0u;
-				first_count += wave_count[v];
+		bound = enough(least_of_lanes<BUILD_WAVES / 2>(reduce[0][lane % BUILD_WAVES]));
+		unsigned long long masks[BUILD_OWN];
+		uint32_t count = 0;
+#pragma unroll
+		for (uint32_t i = 0; i < BUILD_OWN; ++i)
+			if (i < rounds) {
+				masks[i] = __ballot(first_own + i * WAVE < w.k && least[i] <= bound);
+				count += (uint32_t)__popcll(masks[i]);
 			}
-			if (keep) first_list[before + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)j;
-			__syncthreads();
+		if (lane == 0) wave_count[wave] = count;
+		__syncthreads();
+		uint32_t to = 0;
+#pragma unroll
+		for (uint32_t v = 0; v < BUILD_WAVES; ++v) {
+			const uint32_t c = wave_count[v];
+			to += v < wave ? c : 0u;
+			first_count += c;
 		}
+#pragma unroll
+		for (uint32_t i = 0; i < BUILD_OWN; ++i)
+			if (i < rounds) {
+				if (masks[i] >> lane & 1) first_list[to + lanes_before(masks[i])] = (uint16_t)(first_own + i * WAVE);
+				to += (uint32_t)__popcll(masks[i]);
+			}
+		__syncthreads();
 	}
 
 	/* the wavefront's list */
@@ -318,16 +410,16 @@ build_cells_kernel(const CellArgs w)
 			measure(first_list[i], lo, hi, least, most);
 			bound = fminf(bound, most);
 		}
-		for (int off = WAVE / 2; off > 0; off >>= 1) bound = fminf(bound, __shfl_xor(bound, off));
+		bound = enough(least_of_lanes(bound));
 #pragma unroll 4
 		for (uint32_t base = 0; base < first_count; base += WAVE) {
 			const uint32_t i = base + lane;
 			const uint16_t j = first_list[min(i, first_count - 1)];
 			float least, most;
 			measure(j, lo, hi, least, most);
-			const bool keep = i < first_count && least <= enough(bound);
+			const bool keep = i < first_count && least <= bound;
 			const unsigned long long mask = __ballot(keep);
-			const uint32_t to = second_count + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+			const uint32_t to = second_count + lanes_before(mask);
 			if (keep && to < BUILD_SHORT) second_list[to] = j;
 			second_count += (uint32_t)__popcll(mask);
 		}
@@ -336,36 +428,78 @@ build_cells_kernel(const CellArgs w)
 	__builtin_amdgcn_wave_barrier();
 	const bool too_long = second_count > BUILD_SHORT;
 
-	/* the cells' lists: LANES lanes share a cell, a contiguous part of the wavefront's list each */
-	const uint32_t part = lane % LANES;
-	const uint32_t i0 = too_long ? 0u : part * second_count / LANES, i1 = too_long ? 0u : (part + 1) * second_count / LANES;
-	box(lo, hi, at, 1);
-	float bound = __builtin_inff();
-#pragma unroll 4
-	for (uint32_t i = i0; i < i1; ++i) {
-		float least, most;
-		measure(second_list[i], lo, hi, least, most);
-		bound = fminf(bound, most);
-	}
-	for (uint32_t off = LANES / 2; off > 0; off >>= 1) bound = fminf(bound, __shfl_xor(bound, (int)off));
-	bound = enough(bound);
-	uint32_t count = 0;
-	unsigned long long kept = 0; /* which of this lane's first 63 */
-#pragma unroll 4
-	for (uint32_t i = i0; i < i1; ++i) {
-		float least, most;
-		measure(second_list[i], lo, hi, least, most);
-		const bool keep = least <= bound;
-		count += keep ? 1u : 0u;
-		kept |= (unsigned long long)(keep ? 1u : 0u) << min(i - i0, 63u);
-	}
-	uint32_t before = 0, total = 0; /* entries of the lanes before this one, of the cell */
+	/*
+	 * The cells' lists, of all the wavefront's cells at once: a lane per centroid of the list, whose distances from a cell are sums of one of LOW values per
+	 * dimension: 24 additions for the 16 cells of d = 4 (LANES lanes to a cell, a part of the list each and every distance by itself: 16 us of the slowest
+	 * work-group instead of 3.6 at k = 4096).
+	 */
+	const uint32_t turns = too_long ? 0u : (second_count + WAVE - 1) / WAVE;
+	float low_end[D][LOW], high_end[D][LOW];
 #pragma unroll
-	for (uint32_t v = 0; v < LANES; ++v) {
-		const uint32_t c = (uint32_t)__shfl((int)count, (int)(lane - part + v));
-		before += v < part ? c : 0u;
-		total += c;
+	for (int q = 0; q < D; ++q)
+#pragma unroll
+		for (uint32_t l = 0; l < LOW; ++l) {
+			const uint32_t first = (top[q] * MID + mid[q]) * LOW + l;
+			low_end[q][l] = ((float)first - CELL_MARGIN) * width[q];
+			high_end[q][l] = ((float)(first + 1) + CELL_MARGIN) * width[q];
+		}
+	float bounds[LOWS];
+#pragma unroll
+	for (uint32_t c = 0; c < LOWS; ++c) bounds[c] = __builtin_inff();
+	for (uint32_t i = 0; i < turns; ++i) {
+		const uint32_t j = second_list[min(i * WAVE + lane, second_count - 1)];
+		float far[D][LOW], sums[LOWS];
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			const float v = coords[j * D + q];
+#pragma unroll
+			for (uint32_t l = 0; l < LOW; ++l) {
+				const float most = fmaxf(v - low_end[q][l], high_end[q][l] - v);
+				far[q][l] = most * most;
+			}
+		}
+		all_sums<D, LOW>(far, sums);
+#pragma unroll
+		for (uint32_t c = 0; c < LOWS; ++c) bounds[c] = fminf(bounds[c], sums[c]);
 	}
+	const float bound = enough(least_of_each(bounds, lane)); /* of cell lane / LANES */
+#pragma unroll
+	for (uint32_t c = 0; c < LOWS; ++c) bounds[c] = of_lane(bound, c * LANES);
+	uint32_t counts[LOWS], kept[BUILD_SHORT / WAVE / 2]; /* 16 bits a turn, the last turn's lowest: which cells keep this lane's centroid */
+#pragma unroll
+	for (uint32_t c = 0; c < LOWS; ++c) counts[c] = 0;
+#pragma unroll
+	for (uint32_t u = 0; u < BUILD_SHORT / WAVE / 2; ++u) kept[u] = 0;
+	for (uint32_t i = 0; i < turns; ++i) {
+		const bool there = i * WAVE + lane < second_count;
+		const uint32_t j = second_list[min(i * WAVE + lane, second_count - 1)];
+		float out[D][LOW], sums[LOWS];
+#pragma unroll
+		for (int q = 0; q < D; ++q) {
+			const float v = coords[j * D + q];
+#pragma unroll
+			for (uint32_t l = 0; l < LOW; ++l) {
+				const float least = fmaxf(fmaxf(low_end[q][l] - v, v - high_end[q][l]), 0.0f);
+				out[q][l] = least * least;
+				if (q == 0) out[q][l] = there ? out[q][l] : __builtin_inff();
+			}
+		}
+		all_sums<D, LOW>(out, sums);
+		uint32_t bits = 0;
+#pragma unroll
+		for (uint32_t c = 0; c < LOWS; ++c) {
+			const bool keep = sums[c] <= bounds[c];
+			counts[c] += (uint32_t)__popcll(__ballot(keep));
+			bits |= keep ? 1u << c : 0u;
+		}
+#pragma unroll
+		for (uint32_t u = BUILD_SHORT / WAVE / 2 - 1; u > 0; --u) kept[u] = kept[u] << 16 | kept[u - 1] >> 16;
+		kept[0] = kept[0] << 16 | bits;
+	}
+	const uint32_t part = lane % LANES;
+	uint32_t total = 0; /* entries of cell lane / LANES */
+#pragma unroll
+	for (uint32_t c = 0; c < LOWS; ++c) total = lane / LANES == c ? counts[c] : total;
 	uint32_t units = wave < MIDS ? (total + CELL_UNIT - 1) / CELL_UNIT : 0u;
 	const bool fits = units <= CELL_MOST_UNITS && !too_long;
 	if (!fits) units = 0;
@@ -380,29 +514,34 @@ build_cells_kernel(const CellArgs w)
 	if (tid == 0) {
 		uint32_t all = 0;
 		for (uint32_t v = 0; v < BUILD_WAVES; ++v) { const uint32_t u = wave_units[v]; wave_units[v] = all; all += u; }
-		pool_start = CELL_SAMPLE / CELL_UNIT + atomicAdd(w.counters + CELLS_COUNTER, all);
+		constexpr uint32_t GROUPS = power(TOP, D), OWN = (CELL_OWN_UNITS - CELL_SAMPLE / CELL_UNIT) / GROUPS;
+		pool_start = CELL_SAMPLE / CELL_UNIT + (all <= OWN ? blockIdx.x * OWN : GROUPS * OWN + atomicAdd(w.counters + CELLS_COUNTER, all));
 	}
 	__syncthreads();
 	const uint32_t start = pool_start + wave_units[wave] + upto - units; /* (lanes of a cell behind its first: upto counts the cell already) */
 	const bool listed = fits && units > 0 && (uint64_t)start + units <= w.pool_units;
-	if (writes) w.table[cell] = listed ? start | units << 20 : nothing;
-	if (listed && wave < MIDS) {
-		uint16_t* out = w.pool + (size_t)start * CELL_UNIT;
-		uint32_t to = before;
-		kept &= ~(1ull << 63);
-		while (kept) {
-			out[to++] = second_list[i0 + (uint32_t)__builtin_ctzll(kept)];
-			kept &= kept - 1;
+	if (writes) w.table[cell] = listed ? start | units << CELL_START_BITS : nothing;
+	if (listed) /* the last unit is filled up with the row behind the last centroid (which is infinitely far) */
+		for (uint32_t to = total + part; to < units * CELL_UNIT; to += LANES) w.pool[(size_t)start * CELL_UNIT + to] = (uint16_t)w.k;
+	const unsigned long long has_list = __ballot(listed);
+	uint32_t cells = 0; /* that have a list */
+#pragma unroll
+	for (uint32_t c = 0; c < LOWS; ++c) {
+		cells |= (uint32_t)(has_list >> (c * LANES) & 1) << c;
+		counts[c] += (uint32_t)__builtin_amdgcn_readlane((int)(start * CELL_UNIT), (int)(c * LANES)); /* the end of what is still to be written */
+	}
+	for (uint32_t i = turns; i-- > 0;) {
+		const uint16_t j = second_list[min(i * WAVE + lane, second_count - 1)];
+		const uint32_t bits = kept[0] & cells;
+#pragma unroll
+		for (uint32_t u = 0; u < BUILD_SHORT / WAVE / 2; ++u) kept[u] = kept[u] >> 16 | (u + 1 < BUILD_SHORT / WAVE / 2 ? kept[u + 1] << 16 : 0u);
+#pragma unroll
+		for (uint32_t c = 0; c < LOWS; ++c) {
+			const bool keep = bits >> c & 1;
+			const unsigned long long mask = __ballot(keep);
+			counts[c] -= (uint32_t)__popcll(mask);
+			if (keep) w.pool[counts[c] + lanes_before(mask)] = j;
 		}
-		for (uint32_t i = i0 + 63; i < i1; ++i) {
-			const uint16_t j = second_list[i];
-			float least, most;
-			measure(j, lo, hi, least, most);
-			if (least <= bound) out[to++] = j;
-		}
-		/* the lane with the cell's last entry fills the last unit up, with the row behind the last centroid (which is infinitely far) */
-		if (count > 0 && to == total)
-			for (; to < units * CELL_UNIT; ++to) out[to] = (uint16_t)w.k;
 	}
 }
 
@@ -496,7 +635,7 @@ assign_cells_kernel(const CellAssignArgs w)
 		for (uint32_t i = 0; i < CHOICE_EACH; ++i) {
 			bool inside;
 			const uint32_t entry = w.table[locate(sample[i], inside)];
-			uint32_t units = (entry >> 20) & CELL_MOST_UNITS;
+			uint32_t units = (entry >> CELL_START_BITS) & CELL_MOST_UNITS;
 			for (int off = WAVE / 2; off > 0; off >>= 1) units = max(units, (uint32_t)__shfl_xor((int)units, off));
 			most[4] += units * CELL_UNIT;
 			most[5] += (uint32_t)__popcll(__ballot(!inside || (entry & CELL_TRUNCATED)));
@@ -552,8 +691,8 @@ assign_cells_kernel(const CellAssignArgs w)
 		for (int q = 0; q < D; ++q) x[q] = w.data[elem<LD>(w.stride, min(pt, w.n - 1), q)];
 		bool inside;
 		const uint32_t entry = w.table[locate(x, inside)];
-		const uint32_t units = (entry >> 20) & CELL_MOST_UNITS;
-		const uint4* list = (const uint4*)w.pool + (entry & 0xFFFFFu);
+		const uint32_t units = (entry >> CELL_START_BITS) & CELL_MOST_UNITS;
+		const uint4* list = (const uint4*)w.pool + (entry & ((1u << CELL_START_BITS) - 1));
 		float best = __builtin_inff();
 		uint32_t winner = 0; /* as an LDS address */
 		auto compare = [&](const f32x4& c, uint32_t at) {

@@ -186,3 +186,31 @@ def test_recorded_cells_replay(km, orc, gpu, kind):
     g.destroy()
     for b in (d, m, a):
         b.free()
+
+
+@pytest.mark.parametrize("dim", [2, 3, 4])
+@pytest.mark.parametrize("k", [3, 64, 65, 66, 129, 1023, 1024, 1025, 1026, 2049, 6144])
+def test_lists_of_every_length(km, orc, gpu, dim, k):
+    """All centroids but one in one cell, whose list they all are on: 1 to 16 full turns of 64, one less and one more, the longest that is kept
+    (1024 centroids) and the first that is not; and as many centroids as a thread of the building kernel has at most, and at the steps between. The rest of
+    the cells have short lists, which no longer share a counter. The result is the serial scan's, bit for bit."""
+    rng = np.random.default_rng(dim * 101 + k)
+    means = (0.37 + rng.uniform(0, 1e-3, size=(k, dim))).astype(np.float32)
+    means[rng.integers(0, k)] = 1.0
+    n = 4099
+    rows = np.where(rng.random((n, 1)) < 0.5, 0.37 + rng.uniform(-1e-3, 2e-3, size=(n, dim)), rng.uniform(0.2, 1.2, size=(n, dim))).astype(np.float32)
+    want = orc.assign(rows.ravel(), means.ravel(), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    m = km.DeviceBuffer(means.nbytes)
+    a = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for layout in (0, 1):
+            m.write(flat(means, layout))
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, 0, dim, m, layout, km.layout_stride(layout, k, dim), a, dim, k, n)
+            km.sync()
+            assert np.array_equal(a.read(np.uint32, n), want)
+    finally:
+        km.set_two_level_sweep(1)
+    for b in (d, m, a): b.free()
