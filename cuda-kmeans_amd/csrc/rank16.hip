@@ -150,8 +150,8 @@ static int launch_pack16(const AssignArgs& a, Workspace* ws)
 	return KMX_OK;
 }
 
-/* sweeps the points; what is left goes to ws->listed (length in counters[LISTED_COUNTER]), rows of SoA points to ws->queued_rows */
-static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+/* sweeps the points; what is left goes to ws->listed (length in counters[LISTED_COUNTER]), the rows of SoA points to ws->queued_rows: those of listed points, or (copy_all) all */
+static int launch_rank16_sweep(const AssignArgs& a, bool copy_all, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	const uint32_t kb = rank16_kb(a.dim), kp = round_up(a.k, TILE), copy_stride = round_up(a.dim, 8);
 	int rc = reserve_listed(ws, 2 * (size_t)a.n);
@@ -159,7 +159,7 @@ static int launch_rank16_sweep(const AssignArgs& a, kmx_exec_params* exec, Works
 	if (a.layout == KMX_SOA && (rc = reserve_queued_rows(ws, a.n, copy_stride, 0))) return rc;
 	const float* norms = ws->norms16;
 	const Rank16Args w = { a.data, a.stride, (const f16x8*)ws->packed16, norms, norms + rank16_low_offset(kp), norms + rank16_frame_offset(kp), ws->norms16 + rank16_scale_offset(kp),
-	                       a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->queued_rows, copy_stride, a.dim, a.k, kp, a.n, 0,
+	                       a.assignment, ws->listed, ws->counters + LISTED_COUNTER, ws->queued_rows, copy_stride, copy_all, a.dim, a.k, kp, a.n, 0,
 	                       cert_kd_level1(a.dim) + cert_kd_keyed(4) + 8.0f * CERT_UNIT + a.kd_extra, 0 };
 	switch (kb) {
 	case 1: return launch_rank16_1(a, w, exec, ws, dev);
@@ -208,6 +208,7 @@ int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 	/* SoA points go in parts whose copied rows fit the bound of the workspace (1 GiB unless it was set) */
 	const size_t row_bytes = round_up(a.dim, 8) * sizeof(float);
 	const uint32_t part = a.layout == KMX_AOS ? a.n : (uint32_t)std::min<size_t>(a.n, std::max<size_t>(1024, queued_rows_limit() / row_bytes));
+	const bool copy_all = a.rows_out && a.layout == KMX_SOA && part == a.n; /* somebody reads all of them */
 	for (uint32_t first = 0; first < a.n; first += std::min(part, a.n - first)) {
 		AssignArgs p = a;
 		p.n = std::min(part, a.n - first);
@@ -218,7 +219,7 @@ int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 			KMX_LAUNCH_CHECK("clear_word_kernel");
 		}
 		if (first == 0 && (rc = profile_begin(0))) return rc;
-		if ((rc = launch_rank16_sweep(p, exec, ws, dev))) return rc;
+		if ((rc = launch_rank16_sweep(p, copy_all, exec, ws, dev))) return rc;
 		if (first == 0 && (rc = profile_end(0))) return rc;
 		const bool aos = a.layout == KMX_AOS;
 		if (a.points64) rc = launch_listed_exact<double>(p, a.points64 + first, aos ? a.stride : 1, aos ? 1 : a.stride, a.dim, ws, dev);
@@ -227,7 +228,7 @@ int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* 
 		if (rc) return rc;
 	}
 	if (a.settled) *a.settled = true;
-	if (a.rows_out && a.layout == KMX_SOA && part == a.n) *a.rows_out = AosRows{ ws->queued_rows, round_up(a.dim, 8) };
+	if (copy_all) *a.rows_out = AosRows{ ws->queued_rows, round_up(a.dim, 8) };
 	return KMX_OK;
 }
 

@@ -41,6 +41,7 @@ struct Rank16Args {
 	float* scale;          /* S, 1 / S^2; the first work-group puts the maxima of the norms and of the bf16 mid and rest parts behind them */
 	uint32_t* assignment; uint32_t* list; uint32_t* length;
 	float* copies; uint32_t copy_stride; /* SoA: the rows as AoS, zeros behind the coordinates */
+	bool copy_all;         /* of all points, else of the listed ones */
 	uint32_t dim, k, kp, n, chunk_tiles;
 	float kd;
 	uint32_t list_entries; /* of a wavefront's list, resident centroids */
@@ -70,14 +71,15 @@ constexpr uint32_t rank16_slots(uint32_t kb) { return kb >= 12 ? 4 : 2; }
 __host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { return (tiles * NORM_TILE + WAVE - 1) / WAVE; }
 /* what a chunk takes in LDS, its norms behind its operands as whole requests of 64 words */
 __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t tiles) { return tiles * kb * WAVE * 16 + rank16_norm_blocks(tiles) * WAVE * 4; }
+/* SoA: which rows go out as AoS, and how (rank16_copy, copy_listed); AoS: EXCHANGED, to nobody */
+enum Rank16Copies { RANK16_EXCHANGED, RANK16_DIRECT, RANK16_LISTED };
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
-/* direct: SoA rows are not exchanged (rank16_copy) */
-constexpr uint32_t rank16_exchange(uint32_t kb, int layout, bool direct) { return rank16_shared_rows(kb, layout) || (layout == KMX_SOA && !direct) ? RANK16_EXCHANGE : 0; }
-constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, bool direct) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, direct) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_exchange(uint32_t kb, int layout, Rank16Copies copies) { return rank16_shared_rows(kb, layout) || (layout == KMX_SOA && copies == RANK16_EXCHANGED) ? RANK16_EXCHANGE : 0; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, copies) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
 /* the lists of a work-group around resident centroids, lying behind them */
 constexpr uint32_t rank16_list_bytes(uint32_t kb, int layout, uint32_t entries) { return rank16_waves(kb, layout, false) * entries * 8; }
-constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true, false) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
+constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true, RANK16_EXCHANGED) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
  * S for centroids whose coordinates are up to `far` from the frame and up to `size` from the origin, both of a sample: the power of two
@@ -185,17 +187,21 @@ __device__ __forceinline__ void rank16_exchanged() /* LDS keeps the order of a w
 }
 
 /*
- * SoA: the rows go out as AoS on the way, for the exact pass and whatever else reads single rows (coordinates of a listed point lie a
- * cache line each apart; with 9 % of N = 2M, d = 128 listed, gathering them read all data again, 430 us, and was no cheaper right
- * behind the sweep of the point, 360 us. The stores travel behind the matrix instructions). Through LDS, so that four lanes store 64
- * consecutive bytes of a row. `exchange`: RANK16_EXCHANGE words of this wavefront's. Where resident centroids leave no room for it a lane stores
- * its 32 bytes as they are (DIRECT): the centroids would have to stream by otherwise (N = 1M, d = 12, k = 4000 262 us, streamed 368; d = 40,
+ * SoA: rows go out as AoS, for the exact pass (coordinates of a listed point lie a cache line each apart) and whatever else reads single rows.
+ * All of them on the way in, where somebody reads all (the update of an iteration): through LDS, so that four lanes store 64 consecutive bytes of
+ * a row. `exchange`: RANK16_EXCHANGE words of this wavefront's. Where resident centroids leave no room for it a lane stores its 32 bytes as they
+ * are (DIRECT): the centroids would have to stream by otherwise (N = 1M, d = 12, k = 4000 262 us, streamed 368; d = 40,
  * k = 1536 249, 283; d = 64, k = 1150 255, 295; with room for it, d = 64, k = 256, 170 through LDS, 183 without).
+ * For the assignment alone the listed ones are enough (LISTED, see copy_listed in the kernel): writing as many bytes as are read, in the phase in which
+ * the matrix cores wait for the points, cost more than reading the columns' lines of the listed points once more from the memory-side
+ * cache. us per assignment, all rows -> listed ones: N = 2M, d = 128, k = 1024, 9 % listed 854 -> 812 (without any copies 643), 1 % 808 -> 732; d = 32
+ * 256 -> 222; N = 1M, d = 64, k = 500 162 -> 119; d = 90, k = 300 222 -> 157; N = 500000, d = 200, k = 1024 392 -> 331; nearly all listed (coordinates 0 or 1),
+ * d = 64, k = 256 145 -> 89, d = 128, k = 512 193 -> 189.
  */
-template <bool DIRECT>
+template <Rank16Copies COPIES>
 __device__ __forceinline__ void rank16_copy(const Rank16Args& w, const float (&v)[8], uint32_t tile_first, uint32_t kb, uint32_t lane, float* exchange)
 {
-	if (DIRECT) {
+	if (COPIES == RANK16_DIRECT) {
 		const uint32_t pt = tile_first + lane % TILE, d = kb * KBLOCK + lane / TILE * 8;
 		if (pt >= w.n || d >= w.copy_stride) return;
 		float* to = w.copies + (size_t)pt * w.copy_stride + d;
@@ -359,7 +365,7 @@ __device__ __forceinline__ float rank16_both(float v)
  * Rows of up to 64 dimensions and resident centroids: two accumulator sets, the tracking of one tile in pieces behind the matrix
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
-template <int KB, int LD, bool STREAM, bool DIRECT>
+template <int KB, int LD, bool STREAM, Rank16Copies COPIES>
 __global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM) * WAVE, rank16_waves(KB, LD, STREAM) == 12 ? 3 : 2)
 rank16_kernel(const Rank16Args w)
 {
@@ -374,7 +380,7 @@ rank16_kernel(const Rank16Args w)
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
 	__shared__ uint32_t wave_max[4][WAVES];
 	__shared__ uint32_t streamed_lists[STREAM ? WAVES : 1][STREAM ? 2 * RANK16_LIST_STREAMED : 1];
-	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD, DIRECT) ? RANK16_EXCHANGE : 1];
+	__shared__ __attribute__((aligned(16))) float exchanges[WAVES][rank16_exchange(KB, LD, COPIES) ? RANK16_EXCHANGE : 1];
 	uint32_t& claimed = wave_max[3][0];
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
@@ -446,6 +452,96 @@ rank16_kernel(const Rank16Args w)
 	float snap[P][GROUPED ? 1 : SNAP_ROWS];
 	f32x2 kept[P][RANK16_GROUPS / 2]; /* GROUPED: the minima of the leading tile's groups */
 
+	/*
+	 * RANK16_LISTED: the listed points' rows, read again once the sweep has left them: `late`, a bit for each of the 64 points from late_first on.
+	 * Eight lanes a row, LATE_EACH consecutive coordinates each (in LATE_TURNS turns), so that a load touches eight columns: with a lane per
+	 * column every lane had a page of its own (N = 2M, d = 128, k = 1024: 905 against 812 us a call). Up to eight
+	 * rows are requested (request_listed) ahead of the next points and stored
+	 * behind them (store_listed). Many of the 64: their tiles as a whole (copy_tiles).
+	 */
+	constexpr bool LISTED = LD == KMX_SOA && COPIES == RANK16_LISTED;
+	constexpr uint32_t LATE_TURNS = KB > 8 ? 2 : 1, LATE_EACH = KB * KBLOCK / 8 / LATE_TURNS, LATE_VEC = LATE_EACH % 4 == 0 ? 4 : 2, LATE_MANY = 24;
+	static_assert(LATE_EACH % LATE_VEC == 0, "whole stores");
+	uint64_t late = 0;
+	uint32_t late_first = 0;
+	struct Late { float v[LATE_EACH]; uint32_t point; }; /* point: 64 for none */
+	auto late_rows = [&](Late& l) { /* the next eight */
+		l.point = 64;
+#pragma unroll
+		for (uint32_t g = 0; g < 8; ++g) {
+			const uint32_t bit = late ? (uint32_t)__builtin_ctzll(late) : 64u;
+			late &= late - 1; /* (of zero: zero) */
+			l.point = lane / 8 == g ? bit : l.point;
+		}
+	};
+	auto request_listed = [&](Late& l, uint32_t turn) {
+		uint32_t d0 = (turn * 8 + lane % 8) * LATE_EACH;
+		asm volatile("" : "+v"(d0));
+		if (l.point < 64) {
+			const float* src = w.data + late_first + l.point + (size_t)min(d0, w.dim - 1) * w.stride;
+#pragma unroll
+			for (uint32_t q = 0; q < LATE_EACH; ++q) {
+				l.v[q] = *src;
+				src += d0 + q + 1 < w.dim ? w.stride : 0;
+			}
+		}
+	};
+	auto store_listed = [&](const Late& l, uint32_t turn) {
+		uint32_t d0 = (turn * 8 + lane % 8) * LATE_EACH;
+		asm volatile("" : "+v"(d0));
+		if (l.point < 64) {
+			float* to = w.copies + (size_t)(late_first + l.point) * w.copy_stride + d0;
+#pragma unroll
+			for (uint32_t q = 0; q < LATE_EACH; q += LATE_VEC) {
+				typedef float Part __attribute__((ext_vector_type(LATE_VEC)));
+				Part part;
+#pragma unroll
+				for (uint32_t e = 0; e < LATE_VEC; ++e) part[e] = d0 + q + e < w.dim ? l.v[q + e] : 0.0f;
+				if (d0 + q < w.copy_stride) *(Part*)(to + q) = part;
+			}
+		}
+	};
+	auto copy_tiles = [&]() {
+#pragma unroll 1
+		for (uint32_t p = 0; p < P; ++p) {
+			const Rank16Source from = rank16_source<LD, SHARED>(w.data, w.stride, late_first + p * TILE, w.n, lane);
+#pragma unroll 1
+			for (uint32_t kb = 0; kb < KB; ++kb) {
+				float v[8];
+				rank16_request<LD, SHARED, false>(v, from, w.stride, kb, lane, w.dim);
+				rank16_place<LD, SHARED>(v, kb, lane, w.dim);
+				rank16_copy<RANK16_DIRECT>(w, v, late_first + p * TILE, kb, lane, exchange);
+			}
+		}
+		late = 0;
+	};
+	/* copy the listed rows around what fetches the next points */
+	auto copy_listed = [&](auto&& fetch_next) {
+		if constexpr (LISTED) {
+			if (__builtin_popcountll(late) > LATE_MANY) copy_tiles();
+			const bool some = late != 0;
+			Late l;
+			if (some) {
+				late_rows(l);
+				if (LATE_TURNS > 1) {
+					request_listed(l, 1);
+					store_listed(l, 1);
+				}
+				request_listed(l, 0);
+			}
+			fetch_next();
+			if (some) store_listed(l, 0);
+			while (late) {
+				late_rows(l);
+#pragma unroll
+				for (uint32_t turn = 0; turn < LATE_TURNS; ++turn) {
+					request_listed(l, turn);
+					store_listed(l, turn);
+				}
+			}
+		}
+		else fetch_next();
+	};
 	/* A block is converted while the next DEPTH ones are on their way. (Requesting the first of them while the unit before is swept was no gain:
 	 * N = 2M, d = 128, k = 1024: 653 against 618 us, d = 96 440 against 442.) */
 	constexpr int BLOCKS = P * KB, DEPTH = BLOCKS < 8 ? BLOCKS : 8;
@@ -468,7 +564,7 @@ rank16_kernel(const Rank16Args w)
 			__builtin_amdgcn_sched_barrier(0);
 			float (&v)[8] = raw[at % DEPTH];
 			if (!WHOLE) rank16_place<LD, SHARED>(v, kb, lane, dim);
-			if (LD == KMX_SOA) rank16_copy<DIRECT>(w, v, first + p * TILE, kb, lane, exchange);
+			if (LD == KMX_SOA && COPIES != RANK16_LISTED) rank16_copy<COPIES>(w, v, first + p * TILE, kb, lane, exchange);
 			rank16_convert<SHARED>(b[p][kb], v, frame, scale, kb, lane, sums[p], exchange);
 			if (!SHARED) asm volatile("" : "+v"(b[p][kb]));
 			/* the sums exist here: left alone the compiler moves them behind the sweep and keeps the coordinates alive */
@@ -547,6 +643,10 @@ rank16_kernel(const Rank16Args w)
 			if (mine) w.assignment[pt] = idx < w.k ? idx : 0u;
 			const bool flag = mine && !decided;
 			const unsigned long long mask = __ballot(flag);
+			if (LISTED) {
+				late |= (uint64_t)mask << (p * TILE);
+				late_first = first_pt;
+			}
 			if (mask) {
 				const uint32_t add = (uint32_t)__builtin_popcountll(mask);
 				if (flagged + add > list_entries) flush_flags();
@@ -692,7 +792,7 @@ rank16_kernel(const Rank16Args w)
 #pragma unroll
 					for (int kb = 0; kb < KB; ++kb) {
 						rank16_place<LD, SHARED>(raw[p][kb], kb, lane, w.dim);
-						if (LD == KMX_SOA) rank16_copy<DIRECT>(w, raw[p][kb], first + p * TILE, kb, lane, exchange);
+						if (LD == KMX_SOA && COPIES != RANK16_LISTED) rank16_copy<COPIES>(w, raw[p][kb], first + p * TILE, kb, lane, exchange);
 						rank16_convert<SHARED>(b[p][kb], raw[p][kb], frame, scale, kb, lane, sums, exchange);
 					}
 					rank16_total<SHARED>(xx[p], xl[p], sums, lane);
@@ -707,17 +807,18 @@ rank16_kernel(const Rank16Args w)
 				finish(first_point(item));
 				item = next;
 				next = uniform(after);
-				if (item < items) convert(first_point(item));
+				copy_listed([&]() { if (item < items) convert(first_point(item)); });
 			}
 		}
 		else {
 			while (item < items) {
 				const uint32_t after = claim();
-				load_points(first_point(item));
+				copy_listed([&]() { load_points(first_point(item)); });
 				sweep();
 				finish(first_point(item));
 				item = uniform(after);
 			}
+			copy_listed([]() {});
 		}
 	}
 	else {
@@ -796,11 +897,12 @@ rank16_kernel(const Rank16Args w)
 		const uint32_t units = (w.n + WAVES * P * TILE - 1) / (WAVES * P * TILE);
 		for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
 			const uint32_t first = (unit * WAVES + wave) * (P * TILE);
-			load_points(first);
+			copy_listed([&]() { load_points(first); });
 			start();
 			for (uint32_t chunk = 0; chunk < chunks; ++chunk) { next_chunk(); sweep_chunk(chunk); }
 			finish(first);
 		}
+		copy_listed([]() {});
 	}
 	if constexpr (STREAM) staged_but<0>(); /* (nothing may arrive in LDS that is no longer this work-group's) */
 	/* what is left in the lists: one addition per work-group (one per wavefront took 12 us of a launch: 2048 of them to one address) */
@@ -825,23 +927,25 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 {
 	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4, tiles = w.kp / TILE, budget = lds_budget_of(exec, dev);
 	if (budget < rank16_least_bytes(KB, a.layout)) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
-	auto resident = [&](bool direct, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, direct) + rank16_list_bytes(KB, a.layout, entries) <= budget; };
-	const bool direct = KB < 12 && a.layout == KMX_SOA && !resident(false, rank16_list_least(KB)) && resident(true, rank16_list_least(KB));
-	const bool stream_mode = !resident(direct, rank16_list_least(KB));
+	auto resident = [&](Rank16Copies copies, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, copies) + rank16_list_bytes(KB, a.layout, entries) <= budget; };
+	Rank16Copies copies = w.copy_all || a.layout == KMX_AOS ? RANK16_EXCHANGED : RANK16_LISTED;
+	if (KB < 12 && w.copy_all && a.layout == KMX_SOA && !resident(copies, rank16_list_least(KB)) && resident(RANK16_DIRECT, rank16_list_least(KB))) copies = RANK16_DIRECT;
+	const bool stream_mode = !resident(copies, rank16_list_least(KB));
 	w.chunk_tiles = tiles;
 	w.list_entries = RANK16_LIST_MOST;
-	while (!stream_mode && !resident(direct, w.list_entries)) --w.list_entries;
+	while (!stream_mode && !resident(copies, w.list_entries)) --w.list_entries;
 	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, a.layout, w.list_entries);
-	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode, direct);
+	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode, copies);
 	if (stream_mode) {
 		w.chunk_tiles = 1;
 		while (rank16_slots(KB) == 2 && w.chunk_tiles < tiles && static_bytes + 2 * rank16_slot_bytes(KB, w.chunk_tiles + 1) <= budget) ++w.chunk_tiles;
 		lds_bytes = rank16_slots(KB) * rank16_slot_bytes(KB, w.chunk_tiles);
 	}
-	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true, false> : rank16_kernel<KB, KMX_AOS, false, false>)
-	                                                 : (stream_mode ? rank16_kernel<KB, KMX_SOA, true, false> : rank16_kernel<KB, KMX_SOA, false, false>);
+	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true, RANK16_EXCHANGED> : rank16_kernel<KB, KMX_AOS, false, RANK16_EXCHANGED>)
+	                           : copies == RANK16_LISTED ? (stream_mode ? rank16_kernel<KB, KMX_SOA, true, RANK16_LISTED> : rank16_kernel<KB, KMX_SOA, false, RANK16_LISTED>)
+	                                                     : (stream_mode ? rank16_kernel<KB, KMX_SOA, true, RANK16_EXCHANGED> : rank16_kernel<KB, KMX_SOA, false, RANK16_EXCHANGED>);
 	if constexpr (KB < 12)
-		if (direct) kernel = rank16_kernel<KB, KMX_SOA, false, true>;
+		if (copies == RANK16_DIRECT) kernel = rank16_kernel<KB, KMX_SOA, false, RANK16_DIRECT>;
 	const uint32_t waves = rank16_waves(KB, a.layout, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
 	const uint32_t grid = std::min((a.n + unit - 1) / unit, (waves == 4 ? 2 : 1) * dev.compute_units);
 	exec->block_count = grid;

@@ -228,3 +228,32 @@ def test_every_place_of_the_runner_up(km, orc, gpu, dim, k):
     finally:
         km.set_two_level_sweep(1)
     m.free(); out.free()
+
+
+@pytest.mark.parametrize("share", [0.01, 0.12, 0.3, 0.5, 1.0])
+@pytest.mark.parametrize("dim,k,n", [(5, 40, 4099), (17, 40, 4099), (40, 64, 3001), (63, 40, 70003), (90, 64, 3001), (128, 600, 5001), (180, 64, 3001), (250, 200, 5001)])
+def test_listed_rows_of_soa_points_are_copied_behind_the_sweep(km, orc, gpu, dim, k, n, share):
+    """Points halfway between two centroids, which no ranking settles: none, up to eight, more than eight and nearly all of a wavefront's 64."""
+    rng = np.random.default_rng(dim + n + int(100 * share))
+    means = rng.integers(-8, 9, size=(k, dim)).astype(np.float32)
+    near = means[rng.integers(0, k, n)]
+    halfway = rng.random(n) < share
+    rows = np.where(halfway[:, None], (near + means[rng.integers(0, k, n)]) / 2, near + rng.normal(size=(n, dim)).astype(np.float32) * np.float32(0.1)).astype(np.float32)
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, 1))
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 0))
+    a = km.DeviceBuffer(4 * n)
+    km.set_two_level_sweep(2)
+    try:
+        for limit in (1 << 30, 1):
+            a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+            km.set_queued_rows_limit(limit)
+            km.assign(km.ASSIGN_MFMA_BF16X3, d, 1, n, m, 0, dim, a, dim, k, n)
+            km.sync()
+            got = a.read(np.uint32, n)
+            assert np.array_equal(got, want), "%d mismatches" % int((got != want).sum())
+    finally:
+        km.set_two_level_sweep(1)
+        km.set_queued_rows_limit(1 << 30)
+    for b in (d, m, a):
+        b.free()
