@@ -68,9 +68,14 @@ bool takes_cells(const AssignArgs& a, uint32_t lds_budget)
 	return a.dim <= 4 && mode != 0 && (mode == 2 || pays) && cells_support(a, lds_budget);
 }
 
+bool takes_half_sweep(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
+{
+	return bf16_supports(a, lds_budget_of(exec, dev), dev) && takes_rank16(a, lds_budget_of(exec, dev));
+}
+
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
 {
-	return a.layout == KMX_SOA && bf16_supports(a, lds_budget_of(exec, dev), dev) && takes_rank16(a, lds_budget_of(exec, dev)) &&
+	return a.layout == KMX_SOA && takes_half_sweep(a, exec, dev) &&
 	       (size_t)a.n * round_up(a.dim, 8) * sizeof(float) <= queued_rows_limit();
 }
 

@@ -200,6 +200,7 @@ bool takes_cells(const AssignArgs& a, uint32_t lds_budget); /* KMX_ASSIGN_MFMA_B
 bool cells_support(const AssignArgs& a, uint32_t lds_budget);
 int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half, bool choose); /* choose: may leave all points to the packed sweep (WAY_BACK_COUNTER) */
 int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev); /* rank16.hip: all of it */
+bool takes_half_sweep(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST of rows of more than 4 dimensions is the half-precision sweep */
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST would write a.rows_out */
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */
@@ -233,12 +234,14 @@ inline uint32_t lds_budget_of(const kmx_exec_params* exec, const DeviceInfo& dev
 /* means and sizes from the partial sums [chunks][k][dim] and counts [chunks][k] */
 template <typename F>
 int launch_reduce_partials(const F* partial, const uint32_t* partial_counts, uint32_t chunks, F* means, int layout_means, size_t stride_means, uint32_t* sizes, uint32_t dim, uint32_t k, bool divide);
-/* update_sums64.hip: the update of AoS points where the clusters' sums fit LDS as doubles. SUMS64_DONE: means and sizes are finished; SUMS64_OTHERS: not for this
+/* update_sums64.hip: the update where the clusters' sums fit LDS as doubles. SUMS64_DONE: means and sizes are finished; SUMS64_OTHERS: not for this
  * shape; SUMS64_NO_ROOM: a graph is recorded and the partial sums would need a larger work space, so a kernel without any has to do */
 enum Sums64Result { SUMS64_DONE, SUMS64_OTHERS, SUMS64_NO_ROOM };
 template <typename F>
-int launch_update_sums64(const F* data, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
+int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
                          uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, Sums64Result* result);
+/* floats: whether it takes SoA points as they are */
+bool sums64_takes_columns(uint32_t dim, uint32_t k, uint32_t n, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev);
 /* the work space of kmx_update_f32_noalloc on the current device: `partials` is the library's static scratch array */
 int noalloc_workspace(Workspace** ws);
 bool recording_graph(); /* between kmx_graph_begin and kmx_graph_end */

@@ -17,7 +17,8 @@
  *                              with integer LDS atomics, then lane groups walk the sorted list and sum each
  *                              cluster's rows in registers (no atomics at all); per-chunk sums go to a partial
  *                              buffer with plain coalesced stores and reduce_partials_kernel folds them.
- *       update_lds_kernel      fallback for the shapes/layouts the two above do not take (SoA points), and while
+ *                              SoA points: update_columns64_kernel, a lane per point and a request per column.
+ *       update_lds_kernel      fallback for the shapes/layouts the two above do not take, and while
  *                              a graph is recorded and nothing can be allocated: LDS-privatised ds_add_f32.
  *     Points are read exactly once in all three.
  *   reduce_copies_kernel / divide_means_kernel
@@ -797,8 +798,8 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 	const uint32_t budget = exec->shared_mem_bytes ? std::min(exec->shared_mem_bytes, dev.lds_bytes) : dev.lds_bytes;
 
 	Sums64Result sums64 = SUMS64_OTHERS;
-	if (LD == KMX_AOS) {
-		const int rc = launch_update_sums64<float>(u.data, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.n, u.divide, exec, ws, dev, &sums64);
+	{
+		const int rc = launch_update_sums64<float>(u.data, LD, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.n, u.divide, exec, ws, dev, &sums64);
 		if (sums64 == SUMS64_DONE) *state = 2;
 		if (rc || sums64 == SUMS64_DONE) return rc;
 	}
@@ -981,11 +982,11 @@ static int launch_update_t(int variant, const UpdateArgs& u, kmx_exec_params* ex
 }
 
 /*
- * SoA points and the tuned variant: the kernels that read whole rows (sorted chunks, private copies) are 5 to 10 times
+ * SoA points, where update_columns64_kernel does not take them, and the serial-order sums: the kernels that read whole rows are 5 to 10 times
  * faster than anything that adds element by element (measured at N = 2M, d = 32, k = 1024: 0.07 ms against 0.68 ms for the
  * LDS atomics), more than a transposition costs. The points are therefore copied into AoS rows first: tiles of
  * 64 points x 32 dimensions through LDS, reads contiguous along the points, writes contiguous along the dimensions.
- * Rows of fewer than 8 dimensions stay with the element-wise kernel (0.11 ms against 0.15 ms at N = 4M, d = 4, k = 4096).
+ * Rows of fewer than 8 dimensions stay with the element-wise kernel.
  */
 constexpr size_t ROWS_COPY_MAX_BYTES = (size_t)4 << 30; /* larger inputs keep the element-wise kernel */
 
@@ -1074,7 +1075,7 @@ int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Works
 		                                u.dim, u.k, u.n, u.divide, &exec->block_count, dev);
 		return rc ? rc : profile_end(1);
 	}
-	if (update_wants_rows(variant, u, exec, ws, dev)) {
+	if (update_wants_rows(variant, u, exec, ws, dev) && !sums64_takes_columns(u.dim, u.k, u.n, exec, ws, dev)) {
 		const int rc = launch_rows_from_soa(u.data, u.stride, u.dim, u.n, ws, dev);
 		if (rc) return rc;
 		UpdateArgs rows = u;

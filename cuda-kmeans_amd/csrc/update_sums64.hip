@@ -172,6 +172,155 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 	return true;
 }
 
+/* the sum of a row of 16 lanes */
+__device__ __forceinline__ double sums64_of_16(double v)
+{
+	auto turned = [](double x, auto by) -> double { /* row_ror */
+		const int low = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x120 + decltype(by)::value, 0xF, 0xF, true);
+		const int high = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x120 + decltype(by)::value, 0xF, 0xF, true);
+		return __hiloint2double(high, low);
+	};
+	v += turned(v, std::integral_constant<int, 8>{});
+	v += turned(v, std::integral_constant<int, 4>{});
+	v += turned(v, std::integral_constant<int, 2>{});
+	return v + turned(v, std::integral_constant<int, 1>{});
+}
+
+/*
+ * The same for SoA points: a lane takes a point, W columns of 64 points are W requests, and nothing is copied into rows first. Lanes that meet in a column's
+ * sums have any clusters, so a column's sums lie side by side (rows of sums would leave whole banks unused), each in `copies` places for neighbouring
+ * lanes. Points that come sorted by cluster are added up in registers first, 16 at a time: lanes that meet at a sum take turns of 3 cycles each.
+ * What bounds it: memory (N = 8.4M, d = 32, k = 1024 208 us, 5.2 TB/s; AoS 219 on that card) or, from the caches, the conflicts of 64 lanes at random
+ * sums, 26 cycles an addition (N = 2M 72 us). us per update, rows copied first or (d < 8) ds_add_f32 -> this:
+ *   N = 8.4M, d = 32, k = 1024 752 -> 208; N = 250007, d = 50, k = 300 51 -> 22; N = 2M, d = 128, k = 1024 785 -> 212; N = 4M, d = 4, k = 4096 123 -> 29;
+ *   N = 16M, d = 2, k = 2 204 -> 37; N = 1M, d = 64, k = 4000 247 -> 72; N = 2M, d = 32, k = 1024, points sorted by cluster 249 -> 74 (without the sums of 16 355);
+ *   doubles: N = 2M, d = 32, k = 1024 350 -> 131; N = 500000, d = 128, k = 1024 865 -> 116; N = 250000, d = 50, k = 300 143 -> 26.
+ */
+template <int W, typename F>
+__global__ void __launch_bounds__(SUMS64_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+update_columns64_kernel(const F* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment, F* __restrict__ partial, uint32_t* __restrict__ partial_counts,
+                        uint32_t dim, uint32_t k, uint32_t n, uint32_t chunk_points, uint32_t chunks, uint32_t slices, uint32_t copies, uint32_t xcds)
+{
+	constexpr uint32_t SUBS = W >= 8 ? 1 : W >= 4 ? 2 : 4, POINTS = SUBS * WAVE;
+	constexpr int STEPS = sizeof(F) == 8 ? 2 : 3; /* under way */
+	/* W columns of (k + 1) * copies sums (the last ones take what is no cluster's), then as many counts as a column has sums */
+	extern __shared__ __attribute__((aligned(16))) double sums64[];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	/* few slices: those of a chunk, which write to the same lines, on one XCD */
+	const uint32_t at = blockIdx.x / xcds, slice = at % slices, chunk = blockIdx.x % xcds + xcds * (at / slices), column = (k + 1) * copies;
+	if (chunk >= chunks) return;
+	uint32_t* counts = (uint32_t*)(sums64 + W * column);
+	const uint32_t d0 = slice * W, mine = min((uint32_t)W, dim - d0);
+	const uint32_t p_begin = (uint32_t)min((uint64_t)chunk * chunk_points, (uint64_t)n), count = min(chunk_points, n - p_begin);
+	for (uint32_t i = tid; i < W * column; i += SUMS64_THREADS) sums64[i] = 0.0;
+	for (uint32_t i = tid; i < column; i += SUMS64_THREADS) counts[i] = 0u;
+	__syncthreads();
+
+	const char* from[W];
+#pragma unroll
+	for (uint32_t j = 0; j < W; ++j) from[j] = (const char*)(data + (size_t)(d0 + min(j, mine - 1)) * stride + p_begin); /* (behind the row's last column that one again, to sums nobody reads) */
+	const uint32_t* members = assignment + p_begin;
+	const uint32_t steps = (count + POINTS - 1) / POINTS;
+	struct Step { F x[SUBS][W]; uint32_t member[SUBS]; };
+	auto request = [&](Step& s, uint32_t step) {
+#pragma unroll
+		for (uint32_t sub = 0; sub < SUBS; ++sub) {
+			const uint32_t p = step * POINTS + sub * WAVE + lane, inside = min(p, count - 1);
+			s.member[sub] = p < count ? members[p] : k;
+#pragma unroll
+			for (uint32_t j = 0; j < W; ++j) s.x[sub][j] = *(const F*)(from[j] + inside * (uint32_t)sizeof(F));
+		}
+	};
+	auto add = [&](Step& s) {
+#pragma unroll
+		for (uint32_t sub = 0; sub < SUBS; ++sub) {
+			const uint32_t c = min(s.member[sub], k) * copies + lane % copies;
+#pragma unroll
+			for (uint32_t j = 0; j < W; ++j) asm volatile("" : "+v"(s.x[sub][j])); /* (all here before the paths part, so that neither waits for later steps too) */
+			if (slice == 0) atomicAdd(&counts[c], 1u);
+			if (__builtin_amdgcn_ballot_w64(s.member[sub] == sums64_member<16, 0>(s.member[sub])) == ~0ull) {
+				/* 16 neighbours in one cluster, and so all over the wavefront: lanes that meet at a sum would take turns of 3 cycles each */
+#pragma unroll
+				for (uint32_t j = 0; j < W; ++j) {
+					const double sum = sums64_of_16((double)s.x[sub][j]);
+					if (lane % 16 == 0) unsafeAtomicAdd(&sums64[j * column + c], sum);
+				}
+			}
+			else
+#pragma unroll
+				for (uint32_t j = 0; j < W; ++j) unsafeAtomicAdd(&sums64[j * column + c], (double)s.x[sub][j]);
+		}
+	};
+	Step ring[STEPS];
+#pragma unroll
+	for (int i = 0; i < STEPS - 1; ++i)
+		if (wave + SUMS64_WAVES * i < steps) request(ring[i], wave + SUMS64_WAVES * i);
+	for (uint32_t step = wave; step < steps; step += SUMS64_WAVES * STEPS) {
+#pragma unroll
+		for (int i = 0; i < STEPS; ++i) {
+			const uint32_t now = step + SUMS64_WAVES * i, then = now + SUMS64_WAVES * (STEPS - 1);
+			if (then < steps) request(ring[(i + STEPS - 1) % STEPS], then);
+			if (now < steps) add(ring[i]);
+		}
+	}
+	__syncthreads();
+	F* out = partial + (size_t)chunk * k * dim + d0;
+	for (uint32_t i = tid; i < k * W; i += SUMS64_THREADS) {
+		const uint32_t c = i / W, j = i % W;
+		if (j >= mine) continue;
+		const double* sums = sums64 + j * column + c * copies;
+		double sum = sums[0];
+		for (uint32_t q = 1; q < copies; ++q) sum += sums[q];
+		out[(size_t)c * dim + j] = (F)sum;
+	}
+	if (slice == 0)
+		for (uint32_t c = tid; c < k; c += SUMS64_THREADS) {
+			uint32_t size = counts[c * copies];
+			for (uint32_t q = 1; q < copies; ++q) size += counts[c * copies + q];
+			partial_counts[(size_t)chunk * k + c] = size;
+		}
+}
+
+/*
+ * Slices of up to 16 columns, equal as far as they can be. Up to eight of them: as many chunks per XCD as it has compute units for; more: as many chunks as fill
+ * the compute units in one to four rounds (17 slices, 15 chunks). Chunks of as many points as there are clusters at least, as above. Copies while
+ * two points of a wavefront would often meet in one place.
+ */
+constexpr uint32_t COLUMNS64 = 16, COLUMNS64_TOGETHER = 8;
+
+static bool plan_columns64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint32_t budget, uint32_t compute_units, Sums64Plan* plan)
+{
+	if ((uint64_t)(k + 1) * 12 > budget || dim > 8192 || (doubles && n / 200 < k && (uint64_t)k * dim > 8192)) return false;
+	const uint32_t most = std::min<uint32_t>(COLUMNS64, (budget / (k + 1) - 4) / 8), slices = (dim - 1) / most + 1, width = (dim - 1) / slices + 1;
+	const uint32_t bytes = (k + 1) * (8 * width + 4);
+	uint32_t copies = 1, chunks = 0, rounds = 0;
+	while (copies < 32 && copies * k < 256 && 2 * copies * bytes <= std::min<uint32_t>(budget, 64 * 1024)) copies *= 2;
+	if (slices <= COLUMNS64_TOGETHER) chunks = std::max<uint32_t>(1, compute_units / SUMS64_XCDS / slices) * SUMS64_XCDS;
+	else for (uint32_t r = 1; r <= 4; ++r) {
+		const uint32_t fit = compute_units * r / slices;
+		if (fit > 0 && (chunks == 0 || (uint64_t)fit * 20 * rounds > (uint64_t)chunks * 21 * r)) { chunks = fit; rounds = r; }
+	}
+	const uint64_t least_points = std::max<uint64_t>(512, (uint64_t)k * (doubles ? 4 : 1));
+	const uint64_t points = (std::max<uint64_t>(least_points, ((uint64_t)n + std::max(chunks, 1u) - 1) / std::max(chunks, 1u)) + WAVE - 1) / WAVE * WAVE;
+	const uint32_t chunk_points = (uint32_t)std::min<uint64_t>(points, 1u << 28); /* (offsets of 32 bits) */
+	*plan = { width, (dim - 1) / width + 1, copies, (uint32_t)(((uint64_t)n + chunk_points - 1) / chunk_points), chunk_points, copies * bytes };
+	return true;
+}
+
+template <int W, typename F>
+static int launch_columns64(uint32_t width, const F* data, size_t stride, const uint32_t* assignment, F* partial, uint32_t* partial_counts, uint32_t dim, uint32_t k, uint32_t n, const Sums64Plan& p)
+{
+	if constexpr (W > 1)
+		if (width < W) return launch_columns64<W - 1, F>(width, data, stride, assignment, partial, partial_counts, dim, k, n, p);
+	auto kernel = update_columns64_kernel<W, F>;
+	KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds_bytes));
+	const uint32_t xcds = p.slices <= COLUMNS64_TOGETHER ? SUMS64_XCDS : 1;
+	KMX_LAUNCH_KERNEL(kernel, dim3((p.chunks + xcds - 1) / xcds * xcds * p.slices), dim3(SUMS64_THREADS), p.lds_bytes, stream(),
+	                  data, stride, assignment, partial, partial_counts, dim, k, n, p.chunk_points, p.chunks, p.slices, p.copies, xcds);
+	KMX_LAUNCH_CHECK("update_columns64_kernel");
+	return KMX_OK;
+}
+
 template <int LW, bool FULL, typename F>
 static int launch_sums64(const F* data, size_t stride, const uint32_t* assignment, F* partial, uint32_t* partial_counts, uint32_t dim, uint32_t k, uint32_t n, const Sums64Plan& p)
 {
@@ -183,14 +332,25 @@ static int launch_sums64(const F* data, size_t stride, const uint32_t* assignmen
 	return KMX_OK;
 }
 
+static size_t sums64_words(const Sums64Plan& p, uint32_t dim, uint32_t k, size_t item) { return (size_t)p.chunks * k * dim * (item / sizeof(float)) + (size_t)p.chunks * k; }
+
+bool sums64_takes_columns(uint32_t dim, uint32_t k, uint32_t n, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev)
+{
+	Sums64Plan p;
+	return n > 0 && !ws->fixed && plan_columns64(dim, k, n, false, lds_budget_of(exec, dev), dev.compute_units, &p) &&
+	       !(recording_graph() && sums64_words(p, dim, k, sizeof(float)) > ws->partials_cap);
+}
+
 template <typename F>
-int launch_update_sums64(const F* data, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
+int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
                          uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, Sums64Result* result)
 {
 	*result = SUMS64_OTHERS;
 	Sums64Plan p;
-	if (n == 0 || !plan_sums64(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p)) return KMX_OK;
-	const size_t sums = (size_t)p.chunks * k * dim, words = sums * (sizeof(F) / sizeof(float)) + (size_t)p.chunks * k;
+	const bool columns = layout == KMX_SOA;
+	if (n == 0 || (columns && ws->fixed)) return KMX_OK; /* (SoA points are taken there whatever their number of partial sums) */
+	if (!(columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p)) return KMX_OK;
+	const size_t sums = (size_t)p.chunks * k * dim, words = sums64_words(p, dim, k, sizeof(F));
 	if (recording_graph() && words > ws->partials_cap) {
 		*result = SUMS64_NO_ROOM;
 		return KMX_OK;
@@ -203,7 +363,8 @@ int launch_update_sums64(const F* data, size_t stride, const uint32_t* assignmen
 	uint32_t* partial_counts = (uint32_t*)(partial + sums);
 #define KMX_SUMS64(LW) (dim % p.width == 0 && p.width == LW ? launch_sums64<LW, true, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p) \
 	                                                        : launch_sums64<LW, false, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p))
-	rc = p.width <= 1 ? launch_sums64<1, true, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p)
+	if (columns) rc = launch_columns64<COLUMNS64, F>(p.width, data, stride, assignment, partial, partial_counts, dim, k, n, p);
+	else rc = p.width <= 1 ? launch_sums64<1, true, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p)
 	   : p.width <= 2 ? KMX_SUMS64(2) : p.width <= 4 ? KMX_SUMS64(4) : p.width <= 8 ? KMX_SUMS64(8) : p.width <= 16 ? KMX_SUMS64(16)
 	   : p.width <= 32 ? KMX_SUMS64(32) : KMX_SUMS64(64);
 #undef KMX_SUMS64
@@ -211,7 +372,7 @@ int launch_update_sums64(const F* data, size_t stride, const uint32_t* assignmen
 	return launch_reduce_partials<F>(partial, partial_counts, p.chunks, means, layout_means, stride_means, sizes, dim, k, divide);
 }
 
-template int launch_update_sums64<float>(const float*, size_t, const uint32_t*, float*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
-template int launch_update_sums64<double>(const double*, size_t, const uint32_t*, double*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
+template int launch_update_sums64<float>(const float*, int, size_t, const uint32_t*, float*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
+template int launch_update_sums64<double>(const double*, int, size_t, const uint32_t*, double*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
 
 } // namespace kmx

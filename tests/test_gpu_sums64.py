@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 AOS, SOA = 0, 1
 
 
-def check(km, dim, k, n, dtype, stride=None, layout_means=AOS, outside=False, one=False, seed=0):
+def check(km, dim, k, n, dtype, stride=None, layout_means=AOS, outside=False, one=False, seed=0, layout=AOS, by_cluster=False):
     rng = np.random.default_rng(seed + 1000 * dim + k)
     stride = stride or dim
     rows = np.full((n, stride), np.nan, dtype)
@@ -19,12 +19,15 @@ def check(km, dim, k, n, dtype, stride=None, layout_means=AOS, outside=False, on
     if one:
         member[:] = k - 1
     member[-1] = k - 1
-    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    if by_cluster:
+        member.sort()
+    stored = rows if layout == AOS else np.ascontiguousarray(rows[:, :dim].T)
+    d = km.DeviceBuffer(stored.nbytes); d.write(stored.ravel())
     a = km.DeviceBuffer(4 * n); a.write(member)
     stride_means = dim if layout_means == AOS else k
     m = km.DeviceBuffer(rows.itemsize * k * dim); s = km.DeviceBuffer(4 * k)
     m.zero(); s.zero()
-    km.update(km.UPDATE_ATOMIC_SHM, d, AOS, stride, a, m, layout_means, stride_means, s, dim, k, n, None, dtype)
+    km.update(km.UPDATE_ATOMIC_SHM, d, layout, stride if layout == AOS else n, a, m, layout_means, stride_means, s, dim, k, n, None, dtype)
     got = m.read(dtype, k * dim)
     got = got.reshape(k, dim) if layout_means == AOS else got.reshape(dim, k).T
     sizes = s.read(np.uint32, k)
@@ -113,3 +116,13 @@ def test_recorded_without_room_for_partial_sums(km, gpu, dtype):
     g.destroy()
     for b in (d, a, m, s):
         b.free()
+
+
+# columns: one to sixteen at a time, last slices of fewer, sums in up to 32 places, more slices than compute units; points sorted by cluster
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dim,k", [(1, 2), (2, 3), (3, 9), (4, 300), (5, 70), (6, 70), (7, 70), (8, 500), (9, 70), (10, 70), (11, 70), (12, 70), (13, 70), (14, 70), (15, 70), (16, 900),
+                                   (17, 70), (33, 1024), (50, 300), (100, 2500), (4, 4500), (3, 13000), (260, 20), (4200, 3)])
+def test_points_by_columns(km, gpu, dim, k, dtype):
+    for n in (5003, 9001) if dim > 1000 else (20011, 150001):
+        check(km, dim, k, n, dtype, layout=SOA, outside=n == 20011)
+        check(km, dim, k, n, dtype, layout=SOA, layout_means=SOA, by_cluster=True)
