@@ -537,11 +537,11 @@ bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget
 
 /*
  * Up to 128 work-groups of 64 points leave half of the compute units idle: 32 points each (us per iteration, 64 / 32 points: N = 1000, d = 20, k = 128 14.4 / 12.0;
- * N = 5000, d = 32, k = 100 16.5 / 14.5; N = 10240, d = 20, k = 128 16.4 / 16.6: twice the partial sums). Little more than one work-group per compute unit: 16
- * wavefronts each, whose waits for the LDS others cover (eight / 16: N = 10240, d = 20, k = 128 16.4 / 15.2; N = 16384 15.9 / 15.0; N = 20000, k = 100
- * 19.4 / 19.3; N = 32768, d = 8, k = 64 13.6 / 14.6).
+ * N = 5000, d = 32, k = 100 16.5 / 14.5; N = 10240, d = 20, k = 128 16.4 / 16.6: twice the partial sums). One work-group per compute unit at most: 16
+ * wavefronts each, whose waits for the LDS others cover (eight / 16: N = 10240, d = 20, k = 128 16.4 / 15.2; N = 16384 15.9 / 15.0); with two, the waits
+ * are covered already (N = 20000, d = 100, k = 30, SoA 23.3 / 26.7; d = 8, k = 30 12.7 / 15.1; AoS d = 20, k = 100 20.0 / 19.8; N = 32768, d = 8, k = 64 13.6 / 14.6).
  */
-constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 20000;
+constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 256 * SMALL_POINTS;
 
 template <typename F, bool SUMS>
 static int launch_assign_small_t(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
