@@ -73,6 +73,13 @@ __host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { retu
 __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t tiles) { return tiles * kb * WAVE * 16 + rank16_norm_blocks(tiles) * WAVE * 4; }
 /* SoA: which rows go out as AoS, and how (rank16_copy, copy_listed); AoS: EXCHANGED, to nobody */
 enum Rank16Copies { RANK16_EXCHANGED, RANK16_DIRECT, RANK16_LISTED };
+/*
+ * SoA points requested 64 of a column at a time instead of 32 of two columns, from scalar addresses (rank16_request_columns): 128 dimensions, where eight wavefronts
+ * wait for points between streams of centroids, and 256, whose registers hold no vector addresses beside the operands. us per assignment,
+ * N = 2M, d = 128, k = 1024 738 -> 693 (9 % listed 816 -> 782; addresses kept 795); N = 400000, d = 250, k = 130 357 -> 213; N = 262144, d = 256, k = 285 147 -> 133;
+ * but N = 500000, d = 200, k = 1024 330 -> 334; N = 1M, d = 90, k = 300 157 -> 161; d = 40, k = 200 77 -> 81; N = 2M, d = 32, k = 1024 225 -> 230.
+ */
+constexpr bool rank16_whole_columns(uint32_t kb, int layout) { return layout == KMX_SOA && (kb == 8 || kb == 16); }
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
 constexpr uint32_t rank16_exchange(uint32_t kb, int layout, Rank16Copies copies) { return rank16_shared_rows(kb, layout) || (layout == KMX_SOA && copies == RANK16_EXCHANGED) ? RANK16_EXCHANGE : 0; }
@@ -154,6 +161,39 @@ __device__ __forceinline__ void rank16_request(float (&v)[8], const Rank16Source
 			v[j] = *src;
 			src += WHOLE || d0 + j + 1 < dim ? stride : 0;
 		}
+	}
+}
+
+/*
+ * SoA, both tiles of a wavefront's 64 points: lane l requests point l's coordinates j and 8 + j of block kb, 256 consecutive bytes of a column each, from an
+ * address that is the same for all lanes, and the half-waves change places (rank16_halves). `inside`: the lane's point, from the first one on; `column`: the
+ * first point's coordinate 0. FRESH: addresses are formed here and not kept (spilled) from one unit of points to the next.
+ */
+template <bool WHOLE, bool FRESH>
+__device__ __forceinline__ void rank16_request_columns(float (&low)[8], float (&high)[8], const float* column, size_t stride, uint32_t inside, uint32_t kb, uint32_t dim)
+{
+	const uint32_t d0 = kb * KBLOCK;
+	if (FRESH) asm volatile("" : "+s"(stride));
+	const float* at = column + (size_t)(WHOLE ? d0 : min(d0, dim - 1)) * stride;
+#pragma unroll
+	for (uint32_t j = 0; j < 16; ++j) {
+		(j < 8 ? low : high)[j % 8] = *(const float*)((const char*)at + inside * 4u);
+		at += WHOLE || d0 + j + 1 < dim ? stride : 0;
+	}
+}
+/* the requested coordinates as the two tiles' (first tile's to v0), zeros behind the row */
+__device__ __forceinline__ void rank16_halves(float (&v0)[8], float (&v1)[8], uint32_t kb, uint32_t dim)
+{
+	const bool whole = (kb + 1) * KBLOCK <= dim;
+#pragma unroll
+	for (uint32_t j = 0; j < 8; ++j) {
+		if (!whole) {
+			v0[j] = kb * KBLOCK + j < dim ? v0[j] : 0.0f;
+			v1[j] = kb * KBLOCK + 8 + j < dim ? v1[j] : 0.0f;
+		}
+		const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v0[j]), __float_as_uint(v1[j]), false, false);
+		v0[j] = __uint_as_float(r[0]);
+		v1[j] = __uint_as_float(r[1]);
 	}
 }
 
@@ -461,7 +501,7 @@ rank16_kernel(const Rank16Args w)
 	 */
 	constexpr bool LISTED = LD == KMX_SOA && COPIES == RANK16_LISTED;
 	constexpr uint32_t LATE_TURNS = KB > 8 ? 2 : 1, LATE_EACH = KB * KBLOCK / 8 / LATE_TURNS, LATE_VEC = LATE_EACH % 4 == 0 ? 4 : 2, LATE_MANY = 24;
-	static_assert(LATE_EACH % LATE_VEC == 0, "whole stores");
+	static_assert(P == 2 && LATE_EACH % LATE_VEC == 0, "whole stores");
 	uint64_t late = 0;
 	uint32_t late_first = 0;
 	struct Late { float v[LATE_EACH]; uint32_t point; }; /* point: 64 for none */
@@ -547,9 +587,39 @@ rank16_kernel(const Rank16Args w)
 	constexpr int BLOCKS = P * KB, DEPTH = BLOCKS < 8 ? BLOCKS : 8;
 	auto load_points_of = [&](auto whole, uint32_t first, uint32_t dim) {
 		constexpr bool WHOLE = decltype(whole)::value;
+		Rank16Sums sums[P];
+		if constexpr (rank16_whole_columns(KB, LD)) {
+			constexpr int PAIRS = 4; /* blocks of both tiles under way */
+			constexpr bool FRESH = KB == 8;
+			float raw[PAIRS][P][8];
+			const float* column = w.data + rank16_uniform(first);
+			const uint32_t inside = min(lane, w.n - 1 - min(first, w.n - 1));
+#pragma unroll
+			for (int p = 0; p < P; ++p) sums[p] = Rank16Sums{ { 0.0f, 0.0f }, { 0.0f, 0.0f } };
+#pragma unroll
+			for (int kb = 0; kb < PAIRS; ++kb) rank16_request_columns<WHOLE, FRESH>(raw[kb][0], raw[kb][1], column, w.stride, inside, kb, dim);
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb) {
+				__builtin_amdgcn_sched_barrier(0);
+				float (&v)[P][8] = raw[kb % PAIRS];
+				rank16_halves(v[0], v[1], kb, WHOLE ? KB * KBLOCK : dim);
+#pragma unroll
+				for (int p = 0; p < P; ++p) {
+					if (COPIES != RANK16_LISTED) rank16_copy<COPIES>(w, v[p], first + p * TILE, kb, lane, exchange);
+					rank16_convert<SHARED>(b[p][kb], v[p], frame, scale, kb, lane, sums[p], exchange);
+					asm volatile("" : "+v"(b[p][kb]));
+					asm volatile("" : "+v"(sums[p].part[0]), "+v"(sums[p].low[0]));
+				}
+				__builtin_amdgcn_sched_barrier(0);
+				if (kb + PAIRS < KB) rank16_request_columns<WHOLE, FRESH>(raw[kb % PAIRS][0], raw[kb % PAIRS][1], column, w.stride, inside, kb + PAIRS, dim);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int p = 0; p < P; ++p) rank16_total<SHARED>(xx[p], xl[p], sums[p], lane);
+			return;
+		}
 		float raw[DEPTH][8];
 		Rank16Source from[P];
-		Rank16Sums sums[P];
 #pragma unroll
 		for (int p = 0; p < P; ++p) {
 			from[p] = rank16_source<LD, SHARED>(w.data, w.stride, first + p * TILE, w.n, lane);
