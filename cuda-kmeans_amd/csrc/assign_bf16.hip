@@ -40,14 +40,20 @@ namespace kmx {
  *     the exact pass (N = 4M, d = 20, k = 16: 106 -> 141; d = 64, k = 20, N = 1M: 81 -> 67; d = 32, k = 64: 62 -> 51);
  *   - small narrow calls are latency, the same either way (N = 131072, d = 24, k = 128: 24.5 -> 25.5; N = 200k, d = 40, k = 16: 27.5 ->
  *     28.3; N = 65536, d = 20, k = 2000: 62 -> 45; N = 30000, d = 200, k = 512: 81 -> 65);
- *   - SoA points are written out as rows on the way, which many centroids have to pay for (N = 1M, d = 64, k = 64: 116 -> 160;
- *     d = 32, k = 128: 134 -> 82; N = 250k, d = 50, k = 300: 66 -> 55).
+ *   - SoA points, whose listed rows are fetched again: one tile of centroids, or two and narrow rows, are read faster by three products where there are
+ *     many points (N = 1M, d = 64, k = 20: 113 -> 120; N = 2M, d = 40, k = 16: 115 -> 139; N = 4M, d = 20, k = 64: 158 -> 172; d = 30, k = 40: 156 -> 177), the
+ *     rest is not (N = 2M, d = 100, k = 50: 356 -> 249; N = 400000, d = 250, k = 20: 457 -> 221; N = 1M, d = 64, k = 64: 126 -> 109; d = 32, k = 100: 75 -> 65;
+ *     N = 500000, d = 64, k = 20: 74 -> 71; N = 131072, d = 24, k = 100: 32 -> 25).
  */
 static bool rank16_pays(const AssignArgs& a)
 {
-	if (a.layout == KMX_SOA && a.k < 128) return false;
+	const double pairs = (double)a.n * a.k * a.dim;
+	if (a.layout == KMX_SOA) {
+		const bool few = (size_t)a.n * a.dim <= ((size_t)1 << 25); /* points */
+		return a.dim > 32 ? a.dim > 64 || a.k > 32 || few : (a.k >= 96 || (a.k > 32 && few)) && pairs >= 2.5e8;
+	}
 	if (a.dim > 32) return true;
-	return a.k > 32 && (double)a.n * a.k * a.dim >= 5e8;
+	return a.k > 32 && pairs >= 5e8;
 }
 
 static bool takes_rank16(const AssignArgs& a, uint32_t lds_budget)
@@ -68,14 +74,9 @@ bool takes_cells(const AssignArgs& a, uint32_t lds_budget)
 	return a.dim <= 4 && mode != 0 && (mode == 2 || pays) && cells_support(a, lds_budget);
 }
 
-bool takes_half_sweep(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
-{
-	return bf16_supports(a, lds_budget_of(exec, dev), dev) && takes_rank16(a, lds_budget_of(exec, dev));
-}
-
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev)
 {
-	return a.layout == KMX_SOA && takes_half_sweep(a, exec, dev) &&
+	return a.layout == KMX_SOA && bf16_supports(a, lds_budget_of(exec, dev), dev) && takes_rank16(a, lds_budget_of(exec, dev)) &&
 	       (size_t)a.n * round_up(a.dim, 8) * sizeof(float) <= queued_rows_limit();
 }
 

@@ -200,7 +200,6 @@ bool takes_cells(const AssignArgs& a, uint32_t lds_budget); /* KMX_ASSIGN_MFMA_B
 bool cells_support(const AssignArgs& a, uint32_t lds_budget);
 int launch_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, const Cells16& half, bool choose); /* choose: may leave all points to the packed sweep (WAY_BACK_COUNTER) */
 int launch_assign_cells(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev); /* rank16.hip: all of it */
-bool takes_half_sweep(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST of rows of more than 4 dimensions is the half-precision sweep */
 bool sweep_writes_rows(const AssignArgs& a, const kmx_exec_params* exec, const DeviceInfo& dev); /* KMX_ASSIGN_BEST would write a.rows_out */
 int launch_assign_rank16(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* assign_wide.hip: rows of more than 256 dimensions (the split-bf16 variant's launcher passes them on) */

@@ -269,18 +269,18 @@ static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_
 }
 
 /*
- * Assignment and update of SoA points. Where both read columns as they are, they do (us per iteration, all rows written by the sweep -> columns: N = 250007, d = 50,
- * k = 300 75 -> 67; N = 2M, d = 32, k = 1024 316 -> 293; N = 2M, d = 128, k = 1024 1016 -> 936; N = 4M, d = 60, k = 100 1203 -> 581).
- * Otherwise the update reads whole rows: from the half-precision sweep, which has them in its hands, or copied first, for the assignment to read as well.
- * The other sweeps are slower on columns than that copy takes (N = 40000, d = 250, k = 100 107 instead of 82), and so is the one of rows of more than
- * 256 dimensions where columns begin inside a line, or few points make it (rows first -> columns: N = 100000, d = 500, k = 400 327 -> 222,
+ * Assignment and update of SoA points. Both read columns as they are (us per iteration, all rows written by the sweep, or copied ahead of it -> columns: N = 250007,
+ * d = 50, k = 300 75 -> 67; N = 2M, d = 32, k = 1024 316 -> 293; N = 2M, d = 128, k = 1024 1016 -> 936; N = 2M, d = 100, k = 50 1060 -> 400; N = 1M, d = 5,
+ * k = 100 159 -> 59), unless the update has no kernel for them: then it reads whole rows, from the half-precision sweep, which has them in its hands, or copied
+ * first, for the assignment to read as well. So it does where the sweep of more than 256 dimensions would read columns that begin inside a line,
+ * or few points (rows first -> columns: N = 100000, d = 500, k = 400 327 -> 222,
  * d = 300, k = 2000 377 -> 318; N = 131071, d = 512, k = 40 350 -> 355; N = 20000, d = 400, k = 1000 125 -> 136).
  */
 constexpr size_t WIDE_COLUMNS_FLOATS = (size_t)1 << 24;
 static int launch_two_passes_soa(AssignArgs a, UpdateArgs u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	AosRows rows = { nullptr, 0 };
-	const bool reads_columns = u.dim > 256 ? u.stride % 32 == 0 && (size_t)u.n * u.dim >= WIDE_COLUMNS_FLOATS : takes_half_sweep(a, exec, dev);
+	const bool reads_columns = u.dim <= 256 || (u.stride % 32 == 0 && (size_t)u.n * u.dim >= WIDE_COLUMNS_FLOATS);
 	const bool columns = reads_columns && sums64_takes_columns(u.dim, u.k, u.n, exec, ws, dev);
 	if (!columns && update_wants_rows(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev)) {
 		if (sweep_writes_rows(a, exec, dev)) a.rows_out = &rows;

@@ -257,3 +257,9 @@ def test_listed_rows_of_soa_points_are_copied_behind_the_sweep(km, orc, gpu, dim
         km.set_queued_rows_limit(1 << 30)
     for b in (d, m, a):
         b.free()
+
+
+@pytest.mark.parametrize("dim,k,n", [(5, 100, 300001), (7, 500, 40003), (100, 2, 70001), (250, 20, 33001), (60, 20, 40003), (40, 33, 70001), (24, 96, 131072), (64, 20, 530001), (300, 33, 60000)])
+def test_iterations_on_soa_points_with_few_centroids(km, orc, gpu, dim, k, n):
+    """Both sides of the line between the sweeps, and the update of columns behind each of them."""
+    test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, 1)
