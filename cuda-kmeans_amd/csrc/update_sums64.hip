@@ -321,6 +321,253 @@ static int launch_columns64(uint32_t width, const F* data, size_t stride, const 
 	return KMX_OK;
 }
 
+/*
+ * Rows of more coordinates than slices are worth it: a work-group takes the clusters c = range (modulo `ranges`, a power of two) of its part of the points, up to 256
+ * of their coordinates. A wavefront looks through the memberships of its share, lists the points that are the work-group's, and then reads their rows, four
+ * coordinates per lane, eight rows under way while eight are added.
+ * A compute unit reads 50 GB/s at most, twice what all of them together get from memory: a range with many points has to have many work-groups. Each
+ * work-group counts the ranges in the same sample of the memberships (16384 of them, 16 at a place) and finds from that which range it
+ * has and which part of the points (in equal parts, N = 1M, d = 256, k = 1024: 190 us on equal clusters, 758 an iteration on normal ones, 1246 with all points
+ * in one; now 202, 741, 230). What bounds it: memory, 1.07 GB in 188 us of the kernel's 193 (5.6 TB/s), then the fold, 6.
+ */
+constexpr uint32_t RANGES64_LIST = 384, RANGES64_SCAN = 4 * WAVE, RANGES64_ROWS = 8; /* entries of a wavefront's list; points looked at together; rows of a step */
+constexpr uint32_t RANGES64_MOST = 32, RANGES64_SAMPLES = 16;                         /* ranges; places of the sample per 16 lanes */
+typedef float f32x4_row __attribute__((ext_vector_type(4), aligned(4)));
+
+/* partial: [work-group of a slice][its clusters][dim], partial_counts: [work-group][its clusters], starts: a range's first work-group, then their number */
+__global__ void __launch_bounds__(SUMS64_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+update_ranges64_kernel(const float* __restrict__ data, size_t stride, const uint32_t* __restrict__ assignment, float* __restrict__ partial, uint32_t* __restrict__ partial_counts,
+                       uint32_t* __restrict__ starts, uint32_t dim, uint32_t k, uint32_t n, uint32_t groups, uint32_t log_ranges, uint32_t width)
+{
+	/* per cluster of the range four times width / 4 sums (a lane's coordinates lie in each of them), a row more for what fills up a step; counts; lists */
+	extern __shared__ __attribute__((aligned(16))) double sums64[];
+	__shared__ uint32_t in_range[RANGES64_MOST], begin[RANGES64_MOST + 1];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
+	const uint32_t ranges = 1u << log_ranges, most = (k + ranges - 1) >> log_ranges;
+	const uint32_t me = blockIdx.x % groups, slice = blockIdx.x / groups, d0 = slice * width, lanes = min(width, dim - d0) / 4, row = width; /* (whole pieces of four) */
+	uint32_t* counts = (uint32_t*)(sums64 + (most + 1) * row);
+	uint32_t* lists = counts + most;
+	uint32_t* list = lists + wave * (RANGES64_LIST + RANGES64_ROWS);
+	{
+		uint32_t sample[RANGES64_SAMPLES];
+		constexpr uint32_t PLACES = SUMS64_THREADS / 16 * RANGES64_SAMPLES;
+		const bool all = n <= PLACES * 16;
+		const uint32_t whole = (n - min(n, 16u)) / PLACES, rest = (n - min(n, 16u)) % PLACES; /* (n <= 2^24, 2^10 places) */
+#pragma unroll
+		for (uint32_t i = 0; i < RANGES64_SAMPLES; ++i) {
+			const uint32_t place = i * (SUMS64_THREADS / 16) + tid / 16, p = (all ? place * 16 : place * whole + place * rest / PLACES) + tid % 16;
+			sample[i] = p < n ? assignment[p] : ~0u;
+		}
+		for (uint32_t i = tid; i < (most + 1) * row; i += SUMS64_THREADS) sums64[i] = 0.0;
+		for (uint32_t i = tid; i < most; i += SUMS64_THREADS) counts[i] = 0u;
+		for (uint32_t i = tid; i < ranges * WAVE; i += SUMS64_THREADS) lists[i] = 0u; /* a range's points by the lane that saw them */
+		__syncthreads();
+#pragma unroll
+		for (uint32_t i = 0; i < RANGES64_SAMPLES; ++i)
+			if (sample[i] < k) atomicAdd(&lists[(sample[i] & (ranges - 1)) * WAVE + lane], 1u);
+		__syncthreads();
+		for (uint32_t r = wave; r < ranges; r += SUMS64_WAVES) {
+			uint32_t seen = lists[r * WAVE + lane];
+			for (int off = WAVE / 2; off > 0; off >>= 1) seen += (uint32_t)__shfl_xor((int)seen, off);
+			if (lane == 0) in_range[r] = seen;
+		}
+		__syncthreads();
+	}
+	if (wave == 0) {
+		const uint32_t seen = lane < ranges ? in_range[lane] : 0;
+		uint32_t total = seen;
+		for (int off = WAVE / 2; off > 0; off >>= 1) total += (uint32_t)__shfl_xor((int)total, off);
+		/* one work-group each, the others in proportion, those that the rounding leaves to the first ranges */
+		uint32_t share = lane < ranges ? 1 + (uint32_t)((uint64_t)(groups - ranges) * seen / max(total, 1u)) : 0, given = share;
+		for (int off = WAVE / 2; off > 0; off >>= 1) given += (uint32_t)__shfl_xor((int)given, off);
+		const uint32_t left = groups - given;
+		if (lane < ranges) share += left / ranges + (lane < left % ranges ? 1 : 0);
+		uint32_t up_to = share;
+		for (int off = 1; off < WAVE; off <<= 1) {
+			const uint32_t up = (uint32_t)__shfl_up((int)up_to, off);
+			if (lane >= (uint32_t)off) up_to += up;
+		}
+		if (lane < ranges) begin[lane + 1] = up_to;
+		if (lane == 0) begin[0] = 0;
+	}
+	__syncthreads();
+	if (blockIdx.x == 0 && tid <= ranges) starts[tid] = begin[tid];
+	uint32_t range = 0;
+	while (range + 1 < ranges && begin[range + 1] <= me) ++range;
+	const uint32_t parts = begin[range + 1] - begin[range], part = me - begin[range];
+	const uint32_t p_begin = (uint32_t)((uint64_t)part * n / parts), count = (uint32_t)((uint64_t)(part + 1) * n / parts) - p_begin;
+
+	const uint32_t* members = assignment + p_begin;
+	const uint32_t piece = min(lane, lanes - 1);
+	const char* rows = (const char*)(data + (size_t)p_begin * stride + d0) + piece * 16;
+	const bool lane_on = lane < lanes;
+	const uint32_t sums_at = piece * 8;
+	const uint32_t scans = (count + RANGES64_SCAN - 1) / RANGES64_SCAN;
+	uint32_t scan = wave;
+	while (scan < scans) {
+		uint32_t listed = 0;
+		bool room = true;
+		while (room && scan < scans) {
+			uint32_t member[2][4];
+#pragma unroll
+			for (uint32_t s = 0; s < 2; ++s)
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q) {
+					const uint32_t p = (scan + s * SUMS64_WAVES) * RANGES64_SCAN + q * WAVE + lane;
+					member[s][q] = p < count ? members[p] : ~0u;
+				}
+#pragma unroll
+			for (uint32_t s = 0; s < 2; ++s) {
+				room = room && listed + RANGES64_SCAN <= RANGES64_LIST;
+				if (!room) continue;
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q) {
+					const bool mine = member[s][q] < k && (member[s][q] & (ranges - 1)) == range;
+					const unsigned long long mask = __builtin_amdgcn_ballot_w64(mine);
+					if (mine) {
+						const uint32_t c = member[s][q] >> log_ranges;
+						if (slice == 0) atomicAdd(&counts[c], 1u);
+						list[listed + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = c << 24 | (scan * RANGES64_SCAN + q * WAVE + lane);
+					}
+					listed += (uint32_t)__popcll(mask);
+				}
+				scan += SUMS64_WAVES;
+			}
+		}
+		if (listed == 0) continue;
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		const uint32_t last = list[listed - 1] & 0xFFFFFFu;
+		if (lane < RANGES64_ROWS) list[listed + lane] = most << 24 | last; /* the last step's rows beyond the list */
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		struct Step { f32x4_row x[RANGES64_ROWS]; uint32_t to[RANGES64_ROWS]; };
+		auto request = [&](Step& s, uint32_t first) {
+#pragma unroll
+			for (uint32_t u = 0; u < RANGES64_ROWS; ++u) {
+				const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[first + u]);
+				s.to[u] = e >> 24;
+				s.x[u] = *(const f32x4_row*)(rows + (size_t)(e & 0xFFFFFFu) * stride * sizeof(float));
+			}
+		};
+		auto add = [&](Step& s) {
+#pragma unroll
+			for (uint32_t u = 0; u < RANGES64_ROWS; ++u) {
+				char* to = (char*)sums64 + s.to[u] * (row * 8) + sums_at;
+				if (lane_on) {
+#pragma unroll
+					for (uint32_t e = 0; e < 4; ++e) unsafeAtomicAdd((double*)(to + e * (row * 2)), (double)s.x[u][e]);
+				}
+			}
+		};
+		Step a, b;
+		request(a, 0);
+		for (uint32_t first = 0; first < listed; first += 2 * RANGES64_ROWS) {
+			request(b, min(first + RANGES64_ROWS, listed));
+			add(a);
+			request(a, min(first + 2 * RANGES64_ROWS, listed));
+			add(b);
+		}
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+	}
+	__syncthreads();
+	float* out = partial + (size_t)me * most * dim + d0 + piece * 4;
+	for (uint32_t i = wave; i < most; i += SUMS64_WAVES) {
+		const double* sums = sums64 + i * row + piece;
+		if (lane_on) *(f32x4_row*)(out + (size_t)i * dim) = f32x4_row{ (float)sums[0], (float)sums[row / 4], (float)sums[row / 2], (float)sums[row / 4 * 3] };
+	}
+	if (slice == 0)
+		for (uint32_t i = tid; i < most; i += SUMS64_THREADS) partial_counts[(size_t)me * most + i] = counts[i];
+}
+
+/* means and sizes from what update_ranges64_kernel left: a work-group per cluster, four wavefronts share out its range's work-groups */
+template <int LM>
+__global__ void __launch_bounds__(4 * WAVE)
+fold_ranges64_kernel(const float* __restrict__ partial, const uint32_t* __restrict__ partial_counts, const uint32_t* __restrict__ starts, float* __restrict__ means, size_t stride_means,
+                     uint32_t* __restrict__ sizes, uint32_t dim, uint32_t k, uint32_t log_ranges, uint32_t divide)
+{
+	__shared__ double part[4][4][WAVE];
+	const uint32_t c = blockIdx.x, lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, ranges = 1u << log_ranges, most = (k + ranges - 1) >> log_ranges;
+	const uint32_t first = starts[c & (ranges - 1)], last = starts[(c & (ranges - 1)) + 1], local = c >> log_ranges;
+	uint32_t size = 0;
+	for (uint32_t g = first + lane; g < last; g += WAVE) size += partial_counts[(size_t)g * most + local];
+	for (int off = WAVE / 2; off > 0; off >>= 1) size += (uint32_t)__shfl_xor((int)size, off);
+	if (threadIdx.x == 0) sizes[c] = size;
+	for (uint32_t q0 = 0; q0 < dim / 4; q0 += WAVE) {
+		const uint32_t q = min(q0 + lane, dim / 4 - 1);
+		double sum[4] = { 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll 4
+		for (uint32_t g = first + wave; g < last; g += 4) {
+			const f32x4_row v = *(const f32x4_row*)(partial + ((size_t)g * most + local) * dim + q * 4);
+#pragma unroll
+			for (uint32_t e = 0; e < 4; ++e) sum[e] += (double)v[e];
+		}
+#pragma unroll
+		for (uint32_t e = 0; e < 4; ++e) part[wave][e][lane] = sum[e];
+		__syncthreads();
+		/* wavefront `wave` has coordinate `wave` of the lanes' four */
+		const float total = (float)(part[0][wave][lane] + part[1][wave][lane] + part[2][wave][lane] + part[3][wave][lane]);
+		if (q0 + lane < dim / 4) means[elem<LM>(stride_means, c, q * 4 + wave)] = !divide ? total : size ? total / (float)size : 0.0f;
+		__syncthreads();
+	}
+}
+
+/*
+ * Where ranges beat the sorted chunks (update.hip) or slices of 16 coordinates (us per update, those -> ranges; the sample and the fold cost 8 us). Up to 256
+ * dimensions from 25 million floats on: N = 1M, d = 256, k = 1024 234 -> 202; d = 192 191 -> 162; N = 500000, d = 200, k = 1000 104 -> 92; d = 224, k = 2000 135 -> 113;
+ * N = 100000, d = 256, k = 1000 34.7 -> 33.4, but d = 200, k = 600 28 -> 31. More: from 600 clusters on, whose partial sums the sorted chunks
+ * write in 32 copies and more: N = 100000, d = 300, k = 2000 71 -> 45; N = 131071, d = 512, k = 1000 79 -> 60, k = 600 65 -> 58, k = 400 57 -> 59. Half of the points in
+ * one cluster, N = 1M, d = 256, k = 1024 448 -> 216; all of them 702 -> 230; sorted by cluster 292 -> 225. Slices of 16: N = 1M, d = 160, k = 600 128.7 -> 128.3,
+ * N = 300000, d = 144, k = 1000 37.6 -> 40.7: stay.
+ */
+static bool ranges64_pays(uint32_t dim, uint32_t k, uint32_t n, bool planned)
+{
+	return !planned && (dim <= 256 ? (size_t)n * dim >= (3u << 23) : k >= 600);
+}
+
+struct Ranges64Plan { uint32_t width, slices, log_ranges, groups, lds_bytes; };
+
+static size_t ranges64_words(const Ranges64Plan& p, uint32_t dim, uint32_t k)
+{
+	const size_t rows = (size_t)p.groups * (((size_t)k + (1u << p.log_ranges) - 1) >> p.log_ranges);
+	return rows * (dim + 1) + RANGES64_MOST + 1;
+}
+
+static bool plan_ranges64(uint32_t dim, uint32_t k, uint32_t n, uint32_t budget, uint32_t compute_units, Ranges64Plan* plan)
+{
+	if (dim % 4 != 0 || dim <= 128 || dim > 1024 || n > (1u << 24)) return false; /* (numbers of points of 24 bits) */
+	const uint32_t slices = (dim - 1) / 256 + 1, width = ((dim - 1) / slices + 4) / 4 * 4;
+	const uint32_t tables = (2 * RANGES64_MOST + 1) * 4 + 64;
+	static_assert(SUMS64_WAVES * (RANGES64_LIST + RANGES64_ROWS) >= RANGES64_MOST * WAVE, "the sample's counts lie in the lists");
+	for (uint32_t log_ranges = 0; (1u << log_ranges) <= RANGES64_MOST; ++log_ranges) {
+		const uint32_t ranges = 1u << log_ranges, most = (k + ranges - 1) >> log_ranges;
+		const uint64_t bytes = ((uint64_t)most + 1) * width * 8 + (uint64_t)most * 4 + SUMS64_WAVES * (RANGES64_LIST + RANGES64_ROWS) * 4;
+		if (most > 255 || bytes + tables > budget) continue; /* (clusters of eight bits) */
+		const uint64_t wanted = (uint64_t)ranges * std::max<uint64_t>(1, n / std::max<uint32_t>(k, 512));
+		const uint32_t groups = (uint32_t)std::min<uint64_t>(wanted, compute_units / slices);
+		if (groups < ranges) return false;
+		*plan = { width, slices, log_ranges, groups, (uint32_t)bytes };
+		return true;
+	}
+	return false;
+}
+
+static int launch_ranges64(const float* data, size_t stride, const uint32_t* assignment, float* means, int layout_means, size_t stride_means, uint32_t* sizes,
+                           uint32_t dim, uint32_t k, uint32_t n, bool divide, const Ranges64Plan& p, Workspace* ws)
+{
+	const size_t rows = (size_t)p.groups * ((k + (1u << p.log_ranges) - 1) >> p.log_ranges);
+	uint32_t* counts = (uint32_t*)(ws->partials + rows * dim);
+	KMX_HIP(hipFuncSetAttribute((const void*)update_ranges64_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds_bytes));
+	KMX_LAUNCH_KERNEL(update_ranges64_kernel, dim3(p.groups * p.slices), dim3(SUMS64_THREADS), p.lds_bytes, stream(),
+	                  data, stride, assignment, ws->partials, counts, counts + rows, dim, k, n, p.groups, p.log_ranges, p.width);
+	KMX_LAUNCH_CHECK("update_ranges64_kernel");
+	auto fold = layout_means == KMX_AOS ? fold_ranges64_kernel<KMX_AOS> : fold_ranges64_kernel<KMX_SOA>;
+	KMX_LAUNCH_KERNEL(fold, dim3(k), dim3(4 * WAVE), 0, stream(), ws->partials, counts, counts + rows, means, stride_means, sizes, dim, k, p.log_ranges, divide ? 1u : 0u);
+	KMX_LAUNCH_CHECK("fold_ranges64_kernel");
+	return KMX_OK;
+}
+
 template <int LW, bool FULL, typename F>
 static int launch_sums64(const F* data, size_t stride, const uint32_t* assignment, F* partial, uint32_t* partial_counts, uint32_t dim, uint32_t k, uint32_t n, const Sums64Plan& p)
 {
@@ -349,7 +596,23 @@ int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_
 	Sums64Plan p;
 	const bool columns = layout == KMX_SOA;
 	if (n == 0 || (columns && ws->fixed)) return KMX_OK; /* (SoA points are taken there whatever their number of partial sums) */
-	if (!(columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p)) return KMX_OK;
+	const bool planned = (columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p);
+	if constexpr (sizeof(F) == 4) {
+		Ranges64Plan r;
+		if (!columns && ranges64_pays(dim, k, n, planned) && plan_ranges64(dim, k, n, lds_budget_of(exec, dev), dev.compute_units, &r)) {
+			const size_t words = ranges64_words(r, dim, k);
+			if (recording_graph() && words > ws->partials_cap) {
+				*result = SUMS64_NO_ROOM;
+				return KMX_OK;
+			}
+			const int rc = reserve_partials(ws, words);
+			if (rc) return rc;
+			*result = SUMS64_DONE;
+			exec->block_count = r.groups * r.slices;
+			return launch_ranges64(data, stride, assignment, means, layout_means, stride_means, sizes, dim, k, n, divide, r, ws);
+		}
+	}
+	if (!planned) return KMX_OK;
 	const size_t sums = (size_t)p.chunks * k * dim, words = sums64_words(p, dim, k, sizeof(F));
 	if (recording_graph() && words > ws->partials_cap) {
 		*result = SUMS64_NO_ROOM;

@@ -126,3 +126,12 @@ def test_points_by_columns(km, gpu, dim, k, dtype):
     for n in (5003, 9001) if dim > 1000 else (20011, 150001):
         check(km, dim, k, n, dtype, layout=SOA, outside=n == 20011)
         check(km, dim, k, n, dtype, layout=SOA, layout_means=SOA, by_cluster=True)
+
+
+# ranges of clusters: two to 32 of them, one and more slices of up to 256 coordinates, ranges without points or with nearly all
+@pytest.mark.parametrize("dim,k,n", [(260, 700, 20011), (300, 600, 9001), (512, 2000, 20011), (1024, 601, 5003), (516, 640, 1501), (768, 1500, 16385), (200, 610, 126001)])
+def test_ranges_of_clusters(km, gpu, dim, k, n):
+    check(km, dim, k, n, np.float32, outside=True, stride=dim + 3)
+    check(km, dim, k, n, np.float32, one=True, layout_means=SOA)
+    if dim > 256:
+        check(km, dim, k, n, np.float32, by_cluster=True)
