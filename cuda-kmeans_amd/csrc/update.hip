@@ -6,26 +6,26 @@
  *   update_fine_kernel    - one lane per (point, dim) element, global atomics
  *                           (counterpart of updateAtomicFineKernel, reference kernels.cu:770-791)
  *   KMX_UPDATE_ATOMIC_SHM - the tuned variant (counterpart of updateAtomicShmKernel, reference
- *                           kernels.cu:817-858), three kernels chosen by shape. Measured on gfx950: an LDS
+ *                           kernels.cu:817-858), kernels chosen by shape. Measured on gfx950: an LDS
  *                           ds_add_f32 costs ~194 cycles per wavefront instruction whatever the address
  *                           pattern (lanes are serialised), ds_add_u32 4.4 cycles, ds_add_f64 8.2 on rows of
  *                           16 sums, a plain LDS read-add-write 8.2.
  *       update_sums64_kernel   (update_sums64.hip) wherever the clusters' sums fit LDS as doubles, in slices of
  *                              the coordinates if need be: every coordinate one ds_add_f64, the points read in
- *                              the order they lie in.
- *       update_sorted_kernel   larger k * dim: the work-group counting-sorts its chunk of points by cluster
+ *                              the order they lie in (SoA: update_columns64_kernel).
+ *       update_ranges64_kernel (there too) wide rows: a work-group has a range of clusters and reads the rows of its points.
+ *       update_sorted_kernel   the rest: the work-group counting-sorts its chunk of points by cluster
  *                              with integer LDS atomics, then lane groups walk the sorted list and sum each
  *                              cluster's rows in registers (no atomics at all); per-chunk sums go to a partial
  *                              buffer with plain coalesced stores and reduce_partials_kernel folds them.
- *                              SoA points: update_columns64_kernel, a lane per point and a request per column.
- *       update_lds_kernel      fallback for the shapes/layouts the two above do not take, and while
+ *       update_lds_kernel      fallback for the shapes/layouts the others do not take, and while
  *                              a graph is recorded and nothing can be allocated: LDS-privatised ds_add_f32.
- *     Points are read exactly once in all three.
+ *     Points are read exactly once in all of them.
  *   reduce_copies_kernel / divide_means_kernel
  *                         - counterparts of reducePrivCopiesKernel / divideMeansKernel
  *                           (reference kernels.cu:115-135,149-163); empty clusters keep their zero.
  *
- * Partial sums are fp32 and their order differs from the serial order, exactly as in the reference's GPU path
+ * Partial sums are handed over as fp32 and their order differs from the serial order, exactly as in the reference's GPU path
  * (atomics); counts are integers and exact.
  */
 #include "kmx_internal.h"
