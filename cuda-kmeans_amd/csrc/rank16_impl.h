@@ -13,13 +13,17 @@ namespace kmx {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
+/* SoA: which rows go out as AoS, and how (rank16_copy, copy_listed); AoS: EXCHANGED, to nobody */
+enum Rank16Copies { RANK16_EXCHANGED, RANK16_DIRECT, RANK16_LISTED };
+
 /*
  * Rows of up to 32 dimensions around resident centroids: three wavefronts on a SIMD, of which the third also covers the ends of the others'
  * sweeps. That takes tracking in fewer registers (RANK16_GROUPS). us per assignment (N = 2M, Gaussian mixture, centroids after two rounds), two wavefronts with
  * the snapshot -> three: d = 32, k = 1024 219 -> 204; d = 16 174 -> 150; d = 10, k = 100 74 -> 70. The same tracking with two: 220, 165, 78. Wider rows
- * would spill (N = 1M, d = 64, k = 512: 103 -> 114), and so does the copying of SoA points (d = 24, k = 256: 68.6 -> 69.6).
+ * would spill (N = 1M, d = 64, k = 512: 103 -> 114), and so does the copying of
+ * all SoA points (d = 24, k = 256: 68.6 -> 69.6); of the listed ones only (SoA, d = 32, k = 1024 225 -> 215, around its first points 246 -> 230; N = 1M, d = 20, k = 300 70 -> 68).
  */
-constexpr bool rank16_grouped(uint32_t kb, int layout) { return kb == 1 || (kb == 2 && layout == KMX_AOS); }
+constexpr bool rank16_grouped(uint32_t kb, int layout, Rank16Copies copies) { return kb == 1 || (kb == 2 && (layout == KMX_AOS || copies == RANK16_LISTED)); }
 /*
  * Wavefronts of a work-group: otherwise eight around centroids in LDS. Where the centroids stream by (slots of a chunk of tiles that go round, filled by
  * requests straight to LDS, a barrier per chunk), rows of up to 128 dimensions keep that form with two chunks as large as fit, since the
@@ -29,7 +33,7 @@ constexpr bool rank16_grouped(uint32_t kb, int layout) { return kb == 1 || (kb =
  * the matrix cores, and four slots of a tile (N = 1M, d = 256, k = 1024: 549, with eight wavefronts and two chunks of four tiles 569).
  * With chunks through registers and eight wavefronts for all widths: 656, 655, 480, 464.
  */
-constexpr uint32_t rank16_waves(uint32_t kb, int layout, bool stream) { return stream && kb >= 12 ? 4 : !stream && rank16_grouped(kb, layout) ? 12 : 8; }
+constexpr uint32_t rank16_waves(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return stream && kb >= 12 ? 4 : !stream && rank16_grouped(kb, layout, copies) ? 12 : 8; }
 constexpr int RANK16_P = 2; /* point tiles per wavefront: an operand read serves two instructions */
 
 struct Rank16Args {
@@ -71,8 +75,6 @@ constexpr uint32_t rank16_slots(uint32_t kb) { return kb >= 12 ? 4 : 2; }
 __host__ __device__ constexpr uint32_t rank16_norm_blocks(uint32_t tiles) { return (tiles * NORM_TILE + WAVE - 1) / WAVE; }
 /* what a chunk takes in LDS, its norms behind its operands as whole requests of 64 words */
 __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t tiles) { return tiles * kb * WAVE * 16 + rank16_norm_blocks(tiles) * WAVE * 4; }
-/* SoA: which rows go out as AoS, and how (rank16_copy, copy_listed); AoS: EXCHANGED, to nobody */
-enum Rank16Copies { RANK16_EXCHANGED, RANK16_DIRECT, RANK16_LISTED };
 /*
  * SoA points requested 64 of a column at a time instead of 32 of two columns, from scalar addresses (rank16_request_columns): 128 dimensions, where eight wavefronts
  * wait for points between streams of centroids, and 256, whose registers hold no vector addresses beside the operands. us per assignment,
@@ -83,9 +85,9 @@ constexpr bool rank16_whole_columns(uint32_t kb, int layout) { return layout == 
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
 constexpr uint32_t rank16_exchange(uint32_t kb, int layout, Rank16Copies copies) { return rank16_shared_rows(kb, layout) || (layout == KMX_SOA && copies == RANK16_EXCHANGED) ? RANK16_EXCHANGE : 0; }
-constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, copies) + 4) * rank16_waves(kb, layout, stream) + kb * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, copies) + 4) * rank16_waves(kb, layout, stream, copies) + kb * KBLOCK) * 4 + 64; }
 /* the lists of a work-group around resident centroids, lying behind them */
-constexpr uint32_t rank16_list_bytes(uint32_t kb, int layout, uint32_t entries) { return rank16_waves(kb, layout, false) * entries * 8; }
+constexpr uint32_t rank16_list_bytes(uint32_t kb, int layout, Rank16Copies copies, uint32_t entries) { return rank16_waves(kb, layout, false, copies) * entries * 8; }
 constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true, RANK16_EXCHANGED) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
@@ -406,15 +408,15 @@ __device__ __forceinline__ float rank16_both(float v)
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
 template <int KB, int LD, bool STREAM, Rank16Copies COPIES>
-__global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM) * WAVE, rank16_waves(KB, LD, STREAM) == 12 ? 3 : 2)
+__global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM, COPIES) * WAVE, rank16_waves(KB, LD, STREAM, COPIES) == 12 ? 3 : 2)
 rank16_kernel(const Rank16Args w)
 {
-	constexpr uint32_t WAVES = rank16_waves(KB, LD, STREAM), THREADS = WAVES * WAVE;
+	constexpr uint32_t WAVES = rank16_waves(KB, LD, STREAM, COPIES), THREADS = WAVES * WAVE;
 	constexpr int P = RANK16_P;
 	constexpr uint32_t TF = rank16_tile_floats<KB>();
 	constexpr bool PIPE = !STREAM && KB <= 4;
 	constexpr bool SHARED = rank16_shared_rows(KB, LD);
-	constexpr bool GROUPED = PIPE && rank16_grouped(KB, LD);
+	constexpr bool GROUPED = PIPE && rank16_grouped(KB, LD, COPIES);
 	constexpr bool PREFETCH = PIPE && (KB == 1 || (KB == 2 && !GROUPED)); /* the next item's coordinates travel while the current one is swept */
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
@@ -997,14 +999,14 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 {
 	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4, tiles = w.kp / TILE, budget = lds_budget_of(exec, dev);
 	if (budget < rank16_least_bytes(KB, a.layout)) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
-	auto resident = [&](Rank16Copies copies, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, copies) + rank16_list_bytes(KB, a.layout, entries) <= budget; };
+	auto resident = [&](Rank16Copies copies, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, copies) + rank16_list_bytes(KB, a.layout, copies, entries) <= budget; };
 	Rank16Copies copies = w.copy_all || a.layout == KMX_AOS ? RANK16_EXCHANGED : RANK16_LISTED;
 	if (KB < 12 && w.copy_all && a.layout == KMX_SOA && !resident(copies, rank16_list_least(KB)) && resident(RANK16_DIRECT, rank16_list_least(KB))) copies = RANK16_DIRECT;
 	const bool stream_mode = !resident(copies, rank16_list_least(KB));
 	w.chunk_tiles = tiles;
 	w.list_entries = RANK16_LIST_MOST;
 	while (!stream_mode && !resident(copies, w.list_entries)) --w.list_entries;
-	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, a.layout, w.list_entries);
+	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, a.layout, copies, w.list_entries);
 	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode, copies);
 	if (stream_mode) {
 		w.chunk_tiles = 1;
@@ -1016,7 +1018,7 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 	                                                     : (stream_mode ? rank16_kernel<KB, KMX_SOA, true, RANK16_EXCHANGED> : rank16_kernel<KB, KMX_SOA, false, RANK16_EXCHANGED>);
 	if constexpr (KB < 12)
 		if (copies == RANK16_DIRECT) kernel = rank16_kernel<KB, KMX_SOA, false, RANK16_DIRECT>;
-	const uint32_t waves = rank16_waves(KB, a.layout, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
+	const uint32_t waves = rank16_waves(KB, a.layout, stream_mode, copies), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
 	const uint32_t grid = std::min((a.n + unit - 1) / unit, (waves == 4 ? 2 : 1) * dev.compute_units);
 	exec->block_count = grid;
 #define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (half-precision sweep): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u, chunk tiles %u, LDS %u)", \
@@ -1024,7 +1026,7 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 	if (!sizing_only()) {
 		KMX_PLAN(w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1 && KB * KBLOCK >= a.dim);
 		KMX_PLAN(w.chunk_tiles >= 1 && (uint64_t)lds_bytes + static_bytes <= dev.lds_bytes && rank16_tile_floats<KB>() % 4 == 0);
-		KMX_PLAN(stream_mode || (w.list_entries >= RANK16_P * TILE / 2 && rank16_waves(KB, a.layout, false) * 2 * w.list_entries + tiles * (tile_bytes / 4) <= lds_bytes / 4));
+		KMX_PLAN(stream_mode || (w.list_entries >= RANK16_P * TILE / 2 && rank16_waves(KB, a.layout, false, copies) * 2 * w.list_entries + tiles * (tile_bytes / 4) <= lds_bytes / 4));
 		KMX_PLAN(ws->packed16 && (size_t)tiles * KB * WAVE * 4 <= ws->packed16_cap);
 		KMX_PLAN(!stream_mode || ((rank16_slots(KB) == 2 || w.chunk_tiles == 1) && /* whole requests of norms, the last chunk's too */
 		                          (size_t)(tiles - 1) / w.chunk_tiles * w.chunk_tiles * NORM_TILE + rank16_norm_blocks(w.chunk_tiles) * WAVE <= ws->norms16_cap));
