@@ -985,29 +985,46 @@ static int launch_update_t(int variant, const UpdateArgs& u, kmx_exec_params* ex
  * SoA points, where update_columns64_kernel does not take them, and the serial-order sums: the kernels that read whole rows are 5 to 10 times
  * faster than anything that adds element by element (measured at N = 2M, d = 32, k = 1024: 0.07 ms against 0.68 ms for the
  * LDS atomics), more than a transposition costs. The points are therefore copied into AoS rows first: tiles of
- * 64 points x 32 dimensions through LDS, reads contiguous along the points, writes contiguous along the dimensions.
+ * 64 points x 32 dimensions through LDS, reads contiguous along the points, writes contiguous along the dimensions. A wavefront has a tile of its own: 32
+ * requests under way per lane, 16 bytes a store, and nobody waits at a barrier (iterations, a work-group per tile -> this: N = 131071, d = 512, k = 40
+ * 342 -> 320 us; N = 99999, d = 500, k = 400 301 -> 273; bound by memory, as many bytes written as read).
  * Rows of fewer than 8 dimensions stay with the element-wise kernel.
  */
 constexpr size_t ROWS_COPY_MAX_BYTES = (size_t)4 << 30; /* larger inputs keep the element-wise kernel */
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(4 * WAVE)
 rows_from_soa_kernel(const float* __restrict__ data, size_t stride, float* __restrict__ rows, uint32_t dim, uint32_t n)
 {
-	__shared__ float tile[32][65];
+	__shared__ float tiles_of[4][32][65];
+	const uint32_t lane = threadIdx.x % WAVE, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+	float (&tile)[32][65] = tiles_of[wave];
 	const uint32_t tiles_q = (dim + 31) / 32;
 	const size_t tiles = (size_t)((n + 63) / 64) * tiles_q;
-	for (size_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-		const uint32_t p0 = (uint32_t)(t / tiles_q) * 64, q0 = (uint32_t)(t % tiles_q) * 32;
-		__syncthreads(); /* the previous tile has been written out */
-		for (uint32_t q = threadIdx.x / 64; q < 32; q += 4) {
-			const uint32_t p = threadIdx.x % 64;
-			if (q0 + q < dim && p0 + p < n) tile[q][p] = data[(size_t)(q0 + q) * stride + p0 + p];
+	for (size_t t = (size_t)blockIdx.x * 4 + wave; t < tiles; t += (size_t)gridDim.x * 4) {
+		const uint32_t p0 = (uint32_t)(t / tiles_q) * 64, q0 = (uint32_t)(t % tiles_q) * 32, columns = min(32u, dim - q0);
+		const float* src = data + (size_t)q0 * stride + min(p0 + lane, n - 1);
+		float v[32];
+#pragma unroll
+		for (uint32_t q = 0; q < 32; ++q) v[q] = src[(size_t)min(q, columns - 1) * stride];
+#pragma unroll
+		for (uint32_t q = 0; q < 32; ++q) tile[q][lane] = v[q];
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		float* out = rows + (size_t)p0 * dim + q0;
+		if (dim % 4 == 0) {
+			const uint32_t q = lane % 8 * 4;
+#pragma unroll
+			for (uint32_t p = lane / 8; p < 64; p += 8)
+				if (q < columns && p0 + p < n) *(f32x4*)(out + (size_t)p * dim + q) = f32x4{ tile[q][p], tile[q + 1][p], tile[q + 2][p], tile[q + 3][p] };
 		}
-		__syncthreads();
-		for (uint32_t p = threadIdx.x / 32; p < 64; p += 8) {
-			const uint32_t q = threadIdx.x % 32;
-			if (q0 + q < dim && p0 + p < n) rows[(size_t)(p0 + p) * dim + q0 + q] = tile[q][p];
+		else {
+			const uint32_t q = lane % 32;
+#pragma unroll 8
+			for (uint32_t p = lane / 32; p < 64; p += 2)
+				if (q < columns && p0 + p < n) out[(size_t)p * dim + q] = tile[q][p];
 		}
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
 	}
 }
 
@@ -1057,7 +1074,7 @@ int launch_rows_from_soa(const float* data, size_t stride, uint32_t dim, uint32_
 	int rc = reserve_rows_copy(ws, (size_t)n * dim);
 	if (rc) return rc;
 	const size_t tiles = (size_t)((n + 63) / 64) * ((dim + 31) / 32);
-	KMX_LAUNCH_KERNEL(rows_from_soa_kernel, dim3((uint32_t)std::min<size_t>(tiles, (size_t)dev.compute_units * 32)), dim3(256), 0, stream(),
+	KMX_LAUNCH_KERNEL(rows_from_soa_kernel, dim3((uint32_t)std::min<size_t>((tiles + 3) / 4, (size_t)dev.compute_units * 16)), dim3(4 * WAVE), 0, stream(),
 	                   data, stride, ws->rows_copy, dim, n);
 	KMX_LAUNCH_CHECK("rows_from_soa_kernel");
 	return KMX_OK;
