@@ -274,13 +274,14 @@ static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_
  * k = 100 159 -> 59), unless the update has no kernel for them: then it reads whole rows, from the half-precision sweep, which has them in its hands, or copied
  * first, for the assignment to read as well. So it does where the sweep of more than 256 dimensions would read columns that begin inside a line,
  * or few points (rows first -> columns: N = 100000, d = 500, k = 400 327 -> 222,
- * d = 300, k = 2000 377 -> 318; N = 131071, d = 512, k = 40 350 -> 355; N = 20000, d = 400, k = 1000 125 -> 136).
+ * d = 300, k = 2000 377 -> 318; N = 131071, d = 512, k = 40 320 -> 355; N = 99999, d = 500, k = 400 273 -> 301; N = 20000, d = 400, k = 1000 120 -> 136).
  */
 constexpr size_t WIDE_COLUMNS_FLOATS = (size_t)1 << 24;
 static int launch_two_passes_soa(AssignArgs a, UpdateArgs u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	AosRows rows = { nullptr, 0 };
-	const bool reads_columns = u.dim <= 256 || (u.stride % 32 == 0 && (size_t)u.n * u.dim >= WIDE_COLUMNS_FLOATS);
+	const bool no_room = recording_graph() && (size_t)u.n * u.dim > ws->rows_copy_cap; /* (the room was made for columns without a stride of their own) */
+	const bool reads_columns = u.dim <= 256 || no_room || (u.stride % 32 == 0 && (size_t)u.n * u.dim >= WIDE_COLUMNS_FLOATS);
 	const bool columns = reads_columns && sums64_takes_columns(u.dim, u.k, u.n, exec, ws, dev);
 	if (!columns && update_wants_rows(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev)) {
 		if (sweep_writes_rows(a, exec, dev)) a.rows_out = &rows;

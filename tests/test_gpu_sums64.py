@@ -135,3 +135,37 @@ def test_ranges_of_clusters(km, gpu, dim, k, n):
     check(km, dim, k, n, np.float32, one=True, layout_means=SOA)
     if dim > 256:
         check(km, dim, k, n, np.float32, by_cluster=True)
+
+
+@pytest.mark.parametrize("dim,k,n,layout,pad", [(300, 600, 60032, SOA, 5), (50, 300, 40000, SOA, 5), (260, 600, 20000, AOS, 0)])
+def test_recorded_iterations_in_reserved_room(km, orc, gpu, dim, k, n, layout, pad):
+    """The room is sized for columns without a stride of their own; padded columns, which copy rows first otherwise, have to do with it."""
+    rng = np.random.default_rng(dim + n)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    cents = rows[rng.choice(n, k, replace=False)].copy()
+    stride = dim if layout == AOS else n + pad
+    stored = rows
+    if layout == SOA:
+        stored = np.full((dim, stride), np.nan, np.float32)
+        stored[:, :n] = rows.T
+    d = km.DeviceBuffer(stored.nbytes); d.write(stored.ravel())
+    m = km.DeviceBuffer(4 * k * dim); m.write(cents.ravel())
+    a = km.DeviceBuffer(4 * n); out = km.DeviceBuffer(4 * k * dim); sizes = km.DeviceBuffer(4 * k)
+    want = orc.assign(rows.ravel(), cents.ravel(), dim, k, n, threads=0, fast=True)
+    counts = np.bincount(want, minlength=k)
+    sums = np.zeros((k, dim)); np.add.at(sums, want, rows.astype(np.float64))
+    km.sync()
+    km.check(km.hip_lib().kmx_shutdown())
+    km.reserve(km.ASSIGN_BEST, km.UPDATE_ATOMIC_SHM, layout, AOS, dim, k, n)
+    with km.Graph() as g:
+        km.iteration(d, layout, stride, m, out, AOS, dim, a, sizes, dim, k, n)
+    for _ in range(3):
+        a.write(np.full(n, 0xFFFFFFF1, np.uint32)); out.write(np.full(k * dim, np.nan, np.float32)); sizes.write(np.full(k, 7, np.uint32))
+        g.launch()
+        km.sync()
+        assert np.array_equal(a.read(np.uint32, n), want)
+        assert np.array_equal(sizes.read(np.uint32, k), counts)
+        assert np.allclose(out.read(np.float32, k * dim).reshape(k, dim), sums / counts[:, None], rtol=1e-5, atol=1e-6)
+    g.destroy()
+    for b in (d, m, a, out, sizes):
+        b.free()
