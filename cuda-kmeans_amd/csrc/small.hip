@@ -521,17 +521,17 @@ constexpr uint32_t SMALL_FEW_CENTROIDS = 12; /* up to here a tile of one point t
  * compute unit, so fewer than 256 of them leave units idle. Us per iteration near the line, these kernels / the general path: N = 40000, d = 32, k = 100
  * (effort 504 million) 28.7 / 40.3; N = 32768, d = 32, k = 128 (528) 27.1 / 31.5; N = 65536, d = 16, k = 100 (511) 27.2 / 32.0; N = 50000, d = 16, k = 128 (499)
  * 29.9 / 28.3; N = 65536, d = 8, k = 200 (708) 33.8 / 29.3. Wider rows, per assignment: N = 65536, d = 64, k = 50 (727) 20.4 / 22.6; N = 40000, d = 64, k = 80
- * (710) 20.2 / 21.7; N = 20000, d = 64, k = 200 (888) 32.1 / 22.7. Twice that for doubles.
+ * (710) 20.2 / 21.7; N = 20000, d = 64, k = 200 (888) 32.1 / 22.7. Doubles: twice 450 million.
  * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
  */
 constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
-constexpr uint64_t SMALL_EFFORT = 530000000;
+constexpr uint64_t SMALL_EFFORT = 530000000, SMALL_EFFORT_DOUBLES = 450000000; /* (doubles, N = 56478, d = 56, k = 128, 475: 87 us per iteration, general path 54) */
 template <typename F>
 bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
 	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
 	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
-	const uint64_t limit = SMALL_EFFORT * (dim > 32 ? 3 : 2) / 2 * (sizeof(F) / 4);
+	const uint64_t limit = (sizeof(F) == 8 ? 2 * SMALL_EFFORT_DOUBLES : SMALL_EFFORT) * (dim > 32 ? 3 : 2) / 2;
 	return effort <= limit && assign_small_lds<F>(dim, k, SMALL_POINTS, false) + assign_small_static<F>() <= lds_budget;
 }
 

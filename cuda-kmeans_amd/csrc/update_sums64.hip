@@ -135,7 +135,8 @@ update_sums64_kernel(const F* __restrict__ data, size_t stride, const uint32_t* 
  * A chunk has as many points as there are clusters, 512 at least: its sums are written and read once more (N = 200000, d = 4, k = 4000: 256 chunks 17 us, 50
  * 14, sorted chunks 31; N = 50000, d = 32, k = 1000: 17, 14, 16); where that leaves compute units over and a slice is wide, more slices (N = 100000, d = 32,
  * k = 500: one slice 16, two 13). Sums of doubles are twice as dear: four times as many points, and few points are left to the kernels that add to the means
- * where they lie (N = 400000, d = 32, k = 1000 33.2, those 34.2; N = 100000, k = 500 17.4, 17.1; N = 200000, d = 4, k = 4000 19.0, 16.2).
+ * where they lie (N = 400000, d = 32, k = 1000 33.2, those 34.2; N = 100000, k = 500 17.4, 17.1; N = 200000, d = 4, k = 4000 19.0, 16.2;
+ * rows of one slice of 16: N = 225824, d = 11, k = 1105 23.9, 15.1; k = 700 18.5, 16.7; N = 500000, k = 1105 24.9, 27.9; d = 8 15.7, 18.5).
  * Few clusters: the rows of a request mostly meet at the same sums, which costs an LDS cycle each; copies of them, as many as rows (N = 16M, d = 2,
  * k = 2: 90 us without, 34 with).
  */
@@ -148,6 +149,7 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 	auto slices_of = [&](uint32_t width) -> uint32_t { return (dim - 1) / width + 1; };
 	auto chunks_of = [&](uint32_t width) -> uint32_t { return std::max<uint32_t>(1, compute_units / SUMS64_XCDS / slices_of(width)) * SUMS64_XCDS; };
 	if (dim > SUMS64_SLICES * SUMS64_LANES || (doubles && n / 200 < k && (uint64_t)k * dim > 8192)) return false;
+	if (doubles && dim <= 16 && dim != 8 && n / 400 < k && (uint64_t)k * dim > 6144) return false; /* (one slice: as many work-groups as chunks) */
 	const uint64_t least_points = std::max<uint64_t>(512, (uint64_t)k * (doubles ? 4 : 1));
 	/* doubles whose sums do not fit as a whole */
 	const bool parts = doubles && bytes(dim) > budget, eights = parts && dim <= 56 && dim % 4 == 0 && dim % 16 != 0;
