@@ -137,6 +137,8 @@ update_sums64_kernel(const F* __restrict__ data, size_t stride, const uint32_t* 
  * k = 500: one slice 16, two 13). Sums of doubles are twice as dear: four times as many points, and few points are left to the kernels that add to the means
  * where they lie (N = 400000, d = 32, k = 1000 33.2, those 34.2; N = 100000, k = 500 17.4, 17.1; N = 200000, d = 4, k = 4000 19.0, 16.2;
  * rows of one slice of 16: N = 225824, d = 11, k = 1105 23.9, 15.1; k = 700 18.5, 16.7; N = 500000, k = 1105 24.9, 27.9; d = 8 15.7, 18.5).
+ * Unaligned slices of a middling number of points: N = 100000, d = 100, k = 500 26.1, sorted chunks 21.9; N = 143310, d = 160, k = 354 31.5, 27.1; but N = 300000, d = 148 42.4,
+ * 45.5; N = 30000, d = 140, k = 300 13.0, 16.6; N = 100000, d = 200, k = 100 22.8, 24.3.
  * Few clusters: the rows of a request mostly meet at the same sums, which costs an LDS cycle each; copies of them, as many as rows (N = 16M, d = 2,
  * k = 2: 90 us without, 34 with).
  */
@@ -165,6 +167,8 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 		width = w;
 	}
 	if (width == 0) return false;
+	/* three slices and more that begin inside a line, and sums to write that are a fifth of what is read: the sorted chunks, while the points lie in the caches */
+	if (!doubles && width > 32 && width % 16 != 0 && slices_of(width) >= 3 && k >= 300 && (uint64_t)n * dim >= (1u << 23) && (uint64_t)n * dim < (1u << 25)) return false;
 	uint32_t lanes = 1, copies = 1;
 	while (lanes < width) lanes *= 2;
 	while (copies * 2 <= WAVE / lanes && 2 * copies * bytes(width) <= std::min<uint32_t>(budget, 48 * 1024)) copies *= 2;
@@ -516,16 +520,16 @@ fold_ranges64_kernel(const float* __restrict__ partial, const uint32_t* __restri
 }
 
 /*
- * Where ranges beat the sorted chunks (update.hip) or slices of 16 coordinates (us per update, those -> ranges; the sample and the fold cost 8 us). Up to 256
- * dimensions from 25 million floats on: N = 1M, d = 256, k = 1024 234 -> 202; d = 192 191 -> 162; N = 500000, d = 200, k = 1000 104 -> 92; d = 224, k = 2000 135 -> 113;
- * N = 100000, d = 256, k = 1000 34.7 -> 33.4, but d = 200, k = 600 28 -> 31. More: from 600 clusters on, whose partial sums the sorted chunks
- * write in 32 copies and more: N = 100000, d = 300, k = 2000 71 -> 45; N = 131071, d = 512, k = 1000 79 -> 60, k = 600 65 -> 58, k = 400 57 -> 59. Half of the points in
+ * Where ranges beat the sorted chunks (update.hip) or slices of 16 coordinates (us per update, those -> ranges; the sample and the fold cost 8 us): from 600 clusters on.
+ * Up to 256 dimensions from 25 million floats on: N = 1M, d = 256, k = 1024 234 -> 202; d = 192 191 -> 162; N = 500000, d = 200, k = 1000 104 -> 92; d = 224, k = 2000 135 -> 113;
+ * N = 100000, d = 256, k = 1000 34.7 -> 33.4, but d = 200, k = 600 28 -> 31; N = 190000, d = 148, k = 354 34 -> 37. More,
+ * of whose clusters the sorted chunks write 32 sets of partial sums and more: N = 100000, d = 300, k = 2000 71 -> 45; N = 131071, d = 512, k = 1000 79 -> 60, k = 600 65 -> 58, k = 400 57 -> 59. Half of the points in
  * one cluster, N = 1M, d = 256, k = 1024 448 -> 216; all of them 702 -> 230; sorted by cluster 292 -> 225. Slices of 16: N = 1M, d = 160, k = 600 128.7 -> 128.3,
  * N = 300000, d = 144, k = 1000 37.6 -> 40.7: stay.
  */
 static bool ranges64_pays(uint32_t dim, uint32_t k, uint32_t n, bool planned)
 {
-	return !planned && (dim <= 256 ? (size_t)n * dim >= (3u << 23) : k >= 600);
+	return !planned && k >= 600 && (dim > 256 || (size_t)n * dim >= (3u << 23));
 }
 
 struct Ranges64Plan { uint32_t width, slices, log_ranges, groups, lds_bytes; };
