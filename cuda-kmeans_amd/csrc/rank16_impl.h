@@ -7,6 +7,7 @@
 #define KMX_RANK16_IMPL_H
 
 #include "assign_bf16_impl.h"
+#include "rank16_columns.h"
 
 namespace kmx {
 
@@ -168,8 +169,8 @@ __device__ __forceinline__ void rank16_request(float (&v)[8], const Rank16Source
 
 /*
  * SoA, both tiles of a wavefront's 64 points: lane l requests point l's coordinates j and 8 + j of block kb, 256 consecutive bytes of a column each, from an
- * address that is the same for all lanes, and the half-waves change places (rank16_halves). `inside`: the lane's point, from the first one on; `column`: the
- * first point's coordinate 0. FRESH: addresses are formed here and not kept (spilled) from one unit of points to the next.
+ * address that is the same for all lanes, and the half-waves change places (rank16_halves). `inside`: the lane's point, from rank16_column_base on; `column`: that
+ * point's coordinate 0. FRESH: addresses are formed here and not kept (spilled) from one unit of points to the next.
  */
 template <bool WHOLE, bool FRESH>
 __device__ __forceinline__ void rank16_request_columns(float (&low)[8], float (&high)[8], const float* column, size_t stride, uint32_t inside, uint32_t kb, uint32_t dim)
@@ -594,8 +595,8 @@ rank16_kernel(const Rank16Args w)
 			constexpr int PAIRS = 4; /* blocks of both tiles under way */
 			constexpr bool FRESH = KB == 8;
 			float raw[PAIRS][P][8];
-			const float* column = w.data + rank16_uniform(first);
-			const uint32_t inside = min(lane, w.n - 1 - min(first, w.n - 1));
+			const uint32_t base = rank16_column_base(rank16_uniform(first), w.n), inside = rank16_column_inside(base, lane, w.n);
+			const float* column = w.data + base;
 #pragma unroll
 			for (int p = 0; p < P; ++p) sums[p] = Rank16Sums{ { 0.0f, 0.0f }, { 0.0f, 0.0f } };
 #pragma unroll

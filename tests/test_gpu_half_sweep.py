@@ -263,3 +263,10 @@ def test_listed_rows_of_soa_points_are_copied_behind_the_sweep(km, orc, gpu, dim
 def test_iterations_on_soa_points_with_few_centroids(km, orc, gpu, dim, k, n):
     """Both sides of the line between the sweeps, and the update of columns behind each of them."""
     test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, 1)
+
+
+@pytest.mark.parametrize("dim,k", [(97, 40), (128, 600), (200, 40), (250, 600)])
+@pytest.mark.parametrize("n", [65, 192, 520, 577, 5001, 33281])
+def test_columns_read_by_wavefronts_without_points(km, orc, gpu, dim, k, n):
+    """Numbers of points that leave one to seven wavefronts of the last unit without any, centroids in LDS and streamed: those read the last point again."""
+    test_listed_rows_of_soa_points_are_copied_behind_the_sweep(km, orc, gpu, dim, k, n, 0.12)
