@@ -1295,7 +1295,7 @@ extern "C" int kmx_assign_f64(int variant,
 		Workspace* ws = nullptr;
 		if ((rc = workspace(&ws))) return rc;
 		if ((rc = profile_begin(0))) return rc;
-		rc = launch_assign_small<double>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, ws->counters, &exec->block_count, *dev);
+		rc = launch_assign_small<double>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, ws->counters, &exec->block_count, lds_budget_of(exec, *dev));
 		return rc ? rc : profile_end(0);
 	}
 	const bool float_ranking = variant == KMX_ASSIGN_MFMA || variant == KMX_ASSIGN_MFMA_BF16X3 || variant == KMX_ASSIGN_BEST;

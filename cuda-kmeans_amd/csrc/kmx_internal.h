@@ -213,16 +213,16 @@ int launch_assign_lds_fma(const AssignArgs& a, kmx_exec_params* exec, Workspace*
 /* small.hip: small inputs in one launch each (assignment, update), floats and doubles */
 template <typename F> bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget);
 template <typename F> bool small_update_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget, const DeviceInfo& dev);
+/* lds_budget: the one that small_assign_fits or small_iteration_fits was asked with */
 template <typename F>
 int launch_assign_small(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
-                        uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, uint32_t* blocks, const DeviceInfo& dev);
+                        uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, uint32_t* blocks, uint32_t lds_budget);
 template <typename F>
 int launch_update_small(const F* data, int layout, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
                         uint32_t dim, uint32_t k, uint32_t n, bool divide, uint32_t* blocks, const DeviceInfo& dev);
 /* the assignment of small inputs that also adds its points up: partial sums and counts of *blocks work-groups (at most
- * assign_small_max_blocks(n)), for launch_reduce_partials */
-int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, const DeviceInfo& dev);
-uint32_t assign_small_max_blocks(uint32_t n);
+ * assign_small_max_blocks(n), small_plan.h), for launch_reduce_partials */
+int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, uint32_t lds_budget);
 bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget);
 inline uint32_t lds_budget_of(const kmx_exec_params* exec, const DeviceInfo& dev)
 {

@@ -4,6 +4,7 @@
  */
 #include "kmx_internal.h"
 #include "certificate.h"
+#include "small_plan.h"
 
 #include <cstdarg>
 #include <cstring>
@@ -201,7 +202,7 @@ int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Wor
 		int rc = profile_begin(0);
 		if (rc) return rc;
 		rc = launch_assign_small<float>(a.data, a.layout, a.stride, a.means, a.layout_means, a.stride_means, a.assignment, a.dim, a.k, a.n,
-		                                ws->counters, &exec->block_count, dev);
+		                                ws->counters, &exec->block_count, lds_budget_of(exec, dev));
 		return rc ? rc : profile_end(0);
 	}
 	if (variant == KMX_ASSIGN_BEST) {
@@ -263,7 +264,7 @@ static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_
 	g_last_assign_variant = KMX_ASSIGN_BASE;
 	uint32_t* partial_counts = (uint32_t*)(ws->partials + most * elements);
 	if ((rc = profile_begin(0))) return rc;
-	if ((rc = launch_assign_small_sums(a, ws->partials, partial_counts, &exec->block_count, ws->counters, dev))) return rc;
+	if ((rc = launch_assign_small_sums(a, ws->partials, partial_counts, &exec->block_count, ws->counters, lds_budget_of(exec, dev)))) return rc;
 	if ((rc = profile_end(0))) return rc;
 	return launch_reduce_partials<float>(ws->partials, partial_counts, exec->block_count, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.divide);
 }

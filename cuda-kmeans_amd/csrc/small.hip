@@ -12,6 +12,7 @@
  * Where the general paths take over is measured; see small_assign_fits and small_update_fits.
  */
 #include "kmx_internal.h"
+#include "small_plan.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -19,9 +20,6 @@
 #pragma clang fp contract(off)
 
 namespace kmx {
-
-constexpr uint32_t SMALL_THREADS = 512;
-constexpr uint32_t SMALL_WAVES = SMALL_THREADS / WAVE;
 
 template <typename F> struct SmallVec;
 template <> struct SmallVec<float> { typedef float type __attribute__((ext_vector_type(4))); };
@@ -64,7 +62,7 @@ template <> struct SqrtMargin<float> { static constexpr float ratio = 0.9999995f
 template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e-15, tiny = 1e-290; };
 
 /*
- * A work-group owns 64 points (or 32, see SMALL_HALF_POINTS), whose rows it stages in LDS next to a chunk of the centroids. A wavefront is 16 x 4 lanes with
+ * A work-group owns 64 points (or 32, see small_shape), whose rows it stages in LDS next to a chunk of the centroids. A wavefront is 16 x 4 lanes with
  * T points times T centroids each, so it covers 16 T points and 4 T centroids at a time; of 64 points, the eight wavefronts are 4 / T groups of
  * points times 2 T shares of the centroids. Per four dimensions a lane reads 2 T pieces of 16 bytes for its T^2 pairs: with T = 2
  * (192 ALU cycles against 128 of the LDS that four SIMDs share) the vector ALU sets the pace, T = 1 (48 against 64) is for a
@@ -82,8 +80,6 @@ template <> struct SqrtMargin<double> { static constexpr double ratio = 1.0 - 1e
  * times rows on the fp32 matrix instruction, which keeps the vector ALU, took 2.1 instead of 0.5 us of a work-group: N = 10240, d = 20, k = 128 17.7 -> 16.4 us per
  * iteration, N = 65536, d = 8, k = 64 20.5 -> 18.4, N = 20000, d = 20, k = 100 22.3 -> 19.4).
  */
-constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading the memberships again (update_small_kernel) is cheaper than as many partial sums */
-constexpr uint32_t SMALL_POINTS = WAVE;
 
 /*
  * `count` rows of dim elements on their way to LDS rows of row_stride: AoS rows `stride` apart, or columns (row r of column q at src[q * stride + r];
@@ -227,12 +223,13 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
                     uint32_t magic, uint32_t vec4, uint32_t* __restrict__ counters, F* __restrict__ partial, uint32_t* __restrict__ partial_counts)
 {
 	typedef typename SmallVec<F>::type F4;
-	constexpr uint32_t WAVES = THREADS / WAVE, PG = POINTS / 16 / T, CW = WAVES / PG; /* groups of points, shares of the centroids */
+	constexpr uint32_t PG = POINTS / 16 / T, CW = small_shares(T, POINTS, THREADS); /* groups of points, shares of the centroids */
 	extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
 	F* rows = (F*)lds_raw;
 	F* cents = rows + (size_t)POINTS * row_stride; /* chunk rows; with SUMS later k * dim doubles and k counts */
 	__shared__ SmallKey<F> cand[CW][POINTS];
 	__shared__ __attribute__((aligned(16))) uint32_t member[POINTS];
+	static_assert(sizeof(cand) + sizeof(member) == small_static_bytes(sizeof(F), T, POINTS, THREADS), "the plan's static arrays");
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
 	const uint32_t pg = wave % PG, cw = wave / PG;
@@ -497,95 +494,44 @@ update_small_kernel(const F* __restrict__ data, size_t stride, const uint32_t* _
 	if (tid < mine) sizes[c0 + tid] = count[tid];
 }
 
-static uint32_t small_row_stride(uint32_t dim) { return (((dim + 3) / 4) | 1u) * 4; }
-template <typename F> static uint32_t assign_small_static()
-{
-	return SMALL_WAVES * SMALL_POINTS * ((uint32_t)sizeof(F) + 4) + SMALL_POINTS * 4 + 64;
-}
-/* LDS next to the static arrays: the rows of the points and as many centroids as 32 KB hold (at least 32: one step of all wavefronts) */
-template <typename F> static uint32_t assign_small_chunk(uint32_t dim, uint32_t k)
-{
-	const uint32_t fit = 32 * 1024 / (small_row_stride(dim) * (uint32_t)sizeof(F)) / 32 * 32;
-	return std::min(k, std::max(32u, fit));
-}
-template <typename F> static uint32_t assign_small_lds(uint32_t dim, uint32_t k, uint32_t points, bool sums)
-{
-	const uint32_t centroids = assign_small_chunk<F>(dim, k) * small_row_stride(dim) * (uint32_t)sizeof(F);
-	return points * small_row_stride(dim) * (uint32_t)sizeof(F) + (sums ? std::max(centroids, k * dim * 8 + k * 4) : centroids);
-}
-
-constexpr uint32_t SMALL_FEW_CENTROIDS = 12; /* up to here a tile of one point times one centroid per lane */
-
-/*
- * Every pair costs 3 dim operations and about 30 to compare and keep, four cycles each on a SIMD; a work-group of 64 points keeps one
- * compute unit, so fewer than 256 of them leave units idle. Us per iteration near the line, these kernels / the general path: N = 40000, d = 32, k = 100
- * (effort 504 million) 28.7 / 40.3; N = 32768, d = 32, k = 128 (528) 27.1 / 31.5; N = 65536, d = 16, k = 100 (511) 27.2 / 32.0; N = 50000, d = 16, k = 128 (499)
- * 29.9 / 28.3; N = 65536, d = 8, k = 200 (708) 33.8 / 29.3. Wider rows, per assignment: N = 65536, d = 64, k = 50 (727) 20.4 / 22.6; N = 40000, d = 64, k = 80
- * (710) 20.2 / 21.7; N = 20000, d = 64, k = 200 (888) 32.1 / 22.7. Doubles: twice 450 million.
- * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
- */
-constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
-constexpr uint64_t SMALL_EFFORT = 530000000, SMALL_EFFORT_DOUBLES = 450000000; /* (doubles, N = 56478, d = 56, k = 128, 475: 87 us per iteration, general path 54) */
 template <typename F>
-bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
-{
-	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
-	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
-	const uint64_t limit = (sizeof(F) == 8 ? 2 * SMALL_EFFORT_DOUBLES : SMALL_EFFORT) * (dim > 32 ? 3 : 2) / 2;
-	return effort <= limit && assign_small_lds<F>(dim, k, SMALL_POINTS, false) + assign_small_static<F>() <= lds_budget;
-}
-
-/*
- * Up to 128 work-groups of 64 points leave half of the compute units idle: 32 points each (us per iteration, 64 / 32 points: N = 1000, d = 20, k = 128 14.4 / 12.0;
- * N = 5000, d = 32, k = 100 16.5 / 14.5; N = 10240, d = 20, k = 128 16.4 / 16.6: twice the partial sums). One work-group per compute unit at most: 16
- * wavefronts each, whose waits for the LDS others cover (eight / 16: N = 10240, d = 20, k = 128 16.4 / 15.2; N = 16384 15.9 / 15.0); with two, the waits
- * are covered already (N = 20000, d = 100, k = 30, SoA 23.3 / 26.7; d = 8, k = 30 12.7 / 15.1; AoS d = 20, k = 100 20.0 / 19.8; N = 32768, d = 8, k = 64 13.6 / 14.6).
- */
-constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 256 * SMALL_POINTS;
+bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget) { return small_assign_accepts(sizeof(F), dim, k, n, lds_budget); }
 
 template <typename F, bool SUMS>
 static int launch_assign_small_t(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
-                                 uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, F* partial, uint32_t* partial_counts, uint32_t* blocks, const DeviceInfo& dev)
+                                 uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, F* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t lds_budget)
 {
-	const bool half = n <= SMALL_HALF_POINTS, wide = !half && n <= SMALL_WIDE_POINTS;
-	const uint32_t points = half ? SMALL_POINTS / 2 : SMALL_POINTS;
-	const uint32_t lds = assign_small_lds<F>(dim, k, points, SUMS);
-	*blocks = (n + points - 1) / points;
+	const SmallShape shape = small_shape(sizeof(F), dim, k, n, SUMS, lds_budget);
+	*blocks = (n + shape.points - 1) / shape.points;
 	const uint32_t align = 4 * sizeof(F) - 1;
 	const uint32_t vec4 = (dim % 4 == 0 && stride % 4 == 0 && ((uintptr_t)data & align) == 0 ? 1u : 0u) | (dim % 4 == 0 && stride_means % 4 == 0 && ((uintptr_t)means & align) == 0 ? 2u : 0u);
 	void (*kernel)(const F*, size_t, const F*, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t*, F*, uint32_t*) = nullptr;
 #define KMX_PICK(P, Q, W) (layout == KMX_AOS ? (layout_means == KMX_AOS ? assign_small_kernel<F, P, Q, W, KMX_AOS, KMX_AOS, SUMS> : assign_small_kernel<F, P, Q, W, KMX_AOS, KMX_SOA, SUMS>) \
                                        : (layout_means == KMX_AOS ? assign_small_kernel<F, P, Q, W, KMX_SOA, KMX_AOS, SUMS> : assign_small_kernel<F, P, Q, W, KMX_SOA, KMX_SOA, SUMS>))
-	const bool few = k <= SMALL_FEW_CENTROIDS;
-	kernel = half ? (few ? KMX_PICK(1, 32, 512) : KMX_PICK(2, 32, 512)) : wide ? (few ? KMX_PICK(1, 64, 1024) : KMX_PICK(2, 64, 1024)) : few ? KMX_PICK(1, 64, 512) : KMX_PICK(2, 64, 512);
+	const bool few = shape.tile == 1;
+	kernel = shape.points == 32 ? (few ? KMX_PICK(1, 32, 512) : KMX_PICK(2, 32, 512)) : shape.threads == 1024 ? (few ? KMX_PICK(1, 64, 1024) : KMX_PICK(2, 64, 1024)) : few ? KMX_PICK(1, 64, 512) : KMX_PICK(2, 64, 512);
 #undef KMX_PICK
-	if (lds > 48 * 1024) KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(wide ? 1024 : SMALL_THREADS), lds, stream(), data, stride, means, stride_means, assignment, dim, k, n,
-	                   small_row_stride(dim), assign_small_chunk<F>(dim, k), (uint32_t)((0x100000000ull + dim - 1) / dim), vec4, counters, partial, partial_counts);
+	if (shape.lds_bytes > 48 * 1024) KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.lds_bytes));
+	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(shape.threads), shape.lds_bytes, stream(), data, stride, means, stride_means, assignment, dim, k, n,
+	                   small_row_stride(dim), assign_small_chunk(sizeof(F), dim, k), (uint32_t)((0x100000000ull + dim - 1) / dim), vec4, counters, partial, partial_counts);
 	KMX_LAUNCH_CHECK("assign_small_kernel");
 	return KMX_OK;
 }
 
 template <typename F>
 int launch_assign_small(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
-                        uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, uint32_t* blocks, const DeviceInfo& dev)
+                        uint32_t dim, uint32_t k, uint32_t n, uint32_t* counters, uint32_t* blocks, uint32_t lds_budget)
 {
-	return launch_assign_small_t<F, false>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, counters, nullptr, nullptr, blocks, dev);
+	return launch_assign_small_t<F, false>(data, layout, stride, means, layout_means, stride_means, assignment, dim, k, n, counters, nullptr, nullptr, blocks, lds_budget);
 }
 
 /* the single-pass iteration of small inputs: partial sums and counts of *blocks work-groups, at most assign_small_max_blocks(n), for launch_reduce_partials */
-int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, const DeviceInfo& dev)
+int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, uint32_t lds_budget)
 {
 	return launch_assign_small_t<float, true>(a.data, a.layout, a.stride, a.means, a.layout_means, a.stride_means, a.assignment, a.dim, a.k, a.n,
-	                                          counters, partial, partial_counts, blocks, dev);
+	                                          counters, partial, partial_counts, blocks, lds_budget);
 }
-uint32_t assign_small_max_blocks(uint32_t n) { return n <= SMALL_HALF_POINTS ? (n + SMALL_POINTS / 2 - 1) / (SMALL_POINTS / 2) : (n + SMALL_POINTS - 1) / SMALL_POINTS; }
-/* (the partial sums of all work-groups are written and read once) */
-bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
-{
-	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * ((n + SMALL_POINTS - 1) / SMALL_POINTS) <= (2u << 20) && small_assign_fits<float>(dim, k, n, lds_budget) &&
-	       assign_small_lds<float>(dim, k, SMALL_POINTS, true) + assign_small_static<float>() <= lds_budget;
-}
+bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget) { return small_iteration_accepts(dim, k, n, lds_budget); }
 
 /*
  * The members of a cluster come from one compute unit, so the largest cluster sets the time: everything in one cluster is
@@ -640,7 +586,7 @@ int launch_update_small(const F* data, int layout, size_t stride, const uint32_t
 #define KMX_SMALL_INSTANCES(F)                                                                                                                                   \
 	template bool small_assign_fits<F>(uint32_t, uint32_t, uint32_t, uint32_t);                                                                                  \
 	template bool small_update_fits<F>(uint32_t, uint32_t, uint32_t, uint32_t, const DeviceInfo&);                                                               \
-	template int launch_assign_small<F>(const F*, int, size_t, const F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, const DeviceInfo&); \
+	template int launch_assign_small<F>(const F*, int, size_t, const F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, uint32_t); \
 	template int launch_update_small<F>(const F*, int, size_t, const uint32_t*, F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, uint32_t*, const DeviceInfo&);
 KMX_SMALL_INSTANCES(float)
 KMX_SMALL_INSTANCES(double)

@@ -1,0 +1,93 @@
+/*
+ * Which small inputs assign_small_kernel (small.hip) takes and with which work-groups, and the LDS they need. Plain host code without a HIP
+ * header: the tests look at every shape that is accepted. value_bytes: 4 for floats, 8 for doubles.
+ */
+#ifndef KMX_SMALL_PLAN_H
+#define KMX_SMALL_PLAN_H
+
+#include <algorithm>
+#include <cstdint>
+
+namespace kmx {
+
+constexpr uint32_t SMALL_WAVE = 64, SMALL_POINTS = SMALL_WAVE;
+constexpr uint32_t SMALL_THREADS = 512, SMALL_WIDE_THREADS = 1024;
+constexpr uint32_t SMALL_SUMS = 4096; /* elements of the sums: beyond, reading the memberships again (update_small_kernel) is cheaper than as many partial sums */
+constexpr uint32_t SMALL_FEW_CENTROIDS = 12; /* up to here a tile of one point times one centroid per lane */
+
+/* a candidate: a root and its centroid's number, floats as 64 bits (SmallKey) */
+constexpr uint32_t small_key_bytes(uint32_t value_bytes) { return value_bytes == 4 ? 8 : 16; }
+/* shares of the centroids: a wavefront has 16 * tile of the points */
+constexpr uint32_t small_shares(uint32_t tile, uint32_t points, uint32_t threads) { return threads / SMALL_WAVE / (points / 16 / tile); }
+/* the kernel's static arrays: a candidate per share and point, a membership per point */
+constexpr uint32_t small_static_bytes(uint32_t value_bytes, uint32_t tile, uint32_t points, uint32_t threads)
+{
+	return small_shares(tile, points, threads) * points * small_key_bytes(value_bytes) + points * 4;
+}
+
+constexpr uint32_t small_row_stride(uint32_t dim) { return (((dim + 3) / 4) | 1u) * 4; }
+/* LDS next to the static arrays: the rows of the points and as many centroids as 32 KB hold (at least 32: one step of all wavefronts) */
+inline uint32_t assign_small_chunk(uint32_t value_bytes, uint32_t dim, uint32_t k)
+{
+	const uint32_t fit = 32 * 1024 / (small_row_stride(dim) * value_bytes) / 32 * 32;
+	return std::min(k, std::max(32u, fit));
+}
+inline uint32_t assign_small_lds(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t points, bool sums)
+{
+	const uint32_t centroids = assign_small_chunk(value_bytes, dim, k) * small_row_stride(dim) * value_bytes;
+	return points * small_row_stride(dim) * value_bytes + (sums ? std::max(centroids, k * dim * 8 + k * 4) : centroids);
+}
+
+/*
+ * Every pair costs 3 dim operations and about 30 to compare and keep, four cycles each on a SIMD; a work-group of 64 points keeps one
+ * compute unit, so fewer than 256 of them leave units idle. Us per iteration near the line, these kernels / the general path: N = 40000, d = 32, k = 100
+ * (effort 504 million) 28.7 / 40.3; N = 32768, d = 32, k = 128 (528) 27.1 / 31.5; N = 65536, d = 16, k = 100 (511) 27.2 / 32.0; N = 50000, d = 16, k = 128 (499)
+ * 29.9 / 28.3; N = 65536, d = 8, k = 200 (708) 33.8 / 29.3. Wider rows, per assignment: N = 65536, d = 64, k = 50 (727) 20.4 / 22.6; N = 40000, d = 64, k = 80
+ * (710) 20.2 / 21.7; N = 20000, d = 64, k = 200 (888) 32.1 / 22.7. Doubles: twice 450 million.
+ * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
+ */
+constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
+constexpr uint64_t SMALL_EFFORT = 530000000, SMALL_EFFORT_DOUBLES = 450000000; /* (doubles, N = 56478, d = 56, k = 128, 475: 87 us per iteration, general path 54) */
+/* what the rule leaves for the static arrays: those of every work-group of eight wavefronts fit; one of 16 is taken only where its own do (small_shape) */
+constexpr uint32_t small_static_room(uint32_t value_bytes) { return SMALL_THREADS / SMALL_WAVE * SMALL_POINTS * (value_bytes + 4) + SMALL_POINTS * 4 + 64; }
+constexpr bool small_static_fits(uint32_t value_bytes, uint32_t tile, uint32_t points) { return small_static_bytes(value_bytes, tile, points, SMALL_THREADS) <= small_static_room(value_bytes); }
+static_assert(small_static_fits(4, 1, 64) && small_static_fits(4, 2, 64) && small_static_fits(4, 1, 32) && small_static_fits(4, 2, 32) &&
+              small_static_fits(8, 1, 64) && small_static_fits(8, 2, 64) && small_static_fits(8, 1, 32) && small_static_fits(8, 2, 32), "eight wavefronts");
+
+inline bool small_assign_accepts(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
+{
+	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
+	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
+	const uint64_t limit = (value_bytes == 8 ? 2 * SMALL_EFFORT_DOUBLES : SMALL_EFFORT) * (dim > 32 ? 3 : 2) / 2;
+	return effort <= limit && assign_small_lds(value_bytes, dim, k, SMALL_POINTS, false) + small_static_room(value_bytes) <= lds_budget;
+}
+/* floats, points added up too (the partial sums of all work-groups are written and read once) */
+inline bool small_iteration_accepts(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
+{
+	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * ((n + SMALL_POINTS - 1) / SMALL_POINTS) <= (2u << 20) && small_assign_accepts(4, dim, k, n, lds_budget) &&
+	       assign_small_lds(4, dim, k, SMALL_POINTS, true) + small_static_room(4) <= lds_budget;
+}
+
+/*
+ * Up to 128 work-groups of 64 points leave half of the compute units idle: 32 points each (us per iteration, 64 / 32 points: N = 1000, d = 20, k = 128 14.4 / 12.0;
+ * N = 5000, d = 32, k = 100 16.5 / 14.5; N = 10240, d = 20, k = 128 16.4 / 16.6: twice the partial sums). One work-group per compute unit at most: 16
+ * wavefronts each, whose waits for the LDS others cover (eight / 16: N = 10240, d = 20, k = 128 16.4 / 15.2; N = 16384 15.9 / 15.0); with two, the waits
+ * are covered already (N = 20000, d = 100, k = 30, SoA 23.3 / 26.7; d = 8, k = 30 12.7 / 15.1; AoS d = 20, k = 100 20.0 / 19.8; N = 32768, d = 8, k = 64 13.6 / 14.6).
+ * 16 wavefronts have twice as many candidates in LDS, which rows of around 200 doubles leave no room for: eight there.
+ */
+constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 256 * SMALL_POINTS;
+
+struct SmallShape { uint32_t tile, points, threads, lds_bytes; /* without the static arrays */ };
+
+inline SmallShape small_shape(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t n, bool sums, uint32_t lds_budget)
+{
+	const uint32_t tile = k > SMALL_FEW_CENTROIDS ? 2 : 1, points = n <= SMALL_HALF_POINTS ? SMALL_POINTS / 2 : SMALL_POINTS;
+	const uint32_t lds = assign_small_lds(value_bytes, dim, k, points, sums);
+	const bool wide = n > SMALL_HALF_POINTS && n <= SMALL_WIDE_POINTS && lds + small_static_bytes(value_bytes, tile, points, SMALL_WIDE_THREADS) <= lds_budget;
+	return SmallShape{ tile, points, wide ? SMALL_WIDE_THREADS : SMALL_THREADS, lds };
+}
+inline uint32_t assign_small_max_blocks(uint32_t n) { return n <= SMALL_HALF_POINTS ? (n + SMALL_POINTS / 2 - 1) / (SMALL_POINTS / 2) : (n + SMALL_POINTS - 1) / SMALL_POINTS; }
+
+} // namespace kmx
+
+#endif

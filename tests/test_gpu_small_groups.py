@@ -47,3 +47,33 @@ def test_both_sides_of_the_lines(km, orc, gpu, dim, k, n, layout):
             out.free(); sizes.free()
         for b in (d, m, a):
             b.free()
+
+
+@pytest.mark.parametrize("dim,k", [(196, 128), (197, 132), (200, 64), (204, 100), (204, 32), (205, 28), (237, 16), (250, 14), (252, 12), (256, 14)])
+@pytest.mark.parametrize("n", [8192, 8193, 10000, 16384, 16385])
+def test_wide_rows_beside_what_lds_holds(km, orc, gpu, dim, k, n):
+    """Rows of around 200 doubles, where 16 wavefronts' candidates do not fit beside them."""
+    for layout in (0, 1):
+        test_both_sides_of_the_lines(km, orc, gpu, dim, k, n, layout)
+
+
+@pytest.mark.parametrize("budget", [48 * 1024, 72 * 1024, 100 * 1024])
+@pytest.mark.parametrize("dim,k", [(20, 13), (48, 64), (64, 64), (100, 40)])
+def test_small_inputs_under_a_callers_budget(km, orc, gpu, dim, k, budget):
+    n = 10000
+    rng = np.random.default_rng(dim + budget)
+    rows = np.round(rng.normal(size=(n, dim)) * 4) / 4
+    means = rows[rng.permutation(n)[:k]].copy()
+    execution = km.ExecParams()
+    execution.shared_mem_bytes = budget
+    for dtype, fn in ((np.float32, orc.assign), (np.float64, orc.assign_f64)):
+        item = np.dtype(dtype).itemsize
+        want = fn(rows.astype(dtype).ravel(), means.astype(dtype).ravel(), dim, k, n, threads=0)
+        d = km.DeviceBuffer(item * n * dim); d.write(rows.astype(dtype).ravel())
+        m = km.DeviceBuffer(item * k * dim); m.write(means.astype(dtype).ravel())
+        a = km.DeviceBuffer(4 * n); a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+        km.assign(km.ASSIGN_BEST, d, 0, dim, m, 0, dim, a, dim, k, n, execution, dtype)
+        km.sync()
+        assert np.array_equal(a.read(np.uint32, n), want)
+        for b in (d, m, a):
+            b.free()

@@ -1,0 +1,58 @@
+"""Small inputs (csrc/small_plan.h): every shape that the rule accepts is launched with work-groups whose LDS fits the budget, static arrays included, and
+with as many partial sums as there is room for (no GPU needed: all shapes are enumerated)."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = """
+#include "small_plan.h"
+using namespace kmx;
+/* number of accepted shapes, and of those whose launch asks for more than the budget; always_wide: as if 16 wavefronts were taken whatever they need */
+extern "C" void count(uint32_t value_bytes, int sums, uint32_t budget, int always_wide, uint64_t* accepted, uint64_t* beyond, uint64_t* wide)
+{
+	*accepted = *beyond = *wide = 0;
+	const uint32_t points[] = { 1, 31, 32, 33, 64, 1000, 8191, 8192, 8193, 10000, 16383, 16384, 16385, 30000, 65535, 65536, 65537 };
+	for (uint32_t n : points)
+		for (uint32_t dim = 1; dim <= 257; ++dim)
+			for (uint32_t k = 1; k <= 1200; k += k < 300 ? 1 : 37) {
+				if (!(sums ? value_bytes == 4 && small_iteration_accepts(dim, k, n, budget) : small_assign_accepts(value_bytes, dim, k, n, budget))) continue;
+				++*accepted;
+				const SmallShape s = small_shape(value_bytes, dim, k, n, sums != 0, budget);
+				const uint32_t threads = always_wide && n > SMALL_HALF_POINTS && n <= SMALL_WIDE_POINTS ? SMALL_WIDE_THREADS : s.threads;
+				*beyond += s.lds_bytes + small_static_bytes(value_bytes, s.tile, s.points, threads) > budget || (n + s.points - 1) / s.points > assign_small_max_blocks(n);
+				*wide += threads == SMALL_WIDE_THREADS;
+			}
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def count(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("small")
+    src, lib = folder / "small.cpp", folder / "libsmall.so"
+    src.write_text(SOURCE)
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "cuda-kmeans_amd", "csrc"), str(src), "-o", str(lib)])
+    fn = ctypes.CDLL(str(lib)).count
+    fn.restype = None
+
+    def call(value_bytes, sums, budget, always_wide=False):
+        out = [ctypes.c_uint64() for _ in range(3)]
+        fn(value_bytes, int(sums), budget, int(always_wide), *[ctypes.byref(v) for v in out])
+        return [v.value for v in out]
+    return call
+
+
+@pytest.mark.parametrize("value_bytes,sums", [(4, False), (4, True), (8, False)])
+@pytest.mark.parametrize("budget", [160 * 1024, 128 * 1024, 64 * 1024 + 8, 48 * 1024, 16 * 1024])
+def test_what_is_accepted_fits(count, value_bytes, sums, budget):
+    accepted, beyond, wide = count(value_bytes, sums, budget)
+    assert accepted > 0 and beyond == 0
+    assert wide > 0                                                     # the rule is not kept by never taking 16 wavefronts
+
+
+def test_candidates_that_are_not_counted_would_be_noticed(count):
+    """16 wavefronts whatever they need: more than there is, for rows of around 200 doubles."""
+    assert count(8, False, 160 * 1024, always_wide=True)[1] > 0
