@@ -278,11 +278,9 @@ static int launch_iteration_small(const AssignArgs& a, const UpdateArgs& u, kmx_
  * d = 300, k = 2000 377 -> 318; N = 131071, d = 512, k = 40 320 -> 355; N = 99999, d = 500, k = 400 273 -> 301; N = 20000, d = 400, k = 1000 120 -> 136).
  */
 constexpr size_t WIDE_COLUMNS_FLOATS = (size_t)1 << 24;
-static int launch_two_passes_soa(AssignArgs a, UpdateArgs u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+static int launch_two_passes_soa(AssignArgs a, UpdateArgs u, bool reads_columns, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
 {
 	AosRows rows = { nullptr, 0 };
-	const bool no_room = recording_graph() && (size_t)u.n * u.dim > ws->rows_copy_cap; /* (the room was made for columns without a stride of their own) */
-	const bool reads_columns = u.dim <= 256 || no_room || (u.stride % 32 == 0 && (size_t)u.n * u.dim >= WIDE_COLUMNS_FLOATS);
 	const bool columns = reads_columns && sums64_takes_columns(u.dim, u.k, u.n, exec, ws, dev);
 	if (!columns && update_wants_rows(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev)) {
 		if (sweep_writes_rows(a, exec, dev)) a.rows_out = &rows;
@@ -297,6 +295,18 @@ static int launch_two_passes_soa(AssignArgs a, UpdateArgs u, kmx_exec_params* ex
 	if (rc) return rc;
 	if (rows.data) { u.data = rows.data; u.stride = rows.stride; u.layout = KMX_AOS; }
 	return launch_update(KMX_UPDATE_ATOMIC_SHM, u, exec, ws, dev);
+}
+
+static int launch_two_passes_soa(const AssignArgs& a, const UpdateArgs& u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev)
+{
+	const bool enough = (size_t)u.n * u.dim >= WIDE_COLUMNS_FLOATS;
+	if (u.dim > 256 && enough && sizing_only()) {
+		/* the stride decides, and the room is for calls with any */
+		const int rc = launch_two_passes_soa(a, u, false, exec, ws, dev);
+		return rc ? rc : launch_two_passes_soa(a, u, true, exec, ws, dev);
+	}
+	const bool no_room = recording_graph() && (size_t)u.n * u.dim > ws->rows_copy_cap; /* for rows */
+	return launch_two_passes_soa(a, u, u.dim <= 256 || no_room || (u.stride % 32 == 0 && enough), exec, ws, dev);
 }
 
 } // namespace kmx

@@ -107,3 +107,34 @@ def test_noalloc_update_refuses_what_does_not_fit(km, gpu):
     assert s.read(np.uint32, k)[0] == n
     for b in (d, a, m, s):
         b.free()
+
+
+@pytest.mark.parametrize("dim,k,n", [(300, 200, 65536), (512, 400, 32800), (300, 2000, 60001), (200, 300, 90000)])
+def test_reserved_room_is_enough_for_columns_of_any_stride(km, orc, gpu, dim, k, n):
+    """kmx_reserve_f32 names no stride, and that of SoA points decides whether an iteration reads them by columns or by rows (more than 256 dimensions):
+    after the reservation neither allocates anything."""
+    rng = np.random.default_rng(dim + n)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    cents = rows[rng.choice(n, k, replace=False)].copy()
+    want = orc.assign(rows.ravel(), cents.ravel(), dim, k, n, threads=0, fast=True)
+    m = km.DeviceBuffer(4 * k * dim); m.write(cents.ravel())
+    a = km.DeviceBuffer(4 * n); out = km.DeviceBuffer(4 * k * dim); sizes = km.DeviceBuffer(4 * k)
+    for stride in (n, n + 5, (n + 32) // 32 * 32):
+        stored = np.full((dim, stride), np.nan, np.float32)
+        stored[:, :n] = rows.T
+        d = km.DeviceBuffer(stored.nbytes); d.write(stored.ravel())
+        km.iteration(d, SOA, stride, m, out, AOS, dim, a, sizes, dim, k, n)   # (the runtime keeps memory of its own for the kernels)
+        km.sync()
+        km.check(km.hip_lib().kmx_shutdown())
+        km.reserve(km.ASSIGN_BEST, km.UPDATE_ATOMIC_SHM, SOA, AOS, dim, k, n)
+        a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+        km.sync()
+        before = device_memory_in_use()
+        km.iteration(d, SOA, stride, m, out, AOS, dim, a, sizes, dim, k, n)
+        km.sync()
+        assert device_memory_in_use() == before, stride
+        assert np.array_equal(a.read(np.uint32, n), want)
+        assert np.array_equal(sizes.read(np.uint32, k), np.bincount(want, minlength=k))
+        d.free()
+    for b in (m, a, out, sizes):
+        b.free()
