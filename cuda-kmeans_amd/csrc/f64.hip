@@ -1413,12 +1413,12 @@ static int update_f64_call(const char* who, bool divide, int variant,
 		rc = launch_update_small<double>(data, layout, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n, divide, &exec->block_count, *dev);
 		return rc ? rc : profile_end(1);
 	}
-	if (variant == KMX_UPDATE_ATOMIC_SHM && (!recording_graph() || workspace_exists())) {
+	if (variant == KMX_UPDATE_ATOMIC_SHM) {
 		Workspace* ws = nullptr;
-		if ((rc = workspace(&ws))) return rc;
-		Sums64Result result = SUMS64_OTHERS;
-		rc = launch_update_sums64<double>(data, layout, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n, divide, exec, ws, *dev, &result);
-		if (rc || result == SUMS64_DONE) return rc ? rc : profile_end(1);
+		if (!launches_recorded() && (rc = workspace(&ws))) return rc;
+		bool done = false;
+		rc = launch_update_sums64<double>(data, layout, stride, assignment, means, layout_means, stride_means, cluster_sizes, dim, k, n, divide, exec, ws, *dev, &done);
+		if (rc || done) return rc ? rc : profile_end(1);
 	}
 #define KMX_F64_UPDATE(LD, LM) \
 	launch_update_f64_t<LD, LM>(variant, data, stride, assignment, means, stride_means, cluster_sizes, dim, k, n, exec, *dev, divide)

@@ -72,7 +72,6 @@ struct Workspace {
 	bool fixed = false; /* the work space of the entry point that allocates nothing: its buffers never grow, a call that needs more is refused */
 };
 int workspace(Workspace** ws);
-bool workspace_exists(); /* workspace() would allocate nothing */
 int reserve_queue(Workspace* ws, size_t entries);
 int reserve_packed(Workspace* ws, size_t packed_floats, size_t norm_floats, size_t transposed_floats);
 int reserve_cells(Workspace* ws, size_t words);
@@ -233,17 +232,18 @@ inline uint32_t lds_budget_of(const kmx_exec_params* exec, const DeviceInfo& dev
 /* means and sizes from the partial sums [chunks][k][dim] and counts [chunks][k] */
 template <typename F>
 int launch_reduce_partials(const F* partial, const uint32_t* partial_counts, uint32_t chunks, F* means, int layout_means, size_t stride_means, uint32_t* sizes, uint32_t dim, uint32_t k, bool divide);
-/* update_sums64.hip: the update where the clusters' sums fit LDS as doubles. SUMS64_DONE: means and sizes are finished; SUMS64_OTHERS: not for this
- * shape; SUMS64_NO_ROOM: a graph is recorded and the partial sums would need a larger work space, so a kernel without any has to do */
-enum Sums64Result { SUMS64_DONE, SUMS64_OTHERS, SUMS64_NO_ROOM };
+/* update_sums64.hip: the update where the clusters' sums fit LDS as doubles. *done: means and sizes are finished; otherwise it is not for this shape.
+ * Doubles whose launches are recorded take no work space (ws may be null) */
 template <typename F>
 int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
-                         uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, Sums64Result* result);
+                         uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, bool* done);
 /* floats: whether it takes SoA points as they are */
 bool sums64_takes_columns(uint32_t dim, uint32_t k, uint32_t n, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev);
 /* the work space of kmx_update_f32_noalloc on the current device: `partials` is the library's static scratch array */
 int noalloc_workspace(Workspace** ws);
+Workspace* fixed_scratch(); /* the same where its address is known, else null */
 bool recording_graph(); /* between kmx_graph_begin and kmx_graph_end */
+bool launches_recorded(); /* the same, or the caller records the stream it has set */
 int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* whether launch_update would copy the SoA points of u into AoS rows first, and that copy: ws->rows_copy, rows of dim floats */
 bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev);

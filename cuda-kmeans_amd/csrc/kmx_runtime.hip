@@ -34,6 +34,14 @@ static bool g_capturing = false;
 hipStream_t stream() { return g_capturing ? g_capture_stream : g_stream; }
 bool recording_graph() { return g_capturing; }
 
+bool launches_recorded()
+{
+	if (g_capturing || !g_stream) return g_capturing; /* (the legacy stream cannot be recorded) */
+	hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(g_stream, &status) != hipSuccess) { (void)hipGetLastError(); return false; }
+	return status == hipStreamCaptureStatusActive;
+}
+
 #define KMX_NOT_WHILE_CAPTURING(name)                                                                          \
 	do {                                                                                                       \
 		if (g_capturing) return fail(KMX_ERR_INVALID_ARGUMENT, name ": not allowed between kmx_graph_begin and kmx_graph_end"); \
@@ -80,8 +88,6 @@ int device_info(const DeviceInfo** out)
 	*out = &g_dev;
 	return KMX_OK;
 }
-
-bool workspace_exists() { return g_ws.counters != nullptr; }
 
 int workspace(Workspace** ws)
 {
@@ -801,6 +807,8 @@ int kmx_graph_begin(void)
 {
 	clear_error();
 	KMX_NOT_WHILE_CAPTURING("kmx_graph_begin");
+	Workspace* scratch = nullptr;
+	if (noalloc_workspace(&scratch)) clear_error(); /* the address of the scratch array that recorded updates use (they do without if it has none) */
 	if (!g_capture_stream) KMX_HIP(hipStreamCreateWithFlags(&g_capture_stream, hipStreamNonBlocking));
 	/* work already queued on the caller's stream stays ahead of whatever the graph will do: the graph is launched
 	 * on that stream; recording itself runs nothing */

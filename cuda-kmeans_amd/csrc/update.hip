@@ -18,8 +18,7 @@
  *                              with integer LDS atomics, then lane groups walk the sorted list and sum each
  *                              cluster's rows in registers (no atomics at all); per-chunk sums go to a partial
  *                              buffer with plain coalesced stores and reduce_partials_kernel folds them.
- *       update_lds_kernel      fallback for the shapes/layouts the others do not take, and while
- *                              a graph is recorded and nothing can be allocated: LDS-privatised ds_add_f32.
+ *       update_lds_kernel      fallback for the shapes/layouts the others do not take: LDS-privatised ds_add_f32.
  *     Points are read exactly once in all of them.
  *   reduce_copies_kernel / divide_means_kernel
  *                         - counterparts of reducePrivCopiesKernel / divideMeansKernel
@@ -797,14 +796,14 @@ static int launch_update_tuned(const UpdateArgs& u, kmx_exec_params* exec, Works
 	*state = 1;
 	const uint32_t budget = exec->shared_mem_bytes ? std::min(exec->shared_mem_bytes, dev.lds_bytes) : dev.lds_bytes;
 
-	Sums64Result sums64 = SUMS64_OTHERS;
 	{
-		const int rc = launch_update_sums64<float>(u.data, LD, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.n, u.divide, exec, ws, dev, &sums64);
-		if (sums64 == SUMS64_DONE) *state = 2;
-		if (rc || sums64 == SUMS64_DONE) return rc;
+		bool done = false;
+		const int rc = launch_update_sums64<float>(u.data, LD, u.stride, u.assignment, u.means, u.layout_means, u.stride_means, u.cluster_sizes, u.dim, u.k, u.n, u.divide, exec, ws, dev, &done);
+		if (done) *state = 2;
+		if (rc || done) return rc;
 	}
 
-	if (LD == KMX_AOS && sums64 != SUMS64_NO_ROOM && u.k < (1u << (32 - SORT_SHIFT)) && (uint64_t)(u.k + 36) * 4 + 1024 * 4 + 1024 * 5 * 4 <= budget) {
+	if (LD == KMX_AOS && u.k < (1u << (32 - SORT_SHIFT)) && (uint64_t)(u.k + 36) * 4 + 1024 * 4 + 1024 * 5 * 4 <= budget) {
 		const uint32_t slices = (u.dim + 31) / 32;
 		/* rows of 33 to 256 dimensions: the work-groups of a chunk take ranges of clusters and read whole rows (measured at
 		 * N = 1M, d = 256, k = 1024: 0.29 ms in slices of 32 dimensions) */
@@ -1029,7 +1028,7 @@ rows_from_soa_kernel(const float* __restrict__ data, size_t stride, float* __res
 }
 
 /*
- * Scratch memory of kmx_update_f32_noalloc: the per-chunk partial sums and counts of update_sorted_kernel, the only
+ * Scratch memory of kmx_update_f32_noalloc, and of recorded updates (update_sums64.hip): the per-chunk partial sums and counts, the only
  * device memory beyond inputs and outputs the update uses with AoS points. One copy per GPU, held until the process
  * ends. In host code the array's name is only a stand-in: its device address on the current device comes from
  * hipGetSymbolAddress, once per device, and that pointer is what the kernels get.
@@ -1059,6 +1058,14 @@ int noalloc_workspace(Workspace** ws)
 	}
 	*ws = &w;
 	return KMX_OK;
+}
+
+Workspace* fixed_scratch()
+{
+	int device = 0;
+	if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= NOALLOC_MAX_DEVICES) return nullptr;
+	Workspace& w = g_noalloc_ws[device];
+	return w.partials ? &w : nullptr;
 }
 
 bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev)

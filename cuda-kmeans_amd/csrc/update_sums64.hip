@@ -560,16 +560,16 @@ static bool plan_ranges64(uint32_t dim, uint32_t k, uint32_t n, uint32_t budget,
 }
 
 static int launch_ranges64(const float* data, size_t stride, const uint32_t* assignment, float* means, int layout_means, size_t stride_means, uint32_t* sizes,
-                           uint32_t dim, uint32_t k, uint32_t n, bool divide, const Ranges64Plan& p, Workspace* ws)
+                           uint32_t dim, uint32_t k, uint32_t n, bool divide, const Ranges64Plan& p, float* partials)
 {
 	const size_t rows = (size_t)p.groups * ((k + (1u << p.log_ranges) - 1) >> p.log_ranges);
-	uint32_t* counts = (uint32_t*)(ws->partials + rows * dim);
+	uint32_t* counts = (uint32_t*)(partials + rows * dim);
 	KMX_HIP(hipFuncSetAttribute((const void*)update_ranges64_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds_bytes));
 	KMX_LAUNCH_KERNEL(update_ranges64_kernel, dim3(p.groups * p.slices), dim3(SUMS64_THREADS), p.lds_bytes, stream(),
-	                  data, stride, assignment, ws->partials, counts, counts + rows, dim, k, n, p.groups, p.log_ranges, p.width);
+	                  data, stride, assignment, partials, counts, counts + rows, dim, k, n, p.groups, p.log_ranges, p.width);
 	KMX_LAUNCH_CHECK("update_ranges64_kernel");
 	auto fold = layout_means == KMX_AOS ? fold_ranges64_kernel<KMX_AOS> : fold_ranges64_kernel<KMX_SOA>;
-	KMX_LAUNCH_KERNEL(fold, dim3(k), dim3(4 * WAVE), 0, stream(), ws->partials, counts, counts + rows, means, stride_means, sizes, dim, k, p.log_ranges, divide ? 1u : 0u);
+	KMX_LAUNCH_KERNEL(fold, dim3(k), dim3(4 * WAVE), 0, stream(), partials, counts, counts + rows, means, stride_means, sizes, dim, k, p.log_ranges, divide ? 1u : 0u);
 	KMX_LAUNCH_CHECK("fold_ranges64_kernel");
 	return KMX_OK;
 }
@@ -587,48 +587,68 @@ static int launch_sums64(const F* data, size_t stride, const uint32_t* assignmen
 
 static size_t sums64_words(const Sums64Plan& p, uint32_t dim, uint32_t k, size_t item) { return (size_t)p.chunks * k * dim * (item / sizeof(float)) + (size_t)p.chunks * k; }
 
+/*
+ * Where the partial sums of a call lie (null: a kernel without any has to do). A recording keeps the addresses of its moment, and the work space moves when a
+ * later call needs more of it: recorded sums lie in the static scratch array, which holds all but those of SoA points with thousands of dimensions. Those of
+ * floats take the work space (as the copied rows did), doubles the kernels of f64.hip, which need none.
+ */
+static bool recorded_sums_fit(size_t words)
+{
+	const Workspace* fixed = fixed_scratch();
+	return fixed && words <= fixed->partials_cap;
+}
+
+template <typename F>
+static int place_sums(Workspace* ws, size_t words, float** partials)
+{
+	*partials = nullptr;
+	if (launches_recorded()) {
+		if (recorded_sums_fit(words)) {
+			*partials = fixed_scratch()->partials;
+			return KMX_OK;
+		}
+		if (sizeof(F) == 8) return KMX_OK;
+	}
+	const int rc = reserve_partials(ws, words);
+	*partials = ws->partials;
+	return rc;
+}
+
 bool sums64_takes_columns(uint32_t dim, uint32_t k, uint32_t n, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev)
 {
 	Sums64Plan p;
-	return n > 0 && !ws->fixed && plan_columns64(dim, k, n, false, lds_budget_of(exec, dev), dev.compute_units, &p) &&
-	       !(recording_graph() && sums64_words(p, dim, k, sizeof(float)) > ws->partials_cap);
+	if (n == 0 || ws->fixed || !plan_columns64(dim, k, n, false, lds_budget_of(exec, dev), dev.compute_units, &p)) return false;
+	const size_t words = sums64_words(p, dim, k, sizeof(float));
+	return !launches_recorded() || recorded_sums_fit(words) || words <= ws->partials_cap;
 }
 
 template <typename F>
 int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_t* assignment, F* means, int layout_means, size_t stride_means, uint32_t* sizes,
-                         uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, Sums64Result* result)
+                         uint32_t dim, uint32_t k, uint32_t n, bool divide, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, bool* done)
 {
-	*result = SUMS64_OTHERS;
+	*done = false;
 	Sums64Plan p;
+	float* partials = nullptr;
 	const bool columns = layout == KMX_SOA;
-	if (n == 0 || (columns && ws->fixed)) return KMX_OK; /* (SoA points are taken there whatever their number of partial sums) */
+	if (n == 0 || (columns && ws && ws->fixed)) return KMX_OK; /* (SoA points are taken there whatever their number of partial sums) */
 	const bool planned = (columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p);
 	if constexpr (sizeof(F) == 4) {
 		Ranges64Plan r;
 		if (!columns && ranges64_pays(dim, k, n, planned) && plan_ranges64(dim, k, n, lds_budget_of(exec, dev), dev.compute_units, &r)) {
-			const size_t words = ranges64_words(r, dim, k);
-			if (recording_graph() && words > ws->partials_cap) {
-				*result = SUMS64_NO_ROOM;
-				return KMX_OK;
-			}
-			const int rc = reserve_partials(ws, words);
+			const int rc = place_sums<F>(ws, ranges64_words(r, dim, k), &partials);
 			if (rc) return rc;
-			*result = SUMS64_DONE;
+			*done = true;
 			exec->block_count = r.groups * r.slices;
-			return launch_ranges64(data, stride, assignment, means, layout_means, stride_means, sizes, dim, k, n, divide, r, ws);
+			return launch_ranges64(data, stride, assignment, means, layout_means, stride_means, sizes, dim, k, n, divide, r, partials);
 		}
 	}
 	if (!planned) return KMX_OK;
-	const size_t sums = (size_t)p.chunks * k * dim, words = sums64_words(p, dim, k, sizeof(F));
-	if (recording_graph() && words > ws->partials_cap) {
-		*result = SUMS64_NO_ROOM;
-		return KMX_OK;
-	}
-	int rc = reserve_partials(ws, words);
-	if (rc) return rc;
-	*result = SUMS64_DONE;
+	const size_t sums = (size_t)p.chunks * k * dim;
+	int rc = place_sums<F>(ws, sums64_words(p, dim, k, sizeof(F)), &partials);
+	if (rc || !partials) return rc;
+	*done = true;
 	exec->block_count = p.chunks * p.slices;
-	F* partial = (F*)ws->partials;
+	F* partial = (F*)partials;
 	uint32_t* partial_counts = (uint32_t*)(partial + sums);
 #define KMX_SUMS64(LW) (dim % p.width == 0 && p.width == LW ? launch_sums64<LW, true, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p) \
 	                                                        : launch_sums64<LW, false, F>(data, stride, assignment, partial, partial_counts, dim, k, n, p))
@@ -641,7 +661,7 @@ int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_
 	return launch_reduce_partials<F>(partial, partial_counts, p.chunks, means, layout_means, stride_means, sizes, dim, k, divide);
 }
 
-template int launch_update_sums64<float>(const float*, int, size_t, const uint32_t*, float*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
-template int launch_update_sums64<double>(const double*, int, size_t, const uint32_t*, double*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, Sums64Result*);
+template int launch_update_sums64<float>(const float*, int, size_t, const uint32_t*, float*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, bool*);
+template int launch_update_sums64<double>(const double*, int, size_t, const uint32_t*, double*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, kmx_exec_params*, Workspace*, const DeviceInfo&, bool*);
 
 } // namespace kmx

@@ -150,7 +150,7 @@ int kmx_assign_f32(int variant,
  * kmx_update_f32 calls of this shape and these variants and for kmx_iteration_f32 and kmx_fused_f32 calls of this shape, so that
  * those calls allocate nothing afterwards
  * (no counterpart in the reference, whose runners allocate nothing: cuda.hpp:54-64 allocates everything in initialize()).
- * Without it the first call of a shape grows the work space itself, which waits for the stream and calls hipMalloc; a
+ * Points and centroids may have any stride. Without it the first call of a shape grows the work space itself, which waits for the stream and calls hipMalloc; a
  * call with a different LDS budget (shared_mem_bytes) than the default may still grow it. Not while a graph is recorded.
  */
 int kmx_reserve_f32(int assign_variant, int update_variant, int layout, int layout_means, uint32_t dim, uint32_t k, uint32_t n);
@@ -188,7 +188,8 @@ int kmx_update_f32(int variant,
  * work space that kmx_update_f32 grows with hipMalloc. The call allocates and frees nothing; a shape whose partial
  * sums do not fit is refused with KMX_ERR_UNSUPPORTED (the message names both sizes). SoA points skip the AoS copy
  * kmx_update_f32 makes of them and run the element-wise kernels (slower, same results). Per-kernel profiling
- * (kmx_set_profiling) does not cover this call. All calls on one GPU share that GPU's array: calls that overlap in
+ * (kmx_set_profiling) does not cover this call. All calls on one GPU share that GPU's array, also with recorded updates (see
+ * kmx_graph_begin): calls and replays that overlap in
  * time on one GPU (different streams, different threads) race; calls on the library's one stream do not.
  * The address of a device's array is looked up once per device: by kmx_set_device, by kmx_reserve_f32, or else by the
  * first call of this function on the device, which is therefore refused (KMX_ERR_INVALID_ARGUMENT) between kmx_graph_begin
@@ -263,8 +264,10 @@ int kmx_iteration_last_passes(int* passes);
  *   KMX_ASSIGN_LDS_FMA ranks with fp64 FMAs; KMX_ASSIGN_MFMA, _MFMA_BF16X3 and _BEST rank float copies of the inputs with the
  *   float sweeps (work space: n * dim + k * dim floats); all hand the points they cannot certify to the serial arithmetic
  *   on the doubles.
- * kmx_update_f64: ATOMIC_POINT / _FINE / _SHM; ATOMIC_SHM privatises the sums in LDS (whole when k * dim doubles fit 32 KB,
- *   in ranges of clusters of that size beyond), the others (and more than 256 ranges) use fp64 atomics in global memory. privatized_copies > 1: KMX_ERR_UNSUPPORTED.
+ * kmx_update_f64: ATOMIC_POINT / _FINE / _SHM / SERIAL_ORDER; ATOMIC_SHM keeps the sums in LDS: slices of the coordinates of all clusters where ten of
+ *   them fit (SoA points: as many as there are), whose partial sums take the library's work space (at most 256 times k * dim doubles; grown on demand,
+ *   kmx_reserve_f32 does not size it); otherwise whole sums of up to 32 KB or ranges of clusters of that size, without work space. ATOMIC_POINT / _FINE (and more than 256 ranges) use
+ *   fp64 atomics in global memory. privatized_copies > 1: KMX_ERR_UNSUPPORTED.
  *   Precondition as for kmx_update_f32: means and cluster_sizes are zero (kmx_fill_zero_u32 with twice the count).
  * kmx_fused_f64: KMX_FUSED_TWO_PASS / KMX_FUSED_BEST (assignment into the work space, then the update);
  *   KMX_FUSED_ONE_PASS is float-only: KMX_ERR_UNSUPPORTED.
@@ -316,6 +319,11 @@ int kmx_event_elapsed_ms(void* start, void* stop, float* ms); /* waits for `stop
  * (the host driver records two ping-pong iterations once and replays them). Everything that allocates, copies or
  * waits is refused while recording; a call whose work space would have to grow is refused too -- make the same
  * calls once before recording. Per-kernel profiling events are not recorded.
+ * A recording holds the addresses of its moment: those of its buffers, and of the work space where a call uses it, which a later call that needs more
+ * of it, and kmx_shutdown, release. It is not launched after that; kmx_reserve_f32 for the largest shape beforehand keeps the work space where it is.
+ * Updates with KMX_UPDATE_ATOMIC_SHM (kmx_update_f32, kmx_update_f64) whose sums fit LDS take their scratch memory from the static array of kmx_update_f32_noalloc instead, so
+ * recordings of nothing else stay valid. The same holds where the caller records the stream of kmx_set_stream with the runtime's own means, except that kmx_set_device,
+ * kmx_reserve_f32 or kmx_graph_begin has to come first (the array's address) and that replays are the caller's to keep from overlapping with other users of the array.
  */
 int kmx_graph_begin(void);
 int kmx_graph_end(void** graph);

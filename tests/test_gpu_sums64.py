@@ -3,6 +3,8 @@ steps, copies of the sums, members of no cluster, against sums in 64 bits.
 
 The bound: a chunk's sums are exact to a double's rounding and rounded to the result's type once, then at most 256 chunks are added one after the other and the
 sum is divided: 258 roundings of at most the sum of the magnitudes (doubles: one more per member)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -169,3 +171,100 @@ def test_recorded_iterations_in_reserved_room(km, orc, gpu, dim, k, n, layout, p
     g.destroy()
     for b in (d, m, a, out, sizes):
         b.free()
+
+
+# shapes whose update used no work space until its sums lay in LDS as doubles: few clusters, columns of fewer than eight dimensions, doubles
+NO_WORK_SPACE = [(16, 16, 1 << 16, AOS, np.float32), (4, 300, 70001, SOA, np.float32), (32, 200, 70001, AOS, np.float64), (20, 300, 70001, SOA, np.float64)]
+
+
+def runtime():
+    """The HIP runtime this process has loaded."""
+    return ctypes.CDLL("libamdhip64.so")
+
+
+def own_stream():
+    stream = ctypes.c_void_p()
+    assert runtime().hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0   # (non-blocking)
+    return stream
+
+
+class Prepared:
+    def __init__(self, km, dim, k, n, layout, dtype, seed):
+        rng = np.random.default_rng(seed)
+        rows = rng.normal(size=(n, dim)).astype(dtype)
+        self.member = rng.integers(0, k, size=n).astype(np.uint32)
+        self.member[:k] = np.arange(k)
+        self.want = np.zeros((k, dim)); np.add.at(self.want, self.member, rows.astype(np.float64))
+        self.want /= np.bincount(self.member, minlength=k)[:, None]
+        self.args = (dim, k, n); self.dtype = dtype; self.layout = layout
+        self.d = km.DeviceBuffer(rows.nbytes); self.d.write(rows.ravel() if layout == AOS else rows.T.copy().ravel())
+        self.a = km.DeviceBuffer(4 * n); self.a.write(self.member)
+        self.m = km.DeviceBuffer(rows.itemsize * k * dim); self.s = km.DeviceBuffer(4 * k)
+
+    def update(self, km):
+        dim, k, n = self.args
+        km.update(km.UPDATE_ATOMIC_SHM, self.d, self.layout, dim if self.layout == AOS else n, self.a, self.m, AOS, dim, self.s, dim, k, n, None, self.dtype)
+
+    def spoil(self):
+        dim, k, n = self.args
+        self.m.write(np.full(k * dim, np.nan, self.dtype)); self.s.write(np.full(k, 7, np.uint32))
+
+    def check(self):
+        dim, k, n = self.args
+        assert np.array_equal(self.s.read(np.uint32, k), np.bincount(self.member, minlength=k))
+        assert np.abs(self.m.read(self.dtype, k * dim).reshape(k, dim) - self.want).max() < 1e-5   # (|x| < 6: sums of a thousandth of that per rounding)
+
+    def free(self):
+        for b in (self.d, self.a, self.m, self.s):
+            b.free()
+
+
+@pytest.mark.parametrize("dim,k,n,layout,dtype", NO_WORK_SPACE)
+def test_recorded_updates_outlive_the_work_space(km, gpu, dim, k, n, layout, dtype):
+    """Recorded with room for the partial sums in the work space, which then moves (a larger call) and goes (kmx_shutdown)."""
+    p = Prepared(km, dim, k, n, layout, dtype, 5)
+    large = Prepared(km, 24, 500, 1 << 18, AOS, np.float64, 6)
+    p.update(km)
+    km.sync()
+    with km.Graph() as g:
+        p.m.zero(); p.s.zero()
+        p.update(km)
+    for _ in range(2):
+        large.update(km)
+        large.check()
+        for _ in range(2):
+            p.spoil()
+            g.launch()
+            km.sync()
+            p.check()
+        km.check(km.hip_lib().kmx_shutdown())
+    g.destroy()
+    p.free(); large.free()
+
+
+def test_doubles_on_a_stream_that_the_caller_records(km, gpu):
+    """Without a work space: nothing is allocated, and nothing is left in the recording that would not run."""
+    hip, lib = runtime(), km.hip_lib()
+    for dim, k, n, layout in ((32, 200, 70001, AOS), (20, 300, 70001, SOA)):
+        p = Prepared(km, dim, k, n, layout, np.float64, 9)
+        p.update(km)                                      # (kernels are loaded)
+        km.sync()
+        km.check(lib.kmx_shutdown())
+        stream, graph, launched = own_stream(), ctypes.c_void_p(), ctypes.c_void_p()
+        assert hip.hipStreamBeginCapture(stream, 0) == 0  # (the strictest mode)
+        try:
+            km.check(lib.kmx_set_stream(stream))
+            p.m.zero(); p.s.zero()
+            p.update(km)
+        finally:
+            km.check(lib.kmx_set_stream(None))
+            assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(launched), graph, None, None, ctypes.c_size_t(0)) == 0
+        for _ in range(3):
+            p.spoil()
+            km.sync()
+            assert hip.hipGraphLaunch(launched, stream) == 0
+            km.sync()
+            p.check()
+        assert hip.hipGraphExecDestroy(launched) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+        p.free()
