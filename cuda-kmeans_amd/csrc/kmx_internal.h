@@ -244,6 +244,7 @@ int noalloc_workspace(Workspace** ws);
 Workspace* fixed_scratch(); /* the same where its address is known, else null */
 bool recording_graph(); /* between kmx_graph_begin and kmx_graph_end */
 bool launches_recorded(); /* the same, or the caller records the stream it has set */
+void scratch_recorded(); /* the launches that are recorded use the static scratch array */
 int launch_update(int variant, const UpdateArgs& u, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 /* whether launch_update would copy the SoA points of u into AoS rows first, and that copy: ws->rows_copy, rows of dim floats */
 bool update_wants_rows(int variant, const UpdateArgs& u, const kmx_exec_params* exec, const Workspace* ws, const DeviceInfo& dev);

@@ -136,6 +136,23 @@ int reserve_packed16(Workspace* ws, size_t packed_floats, size_t norm_floats)
 	return rc ? rc : grow(&ws->norms16, &ws->norms16_cap, norm_floats);
 }
 
+/*
+ * The partial sums of all streams lie in one array, and those of all recordings in another: the first use of either on another stream than the last one's
+ * waits for the device. (Not for an event of that stream: it may have been destroyed since, and only its name is kept.)
+ */
+static hipStream_t g_scratch_stream = nullptr;
+static bool g_scratch_used = false, g_scratch_recorded = false;
+void scratch_recorded() { g_scratch_recorded = true; }
+
+static int order_scratch()
+{
+	if (g_sizing || launches_recorded()) return KMX_OK; /* (nothing runs now) */
+	if (g_scratch_used && g_scratch_stream != g_stream) KMX_HIP(hipDeviceSynchronize());
+	g_scratch_stream = g_stream;
+	g_scratch_used = true;
+	return KMX_OK;
+}
+
 int reserve_partials(Workspace* ws, size_t floats)
 {
 	if (ws->fixed) {
@@ -143,7 +160,8 @@ int reserve_partials(Workspace* ws, size_t floats)
 		return fail(KMX_ERR_UNSUPPORTED, "the call needs %zu bytes of scratch memory for its partial sums; the entry point that allocates nothing holds %zu",
 		            floats * sizeof(float), ws->partials_cap * sizeof(float));
 	}
-	return grow(&ws->partials, &ws->partials_cap, floats);
+	const int rc = order_scratch();
+	return rc ? rc : grow(&ws->partials, &ws->partials_cap, floats);
 }
 int reserve_fused_assignment(Workspace* ws, size_t entries) { return grow(&ws->fused_assignment, &ws->fused_cap, entries); }
 int reserve_bucket_sizes(Workspace* ws, size_t entries) { return grow(&ws->bucket_sizes, &ws->bucket_cap, entries); }
@@ -848,6 +866,8 @@ int kmx_graph_launch(void* graph)
 	clear_error();
 	KMX_NOT_WHILE_CAPTURING("kmx_graph_launch");
 	if (!graph) return fail(KMX_ERR_INVALID_ARGUMENT, "kmx_graph_launch: null graph");
+	const int rc = g_scratch_recorded ? order_scratch() : KMX_OK;
+	if (rc) return rc;
 	KMX_HIP(hipGraphLaunch((hipGraphExec_t)graph, g_stream));
 	return KMX_OK;
 }

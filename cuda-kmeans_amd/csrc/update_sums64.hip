@@ -605,6 +605,7 @@ static int place_sums(Workspace* ws, size_t words, float** partials)
 	if (launches_recorded()) {
 		if (recorded_sums_fit(words)) {
 			*partials = fixed_scratch()->partials;
+			scratch_recorded();
 			return KMX_OK;
 		}
 		if (sizeof(F) == 8) return KMX_OK;

@@ -18,6 +18,9 @@
  *     called) and the calls return without waiting, except kmx_sync, kmx_d2h and
  *     kmx_event_elapsed_ms. Stream order is the only dependency mechanism, as in the reference
  *     (cuda.hpp:70-88: one cudaDeviceSynchronize after the iteration loop).
+ *     All streams share the library's work space, so assignments and whole iterations may not overlap on
+ *     several of them. Updates may: where their partial sums need the work space, or a graph is launched that holds some, the first
+ *     call on another stream than the last one's waits for the device.
  *   - Not thread-safe: one host thread drives one device, as in the reference. The library keeps one work space, one
  *     stream and the properties of one device per process; kmx_set_device to another device is refused until
  *     kmx_shutdown() has released the work space.

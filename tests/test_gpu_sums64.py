@@ -242,6 +242,44 @@ def test_recorded_updates_outlive_the_work_space(km, gpu, dim, k, n, layout, dty
     p.free(); large.free()
 
 
+@pytest.mark.parametrize("dim,k,n,layout,dtype", NO_WORK_SPACE)
+def test_updates_on_two_streams(km, gpu, dim, k, n, layout, dtype):
+    """The calls of two streams share the partial sums' array: the second waits for the first, eager or recorded."""
+    pair = [Prepared(km, dim, k, n, layout, dtype, seed) for seed in (7, 8)]
+    streams = [own_stream() for _ in pair]
+    graphs = []
+    for p in pair:
+        p.update(km)
+        with km.Graph() as g:
+            p.m.zero(); p.s.zero()
+            p.update(km)
+        graphs.append(g)
+    lib = km.hip_lib()
+    try:
+        for recorded in (False, True):
+            for p in pair:
+                p.spoil()
+            km.sync()
+            for _ in range(20):
+                for p, stream, g in zip(pair, streams, graphs):
+                    km.check(lib.kmx_set_stream(stream))
+                    g.launch() if recorded else p.update(km)
+            km.sync()
+            for p in pair:
+                p.check()
+    finally:
+        km.check(lib.kmx_set_stream(None))
+    km.sync()
+    for g in graphs:
+        g.destroy()
+    for stream in streams:
+        assert runtime().hipStreamDestroy(stream) == 0
+    for p in pair:
+        p.update(km)                                      # (the stream that used the array last is gone)
+        p.check()
+        p.free()
+
+
 def test_doubles_on_a_stream_that_the_caller_records(km, gpu):
     """Without a work space: nothing is allocated, and nothing is left in the recording that would not run."""
     hip, lib = runtime(), km.hip_lib()
