@@ -123,11 +123,37 @@ update_sums64_kernel(const F* __restrict__ data, size_t stride, const uint32_t* 
 }
 
 /*
+ * Where the sorted chunks (update.hip) are ahead of slices (floats; us per call, slices / sorted chunks):
+ *   - wide slices whose sums to write are an eighth of what is read and more (N = 140625, d = 128, k = 300 29.3 / 24.1; N = 162500, d = 80, k = 500 28.9 / 23.9; N = 250000, d = 128,
+ *     k = 300, a seventh, 37.0 / 33.4; N = 400000, d = 70, k = 300, a tenth, 34.8 / 40.7), of 32 coordinates and fewer nearly a half (N = 82000, d = 110, k = 600
+ *     22.4 / 20.5; N = 102000, d = 127, k = 600, three eighths, 25.5 / 25.8);
+ *   - slices that are parts of a line, from 2^26 floats on, which the caches do not hold: of 16 that begin inside lines, up to 2^27 floats, and while they leave a tenth of the compute units
+ *     over up to 200 million (sorted chunks in shares of the slices' time: d = 100, k = 1000, seven slices x 32 chunks: N = 720000 0.87, 900000 0.85, 1.8M 0.94, 2.4M 1.18; d = 90,
+ *     six x 40: N = 1M 0.91, 1.3M 1.00, 2.2M 1.05; d = 120, eight x 32: N = 600000 1.02, 1M 1.02); of 8 of rows of whole lines (N = 6.25M, d = 32, k = 2000 0.90; N = 1.9M, d = 48
+ *     0.92; but d = 36 1.05) and of 4 (N = 6.25M, d = 32, k = 4000 0.78; N = 2.5M, d = 36 0.88; but N = 7.1M, d = 28 1.11).
+ */
+static bool sorted_pays(uint32_t dim, uint32_t k, uint32_t n, uint32_t width, uint32_t slices, uint32_t chunks, uint32_t compute_units)
+{
+	const uint64_t written = (uint64_t)chunks * k; /* rows of sums */
+	if (width > 32 ? slices >= 2 && written * 8 > n : width > 16 && written * 20 > (uint64_t)n * 9) return true;
+	const uint64_t floats = (uint64_t)n * dim;
+	if (floats < (1u << 26)) return false;
+	if (width == 16 && dim > 64 && dim % 16 != 0) {
+		const uint32_t busy = slices * chunks;
+		return floats < (busy * 10 < compute_units * 9 ? 200000000u : busy < compute_units ? 1u << 27 : 0u);
+	}
+	return dim >= 32 && (width <= 4 || (width == 8 && dim % 16 == 0));
+}
+
+/*
  * A work-group per compute unit: slices of the coordinates x chunks of the points, as few slices as let their sums fit LDS, ten at most (d = 160, k = 600: ten
  * 139 us, five 129, sorted chunks 158; d = 256, k = 1024: sixteen 277, sorted chunks 242; N = 1M here and below). Slices are equal, or, in floats, of whole 64
  * bytes up to 32 coordinates (sorted chunks / equal / these: d = 33, k = 1000 54 / 41 / 35; d = 80, k = 1000 86 / 101 / 77; wider ones d = 100, k = 100,
- * N = 500000: 50 + 50 38, 64 + 36 46). Rows of up to 48 floats go in slices of 16, doubles in slices of 32 or two, even where the whole row fits (d = 40,
- * k = 300: 34, whole 37; doubles, N = 2M, d = 32, k = 500: 103, 113): the sums to write are fewer. Doubles whose sums do not fit as a whole: 16 at a time (N = 500000,
+ * N = 500000: 50 + 50 38, 64 + 36 46; d = 112, N = 392857 56 + 56 34.5, 64 + 48 36.6), and of whole 64 bytes where rows consist of such in three slices and more (d = 160, k = 100: N = 412500
+ * 54 + 54 + 52 60, 64 + 64 + 32 49.5, sorted chunks 53; N = 1.25M 180, 156, 164). Rows of up to 48 floats go in slices of 16, doubles in slices of 32 or two, even where the whole row fits (d = 40,
+ * k = 300: 34, whole 37; doubles, N = 2M, d = 32, k = 500: 103, 113): the sums to write are fewer. But from some 60 million floats on, which the memory-side cache
+ * does not hold, a row that begins anywhere is read once (slices of 16 / whole: d = 36, k = 18, N = 1.6M 43.6 / 42.8, N = 1.9M 64.6 / 53.4, N = 2.8M 113 / 86; d = 18 58.8 / 58.6
+ * at 68 million, 81 / 75 at 80; d = 44, N = 1.3M 41 / 44, N = 1.5M 64 / 53; d = 48, k = 200, N = 3.3M 135 / 129; d = 32, N = 5M 128 / 126). Doubles whose sums do not fit as a whole: 16 at a time (N = 500000,
  * d = 128, k = 1024: 123, slices of 19 142, sums of ranges of clusters 204), equal where the last would be narrow (N = 1M, d = 33, k = 1000: 73,
  * 16 + 16 + 1 86, ranges 77), eight at a time where rows are odd multiples of 32 bytes and short (N = 1M, d = 24, k = 1200: 43, 12 + 12 47, ranges 53). Rows of more than 192 floats in slices of 32 and less lose
  * (N = 500000, d = 256, k = 600: 123 against 121).
@@ -137,8 +163,6 @@ update_sums64_kernel(const F* __restrict__ data, size_t stride, const uint32_t* 
  * k = 500: one slice 16, two 13). Sums of doubles are twice as dear: four times as many points, and few points are left to the kernels that add to the means
  * where they lie (N = 400000, d = 32, k = 1000 33.2, those 34.2; N = 100000, k = 500 17.4, 17.1; N = 200000, d = 4, k = 4000 19.0, 16.2;
  * rows of one slice of 16: N = 225824, d = 11, k = 1105 23.9, 15.1; k = 700 18.5, 16.7; N = 500000, k = 1105 24.9, 27.9; d = 8 15.7, 18.5).
- * Unaligned slices of a middling number of points: N = 100000, d = 100, k = 500 26.1, sorted chunks 21.9; N = 143310, d = 160, k = 354 31.5, 27.1; but N = 300000, d = 148 42.4,
- * 45.5; N = 30000, d = 140, k = 300 13.0, 16.6; N = 100000, d = 200, k = 100 22.8, 24.3.
  * Few clusters: the rows of a request mostly meet at the same sums, which costs an LDS cycle each; copies of them, as many as rows (N = 16M, d = 2,
  * k = 2: 90 us without, 34 with).
  */
@@ -156,25 +180,25 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 	/* doubles whose sums do not fit as a whole */
 	const bool parts = doubles && bytes(dim) > budget, eights = parts && dim <= 56 && dim % 4 == 0 && dim % 16 != 0;
 	if (parts && slices_of(16) == 7 && dim % 16 != 0 && dim % 16 <= 8) return false;
-	const uint32_t fewest = dim <= 16 ? 1 : parts ? slices_of(eights ? 8 : 16) : doubles ? std::max<uint32_t>(2, slices_of(32)) : dim <= 48 ? slices_of(16) : slices_of(SUMS64_LANES);
+	const bool whole_row = !doubles && dim > 16 && dim <= 48 && bytes(dim) <= budget && (uint64_t)n * dim >= 60000000;
+	const uint32_t fewest = dim <= 16 || whole_row ? 1 : parts ? slices_of(eights ? 8 : 16) : doubles ? std::max<uint32_t>(2, slices_of(32)) : dim <= 48 ? slices_of(16) : slices_of(SUMS64_LANES);
 	uint32_t width = 0;
 	for (uint32_t slices = fewest; slices <= SUMS64_SLICES && (width == 0 || width > 16); ++slices) {
 		const uint32_t equal = (dim - 1) / slices + 1, whole = equal > 8 ? (equal + 15) / 16 * 16 : equal > 4 ? 8 : 4;
-		const bool as_is = doubles ? !eights && !(parts && equal > 8 && (dim - 1) % 16 >= 7) : equal > 32;
-		const uint32_t w = dim <= 16 || as_is ? equal : whole;
+		const bool as_is = doubles ? !eights && !(parts && equal > 8 && (dim - 1) % 16 >= 7) : equal > 32 && !(dim % 16 == 0 && slices >= 3);
+		const uint32_t w = dim <= 16 || slices == 1 || as_is ? equal : whole;
 		if (bytes(w) > budget || (dim > 192 && w <= 32 && !doubles)) continue;
 		if (width != 0 && least_points * 2 * chunks_of(width) <= n) break; /* enough points for this many work-groups */
 		width = w;
 	}
 	if (width == 0) return false;
-	/* three slices and more that begin inside a line, and sums to write that are a fifth of what is read: the sorted chunks, while the points lie in the caches */
-	if (!doubles && width > 32 && width % 16 != 0 && slices_of(width) >= 3 && k >= 300 && (uint64_t)n * dim >= (1u << 23) && (uint64_t)n * dim < (1u << 25)) return false;
 	uint32_t lanes = 1, copies = 1;
 	while (lanes < width) lanes *= 2;
 	while (copies * 2 <= WAVE / lanes && 2 * copies * bytes(width) <= std::min<uint32_t>(budget, 48 * 1024)) copies *= 2;
 	const uint64_t points = (std::max<uint64_t>(least_points, ((uint64_t)n + chunks_of(width) - 1) / chunks_of(width)) + WAVE - 1) / WAVE * WAVE;
-	const uint32_t chunk_points = (uint32_t)std::min<uint64_t>(points, 1u << 31);
-	*plan = { width, slices_of(width), copies, (uint32_t)(((uint64_t)n + chunk_points - 1) / chunk_points), chunk_points, (uint32_t)(copies * bytes(width)) };
+	const uint32_t chunk_points = (uint32_t)std::min<uint64_t>(points, 1u << 31), chunks = (uint32_t)(((uint64_t)n + chunk_points - 1) / chunk_points);
+	if (!doubles && sorted_pays(dim, k, n, width, slices_of(width), chunks, compute_units)) return false;
+	*plan = { width, slices_of(width), copies, chunks, chunk_points, (uint32_t)(copies * bytes(width)) };
 	return true;
 }
 

@@ -306,3 +306,31 @@ def test_doubles_on_a_stream_that_the_caller_records(km, gpu):
             p.check()
         assert hip.hipGraphExecDestroy(launched) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
         p.free()
+
+
+@pytest.mark.parametrize("dim,k", [(17, 70), (37, 300), (48, 400), (37, 900)])
+def test_whole_rows_of_many_points(km, gpu, dim, k):
+    """Both sides of the line from which rows of 17 to 48 floats go as a whole (37 x 900 sums do not fit so). Small whole numbers: every sum is exact."""
+    line = -(-60000000 // dim)
+    rng = np.random.default_rng(dim + k)
+    rows = rng.integers(-8, 9, size=(line, dim), dtype=np.int8).astype(np.float32)
+    member = rng.integers(0, k, size=line).astype(np.uint32)
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * line); a.write(member)
+    m = km.DeviceBuffer(4 * k * dim); s = km.DeviceBuffer(4 * k)
+    for n in (line, line - 1):
+        m.write(np.full(k * dim, np.nan, np.float32)); s.write(np.full(k, 7, np.uint32))
+        km.update(km.UPDATE_ATOMIC_SHM, d, AOS, dim, a, m, AOS, dim, s, dim, k, n)
+        counts = np.bincount(member[:n], minlength=k)
+        want = np.stack([np.bincount(member[:n], weights=rows[:n, q], minlength=k) for q in range(dim)], axis=1)
+        assert np.array_equal(s.read(np.uint32, k), counts)
+        assert np.array_equal(m.read(np.float32, k * dim).reshape(k, dim), want.astype(np.float32) / counts.astype(np.float32)[:, None])
+    for b in (d, a, m, s):
+        b.free()
+
+
+@pytest.mark.parametrize("dim,k,n", [(160, 100, 150001), (176, 60, 150001), (144, 30, 100003), (192, 200, 200001), (128, 400, 300001), (112, 100, 100003), (160, 100, 20011)])
+def test_slices_of_whole_lines(km, gpu, dim, k, n):
+    """Rows of whole 64 bytes in three slices and more, the last one narrower; the last two: equal slices, and slices of 32."""
+    check(km, dim, k, n, np.float32, outside=True)
+    check(km, dim, k, n, np.float32, layout_means=SOA, stride=dim + 3)
