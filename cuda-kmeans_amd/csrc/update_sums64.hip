@@ -196,9 +196,8 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 	while (lanes < width) lanes *= 2;
 	while (copies * 2 <= WAVE / lanes && 2 * copies * bytes(width) <= std::min<uint32_t>(budget, 48 * 1024)) copies *= 2;
 	const uint64_t points = (std::max<uint64_t>(least_points, ((uint64_t)n + chunks_of(width) - 1) / chunks_of(width)) + WAVE - 1) / WAVE * WAVE;
-	const uint32_t chunk_points = (uint32_t)std::min<uint64_t>(points, 1u << 31), chunks = (uint32_t)(((uint64_t)n + chunk_points - 1) / chunk_points);
-	if (!doubles && sorted_pays(dim, k, n, width, slices_of(width), chunks, compute_units)) return false;
-	*plan = { width, slices_of(width), copies, chunks, chunk_points, (uint32_t)(copies * bytes(width)) };
+	const uint32_t chunk_points = (uint32_t)std::min<uint64_t>(points, 1u << 31);
+	*plan = { width, slices_of(width), copies, (uint32_t)(((uint64_t)n + chunk_points - 1) / chunk_points), chunk_points, (uint32_t)(copies * bytes(width)) };
 	return true;
 }
 
@@ -656,7 +655,9 @@ int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_
 	float* partials = nullptr;
 	const bool columns = layout == KMX_SOA;
 	if (n == 0 || (columns && ws && ws->fixed)) return KMX_OK; /* (SoA points are taken there whatever their number of partial sums) */
-	const bool planned = (columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p);
+	bool planned = (columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p);
+	/* (the sorted chunks' partial sums may be several times as many, and would not fit the scratch array) */
+	if (planned && !columns && sizeof(F) == 4 && !ws->fixed && !launches_recorded()) planned = !sorted_pays(dim, k, n, p.width, p.slices, p.chunks, dev.compute_units);
 	if constexpr (sizeof(F) == 4) {
 		Ranges64Plan r;
 		if (!columns && ranges64_pays(dim, k, n, planned) && plan_ranges64(dim, k, n, lds_budget_of(exec, dev), dev.compute_units, &r)) {

@@ -334,3 +334,36 @@ def test_slices_of_whole_lines(km, gpu, dim, k, n):
     """Rows of whole 64 bytes in three slices and more, the last one narrower; the last two: equal slices, and slices of 32."""
     check(km, dim, k, n, np.float32, outside=True)
     check(km, dim, k, n, np.float32, layout_means=SOA, stride=dim + 3)
+
+
+def test_many_clusters_of_many_points_without_allocation(km, gpu):
+    """Slices of four coordinates, where the sorted chunks are faster but their partial sums would not fit the scratch array: taken there and while recorded, as slices."""
+    dim, k, n = 32, 4000, (1 << 21) + 5
+    rng = np.random.default_rng(11)
+    rows = rng.integers(-8, 9, size=(n, dim), dtype=np.int8).astype(np.float32)
+    member = rng.integers(0, k, size=n).astype(np.uint32)
+    counts = np.bincount(member, minlength=k)
+    want = np.stack([np.bincount(member, weights=rows[:, q], minlength=k) for q in range(dim)], axis=1).astype(np.float32) / counts.astype(np.float32)[:, None]
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * n); a.write(member)
+    m = km.DeviceBuffer(4 * k * dim); s = km.DeviceBuffer(4 * k)
+
+    def check_result():
+        assert np.array_equal(s.read(np.uint32, k), counts)
+        assert np.array_equal(m.read(np.float32, k * dim).reshape(k, dim), want)       # (whole numbers: every sum is exact)
+        m.write(np.full(k * dim, np.nan, np.float32)); s.write(np.full(k, 7, np.uint32))
+    for fn in (km.update, km.update_noalloc):
+        fn(km.UPDATE_ATOMIC_SHM, d, AOS, dim, a, m, AOS, dim, s, dim, k, n)
+        check_result()
+    km.sync()
+    km.check(km.hip_lib().kmx_shutdown())
+    km.update(km.UPDATE_ATOMIC_SHM, d, AOS, dim, a, m, AOS, dim, s, dim, k, 64)
+    with km.Graph() as g:
+        km.update(km.UPDATE_ATOMIC_SHM, d, AOS, dim, a, m, AOS, dim, s, dim, k, n)
+    for _ in range(3):
+        g.launch()
+        km.sync()
+        check_result()
+    g.destroy()
+    for b in (d, a, m, s):
+        b.free()
