@@ -155,14 +155,18 @@ static bool sorted_pays(uint32_t dim, uint32_t k, uint32_t n, uint32_t width, ui
  * does not hold, a row that begins anywhere is read once (slices of 16 / whole: d = 36, k = 18, N = 1.6M 43.6 / 42.8, N = 1.9M 64.6 / 53.4, N = 2.8M 113 / 86; d = 18 58.8 / 58.6
  * at 68 million, 81 / 75 at 80; d = 44, N = 1.3M 41 / 44, N = 1.5M 64 / 53; d = 48, k = 200, N = 3.3M 135 / 129; d = 32, N = 5M 128 / 126). Doubles whose sums do not fit as a whole: 16 at a time (N = 500000,
  * d = 128, k = 1024: 123, slices of 19 142, sums of ranges of clusters 204), equal where the last would be narrow (N = 1M, d = 33, k = 1000: 73,
- * 16 + 16 + 1 86, ranges 77), eight at a time where rows are odd multiples of 32 bytes and short (N = 1M, d = 24, k = 1200: 43, 12 + 12 47, ranges 53). Rows of more than 192 floats in slices of 32 and less lose
+ * 16 + 16 + 1 86, ranges 77), eight at a time where rows are odd multiples of 32 bytes and short (N = 1M, d = 24, k = 1200: 43, 12 + 12 47, ranges 53).
+ * Seven slices leave an eighth of the compute units over: where rows begin inside lines and the caches do not hold them, the ranges (d = 100, k = 600: N = 500000 103, ranges 91,
+ * N = 1M 192, 176, but N = 300000 48, 52, N = 150000 30, 34; d = 105 105, 93, 197, 180, but 51, 54 and 31, 35). Rows of more than 192 floats in slices of 32 and less lose
  * (N = 500000, d = 256, k = 600: 123 against 121).
  * As many chunks per XCD as it has compute units for: one more somewhere comes alone at the end (d = 48, k = 1024: 85 chunks of three slices 62, 80 42).
  * A chunk has as many points as there are clusters, 512 at least: its sums are written and read once more (N = 200000, d = 4, k = 4000: 256 chunks 17 us, 50
  * 14, sorted chunks 31; N = 50000, d = 32, k = 1000: 17, 14, 16); where that leaves compute units over and a slice is wide, more slices (N = 100000, d = 32,
  * k = 500: one slice 16, two 13). Sums of doubles are twice as dear: four times as many points, and few points are left to the kernels that add to the means
  * where they lie (N = 400000, d = 32, k = 1000 33.2, those 34.2; N = 100000, k = 500 17.4, 17.1; N = 200000, d = 4, k = 4000 19.0, 16.2;
- * rows of one slice of 16: N = 225824, d = 11, k = 1105 23.9, 15.1; k = 700 18.5, 16.7; N = 500000, k = 1105 24.9, 27.9; d = 8 15.7, 18.5).
+ * rows of one slice, whose work-groups are as few as the chunks, unless they are 4 or 8 doubles, which a group of lanes reads without a gap: d = 11, N = 225824, k = 1105 24.2, 16.0; N = 300000
+ * 24.3, 20.9; N = 400000, k = 2000 28.2, 28.7; d = 6, N = 400000, k = 2000 26.3, 16.2; d = 13, N = 225824, k = 700 18.8, 21.1; but d = 8, N = 225824, k = 1105 15.7, 18.5;
+ * d = 4, N = 300000, k = 2000 15.4, 18.3).
  * Few clusters: the rows of a request mostly meet at the same sums, which costs an LDS cycle each; copies of them, as many as rows (N = 16M, d = 2,
  * k = 2: 90 us without, 34 with).
  */
@@ -175,11 +179,11 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 	auto slices_of = [&](uint32_t width) -> uint32_t { return (dim - 1) / width + 1; };
 	auto chunks_of = [&](uint32_t width) -> uint32_t { return std::max<uint32_t>(1, compute_units / SUMS64_XCDS / slices_of(width)) * SUMS64_XCDS; };
 	if (dim > SUMS64_SLICES * SUMS64_LANES || (doubles && n / 200 < k && (uint64_t)k * dim > 8192)) return false;
-	if (doubles && dim <= 16 && dim != 8 && n / 400 < k && (uint64_t)k * dim > 6144) return false; /* (one slice: as many work-groups as chunks) */
+	if (doubles && dim <= 16 && dim != 4 && dim != 8 && n / 300 < k && (uint64_t)k * dim > 6144) return false; /* (one slice: as many work-groups as chunks) */
 	const uint64_t least_points = std::max<uint64_t>(512, (uint64_t)k * (doubles ? 4 : 1));
 	/* doubles whose sums do not fit as a whole */
 	const bool parts = doubles && bytes(dim) > budget, eights = parts && dim <= 56 && dim % 4 == 0 && dim % 16 != 0;
-	if (parts && slices_of(16) == 7 && dim % 16 != 0 && dim % 16 <= 8) return false;
+	if (parts && slices_of(16) == 7 && dim % 16 != 0 && (uint64_t)n * dim >= 40000000) return false;
 	const bool whole_row = !doubles && dim > 16 && dim <= 48 && bytes(dim) <= budget && (uint64_t)n * dim >= 60000000;
 	const uint32_t fewest = dim <= 16 || whole_row ? 1 : parts ? slices_of(eights ? 8 : 16) : doubles ? std::max<uint32_t>(2, slices_of(32)) : dim <= 48 ? slices_of(16) : slices_of(SUMS64_LANES);
 	uint32_t width = 0;

@@ -367,3 +367,9 @@ def test_many_clusters_of_many_points_without_allocation(km, gpu):
     g.destroy()
     for b in (d, a, m, s):
         b.free()
+
+
+# both sides of the lines between slices of doubles and the kernels without partial sums
+@pytest.mark.parametrize("dim,k,n", [(100, 300, 399999), (100, 300, 400001), (105, 600, 380001), (105, 600, 381001), (97, 1000, 300001), (4, 2000, 300001), (8, 2000, 500001), (11, 1105, 331499), (11, 1105, 331500), (6, 2000, 400001)])
+def test_doubles_beside_the_lines(km, gpu, dim, k, n):
+    check(km, dim, k, n, np.float64, outside=True)
