@@ -1290,7 +1290,7 @@ extern "C" int kmx_assign_f64(int variant,
 	const DeviceInfo* dev = nullptr;
 	rc = device_info(&dev);
 	if (rc) return rc;
-	if (variant == KMX_ASSIGN_BEST && small_assign_fits<double>(dim, k, n, lds_budget_of(exec, *dev))) {
+	if (variant == KMX_ASSIGN_BEST && small_assign_fits<double>(layout, dim, k, n, lds_budget_of(exec, *dev))) {
 		/* small inputs: the serial arithmetic for every pair in one launch (small.hip) */
 		Workspace* ws = nullptr;
 		if ((rc = workspace(&ws))) return rc;

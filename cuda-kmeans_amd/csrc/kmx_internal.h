@@ -210,7 +210,7 @@ bool lds_fma_reads_through_scalar_cache(const AssignArgs& a); /* a handful of ce
 int launch_assign_lds_fma(const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev);
 
 /* small.hip: small inputs in one launch each (assignment, update), floats and doubles */
-template <typename F> bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget);
+template <typename F> bool small_assign_fits(int layout, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget);
 template <typename F> bool small_update_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget, const DeviceInfo& dev);
 /* lds_budget: the one that small_assign_fits or small_iteration_fits was asked with */
 template <typename F>
@@ -222,7 +222,7 @@ int launch_update_small(const F* data, int layout, size_t stride, const uint32_t
 /* the assignment of small inputs that also adds its points up: partial sums and counts of *blocks work-groups (at most
  * assign_small_max_blocks(n), small_plan.h), for launch_reduce_partials */
 int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* partial_counts, uint32_t* blocks, uint32_t* counters, uint32_t lds_budget);
-bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget);
+bool small_iteration_fits(int layout, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget);
 inline uint32_t lds_budget_of(const kmx_exec_params* exec, const DeviceInfo& dev)
 {
 	return exec->shared_mem_bytes && exec->shared_mem_bytes < dev.lds_bytes ? exec->shared_mem_bytes : dev.lds_bytes;

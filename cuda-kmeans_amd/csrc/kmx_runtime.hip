@@ -219,7 +219,7 @@ namespace kmx {
 
 int dispatch_assign(int variant, const AssignArgs& a, kmx_exec_params* exec, Workspace* ws, const DeviceInfo& dev, int* chosen)
 {
-	if (variant == KMX_ASSIGN_BEST && !a.ranking_only && small_assign_fits<float>(a.dim, a.k, a.n, lds_budget_of(exec, dev))) {
+	if (variant == KMX_ASSIGN_BEST && !a.ranking_only && small_assign_fits<float>(a.layout, a.dim, a.k, a.n, lds_budget_of(exec, dev))) {
 		/* small inputs: the serial arithmetic for every pair in one launch (small.hip) */
 		g_last_assign_variant = KMX_ASSIGN_BASE;
 		if (chosen) *chosen = KMX_ASSIGN_BASE;
@@ -735,7 +735,7 @@ int kmx_fused_f32(int variant,
 		if (rc) return rc;
 		AssignArgs a{ data, layout, stride, means_in, layout_means, stride_means, ws->fused_assignment, dim, k, n };
 		UpdateArgs small{ data, layout, stride, ws->fused_assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
-		if (small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) return launch_iteration_small(a, small, exec, ws, *dev);
+		if (small_iteration_fits(layout, dim, k, n, lds_budget_of(exec, *dev))) return launch_iteration_small(a, small, exec, ws, *dev);
 		return launch_fused_small(a, means_out, cluster_sizes, 0, exec, ws, *dev);
 	}
 	return two_passes(data, layout, stride, means_in, means_out, layout_means, stride_means, ws->fused_assignment, cluster_sizes, dim, k, n, exec);
@@ -765,7 +765,7 @@ int kmx_iteration_f32(const float* data, int layout, size_t stride,
 		rc = workspace(&ws);
 		if (rc) return rc;
 		UpdateArgs u{ data, layout, stride, assignment, means_out, layout_means, stride_means, cluster_sizes, dim, k, n };
-		if (small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) {
+		if (small_iteration_fits(layout, dim, k, n, lds_budget_of(exec, *dev))) {
 			AssignArgs small{ data, layout, stride, means_in, layout_means, stride_means, assignment, dim, k, n };
 			g_last_iteration_passes = 1;
 			return launch_iteration_small(small, u, exec, ws, *dev);
@@ -779,7 +779,7 @@ int kmx_iteration_f32(const float* data, int layout, size_t stride,
 	const DeviceInfo* dev = nullptr;
 	int rc = device_info(&dev);
 	if (rc) return rc;
-	if (n > 0 && small_iteration_fits(dim, k, n, lds_budget_of(exec, *dev))) {
+	if (n > 0 && small_iteration_fits(layout, dim, k, n, lds_budget_of(exec, *dev))) {
 		if ((rc = check_layout("kmx_iteration_f32", "data", layout, stride, n, dim))) return rc;
 		if ((rc = check_layout("kmx_iteration_f32", "means", layout_means, stride_means, k, dim))) return rc;
 		Workspace* ws = nullptr;

@@ -495,7 +495,7 @@ update_small_kernel(const F* __restrict__ data, size_t stride, const uint32_t* _
 }
 
 template <typename F>
-bool small_assign_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget) { return small_assign_accepts(sizeof(F), dim, k, n, lds_budget); }
+bool small_assign_fits(int layout, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget) { return small_assign_accepts(sizeof(F), layout == KMX_SOA, dim, k, n, lds_budget); }
 
 template <typename F, bool SUMS>
 static int launch_assign_small_t(const F* data, int layout, size_t stride, const F* means, int layout_means, size_t stride_means, uint32_t* assignment,
@@ -531,7 +531,7 @@ int launch_assign_small_sums(const AssignArgs& a, float* partial, uint32_t* part
 	return launch_assign_small_t<float, true>(a.data, a.layout, a.stride, a.means, a.layout_means, a.stride_means, a.assignment, a.dim, a.k, a.n,
 	                                          counters, partial, partial_counts, blocks, lds_budget);
 }
-bool small_iteration_fits(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget) { return small_iteration_accepts(dim, k, n, lds_budget); }
+bool small_iteration_fits(int layout, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget) { return small_iteration_accepts(layout == KMX_SOA, dim, k, n, lds_budget); }
 
 /*
  * The members of a cluster come from one compute unit, so the largest cluster sets the time: everything in one cluster is
@@ -584,7 +584,7 @@ int launch_update_small(const F* data, int layout, size_t stride, const uint32_t
 }
 
 #define KMX_SMALL_INSTANCES(F)                                                                                                                                   \
-	template bool small_assign_fits<F>(uint32_t, uint32_t, uint32_t, uint32_t);                                                                                  \
+	template bool small_assign_fits<F>(int, uint32_t, uint32_t, uint32_t, uint32_t);                                                                             \
 	template bool small_update_fits<F>(uint32_t, uint32_t, uint32_t, uint32_t, const DeviceInfo&);                                                               \
 	template int launch_assign_small<F>(const F*, int, size_t, const F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, uint32_t); \
 	template int launch_update_small<F>(const F*, int, size_t, const uint32_t*, F*, int, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, bool, uint32_t*, const DeviceInfo&);

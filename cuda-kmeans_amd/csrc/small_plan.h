@@ -40,31 +40,38 @@ inline uint32_t assign_small_lds(uint32_t value_bytes, uint32_t dim, uint32_t k,
 
 /*
  * Every pair costs 3 dim operations and about 30 to compare and keep, four cycles each on a SIMD; a work-group of 64 points keeps one
- * compute unit, so fewer than 256 of them leave units idle. Us per iteration near the line, these kernels / the general path: N = 40000, d = 32, k = 100
- * (effort 504 million) 28.7 / 40.3; N = 32768, d = 32, k = 128 (528) 27.1 / 31.5; N = 65536, d = 16, k = 100 (511) 27.2 / 32.0; N = 50000, d = 16, k = 128 (499)
- * 29.9 / 28.3; N = 65536, d = 8, k = 200 (708) 33.8 / 29.3. Wider rows, per assignment: N = 65536, d = 64, k = 50 (727) 20.4 / 22.6; N = 40000, d = 64, k = 80
- * (710) 20.2 / 21.7; N = 20000, d = 64, k = 200 (888) 32.1 / 22.7. Doubles: twice 450 million.
+ * compute unit, so fewer than 256 of them leave units idle. The line is 450 million, 530 million where small_more says so, and three halves of either for more than 32 dimensions.
+ * Between the two, 2145 shapes, these kernels in shares of the general path's time: work-groups a little more than 256, whose second
+ * round is nearly empty, 1.0 to 1.75 (N = 17391, d = 14, k = 420 34.6 / 24.2 us; N = 19340, d = 42, k = 261 38.4 / 21.9); else rows of 5 to 16 floats 0.85 to 1.32, 1.08 in the mean; of up to
+ * 4 0.76 to 1.0, of 17 to 32 0.59 to 1.05 (N = 40000, d = 32, k = 100 28.7 / 40.3 us per iteration), wider 0.82 to 1.56, 1.1 in the mean; columns, 5 to 8 of them 0.89 to 1.11, 9 to 16
+ * 0.76 to 1.01, 129 to 192 0.58 to 0.96, others beyond 32 0.86 to 1.58. Doubles: twice 450 million.
  * From 65536 points on the work-groups run in rounds and the general path's larger ones are ahead.
  */
 constexpr uint32_t SMALL_MAX_POINTS = 1u << 16;
-constexpr uint64_t SMALL_EFFORT = 530000000, SMALL_EFFORT_DOUBLES = 450000000; /* (doubles, N = 56478, d = 56, k = 128, 475: 87 us per iteration, general path 54) */
+constexpr uint64_t SMALL_EFFORT = 450000000, SMALL_EFFORT_MORE = 530000000; /* (doubles, N = 56478, d = 56, k = 128, 475: 87 us per iteration, general path 54) */
+/* `columns`: SoA points */
+constexpr bool small_more(bool columns, uint32_t dim, uint32_t n)
+{
+	if (dim > 32) return columns && dim > 128 && dim <= 192;
+	return columns ? (dim > 16 && n > 20480) || (n > 24576 && (dim <= 4 || dim > 8)) : n > 24576 && (dim <= 4 || dim > 16);
+}
 /* what the rule leaves for the static arrays: those of every work-group of eight wavefronts fit; one of 16 is taken only where its own do (small_shape) */
 constexpr uint32_t small_static_room(uint32_t value_bytes) { return SMALL_THREADS / SMALL_WAVE * SMALL_POINTS * (value_bytes + 4) + SMALL_POINTS * 4 + 64; }
 constexpr bool small_static_fits(uint32_t value_bytes, uint32_t tile, uint32_t points) { return small_static_bytes(value_bytes, tile, points, SMALL_THREADS) <= small_static_room(value_bytes); }
 static_assert(small_static_fits(4, 1, 64) && small_static_fits(4, 2, 64) && small_static_fits(4, 1, 32) && small_static_fits(4, 2, 32) &&
               small_static_fits(8, 1, 64) && small_static_fits(8, 2, 64) && small_static_fits(8, 1, 32) && small_static_fits(8, 2, 32), "eight wavefronts");
 
-inline bool small_assign_accepts(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
+inline bool small_assign_accepts(uint32_t value_bytes, bool columns, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
 	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
 	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
-	const uint64_t limit = (value_bytes == 8 ? 2 * SMALL_EFFORT_DOUBLES : SMALL_EFFORT) * (dim > 32 ? 3 : 2) / 2;
+	const uint64_t limit = (value_bytes == 8 ? 2 * SMALL_EFFORT : small_more(columns, dim, n) ? SMALL_EFFORT_MORE : SMALL_EFFORT) * (dim > 32 ? 3 : 2) / 2;
 	return effort <= limit && assign_small_lds(value_bytes, dim, k, SMALL_POINTS, false) + small_static_room(value_bytes) <= lds_budget;
 }
 /* floats, points added up too (the partial sums of all work-groups are written and read once) */
-inline bool small_iteration_accepts(uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
+inline bool small_iteration_accepts(bool columns, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
-	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * ((n + SMALL_POINTS - 1) / SMALL_POINTS) <= (2u << 20) && small_assign_accepts(4, dim, k, n, lds_budget) &&
+	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * ((n + SMALL_POINTS - 1) / SMALL_POINTS) <= (2u << 20) && small_assign_accepts(4, columns, dim, k, n, lds_budget) &&
 	       assign_small_lds(4, dim, k, SMALL_POINTS, true) + small_static_room(4) <= lds_budget;
 }
 
