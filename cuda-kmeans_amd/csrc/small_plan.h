@@ -80,7 +80,9 @@ inline bool small_iteration_accepts(bool columns, uint32_t dim, uint32_t k, uint
  * N = 5000, d = 32, k = 100 16.5 / 14.5; N = 10240, d = 20, k = 128 16.4 / 16.6: twice the partial sums). One work-group per compute unit at most: 16
  * wavefronts each, whose waits for the LDS others cover (eight / 16: N = 10240, d = 20, k = 128 16.4 / 15.2; N = 16384 15.9 / 15.0); with two, the waits
  * are covered already (N = 20000, d = 100, k = 30, SoA 23.3 / 26.7; d = 8, k = 30 12.7 / 15.1; AoS d = 20, k = 100 20.0 / 19.8; N = 32768, d = 8, k = 64 13.6 / 14.6).
- * 16 wavefronts have twice as many candidates in LDS, which rows of around 200 doubles leave no room for: eight there.
+ * 16 wavefronts have twice as many candidates in LDS, which rows of around 200 doubles leave no room for: eight there. Candidates of doubles have 16 bytes, and merging twice as
+ * many costs more than the waits unless there are many centroids (1368 shapes of 8193 to 16384 points, 16 wavefronts in shares of the time of eight: 13 to 200 centroids 0.95 to 1.24, 1.07
+ * in the mean, more than that in up to 64 dimensions 0.92 to 1.10, 0.97 in the mean, beyond 0.99 to 1.06; up to 12 centroids 0.94 to 1.04 in up to 16 dimensions, beyond 0.96 to 1.24).
  */
 constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 256 * SMALL_POINTS;
 
@@ -90,7 +92,8 @@ inline SmallShape small_shape(uint32_t value_bytes, uint32_t dim, uint32_t k, ui
 {
 	const uint32_t tile = k > SMALL_FEW_CENTROIDS ? 2 : 1, points = n <= SMALL_HALF_POINTS ? SMALL_POINTS / 2 : SMALL_POINTS;
 	const uint32_t lds = assign_small_lds(value_bytes, dim, k, points, sums);
-	const bool wide = n > SMALL_HALF_POINTS && n <= SMALL_WIDE_POINTS && lds + small_static_bytes(value_bytes, tile, points, SMALL_WIDE_THREADS) <= lds_budget;
+	const bool many = value_bytes == 4 || (k > 200 && dim <= 64) || (k <= SMALL_FEW_CENTROIDS && dim <= 16);
+	const bool wide = many && n > SMALL_HALF_POINTS && n <= SMALL_WIDE_POINTS && lds + small_static_bytes(value_bytes, tile, points, SMALL_WIDE_THREADS) <= lds_budget;
 	return SmallShape{ tile, points, wide ? SMALL_WIDE_THREADS : SMALL_THREADS, lds };
 }
 inline uint32_t assign_small_max_blocks(uint32_t n) { return n <= SMALL_HALF_POINTS ? (n + SMALL_POINTS / 2 - 1) / (SMALL_POINTS / 2) : (n + SMALL_POINTS - 1) / SMALL_POINTS; }

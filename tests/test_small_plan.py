@@ -12,6 +12,7 @@ SOURCE = """
 using namespace kmx;
 /* number of accepted shapes, and of those whose launch asks for more than the budget; always_wide: as if 16 wavefronts were taken whatever they need */
 extern "C" int accepts(uint32_t value_bytes, int columns, uint32_t dim, uint32_t k, uint32_t n) { return small_assign_accepts(value_bytes, columns != 0, dim, k, n, 160 * 1024); }
+extern "C" uint32_t threads(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t n) { return small_shape(value_bytes, dim, k, n, false, 160 * 1024).threads; }
 extern "C" void count(uint32_t value_bytes, int columns, int sums, uint32_t budget, int always_wide, uint64_t* accepted, uint64_t* beyond, uint64_t* wide)
 {
 	*accepted = *beyond = *wide = 0;
@@ -75,3 +76,9 @@ def test_work_groups_a_little_more_than_compute_units_go_to_the_general_path(lib
 @pytest.mark.parametrize("columns,dim,k,n", [(0, 32, 100, 40000), (0, 4, 190, 65536), (1, 150, 24, 65536)])
 def test_shapes_beyond_the_lower_line_that_stay(library, columns, dim, k, n):
     assert library.accepts(4, columns, dim, k, n)
+
+
+# doubles, us of 16 wavefronts / eight: 10.2 / 8.3, 6.3 / 5.1; 30.8 / 32.0 and more with many centroids
+@pytest.mark.parametrize("dim,k,n,threads", [(34, 46, 15066, 512), (60, 8, 12485, 512), (36, 46, 11715, 512), (20, 387, 14211, 1024), (4, 8, 15075, 1024)])
+def test_doubles_take_16_wavefronts_for_many_centroids(library, dim, k, n, threads):
+    assert library.threads(8, dim, k, n) == threads
