@@ -1003,7 +1003,12 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 	auto resident = [&](Rank16Copies copies, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, copies) + rank16_list_bytes(KB, a.layout, copies, entries) <= budget; };
 	Rank16Copies copies = w.copy_all || a.layout == KMX_AOS ? RANK16_EXCHANGED : RANK16_LISTED;
 	if (KB < 12 && w.copy_all && a.layout == KMX_SOA && !resident(copies, rank16_list_least(KB)) && resident(RANK16_DIRECT, rank16_list_least(KB))) copies = RANK16_DIRECT;
-	const bool stream_mode = !resident(copies, rank16_list_least(KB));
+	/*
+	 * Without room to exchange rows, SoA points have a tile more in LDS. Beyond 128 dimensions that is too dear: what is left holds short lists, where the streamed form
+	 * has two work-groups of four wavefronts and whole ones (us per assignment, resident -> streamed: N = 192644, d = 133, k = 375 110 -> 79; N = 56454, d = 169, k = 368
+	 * 66 -> 49; N = 28000, d = 204, k = 274 1.13 of the time; up to 128 dimensions 0.90 to 1.06).
+	 */
+	const bool stream_mode = !resident(KB >= 12 && copies == RANK16_LISTED ? RANK16_EXCHANGED : copies, rank16_list_least(KB));
 	w.chunk_tiles = tiles;
 	w.list_entries = RANK16_LIST_MOST;
 	while (!stream_mode && !resident(copies, w.list_entries)) --w.list_entries;

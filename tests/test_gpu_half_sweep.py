@@ -270,3 +270,27 @@ def test_iterations_on_soa_points_with_few_centroids(km, orc, gpu, dim, k, n):
 def test_columns_read_by_wavefronts_without_points(km, orc, gpu, dim, k, n):
     """Numbers of points that leave one to seven wavefronts of the last unit without any, centroids in LDS and streamed: those read the last point again."""
     test_listed_rows_of_soa_points_are_copied_behind_the_sweep(km, orc, gpu, dim, k, n, 0.12)
+
+
+# rows of 12 and 16 blocks: as many centroids as are kept in LDS, one more, and as many as would just fit without room to exchange rows
+@pytest.mark.parametrize("dim,k,streamed", [(150, 352, False), (150, 353, True), (185, 384, True), (250, 256, False), (250, 257, True), (200, 288, True)])
+def test_wide_soa_rows_around_as_many_centroids_as_fit(km, orc, gpu, dim, k, streamed):
+    n = 4099
+    rng = np.random.default_rng(dim + k)
+    means = rng.normal(size=(k, dim)).astype(np.float32) * np.float32(3)
+    rows = (means[rng.integers(0, k, n)] + rng.normal(size=(n, dim)) * 0.5).astype(np.float32)
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, 1))
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 0))
+    a = km.DeviceBuffer(4 * n); a.write(np.full(n, 0xFFFFFFF1, np.uint32))
+    ex = km.ExecParams()
+    km.set_two_level_sweep(2)
+    try:
+        km.assign(km.ASSIGN_MFMA_BF16X3, d, 1, n, m, 0, dim, a, dim, k, n, ex)
+        km.sync()
+    finally:
+        km.set_two_level_sweep(1)
+    assert np.array_equal(a.read(np.uint32, n), want)
+    assert ex.block_count == -(-n // (256 if streamed else 512))        # units of four or of eight wavefronts
+    for b in (d, m, a):
+        b.free()
