@@ -552,11 +552,13 @@ fold_ranges64_kernel(const float* __restrict__ partial, const uint32_t* __restri
  * N = 100000, d = 256, k = 1000 34.7 -> 33.4, but d = 200, k = 600 28 -> 31; N = 190000, d = 148, k = 354 34 -> 37. More,
  * of whose clusters the sorted chunks write 32 sets of partial sums and more: N = 100000, d = 300, k = 2000 71 -> 45; N = 131071, d = 512, k = 1000 79 -> 60, k = 600 65 -> 58, k = 400 57 -> 59. Half of the points in
  * one cluster, N = 1M, d = 256, k = 1024 448 -> 216; all of them 702 -> 230; sorted by cluster 292 -> 225. Slices of 16: N = 1M, d = 160, k = 600 128.7 -> 128.3,
- * N = 300000, d = 144, k = 1000 37.6 -> 40.7: stay.
+ * N = 300000, d = 144, k = 1000 37.6 -> 40.7: stay. More than 256 dimensions, few points: the sorted chunks' sums are fewer (802 shapes of 1 to 26 million floats; N = 8830, d = 372, k = 606
+ * 18.1 -> 22.6, N = 16343, d = 304, k = 717 19.9 -> 23.3, but N = 6706, d = 400, k = 1585 27.9 -> 21.2): ranges from 280000 sums or 5 million floats on; below 1.10 in the mean, from there 0.75.
  */
 static bool ranges64_pays(uint32_t dim, uint32_t k, uint32_t n, bool planned)
 {
-	return !planned && k >= 600 && (dim > 256 || (size_t)n * dim >= (3u << 23));
+	const size_t floats = (size_t)n * dim;
+	return !planned && k >= 600 && (dim > 256 ? floats >= 5000000 || (size_t)k * dim >= 280000 : floats >= (3u << 23));
 }
 
 struct Ranges64Plan { uint32_t width, slices, log_ranges, groups, lds_bytes; };

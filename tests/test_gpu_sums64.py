@@ -373,3 +373,27 @@ def test_many_clusters_of_many_points_without_allocation(km, gpu):
 @pytest.mark.parametrize("dim,k,n", [(100, 300, 399999), (100, 300, 400001), (105, 600, 380001), (105, 600, 381001), (97, 1000, 300001), (4, 2000, 300001), (8, 2000, 500001), (11, 1105, 331499), (11, 1105, 331500), (6, 2000, 400001)])
 def test_doubles_beside_the_lines(km, gpu, dim, k, n):
     check(km, dim, k, n, np.float64, outside=True)
+
+
+def work_groups(km, dim, k, n, dtype=np.float32, stride=None):
+    """Of an update of AoS points (all in cluster 0)."""
+    stride = stride or dim
+    item = np.dtype(dtype).itemsize
+    bufs = [km.DeviceBuffer(b) for b in (item * n * stride, 4 * n, item * k * dim, 4 * k)]
+    for b in bufs:
+        b.zero()
+    ex = km.ExecParams()
+    km.update(km.UPDATE_ATOMIC_SHM, bufs[0], AOS, stride, bufs[1], bufs[2], AOS, dim, bufs[3], dim, k, n, ex, dtype)
+    km.sync()
+    for b in bufs:
+        b.free()
+    return ex.block_count
+
+
+# both sides of the lines between ranges of clusters and the sorted chunks (us, ranges / sorted chunks: 22.6 / 18.1, 23.3 / 19.9; 21.2 / 27.9)
+@pytest.mark.parametrize("dim,k,n,ranges", [(372, 606, 8830, False), (304, 717, 16343, False), (304, 717, 16448, True), (400, 1585, 6706, True), (400, 700, 6706, True), (400, 699, 6706, False)])
+def test_wide_rows_of_few_points(km, gpu, dim, k, n, ranges):
+    check(km, dim, k, n, np.float32, outside=True)
+    slices = -(-dim // 32)
+    chunk = -(-(-(-n // (gpu.compute_units // slices))) // 1024) * 1024
+    assert (work_groups(km, dim, k, n) != -(-n // chunk) * slices) == ranges
