@@ -153,7 +153,9 @@ static bool sorted_pays(uint32_t dim, uint32_t k, uint32_t n, uint32_t width, ui
  * 54 + 54 + 52 60, 64 + 64 + 32 49.5, sorted chunks 53; N = 1.25M 180, 156, 164). Rows of up to 48 floats go in slices of 16, doubles in slices of 32 or two, even where the whole row fits (d = 40,
  * k = 300: 34, whole 37; doubles, N = 2M, d = 32, k = 500: 103, 113): the sums to write are fewer. But from some 60 million floats on, which the memory-side cache
  * does not hold, a row that begins anywhere is read once (slices of 16 / whole: d = 36, k = 18, N = 1.6M 43.6 / 42.8, N = 1.9M 64.6 / 53.4, N = 2.8M 113 / 86; d = 18 58.8 / 58.6
- * at 68 million, 81 / 75 at 80; d = 44, N = 1.3M 41 / 44, N = 1.5M 64 / 53; d = 48, k = 200, N = 3.3M 135 / 129; d = 32, N = 5M 128 / 126). Doubles whose sums do not fit as a whole: 16 at a time (N = 500000,
+ * at 68 million, 81 / 75 at 80; d = 44, N = 1.3M 41 / 44, N = 1.5M 64 / 53; d = 48, k = 200, N = 3.3M 135 / 129; d = 32, N = 5M 128 / 126). Of rows with a gap
+ * of 16 floats and more behind them, which share fewer lines, the memory that they span counts, from 45 million floats on where the last slice has eight coordinates and fewer (stride dim + 32:
+ * d = 17, N = 1.6M 72 / 55; d = 20, N = 1.5M 65 / 52; d = 34, N = 1.4M, stride 50, 72 / 51; d = 20, N = 577000 level), else from 75 (d = 26, N = 1.2M 1.1; d = 42, N = 1.1M 1.07; d = 30 0.98). Doubles whose sums do not fit as a whole: 16 at a time (N = 500000,
  * d = 128, k = 1024: 123, slices of 19 142, sums of ranges of clusters 204), equal where the last would be narrow (N = 1M, d = 33, k = 1000: 73,
  * 16 + 16 + 1 86, ranges 77), eight at a time where rows are odd multiples of 32 bytes and short (N = 1M, d = 24, k = 1200: 43, 12 + 12 47, ranges 53).
  * Seven slices leave an eighth of the compute units over: where rows begin inside lines and the caches do not hold them, the ranges (d = 100, k = 600: N = 500000 103, ranges 91,
@@ -173,7 +175,7 @@ static bool sorted_pays(uint32_t dim, uint32_t k, uint32_t n, uint32_t width, ui
 struct Sums64Plan { uint32_t width, slices, copies, chunks, chunk_points, lds_bytes; };
 constexpr uint32_t SUMS64_SLICES = 10;
 
-static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint32_t budget, uint32_t compute_units, Sums64Plan* plan)
+static bool plan_sums64(uint32_t dim, size_t stride, uint32_t k, uint32_t n, bool doubles, uint32_t budget, uint32_t compute_units, Sums64Plan* plan)
 {
 	auto bytes = [&](uint32_t width) -> uint64_t { return ((uint64_t)k + 1) * (8 * width + 4); };
 	auto slices_of = [&](uint32_t width) -> uint32_t { return (dim - 1) / width + 1; };
@@ -184,7 +186,8 @@ static bool plan_sums64(uint32_t dim, uint32_t k, uint32_t n, bool doubles, uint
 	/* doubles whose sums do not fit as a whole */
 	const bool parts = doubles && bytes(dim) > budget, eights = parts && dim <= 56 && dim % 4 == 0 && dim % 16 != 0;
 	if (parts && slices_of(16) == 7 && dim % 16 != 0 && (uint64_t)n * dim >= 40000000) return false;
-	const bool whole_row = !doubles && dim > 16 && dim <= 48 && bytes(dim) <= budget && (uint64_t)n * dim >= 60000000;
+	const bool beyond_caches = (uint64_t)n * dim >= 60000000 || (stride >= dim + 16 && n * std::min<uint64_t>(stride, dim + 32) >= ((dim - 1) % 16 < 8 ? 45000000 : 75000000));
+	const bool whole_row = !doubles && dim > 16 && dim <= 48 && bytes(dim) <= budget && beyond_caches;
 	const uint32_t fewest = dim <= 16 || whole_row ? 1 : parts ? slices_of(eights ? 8 : 16) : doubles ? std::max<uint32_t>(2, slices_of(32)) : dim <= 48 ? slices_of(16) : slices_of(SUMS64_LANES);
 	uint32_t width = 0;
 	for (uint32_t slices = fewest; slices <= SUMS64_SLICES && (width == 0 || width > 16); ++slices) {
@@ -661,12 +664,13 @@ int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_
 	float* partials = nullptr;
 	const bool columns = layout == KMX_SOA;
 	if (n == 0 || (columns && ws && ws->fixed)) return KMX_OK; /* (SoA points are taken there whatever their number of partial sums) */
-	bool planned = (columns ? plan_columns64 : plan_sums64)(dim, k, n, sizeof(F) == 8, lds_budget_of(exec, dev), dev.compute_units, &p);
+	const uint32_t budget = lds_budget_of(exec, dev);
+	bool planned = columns ? plan_columns64(dim, k, n, sizeof(F) == 8, budget, dev.compute_units, &p) : plan_sums64(dim, stride, k, n, sizeof(F) == 8, budget, dev.compute_units, &p);
 	/* (the sorted chunks' partial sums may be several times as many, and would not fit the scratch array) */
 	if (planned && !columns && sizeof(F) == 4 && !ws->fixed && !launches_recorded()) planned = !sorted_pays(dim, k, n, p.width, p.slices, p.chunks, dev.compute_units);
 	if constexpr (sizeof(F) == 4) {
 		Ranges64Plan r;
-		if (!columns && ranges64_pays(dim, k, n, planned) && plan_ranges64(dim, k, n, lds_budget_of(exec, dev), dev.compute_units, &r)) {
+		if (!columns && ranges64_pays(dim, k, n, planned) && plan_ranges64(dim, k, n, budget, dev.compute_units, &r)) {
 			const int rc = place_sums<F>(ws, ranges64_words(r, dim, k), &partials);
 			if (rc) return rc;
 			*done = true;
@@ -675,6 +679,14 @@ int launch_update_sums64(const F* data, int layout, size_t stride, const uint32_
 		}
 	}
 	if (!planned) return KMX_OK;
+	if (sizing_only() && !columns && sizeof(F) == 4) {
+		/* the stride may decide whether rows go as a whole, and the room is for calls with any */
+		Sums64Plan spread;
+		if (plan_sums64(dim, (size_t)dim + 32, k, n, false, budget, dev.compute_units, &spread)) {
+			const int rc = reserve_partials(ws, sums64_words(spread, dim, k, sizeof(F)));
+			if (rc) return rc;
+		}
+	}
 	const size_t sums = (size_t)p.chunks * k * dim;
 	int rc = place_sums<F>(ws, sums64_words(p, dim, k, sizeof(F)), &partials);
 	if (rc || !partials) return rc;

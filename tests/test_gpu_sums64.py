@@ -397,3 +397,28 @@ def test_wide_rows_of_few_points(km, gpu, dim, k, n, ranges):
     slices = -(-dim // 32)
     chunk = -(-(-(-n // (gpu.compute_units // slices))) // 1024) * 1024
     assert (work_groups(km, dim, k, n) != -(-n // chunk) * slices) == ranges
+
+
+# rows with a gap behind them, on both sides of the lines from which they go as a whole: a work-group per compute unit, not a third or half of it per slice
+@pytest.mark.parametrize("dim,k,stride,whole", [(17, 52, 49, True), (20, 41, 36, True), (20, 41, 35, False), (34, 66, 50, True), (42, 30, 74, True), (26, 40, 46, False)])
+def test_rows_with_gaps_behind_them(km, gpu, dim, k, stride, whole):
+    line = -(-(45000000 if (dim - 1) % 16 < 8 else 75000000) // stride)
+    n = line if whole or stride < dim + 16 else line - 1
+    rng = np.random.default_rng(dim + k)
+    member = rng.integers(0, k, size=n).astype(np.uint32)
+    rows = np.full((n, stride), np.nan, np.float32)
+    rows[:, :dim] = rng.integers(-8, 9, size=(n, dim), dtype=np.int8)
+    d = km.DeviceBuffer(rows.nbytes); d.write(rows.ravel())
+    a = km.DeviceBuffer(4 * n); a.write(member)
+    m = km.DeviceBuffer(4 * k * dim); s = km.DeviceBuffer(4 * k)
+    ex = km.ExecParams()
+    km.update(km.UPDATE_ATOMIC_SHM, d, AOS, stride, a, m, AOS, dim, s, dim, k, n, ex)
+    counts = np.bincount(member, minlength=k)
+    want = np.stack([np.bincount(member, weights=rows[:, q], minlength=k) for q in range(dim)], axis=1)   # (whole numbers: every sum is exact)
+    assert np.array_equal(s.read(np.uint32, k), counts)
+    assert np.array_equal(m.read(np.float32, k * dim).reshape(k, dim), want.astype(np.float32) / counts.astype(np.float32)[:, None])
+    slices = 1 if whole else -(-dim // 16)
+    chunk = -(-n // (gpu.compute_units // 8 // slices * 8) // 64) * 64                 # whole wavefronts of points
+    assert ex.block_count == -(-n // chunk) * slices
+    for b in (d, a, m, s):
+        b.free()

@@ -138,3 +138,23 @@ def test_reserved_room_is_enough_for_columns_of_any_stride(km, orc, gpu, dim, k,
         d.free()
     for b in (m, a, out, sizes):
         b.free()
+
+
+@pytest.mark.parametrize("dim,k,n", [(17, 1000, 920000), (34, 66, 900001)])
+def test_reserved_room_is_enough_for_rows_with_gaps(km, gpu, dim, k, n):
+    """A gap behind the rows makes more of them go as a whole, with more partial sums: after the reservation those do not allocate either."""
+    stride = dim + 33
+    d = km.DeviceBuffer(4 * n * stride); d.zero()
+    a = km.DeviceBuffer(4 * n); a.zero()
+    m = km.DeviceBuffer(4 * k * dim); s = km.DeviceBuffer(4 * k)
+    call = lambda: (km.update(km.UPDATE_ATOMIC_SHM, d, AOS, stride, a, m, AOS, dim, s, dim, k, n), km.sync())
+    call()
+    km.check(km.hip_lib().kmx_shutdown())
+    km.reserve(km.ASSIGN_BEST, km.UPDATE_ATOMIC_SHM, AOS, AOS, dim, k, n)
+    km.sync()
+    before = device_memory_in_use()
+    call()
+    assert device_memory_in_use() == before
+    assert s.read(np.uint32, k)[0] == n
+    for b in (d, a, m, s):
+        b.free()
