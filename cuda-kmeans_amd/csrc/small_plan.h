@@ -41,7 +41,7 @@ inline uint32_t assign_small_lds(uint32_t value_bytes, uint32_t dim, uint32_t k,
 /*
  * Every pair costs 3 dim operations and about 30 to compare and keep, four cycles each on a SIMD; a work-group of 64 points keeps one
  * compute unit, so fewer than 256 of them leave units idle. The line is 450 million, 530 million where small_more says so, and three halves of either for more than 32 dimensions.
- * Between the two, 2145 shapes, these kernels in shares of the general path's time: work-groups a little more than 256, whose second
+ * Between the two, 3236 shapes, these kernels in shares of the general path's time: up to 256 work-groups 0.43 to 1.13, 0.69 in the mean; a little more of them, whose second
  * round is nearly empty, 1.0 to 1.75 (N = 17391, d = 14, k = 420 34.6 / 24.2 us; N = 19340, d = 42, k = 261 38.4 / 21.9); else rows of 5 to 16 floats 0.85 to 1.32, 1.08 in the mean; of up to
  * 4 0.76 to 1.0, of 17 to 32 0.59 to 1.05 (N = 40000, d = 32, k = 100 28.7 / 40.3 us per iteration), wider 0.82 to 1.56, 1.1 in the mean; columns, 5 to 8 of them 0.89 to 1.11, 9 to 16
  * 0.76 to 1.01, 129 to 192 0.58 to 0.96, others beyond 32 0.86 to 1.58. Doubles: twice 450 million.
@@ -52,6 +52,7 @@ constexpr uint64_t SMALL_EFFORT = 450000000, SMALL_EFFORT_MORE = 530000000; /* (
 /* `columns`: SoA points */
 constexpr bool small_more(bool columns, uint32_t dim, uint32_t n)
 {
+	if (n <= 256 * SMALL_POINTS) return true;
 	if (dim > 32) return columns && dim > 128 && dim <= 192;
 	return columns ? (dim > 16 && n > 20480) || (n > 24576 && (dim <= 4 || dim > 8)) : n > 24576 && (dim <= 4 || dim > 16);
 }

@@ -82,3 +82,10 @@ def test_shapes_beyond_the_lower_line_that_stay(library, columns, dim, k, n):
 @pytest.mark.parametrize("dim,k,n,threads", [(34, 46, 15066, 512), (60, 8, 12485, 512), (36, 46, 11715, 512), (20, 387, 14211, 1024), (4, 8, 15075, 1024)])
 def test_doubles_take_16_wavefronts_for_many_centroids(library, dim, k, n, threads):
     assert library.threads(8, dim, k, n) == threads
+
+
+# one work-group per compute unit: half of the general path's time and less
+@pytest.mark.parametrize("columns", [0, 1])
+@pytest.mark.parametrize("dim,k,n", [(2, 840, 3000), (4, 740, 8192), (20, 330, 16384), (90, 157, 5458), (254, 61, 8307)])
+def test_few_work_groups_stay(library, columns, dim, k, n):
+    assert library.accepts(4, columns, dim, k, n)
