@@ -14,17 +14,16 @@ namespace kmx {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-/* SoA: which rows go out as AoS, and how (rank16_copy, copy_listed); AoS: EXCHANGED, to nobody */
-enum Rank16Copies { RANK16_EXCHANGED, RANK16_DIRECT, RANK16_LISTED };
+/* SoA: which rows go out as AoS (copy_listed, rank16_copy): the listed points', or all of them; AoS: none */
+enum Rank16Copies { RANK16_NONE, RANK16_LISTED, RANK16_ALL };
 
 /*
  * Rows of up to 32 dimensions around resident centroids: three wavefronts on a SIMD, of which the third also covers the ends of the others'
  * sweeps. That takes tracking in fewer registers (RANK16_GROUPS). us per assignment (N = 2M, Gaussian mixture, centroids after two rounds), two wavefronts with
  * the snapshot -> three: d = 32, k = 1024 219 -> 204; d = 16 174 -> 150; d = 10, k = 100 74 -> 70. The same tracking with two: 220, 165, 78. Wider rows
- * would spill (N = 1M, d = 64, k = 512: 103 -> 114), and so does the copying of
- * all SoA points (d = 24, k = 256: 68.6 -> 69.6); of the listed ones only (SoA, d = 32, k = 1024 225 -> 215, around its first points 246 -> 230; N = 1M, d = 20, k = 300 70 -> 68).
+ * would spill (N = 1M, d = 64, k = 512: 103 -> 114). SoA: d = 32, k = 1024 225 -> 215, around its first points 246 -> 230; N = 1M, d = 20, k = 300 70 -> 68.
  */
-constexpr bool rank16_grouped(uint32_t kb, int layout, Rank16Copies copies) { return kb == 1 || (kb == 2 && (layout == KMX_AOS || copies == RANK16_LISTED)); }
+constexpr bool rank16_grouped(uint32_t kb) { return kb <= 2; }
 /*
  * Wavefronts of a work-group: otherwise eight around centroids in LDS. Where the centroids stream by (slots of a chunk of tiles that go round, filled by
  * requests straight to LDS, a barrier per chunk), rows of up to 128 dimensions keep that form with two chunks as large as fit, since the
@@ -34,7 +33,7 @@ constexpr bool rank16_grouped(uint32_t kb, int layout, Rank16Copies copies) { re
  * the matrix cores, and four slots of a tile (N = 1M, d = 256, k = 1024: 549, with eight wavefronts and two chunks of four tiles 569).
  * With chunks through registers and eight wavefronts for all widths: 656, 655, 480, 464.
  */
-constexpr uint32_t rank16_waves(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return stream && kb >= 12 ? 4 : !stream && rank16_grouped(kb, layout, copies) ? 12 : 8; }
+constexpr uint32_t rank16_waves(uint32_t kb, bool stream) { return stream && kb >= 12 ? 4 : !stream && rank16_grouped(kb) ? 12 : 8; }
 constexpr int RANK16_P = 2; /* point tiles per wavefront: an operand read serves two instructions */
 
 struct Rank16Args {
@@ -85,11 +84,11 @@ __host__ __device__ constexpr uint32_t rank16_slot_bytes(uint32_t kb, uint32_t t
 constexpr bool rank16_whole_columns(uint32_t kb, int layout) { return layout == KMX_SOA && (kb == 8 || kb == 16); }
 constexpr uint32_t RANK16_EXCHANGE = 256; /* words per wavefront in which the lanes exchange a block of a tile of points */
 constexpr bool rank16_shared_rows(uint32_t kb, int layout) { return layout == KMX_AOS && kb >= 12; }
-constexpr uint32_t rank16_exchange(uint32_t kb, int layout, Rank16Copies copies) { return rank16_shared_rows(kb, layout) || (layout == KMX_SOA && copies == RANK16_EXCHANGED) ? RANK16_EXCHANGE : 0; }
-constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, copies) + 4) * rank16_waves(kb, layout, stream, copies) + kb * KBLOCK) * 4 + 64; }
+constexpr uint32_t rank16_exchange(uint32_t kb, int layout, Rank16Copies copies) { return rank16_shared_rows(kb, layout) || copies == RANK16_ALL ? RANK16_EXCHANGE : 0; }
+constexpr uint32_t rank16_static_bytes(uint32_t kb, int layout, bool stream, Rank16Copies copies) { return ((2 * (stream ? RANK16_LIST_STREAMED : 0) + rank16_exchange(kb, layout, copies) + 4) * rank16_waves(kb, stream) + kb * KBLOCK) * 4 + 64; }
 /* the lists of a work-group around resident centroids, lying behind them */
-constexpr uint32_t rank16_list_bytes(uint32_t kb, int layout, Rank16Copies copies, uint32_t entries) { return rank16_waves(kb, layout, false, copies) * entries * 8; }
-constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true, RANK16_EXCHANGED) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
+constexpr uint32_t rank16_list_bytes(uint32_t kb, uint32_t entries) { return rank16_waves(kb, false) * entries * 8; }
+constexpr uint32_t rank16_least_bytes(uint32_t kb, int layout) { return rank16_static_bytes(kb, layout, true, layout == KMX_SOA ? RANK16_ALL : RANK16_NONE) + rank16_slots(kb) * rank16_slot_bytes(kb, 1); }
 
 /*
  * S for centroids whose coordinates are up to `far` from the frame and up to `size` from the origin, both of a sample: the power of two
@@ -230,21 +229,20 @@ __device__ __forceinline__ void rank16_exchanged() /* LDS keeps the order of a w
 }
 
 /*
- * SoA: rows go out as AoS, for the exact pass (coordinates of a listed point lie a cache line each apart) and whatever else reads single rows.
- * All of them on the way in, where somebody reads all (the update of an iteration): through LDS, so that four lanes store 64 consecutive bytes of
- * a row. `exchange`: RANK16_EXCHANGE words of this wavefront's. Where resident centroids leave no room for it a lane stores its 32 bytes as they
- * are (DIRECT): the centroids would have to stream by otherwise (N = 1M, d = 12, k = 4000 262 us, streamed 368; d = 40,
- * k = 1536 249, 283; d = 64, k = 1150 255, 295; with room for it, d = 64, k = 256, 170 through LDS, 183 without).
- * For the assignment alone the listed ones are enough (LISTED, see copy_listed in the kernel): writing as many bytes as are read, in the phase in which
+ * SoA: rows go out as AoS, for the exact pass (coordinates of a listed point lie a cache line each apart) and whatever else reads single rows: those of the
+ * listed points, behind the sweep (LISTED, see copy_listed in the kernel). Writing as many bytes as are read, in the phase in which
  * the matrix cores wait for the points, cost more than reading the columns' lines of the listed points once more from the memory-side
  * cache. us per assignment, all rows -> listed ones: N = 2M, d = 128, k = 1024, 9 % listed 854 -> 812 (without any copies 643), 1 % 808 -> 732; d = 32
  * 256 -> 222; N = 1M, d = 64, k = 500 162 -> 119; d = 90, k = 300 222 -> 157; N = 500000, d = 200, k = 1024 392 -> 331; nearly all listed (coordinates 0 or 1),
- * d = 64, k = 256 145 -> 89, d = 128, k = 512 193 -> 189.
+ * d = 64, k = 256 145 -> 89, d = 128, k = 512 193 -> 189; 1768 calls of up to 150000 points and 33 to 256 dimensions 0.96 in the mean, up to 1.22 where points that come together are
+ * listed and a work-group has no further points meanwhile (N = 52692, d = 237, k = 284).
+ * All of them (ALL), on the way in and through LDS, so that four lanes store 64 consecutive bytes of a row, where the update behind it reads whole rows: iterations
+ * with more centroids than fit a column's sums. `exchange`: RANK16_EXCHANGE words of this wavefront's. Otherwise a lane stores its 32 bytes as they are.
  */
-template <Rank16Copies COPIES>
+template <bool EXCHANGED>
 __device__ __forceinline__ void rank16_copy(const Rank16Args& w, const float (&v)[8], uint32_t tile_first, uint32_t kb, uint32_t lane, float* exchange)
 {
-	if (COPIES == RANK16_DIRECT) {
+	if (!EXCHANGED) {
 		const uint32_t pt = tile_first + lane % TILE, d = kb * KBLOCK + lane / TILE * 8;
 		if (pt >= w.n || d >= w.copy_stride) return;
 		float* to = w.copies + (size_t)pt * w.copy_stride + d;
@@ -409,15 +407,15 @@ __device__ __forceinline__ float rank16_both(float v)
  * instructions of the next (the fenced step). Otherwise one chain per tile whose tracking the partner wavefront of the SIMD covers.
  */
 template <int KB, int LD, bool STREAM, Rank16Copies COPIES>
-__global__ void __launch_bounds__(rank16_waves(KB, LD, STREAM, COPIES) * WAVE, rank16_waves(KB, LD, STREAM, COPIES) == 12 ? 3 : 2)
+__global__ void __launch_bounds__(rank16_waves(KB, STREAM) * WAVE, rank16_waves(KB, STREAM) == 12 ? 3 : 2)
 rank16_kernel(const Rank16Args w)
 {
-	constexpr uint32_t WAVES = rank16_waves(KB, LD, STREAM, COPIES), THREADS = WAVES * WAVE;
+	constexpr uint32_t WAVES = rank16_waves(KB, STREAM), THREADS = WAVES * WAVE;
 	constexpr int P = RANK16_P;
 	constexpr uint32_t TF = rank16_tile_floats<KB>();
 	constexpr bool PIPE = !STREAM && KB <= 4;
 	constexpr bool SHARED = rank16_shared_rows(KB, LD);
-	constexpr bool GROUPED = PIPE && rank16_grouped(KB, LD, COPIES);
+	constexpr bool GROUPED = PIPE && rank16_grouped(KB);
 	constexpr bool PREFETCH = PIPE && (KB == 1 || (KB == 2 && !GROUPED)); /* the next item's coordinates travel while the current one is swept */
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	__shared__ __attribute__((aligned(16))) float frame[KB * KBLOCK]; /* S m */
@@ -502,7 +500,8 @@ rank16_kernel(const Rank16Args w)
 	 * rows are requested (request_listed) ahead of the next points and stored
 	 * behind them (store_listed). Many of the 64: their tiles as a whole (copy_tiles).
 	 */
-	constexpr bool LISTED = LD == KMX_SOA && COPIES == RANK16_LISTED;
+	constexpr bool LISTED = COPIES == RANK16_LISTED;
+	static_assert(COPIES == RANK16_NONE ? LD == KMX_AOS : LD == KMX_SOA && (LISTED || STREAM), "all rows go out around centroids that stream by");
 	constexpr uint32_t LATE_TURNS = KB > 8 ? 2 : 1, LATE_EACH = KB * KBLOCK / 8 / LATE_TURNS, LATE_VEC = LATE_EACH % 4 == 0 ? 4 : 2, LATE_MANY = 24;
 	static_assert(P == 2 && LATE_EACH % LATE_VEC == 0, "whole stores");
 	uint64_t late = 0;
@@ -553,7 +552,7 @@ rank16_kernel(const Rank16Args w)
 				float v[8];
 				rank16_request<LD, SHARED, false>(v, from, w.stride, kb, lane, w.dim);
 				rank16_place<LD, SHARED>(v, kb, lane, w.dim);
-				rank16_copy<RANK16_DIRECT>(w, v, late_first + p * TILE, kb, lane, exchange);
+				rank16_copy<false>(w, v, late_first + p * TILE, kb, lane, exchange);
 			}
 		}
 		late = 0;
@@ -608,7 +607,7 @@ rank16_kernel(const Rank16Args w)
 				rank16_halves(v[0], v[1], kb, WHOLE ? KB * KBLOCK : dim);
 #pragma unroll
 				for (int p = 0; p < P; ++p) {
-					if (COPIES != RANK16_LISTED) rank16_copy<COPIES>(w, v[p], first + p * TILE, kb, lane, exchange);
+					if (COPIES == RANK16_ALL) rank16_copy<true>(w, v[p], first + p * TILE, kb, lane, exchange);
 					rank16_convert<SHARED>(b[p][kb], v[p], frame, scale, kb, lane, sums[p], exchange);
 					asm volatile("" : "+v"(b[p][kb]));
 					asm volatile("" : "+v"(sums[p].part[0]), "+v"(sums[p].low[0]));
@@ -637,7 +636,7 @@ rank16_kernel(const Rank16Args w)
 			__builtin_amdgcn_sched_barrier(0);
 			float (&v)[8] = raw[at % DEPTH];
 			if (!WHOLE) rank16_place<LD, SHARED>(v, kb, lane, dim);
-			if (LD == KMX_SOA && COPIES != RANK16_LISTED) rank16_copy<COPIES>(w, v, first + p * TILE, kb, lane, exchange);
+			if (COPIES == RANK16_ALL) rank16_copy<true>(w, v, first + p * TILE, kb, lane, exchange);
 			rank16_convert<SHARED>(b[p][kb], v, frame, scale, kb, lane, sums[p], exchange);
 			if (!SHARED) asm volatile("" : "+v"(b[p][kb]));
 			/* the sums exist here: left alone the compiler moves them behind the sweep and keeps the coordinates alive */
@@ -865,7 +864,6 @@ rank16_kernel(const Rank16Args w)
 #pragma unroll
 					for (int kb = 0; kb < KB; ++kb) {
 						rank16_place<LD, SHARED>(raw[p][kb], kb, lane, w.dim);
-						if (LD == KMX_SOA && COPIES != RANK16_LISTED) rank16_copy<COPIES>(w, raw[p][kb], first + p * TILE, kb, lane, exchange);
 						rank16_convert<SHARED>(b[p][kb], raw[p][kb], frame, scale, kb, lane, sums, exchange);
 					}
 					rank16_total<SHARED>(xx[p], xl[p], sums, lane);
@@ -1000,31 +998,29 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 {
 	const uint32_t tile_bytes = (rank16_tile_floats<KB>() + NORM_TILE) * 4, tiles = w.kp / TILE, budget = lds_budget_of(exec, dev);
 	if (budget < rank16_least_bytes(KB, a.layout)) return fail(KMX_ERR_UNSUPPORTED, "assign (half-precision sweep): LDS budget of %u bytes is too small", budget);
-	auto resident = [&](Rank16Copies copies, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, copies) + rank16_list_bytes(KB, a.layout, copies, entries) <= budget; };
-	Rank16Copies copies = w.copy_all || a.layout == KMX_AOS ? RANK16_EXCHANGED : RANK16_LISTED;
-	if (KB < 12 && w.copy_all && a.layout == KMX_SOA && !resident(copies, rank16_list_least(KB)) && resident(RANK16_DIRECT, rank16_list_least(KB))) copies = RANK16_DIRECT;
+	const Rank16Copies copies = a.layout == KMX_AOS ? RANK16_NONE : w.copy_all ? RANK16_ALL : RANK16_LISTED;
+	auto resident = [&](Rank16Copies room, uint32_t entries) { return (uint64_t)tiles * tile_bytes + rank16_static_bytes(KB, a.layout, false, room) + rank16_list_bytes(KB, entries) <= budget; };
 	/*
-	 * Without room to exchange rows, SoA points have a tile more in LDS. Beyond 128 dimensions that is too dear: what is left holds short lists, where the streamed form
-	 * has two work-groups of four wavefronts and whole ones (us per assignment, resident -> streamed: N = 192644, d = 133, k = 375 110 -> 79; N = 56454, d = 169, k = 368
-	 * 66 -> 49; N = 28000, d = 204, k = 274 1.13 of the time; up to 128 dimensions 0.90 to 1.06).
+	 * All rows go out only where the update has no columns' sums: more centroids than those fit LDS, and so than fit it here (or a recording without room for them). Without room to exchange rows, SoA points have a tile more in LDS.
+	 * Beyond 128 dimensions that is too dear: what is left holds short lists, where the streamed form has two work-groups of four wavefronts and whole ones (us per assignment,
+	 * resident -> streamed: N = 192644, d = 133, k = 375 110 -> 79; N = 56454, d = 169, k = 368 66 -> 49; N = 28000, d = 204, k = 274 1.13 of the time; up to 128 dimensions
+	 * 0.90 to 1.06).
 	 */
-	const bool stream_mode = !resident(KB >= 12 && copies == RANK16_LISTED ? RANK16_EXCHANGED : copies, rank16_list_least(KB));
+	const bool stream_mode = copies == RANK16_ALL || !resident(KB >= 12 && copies == RANK16_LISTED ? RANK16_ALL : copies, rank16_list_least(KB));
 	w.chunk_tiles = tiles;
 	w.list_entries = RANK16_LIST_MOST;
 	while (!stream_mode && !resident(copies, w.list_entries)) --w.list_entries;
-	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, a.layout, copies, w.list_entries);
+	uint32_t lds_bytes = tiles * tile_bytes + rank16_list_bytes(KB, w.list_entries);
 	const uint32_t static_bytes = rank16_static_bytes(KB, a.layout, stream_mode, copies);
 	if (stream_mode) {
 		w.chunk_tiles = 1;
 		while (rank16_slots(KB) == 2 && w.chunk_tiles < tiles && static_bytes + 2 * rank16_slot_bytes(KB, w.chunk_tiles + 1) <= budget) ++w.chunk_tiles;
 		lds_bytes = rank16_slots(KB) * rank16_slot_bytes(KB, w.chunk_tiles);
 	}
-	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true, RANK16_EXCHANGED> : rank16_kernel<KB, KMX_AOS, false, RANK16_EXCHANGED>)
-	                           : copies == RANK16_LISTED ? (stream_mode ? rank16_kernel<KB, KMX_SOA, true, RANK16_LISTED> : rank16_kernel<KB, KMX_SOA, false, RANK16_LISTED>)
-	                                                     : (stream_mode ? rank16_kernel<KB, KMX_SOA, true, RANK16_EXCHANGED> : rank16_kernel<KB, KMX_SOA, false, RANK16_EXCHANGED>);
-	if constexpr (KB < 12)
-		if (copies == RANK16_DIRECT) kernel = rank16_kernel<KB, KMX_SOA, false, RANK16_DIRECT>;
-	const uint32_t waves = rank16_waves(KB, a.layout, stream_mode, copies), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
+	void (*kernel)(Rank16Args) = a.layout == KMX_AOS ? (stream_mode ? rank16_kernel<KB, KMX_AOS, true, RANK16_NONE> : rank16_kernel<KB, KMX_AOS, false, RANK16_NONE>)
+	                           : copies == RANK16_ALL ? rank16_kernel<KB, KMX_SOA, true, RANK16_ALL>
+	                           : stream_mode ? rank16_kernel<KB, KMX_SOA, true, RANK16_LISTED> : rank16_kernel<KB, KMX_SOA, false, RANK16_LISTED>;
+	const uint32_t waves = rank16_waves(KB, stream_mode), unit = (stream_mode || KB > 4 ? waves : 1) * RANK16_P * TILE;
 	const uint32_t grid = std::min((a.n + unit - 1) / unit, (waves == 4 ? 2 : 1) * dev.compute_units);
 	exec->block_count = grid;
 #define KMX_PLAN(cond) do { if (!(cond)) return fail(KMX_ERR_DEVICE, "assign (half-precision sweep): launch refused, the plan breaks \"%s\" (dim %u, k %u, kp %u, n %u, chunk tiles %u, LDS %u)", \
@@ -1032,7 +1028,7 @@ static int launch_rank16_kb(const AssignArgs& a, Rank16Args w, kmx_exec_params* 
 	if (!sizing_only()) {
 		KMX_PLAN(w.kp % TILE == 0 && w.kp >= a.k && w.kp - a.k < TILE && a.n >= 1 && KB * KBLOCK >= a.dim);
 		KMX_PLAN(w.chunk_tiles >= 1 && (uint64_t)lds_bytes + static_bytes <= dev.lds_bytes && rank16_tile_floats<KB>() % 4 == 0);
-		KMX_PLAN(stream_mode || (w.list_entries >= RANK16_P * TILE / 2 && rank16_waves(KB, a.layout, false, copies) * 2 * w.list_entries + tiles * (tile_bytes / 4) <= lds_bytes / 4));
+		KMX_PLAN(stream_mode || (w.list_entries >= RANK16_P * TILE / 2 && rank16_waves(KB, false) * 2 * w.list_entries + tiles * (tile_bytes / 4) <= lds_bytes / 4));
 		KMX_PLAN(ws->packed16 && (size_t)tiles * KB * WAVE * 4 <= ws->packed16_cap);
 		KMX_PLAN(!stream_mode || ((rank16_slots(KB) == 2 || w.chunk_tiles == 1) && /* whole requests of norms, the last chunk's too */
 		                          (size_t)(tiles - 1) / w.chunk_tiles * w.chunk_tiles * NORM_TILE + rank16_norm_blocks(w.chunk_tiles) * WAVE <= ws->norms16_cap));
