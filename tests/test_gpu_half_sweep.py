@@ -76,8 +76,8 @@ def test_half_precision_products_accumulate_as_the_certificate_assumes(km, gpu, 
 
 
 @pytest.mark.parametrize("dim,k,n,mode", [(8, 130, 40001, 1), (50, 300, 70007, 1), (50, 60, 40003, 1), (9, 40, 33000, 1), (256, 129, 33001, 1), (300, 20, 33003, 1), (50, 300, 40000, 0), (390, 70, 33001, 0)])
-def test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, mode, budget=0):
-    """The columns, the assignment's copy of the rows, or the one made ahead of it, are what the update adds up."""
+def test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, mode):
+    """The assignment's copy of the rows, or the one made ahead of it, is what the update adds up."""
     rng = np.random.default_rng(dim + k)
     rows = rng.normal(size=(n, dim)).astype(np.float32)
     means = np.ascontiguousarray(rows[rng.choice(n, k, replace=False)])
@@ -87,14 +87,13 @@ def test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, k, n, mode
     o = km.DeviceBuffer(means.nbytes); a = km.DeviceBuffer(4 * n); s = km.DeviceBuffer(4 * k)
     km.set_two_level_sweep(mode)
     try:
-        km.iteration(d, 1, n, m, o, 1, k, a, s, dim, k, n, km.ExecParams(shared_mem_bytes=budget))
+        km.iteration(d, 1, n, m, o, 1, k, a, s, dim, k, n)
         km.sync()
     finally:
         km.set_two_level_sweep(1)
     assert np.array_equal(a.read(np.uint32, n), want)
     counts = np.bincount(want, minlength=k)
     assert np.array_equal(s.read(np.uint32, k), counts)
-    counts = np.maximum(counts, 1)
     sums = np.zeros((k, dim)); np.add.at(sums, want, rows.astype(np.float64))
     got = o.read(np.float32, k * dim).reshape(dim, k).T
     assert np.allclose(got, sums / counts[:, None], rtol=1e-5, atol=1e-6)
@@ -301,4 +300,25 @@ def test_wide_soa_rows_around_as_many_centroids_as_fit(km, orc, gpu, dim, k, str
 @pytest.mark.parametrize("dim", [12, 30, 45, 64, 90, 120, 180, 250])
 @pytest.mark.parametrize("n", [12011, 8191])
 def test_iterations_around_more_centroids_than_sums_fit(km, orc, gpu, dim, n):
-    test_iterations_on_soa_points_match_the_oracle(km, orc, gpu, dim, 6850, n, 2, 80 * 1024)
+    k = 6850
+    rng = np.random.default_rng(dim + k)
+    rows = rng.normal(size=(n, dim)).astype(np.float32)
+    means = np.ascontiguousarray(rows[rng.choice(n, k, replace=False)])
+    want = orc.assign(flat(rows, 0), flat(means, 0), dim, k, n, threads=0, fast=True)
+    d = km.DeviceBuffer(rows.nbytes); d.write(flat(rows, 1))
+    m = km.DeviceBuffer(means.nbytes); m.write(flat(means, 1))
+    o = km.DeviceBuffer(means.nbytes); a = km.DeviceBuffer(4 * n); s = km.DeviceBuffer(4 * k)
+    km.set_two_level_sweep(2)
+    try:
+        km.iteration(d, 1, n, m, o, 1, k, a, s, dim, k, n, km.ExecParams(shared_mem_bytes=80 * 1024))
+        km.sync()
+    finally:
+        km.set_two_level_sweep(1)
+    assert np.array_equal(a.read(np.uint32, n), want)
+    counts = np.bincount(want, minlength=k)
+    assert np.array_equal(s.read(np.uint32, k), counts)
+    sums = np.zeros((k, dim)); np.add.at(sums, want, rows.astype(np.float64))
+    got = o.read(np.float32, k * dim).reshape(dim, k).T
+    assert np.allclose(got, sums / np.maximum(counts, 1)[:, None], rtol=1e-5, atol=1e-6)
+    for b in (d, m, o, a, s):
+        b.free()
