@@ -9,7 +9,7 @@
  *   update_small_kernel  a work-group per range of clusters reads ALL memberships, lists its members, adds their rows and writes
  *                        finished centroids and sizes: no partial sums, nothing cleared before, nothing divided after.
  *
- * Where the general paths take over is measured; see small_assign_fits and small_update_fits.
+ * Where the general paths take over is measured; see small_assign_accepts (small_plan.h) and small_update_fits.
  */
 #include "kmx_internal.h"
 #include "small_plan.h"
