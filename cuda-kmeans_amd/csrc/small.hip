@@ -220,13 +220,14 @@ template <typename F, int T, int POINTS, uint32_t THREADS, int LD, int LM, bool 
 __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(F) == 4 && THREADS == 512 ? 8 : 4)))
 assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restrict__ means, size_t stride_means,
                     uint32_t* __restrict__ assignment, uint32_t dim, uint32_t k, uint32_t n, uint32_t row_stride, uint32_t chunk,
-                    uint32_t magic, uint32_t vec4, uint32_t* __restrict__ counters, F* __restrict__ partial, uint32_t* __restrict__ partial_counts)
+                    uint32_t magic, uint32_t vec4, uint32_t* __restrict__ counters, F* __restrict__ partial, uint32_t* __restrict__ partial_counts,
+                    uint32_t sums_width, uint32_t magic_width)
 {
 	typedef typename SmallVec<F>::type F4;
 	constexpr uint32_t PG = POINTS / 16 / T, CW = small_shares(T, POINTS, THREADS); /* groups of points, shares of the centroids */
 	extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
 	F* rows = (F*)lds_raw;
-	F* cents = rows + (size_t)POINTS * row_stride; /* chunk rows; with SUMS later k * dim doubles and k counts */
+	F* cents = rows + (size_t)POINTS * row_stride; /* chunk rows; with SUMS later k * sums_width doubles and k counts */
 	__shared__ SmallKey<F> cand[CW][POINTS];
 	__shared__ __attribute__((aligned(16))) uint32_t member[POINTS];
 	static_assert(sizeof(cand) + sizeof(member) == small_static_bytes(sizeof(F), T, POINTS, THREADS), "the plan's static arrays");
@@ -344,10 +345,10 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 		if (lc == 0) cand[cw][pg * (16 * T) + lp + 16 * p] = key;
 	}
 	__syncthreads();
-	double* sums = (double*)cents; /* SUMS: k * dim of them, then k counts; the centroids are no longer needed */
-	uint32_t* counts = (uint32_t*)(sums + k * dim);
+	double* sums = (double*)cents; /* SUMS: k * sums_width of them, then k counts; the centroids are no longer needed */
+	uint32_t* counts = (uint32_t*)(sums + k * sums_width);
 	if constexpr (SUMS) {
-		for (uint32_t i = tid; i < k * dim; i += THREADS) sums[i] = 0.0;
+		for (uint32_t i = tid; i < k * sums_width; i += THREADS) sums[i] = 0.0;
 		for (uint32_t i = tid; i < k; i += THREADS) counts[i] = 0u;
 	}
 	if (tid < POINTS) {
@@ -360,15 +361,33 @@ assign_small_kernel(const F* __restrict__ data, size_t stride, const F* __restri
 	}
 
 	if constexpr (SUMS) {
-		__syncthreads();
-		for (uint32_t e = tid; e < here * dim; e += THREADS) {
-			const uint32_t p = dim == 1 ? e : __umulhi(e, magic), q = e - p * dim;
-			unsafeAtomicAdd(&sums[member[p] * dim + q], (double)rows[p * row_stride + q]);
-		}
-		if (tid < here) atomicAdd(&counts[member[tid]], 1u);
-		__syncthreads();
 		F* out = partial + (size_t)blockIdx.x * k * dim;
-		for (uint32_t e = tid; e < k * dim; e += THREADS) out[e] = (F)sums[e];
+		if (sums_width == dim) {
+			__syncthreads();
+			for (uint32_t e = tid; e < here * dim; e += THREADS) {
+				const uint32_t p = dim == 1 ? e : __umulhi(e, magic), q = e - p * dim;
+				unsafeAtomicAdd(&sums[member[p] * dim + q], (double)rows[p * row_stride + q]);
+			}
+			if (tid < here) atomicAdd(&counts[member[tid]], 1u);
+			__syncthreads();
+			for (uint32_t e = tid; e < k * dim; e += THREADS) out[e] = (F)sums[e];
+		}
+		else { /* parts of two coordinates and more, the last one may be narrower (small_shape) */
+			for (uint32_t from = 0; from < dim; from += sums_width) {
+				__syncthreads();
+				for (uint32_t e = tid; e < here * sums_width; e += THREADS) {
+					const uint32_t p = __umulhi(e, magic_width), q = e - p * sums_width;
+					if (from + q < dim) unsafeAtomicAdd(&sums[member[p] * sums_width + q], (double)rows[p * row_stride + from + q]);
+				}
+				if (from == 0 && tid < here) atomicAdd(&counts[member[tid]], 1u);
+				__syncthreads();
+				for (uint32_t e = tid; e < k * sums_width; e += THREADS) {
+					const uint32_t c = __umulhi(e, magic_width), q = e - c * sums_width;
+					if (from + q < dim) out[c * dim + from + q] = (F)sums[e];
+					sums[e] = 0.0;
+				}
+			}
+		}
 		for (uint32_t i = tid; i < k; i += THREADS) partial_counts[(size_t)blockIdx.x * k + i] = counts[i];
 	}
 }
@@ -505,7 +524,7 @@ static int launch_assign_small_t(const F* data, int layout, size_t stride, const
 	*blocks = (n + shape.points - 1) / shape.points;
 	const uint32_t align = 4 * sizeof(F) - 1;
 	const uint32_t vec4 = (dim % 4 == 0 && stride % 4 == 0 && ((uintptr_t)data & align) == 0 ? 1u : 0u) | (dim % 4 == 0 && stride_means % 4 == 0 && ((uintptr_t)means & align) == 0 ? 2u : 0u);
-	void (*kernel)(const F*, size_t, const F*, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t*, F*, uint32_t*) = nullptr;
+	void (*kernel)(const F*, size_t, const F*, size_t, uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t*, F*, uint32_t*, uint32_t, uint32_t) = nullptr;
 #define KMX_PICK(P, Q, W) (layout == KMX_AOS ? (layout_means == KMX_AOS ? assign_small_kernel<F, P, Q, W, KMX_AOS, KMX_AOS, SUMS> : assign_small_kernel<F, P, Q, W, KMX_AOS, KMX_SOA, SUMS>) \
                                        : (layout_means == KMX_AOS ? assign_small_kernel<F, P, Q, W, KMX_SOA, KMX_AOS, SUMS> : assign_small_kernel<F, P, Q, W, KMX_SOA, KMX_SOA, SUMS>))
 	const bool few = shape.tile == 1;
@@ -513,7 +532,8 @@ static int launch_assign_small_t(const F* data, int layout, size_t stride, const
 #undef KMX_PICK
 	if (shape.lds_bytes > 48 * 1024) KMX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.lds_bytes));
 	KMX_LAUNCH_KERNEL(kernel, dim3(*blocks), dim3(shape.threads), shape.lds_bytes, stream(), data, stride, means, stride_means, assignment, dim, k, n,
-	                   small_row_stride(dim), assign_small_chunk(sizeof(F), dim, k), (uint32_t)((0x100000000ull + dim - 1) / dim), vec4, counters, partial, partial_counts);
+	                   small_row_stride(dim), assign_small_chunk(sizeof(F), dim, k), (uint32_t)((0x100000000ull + dim - 1) / dim), vec4, counters, partial, partial_counts,
+	                   shape.sums_width, shape.sums_width ? (uint32_t)((0x100000000ull + shape.sums_width - 1) / shape.sums_width) : 0u);
 	KMX_LAUNCH_CHECK("assign_small_kernel");
 	return KMX_OK;
 }

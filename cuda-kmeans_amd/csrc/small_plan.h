@@ -32,10 +32,11 @@ inline uint32_t assign_small_chunk(uint32_t value_bytes, uint32_t dim, uint32_t 
 	const uint32_t fit = 32 * 1024 / (small_row_stride(dim) * value_bytes) / 32 * 32;
 	return std::min(k, std::max(32u, fit));
 }
-inline uint32_t assign_small_lds(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t points, bool sums)
+/* sums_width: coordinates whose sums lie in LDS at a time, where the centroids were; 0: no sums */
+inline uint32_t assign_small_lds(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t points, uint32_t sums_width)
 {
 	const uint32_t centroids = assign_small_chunk(value_bytes, dim, k) * small_row_stride(dim) * value_bytes;
-	return points * small_row_stride(dim) * value_bytes + (sums ? std::max(centroids, k * dim * 8 + k * 4) : centroids);
+	return points * small_row_stride(dim) * value_bytes + (sums_width ? std::max(centroids, k * sums_width * 8 + k * 4) : centroids);
 }
 
 /*
@@ -67,13 +68,13 @@ inline bool small_assign_accepts(uint32_t value_bytes, bool columns, uint32_t di
 	if (n == 0 || n > SMALL_MAX_POINTS || dim > 256 || k > (1u << 20)) return false;
 	const uint64_t effort = std::max<uint64_t>(n, 256 * SMALL_POINTS) * k * (3 * (uint64_t)dim + 30);
 	const uint64_t limit = (value_bytes == 8 ? 2 * SMALL_EFFORT : small_more(columns, dim, n) ? SMALL_EFFORT_MORE : SMALL_EFFORT) * (dim > 32 ? 3 : 2) / 2;
-	return effort <= limit && assign_small_lds(value_bytes, dim, k, SMALL_POINTS, false) + small_static_room(value_bytes) <= lds_budget;
+	return effort <= limit && assign_small_lds(value_bytes, dim, k, SMALL_POINTS, 0) + small_static_room(value_bytes) <= lds_budget;
 }
 /* floats, points added up too (the partial sums of all work-groups are written and read once) */
 inline bool small_iteration_accepts(bool columns, uint32_t dim, uint32_t k, uint32_t n, uint32_t lds_budget)
 {
 	return (uint64_t)k * dim <= SMALL_SUMS && (uint64_t)k * dim * ((n + SMALL_POINTS - 1) / SMALL_POINTS) <= (2u << 20) && small_assign_accepts(4, columns, dim, k, n, lds_budget) &&
-	       assign_small_lds(4, dim, k, SMALL_POINTS, true) + small_static_room(4) <= lds_budget;
+	       assign_small_lds(4, dim, k, SMALL_POINTS, dim) + small_static_room(4) <= lds_budget;
 }
 
 /*
@@ -87,15 +88,31 @@ inline bool small_iteration_accepts(bool columns, uint32_t dim, uint32_t k, uint
  */
 constexpr uint32_t SMALL_HALF_POINTS = 128 * SMALL_POINTS, SMALL_WIDE_POINTS = 256 * SMALL_POINTS;
 
-struct SmallShape { uint32_t tile, points, threads, lds_bytes; /* without the static arrays */ };
+/* How many times all compute units are filled: work-groups of 512 lanes whose LDS, static arrays included, is given out in pieces of 1280 bytes, four a compute unit at most. */
+constexpr uint32_t small_rounds(uint32_t groups, uint32_t lds_bytes)
+{
+	const uint32_t each = 160 * 1024 / ((lds_bytes + 1279) / 1280 * 1280), resident = 256 * (each < 4 ? each : 4);
+	return resident ? (groups + resident - 1) / resident : groups;
+}
+
+struct SmallShape { uint32_t tile, points, threads, lds_bytes /* without the static arrays */, sums_width; };
 
 inline SmallShape small_shape(uint32_t value_bytes, uint32_t dim, uint32_t k, uint32_t n, bool sums, uint32_t lds_budget)
 {
 	const uint32_t tile = k > SMALL_FEW_CENTROIDS ? 2 : 1, points = n <= SMALL_HALF_POINTS ? SMALL_POINTS / 2 : SMALL_POINTS;
-	const uint32_t lds = assign_small_lds(value_bytes, dim, k, points, sums);
+	/*
+	 * Sums of doubles need more LDS than the centroids they replace. Where that takes a round of work-groups more, they are added up and written in parts of the coordinates, as few as make
+	 * up for it (us per iteration, whole / in parts / whole in floats, before: N = 24497, d = 220, k = 15 39.4 / 27.3 / 26.6; N = 38139, d = 208, k = 16 51.0 / 40.1 / 38.3;
+	 * N = 48841, d = 187, k = 3, SoA 32.1 / 26.2 / 25.7; assignment and update by themselves 26.5, 37.9, 30.6).
+	 */
+	uint32_t width = sums ? dim : 0;
+	const uint32_t groups = (n + points - 1) / points, held = small_static_bytes(value_bytes, tile, points, SMALL_THREADS);
+	const uint32_t least = small_rounds(groups, assign_small_lds(value_bytes, dim, k, points, 0) + held);
+	for (uint32_t parts = 2; sums && parts <= 4 && parts < dim && small_rounds(groups, assign_small_lds(value_bytes, dim, k, points, width) + held) > least; ++parts) width = (dim - 1) / parts + 1;
+	const uint32_t lds = assign_small_lds(value_bytes, dim, k, points, width);
 	const bool many = value_bytes == 4 || (k > 200 && dim <= 64) || (k <= SMALL_FEW_CENTROIDS && dim <= 16);
 	const bool wide = many && n > SMALL_HALF_POINTS && n <= SMALL_WIDE_POINTS && lds + small_static_bytes(value_bytes, tile, points, SMALL_WIDE_THREADS) <= lds_budget;
-	return SmallShape{ tile, points, wide ? SMALL_WIDE_THREADS : SMALL_THREADS, lds };
+	return SmallShape{ tile, points, wide ? SMALL_WIDE_THREADS : SMALL_THREADS, lds, width };
 }
 inline uint32_t assign_small_max_blocks(uint32_t n) { return n <= SMALL_HALF_POINTS ? (n + SMALL_POINTS / 2 - 1) / (SMALL_POINTS / 2) : (n + SMALL_POINTS - 1) / SMALL_POINTS; }
 

@@ -77,3 +77,10 @@ def test_small_inputs_under_a_callers_budget(km, orc, gpu, dim, k, budget):
         assert np.array_equal(a.read(np.uint32, n), want)
         for b in (d, m, a):
             b.free()
+
+
+@pytest.mark.parametrize("dim,k,n", [(220, 15, 24497), (221, 15, 16385), (208, 16, 38139), (252, 12, 25494), (187, 3, 48841), (164, 12, 34223), (255, 14, 32700), (136, 4, 60177)])
+def test_sums_in_parts_of_the_coordinates(km, orc, gpu, dim, k, n):
+    """Whole sums would take a round of work-groups more (small_shape)."""
+    for layout in (0, 1):
+        test_both_sides_of_the_lines(km, orc, gpu, dim, k, n, layout)

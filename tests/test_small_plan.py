@@ -89,3 +89,50 @@ def test_doubles_take_16_wavefronts_for_many_centroids(library, dim, k, n, threa
 @pytest.mark.parametrize("dim,k,n", [(2, 840, 3000), (4, 740, 8192), (20, 330, 16384), (90, 157, 5458), (254, 61, 8307)])
 def test_few_work_groups_stay(library, columns, dim, k, n):
     assert library.accepts(4, columns, dim, k, n)
+
+
+ROUNDS = """
+#include "small_plan.h"
+using namespace kmx;
+/* iterations whose sums, were they all in LDS at once, would take a round of work-groups more than the assignment, and of those the ones that still do; width: the least of all */
+extern "C" void rounds(int columns, uint64_t* whole, uint64_t* still, uint32_t* width)
+{
+	*whole = *still = 0;
+	*width = 1u << 30;
+	for (uint32_t n = 16385; n <= 65536; n += 997)
+		for (uint32_t dim = 1; dim <= 256; ++dim)
+			for (uint32_t k = 1; k * dim <= SMALL_SUMS; ++k) {
+				if (!small_iteration_accepts(columns != 0, dim, k, n, 160 * 1024)) continue;
+				const SmallShape s = small_shape(4, dim, k, n, true, 160 * 1024);
+				const uint32_t groups = (n + s.points - 1) / s.points, held = small_static_bytes(4, s.tile, s.points, s.threads);
+				const uint32_t least = small_rounds(groups, assign_small_lds(4, dim, k, s.points, 0) + held);
+				*whole += small_rounds(groups, assign_small_lds(4, dim, k, s.points, dim) + held) > least;
+				*still += small_rounds(groups, s.lds_bytes + held) > least;
+				if (s.sums_width < dim) *width = std::min(*width, s.sums_width);
+			}
+}
+extern "C" uint32_t width(uint32_t dim, uint32_t k, uint32_t n) { return small_shape(4, dim, k, n, true, 160 * 1024).sums_width; }
+"""
+
+
+@pytest.fixture(scope="module")
+def plan_of_sums(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("rounds")
+    src, lib = folder / "rounds.cpp", folder / "librounds.so"
+    src.write_text(ROUNDS)
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "cuda-kmeans_amd", "csrc"), str(src), "-o", str(lib)])
+    return ctypes.CDLL(str(lib))
+
+
+@pytest.mark.parametrize("columns", [0, 1])
+def test_sums_take_no_round_of_work_groups_more(plan_of_sums, columns):
+    whole, still, width = ctypes.c_uint64(), ctypes.c_uint64(), ctypes.c_uint32()
+    plan_of_sums.rounds(columns, ctypes.byref(whole), ctypes.byref(still), ctypes.byref(width))
+    assert whole.value > 0 and still.value == 0
+    assert width.value >= 2                                             # the kernel's division by the width
+
+
+# in parts where whole sums were slower, whole where they cost nothing
+@pytest.mark.parametrize("dim,k,n,parts", [(220, 15, 24497, 2), (208, 16, 38139, 2), (187, 3, 48841, 2), (20, 128, 10240, 1), (8, 64, 65536, 1), (100, 30, 20000, 1)])
+def test_sums_in_parts(plan_of_sums, dim, k, n, parts):
+    assert plan_of_sums.width(dim, k, n) == (dim if parts == 1 else (dim - 1) // parts + 1)
