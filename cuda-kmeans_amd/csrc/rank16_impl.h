@@ -234,8 +234,8 @@ __device__ __forceinline__ void rank16_exchanged() /* LDS keeps the order of a w
  * the matrix cores wait for the points, cost more than reading the columns' lines of the listed points once more from the memory-side
  * cache. us per assignment, all rows -> listed ones: N = 2M, d = 128, k = 1024, 9 % listed 854 -> 812 (without any copies 643), 1 % 808 -> 732; d = 32
  * 256 -> 222; N = 1M, d = 64, k = 500 162 -> 119; d = 90, k = 300 222 -> 157; N = 500000, d = 200, k = 1024 392 -> 331; nearly all listed (coordinates 0 or 1),
- * d = 64, k = 256 145 -> 89, d = 128, k = 512 193 -> 189; 1768 calls of up to 150000 points and 33 to 256 dimensions 0.96 in the mean, up to 1.22 where points that come together are
- * listed and a work-group has no further points meanwhile (N = 52692, d = 237, k = 284).
+ * d = 64, k = 256 145 -> 89, d = 128, k = 512 193 -> 189; 950 calls of 3000 to 300000 points and 24 to 256 dimensions 0.98 in the mean, 0.82 to 1.06, dearest where points that come
+ * together are listed and a work-group has no further points meanwhile (N = 52692, d = 237, k = 300, uniform points 61 -> 64).
  * All of them (ALL), on the way in and through LDS, so that four lanes store 64 consecutive bytes of a row, where the update behind it reads whole rows: iterations
  * with more centroids than fit a column's sums. `exchange`: RANK16_EXCHANGE words of this wavefront's. Otherwise a lane stores its 32 bytes as they are.
  */
